@@ -10,6 +10,7 @@
 
 #include "../../include/qtip_hip.h"
 #include "qtip_device.h"
+#include "qtip_setup.h"
 #include "qtip_wht.h"
 
 using namespace qtip;
@@ -1426,6 +1427,7 @@ Ready ready(bool launching, hipStream_t st) {
   int cus = 0;
   hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (e == hipSuccess) e = allow_lds_all();
+  if (e == hipSuccess) e = qtip_rht_allow_lds();
   float* sp = nullptr;
   if (e == hipSuccess) e = hipGetSymbolAddress(reinterpret_cast<void**>(&sp), HIP_SYMBOL(scratch));
   if (e == hipSuccess && !sp) e = hipErrorInvalidSymbol;
@@ -1491,6 +1493,12 @@ int choose_split(int m, int k, int bits, int cus, bool summed) {
 }
 
 }  // namespace
+
+int qtip_device_ready(void* stream, int* cus) {
+  const Ready r = ready(stream);
+  *cus = r.cus;
+  return r.rc;
+}
 
 extern "C" {
 

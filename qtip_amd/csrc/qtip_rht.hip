@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "../../include/qtip_hip.h"
+#include "qtip_setup.h"
 #include "qtip_wht.h"
 
 using namespace qtip_wht;
@@ -726,8 +727,55 @@ int launch_rht_rows(const RhtParams& P, int rows, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+#include "qtip_rht_mix.h"
+
+constexpr int mix_class(int kt) { return kt <= 2 ? 2 : (kt <= 4 ? 4 : 8); }
+
+template <typename TI, typename TO, int MODE>
+int launch_mix(const RhtParams& P, const MixShape& M, int kt, int rows, int cus, hipStream_t st) {
+  const int ktc = mix_class(kt);
+  const size_t lds = mix_lds(ktc, P.order);
+  // workgroups a CU holds: LDS, and four waves of 128 registers per SIMD
+  const int fit = (int)((160u * 1024) / lds) < kMixMaxKT / kt ? (int)((160u * 1024) / lds) : kMixMaxKT / kt;
+  const int most = cus * (fit < 1 ? 1 : fit) >> M.logS;
+  const int gx = M.npass < most ? M.npass : (most < 1 ? 1 : most);
+  const dim3 grid((unsigned)gx, 1u << M.logS);
+  if (ktc == 2) rht_mix_kernel<TI, TO, MODE, 2><<<grid, 128 * kt, lds, st>>>(P, M, rows);
+  else if (ktc == 4) rht_mix_kernel<TI, TO, MODE, 4><<<grid, 128 * kt, lds, st>>>(P, M, rows);
+  else rht_mix_kernel<TI, TO, MODE, 8><<<grid, 128 * kt, lds, st>>>(P, M, rows);
+  return (int)hipGetLastError();
+}
+
+// shape of the matrix form for `rows` rows; false where it does not apply
+bool mix_shape(int n, int order, int rows, MixShape& M, int& kt) {
+  int logp = 0;
+  while ((n / order) >> (logp + 1)) ++logp;
+  if (logp < 3 || order > 32 * kMixMaxKT) return false;
+  int logpp = logp < 7 ? logp : 7;
+  // fill the 32 rows of a wave before widening the columns
+  while (logpp > 3 && ((long)order << (logp - logpp)) < 32) --logpp;
+  M.logpp = logpp;
+  M.logA2 = logp - logpp;
+  M.logS = 0;
+  while (((long)order << M.logA2) > 32 * kMixMaxKT) {
+    --M.logA2;
+    ++M.logS;
+  }
+  kt = ((order << M.logA2) + 31) >> 5;
+  const int rpp = kMixCols >> logpp;
+  M.npass = (rows + rpp - 1) / rpp;
+  return true;
+}
+
 // rows from which the one-workgroup-per-row form is used for the power-of-two sizes it covers
 constexpr int kRowsFormMin = 8;
+
+// Rows from which the matrix form is faster than one launch of order * A workgroups per row, which
+// each read the whole row.  Measured (us, that form / matrix form): fp16 rows of 12288 = 12 * 1024
+// 7.1 / 6.9 at 8 rows, 9.8 / 6.9 at 16; 28672 = 28 * 1024 9.2 / 11.2 at 8, 16.5 / 11.3 at 16;
+// 11008 = 172 * 64 15.4 / 10.8 at 8.  fp32 rows take three planes: 28672 16.5 / 21 at 16, 42 / 22 at
+// 45; 11008 15.4 / 19 at 8, 26 / 19 at 16.
+constexpr int mix_rows_min(int order, bool f16) { return order >= 100 ? (f16 ? 8 : 12) : (f16 ? 12 : 24); }
 
 int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream) {
   if (!P.out || !P.in) return QTIP_E_NULL;
@@ -769,6 +817,28 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
       if (in_dtype == QTIP_F16) return launch_rht_rows<_Float16, float>(P, rows, st);
       if (out_dtype == QTIP_F16) return launch_rht_rows<float, _Float16>(P, rows, st);
       return launch_rht_rows<float, float>(P, rows, st);
+    }
+  }
+  if (rows >= mix_rows_min(order, in_dtype == QTIP_F16)) {
+    const size_t ez = in_dtype == QTIP_F16 ? 2 : 4;
+    MixShape M{};
+    int kt = 0;
+    auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    const bool ok = (n & 7) == 0 && al(P.in) && al(P.out) && al(P.pre) && al(P.post) && al(P.norm_w) && al(P.residual) &&
+                    ((P.in_row_stride * ez) & 15u) == 0 && ((P.part_stride * ez) & 15u) == 0 &&
+                    ((P.pre_row_stride * 2) & 15u) == 0 && ((P.post_row_stride * 4) & 15u) == 0 &&
+                    !(P.pre_mode != PRE_NONE && in_dtype != QTIP_F16) && !(fused && out_dtype != QTIP_F16) &&
+                    mix_shape(n, order, rows, M, kt);
+    if (ok) {
+      int cus = 0;
+      const int rc = qtip_device_ready(stream, &cus);
+      if (rc) return rc;
+      if (P.pre_mode == PRE_RMSNORM) return launch_mix<_Float16, _Float16, PRE_RMSNORM>(P, M, kt, rows, cus, st);
+      if (P.pre_mode == PRE_SILU_MUL) return launch_mix<_Float16, _Float16, PRE_SILU_MUL>(P, M, kt, rows, cus, st);
+      if (in_dtype == QTIP_F16 && out_dtype == QTIP_F16) return launch_mix<_Float16, _Float16, PRE_NONE>(P, M, kt, rows, cus, st);
+      if (in_dtype == QTIP_F16) return launch_mix<_Float16, float, PRE_NONE>(P, M, kt, rows, cus, st);
+      if (out_dtype == QTIP_F16) return launch_mix<float, _Float16, PRE_NONE>(P, M, kt, rows, cus, st);
+      return launch_mix<float, float, PRE_NONE>(P, M, kt, rows, cus, st);
     }
   }
   if (fused && out_dtype != QTIP_F16) return QTIP_E_DTYPE;  // fused forms exist for the combinations the decode loop uses
@@ -912,6 +982,22 @@ __global__ __launch_bounds__(kRhtThreads) void rht_chain_kernel(
 }
 
 }  // namespace
+
+// LDS opt-in of this file's kernels, part of the device set-up
+hipError_t qtip_rht_allow_lds() {
+#define QTIP_MIX3(TI, TO, MODE)                                                                       \
+  (const void*)rht_mix_kernel<TI, TO, MODE, 2>, (const void*)rht_mix_kernel<TI, TO, MODE, 4>, \
+      (const void*)rht_mix_kernel<TI, TO, MODE, 8>
+  const void* fns[] = {QTIP_MIX3(_Float16, _Float16, PRE_RMSNORM), QTIP_MIX3(_Float16, _Float16, PRE_SILU_MUL),
+                       QTIP_MIX3(_Float16, _Float16, PRE_NONE),    QTIP_MIX3(_Float16, float, PRE_NONE),
+                       QTIP_MIX3(float, _Float16, PRE_NONE),       QTIP_MIX3(float, float, PRE_NONE)};
+#undef QTIP_MIX3
+  for (const void* f : fns) {
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix_lds(kMixMaxKT, 172));
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
 
 extern "C" {
 

@@ -1,0 +1,79 @@
+"""Transforms of many rows on the matrix cores against float64 matrices, at the edges of their tiling."""
+import numpy as np
+import pytest
+import scipy.linalg
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _transform(x, n, transpose):
+    """sqrt(n) * (H_K (x) H_p) x in float64 on the device (x: float64 rows)."""
+    from qtip_amd.utils.matmul_had import get_hadK
+    had, K = get_hadK(n)
+    p = n // K
+    z = x.view(-1, K, p) @ torch.from_numpy(scipy.linalg.hadamard(p).astype(np.float64)).cuda()
+    if had is not None:
+        h = had.double().cuda()
+        z = (h.T if transpose else h) @ z
+    return z.reshape(-1, n)
+
+
+# power-of-two parts of 8 to 2048: one to sixteen rows per pass, table orders that fill their k tiles and
+# ones that leave 4 to 28 padding rows, one and two slices (53248, 57344), a workgroup of one to eight tiles
+@pytest.mark.parametrize("n", [256, 832, 928, 1120, 1248, 3328, 5120, 10240, 11008, 12288, 14336, 16384, 22016, 28672,
+                               53248, 57344])
+@pytest.mark.parametrize("rows", [24, 37])
+def test_rows_against_float64(n, rows):
+    from qtip_amd import ops
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    had, K = get_hadK(n)
+    g = torch.Generator(device="cuda").manual_seed(n + rows)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    for dt_in, dt_out, transpose, pre_kind, scale_in in (
+            (torch.float16, torch.float16, True, "sign", 1.0), (torch.float16, torch.float32, False, "real", 1.0),
+            (torch.float32, torch.float16, True, "sign", 1.0), (torch.float32, torch.float32, False, "real", 1e-6),
+            (torch.float16, torch.float32, False, None, 1.0), (torch.float32, torch.float32, True, None, 1e6)):
+        x = (rnd(rows, n) * scale_in).to(dt_in)
+        pre = post = None
+        if pre_kind:
+            pre = torch.sign(rnd(n) + 1e-5)
+            pre = (pre if pre_kind == "sign" else pre * (0.5 + torch.rand(n, generator=g, device="cuda"))).half()
+            post = rnd(n)
+        got = ops.rht(x, order=K, had_bits=had_bits(had, K, transpose, "cuda") if K > 1 else None, pre=pre, post=post,
+                      out_dtype=dt_out)
+        ref = _transform(x.double() * (1 if pre is None else pre.double()), n, transpose) * n**-0.5
+        ref = ref * (1 if post is None else post.double())
+        # exact products, fp32 sums of n terms (n * 2^-24 in the worst case, sqrt(n) of it in these) and fp16 results
+        tol = 1e-3 if dt_out == torch.float16 else 1e-5
+        assert got.dtype == dt_out and float((got.double() - ref).abs().max()) <= tol * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("n", [928, 4096, 11008, 28672, 57344])
+@pytest.mark.parametrize("sign", [True, False])
+def test_rows_with_prologue_and_residual(n, sign):
+    """The element-wise neighbours folded into the many-row form: same fp16 rounding points as the
+    single-row forms, whose sums run in another order (an fp16 ulp)."""
+    from qtip_amd import ops
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    had, K = get_hadK(n)
+    rows = 29
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    bits = had_bits(had, K, True, "cuda") if K > 1 else None
+    pre = torch.sign(rnd(n) + 1e-5)
+    pre = (pre if sign else pre * 1.25).half()
+    w = (1 + 0.1 * rnd(n)).half()
+    x, gu, res = rnd(rows, n).half(), rnd(rows, 2 * n).half(), rnd(rows, n).half()
+    kw = dict(order=K, had_bits=bits, pre=pre, out_dtype=torch.float16)
+    close = lambda a, b: float((a.float() - b.float()).abs().max()) <= 2e-3 * float(b.float().abs().max())
+    if n <= 16384:  # the single-row form of the norm holds the vector in registers
+        got = ops.rht(x, pre_mode=ops.PRE_RMSNORM, norm_weight=w, eps=1e-5, **kw)
+        one = torch.cat([ops.rht(x[i:i + 1], pre_mode=ops.PRE_RMSNORM, norm_weight=w, eps=1e-5, **kw) for i in (0, 17, 28)])
+        assert close(got[[0, 17, 28]], one)
+    got = ops.rht(gu, pre_mode=ops.PRE_SILU_MUL, **kw)
+    one = torch.cat([ops.rht(gu[i:i + 1], pre_mode=ops.PRE_SILU_MUL, **kw) for i in (0, 17, 28)])
+    assert close(got[[0, 17, 28]], one)
+    got = ops.rht(x, residual=res, **kw)
+    one = torch.cat([ops.rht(x[i:i + 1], residual=res[i:i + 1], **kw) for i in (0, 17, 28)])
+    assert close(got[[0, 17, 28]], one)
