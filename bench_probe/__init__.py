@@ -47,14 +47,7 @@ def build(verbose=True):
 def build_stamped(verbose=True):
     """The timeline build of libqtip_hip.so (same sources and flags, plus -DQTIP_STAMPS)."""
     from qtip_amd import build as qbuild
-    cmd = [os.environ.get("HIPCC", "hipcc")] + qbuild.HIPCC_FLAGS + ["-DQTIP_STAMPS"] + qbuild.SRCS + \
-        ["-o", STAMPED_LIB_PATH + ".tmp"]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + "\n".join(l for l in res.stderr.splitlines() if "packed-fp32-ops" not in l))
-    os.replace(STAMPED_LIB_PATH + ".tmp", STAMPED_LIB_PATH)
+    qbuild.compile_library(STAMPED_LIB_PATH, ["-DQTIP_STAMPS"], verbose)
     return STAMPED_LIB_PATH
 
 

@@ -186,6 +186,12 @@ int qtip_decompress_gemm(float* out, const void* packed, const void* x_f16,
                          const void* tlut, int m, int k, int bits, int batch,
                          int round_f16, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same product with the fp16-rounded results stored as fp16 (what the reference's fp16 GEMM returns
+ * before .float(): half the bytes, and the output transform reads fp16 as it is). */
+int qtip_decompress_gemm_f16(void* out_f16, const void* packed, const void* x_f16, const void* tlut, int m,
+                             int k, int bits, int batch, void* workspace, size_t workspace_bytes,
+                             void* stream);
+
 /* Randomised Hadamard transform of `rows` vectors of length n = order * p
  * (p a power of two, order 1 or a table order):
  *   out[r][:] = post[:] * scale * (H_order (x) H_p) (pre[:] * in[r][:])

@@ -2,31 +2,46 @@
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SRCS = [os.path.join(HERE, "csrc", f) for f in ("qtip_hip.hip", "qtip_rht.hip", "qtip_decoder.hip", "qtip_pack.hip")]
+SRCS = [os.path.join(HERE, "csrc", f)
+        for f in ("qtip_hip.hip", "qtip_gemm.hip", "qtip_rht.hip", "qtip_decoder.hip", "qtip_pack.hip")]
 OUT = os.path.join(HERE, "libqtip_hip.so")
 
 # packed fp32 VALU forms are switched off for every HIP translation unit
 HIPCC_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
 
-def build(verbose=True):
-    hipcc = os.environ.get("HIPCC", "hipcc")
-    cmd = [hipcc] + HIPCC_FLAGS + SRCS + ["-o", OUT + ".tmp"]
+def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     err = "\n".join(l for l in res.stderr.splitlines() if "packed-fp32-ops" not in l)
     if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed:\n{err}")
+        raise RuntimeError(f"{cmd[0]} failed:\n{err}")
     if err.strip() and verbose:
         print(err, file=sys.stderr)
-    os.replace(OUT + ".tmp", OUT)
-    return OUT
+
+
+def compile_library(out, extra=(), verbose=True):
+    """The library's sources, compiled side by side (hipcc takes them one after the other), into `out`."""
+    hipcc = os.environ.get("HIPCC", "hipcc")
+    with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor(len(SRCS)) as pool:
+        objs = [os.path.join(tmp, os.path.basename(s) + ".o") for s in SRCS]
+        list(pool.map(lambda so: _run([hipcc] + HIPCC_FLAGS + list(extra) + ["-c", so[0], "-o", so[1]], verbose),
+                      zip(SRCS, objs)))
+        _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", out + ".tmp"], verbose)
+    os.replace(out + ".tmp", out)
+    return out
+
+
+def build(verbose=True):
+    return compile_library(OUT, verbose=verbose)
 
 
 if __name__ == "__main__":

@@ -137,40 +137,6 @@ __global__ __launch_bounds__(kThreads, 1) void decode_kernel(uint16_t* __restric
 constexpr size_t kMatvecLds = kLut128Bytes + 2 * kWaves * 32 * sizeof(float);
 constexpr size_t kMatvecXBytes = 28 * 1024;  // LDS left for the x values of a workgroup's k range
 
-// Buffer-addressed streaming loads: the address is (SGPR descriptor, SGPR byte
-// offset, per-lane VGPR offset), so walking the stream costs no vector ALU work.
-template <int K>
-__device__ __forceinline__ LaneData<K> load_lane_buf(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff,
-                                                     uint32_t soff) {
-  LaneData<K> r;
-  // Non-temporal where a load instruction covers whole cache lines (one 16-byte load per lane at 2
-  // bits) or nearly so (3 bits): the stream is read once.  At 4 bits a lane's two 16-byte loads
-  // split every line between two instructions, and with the hint the second one fetches the line
-  // from L2 again: plain loads are 10 % faster there (57344x8192: 47.7 -> 41.5 us).
-  constexpr int NT = K == 4 ? 0 : 2;
-  if constexpr (K == 2) {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, NT);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r.d[i] = v[i];
-  } else if constexpr (K == 3) {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, NT);
-    const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(rsrc, voff + 16, soff, NT);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r.d[i] = v[i];
-    r.d[4] = w[0];
-    r.d[5] = w[1];
-  } else {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, NT);
-    const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff + 16, soff, NT);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      r.d[i] = v[i];
-      r.d[4 + i] = w[i];
-    }
-  }
-  return r;
-}
-
 // x for a lane's columns of a wave-load: 4 x (4 consecutive fp16), 16 bytes apart
 __device__ __forceinline__ void load_x_buf(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff,
                                            u32x2 xv[4]) {
@@ -743,592 +709,6 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(float* __restrict__ out,
 }
 
 // ---------------------------------------------------------------------------
-// batched decompress + fp16 MFMA GEMM
-// ---------------------------------------------------------------------------
-// out[b][row] = sum_col x[b][col] * W[row][col] with v_mfma_f32_16x16x32_f16:
-// M = 16 batch rows, N = the 16 lanes of a DPP row, K = 32 columns.
-//
-// The decode leaves, for every (tile row half mh, row half rh, kh), in lane
-// (g, a) the eight weights of matrix row 16*mh + 8*rh + a/2 at columns
-// 32*g' + 16*kh + 4*(a%2) + {0..3, 8..11} (g' = the lane group's tile block):
-// exactly the shape of an MFMA B operand (N index = a, K group = g), except
-// that even and odd lanes hold different columns (the 4*(a%2) term).  Each
-// product is therefore issued twice, once with the activations of columns
-// +0..3 / +8..11 and once with +4..7 / +12..15, into two accumulators; in the
-// first the even lanes' results are meaningful, in the second the odd lanes',
-// and the other half is simply never read.  That spends half of the matrix
-// core's work, which is free here (the kernel is bound by the decode), and
-// needs no data movement between decode and MFMA: the table lookups land in
-// the operand registers.
-//
-// Activations are shared through LDS: a workgroup (8 waves) works on 4 consecutive 32-row blocks
-// at the same columns - wave w takes row block w % 4 and, of each pair of wave-loads, number
-// w / 4 - so one 16*NB x 256 activation tile per stage serves all eight waves (read from L2 once
-// per 128 matrix rows instead of once per 32; the per-wave reads measured 35-50 % of the run
-// time before).  Tiles are double-buffered: loaded to registers two stages ahead, written to
-// LDS one stage ahead, one barrier per stage.  Rows of the tile are 512 bytes with the 16-byte
-// chunk index xor-ed with the row, which keeps both the 16-byte fills and the A-operand reads
-// (16 lanes = 16 rows at the same chunk) free of bank conflicts.
-// Work unit = (group of 4 row blocks, k split s); a workgroup keeps one s, so its sequence of
-// activation tiles is the same for every unit and the pipeline runs across unit boundaries.
-// S > 1 (few row blocks): fp32 partial results go to parts[s][batch][m] and are summed afterwards.
-constexpr int kGemmRB = 4;  // row blocks per group
-// Two shapes of workgroup: 8 waves (2 k slices, up to 256 VGPRs: two batch tiles) and 16 waves
-// (4 k slices, 128 VGPRs: one batch tile, twice the waves to hide the latencies of a stage).
-constexpr size_t kGemmTileBytes = 16 * 1024;  // 16*NB batch rows x 256*KS columns fp16, NB*KS == 4
-constexpr size_t kGemmLds = kLut128Bytes + 2 * kGemmTileBytes;
-
-template <int K, int NB, int DEPTH, int WAVES>
-__global__ __launch_bounds__(WAVES * 64, 1) void gemm_kernel(
-    float* __restrict__ dst, const uint8_t* __restrict__ packed, const uint16_t* __restrict__ x,
-    const uint32_t* __restrict__ tlut, int m, int k, int batch, int round_f16, int wl_per, int upw_q,
-    int upw_r) {
-  constexpr int THREADS = WAVES * 64;
-  constexpr int KS = WAVES / kGemmRB;          // wave-loads per stage
-  constexpr int ROWB = KS * 256;               // bytes per tile row
-  constexpr int CPR = ROWB / 16;               // 16-byte chunks per tile row
-  constexpr uint32_t TILE = 16 * NB * ROWB;
-  static_assert(2 * TILE <= 2 * kGemmTileBytes, "tiles do not fit");
-  static_assert(16 * NB * CPR == NB * THREADS, "NB chunks per thread and tile");
-  extern __shared__ __align__(16) uint8_t smem[];
-  uint32_t* lut = reinterpret_cast<uint32_t*>(smem);
-  uint8_t* tiles = smem + kLut128Bytes;  // [2][16*NB rows][ROWB bytes]
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rbi = wave & (kGemmRB - 1), ks = wave >> 2;
-  const int a = lane & 15, g = lane >> 4;
-  const uint32_t slot4 = lds_address(lut) + ((uint32_t)(lane & 31) << 2);
-  const int nkb = k >> 5;
-  const int nwl = (nkb + 3) >> 2;  // wave-loads per row block; a partial last one meets zero activations
-  const int nrb = m >> 5;
-  const int ngroups = (nrb + kGemmRB - 1) / kGemmRB;
-  const uint32_t rb_bytes = (uint32_t)nkb * 128 * K;
-  constexpr uint32_t WL_BYTES = 512 * K;
-  const uint32_t loff = (uint32_t)lane * 8 * K;
-  const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(packed), 0, (int)((size_t)nrb * rb_bytes), 0x00020000);
-
-  // grid = (S, workgroups per k range); unit counts as quotient and remainder from the host:
-  // no integer division on the way to the first loads
-  const int s = blockIdx.x;
-  const int g0 = blockIdx.y, gstep = gridDim.y;
-  const int wl0 = s * wl_per;                                   // wl_per is a multiple of KS
-  const int wl1 = wl0 + wl_per < nwl ? wl0 + wl_per : nwl;
-  const int nst = wl1 > wl0 ? (wl1 - wl0 + KS - 1) / KS : 0;    // stages (KS wave-loads each) per unit
-  const int upw = upw_q + (g0 < upw_r ? 1 : 0);  // units of this workgroup: ceil((ngroups - g0) / gstep)
-  const int T = upw * nst;
-  float* out_s = dst + (size_t)s * batch * m;
-
-  // ---- weight stream of this wave: item q = (unit q / nst, stage q % nst), DEPTH in flight
-  int l_t = 0, l_q = 0, l_grp = g0;
-  LaneData<K> buf[DEPTH];
-  auto issue = [&](int d) {
-    const int rb = l_grp * kGemmRB + rbi;
-    const int wl = wl0 + KS * l_t + ks;
-    const bool valid = l_q < T && rb < nrb && wl < wl1;
-    // padding items, and the lanes past the row's end in a partial last wave-load (k / 32 not a
-    // multiple of 4): a lane offset that is out of range by itself, zeros without a memory access
-    const bool lane_ok = valid && 4 * wl + g < nkb;
-    buf[d] = load_lane_buf<K>(rs_w, lane_ok ? loff : 0x7FFFFF00u,
-                              valid ? (uint32_t)rb * rb_bytes + (uint32_t)wl * WL_BYTES : 0u);
-    ++l_q;
-    if (++l_t == nst) {
-      l_t = 0;
-      l_grp += gstep;
-    }
-  };
-  // table words first (their loads return before the stream's), one stage of the stream before the
-  // table is built, the others once the workgroup is past its first barrier
-  constexpr int NTW = kLutEntries * 4 / THREADS;  // distinct table words per thread
-  uint32_t tw[NTW];
-#pragma unroll
-  for (int j = 0; j < NTW; ++j) {
-    // the wave's eight words of a pass through the scalar cache (uniform address), lane l keeps word l / 8
-    const uint32_t* tp = tlut + j * (THREADS / 8) + wave * 8;
-    uint32_t v = tp[0];
-#pragma unroll
-    for (int e = 1; e < 8; ++e) v = ((lane >> 3) == e) ? tp[e] : v;
-    tw[j] = v;
-  }
-  issue(0);
-
-  // ---- activation tiles: thread fills NB 16-byte chunks per tile
-
-  static_assert(DEPTH % 2 == 0, "stage parity must be static inside the unrolled loop");
-  u32x4 xg[2][NB];  // tiles on their way: [parity of the stage][chunk]
-  auto load_tile = [&](int slot, int t) {  // stage t of a unit -> registers
-    const int col0 = 128 * (wl0 + KS * t);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int idx = i * THREADS + tid;
-      const int b = idx / CPR, c = idx % CPR;
-      const int col = col0 + 8 * c;
-      u32x4 v = {0u, 0u, 0u, 0u};
-      if (b < batch && col < k) v = *reinterpret_cast<const u32x4*>(x + (size_t)b * k + col);
-      xg[slot][i] = v;
-    }
-  };
-  auto store_tile = [&](int slot, int bufi) {  // registers -> LDS buffer
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int idx = i * THREADS + tid;
-      const int b = idx / CPR, c = idx % CPR;
-      *reinterpret_cast<u32x4*>(tiles + bufi * TILE + b * ROWB + ((c ^ (b & 7)) << 4)) = xg[slot][i];
-    }
-  };
-  load_tile(0, 0);
-  load_tile(1, nst > 1 ? 1 : 0);
-#pragma unroll
-  for (int it = 0; it < kLutEntries * 8 / THREADS; ++it) {
-    // item it*THREADS + tid belongs to entry it*THREADS/8 + tid/8; entries e and e+512 share a word
-    const uint32_t w = tw[it % NTW] ^ ((uint32_t)(it / NTW) << 15);
-    const u32x4 v = {w, w, w, w};
-    reinterpret_cast<u32x4*>(lut)[it * THREADS + tid] = v;
-  }
-  store_tile(0, 0);
-  __syncthreads();
-#pragma unroll
-  for (int d = 1; d < DEPTH; ++d) issue(d);
-
-  float4_t acc[2][2][2][NB];  // [mh][rh][column half][batch tile]
-#pragma unroll
-  for (int i = 0; i < 8 * NB; ++i) (&acc[0][0][0][0])[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-  // LDS byte offset (inside a tile) of this lane's A-operand chunks: row 16*nb + a, chunk 16*ks + 4*g + 2*kh + h
-  uint32_t arow[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) arow[nb] = (uint32_t)(16 * nb + a) * ROWB;
-  const uint32_t a7 = (uint32_t)(a & 7);
-  const uint32_t tiles_addr = lds_address(tiles);
-
-  int c_t = 0, c_grp = g0;
-  for (int q = 0; q < T; q += DEPTH) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      const bool live = q + d < T;  // uniform over the workgroup
-      if (live) {
-        // tile of stage q+d+2 to registers (slot = parity of that stage = parity of q+d)
-        {
-          int t2 = c_t + 2;
-          if (t2 >= nst) t2 -= nst;
-          if (t2 >= nst) t2 -= nst;  // nst == 1
-          load_tile((q + d) & 1, t2);
-        }
-        const int rb = c_grp * kGemmRB + rbi;
-        const int wl = wl0 + KS * c_t + ks;
-        if (rb < nrb && wl < wl1) {
-          typedef __attribute__((address_space(3))) const u32x4 lds_u32x4_t;
-          const uint32_t tb = tiles_addr + (uint32_t)((q + d) & 1) * TILE;
-          uint32_t P[16], W[32];
-          packed_states<K>(buf[d], P);
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const uint32_t hq = pk_hash(P[i]) & 0xFFC0FFC0u;
-            W[2 * i] = lds_word_abs(lut128_addr_lo(hq, slot4));
-            W[2 * i + 1] = lds_word_abs(lut128_addr_hi(hq, slot4));
-          }
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int kh = 0; kh < 2; ++kh) {
-            u32x4 xa[NB][2];
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-              for (int h = 0; h < 2; ++h) {
-                const uint32_t c = (uint32_t)(16 * ks + 4 * g + 2 * kh + h) ^ a7;
-                xa[nb][h] = *(lds_u32x4_t*)(uintptr_t)(tb + arow[nb] + (c << 4));
-              }
-#pragma unroll
-            for (int mh = 0; mh < 2; ++mh)
-#pragma unroll
-              for (int rh = 0; rh < 2; ++rh) {
-                const int tt = 2 * kh + mh;
-                const u32x4 wv = {W[w_index<K>(0, tt, rh)], W[w_index<K>(1, tt, rh)],
-                                  W[w_index<K>(0, tt, 2 + rh)], W[w_index<K>(1, tt, 2 + rh)]};
-                const half8_t bop = __builtin_bit_cast(half8_t, wv);
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                  for (int ch = 0; ch < 2; ++ch) {
-                    // columns +4*ch+{0..3} and +8+4*ch+{0..3} of the 16 loaded ones
-                    const u32x4 xv = {xa[nb][0][2 * ch], xa[nb][0][2 * ch + 1], xa[nb][1][2 * ch],
-                                      xa[nb][1][2 * ch + 1]};
-                    acc[mh][rh][ch][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                        __builtin_bit_cast(half8_t, xv), bop, acc[mh][rh][ch][nb], 0, 0, 0);
-                  }
-              }
-          }
-        }
-      }
-      issue(d);
-      if (live) {
-        // tile of the next stage (in registers since the previous stage) into the other buffer
-        store_tile((q + d + 1) & 1, (q + d + 1) & 1);
-        __syncthreads();
-        if (++c_t == nst) {
-          // ---- end of a unit: the k slices of a row block meet in the buffer this stage used
-          // (the next tile sits in the other one): slices 1 .. KS-1 hand their sums over in turn,
-          // the wave of slice 0 adds them in that order, rounds and stores
-          float* xch = reinterpret_cast<float*>(tiles + ((q + d) & 1) * TILE) + rbi * (16 * NB * 32);
-          float vals[2][2][NB][4];
-#pragma unroll
-          for (int mh = 0; mh < 2; ++mh)
-#pragma unroll
-            for (int rh = 0; rh < 2; ++rh)
-#pragma unroll
-              for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                  // even lanes: own sum of the even columns + the odd neighbour's sum of the odd columns
-                  // (no per-lane choice before the exchange, see matvec_kernel)
-                  vals[mh][rh][nb][i] = acc[mh][rh][0][nb][i] + dpp_xor1(acc[mh][rh][1][nb][i]);
-                  acc[mh][rh][0][nb][i] = 0.f;
-                  acc[mh][rh][1][nb][i] = 0.f;
-                }
-          const int e0 = ((a >> 1) + 8 * g) * (16 * NB);  // even lanes: 32 slots of 16*NB floats
-          for (int turn = 1; turn < KS; ++turn) {
-            if (ks == turn && (a & 1) == 0) {
-#pragma unroll
-              for (int mh = 0; mh < 2; ++mh)
-#pragma unroll
-                for (int rh = 0; rh < 2; ++rh)
-#pragma unroll
-                  for (int nb = 0; nb < NB; ++nb)
-                    *reinterpret_cast<float4_t*>(xch + e0 + ((mh * 2 + rh) * NB + nb) * 4) =
-                        float4_t{vals[mh][rh][nb][0], vals[mh][rh][nb][1], vals[mh][rh][nb][2], vals[mh][rh][nb][3]};
-            }
-            __syncthreads();
-            if (ks == 0 && (a & 1) == 0) {
-#pragma unroll
-              for (int mh = 0; mh < 2; ++mh)
-#pragma unroll
-                for (int rh = 0; rh < 2; ++rh)
-#pragma unroll
-                  for (int nb = 0; nb < NB; ++nb) {
-                    const float4_t o = *reinterpret_cast<const float4_t*>(xch + e0 + ((mh * 2 + rh) * NB + nb) * 4);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) vals[mh][rh][nb][i] += o[i];
-                  }
-            }
-            __syncthreads();  // the next slice may overwrite; after the last turn the buffer becomes a tile again
-          }
-          const int rb = c_grp * kGemmRB + rbi;
-          if (ks == 0 && (a & 1) == 0 && rb < nrb) {
-#pragma unroll
-            for (int mh = 0; mh < 2; ++mh)
-#pragma unroll
-              for (int rh = 0; rh < 2; ++rh)
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                  for (int i = 0; i < 4; ++i) {
-                    float sum = vals[mh][rh][nb][i];
-                    if (round_f16) sum = (float)(_Float16)sum;
-                    // lane (g, a even): batch row 16*nb + 4*g + i, matrix row 16*mh + 8*rh + a/2
-                    const int bb = 16 * nb + 4 * g + i;
-                    if (bb < batch) out_s[(size_t)bb * m + rb * 32 + 16 * mh + 8 * rh + (a >> 1)] = sum;
-                  }
-          }
-          c_t = 0;
-          c_grp += gstep;
-        }
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// 4-bit batched decompress + GEMM on a row-split lane map: no product is computed twice
-// ---------------------------------------------------------------------------
-// In gemm_kernel the two lanes that share a matrix row hold different column halves of it, which
-// costs every product twice (and 64 accumulator registers for 32 batch rows, hence 8 waves).
-// Here the two lanes of a pair load the SAME 64 bytes - the four reference lanes of one row of a
-// 2x2 tile block, i.e. all 16 columns of that row in each of the four tiles - and split the
-// STATES: a 32-bit chunk holds four states, the even lane decodes states 0 and 2 (rows r), the
-// odd lane states 1 and 3 (rows r + 8).  A byte permutation with a per-lane selector puts the
-// lane's two states of a chunk into one register, so the decode costs what it costs in
-// gemm_kernel (32 lookups per lane and wave-load).  The 16 lanes of a DPP row now hold the same
-// 8 columns of 16 different rows: a v_mfma_f32_16x16x32_f16 B operand whose every output is
-// wanted.  Per wave-load and 16 batch rows: 8 products instead of 16, 8 accumulator registers
-// instead of 32, so 32 batch rows run on the 16-wave workgroup (4 waves per SIMD).
-// Lane (g, a): tile block g of the wave-load, row r = a / 2 (+ 8 for odd a) of either tile row
-// half; registers D[cp][t]: reference lane 4 r + cp (columns 2 cp, 2 cp + 1 of an 8-column
-// group), tile t = 2 kh + mh.  The successor chunk of cp = 3 sits two lanes on (row r + 1, the
-// ring of 32 reference lanes closing inside the 16-lane row).
-// The two lanes of a pair read the same bytes and the four 16-byte loads of a lane walk the same
-// cache lines, so the loads are plain (cached) ones: with the non-temporal hint of the other
-// kernels every load instruction fetched its lines from L2 again (43 us instead of 29 us at batch
-// 8).  HBM traffic is unchanged.
-// One activation tile (16 NB batch rows x 1024 columns) in LDS, single-buffered: the next tile
-// waits in registers while the current one is used, two barriers per stage.
-constexpr int kGemm4Waves = 16, kGemm4KS = 4;
-constexpr size_t kGemm4TileBytes = 32 * 1024;
-constexpr size_t kGemm4Lds = kLut128Bytes + kGemm4TileBytes;
-
-template <int NB>
-__global__ __launch_bounds__(kThreads, 1) void gemm4_kernel(
-    float* __restrict__ dst, const uint8_t* __restrict__ packed, const uint16_t* __restrict__ x,
-    const uint32_t* __restrict__ tlut, int m, int k, int batch, int round_f16, int wl_per, int upw_q,
-    int upw_r) {
-  constexpr int K = 4, DEPTH = 2, KS = kGemm4KS;
-  constexpr int ROWB = KS * 256;  // bytes per tile row
-  constexpr int CPR = ROWB / 16;  // 16-byte chunks per tile row
-  constexpr uint32_t TILE = 16 * NB * ROWB;
-  constexpr bool DB = 2 * TILE <= kGemm4TileBytes;  // room for two tiles: one barrier per stage instead of two
-  static_assert(TILE <= kGemm4TileBytes, "tile does not fit");
-  static_assert(16 * NB * CPR == NB * kThreads, "NB chunks per thread and tile");
-  extern __shared__ __align__(16) uint8_t smem[];
-  uint32_t* lut = reinterpret_cast<uint32_t*>(smem);
-  uint8_t* tile = smem + kLut128Bytes;  // [1 or 2][16*NB rows][ROWB bytes]
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rbi = wave & (kGemmRB - 1), ks = wave >> 2;
-  const int a = lane & 15, g = lane >> 4;
-  const uint32_t slot4 = lds_address(lut) + ((uint32_t)(lane & 31) << 2);
-  const int nkb = k >> 5;
-  const int nwl = (nkb + 3) >> 2;
-  const int nrb = m >> 5;
-  const int ngroups = (nrb + kGemmRB - 1) / kGemmRB;
-  const uint32_t rb_bytes = (uint32_t)nkb * 128 * K;
-  constexpr uint32_t WL_BYTES = 512 * K;
-  const uint32_t loff = (uint32_t)g * (128 * K) + (uint32_t)(a >> 1) * (16 * K);  // the row's four reference lanes
-  const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(packed), 0, (int)((size_t)nrb * rb_bytes), 0x00020000);
-  // states 0 | 2 of a chunk for even lanes (the chunk as it is), 1 | 3 for odd lanes (chunk bytes
-  // 2 1 | chunk byte 0, successor byte 3)
-  const uint32_t sel = (a & 1) ? 0x06050403u : 0x07060504u;
-
-  const int s = blockIdx.x;
-  const int g0 = blockIdx.y, gstep = gridDim.y;
-  const int wl0 = s * wl_per;  // wl_per is a multiple of KS
-  const int wl1 = wl0 + wl_per < nwl ? wl0 + wl_per : nwl;
-  const int nst = wl1 > wl0 ? (wl1 - wl0 + KS - 1) / KS : 0;  // stages per unit
-  const int upw = upw_q + (g0 < upw_r ? 1 : 0);
-  const int T = upw * nst;
-  float* out_s = dst + (size_t)s * batch * m;
-
-  struct Raw {
-    uint32_t d[4][4];  // [cp][t]
-  };
-  int l_t = 0, l_q = 0, l_grp = g0;
-  Raw buf[DEPTH];
-  auto issue = [&](int d) {
-    const int rb = l_grp * kGemmRB + rbi;
-    const int wl = wl0 + KS * l_t + ks;
-    const bool valid = l_q < T && rb < nrb && wl < wl1;
-    // padding items, and the lanes past the row's end in a partial last wave-load: a lane offset
-    // that is out of range by itself, zeros without a memory access
-    const uint32_t vo = (valid && 4 * wl + g < nkb) ? loff : 0x7FFFFF00u;
-    const uint32_t so = valid ? (uint32_t)rb * rb_bytes + (uint32_t)wl * WL_BYTES : 0u;
-#pragma unroll
-    for (int cp = 0; cp < 4; ++cp) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs_w, vo + 16 * cp, so, 0);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) buf[d].d[cp][t] = v[t];
-    }
-    ++l_q;
-    if (++l_t == nst) {
-      l_t = 0;
-      l_grp += gstep;
-    }
-  };
-  // table words through the scalar cache first, one stage of the stream before the table is built
-  uint32_t tw[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t* tp = tlut + j * 128 + wave * 8;
-    uint32_t v = tp[0];
-#pragma unroll
-    for (int e = 1; e < 8; ++e) v = ((lane >> 3) == e) ? tp[e] : v;
-    tw[j] = v;
-  }
-  issue(0);
-
-  static_assert(DEPTH % 2 == 0, "stage parity must be static inside the unrolled loop");
-  u32x4 xg[2][NB];  // tiles on their way: [parity of the stage][chunk], requested two stages ahead
-  auto load_tile = [&](int slot, int t) {  // stage t of a unit -> registers
-    const int col0 = 128 * (wl0 + KS * t);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int idx = i * kThreads + tid;
-      const int b = idx / CPR, c = idx % CPR;
-      const int col = col0 + 8 * c;
-      u32x4 v = {0u, 0u, 0u, 0u};
-      if (b < batch && col < k) v = *reinterpret_cast<const u32x4*>(x + (size_t)b * k + col);
-      xg[slot][i] = v;
-    }
-  };
-  // registers -> LDS buffer (the buffer of the stage's parity when there are two), chunk index
-  // xor-ed with the row: conflict-free both ways
-  auto store_tile = [&](int slot) {
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int idx = i * kThreads + tid;
-      const int b = idx / CPR, c = idx % CPR;
-      *reinterpret_cast<u32x4*>(tile + (DB ? slot * TILE : 0u) + b * ROWB + ((c ^ (b & 7)) << 4)) = xg[slot][i];
-    }
-  };
-  load_tile(0, 0);
-  load_tile(1, nst > 1 ? 1 : 0);
-#pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const uint32_t w = tw[it & 3] ^ ((uint32_t)(it >> 2) << 15);
-    const u32x4 v = {w, w, w, w};
-    reinterpret_cast<u32x4*>(lut)[it * kThreads + tid] = v;
-  }
-  store_tile(0);
-  __syncthreads();
-  issue(1);
-
-  float4_t acc[2][NB];  // [mh][batch tile]
-#pragma unroll
-  for (int i = 0; i < 2 * NB; ++i) (&acc[0][0])[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-  uint32_t arow[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) arow[nb] = (uint32_t)(16 * nb + a) * ROWB;
-  const uint32_t a7 = (uint32_t)(a & 7);
-  const uint32_t tile_addr = lds_address(tile);
-  typedef __attribute__((address_space(3))) const u32x4 lds_u32x4_t;
-
-  int c_t = 0, c_grp = g0;
-  for (int q = 0; q < T; q += DEPTH) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      const bool live = q + d < T;  // uniform over the workgroup
-      if (live) {
-        const int rb = c_grp * kGemmRB + rbi;
-        const int wl = wl0 + KS * c_t + ks;
-        if (rb < nrb && wl < wl1) {
-          const Raw& R = buf[d];
-          const uint32_t tb = tile_addr + (DB ? (uint32_t)((q + d) & 1) * TILE : 0u);
-          uint32_t W[4][4][2];  // [cp][t][jh]
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            // successor of reference lane 4 r + 3: reference lane 4 (r + 1), two lanes on in the row
-            const uint32_t nx = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)R.d[0][t], 0x12E /* row_ror:14 */,
-                                                                      0xF, 0xF, false);
-#pragma unroll
-            for (int cp = 0; cp < 4; ++cp) {
-              const uint32_t c = R.d[cp][t];
-              const uint32_t cn = cp < 3 ? R.d[cp + 1][t] : nx;
-              const uint32_t P = perm(c, cn, sel);  // high half: state 0 or 1, low half: state 2 or 3
-              const uint32_t hq = pk_hash(P) & 0xFFC0FFC0u;
-              W[cp][t][0] = lds_word_abs(lut128_addr_hi(hq, slot4));
-              W[cp][t][1] = lds_word_abs(lut128_addr_lo(hq, slot4));
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-            for (int jh = 0; jh < 2; ++jh) {
-              u32x4 xa[NB];
-              const uint32_t c = (uint32_t)(16 * ks + 4 * g + 2 * kh + jh) ^ a7;
-#pragma unroll
-              for (int nb = 0; nb < NB; ++nb)
-                xa[nb] = *(lds_u32x4_t*)(uintptr_t)(tb + arow[nb] + (c << 4));
-#pragma unroll
-              for (int mh = 0; mh < 2; ++mh) {
-                const int t = 2 * kh + mh;
-                const u32x4 wv = {W[0][t][jh], W[1][t][jh], W[2][t][jh], W[3][t][jh]};
-                const half8_t bop = __builtin_bit_cast(half8_t, wv);
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                  acc[mh][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xa[nb]), bop,
-                                                                       acc[mh][nb], 0, 0, 0);
-              }
-            }
-        }
-      }
-      issue(d);
-      if (live) {
-        if constexpr (DB) {
-          // the next tile (in registers since the previous stage) into the other buffer, the one
-          // after it on its way (slot = parity of that stage = parity of this one)
-          store_tile((q + d + 1) & 1);
-          int t2 = c_t + 2;
-          if (t2 >= nst) t2 -= nst;
-          if (t2 >= nst) t2 -= nst;  // nst == 1
-          load_tile((q + d) & 1, t2);
-        }
-        __syncthreads();  // every wave has read this stage's tile (and, with two buffers, written the next)
-        const int rb = c_grp * kGemmRB + rbi;
-        if (++c_t == nst) {
-          // ---- end of a unit: the k slices of a row block meet in the tile buffer (free between the
-          // two barriers of a stage): slices 1 .. KS-1 hand their sums over in turn, the wave of
-          // slice 0 adds them in that order, rounds and stores
-          float* xch = reinterpret_cast<float*>(tile + (DB ? (uint32_t)((q + d) & 1) * TILE : 0u)) + rbi * (64 * 8 * NB);
-          float4_t vals[2][NB];
-#pragma unroll
-          for (int mh = 0; mh < 2; ++mh)
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-              vals[mh][nb] = acc[mh][nb];
-              acc[mh][nb] = float4_t{0.f, 0.f, 0.f, 0.f};
-            }
-          for (int turn = 1; turn < KS; ++turn) {
-            if (ks == turn) {
-#pragma unroll
-              for (int mh = 0; mh < 2; ++mh)
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                  *reinterpret_cast<float4_t*>(xch + ((mh * NB + nb) * 64 + lane) * 4) = vals[mh][nb];
-            }
-            __syncthreads();
-            if (ks == 0) {
-#pragma unroll
-              for (int mh = 0; mh < 2; ++mh)
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) {
-                  const float4_t o = *reinterpret_cast<const float4_t*>(xch + ((mh * NB + nb) * 64 + lane) * 4);
-                  vals[mh][nb] += o;
-                }
-            }
-            __syncthreads();
-          }
-          if (ks == 0 && rb < nrb) {
-#pragma unroll
-            for (int mh = 0; mh < 2; ++mh)
-#pragma unroll
-              for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                  float sum = vals[mh][nb][i];
-                  if (round_f16) sum = (float)(_Float16)sum;
-                  // lane (g, a): batch row 16*nb + 4*g + i, matrix row 16*mh + 8*(a%2) + a/2
-                  const int bb = 16 * nb + 4 * g + i;
-                  if (bb < batch) out_s[(size_t)bb * m + rb * 32 + 16 * mh + 8 * (a & 1) + (a >> 1)] = sum;
-                }
-          }
-          c_t = 0;
-          c_grp += gstep;
-        }
-        if constexpr (!DB) {
-          // one buffer: the next tile (in registers since the previous stage) goes in now, the one
-          // after it on its way (slot = parity of that stage = parity of this one)
-          store_tile((q + d + 1) & 1);
-          int t2 = c_t + 1;
-          if (t2 >= nst) t2 -= nst;
-          load_tile((q + d) & 1, t2);
-          __syncthreads();  // the next tile is complete
-        }
-      }
-    }
-  }
-}
-
-// out[i] = parts[0][i] + ... (+ rounding through fp16) for the split-k GEMM
-__global__ __launch_bounds__(256) void sum_parts_round_kernel(float* __restrict__ out,
-                                                              const float* __restrict__ parts, long n,
-                                                              int S, int round_f16) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  float sum = parts[i];
-  for (int s = 1; s < S; ++s) sum += parts[(size_t)s * n + i];
-  out[i] = round_f16 ? (float)(_Float16)sum : sum;
-}
-
-// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 // Device memory the allocation-free entry point keeps its split-k partial sums in: one copy per
@@ -1373,12 +753,6 @@ hipError_t allow_lds_all() {
   QTIP_ALLOW((matvec_kernel<2, 2, true, 2>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<3, 2, true, 2>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<4, 2, true, 2>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((gemm_kernel<2, 1, 4, 16>), kGemmLds)
-  QTIP_ALLOW((gemm_kernel<2, 2, 4, 8>), kGemmLds)
-  QTIP_ALLOW((gemm_kernel<3, 1, 2, 16>), kGemmLds)
-  QTIP_ALLOW((gemm_kernel<3, 2, 4, 8>), kGemmLds)
-  QTIP_ALLOW((gemm4_kernel<1>), kGemm4Lds)
-  QTIP_ALLOW((gemm4_kernel<2>), kGemm4Lds)
 #undef QTIP_ALLOW
   return hipSuccess;
 }
@@ -1428,6 +802,7 @@ Ready ready(bool launching, hipStream_t st) {
   hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (e == hipSuccess) e = allow_lds_all();
   if (e == hipSuccess) e = qtip_rht_allow_lds();
+  if (e == hipSuccess) e = qtip_gemm_allow_lds();
   float* sp = nullptr;
   if (e == hipSuccess) e = hipGetSymbolAddress(reinterpret_cast<void**>(&sp), HIP_SYMBOL(scratch));
   if (e == hipSuccess && !sp) e = hipErrorInvalidSymbol;
@@ -1448,17 +823,6 @@ int query_cus() {
   if (d.done.load(std::memory_order_acquire)) return d.cus;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
   return cus > 0 ? cus : 256;
-}
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
-int check_common(const void* a, const void* b, const void* c, const void* d, int m, int k,
-                 int bits) {
-  if (!a || !b || !c || !d) return QTIP_E_NULL;
-  if (bits < 2 || bits > 4) return QTIP_E_SHAPE;
-  if (m <= 0 || k <= 0 || (m & 31) || (k & 31)) return QTIP_E_SHAPE;
-  if ((long)m * k * bits / 8 >= (1L << 31)) return QTIP_E_SHAPE;  // 32-bit buffer offsets
-  return QTIP_OK;
 }
 
 // k split S for the shape: a workgroup walks `rounds` units of nwl/S wave-loads, and when the
@@ -1494,6 +858,8 @@ int choose_split(int m, int k, int bits, int cus, bool summed) {
 
 }  // namespace
 
+int qtip_device_cus() { return query_cus(); }
+
 int qtip_device_ready(void* stream, int* cus) {
   const Ready r = ready(stream);
   *cus = r.cus;
@@ -1502,7 +868,7 @@ int qtip_device_ready(void* stream, int* cus) {
 
 extern "C" {
 
-int qtip_abi_version(void) { return 20; }
+int qtip_abi_version(void) { return 21; }
 
 int qtip_init(void) { return ready(false, nullptr).rc; }
 
@@ -1918,96 +1284,6 @@ int qtip_decompress_matvec_noalloc(float* out, const void* packed, const void* x
   if (rc) return rc;
   sum_parts_kernel<<<(m + 255) / 256, 256, 0, st>>>(out, parts, m, S);
   return (int)hipGetLastError();
-}
-
-// k split of the batched GEMM: groups of 4 row blocks are the parallel units, so matrices with
-// few rows are also cut along k (only when the caller provides room for the partial results)
-static int gemm_split(int m, int k, int cus) {
-  const int ngroups = ((m >> 5) + kGemmRB - 1) / kGemmRB;
-  const int nwl = ((k >> 5) + 3) >> 2;
-  int S = 1;
-  while (S < kMaxSplit && ngroups * S * 2 <= cus && nwl / (S * 2) >= 8) S *= 2;
-  return S;
-}
-
-size_t qtip_gemm_workspace_bytes(int m, int k, int bits, int batch) {
-  if (m <= 0 || k <= 0 || (m & 31) || (k & 31) || bits < 2 || bits > 4 || batch < 1) return 0;
-  const int cus = query_cus();
-  if (!cus) return 0;
-  const int S = gemm_split(m, k, cus);
-  return S > 1 ? (size_t)S * (batch < 32 ? batch : 32) * m * sizeof(float) : 0;
-}
-
-int qtip_decompress_gemm(float* out, const void* packed, const void* x_f16, const void* tlut,
-                         int m, int k, int bits, int batch, int round_f16, void* workspace,
-                         size_t workspace_bytes, void* stream) {
-  int rc = check_common(out, packed, x_f16, tlut, m, k, bits);
-  if (rc) return rc;
-  if (batch < 1 || batch > 65535) return QTIP_E_SHAPE;
-  if (!aligned16(packed) || !aligned16(x_f16) || (reinterpret_cast<uintptr_t>(tlut) & 3u) ||
-      (reinterpret_cast<uintptr_t>(out) & 3u))
-    return QTIP_E_ALIGN;
-  const Ready di = ready(stream);
-  if (di.rc) return di.rc;
-  int S = 1;
-  if (workspace) {
-    S = gemm_split(m, k, di.cus);
-    if (S > 1 && workspace_bytes < (size_t)S * (batch < 32 ? batch : 32) * m * sizeof(float))
-      return QTIP_E_WORKSPACE;
-    if (!aligned16(workspace)) return QTIP_E_ALIGN;
-  }
-  const int ngroups = ((m >> 5) + kGemmRB - 1) / kGemmRB;
-  const int nwl = ((k >> 5) + 3) >> 2;
-  hipStream_t st = (hipStream_t)stream;
-  auto* p = (const uint8_t*)packed;
-  auto* t = (const uint32_t*)tlut;
-  // batch handled in passes of at most 32 rows: two 16-row MFMA tiles on the 8-wave workgroup;
-  // up to 16 rows run on the 16-wave workgroup (4 wave-loads per stage)
-  for (int b0 = 0; b0 < batch; b0 += 32) {
-    const int nb = batch - b0 < 32 ? batch - b0 : 32;
-    const bool rowsplit = bits == 4;  // the 4-bit kernel without duplicated products, 16 waves for every batch
-    const int KS = (rowsplit || nb <= 16) ? 4 : 2;
-    int Sp = S;
-    int wl_per = (nwl + Sp - 1) / Sp;
-    wl_per = (wl_per + KS - 1) / KS * KS;  // stages are groups of KS wave-loads
-    Sp = (nwl + wl_per - 1) / wl_per;      // rounding up may have emptied the last ranges
-    const long units = (long)ngroups * Sp;
-    long grid = units < di.cus ? units : di.cus;
-    grid -= grid % Sp;  // a workgroup keeps one k range
-    const int per_range = (int)(grid / Sp);
-    const dim3 g2((unsigned)Sp, (unsigned)per_range);
-    float* o = out + (size_t)b0 * m;
-    float* d = Sp > 1 ? (float*)workspace : o;
-    const int rnd = Sp > 1 ? 0 : round_f16;
-    const uint16_t* xx = (const uint16_t*)x_f16 + (size_t)b0 * k;
-#define QTIP_GEMM(KB, NBT, WV)                                                                          \
-  gemm_kernel<KB, NBT, (KB == 2 ? 4 : (WV == 16 ? 2 : 4)), WV><<<g2, WV * 64, kGemmLds, st>>>( \
-      d, p, xx, t, m, k, nb, rnd, wl_per, ngroups / per_range, ngroups % per_range)
-#define QTIP_GEMM_K(KB)               \
-  if (nb <= 16) QTIP_GEMM(KB, 1, 16); \
-  else QTIP_GEMM(KB, 2, 8);
-    if (rowsplit) {
-      if (nb <= 16)
-        gemm4_kernel<1><<<g2, kThreads, kGemm4Lds, st>>>(d, p, xx, t, m, k, nb, rnd, wl_per, ngroups / per_range,
-                                                         ngroups % per_range);
-      else
-        gemm4_kernel<2><<<g2, kThreads, kGemm4Lds, st>>>(d, p, xx, t, m, k, nb, rnd, wl_per, ngroups / per_range,
-                                                         ngroups % per_range);
-    } else {
-      if (bits == 2) { QTIP_GEMM_K(2) } else { QTIP_GEMM_K(3) }
-    }
-#undef QTIP_GEMM_K
-#undef QTIP_GEMM
-    hipError_t le = hipGetLastError();
-    if (le != hipSuccess) return (int)le;
-    if (Sp > 1) {
-      const long n = (long)nb * m;
-      sum_parts_round_kernel<<<(int)((n + 255) / 256), 256, 0, st>>>(o, (const float*)workspace, n, Sp, round_f16);
-      le = hipGetLastError();
-      if (le != hipSuccess) return (int)le;
-    }
-  }
-  return QTIP_OK;
 }
 
 }  // extern "C"

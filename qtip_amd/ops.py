@@ -243,15 +243,18 @@ def decompress_matvec_group(packed, x, tlut, m, k, bits, nparts=None):
     return parts
 
 
-def decompress_gemm(packed, x, tlut, m, k, bits, round_f16=True):
-    """(batch, m) fp32 = x[batch,k] (fp16) @ decode(packed)[m,k]^T on the matrix cores."""
+def decompress_gemm(packed, x, tlut, m, k, bits, round_f16=True, out_dtype=torch.float32):
+    """(batch, m) = x[batch,k] (fp16) @ decode(packed)[m,k]^T on the matrix cores: fp32, rounded through
+    fp16 on request, or with out_dtype=torch.float16 the rounded values themselves."""
     _check_packed(packed, m, k, bits)
     _check_tlut(tlut, packed.device)
     require_cuda(x, "x", torch.float16)
     if x.dim() != 2 or x.shape[1] != k or x.device != packed.device:
         raise ValueError(f"x must be (batch, {k}) fp16 on {packed.device}")
+    if out_dtype not in _DT or (out_dtype == torch.float16 and not round_f16):
+        raise ValueError("results are fp32, or fp16 when they are rounded")
     batch = x.shape[0]
-    out = torch.empty((batch, m), dtype=torch.float32, device=packed.device)
+    out = torch.empty((batch, m), dtype=out_dtype, device=packed.device)
     if batch == 0:
         return out
     L = lib()
@@ -262,9 +265,13 @@ def decompress_gemm(packed, x, tlut, m, k, bits, round_f16=True):
             wsp, wsb = _ptr(ws), ws.numel()
         else:
             wsp, wsb = ctypes.c_void_p(0), 0
-        check(L.qtip_decompress_gemm(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, batch,
-                                     int(bool(round_f16)), wsp, wsb, stream_ptr(packed.device)),
-              "qtip_decompress_gemm")
+        if out_dtype == torch.float16:
+            check(L.qtip_decompress_gemm_f16(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, batch, wsp, wsb,
+                                             stream_ptr(packed.device)), "qtip_decompress_gemm_f16")
+        else:
+            check(L.qtip_decompress_gemm(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, batch,
+                                         int(bool(round_f16)), wsp, wsb, stream_ptr(packed.device)),
+                  "qtip_decompress_gemm")
     return out
 
 
