@@ -192,6 +192,12 @@ int qtip_decompress_gemm_f16(void* out_f16, const void* packed, const void* x_f1
                              int k, int bits, int batch, void* workspace, size_t workspace_bytes,
                              void* stream);
 
+/* The HYB table (quantlut_sym): tlut is (2^nbits, 2), contiguous; lut holds the value pair of every 16-bit state,
+ * value v of state s at element s * stride_s + v * stride_v.  dtype: of both tables (expand), of lut (fold: nbits is
+ * 9, entries no state selects become 0). */
+int qtip_expand_table(void* lut, const void* tlut, int dtype, int nbits, long stride_s, long stride_v, void* stream);
+int qtip_fold_table(void* tlut_f16, const void* lut, int dtype, long stride_s, long stride_v, void* stream);
+
 /* Randomised Hadamard transform of `rows` vectors of length n = order * p
  * (p a power of two, order 1 or a table order):
  *   out[r][:] = post[:] * scale * (H_order (x) H_p) (pre[:] * in[r][:])

@@ -137,7 +137,14 @@ class bitshift_codebook(nn.Module):
         return quantlut_sym(self.tlut, self.L, self.tlut_bits)
 
     def recons_lut(self):
-        if self.decode_mode not in _COMPUTED:
+        if self.decode_mode in _COMPUTED:
+            return
+        t = self.tlut
+        if (self.decode_mode == 'quantlut_sym' and t.is_cuda and t.dtype in (torch.float16, torch.float32)
+                and t.shape == (1 << self.tlut_bits, 2) and self.tlut_bits < 16 and t.is_contiguous()
+                and not (torch.is_grad_enabled() and t.requires_grad)):
+            self.lut = ops.expand_table(t, self.tlut_bits)
+        else:
             self.lut = self._expand().T.contiguous()
 
     def recons(self, encoded, **kwargs):

@@ -682,6 +682,30 @@ def decode_natural(packed, lut, m, n, td_x, td_y, K, V):
     return out
 
 
+def expand_table(tlut, nbits):
+    """(2, 65536) value pairs of all states from a (2**nbits, 2) fp16 / fp32 table (quantlut_sym, transposed)."""
+    require_cuda(tlut, "tlut", (torch.float16, torch.float32))
+    if not 1 <= nbits <= 15 or tlut.shape != (1 << nbits, 2):
+        raise ValueError(f"table must be (2**nbits, 2) with nbits up to 15 (got {tuple(tlut.shape)})")
+    lut = torch.empty((2, 1 << 16), dtype=tlut.dtype, device=tlut.device)
+    with torch.cuda.device(tlut.device):
+        check(lib().qtip_expand_table(_ptr(lut), _ptr(tlut), _DT[tlut.dtype], nbits, 1, 1 << 16,
+                                      stream_ptr(tlut.device)), "qtip_expand_table")
+    return lut
+
+
+def fold_table(lut):
+    """(512, 2) fp16 table from the (65536, 2) fp16 / fp32 value pairs of all states, in any strides."""
+    require_cuda(lut, "lut", (torch.float16, torch.float32), contiguous=False)
+    if lut.shape != (1 << 16, 2):
+        raise ValueError(f"lut must be (65536, 2) (got {tuple(lut.shape)})")
+    tlut = torch.empty((512, 2), dtype=torch.float16, device=lut.device)
+    with torch.cuda.device(lut.device):
+        check(lib().qtip_fold_table(_ptr(tlut), _ptr(lut), _DT[lut.dtype], lut.stride(0), lut.stride(1),
+                                    stream_ptr(lut.device)), "qtip_fold_table")
+    return tlut
+
+
 def rht_chain(parts, post, scale_out, residual, norm_weight, eps, pre, scale_in):
     """(x_new, xt) for one hidden-size vector per row, one launch:
     x_new = fp16(residual + fp16(post * scale_out * H(sum(parts)))),

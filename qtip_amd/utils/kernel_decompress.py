@@ -35,6 +35,9 @@ def tlut_from_expanded(expanded_lut):
     """Recover the 512 x 2 tunable table from the (65536, 2) expanded one
     (inverse of quantlut_sym, lib/codebook/bitshift.py:72-80).  Indices no
     state hashes to cannot occur in a stream and are left at zero."""
+    if expanded_lut.is_cuda and expanded_lut.dtype in (torch.float16, torch.float32) \
+            and expanded_lut.shape == (1 << 16, 2):
+        return ops.fold_table(expanded_lut)
     rep, neg, seen = _representatives()
     dev = expanded_lut.device
     t = expanded_lut[rep.to(dev)].clone()

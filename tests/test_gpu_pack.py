@@ -132,3 +132,21 @@ def test_forward_without_fused_kernel(mode, V):
     ref = O.hadamard_transform(xt @ W.T) * (SV.cpu().numpy().astype(np.float64) * 32)
     err = np.abs(y - ref)
     assert err.max() <= 1e-2 * np.abs(ref).max() and err.mean() <= 2e-3 * np.abs(ref).mean()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("nbits", [1, 9, 15])
+def test_expanded_table_on_the_device(dtype, nbits):
+    """Bit for bit the host table, and (9 bits) back again from any strides."""
+    from qtip_amd.codebook.bitshift import bitshift_codebook, quantlut_sym
+    from qtip_amd.utils.kernel_decompress import tlut_from_expanded
+    t = torch.randn(1 << nbits, 2, generator=torch.Generator().manual_seed(nbits)).to(dtype)
+    want = quantlut_sym(t, 16, nbits)
+    cb = bitshift_codebook(16, 2, 2, nbits, "quantlut_sym", tlut=t.to(_dev()))
+    assert cb.lut.shape == (2, 65536) and cb.lut.is_contiguous() and cb.lut.dtype == dtype
+    assert torch.equal(cb.lut.cpu(), want.T)
+    if nbits == 9:
+        wide = torch.zeros(65536, 3, dtype=dtype, device=_dev())
+        wide[:, ::2] = cb.lut.T
+        for lut in (cb.lut.T, cb.lut.T.contiguous(), wide[:, ::2]):
+            assert torch.equal(tlut_from_expanded(lut).cpu(), tlut_from_expanded(want))
