@@ -198,6 +198,12 @@ int qtip_decompress_gemm_f16(void* out_f16, const void* packed, const void* x_f1
 int qtip_expand_table(void* lut, const void* tlut, int dtype, int nbits, long stride_s, long stride_v, void* stream);
 int qtip_fold_table(void* tlut_f16, const void* lut, int dtype, long stride_s, long stride_v, void* stream);
 
+/* Backward of y = x * s over the columns of a (rows, n) fp32 matrix, s fp16 or fp32, n a multiple of 4:
+ * gx = g * s, gs[c] = sum over rows of g * x (fp32, summed in a fixed order). */
+size_t qtip_scale_columns_grad_workspace_bytes(int rows, int n);
+int qtip_scale_columns_grad(float* gx, float* gs, const float* g, const float* x, const void* s, int s_dtype, int rows,
+                            int n, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Randomised Hadamard transform of `rows` vectors of length n = order * p
  * (p a power of two, order 1 or a table order):
  *   out[r][:] = post[:] * scale * (H_order (x) H_p) (pre[:] * in[r][:])

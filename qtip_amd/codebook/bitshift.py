@@ -15,7 +15,7 @@ from torch import nn
 
 from .. import ops
 from ..utils.kernel_check import has_kernel as _has_kernel
-from ..utils.matmul_had import had_bits, matmul_hadU_cuda, matmul_hadUt_cuda
+from ..utils.matmul_had import had_bits, hadU_cast, matmul_hadU_cuda, scale_columns
 
 
 def quantlut_sym(tlut, L, nbits):
@@ -347,22 +347,22 @@ class BitshiftLinear(nn.Module):
         vectors SU / SV; the trellis is fixed and the table gets no gradient on the kernel path
         (BitshiftLinearKernelAG returns None for it, :491-505)."""
         n, m = len(SU), len(SV)
-        x = input.reshape(-1, n).to(torch.float32) * SU
+        x = scale_columns(input.reshape(-1, n).to(torch.float32), SU)
         if rcp == 1:
-            x = matmul_hadUt_cuda(x.reshape(-1, n // tp_rank), had_left, K_left).reshape(x.shape) / self.scale
-        else:
-            x = matmul_hadUt_cuda(x, had_left, K_left) / self.scale
+            x = x.reshape(-1, n // tp_rank)
+        # the product takes its input in fp16 and gives fp16: both casts belong to the transforms' launches
+        cast = torch.float16 if self.has_kernel else torch.float32
+        x = hadU_cast(x, had_left, K_left, True, 1 / self.scale, cast).reshape(-1, n)
         if self.has_kernel:
             x = BitshiftLinearKernelAG.apply(x, trellis, m, n, self.cb.L, self.cb.tlut_bits, self.cb.K, self.V,
-                                             self.cb.lut).float()
+                                             self.cb.lut)
         else:
             hatW = self.get_hatW_natural(trellis, m, n) if mode == 'eval' else self.get_hatW(trellis, m, n)
             x = (x.to(hatW.dtype) @ hatW.T).float()
         if rcp == 2:
-            x = matmul_hadU_cuda(x.reshape(-1, m // tp_rank), had_right, K_right).reshape(x.shape)
-        else:
-            x = matmul_hadU_cuda(x, had_right, K_right)
-        x = x.to(SV.device) * (SV * self.scale)
+            x = x.reshape(-1, m // tp_rank)
+        x = hadU_cast(x, had_right, K_right, False, 1.0, torch.float32).reshape(-1, m)
+        x = scale_columns(x.to(SV.device), SV * self.scale)
         return x.view(*input.shape[:-1], m).to(input.dtype)
 
 

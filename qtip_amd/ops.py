@@ -706,6 +706,24 @@ def fold_table(lut):
     return tlut
 
 
+def scale_columns_grad(g, x, s):
+    """(gx, gs) of y = x * s: g * s (rows, n) and the column sums of g * x (n,), fp32; g and x fp32, s fp16 / fp32."""
+    require_cuda(g, "g", torch.float32)
+    require_cuda(x, "x", torch.float32)
+    require_cuda(s, "s", (torch.float16, torch.float32))
+    if g.dim() != 2 or x.shape != g.shape or s.numel() != g.shape[1] or x.device != g.device or s.device != g.device:
+        raise ValueError("g and x must be (rows, n) and s hold n values, on one device")
+    rows, n = g.shape
+    gx = torch.empty_like(g)
+    gs = torch.empty(n, dtype=torch.float32, device=g.device)
+    L = lib()
+    ws = torch.empty(L.qtip_scale_columns_grad_workspace_bytes(rows, n), dtype=torch.uint8, device=g.device)
+    with torch.cuda.device(g.device):
+        check(L.qtip_scale_columns_grad(_ptr(gx), _ptr(gs), _ptr(g), _ptr(x), _ptr(s), _DT[s.dtype], rows, n, _ptr(ws),
+                                        ws.numel(), stream_ptr(g.device)), "qtip_scale_columns_grad")
+    return gx, gs
+
+
 def rht_chain(parts, post, scale_out, residual, norm_weight, eps, pre, scale_in):
     """(x_new, xt) for one hidden-size vector per row, one launch:
     x_new = fp16(residual + fp16(post * scale_out * H(sum(parts)))),

@@ -184,6 +184,68 @@ def _hadU(X, hadK, K, transpose):
     return out.to(X.dtype).reshape(X.shape)
 
 
+class _HadamardCastFn(torch.autograd.Function):
+    """_HadamardFn of a (rows, n) fp16 / fp32 tensor with the scale and the cast that follow it in the same
+    launch: out_dtype(scale * (H_K (x) H_{n/K}) x / sqrt(n)); the gradient takes the way back with its cast."""
+
+    @staticmethod
+    def forward(ctx, X, hadK, K, transpose, scale, out_dtype):
+        ctx.args = (hadK, K, transpose, scale, X.dtype)
+        return _hadU_cast(X, hadK, K, transpose, scale, out_dtype)
+
+    @staticmethod
+    def backward(ctx, grad):
+        hadK, K, transpose, scale, in_dtype = ctx.args
+        args = (grad, hadK, K, not transpose, scale, in_dtype)
+        # (with create_graph the way back is itself recorded)
+        gx = _HadamardCastFn.apply(*args) if torch.is_grad_enabled() else _hadU_cast(*args)
+        return gx, None, None, None, None, None
+
+
+def _hadU_cast(X, hadK, K, transpose, scale, out_dtype):
+    n = X.shape[-1]
+    bits = had_bits(hadK, K, transpose, X.device) if K > 1 else None
+    return ops.rht(X.contiguous(), order=K, had_bits=bits, scale=n**-0.5 * scale, out_dtype=out_dtype)
+
+
+def hadU_cast(X, hadK, K, transpose, scale, out_dtype):
+    """out_dtype(scale * matmul_hadU_cuda(X)), one launch; differentiable with respect to X."""
+    if X.dtype not in (torch.float16, torch.float32):
+        return (matmul_hadU_cuda(X, hadK, K, transpose) * scale).to(out_dtype)
+    return _HadamardCastFn.apply(X, hadK, K, transpose, scale, out_dtype)
+
+
+class _ScaleColumnsFn(torch.autograd.Function):
+    """x * s over the columns of a (rows, n) fp32 tensor; both gradients in one pass over grad and x."""
+
+    @staticmethod
+    def forward(ctx, x, s):
+        ctx.save_for_backward(x, s)
+        return x * s
+
+    @staticmethod
+    def backward(ctx, grad):
+        x, s = ctx.saved_tensors
+        if torch.is_grad_enabled() or grad.numel() == 0:
+            return grad * s, (grad * x).sum(0).to(s.dtype)
+        gx, gs = ops.scale_columns_grad(*(_aligned(t) for t in (grad, x, s)))
+        return gx, gs.to(s.dtype)
+
+
+def _aligned(t):
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def scale_columns(x, s):
+    """x * s for x (rows, n) and s (n,)."""
+    if (x.requires_grad and s.requires_grad and x.is_cuda and s.device == x.device and x.dim() == 2
+            and x.dtype == torch.float32 and s.dtype in (torch.float16, torch.float32) and s.shape == x.shape[1:]
+            and x.shape[1] % 4 == 0):
+        return _ScaleColumnsFn.apply(x, s)
+    return x * s
+
+
 def matmul_hadU_cuda(X, hadK, K, transpose=False):
     """(H_K (x) H_{n/K}) X / sqrt(n) along the last axis (lib/utils/matmul_had.py:105-115);
     differentiable with respect to X."""

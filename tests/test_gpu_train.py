@@ -87,3 +87,40 @@ def test_train_fixW_mode_matches_eval():
         outs[mode] = lin(x).float()
     err = (outs["eval"] - outs["train-fixW"]).abs().max() / outs["eval"].abs().max()
     assert err < 2e-2
+
+
+@pytest.mark.parametrize("rows,n", [(1, 32), (3, 96), (17, 256), (16, 260), (300, 1248), (2049, 4992)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_scale_columns_gradients(rows, n, dtype):
+    """Both gradients of x * s in one pass.  The column sum of r products errs by r 2^-24 times the sum of
+    their magnitudes at most."""
+    from qtip_amd.utils.matmul_had import scale_columns
+    g = torch.Generator(device="cuda").manual_seed(rows + n)
+    x = torch.randn(rows, n, generator=g, device="cuda").requires_grad_(True)
+    s = torch.randn(n, generator=g, device="cuda").to(dtype).requires_grad_(True)
+    gy = torch.randn(n, rows, generator=g, device="cuda").T  # a strided gradient
+    y = scale_columns(x, s)
+    gx, gs = torch.autograd.grad(y, (x, s), gy)
+    assert torch.equal(y, x * s) and torch.equal(gx, gy * s) and gs.dtype == dtype
+    prod = gy.double() * x.detach().double()
+    tol = prod.abs().sum(0) * rows * 2.0**-24 + prod.sum(0).abs() * (2.0**-11 if dtype == torch.float16 else 0)
+    assert bool(((gs.double() - prod.sum(0)).abs() <= tol).all())
+
+
+def test_second_derivatives_pass_through_the_fused_steps():
+    from qtip_amd.utils import matmul_had as mh
+    n = 96
+    had, K = mh.get_hadK(n)
+    x = torch.randn(6, n, device="cuda", requires_grad=True)
+    s = torch.randn(n, device="cuda", requires_grad=True)
+
+    def grads(f):
+        y = f(x, s)
+        gx, gs = torch.autograd.grad((y**2).sum(), (x, s), create_graph=True)
+        return torch.autograd.grad((gx**2).sum() + (gs**2).sum(), (x, s))
+
+    fused = grads(lambda x, s: mh.hadU_cast(mh.scale_columns(x, s), had, K, True, 0.25, torch.float32))
+    M = _matrix(n, True).float().cuda()
+    plain = grads(lambda x, s: (x * s) @ M.T * 0.25)
+    for a, b in zip(fused, plain):
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-4 * float(b.abs().max()))
