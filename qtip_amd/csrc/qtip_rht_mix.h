@@ -404,7 +404,9 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           b[i] = __builtin_bit_cast(uint32_t, v[i][e]);
-          v[i][e] -= __builtin_bit_cast(float, b[i] & 0xFFFF0000u);
+          // (nothing is left of an infinity: the difference would turn it into a NaN)
+          const float rest = v[i][e] - __builtin_bit_cast(float, b[i] & 0xFFFF0000u);
+          v[i][e] = __builtin_isinf(v[i][e]) ? 0.f : rest;
           left |= __builtin_bit_cast(uint32_t, v[i][e]);
         }
         uint2 w;

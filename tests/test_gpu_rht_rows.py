@@ -77,3 +77,23 @@ def test_rows_with_prologue_and_residual(n, sign):
     got = ops.rht(x, residual=res, **kw)
     one = torch.cat([ops.rht(x[i:i + 1], residual=res[i:i + 1], **kw) for i in (0, 17, 28)])
     assert close(got[[0, 17, 28]], one)
+
+
+@pytest.mark.parametrize("n", [11008, 832, 14336])
+def test_infinities_and_nan_stay_what_they_are(n):
+    """One infinity in a row of fp32 values makes every element of its transform infinite (a sum of it and finite
+    values), with the signs the single-row form gives; a NaN fills its own row only."""
+    from qtip_amd import ops
+    from qtip_amd.utils import matmul_had as mh
+    had, order = mh.get_hadK(n)
+    bits = mh.had_bits(had, order, False, "cuda")
+    x = torch.randn(48, n, generator=torch.Generator().manual_seed(n)).cuda()
+    x[3, 7] = float("inf")
+    x[20, n - 1] = -float("inf")
+    x[41, 100] = float("nan")
+    y = ops.rht(x, order=order, had_bits=bits)
+    for r in (3, 20):
+        assert torch.equal(y[r:r + 1], ops.rht(x[r:r + 1].clone(), order=order, had_bits=bits))
+        assert bool(torch.isinf(y[r]).all())
+    bad = ~torch.isfinite(y).all(1)
+    assert torch.isnan(y[41]).all() and bad.nonzero().flatten().tolist() == [3, 20, 41]
