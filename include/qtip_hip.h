@@ -204,6 +204,15 @@ size_t qtip_scale_columns_grad_workspace_bytes(int rows, int n);
 int qtip_scale_columns_grad(float* gx, float* gs, const float* g, const float* x, const void* s, int s_dtype, int rows,
                             int n, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Attention of n new tokens (a prompt, or a piece of one): rotary embedding of q and k (fp16 arithmetic; cos and sin
+ * (n, head_dim) fp16), k and v into slots pos[0..n) of the caches (kv_heads, slots, head_dim), then every query i
+ * against the cache slots up to pos[i].  q, k, v: fp16 rows, strides in elements (multiples of 8); out (n, heads *
+ * head_dim).  head_dim 64 or 128.  Positions outside the cache are not written. */
+int qtip_prefill_attention(void* out_f16, const void* q_f16, const void* k_f16, const void* v_f16, int q_stride,
+                           int k_stride, int v_stride, const void* cos_f16, const void* sin_f16, void* k_cache_f16,
+                           void* v_cache_f16, const int64_t* pos, int n, int heads, int kv_heads, int head_dim,
+                           int slots, void* stream);
+
 /* Randomised Hadamard transform of `rows` vectors of length n = order * p
  * (p a power of two, order 1 or a table order):
  *   out[r][:] = post[:] * scale * (H_order (x) H_p) (pre[:] * in[r][:])

@@ -13,7 +13,7 @@ LIB_PATH = os.environ.get("QTIP_HIP_LIBRARY") or os.path.join(_HERE, "libqtip_hi
 
 QTIP_F16 = 0
 QTIP_F32 = 1
-ABI_VERSION = 23
+ABI_VERSION = 24
 
 _lib = None
 
@@ -56,6 +56,8 @@ _SIGNATURES = {
     "qtip_scale_columns_grad_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 2),
     "qtip_scale_columns_grad": (ctypes.c_int, [ctypes.c_void_p] * 5 + [ctypes.c_int] * 3 +
                                 [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "qtip_prefill_attention": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_int] * 3 + [ctypes.c_void_p] * 5 +
+                               [ctypes.c_int] * 5 + [ctypes.c_void_p]),
     "qtip_rht": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                                 ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
                                 ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p]),

@@ -306,14 +306,8 @@ class BitshiftLinear(nn.Module):
                 # partial sums (if any) are added by the output transform on load
                 y = ops.decompress_matvec_parts(trellis.reshape(-1), xt.reshape(-1), tl.reshape(-1), m, n, self.cb.K)
                 in_parts = y.shape[0]
-            elif bs < self.dense_rows_min:
-                y = ops.decompress_gemm(trellis.reshape(-1), xt, tl, m, n, self.cb.K, out_dtype=torch.float16)
             else:
-                # many rows: decode once to dense fp16 and let the BLAS library multiply, which is
-                # what the reference does for every batch (bitshift.py:476-489)
-                hatW = ops.decode(trellis.reshape(-1), tl.reshape(-1), m, n, self.cb.K)
-                y = xt @ hatW.T  # fp16, which the output transform takes as it is
-                del hatW
+                y = self.rows_product(xt, trellis, tl, m, n)
         else:
             if mode == 'eval':
                 hatW = self.get_hatW_natural(trellis, m, n)
@@ -340,6 +334,14 @@ class BitshiftLinear(nn.Module):
             out = (yt.to(SV.device) * (SV * self.scale)).to(input.dtype)
         return out.view(*input.shape[:-1], m)
 
+
+    def rows_product(self, xt, trellis, tlut, m, n):
+        """(rows, m) fp16 = xt (rows, n) fp16 @ decode(trellis)^T, for two rows or more."""
+        if xt.shape[0] < self.dense_rows_min:
+            return ops.decompress_gemm(trellis.reshape(-1), xt, tlut, m, n, self.cb.K, out_dtype=torch.float16)
+        # many rows: decode once to dense fp16 and let the BLAS library multiply, which is what the reference does
+        # for every batch (bitshift.py:476-489); fp16, which the output transform takes as it is
+        return xt @ ops.decode(trellis.reshape(-1), tlut.reshape(-1), m, n, self.cb.K).T
 
     def _forward_autograd(self, input, trellis, SU, SV, had_left, had_right, K_left, K_right, rcp, tp_rank, mode):
         """The same forward as a chain of differentiable steps, as the reference runs it when

@@ -868,7 +868,7 @@ int qtip_device_ready(void* stream, int* cus) {
 
 extern "C" {
 
-int qtip_abi_version(void) { return 23; }
+int qtip_abi_version(void) { return 24; }
 
 int qtip_init(void) { return ready(false, nullptr).rc; }
 

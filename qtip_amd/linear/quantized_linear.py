@@ -62,26 +62,30 @@ class QuantizedLinear(nn.Module):
             return torch.utils.checkpoint.checkpoint(self.no_ckpt_forward, input, use_reentrant=True)
         return self.no_ckpt_forward(input)
 
+    def build_codebook_class(self):
+        """Set-up on first use."""
+        self.codebook_class = bitshift.BitshiftLinear(self.td_x, self.td_y, self.L, self.K, self.V, self.tlut_bits,
+                                                      self.decode_mode, dtype=self.dtype, tlut=self.tlut,
+                                                      has_kernel=self.has_kernel)
+        # rcp becomes a python int on first use (one host sync, outside any graph capture)
+        rcp = int(self.rcp.item())
+        del self.rcp
+        self.rcp = rcp
+        tp_rank = int(self.tp_rank.item())
+        del self.tp_rank
+        self.tp_rank = tp_rank
+        if self.mode == 'train-fixW':
+            self.codebook_class.cache_hatW(self.trellis, self.had_left, self.had_right, self.K_left, self.K_right,
+                                           len(self.SV), len(self.SU), self.rcp, self.tp_rank)
+        elif self.mode == 'train-recons' and not self.has_kernel:
+            self.trellis = self.codebook_class.cb.unpack_trellis(self.trellis, self.td_x * self.td_y)
+        elif self.mode not in ('eval', 'train-recons'):
+            raise Exception(f"unknown mode {self.mode}")
+        self.built_codebook_class = True
+
     def no_ckpt_forward(self, input):
         if not self.built_codebook_class:
-            self.codebook_class = bitshift.BitshiftLinear(self.td_x, self.td_y, self.L, self.K, self.V, self.tlut_bits,
-                                                          self.decode_mode, dtype=self.dtype, tlut=self.tlut,
-                                                          has_kernel=self.has_kernel)
-            # rcp becomes a python int on first use (one host sync, outside any graph capture)
-            rcp = int(self.rcp.item())
-            del self.rcp
-            self.rcp = rcp
-            tp_rank = int(self.tp_rank.item())
-            del self.tp_rank
-            self.tp_rank = tp_rank
-            if self.mode == 'train-fixW':
-                self.codebook_class.cache_hatW(self.trellis, self.had_left, self.had_right, self.K_left, self.K_right,
-                                               len(self.SV), len(self.SU), self.rcp, self.tp_rank)
-            elif self.mode == 'train-recons' and not self.has_kernel:
-                self.trellis = self.codebook_class.cb.unpack_trellis(self.trellis, self.td_x * self.td_y)
-            elif self.mode not in ('eval', 'train-recons'):
-                raise Exception(f"unknown mode {self.mode}")
-            self.built_codebook_class = True
+            self.build_codebook_class()
         # the reference adds 0 so that a graph's static output is never aliased; the
         # output transform here already writes a fresh tensor
         result = self.codebook_class(input, self.trellis, self.SU, self.SV, self.had_left, self.had_right, self.K_left,

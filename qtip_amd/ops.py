@@ -553,6 +553,34 @@ def decode_attention_rht3(parts, post, scale, had_bits, order, k_cache, v_cache,
     return out
 
 
+def prefill_attention(q, k, v, cos, sin, k_cache, v_cache, pos, heads, kv_heads, head_dim):
+    """Causal attention of n new tokens against the cache, which gets their keys and values first: q (n, heads *
+    head_dim), k / v (n, kv_heads * head_dim) fp16 with contiguous rows, cos / sin (n, head_dim) fp16, pos (n,) int64
+    cache slots, caches (1, kv_heads, slots, head_dim) fp16.  Returns (n, heads * head_dim)."""
+    n, slots = q.shape[0], k_cache.shape[2]
+    for t, name, width in ((q, "q", heads * head_dim), (k, "k", kv_heads * head_dim), (v, "v", kv_heads * head_dim)):
+        require_cuda(t, name, torch.float16, contiguous=False)
+        if t.shape != (n, width) or t.stride(1) != 1:
+            raise ValueError(f"{name} must be ({n}, {width}) with contiguous rows")
+    for t, name in ((cos, "cos"), (sin, "sin")):
+        require_cuda(t, name, torch.float16)
+        if t.numel() != n * head_dim:
+            raise ValueError(f"{name} must be ({n}, {head_dim})")
+    for t, name in ((k_cache, "k_cache"), (v_cache, "v_cache")):
+        require_cuda(t, name, torch.float16)
+        if t.shape != (1, kv_heads, slots, head_dim):
+            raise ValueError(f"{name} must be (1, {kv_heads}, slots, {head_dim})")
+    require_cuda(pos, "pos", torch.int64)
+    if pos.shape != (n,):
+        raise ValueError(f"pos must hold {n} cache slots")
+    out = torch.empty((n, heads * head_dim), dtype=torch.float16, device=q.device)
+    with torch.cuda.device(q.device):
+        check(lib().qtip_prefill_attention(_ptr(out), _ptr(q), _ptr(k), _ptr(v), q.stride(0), k.stride(0), v.stride(0),
+                                           _ptr(cos), _ptr(sin), _ptr(k_cache), _ptr(v_cache), _ptr(pos), n, heads,
+                                           kv_heads, head_dim, slots, stream_ptr(q.device)), "qtip_prefill_attention")
+    return out
+
+
 def rmsnorm(x, weight, eps):
     """weight * fp16(x * rsqrt(mean(x^2) + eps)) for one fp16 vector (model/llama.py:129-135)."""
     require_cuda(x, "x", torch.float16)

@@ -1,0 +1,96 @@
+"""The prompt's attention kernel and the fused launches of a decoder layer over many tokens."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rotate(x, cos, sin):
+    h = x.shape[-1] // 2
+    return x * cos + torch.cat([-x[..., h:], x[..., :h]], -1) * sin
+
+
+@pytest.mark.parametrize("n,past,slots,heads,kv,hd", [
+    (1, 0, 1, 1, 1, 64), (12, 0, 32, 4, 4, 128), (63, 0, 64, 4, 1, 64), (64, 1, 65, 2, 2, 128), (65, 130, 200, 8, 2, 128),
+    (200, 0, 333, 4, 2, 64), (129, 900, 1088, 2, 1, 128), (3, 2000, 4096, 4, 4, 128)])
+def test_prefill_attention(n, past, slots, heads, kv, hd):
+    """Keys bit for bit the fp16 rotary embedding, values copied, output against float64 from the rounded queries
+    and keys: probabilities are rounded to fp16 (2^-11 of each), and so is the result."""
+    from qtip_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(n + past)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").half()
+    wide = rand(n, (heads + 2 * kv) * hd + 8)
+    q, k, v = wide[:, :-8].split([heads * hd, kv * hd, kv * hd], -1)
+    kc, vc = rand(1, kv, slots, hd), rand(1, kv, slots, hd)
+    kc[:, :, past + n:] = float("nan")  # slots behind the last query are not looked at
+    vc[:, :, past + n:] = float("nan")
+    pos = torch.arange(past, past + n, device="cuda")
+    f = pos[:, None].float() * torch.rand(hd // 2, generator=g, device="cuda")
+    emb = torch.cat([f, f], -1)
+    cos, sin = emb.cos().half(), emb.sin().half()
+    kc0, vc0 = kc.clone(), vc.clone()
+    out = ops.prefill_attention(q, k, v, cos, sin, kc, vc, pos, heads, kv, hd)
+    rows = lambda t, h: t.reshape(n, h, hd).transpose(0, 1)
+    kc0[0, :, past:past + n] = _rotate(rows(k, kv), cos, sin)
+    vc0[0, :, past:past + n] = rows(v, kv)
+    same = lambda a, b: torch.equal(a.view(torch.int16), b.view(torch.int16))
+    assert same(kc[:, :, :past + n], kc0[:, :, :past + n]) and same(vc[:, :, :past + n], vc0[:, :, :past + n])
+    qr = _rotate(rows(q, heads), cos, sin).double()
+    kk = kc0[0, :, :past + n].double().repeat_interleave(heads // kv, 0)
+    vv = vc0[0, :, :past + n].double().repeat_interleave(heads // kv, 0)
+    s = qr @ kk.transpose(1, 2) / math.sqrt(hd)
+    s.masked_fill_(torch.arange(past + n, device="cuda")[None, :] > pos[:, None], -math.inf)
+    p = s.softmax(-1)
+    want = (p @ vv).transpose(0, 1).reshape(n, -1)
+    bound = (p @ vv.abs()).transpose(0, 1).reshape(n, -1)
+    # roundings of the probabilities and of the result, and the fp32 scores' error in the exponent
+    assert bool(((out.double() - want).abs() <= 2.0**-10 * bound + 1e-6).all())
+
+
+def test_prefill_attention_skips_positions_outside_the_cache():
+    from qtip_amd import ops
+    kc = torch.ones(1, 1, 4, 64, device="cuda", dtype=torch.float16)
+    vc = kc.clone()
+    x = torch.randn(3, 64, device="cuda").half()
+    one, zero = torch.ones_like(x), torch.zeros_like(x)
+    out = ops.prefill_attention(x, x, x, one, zero, kc, vc, torch.tensor([-1, 4, 2**32 + 1], device="cuda"), 1, 1, 64)
+    assert bool((kc == 1).all()) and bool((vc == 1).all()) and bool((out[1:] == 1).all())
+
+
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("hidden,heads,kv,ffn,n", [(256, 4, 2, 832, 12), (512, 4, 4, 1376, 77), (640, 5, 5, 1728, 40),
+                                                   (256, 2, 1, 832, 300)])
+def test_layer_over_many_tokens(hidden, heads, kv, ffn, n, fused):
+    """The fused launches against the module-by-module layer (which a forward hook makes it take), whole and in two
+    pieces; fp16 rounding points are the same, sums are in another order."""
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder
+    cfg = LlamaConfig(hidden=hidden, heads=heads, kv_heads=kv, layers=2, ffn=ffn, vocab=96)
+    model = LlamaDecoder(cfg, max_cache_len=n + 9, seed=n, fused=fused)
+    ids = torch.randint(0, 96, (1, n), generator=torch.Generator().manual_seed(1)).cuda()
+    at = torch.arange(n, device="cuda")
+
+    def run(cut=None):
+        for c in model.k_cache + model.v_cache:
+            c.zero_()
+        with torch.no_grad():
+            if cut:
+                lg = torch.cat([model(ids[:, :cut], at[:cut]), model(ids[:, cut:], at[cut:])], 1)
+            else:
+                lg = model(ids, at)
+        return [lg] + [c.clone() for c in model.k_cache + model.v_cache]
+
+    with torch.no_grad():
+        assert model.layers[0].rows_ok(model.embed[ids][0], model.k_cache[0], model.v_cache[0], at)
+    got = run()
+    pieces = run(n // 2) if n >= 24 else got
+    seen = []
+    hooks = [l.o.register_forward_hook(lambda *a: seen.append(1)) for l in model.layers]
+    want = run()
+    for h in hooks:
+        h.remove()
+    assert len(seen) == 2
+    for other in (got, pieces):
+        for a, b in zip(other, want):
+            assert float((a.double() - b.double()).norm() / b.double().norm()) <= 5e-3
