@@ -192,6 +192,18 @@ int qtip_decompress_gemm_f16(void* out_f16, const void* packed, const void* x_f1
                              int k, int bits, int batch, void* workspace, size_t workspace_bytes,
                              void* stream);
 
+/* A whole quantized projection (lib/codebook/bitshift.py:415-472 with rcp 0): out[rows][m] in x's dtype =
+ * sv * scale_out * H_out(fp16(scale_in * H_in(su * x)) @ decode(packed)^T), H of order_in x k / order_in and
+ * order_out x m / order_out with sign bits as qtip_rht takes them (NULL for order 1).  The launches are those of
+ * qtip_rht, qtip_decompress_matvec_parts (one row; with the input transform inside where
+ * qtip_decompress_matvec_parts_rht covers it) or qtip_decompress_gemm_f16, qtip_rht, and so are the results.
+ * workspace: qtip_linear_workspace_bytes(...) bytes of scratch, 16-byte aligned, 0 bytes for a refused shape. */
+size_t qtip_linear_workspace_bytes(int m, int k, int bits, int rows, int order_in, int x_dtype);
+int qtip_linear(void* out, const void* x, int x_dtype, const void* packed, const void* tlut, const void* su_f16,
+                const float* sv, const uint32_t* had_in, int order_in, const uint32_t* had_out, int order_out, int m,
+                int k, int bits, int rows, float scale_in, float scale_out, void* workspace, size_t workspace_bytes,
+                void* stream);
+
 /* The HYB table (quantlut_sym): tlut is (2^nbits, 2), contiguous; lut holds the value pair of every 16-bit state,
  * value v of state s at element s * stride_s + v * stride_v.  dtype: of both tables (expand), of lut (fold: nbits is
  * 9, entries no state selects become 0). */

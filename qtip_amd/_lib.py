@@ -50,6 +50,10 @@ _SIGNATURES = {
                              [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "qtip_decompress_gemm_f16": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 +
                                  [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "qtip_linear_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 6),
+    "qtip_linear": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] + [ctypes.c_void_p] * 5 +
+                    [ctypes.c_int, ctypes.c_void_p] + [ctypes.c_int] * 5 + [ctypes.c_float] * 2 +
+                    [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "qtip_expand_table": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2 + [ctypes.c_long] * 2 +
                           [ctypes.c_void_p]),
     "qtip_fold_table": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] + [ctypes.c_long] * 2 + [ctypes.c_void_p]),
@@ -143,8 +147,10 @@ def check(code, what):
 def stream_ptr(device):
     """Current stream of `device` as the launchers take it; also the point where a device the
     library has not met yet gets its one-time set-up (every launch passes through here)."""
-    init_device(device)
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    index = device.index
+    if index not in _INITIALISED:
+        init_device(device)
+    return torch.cuda.current_stream(index).cuda_stream
 
 
 def require_cuda(t, name, dtype=None, contiguous=True):

@@ -7,7 +7,8 @@ from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRCS = [os.path.join(HERE, "csrc", f)
-        for f in ("qtip_hip.hip", "qtip_gemm.hip", "qtip_rht.hip", "qtip_decoder.hip", "qtip_pack.hip", "qtip_prefill.hip", "qtip_train.hip")]
+        for f in ("qtip_hip.hip", "qtip_gemm.hip", "qtip_rht.hip", "qtip_decoder.hip", "qtip_pack.hip", "qtip_prefill.hip", "qtip_train.hip",
+                  "qtip_linear.hip")]
 OUT = os.path.join(HERE, "libqtip_hip.so")
 
 # packed fp32 VALU forms are switched off for every HIP translation unit

@@ -273,6 +273,18 @@ class BitshiftLinear(nn.Module):
                                  rcp, tp_rank, mode=mode, **kwargs) for i in range(0, bs, self.max_rows)]
             return torch.cat(outs, dim=0).view(*input.shape[:-1], m)
 
+        if (self.has_kernel and rcp not in (1, 2) and bs < self.dense_rows_min and SU.dtype == torch.float16
+                and SV.dtype == torch.float32 and SV.device == dev and x.dtype in (torch.float16, torch.float32)):
+            # both transforms and the product by one call of the library: what bounds such a call otherwise is the
+            # host.  (From dense_rows_min rows on the product is the BLAS library's.)  us per call, launch by launch /
+            # here: 4096x4096, 2 bits, one row 40 / 27; 28672x8192, 4 bits, 16 rows 59 / 44; 4096x11008, 3 bits, 45
+            # rows 65 / 35
+            return ops.linear(x.contiguous(), trellis.contiguous(), self._tlut16(dev), SU.contiguous(), SV.contiguous(),
+                              had_bits(had_left, K_left, True, dev) if K_left > 1 else None, K_left,
+                              had_bits(had_right, K_right, False, dev) if K_right > 1 else None, K_right,
+                              m, n, self.cb.K, (n**-0.5) / self.scale, (m**-0.5) * self.scale
+                              ).view(*input.shape[:-1], m)
+
         # ---- input transform: fp16(H_L^T (x * SU) / sqrt(n) / 32)
         fused_in = (rcp != 1 and SU.dtype == torch.float16 and x.dtype in (torch.float16, torch.float32))
         # one token, power-of-two input size: the matvec kernel transforms its input itself

@@ -1,0 +1,71 @@
+// A quantized projection as one library call (qtip_linear): the launches of the transforms and the product, with
+// the scratch between them.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "../../include/qtip_hip.h"
+#include "qtip_setup.h"
+
+namespace {
+
+// Scratch of a call: the transformed input (unless the matvec makes it), the product, the GEMM's partial sums.
+struct LinearPlan {
+  bool in_matvec;
+  int S;
+  size_t y_off, ws_off, ws_bytes, total;
+};
+
+LinearPlan linear_plan(int m, int k, int bits, int rows, int order_in, int x_dtype) {
+  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  LinearPlan p{};
+  p.S = rows == 1 ? qtip_matvec_split(m, k, bits) : 1;
+  p.in_matvec = rows == 1 && order_in == 1 && x_dtype == QTIP_F16 && (k == 2048 || k == 4096 || k == 8192);
+  p.y_off = p.in_matvec ? 0 : up((size_t)rows * k * 2);
+  p.ws_off = p.y_off + up(rows == 1 ? (size_t)p.S * m * sizeof(float) : (size_t)rows * m * 2);
+  p.ws_bytes = rows == 1 ? 0 : qtip_gemm_workspace_bytes(m, k, bits, rows);
+  p.total = p.ws_off + p.ws_bytes;
+  return p;
+}
+
+bool linear_shape_ok(int m, int k, int bits, int rows) {
+  return m > 0 && k > 0 && !((m | k) & 31) && bits >= 2 && bits <= 4 && rows >= 1 && rows <= 65535 &&
+         (long)m * k * bits / 8 < (1L << 31);
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t qtip_linear_workspace_bytes(int m, int k, int bits, int rows, int order_in, int x_dtype) {
+  return linear_shape_ok(m, k, bits, rows) ? linear_plan(m, k, bits, rows, order_in, x_dtype).total : 0;
+}
+
+int qtip_linear(void* out, const void* x, int x_dtype, const void* packed, const void* tlut, const void* su_f16,
+                const float* sv, const uint32_t* had_in, int order_in, const uint32_t* had_out, int order_out, int m,
+                int k, int bits, int rows, float scale_in, float scale_out, void* workspace, size_t workspace_bytes,
+                void* stream) {
+  if (!out || !x || !packed || !tlut || !su_f16 || !sv || !workspace) return QTIP_E_NULL;
+  if (!linear_shape_ok(m, k, bits, rows)) return QTIP_E_SHAPE;
+  if (x_dtype != QTIP_F16 && x_dtype != QTIP_F32) return QTIP_E_DTYPE;
+  if (!aligned16(workspace)) return QTIP_E_ALIGN;
+  const LinearPlan p = linear_plan(m, k, bits, rows, order_in, x_dtype);
+  if (rows == 1 && p.S < 1) return QTIP_E_SHAPE;
+  if (workspace_bytes < p.total) return QTIP_E_WORKSPACE;
+  uint8_t* ws = (uint8_t*)workspace;
+  void* y = ws + p.y_off;
+  int rc;
+  if (p.in_matvec) {
+    rc = qtip_decompress_matvec_parts_rht((float*)y, packed, x, su_f16, scale_in, tlut, m, k, bits, p.S, stream);
+  } else {
+    rc = qtip_rht(ws, QTIP_F16, x, x_dtype, 1, rows, k, order_in, had_in, su_f16, nullptr, scale_in, stream);
+    if (rc) return rc;
+    rc = rows == 1 ? qtip_decompress_matvec_parts((float*)y, packed, ws, tlut, m, k, bits, p.S, stream)
+                   : qtip_decompress_gemm_f16(y, packed, ws, tlut, m, k, bits, rows, p.ws_bytes ? ws + p.ws_off : nullptr,
+                                              p.ws_bytes, stream);
+  }
+  if (rc) return rc;
+  return qtip_rht(out, x_dtype, y, rows == 1 ? QTIP_F32 : QTIP_F16, p.S, rows, m, order_out, had_out, nullptr, sv,
+                  scale_out, stream);
+}
+
+}  // extern "C"

@@ -4,6 +4,7 @@ Every function launches on the current stream of the tensors' device and
 returns without synchronising.  Inputs are checked here (device, dtype,
 contiguity, sizes) so that a bad argument raises instead of reaching a kernel.
 """
+import contextlib
 import ctypes
 import math
 
@@ -21,12 +22,12 @@ _WORKSPACE_BYTES = 8 << 20
 _SPLIT = {}
 
 
-def _workspace(device, need):
-    """Scratch of at least `need` bytes for the current stream.  A request beyond the current
+def _workspace(device, need, stream=None):
+    """Scratch of at least `need` bytes for the current stream (`stream`, if the caller has looked it up).  A request beyond the current
     buffer gets a larger one, and the smaller ones stay alive for the life of the process: a
     HIP graph recorded earlier still holds their addresses."""
     dev = device.index if device.index is not None else torch.cuda.current_device()
-    key = (dev, torch.cuda.current_stream(device).cuda_stream)
+    key = (dev, stream_ptr(device) if stream is None else stream)
     held = _WORKSPACE.setdefault(key, [])
     if not held or held[-1].numel() < need:
         held.append(torch.empty(max(need, _WORKSPACE_BYTES), dtype=torch.uint8, device=device))
@@ -38,7 +39,7 @@ def matvec_split(m, k, bits, device):
     key = (m, k, bits, device.index)
     s = _SPLIT.get(key)
     if s is None:
-        with torch.cuda.device(device):
+        with _on(device):
             s = lib().qtip_matvec_split(m, k, bits)
         if s < 1:
             raise ValueError(f"unsupported matvec shape {m}x{k} at {bits} bits")
@@ -47,7 +48,15 @@ def matvec_split(m, k, bits, device):
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(device):
+    """torch.cuda.device(device), which costs two device switches, only where that is not the current one."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def _check_packed(packed, m, k, bits):
@@ -74,7 +83,7 @@ def decode(packed, tlut, m, k, bits):
     _check_packed(packed, m, k, bits)
     _check_tlut(tlut, packed.device)
     out = torch.empty((m, k), dtype=torch.float16, device=packed.device)
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         check(lib().qtip_decode(_ptr(out), _ptr(packed), _ptr(tlut), m, k, bits, stream_ptr(packed.device)),
               "qtip_decode")
     return out
@@ -94,14 +103,14 @@ def decompress_matvec(packed, x, tlut, m, k, bits, out=None, split_k=True):
         if out.numel() != m:
             raise ValueError(f"out must hold {m} fp32 values")
     L = lib()
+    stream = stream_ptr(packed.device)
+    wsp, wsb = None, 0
     if split_k and matvec_split(m, k, bits, packed.device) > 1:
-        ws = _workspace(packed.device, 16 * m * 4)
+        ws = _workspace(packed.device, 16 * m * 4, stream)
         wsp, wsb = _ptr(ws), ws.numel()
-    else:
-        wsp, wsb = ctypes.c_void_p(0), 0
-    with torch.cuda.device(packed.device):
-        check(L.qtip_decompress_matvec(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, wsp, wsb,
-                                       stream_ptr(packed.device)), "qtip_decompress_matvec")
+    with _on(packed.device):
+        check(L.qtip_decompress_matvec(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, wsp, wsb, stream),
+              "qtip_decompress_matvec")
     return out
 
 
@@ -115,7 +124,7 @@ def decompress_matvec_parts(packed, x, tlut, m, k, bits, nparts=None):
         raise ValueError(f"x must hold {k} fp16 values on {packed.device}")
     S = int(nparts) if nparts is not None else matvec_split(m, k, bits, packed.device)
     parts = torch.empty((S, m), dtype=torch.float32, device=packed.device)
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         check(lib().qtip_decompress_matvec_parts(_ptr(parts), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, S,
                                                  stream_ptr(packed.device)), "qtip_decompress_matvec_parts")
     return parts
@@ -137,7 +146,7 @@ def decompress_matvec_parts_rht(packed, x_raw, su, scale, tlut, m, k, bits, npar
         raise ValueError(f"x and su must be on {packed.device}")
     S = int(nparts) if nparts is not None else matvec_split(m, k, bits, packed.device)
     parts = torch.empty((S, m), dtype=torch.float32, device=packed.device)
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         check(lib().qtip_decompress_matvec_parts_rht(_ptr(parts), _ptr(packed), _ptr(x_raw), _ptr(su),
                                                      ctypes.c_float(scale), _ptr(tlut), m, k, bits, S,
                                                      stream_ptr(packed.device)), "qtip_decompress_matvec_parts_rht")
@@ -167,7 +176,7 @@ def decompress_matvec_parts_chain(packed, tlut, m, k, bits, prev_parts, post, sc
     S = int(nparts) if nparts is not None else matvec_split(m, k, bits, packed.device)
     parts = torch.empty((S, m), dtype=torch.float32, device=packed.device)
     x_new = torch.empty((1, k), dtype=torch.float16, device=packed.device)
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         check(lib().qtip_decompress_matvec_parts_chain(
             _ptr(parts), _ptr(packed), _ptr(tlut), m, k, bits, S, _ptr(pp), pp.shape[0], ctypes.c_size_t(pp.stride(0)),
             _ptr(post), ctypes.c_float(scale_out), _ptr(residual), _ptr(norm_weight), ctypes.c_float(eps), _ptr(su),
@@ -205,7 +214,7 @@ def decompress_matvec_group_chain(packed, tlut, m, k, bits, prev_parts, post, sc
     parts = torch.empty((S, m_total), dtype=torch.float32, device=dev)
     x_new = torch.empty((1, k), dtype=torch.float16, device=dev)
     ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(lib().qtip_decompress_matvec_group_chain(
             _ptr(parts), n, ptrs(packed), ptrs(tlut), ptrs(su), (ctypes.c_int * n)(*[int(v) for v in m]), k, bits, S,
             _ptr(pp), pp.shape[0], ctypes.c_size_t(pp.stride(0)), _ptr(post), ctypes.c_float(scale_out),
@@ -236,7 +245,7 @@ def decompress_matvec_group(packed, x, tlut, m, k, bits, nparts=None):
             S *= 2
     parts = torch.empty((S, m_total), dtype=torch.float32, device=dev)
     ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(lib().qtip_decompress_matvec_group(_ptr(parts), n, ptrs(packed), ptrs(x), ptrs(tlut),
                                                  (ctypes.c_int * n)(*[int(v) for v in m]), k, bits, S,
                                                  stream_ptr(dev)), "qtip_decompress_matvec_group")
@@ -258,20 +267,55 @@ def decompress_gemm(packed, x, tlut, m, k, bits, round_f16=True, out_dtype=torch
     if batch == 0:
         return out
     L = lib()
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         need = L.qtip_gemm_workspace_bytes(m, k, bits, batch)
+        stream = stream_ptr(packed.device)
+        wsp, wsb = None, 0
         if need:
-            ws = _workspace(packed.device, need)
+            ws = _workspace(packed.device, need, stream)
             wsp, wsb = _ptr(ws), ws.numel()
-        else:
-            wsp, wsb = ctypes.c_void_p(0), 0
         if out_dtype == torch.float16:
             check(L.qtip_decompress_gemm_f16(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, batch, wsp, wsb,
-                                             stream_ptr(packed.device)), "qtip_decompress_gemm_f16")
+                                             stream), "qtip_decompress_gemm_f16")
         else:
             check(L.qtip_decompress_gemm(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, batch,
-                                         int(bool(round_f16)), wsp, wsb, stream_ptr(packed.device)),
-                  "qtip_decompress_gemm")
+                                         int(bool(round_f16)), wsp, wsb, stream), "qtip_decompress_gemm")
+    return out
+
+
+def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out):
+    """A whole quantized projection in one call of the library: out (rows, m) in x's dtype = sv * scale_out * H_out(
+    fp16(scale_in * H_in(su * x)) @ decode(packed)^T) for x (rows, k) fp16 / fp32; the launches, and the results bit
+    for bit, of rht, decompress_matvec_parts[_rht] (one row) or decompress_gemm (more), rht.  had_in / had_out: sign
+    bits of the table orders (None for order 1)."""
+    dev, rows = packed.device, x.shape[0]
+    _check_packed(packed, m, k, bits)
+    _check_tlut(tlut, dev)
+    require_cuda(x, "x", (torch.float16, torch.float32))
+    require_cuda(su, "su", torch.float16)
+    require_cuda(sv, "sv", torch.float32)
+    if x.shape != (rows, k) or not 1 <= rows <= 65535 or su.numel() != k or sv.numel() != m:
+        raise ValueError(f"x must be (rows, {k}) with 1 to 65535 rows, su hold {k} and sv {m} values")
+    if x.device != dev or su.device != dev or sv.device != dev:
+        raise ValueError(f"x, su and sv must be on {dev}")
+    for bits_t, order, n in ((had_in, order_in, k), (had_out, order_out, m)):
+        p = n // order
+        if n % order or p & (p - 1):
+            raise ValueError(f"{n} is not {order} times a power of two")
+        if order > 1:
+            require_cuda(bits_t, "sign bits", torch.int32)
+            if bits_t.numel() * 32 < order * order:
+                raise ValueError("sign bits too short")
+    dt = _DT[x.dtype]
+    out = torch.empty((rows, m), dtype=x.dtype, device=dev)
+    L = lib()
+    with _on(dev):
+        stream = stream_ptr(dev)
+        need = L.qtip_linear_workspace_bytes(m, k, bits, rows, order_in, dt)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        check(L.qtip_linear(out.data_ptr(), x.data_ptr(), dt, packed.data_ptr(), tlut.data_ptr(), su.data_ptr(),
+                            sv.data_ptr(), _ptr(had_in), order_in, _ptr(had_out), order_out, m, k, bits, rows, scale_in,
+                            scale_out, ws.data_ptr(), need, stream), "qtip_linear")
     return out
 
 
@@ -332,7 +376,7 @@ def rht(x, order=1, had_bits=None, pre=None, post=None, scale=None, out_dtype=No
     if scale is None:
         scale = n ** -0.5
     L = lib()
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         width = x.shape[-1]
         xf = x.reshape(in_parts, rows, width) if in_parts > 1 else x.reshape(rows, width)
         of = out.reshape(rows, n)
@@ -371,7 +415,7 @@ def rht_fused_pre_rows(x, pre_rows, norm_weight, eps, order=1, had_bits=None, sc
     if order > 1:
         require_cuda(had_bits, "had_bits", torch.int32)
     out = torch.empty_like(pre_rows)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         check(lib().qtip_rht_fused_pre_rows(_ptr(out), _ptr(x), pre_rows.shape[0], n, order, _ptr(had_bits),
                                             _ptr(pre_rows), ctypes.c_float(scale if scale is not None else n ** -0.5),
                                             _ptr(norm_weight), ctypes.c_float(eps), stream_ptr(x.device)),
@@ -393,7 +437,7 @@ def rht_post_rows(parts, post_rows, order=1, had_bits=None, scale=None, out_dtyp
     if order > 1:
         require_cuda(had_bits, "had_bits", torch.int32)
     out = torch.empty((rows, n), dtype=out_dtype, device=parts.device)
-    with torch.cuda.device(parts.device):
+    with _on(parts.device):
         check(lib().qtip_rht_post_rows(_ptr(out), _DT[out_dtype], _ptr(parts), _DT[torch.float32], S, rows, n, order,
                                        _ptr(had_bits), _ptr(post_rows),
                                        ctypes.c_float(scale if scale is not None else n ** -0.5),
@@ -414,7 +458,7 @@ def rht_silu_pair(parts, post, order=1, had_bits=None, scale=None):
     if order > 1:
         require_cuda(had_bits, "had_bits", torch.int32)
     out = torch.empty(n if two else n // 2, dtype=torch.float16, device=parts.device)
-    with torch.cuda.device(parts.device):
+    with _on(parts.device):
         check(lib().qtip_rht_silu_pair(_ptr(out), _ptr(parts), S, int(two), n, order, _ptr(had_bits), _ptr(post),
                                        ctypes.c_float(scale if scale is not None else n ** -0.5),
                                        stream_ptr(parts.device)), "qtip_rht_silu_pair")
@@ -474,7 +518,7 @@ def decode_attention(qkv, k_cache, v_cache, pos, inv_freq, heads, kv_heads, head
         raise ValueError("decode_attention: inconsistent shapes")
     out = torch.empty(heads * head_dim, dtype=torch.float16, device=qkv.device)
     ws = _split_workspace(qkv.device, heads, head_dim, key_splits)
-    with torch.cuda.device(qkv.device):
+    with _on(qkv.device):
         check(lib().qtip_decode_attention(_ptr(out), _ptr(qkv), _ptr(k_cache), _ptr(v_cache), _ptr(pos),
                                           _ptr(inv_freq), heads, kv_heads, head_dim, max_len, key_splits, _ptr(ws),
                                           stream_ptr(qkv.device)), "qtip_decode_attention")
@@ -504,7 +548,7 @@ def decode_attention_rht(parts, post, scale, had_bits, order, k_cache, v_cache, 
         raise ValueError("decode_attention_rht: inconsistent shapes")
     out = torch.empty(heads * head_dim, dtype=torch.float16, device=parts.device)
     ws = _split_workspace(parts.device, heads, head_dim, key_splits)
-    with torch.cuda.device(parts.device):
+    with _on(parts.device):
         check(lib().qtip_decode_attention_rht(_ptr(out), _ptr(parts), parts.shape[0], parts.stride(0),
                                               _ptr(post) if post is not None else None, float(scale),
                                               _ptr(had_bits) if had_bits is not None else None, int(order),
@@ -543,7 +587,7 @@ def decode_attention_rht3(parts, post, scale, had_bits, order, k_cache, v_cache,
     out = torch.empty(heads * head_dim, dtype=torch.float16, device=dev)
     ws = _split_workspace(dev, heads, head_dim, key_splits)
     vp = lambda ts: (ctypes.c_void_p * 3)(*[t.data_ptr() if t is not None else None for t in ts])
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(lib().qtip_decode_attention_rht3(_ptr(out), vp(parts), parts[0].shape[0], parts[0].stride(0), vp(post),
                                                (ctypes.c_float * 3)(*[float(v) for v in scale]), vp(had_bits),
                                                (ctypes.c_int * 3)(*[int(v) for v in order]), _ptr(k_cache),
@@ -574,7 +618,7 @@ def prefill_attention(q, k, v, cos, sin, k_cache, v_cache, pos, heads, kv_heads,
     if pos.shape != (n,):
         raise ValueError(f"pos must hold {n} cache slots")
     out = torch.empty((n, heads * head_dim), dtype=torch.float16, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         check(lib().qtip_prefill_attention(_ptr(out), _ptr(q), _ptr(k), _ptr(v), q.stride(0), k.stride(0), v.stride(0),
                                            _ptr(cos), _ptr(sin), _ptr(k_cache), _ptr(v_cache), _ptr(pos), n, heads,
                                            kv_heads, head_dim, slots, stream_ptr(q.device)), "qtip_prefill_attention")
@@ -588,7 +632,7 @@ def rmsnorm(x, weight, eps):
     if x.numel() != weight.numel():
         raise ValueError("rmsnorm: x and weight differ in length")
     out = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         check(lib().qtip_rmsnorm(_ptr(out), _ptr(x), _ptr(weight), float(eps), x.numel(), stream_ptr(x.device)),
               "qtip_rmsnorm")
     return out
@@ -605,7 +649,7 @@ def greedy_pick(logits, tok, pos, history=None, history_base=0):
         require_cuda(history, "history", torch.int64)
     if tok.numel() != 1 or pos.numel() != 1:
         raise ValueError("greedy_pick: tok and pos hold one element each")
-    with torch.cuda.device(logits.device):
+    with _on(logits.device):
         check(lib().qtip_greedy_pick(_ptr(logits), logits.numel(), _ptr(tok), _ptr(pos),
                                      _ptr(history) if history is not None else None,
                                      history.numel() if history is not None else 0, int(history_base),
@@ -628,7 +672,7 @@ def sample_pick(logits, temperature, top_k, seed, counter, tok, pos, history=Non
     k = 0 if top_k is None else int(top_k)
     if tok.numel() != 1 or pos.numel() != 1 or counter.numel() != 1 or not (0 <= k <= SAMPLE_PICK_MAX_TOP_K):
         raise ValueError("sample_pick: tok, pos and counter hold one element each, top_k at most 64")
-    with torch.cuda.device(logits.device):
+    with _on(logits.device):
         check(lib().qtip_sample_pick(_ptr(logits), logits.numel(), ctypes.c_float(temperature), k,
                                      ctypes.c_uint(int(seed) & 0xffffffff), _ptr(counter), _ptr(tok), _ptr(pos),
                                      _ptr(history) if history is not None else None,
@@ -644,7 +688,7 @@ def repack(packed, m, k, bits, to_kernel=True):
     (lib/utils/kernel_decompress.py:19-24)."""
     _check_packed(packed, m, k, bits)
     out = torch.empty_like(packed)
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         check(lib().qtip_repack(_ptr(out), _ptr(packed), m, k, bits, 1 if to_kernel else 0,
                                 stream_ptr(packed.device)), "qtip_repack")
     return out
@@ -665,7 +709,7 @@ def unpack_trellis(packed, T, K, V):
     (lib/codebook/bitshift.py:329-353)."""
     ntiles = _check_natural(packed, T, K, V)
     states = torch.empty((ntiles, T // V), dtype=torch.int32, device=packed.device)
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         check(lib().qtip_unpack_trellis(_ptr(states), _ptr(packed), ntiles, T, K, V, stream_ptr(packed.device)),
               "qtip_unpack_trellis")
     return states
@@ -684,7 +728,7 @@ def pack_trellis(states, K, V):
         raise ValueError(f"unsupported natural packing T={T} K={K} V={V}")
     packed = torch.empty((ntiles, T * K // 16), dtype=torch.uint16, device=states.device)
     bad = torch.zeros(1, dtype=torch.int32, device=states.device)
-    with torch.cuda.device(states.device):
+    with _on(states.device):
         check(lib().qtip_pack_trellis(_ptr(packed), _ptr(states), ntiles, T, K, V, _ptr(bad),
                                       stream_ptr(states.device)), "qtip_pack_trellis")
     nbad = int(bad.item())
@@ -704,7 +748,7 @@ def decode_natural(packed, lut, m, n, td_x, td_y, K, V):
     if lut.shape != (V, 65536) or lut.device != packed.device:
         raise ValueError(f"lut must be ({V}, 65536) on {packed.device}")
     out = torch.empty((m, n), dtype=lut.dtype, device=packed.device)
-    with torch.cuda.device(packed.device):
+    with _on(packed.device):
         check(lib().qtip_decode_natural(_ptr(out), _ptr(packed), _ptr(lut), _DT[lut.dtype], m, n, td_x, td_y, K, V,
                                         stream_ptr(packed.device)), "qtip_decode_natural")
     return out
@@ -716,7 +760,7 @@ def expand_table(tlut, nbits):
     if not 1 <= nbits <= 15 or tlut.shape != (1 << nbits, 2):
         raise ValueError(f"table must be (2**nbits, 2) with nbits up to 15 (got {tuple(tlut.shape)})")
     lut = torch.empty((2, 1 << 16), dtype=tlut.dtype, device=tlut.device)
-    with torch.cuda.device(tlut.device):
+    with _on(tlut.device):
         check(lib().qtip_expand_table(_ptr(lut), _ptr(tlut), _DT[tlut.dtype], nbits, 1, 1 << 16,
                                       stream_ptr(tlut.device)), "qtip_expand_table")
     return lut
@@ -728,7 +772,7 @@ def fold_table(lut):
     if lut.shape != (1 << 16, 2):
         raise ValueError(f"lut must be (65536, 2) (got {tuple(lut.shape)})")
     tlut = torch.empty((512, 2), dtype=torch.float16, device=lut.device)
-    with torch.cuda.device(lut.device):
+    with _on(lut.device):
         check(lib().qtip_fold_table(_ptr(tlut), _ptr(lut), _DT[lut.dtype], lut.stride(0), lut.stride(1),
                                     stream_ptr(lut.device)), "qtip_fold_table")
     return tlut
@@ -746,7 +790,7 @@ def scale_columns_grad(g, x, s):
     gs = torch.empty(n, dtype=torch.float32, device=g.device)
     L = lib()
     ws = torch.empty(L.qtip_scale_columns_grad_workspace_bytes(rows, n), dtype=torch.uint8, device=g.device)
-    with torch.cuda.device(g.device):
+    with _on(g.device):
         check(L.qtip_scale_columns_grad(_ptr(gx), _ptr(gs), _ptr(g), _ptr(x), _ptr(s), _DT[s.dtype], rows, n, _ptr(ws),
                                         ws.numel(), stream_ptr(g.device)), "qtip_scale_columns_grad")
     return gx, gs
@@ -770,7 +814,7 @@ def rht_chain(parts, post, scale_out, residual, norm_weight, eps, pre, scale_in)
         require_cuda(pre, "pre", torch.float16)
     x_new = torch.empty((rows, n), dtype=torch.float16, device=parts.device)
     xt = torch.empty((rows, n), dtype=torch.float16, device=parts.device)
-    with torch.cuda.device(parts.device):
+    with _on(parts.device):
         check(lib().qtip_rht_chain(_ptr(xt), _ptr(x_new), _ptr(parts), S, rows, n, _ptr(post), ctypes.c_float(scale_out),
                                    _ptr(residual), _ptr(norm_weight), ctypes.c_float(eps), _ptr(pre),
                                    ctypes.c_float(scale_in), stream_ptr(parts.device)), "qtip_rht_chain")

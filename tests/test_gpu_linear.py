@@ -1,0 +1,53 @@
+"""A whole projection by one call of the library against the same launches made one by one (lib/codebook/bitshift.py:
+415-472)."""
+import pytest
+import torch
+
+from qtip_amd import ops
+from qtip_amd.utils.matmul_had import get_hadK, had_bits
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# one row: input transform inside the matvec (4096) and beside it, split and whole k; more: each batch form and the
+# last row count of the fused product; table orders on either side
+@pytest.mark.parametrize("m,k,rows", [(32, 4096, 1), (4096, 4096, 1), (832, 11008, 1), (11008, 928, 1), (4096, 4096, 2),
+                                      (1120, 832, 17), (11008, 4096, 64), (4096, 11008, 129), (64, 2048, 192)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("bits", [2, 3, 4])
+def test_linear_is_its_launches(m, k, rows, dtype, bits):
+    g = torch.Generator(device=DEV).manual_seed(m + k + rows + bits)
+    packed = torch.randint(-32768, 32768, (m * k * bits // 16,), dtype=torch.int16, generator=g, device=DEV)
+    tlut = torch.randn(1024, generator=g, device=DEV).half()
+    su = (torch.randint(0, 2, (k,), generator=g, device=DEV) * 2 - 1).half()
+    sv = torch.randn(m, generator=g, device=DEV)
+    x = torch.randn(rows, k, generator=g, device=DEV).to(dtype)
+    (tin, oin), (tout, oout) = get_hadK(k), get_hadK(m)
+    bin_ = had_bits(None, oin, True, DEV) if oin > 1 else None
+    bout = had_bits(None, oout, False, DEV) if oout > 1 else None
+    s_in, s_out = k**-0.5 / 32, m**-0.5 * 32
+    got = ops.linear(x, packed, tlut, su, sv, bin_, oin, bout, oout, m, k, bits, s_in, s_out)
+    if rows == 1 and oin == 1 and dtype == torch.float16 and k in ops.RHT_IN_MATVEC_SIZES:
+        y = ops.decompress_matvec_parts_rht(packed, x.reshape(-1), su, s_in, tlut, m, k, bits)
+    else:
+        xt = ops.rht(x, order=oin, had_bits=bin_, pre=su, scale=s_in, out_dtype=torch.float16)
+        y = (ops.decompress_matvec_parts(packed, xt.reshape(-1), tlut, m, k, bits) if rows == 1
+             else ops.decompress_gemm(packed, xt, tlut, m, k, bits, out_dtype=torch.float16))
+    parts = y.shape[0] if rows == 1 else 1
+    want = ops.rht(y if parts > 1 else y.reshape(rows, m), order=oout, had_bits=bout, post=sv, scale=s_out,
+                   out_dtype=dtype, in_parts=parts).reshape(rows, m)
+    assert got.dtype == dtype and torch.equal(got, want)
+
+
+def test_linear_refuses_what_does_not_fit():
+    packed = torch.zeros(64 * 64 * 2 // 16, dtype=torch.int16, device=DEV)
+    args = dict(tlut=torch.zeros(1024, dtype=torch.float16, device=DEV), su=torch.ones(64, dtype=torch.float16, device=DEV),
+                sv=torch.ones(64, device=DEV), had_in=None, order_in=1, had_out=None, order_out=1, m=64, k=64, bits=2,
+                scale_in=1.0, scale_out=1.0)
+    x = torch.zeros(3, 64, dtype=torch.float16, device=DEV)
+    assert ops.linear(x, packed, **args).shape == (3, 64)
+    for bad in (dict(x=x[:, :32]), dict(x=x[:0]), dict(x=x.cpu()), dict(su=args["su"][:32]), dict(sv=args["sv"].half()),
+                dict(bits=3), dict(order_in=3), dict(packed=packed[:-1])):
+        with pytest.raises((ValueError, TypeError)):
+            ops.linear(**{**args, "x": x, "packed": packed, **bad})
