@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/qtip_hip.h"
 #include "qtip_wht.h"
 
@@ -329,21 +331,28 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
   const int sub = tid & 7, kq = tid >> 3;
   constexpr int dper = D >> 3;  // dims per lane (multiple of 8: D % 64 == 0)
   float mx = -INFINITY;
-  // four keys per thread group and round, all of their loads issued before the first use
-  constexpr int KU = 4;
-  for (int t0 = k0; t0 < k1; t0 += KU * (kAttnThreads / 8)) {
-    uint4 raw[KU][dper / 8];
+  // KU keys per thread group and round, all of their loads issued before the first use: two, or one where no more than
+  // RK are left.  (Four keys and eight values in flight, and 64-bit addresses for each, did not fit a thread's 128
+  // registers: the spills cost more than the wider rounds gained.  us, spilling / now, 32 heads of 128 on 32 kv heads,
+  // cold caches: 60 keys 5.8 / 4.4, 500 9.3 / 8.8, 1000 19.4 / 13.7; 64 heads on 8, 900 keys 16.5 / 12.2; 32 heads on 8 in 8
+  // ranges, 2000 keys 14.9 / 14.1, 4000 20.0 / 18.8.)
+  constexpr int KU = 2, RK = kAttnThreads / 8;
+  auto cache_row = [&](const _Float16* base, int t, int d) {  // 32-bit offset from a uniform base
+    const int tc = (t < k1 && t != pos) ? t : 0;              // clamped: the new key comes from LDS
+    return reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base) + (uint32_t)(tc * D + d) * 2u);
+  };
+  auto key_round = [&](auto n, int t0) {
+    constexpr int N = decltype(n)::value;
+    uint4 raw[N][dper / 8];
 #pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int t = t0 + kq + u * (kAttnThreads / 8);
-      const int tc = (t < k1 && t != pos) ? t : 0;  // clamped: the new key comes from LDS
-      const uint4* kr = reinterpret_cast<const uint4*>(kc + (size_t)tc * D + sub * dper);
+    for (int u = 0; u < N; ++u) {
+      const uint4* kr = cache_row(kc, t0 + kq + u * RK, sub * dper);
 #pragma unroll
       for (int d8 = 0; d8 < dper / 8; ++d8) raw[u][d8] = kr[d8];
     }
 #pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int t = t0 + kq + u * (kAttnThreads / 8);
+    for (int u = 0; u < N; ++u) {
+      const int t = t0 + kq + u * RK;
       float s = 0.f;
       if (t == pos) {
         for (int d = 0; d < dper; ++d) s += q_s[sub * dper + d] * k_s[sub * dper + d];
@@ -364,20 +373,20 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
         mx = fmaxf(mx, s);
       }
     }
+  };
+  for (int t0 = k0; t0 < k1; t0 += KU * RK) {
+    if (k1 - t0 <= RK) key_round(std::integral_constant<int, 1>{}, t0);
+    else key_round(std::integral_constant<int, KU>{}, t0);
   }
-  // the values of the first round (keys tg, tg + TG, ...: all of them up to 512 keys) are requested
+  // the values of the first round (keys tg, tg + TG, ...: all of them up to 256 keys of 128 values) are requested
   // here, before the softmax reductions: their addresses do not depend on the scores.  (Requesting
   // the first round of keys ahead of the rotary embedding in the same way measured slower.)
   constexpr int DG = D >> 3, TG = kAttnThreads / DG;  // 16 dim groups, 64 key groups for D = 128
-  constexpr int VU = 8;  // values per thread and round, loaded before the first use
+  constexpr int VU = 4;  // values per thread and round, loaded before the first use
   const int dg = tid % DG, tg = tid / DG;
   uint4 vfirst[VU];
 #pragma unroll
-  for (int u = 0; u < VU; ++u) {
-    const int t = k0 + tg + u * TG;
-    const int tc = (t < k1 && t != pos) ? t : 0;
-    vfirst[u] = *reinterpret_cast<const uint4*>(vc + (size_t)tc * D + dg * 8);
-  }
+  for (int u = 0; u < VU; ++u) vfirst[u] = *cache_row(vc, k0 + tg + u * TG, dg * 8);
   mx = wave_reduce_max(mx);
   if (lane == 0) red[wave] = mx;
   __syncthreads();
@@ -408,11 +417,7 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
       for (int u = 0; u < VU; ++u) raw[u] = vfirst[u];
     } else {
 #pragma unroll
-      for (int u = 0; u < VU; ++u) {
-        const int t = t0 + u * TG;
-        const int tc = (t < k1 && t != pos) ? t : 0;
-        raw[u] = *reinterpret_cast<const uint4*>(vc + (size_t)tc * D + dg * 8);
-      }
+      for (int u = 0; u < VU; ++u) raw[u] = *cache_row(vc, t0 + u * TG, dg * 8);
     }
 #pragma unroll
     for (int u = 0; u < VU; ++u) {

@@ -489,9 +489,9 @@ ATTN_SPLIT_FROM = 1024  # context length from which the key-range form is faster
 
 def attention_key_splits(context):
     """Key ranges per head for decode attention over a context of `context` tokens: one workgroup
-    per head below ATTN_SPLIT_FROM keys (the ranges cost a second small launch: 32 heads of 128,
-    127 keys 5.8 vs 11.5 us), 8 ranges from there on (2047 keys 22.8 -> 12.9 us, 4095 keys
-    40 -> 20.6 us, which is the time the 67 MB of keys and values take to arrive)."""
+    per head below ATTN_SPLIT_FROM keys (the ranges cost a second small launch: 32 heads of 128, 250 keys
+    5.5 vs 7.9 us; 64 heads on 8, 1000 keys 12.6 vs 14.6), 8 ranges from there on (32 heads on 8, 2000 keys
+    22 -> 14 us, 4000 keys 40 -> 19 us)."""
     return 1 if context < ATTN_SPLIT_FROM else 8
 
 
