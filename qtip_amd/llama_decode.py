@@ -160,7 +160,8 @@ class DecoderLayer(nn.Module):
         norms = [self.input_norm, self.post_norm]
         if any(type(l) is not QuantizedLinear for l in lins) or any(type(m) is not RMSNorm for m in norms):
             return False
-        if any(m._forward_hooks or m._forward_pre_hooks or 'forward' in m.__dict__ for m in lins + norms):
+        hooks = nn.modules.module
+        if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or any(map(_watched, lins + norms)):
             return False
         if torch.is_grad_enabled() and (x.requires_grad or any(m.weight.requires_grad for m in norms)
                                         or any(l.SU.requires_grad or l.SV.requires_grad for l in lins)):
@@ -170,6 +171,8 @@ class DecoderLayer(nn.Module):
         for l in lins:
             if not l.built_codebook_class:
                 l.build_codebook_class()
+            if _watched(l.codebook_class):
+                return False
             if not (l.has_kernel and l.bias is None and l.mode == 'eval' and not l.grad_ckpt and l.rcp not in (1, 2)
                     and l.in_features // l.K_left >= 8 and l.out_features // l.K_right >= 8
                     and l.SU.dtype == torch.float16 and l.SV.dtype == torch.float32
@@ -426,6 +429,11 @@ class DecoderLayer(nn.Module):
                                                next_layer.input_norm.weight)
             return x, parts
         return f['down'].transform_out(pd, residual=x), None
+
+
+def _watched(module):
+    """Something runs beside, or in place of, the module's own forward."""
+    return bool(module._forward_hooks or module._forward_pre_hooks or 'forward' in module.__dict__)
 
 
 # tokens from which a prompt takes the fused launches: the row count from which the transform kernel takes an

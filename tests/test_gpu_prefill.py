@@ -94,3 +94,21 @@ def test_layer_over_many_tokens(hidden, heads, kv, ffn, n, fused):
     for other in (got, pieces):
         for a, b in zip(other, want):
             assert float((a.double() - b.double()).norm() / b.double().norm()) <= 5e-3
+
+
+def test_hooks_see_the_modules():
+    """A hook on the inner module of a projection, or on all modules, is called for a prompt as for a token."""
+    from torch.nn.modules.module import register_module_forward_hook
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=1, ffn=832, vocab=96), max_cache_len=32)
+    ids, at = torch.zeros(1, 20, dtype=torch.int64, device="cuda"), torch.arange(20, device="cuda")
+    seen = []
+    with torch.no_grad():
+        model(ids, at)
+        inner = model.layers[0].o.codebook_class
+        for hook in (inner.register_forward_hook(lambda *a: seen.append(a[0])),
+                     register_module_forward_hook(lambda *a: seen.append(a[0]))):
+            seen.clear()
+            model(ids, at)
+            hook.remove()
+            assert any(m is inner for m in seen)
