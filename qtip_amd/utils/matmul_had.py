@@ -8,6 +8,7 @@ kernel launch.  The order-K tables are the reference's
 (lib/utils/matmul_had.py:129-95715), kept as packed sign bits in
 hadamard_tables.npz.
 """
+import functools
 import os
 import weakref
 
@@ -22,12 +23,14 @@ _float_tables = {}
 _bit_cache = {}
 
 
+@functools.lru_cache(maxsize=None)  # one per table order; reading the archive takes 0.1 ms
 def _table_signs(order):
     global _npz
     if _npz is None:
         _npz = np.load(os.path.join(os.path.dirname(os.path.abspath(__file__)), "hadamard_tables.npz"),
                        allow_pickle=False)
     bits = np.unpackbits(_npz[f"had{order}"])[:order * order].reshape(order, order)
+    bits.setflags(write=False)
     return bits  # 1 = -1
 
 
@@ -65,7 +68,7 @@ def had_bits(hadK, K, transpose, device):
 
     hadK may be None (the built-in table of order K is used) or the caller's
     K x K tensor (as QuantizedLinear hands in); a caller-supplied tensor is
-    packed once per (storage, transpose) and must be a +-1 matrix.
+    packed once per storage, for both directions, and must be a +-1 matrix.
     """
     dev = torch.device(device)
     if hadK is None or (K in _float_tables and hadK.data_ptr() == _float_tables[K].data_ptr()):
@@ -79,8 +82,7 @@ def had_bits(hadK, K, transpose, device):
     # that storage lives its address cannot belong to another tensor, and when it is freed the entry
     # goes with it (nothing of the caller's is kept alive).  An in-place change bumps `_version`.
     st = hadK.untyped_storage()
-    key = (st.data_ptr(), hadK.storage_offset(), tuple(hadK.shape), tuple(hadK.stride()), hadK.dtype,
-           bool(transpose), dev)
+    key = (st.data_ptr(), hadK.storage_offset(), tuple(hadK.shape), tuple(hadK.stride()), hadK.dtype, dev)
     hit = _bit_cache.get(key)
     if hit is None or hit[0]() is not st or hit[1] != hadK._version:
         h = hadK.detach().to("cpu", torch.float32).numpy()
@@ -88,15 +90,15 @@ def had_bits(hadK, K, transpose, device):
             raise ValueError("hadK must be a K x K matrix of +-1")
         neg = h < 0
         # a K x K table equal to the built-in one shares the built-in entry
-        if K in _ORDERS and np.array_equal(neg, _table_signs(K).astype(bool)):
-            bits = had_bits(None, K, transpose, dev)
+        if K in _ORDERS and np.array_equal(neg, _table_signs(K)):
+            bits = tuple(had_bits(None, K, t, dev) for t in (False, True))
         else:
-            bits = torch.from_numpy(_pack_bits(neg.T if transpose else neg)).to(dev)
+            bits = tuple(torch.from_numpy(_pack_bits(b)).to(dev) for b in (neg, neg.T))
         if hit is None or hit[0]() is not st:
             weakref.finalize(st, _bit_cache.pop, key, None)
         hit = (weakref.ref(st), hadK._version, bits)
         _bit_cache[key] = hit
-    return hit[2]
+    return hit[2][bool(transpose)]
 
 
 _dense_cache = {}

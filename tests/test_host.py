@@ -299,3 +299,17 @@ def test_generate_refuses_requests_beyond_the_cache():
     assert not long.supports_fused_decode()  # generate() then decodes module by module
     with pytest.raises(ValueError, match="fused decode step covers"):
         long.decode_fused(torch.zeros((1, 1), dtype=torch.int64), torch.tensor([0]))
+
+
+def test_had_bits_reads_a_table_once_for_both_directions(monkeypatch):
+    """A training step needs a table and its transpose: the caller's copy is read back and checked once."""
+    from qtip_amd.utils import matmul_had as mh
+    h, K = mh.get_hadK(12 * 64)
+    for own in (h.clone(), h.flip(0).contiguous()):  # equal to the built-in table, and another one
+        mh.had_bits(own, K, False, "cpu")
+        reads = []
+        monkeypatch.setattr(mh.np, "abs", lambda *a: reads.append(1))
+        bt = mh.had_bits(own, K, True, "cpu")
+        monkeypatch.undo()
+        assert not reads and torch.equal(bt, torch.from_numpy(mh._pack_bits((own.numpy() < 0).T)))
+    assert not mh._table_signs(K).flags.writeable
