@@ -180,8 +180,7 @@ class BitshiftLinear(nn.Module):
 
     max_rows = 65535  # rows per launch of the transform / GEMM kernels (grid limit)
     # from this many rows on the dense decode + library GEMM is taken instead of the fused
-    # decompress-GEMM, which runs in passes of 128 rows.  us, dense / fused: 4096x4096 at 2 bits 47 / 50 for
-    # 192 rows, 36 / 64 for 256; 22016x4096 99 / 84 and 103 / 109; 28672x8192 253 / 144 and 265 / 181
+    # decompress-GEMM, for matrices of ordinary size (dense_rows_from)
     dense_rows_min = 193
 
     def __init__(self, td_x, td_y, L, K, V, tlut_bits, decode_mode, dtype=torch.float16, tlut=None,
@@ -273,10 +272,10 @@ class BitshiftLinear(nn.Module):
                                  rcp, tp_rank, mode=mode, **kwargs) for i in range(0, bs, self.max_rows)]
             return torch.cat(outs, dim=0).view(*input.shape[:-1], m)
 
-        if (self.has_kernel and rcp not in (1, 2) and bs < self.dense_rows_min and SU.dtype == torch.float16
+        if (self.has_kernel and rcp not in (1, 2) and bs < self.dense_rows_from(m, n) and SU.dtype == torch.float16
                 and SV.dtype == torch.float32 and SV.device == dev and x.dtype in (torch.float16, torch.float32)):
             # both transforms and the product by one call of the library: what bounds such a call otherwise is the
-            # host.  (From dense_rows_min rows on the product is the BLAS library's.)  us per call, launch by launch /
+            # host.  (From dense_rows_from rows on the product is the BLAS library's.)  us per call, launch by launch /
             # here: 4096x4096, 2 bits, one row 40 / 27; 28672x8192, 4 bits, 16 rows 59 / 44; 4096x11008, 3 bits, 45
             # rows 65 / 35
             return ops.linear(x.contiguous(), trellis.contiguous(), self._tlut16(dev), SU.contiguous(), SV.contiguous(),
@@ -347,9 +346,30 @@ class BitshiftLinear(nn.Module):
         return out.view(*input.shape[:-1], m)
 
 
+    @staticmethod
+    def _dense_rows_from(m, n, rows_min):
+        """The row count from which an (m, n) matrix is decoded to dense fp16 for a library product: rows_min, and
+        4/3, 5/3 or 8/3 of it (257, 321, 514) for larger matrices.  The fused kernel decodes the matrix once per
+        128 rows, the dense route writes and reads 2 m n bytes once, and the library's product takes long where a
+        large n meets few output tiles.  us at 2 / 3 / 4 bits, dense / fused:
+          4096x4096    193 rows 35/56 35/58 34/55                     (192 rows 46/49 47/50 45/48)
+          22016x4096   256 rows 108/107 111/125 109/114               n < 5120: 193
+          8192x8192    256 rows 106/90 110/96 110/91; 257 rows 97/102 99/109 100/103
+          5120x13824   256 rows 154/99 156/112 157/103; 257 rows 106/114 109/130 109/119
+          28672x8192   320 rows 261/228 260/265 271/249; 385 rows 295/291 302/344 304/314
+          8192x28672   320 rows 336/219 335/252 345/245; 512 rows 426/337 429/393 433/387"""
+        if n < 5120 or m * n < 1 << 26:
+            return rows_min
+        if n < 8192 or m * n < 1 << 27:
+            return rows_min * 4 // 3
+        return rows_min * 5 // 3 if n < 2 * m else rows_min * 8 // 3
+
+    def dense_rows_from(self, m, n):
+        return self._dense_rows_from(m, n, self.dense_rows_min)
+
     def rows_product(self, xt, trellis, tlut, m, n):
         """(rows, m) fp16 = xt (rows, n) fp16 @ decode(trellis)^T, for two rows or more."""
-        if xt.shape[0] < self.dense_rows_min:
+        if xt.shape[0] < self.dense_rows_from(m, n):
             return ops.decompress_gemm(trellis.reshape(-1), xt, tlut, m, n, self.cb.K, out_dtype=torch.float16)
         # many rows: decode once to dense fp16 and let the BLAS library multiply, which is what the reference does
         # for every batch (bitshift.py:476-489); fp16, which the output transform takes as it is
@@ -395,7 +415,7 @@ class BitshiftLinearKernelAG(torch.autograd.Function):
         if x.shape[0] == 1:
             y = ops.decompress_matvec(trellis.reshape(-1), x.reshape(-1), tlut.reshape(-1), m, n, K).view(1, m)
             y = y.to(torch.float16)
-        elif x.shape[0] < BitshiftLinear.dense_rows_min:
+        elif x.shape[0] < BitshiftLinear._dense_rows_from(m, n, BitshiftLinear.dense_rows_min):
             y = ops.decompress_gemm(trellis.reshape(-1), x, tlut.reshape(-1), m, n, K, out_dtype=torch.float16)
         else:
             y = x @ ops.decode(trellis.reshape(-1), tlut.reshape(-1), m, n, K).T

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from qtip_amd import ops
+from qtip_amd.linear.quantized_linear import QuantizedLinear
 from qtip_amd.utils.matmul_had import get_hadK, had_bits
 
 pytestmark = pytest.mark.gpu
@@ -51,3 +52,39 @@ def test_linear_refuses_what_does_not_fit():
                 dict(bits=3), dict(order_in=3), dict(packed=packed[:-1])):
         with pytest.raises((ValueError, TypeError)):
             ops.linear(**{**args, "x": x, "packed": packed, **bad})
+
+
+def test_dense_rows_rule():
+    """The row count of the dense route grows with the matrix and follows an instance's own dense_rows_min."""
+    lin = QuantizedLinear(1024, 512, 16, 16, 16, 2, 2, 9, "quantlut_sym", dtype=torch.float16).cuda()
+    with torch.no_grad():
+        lin(torch.zeros(1, 1024, device="cuda", dtype=torch.float16))
+    book = lin.codebook_class
+    assert [book.dense_rows_from(m, n) for m, n in ((4096, 4096), (57344, 4096), (8192, 8192), (8160, 8192), (28672, 8192),
+                                                    (8192, 28672), (16384, 8192))] == [193, 193, 257, 193, 321, 514, 321]
+    book.dense_rows_min = 2
+    assert book.dense_rows_from(4096, 4096) == 2 and book.dense_rows_from(28672, 8192) == 3
+
+
+@pytest.mark.parametrize("m,k,bits", [(13824, 5120, 3), (16384, 8192, 2), (8192, 16384, 4)])
+def test_rows_around_the_dense_route(m, k, bits):
+    """Either side of the row count from which a large matrix is decoded to dense fp16, against float64 from the decoded
+    weights: fp32 sums of k products (error at most k 2^-24 of the sum of magnitudes, far less in fact) and a rounding to fp16."""
+    g = torch.Generator(device="cuda").manual_seed(m)
+    lin = QuantizedLinear(k, m, 16, 16, 16, bits, 2, 9, "quantlut_sym", dtype=torch.float16).cuda()
+    lin.trellis.copy_(torch.randint(-32768, 32768, lin.trellis.shape, dtype=torch.int16, generator=g, device="cuda"))
+    lin.tlut.copy_(torch.randn(512, 2, generator=g, device="cuda"))
+    with torch.no_grad():
+        lin(torch.zeros(1, k, device="cuda", dtype=torch.float16))
+        book = lin.codebook_class
+        edge = book.dense_rows_from(m, k)
+        assert edge > book.dense_rows_min
+        tl = book._tlut16(torch.device("cuda", 0))
+        pick = torch.arange(0, m, 37, device="cuda")
+        w = ops.decode(lin.trellis.reshape(-1), tl.reshape(-1), m, k, bits)[pick].double()
+        for rows in (edge - 1, edge):
+            x = torch.randn(rows, k, generator=g, device="cuda").half()
+            y = book.rows_product(x, lin.trellis, tl, m, k)
+            assert y.shape == (rows, m) and y.dtype == torch.float16
+            want, size = x.double() @ w.T, x.double().abs() @ w.abs().T
+            assert bool(((y[:, pick].double() - want).abs() <= 2.0**-11 * want.abs() + 2.0**-20 * size).all())
