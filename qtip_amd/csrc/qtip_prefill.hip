@@ -62,11 +62,14 @@ __global__ __launch_bounds__(kBlock) void cache_rows_kernel(
 //            key 32 kk + 4 g + j (j < 4) or 32 kk + 16 + 4 g + j - 4, and V^T is laid out in that order
 // V goes to LDS transposed (four keys of one dim in 8 bytes); dim 8 c + e sits in row 16 e + c, which keeps the
 // writes of a phase on distinct banks and makes tile e hold the dims 8 c + e, so a lane ends with eight
-// consecutive dims per register.  Scores, softmax and sums in fp32, probabilities rounded to fp16 for the product.
+// consecutive dims per register.  Scores, softmax and sums in fp32; a probability enters the second product as two fp16
+// numbers, its rounded value and the rest, 22 bits of it or 2^-25 of the largest: rounded to one, outputs
+// were up to 1.013 times as far from float64 as the library's attention (2.38e-4 and 2.35e-4 at 150 tokens of 32
+// heads of 128), with two they are the correctly rounded ones (1.96e-4).
 // Bound by a wave's chain through a tile (products, maximum, exponentials, products): the latest queries
 // run first, and 16-query waves give two workgroups per CU at 1000 tokens of 32 heads.  us, 1000 tokens, 32
-// heads of 128: 42 and 8 for the caches, where the library's attention under a dense mask took 193 beside
-// about 150 of small passes (rotation, cache writes, copies of heads).
+// heads of 128: 46 (42 with one fp16 number per probability) and 8 for the caches, where the library's attention
+// under a dense mask took 193 beside about 150 of small passes (rotation, cache writes, copies of heads).
 constexpr int kQ = 64, kKeys = 64;
 
 template <int HD>
@@ -188,21 +191,28 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
     sum *= fade;
 #pragma unroll
     for (int e = 0; e < NE; ++e) o[e] *= fade;
-    half8v p[2];
+    half8v p[2], rest[2];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float x = __builtin_amdgcn_exp2f(s[t][r] - mx);
         sum += x;
-        p[t >> 1][4 * (t & 1) + r] = (_Float16)x;
+        const _Float16 h = (_Float16)x;
+        p[t >> 1][4 * (t & 1) + r] = h;
+        rest[t >> 1][4 * (t & 1) + r] = (_Float16)(x - (float)h);
       }
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int e = 0; e < NE; ++e) {
-        const half8v a = *reinterpret_cast<const half8v*>(lds_v + (16 * e + ql) * VSTR + 64 * kk + 16 * g);
-        o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, p[kk], o[e], 0, 0, 0);
+      for (int e0 = 0; e0 < NE; e0 += 4) {  // (four accumulators apart, the two products of one do not wait for each other)
+        half8v a[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = *reinterpret_cast<const half8v*>(lds_v + (16 * (e0 + e) + ql) * VSTR + 64 * kk + 16 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e0 + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[e], rest[kk], o[e0 + e], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e0 + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[e], p[kk], o[e0 + e], 0, 0, 0);
       }
   }
   sum += __shfl_xor(sum, 16);

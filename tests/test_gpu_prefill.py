@@ -49,6 +49,29 @@ def test_prefill_attention(n, past, slots, heads, kv, hd):
     assert bool(((out.double() - want).abs() <= 2.0**-10 * bound + 1e-6).all())
 
 
+@pytest.mark.parametrize("n,heads,kv,hd", [(12, 4, 4, 128), (64, 4, 1, 64), (150, 8, 8, 128), (333, 8, 2, 128)])
+def test_prefill_probabilities_are_not_rounded_to_fp16(n, heads, kv, hd):
+    """Output against float64: one rounding to fp16 (2^-11 of the value, 2^-25 below the normal range) beside the
+    error of fp32 scores and sums: a score of up to 8 errs by hd 2^-24 of its terms' magnitudes at most and by a few 2^-22 in
+    fact, and so does the probability relative to itself, 2^-18 of the weighted magnitudes with room to spare.
+    Probabilities of 11 bits err by 2^-12 of them."""
+    from qtip_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(n + hd)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").half()
+    q, k, v = rand(n, heads * hd), rand(n, kv * hd), rand(n, kv * hd)
+    kc, vc = rand(1, kv, n, hd), rand(1, kv, n, hd)
+    pos = torch.arange(n, device="cuda")
+    one = torch.ones(n, hd, device="cuda").half()
+    out = ops.prefill_attention(q, k, v, one, torch.zeros_like(one), kc, vc, pos, heads, kv, hd)
+    rows = lambda t, h: t.double().reshape(n, h, hd).transpose(0, 1)
+    kk, vv = (rows(t, kv).repeat_interleave(heads // kv, 0) for t in (k, v))
+    s = rows(q, heads) @ kk.transpose(1, 2).contiguous() / math.sqrt(hd)
+    p = s.masked_fill_(pos[None, :] > pos[:, None], -math.inf).softmax(-1)
+    back = lambda t: t.transpose(0, 1).reshape(n, -1)
+    want, size = back(p @ vv), back(p @ vv.abs())
+    assert bool(((out.double() - want).abs() <= 2.0**-11 * want.abs() + 2.0**-25 + 2.0**-18 * size).all())
+
+
 def test_prefill_attention_skips_positions_outside_the_cache():
     from qtip_amd import ops
     kc = torch.ones(1, 1, 4, 64, device="cuda", dtype=torch.float16)
