@@ -324,7 +324,10 @@ class BitshiftLinear(nn.Module):
                 hatW = self.get_hatW_natural(trellis, m, n)
             else:  # the owning module already turned the trellis into states
                 hatW = self.get_hatW(trellis, m, n)
+            # fp16 and fp32 products go to the output transform as they are, those of a wider or bf16 table as fp32
             y = xt.to(hatW.dtype) @ hatW.T
+            if y.dtype not in (torch.float16, torch.float32):
+                y = y.float()
 
         # ---- output transform: (H_R y / sqrt(m)) * SV * 32, cast
         fused_out = (rcp != 2 and SV.dtype == torch.float32 and SV.device == dev

@@ -150,3 +150,28 @@ def test_expanded_table_on_the_device(dtype, nbits):
         wide[:, ::2] = cb.lut.T
         for lut in (cb.lut.T, cb.lut.T.contiguous(), wide[:, ::2]):
             assert torch.equal(tlut_from_expanded(lut).cpu(), tlut_from_expanded(want))
+
+
+@pytest.mark.parametrize("mode,dtype", [("train-recons", torch.bfloat16), ("train-recons", torch.float64),
+                                        ("train-recons", torch.float32), ("eval", torch.bfloat16)])
+@pytest.mark.parametrize("sv_dtype", [torch.float32, torch.float16])
+def test_forward_with_a_table_of_another_type(mode, dtype, sv_dtype):
+    """A module converted to another type hands its table's type to the dense product: the output transform takes fp16
+    and fp32, so any other product goes on as fp32, with either form of the output transform."""
+    from qtip_amd.codebook.bitshift import BitshiftLinear
+    m, k, K = 128, 256, 2
+    g = torch.Generator(device=_dev()).manual_seed(3)
+    tr = torch.randint(-32768, 32768, (m // 16 * k // 16, 256 * K // 16), dtype=torch.int16, generator=g, device=_dev())
+    tl = torch.randn(512, 2, generator=g, device=_dev()).bfloat16()  # (values every type holds)
+    SU = torch.ones(k, dtype=torch.float16, device=_dev())
+    SV = torch.full((m,), 2.0**-4, dtype=sv_dtype, device=_dev())
+    x = torch.randn(3, k, generator=g, device=_dev()).half()
+    y = []
+    for dt in (dtype, torch.float16):
+        mod = BitshiftLinear(16, 16, 16, K, 2, 9, "quantlut_sym", tlut=tl.to(dt), has_kernel=False)
+        t = tr if mode == "eval" else mod.cb.unpack_trellis(tr, 256)
+        with torch.no_grad():
+            y.append(mod(x, t, SU, SV, None, None, 1, 1, 0, 8, mode=mode))
+    assert y[0].dtype == torch.float16
+    # against the fp16 table: the activations' and products' rounding to bf16 (2^-9 each) or fp16, one of the result
+    assert float((y[0].float() - y[1].float()).norm() / y[1].float().norm()) <= 2.0**-8
