@@ -97,3 +97,50 @@ def test_infinities_and_nan_stay_what_they_are(n):
         assert bool(torch.isinf(y[r]).all())
     bad = ~torch.isfinite(y).all(1)
     assert torch.isnan(y[41]).all() and bad.nonzero().flatten().tolist() == [3, 20, 41]
+
+
+@pytest.mark.parametrize("n,K", [(688, 172), (624, 156), (344, 172), (108, 108), (1200, 300), (2048, 512)])
+@pytest.mark.parametrize("rows", [96, 300])
+def test_orders_the_matrix_form_does_not_take(n, K, rows, monkeypatch):
+    """Large orders over parts of fewer than 8 points, and orders above 256, run as library products from the rows on
+    from which those are faster; either route against float64: exact products, fp32 sums of n terms."""
+    from qtip_amd.utils import matmul_had as mh
+    g = torch.Generator(device="cuda").manual_seed(n + rows)
+    had = mh.get_hadK(n)[0].cuda() if K < 256 else torch.randint(0, 2, (K, K), generator=g, device="cuda").float() * 2 - 1
+    taken, many = [], mh.rht_many_rows
+    monkeypatch.setattr(mh, "rht_many_rows", lambda *a, **k: taken.append(1) or many(*a, **k))
+    h64 = torch.from_numpy(scipy.linalg.hadamard(n // K).astype(np.float64)).cuda()
+    for dtype, tol in ((torch.float32, 1e-5), (torch.float16, 2.0**-10)):
+        x = torch.randn(n, rows, generator=g, device="cuda").to(dtype).T  # (no contiguous rows)
+        for transpose in (False, True):
+            z = (had.T if transpose else had).double() @ (x.double().reshape(rows, K, n // K) @ h64)
+            ref = z.reshape(rows, n) / n**0.5
+            taken.clear()
+            outs = [mh.matmul_hadU_cuda(x, had, K, transpose), mh.hadU_cast(x, had, K, transpose, 1.0, dtype)]
+            assert len(taken) == (2 if rows * K >= 24000 else 0)
+            for y in outs:
+                assert y.dtype == dtype and float((y.double() - ref).abs().max()) <= tol * float(ref.abs().max())
+
+
+def test_projection_whose_orders_the_matrix_form_does_not_take(monkeypatch):
+    """A dense-route projection with 172 * 4 outputs and 156 * 4 inputs: 300 rows at once against 50 at a time, which
+    take the kernel (fp16 activations and results: another order of sums moves some by a rounding)."""
+    from qtip_amd.codebook import bitshift
+    from qtip_amd.utils.matmul_had import get_hadK
+    m, k, rows = 688, 624, 300
+    g = torch.Generator(device="cuda").manual_seed(1)
+    tr = torch.randint(-32768, 32768, (m // 16 * k // 16, 32), dtype=torch.int16, generator=g, device="cuda")
+    mod = bitshift.BitshiftLinear(16, 16, 16, 2, 2, 9, "quantlut_sym", has_kernel=False,
+                                  tlut=torch.randn(512, 2, generator=g, device="cuda").half())
+    su = torch.randint(0, 2, (k,), generator=g, device="cuda").half() * 2 - 1
+    sv = torch.randn(m, generator=g, device="cuda")
+    x = torch.randn(rows, k, generator=g, device="cuda").half()
+    (hl, kl), (hr, kr) = get_hadK(k), get_hadK(m)
+    taken, many = [], bitshift.rht_many_rows
+    monkeypatch.setattr(bitshift, "rht_many_rows", lambda *a, **kw: taken.append(1) or many(*a, **kw))
+    call = lambda t: mod(t, tr, su, sv, hl, hr, kl, kr, 0, 8)
+    with torch.no_grad():
+        want = torch.cat([call(x[i:i + 50]) for i in range(0, rows, 50)])
+        assert not taken
+        got = call(x)
+    assert len(taken) == 2 and float((got.float() - want.float()).norm() / want.float().norm()) <= 2.0**-10
