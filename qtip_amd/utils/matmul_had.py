@@ -243,13 +243,8 @@ class _ScaleColumnsFn(torch.autograd.Function):
         x, s = ctx.saved_tensors
         if torch.is_grad_enabled() or grad.numel() == 0:
             return grad * s, (grad * x).sum(0).to(s.dtype)
-        gx, gs = ops.scale_columns_grad(*(_aligned(t) for t in (grad, x, s)))
+        gx, gs = ops.scale_columns_grad(*(ops.aligned16(t.contiguous()) for t in (grad, x, s)))
         return gx, gs.to(s.dtype)
-
-
-def _aligned(t):
-    t = t.contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def scale_columns(x, s):

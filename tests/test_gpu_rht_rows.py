@@ -144,3 +144,37 @@ def test_projection_whose_orders_the_matrix_form_does_not_take(monkeypatch):
         assert not taken
         got = call(x)
     assert len(taken) == 2 and float((got.float() - want.float()).norm() / want.float().norm()) <= 2.0**-10
+
+
+@pytest.mark.parametrize("n", [11008, 4096, 12288])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_many_rows_that_start_off_16_bytes(n, dtype):
+    """Rows and vectors at any element offset take the route of aligned ones, to the same bits."""
+    from qtip_amd import ops
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    had, K = get_hadK(n)
+    bits = had_bits(had, K, True, "cuda") if K > 1 else None
+    rows = 96
+    g = torch.Generator(device="cuda").manual_seed(n)
+
+    def both(*shape, dt):
+        off = torch.empty(int(np.prod(shape)) + 1, dtype=dt, device="cuda")[1:].view(*shape)
+        off.copy_(torch.randn(*shape, generator=g, device="cuda"))
+        assert off.data_ptr() % 16 and off.is_contiguous()
+        return off, off.clone()
+
+    x, pre, post = both(rows, n, dt=dtype), both(n, dt=torch.float16), both(n, dt=torch.float32)
+    got, want = (ops.rht(x[i], order=K, had_bits=bits, pre=pre[i], post=post[i]) for i in (0, 1))
+    assert torch.equal(got, want)
+    if dtype == torch.float16:
+        res, w = both(rows, n, dt=torch.float16), both(n, dt=torch.float16)
+        got, want = (ops.rht(x[i], order=K, had_bits=bits, residual=res[i], pre_mode=ops.PRE_RMSNORM, norm_weight=w[i],
+                             eps=1e-5) for i in (0, 1))
+        assert torch.equal(got, want)
+    m = 64
+    packed = torch.randint(-32768, 32768, (m * n * 2 // 16,), dtype=torch.int16, generator=g, device="cuda")
+    tlut = torch.randn(1024, generator=g, device="cuda").half()
+    sv = both(m, dt=torch.float32)
+    got, want = (ops.linear(x[i], packed, tlut, pre[i], sv[i], bits, K, None, 1, m, n, 2, n**-0.5 / 32, m**-0.5 * 32)
+                 for i in (0, 1))
+    assert torch.equal(got, want)
