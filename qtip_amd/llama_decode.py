@@ -150,7 +150,9 @@ class DecoderLayer(nn.Module):
         if not (ROWS_MIN <= n <= 65535 and x.is_cuda and x.dtype == torch.float16 and cfg.head_dim in (64, 128)
                 and cache_position.dtype == torch.int64 and cache_position.shape == (n,)
                 and cache_position.device == x.device and cache_position.is_contiguous()
-                and all(c.is_contiguous() and c.dtype == torch.float16 and c.device == x.device and c.dim() == 4
+                and not (x.is_contiguous() and x.data_ptr() % 16)  # (a copy to contiguous rows is aligned)
+                and all(c.is_contiguous() and c.data_ptr() % 16 == 0 and c.dtype == torch.float16
+                        and c.device == x.device and c.dim() == 4
                         and c.shape[0] == 1 and c.shape[1] == cfg.kv_heads and c.shape[3] == cfg.head_dim
                         and c.shape == k_cache.shape for c in (k_cache, v_cache))):
             return False

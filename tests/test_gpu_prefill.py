@@ -135,3 +135,36 @@ def test_hooks_see_the_modules():
             model(ids, at)
             hook.remove()
             assert any(m is inner for m in seen)
+
+
+@pytest.mark.parametrize("which", ["k_cache", "v_cache", "both"])
+def test_caches_that_start_off_16_bytes(which):
+    """Such a cache goes module by module, as any other the attention kernel does not take."""
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=2, ffn=832, vocab=96), max_cache_len=32)
+    ids, at = torch.arange(20, device="cuda")[None], torch.arange(20, device="cuda")
+
+    def run():
+        with torch.no_grad():
+            return [model(ids, at)] + [c.clone() for c in model.k_cache + model.v_cache]
+
+    want = run()
+    for name in ("k_cache", "v_cache") if which == "both" else (which,):
+        caches = getattr(model, name)
+        caches[1] = torch.zeros(caches[1].numel() + 3, dtype=torch.float16, device="cuda")[3:].view_as(caches[1])
+    assert not model.layers[1].rows_ok(model.embed[ids][0], model.k_cache[1], model.v_cache[1], at)
+    for a, b in zip(run(), want):  # (sums in another order before the fp16 rounding points)
+        assert float((a.double() - b.double()).norm() / b.double().norm()) <= 5e-3
+
+
+def test_layer_input_that_starts_off_16_bytes():
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=1, ffn=832, vocab=96), max_cache_len=32)
+    at = torch.arange(20, device="cuda")
+    cos, sin = model.rope(at)
+    x = torch.empty(20 * 256 + 1, dtype=torch.float16, device="cuda")[1:].view(1, 20, 256)
+    x.copy_(torch.randn(x.shape, generator=torch.Generator().manual_seed(0)))
+    assert not model.layers[0].rows_ok(x[0], model.k_cache[0], model.v_cache[0], at)
+    with torch.no_grad():
+        got, want = (model.layers[0](t, cos, sin, model.k_cache[0], model.v_cache[0], at, None) for t in (x, x.clone()))
+    assert float((got.double() - want.double()).norm() / want.double().norm()) <= 5e-3
