@@ -14,6 +14,7 @@ the reference's README quotes its decode speed on); lm_head and the embedding
 stay dense fp16.  Decode steps are recorded into one HIP graph, as the
 reference does with torch.compile(mode="max-autotune") (eval/interactive_gen.py:147-149).
 """
+import functools
 import math
 import time
 
@@ -162,8 +163,7 @@ class DecoderLayer(nn.Module):
         norms = [self.input_norm, self.post_norm]
         if any(type(l) is not QuantizedLinear for l in lins) or any(type(m) is not RMSNorm for m in norms):
             return False
-        hooks = nn.modules.module
-        if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or any(map(_watched, lins + norms)):
+        if _all_modules_hooked() or any(map(_watched, lins + norms)):
             return False
         if torch.is_grad_enabled() and (x.requires_grad or any(m.weight.requires_grad for m in norms)
                                         or any(l.SU.requires_grad or l.SV.requires_grad for l in lins)):
@@ -203,13 +203,17 @@ class DecoderLayer(nn.Module):
         up = _rows_linear(self.up_proj, x, ops.PRE_RMSNORM, self.post_norm)
         return _rows_linear(self.down, F.silu(gate) * up, residual=x)
 
-    def forward(self, x, cos, sin, k_cache, v_cache, cache_position, attn_mask):
-        """attn_mask None: a query attends to the cache slots up to its position."""
+    def forward(self, x, cos, sin, k_cache, v_cache, cache_position, attn_mask, causal=False):
+        """causal (or attn_mask None): a query attends to the cache slots up to its position, and attn_mask is that
+        mask or a function that makes it, called if the layer goes module by module."""
         cfg = self.cfg
-        if attn_mask is None:
+        if causal or attn_mask is None:
             if x.shape[0] == 1 and self.rows_ok(x[0], k_cache, v_cache, cache_position):
                 return self._forward_rows(x[0], cos[0, 0], sin[0, 0], k_cache, v_cache, cache_position)[None]
-            attn_mask = _causal_mask(k_cache.shape[2], cache_position)
+            if attn_mask is None:
+                attn_mask = _causal_mask(k_cache.shape[2], cache_position)
+            elif callable(attn_mask):
+                attn_mask = attn_mask()
         q_len = x.shape[1]
         h = self.input_norm(x)
         qkv = self._qkv(h)
@@ -438,6 +442,11 @@ def _watched(module):
     return bool(module._forward_hooks or module._forward_pre_hooks or 'forward' in module.__dict__)
 
 
+def _all_modules_hooked():
+    hooks = nn.modules.module
+    return bool(hooks._global_forward_hooks or hooks._global_forward_pre_hooks)
+
+
 # tokens from which a prompt takes the fused launches: the row count from which the transform kernel takes an
 # element-wise prologue at every size.  1000 tokens through four layers of 4096 (32 heads, 2 bits) and the head:
 # 4670 us module by module, 3100 fused
@@ -635,10 +644,16 @@ class LlamaDecoder(nn.Module):
         """ids (1, q_len) int64, cache_position (q_len,) int64 -> logits (1, q_len, vocab) fp32."""
         x = self.embed[ids]
         cos, sin = self.rope(cache_position)
-        # (from ROWS_MIN tokens on a layer takes its own way or makes the mask itself)
-        mask = _causal_mask(self.max_cache_len, cache_position) if ids.shape[-1] < ROWS_MIN or not ids.is_cuda else None
+        # one mask for all layers, made if something asks for it: from ROWS_MIN tokens on a layer may go without; hooks
+        # and anyone's own layers are handed the tensor
+        mask = functools.lru_cache(maxsize=1)(lambda: _causal_mask(self.max_cache_len, cache_position))
+        few, hooked = ids.shape[-1] < ROWS_MIN or not ids.is_cuda, _all_modules_hooked()
         for i, layer in enumerate(self.layers):
-            x = layer(x, cos, sin, self.k_cache[i], self.v_cache[i], cache_position, mask)
+            args = (x, cos, sin, self.k_cache[i], self.v_cache[i], cache_position)
+            if few or type(layer) is not DecoderLayer or 'forward' in layer.__dict__:
+                x = layer(*args, mask())
+            else:
+                x = layer(*args, mask() if hooked or _watched(layer) else mask, causal=True)
         x = self.norm(x)
         return (x @ self.lm_head.T).float()
 

@@ -168,3 +168,46 @@ def test_layer_input_that_starts_off_16_bytes():
     with torch.no_grad():
         got, want = (model.layers[0](t, cos, sin, model.k_cache[0], model.v_cache[0], at, None) for t in (x, x.clone()))
     assert float((got.double() - want.double()).norm() / want.double().norm()) <= 5e-3
+
+
+def test_one_mask_for_all_layers(monkeypatch):
+    """Layers that go module by module share one mask, plain ones need none; a hook on a layer, and a layer of the
+    caller's own, get the tensor."""
+    from qtip_amd import llama_decode
+    model = llama_decode.LlamaDecoder(llama_decode.LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=3, ffn=832, vocab=96),
+                                      max_cache_len=32)
+    ids, at = torch.zeros(1, 20, dtype=torch.int64, device="cuda"), torch.arange(20, device="cuda")
+    made, masks, make = [], [], llama_decode._causal_mask
+    monkeypatch.setattr(llama_decode, "_causal_mask", lambda *a: made.append(1) or make(*a))
+
+    def run():
+        made.clear()
+        with torch.no_grad():
+            return model(ids, at)
+
+    run()
+    assert not made
+    hooks = [l.o.register_forward_hook(lambda *a: None) for l in model.layers]
+    want = run()
+    assert len(made) == 1
+    for h in hooks:
+        h.remove()
+    hook = model.layers[1].register_forward_hook(lambda mod, args, out: masks.append(args[6]))
+    run()
+    hook.remove()
+    assert len(made) == 1
+
+    class Own(torch.nn.Module):
+
+        def __init__(self, layer):
+            super().__init__()
+            self.layer = layer
+
+        def forward(self, x, cos, sin, k_cache, v_cache, cache_position, attn_mask):
+            masks.append(attn_mask)
+            return self.layer(x, cos, sin, k_cache, v_cache, cache_position, attn_mask)
+
+    model.layers[2] = Own(model.layers[2])
+    got = run()
+    assert len(made) == 1 and float((got - want).norm() / want.norm()) <= 5e-3
+    assert len(masks) == 2 and all(torch.equal(m, make(32, at)) for m in masks)
