@@ -641,7 +641,10 @@ class LlamaDecoder(nn.Module):
         return emb.cos().half()[None, None], emb.sin().half()[None, None]
 
     def forward(self, ids, cache_position):
-        """ids (1, q_len) int64, cache_position (q_len,) int64 -> logits (1, q_len, vocab) fp32."""
+        """ids (1, q_len) int64, cache_position (q_len,) int64, slots below max_cache_len -> logits (1, q_len, vocab)
+        fp32."""
+        if cache_position.numel() > self.max_cache_len:  # (the positions themselves are device memory)
+            raise ValueError(f"{cache_position.numel()} tokens do not fit the key / value cache of {self.max_cache_len} slots")
         x = self.embed[ids]
         cos, sin = self.rope(cache_position)
         # one mask for all layers, made if something asks for it: from ROWS_MIN tokens on a layer may go without; hooks

@@ -301,6 +301,16 @@ def test_generate_refuses_requests_beyond_the_cache():
         long.decode_fused(torch.zeros((1, 1), dtype=torch.int64), torch.tensor([0]))
 
 
+@pytest.mark.parametrize("n", [9, 30])
+def test_forward_refuses_more_tokens_than_the_cache_has_slots(n):
+    """From the shapes alone, before a layer runs: past the cache keys and values would be dropped."""
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=1, ffn=832, vocab=96), max_cache_len=8,
+                         device="cpu", random_init=False)
+    with torch.no_grad(), pytest.raises(ValueError, match="do not fit the key / value cache"):
+        model(torch.zeros(1, n, dtype=torch.int64), torch.arange(n))
+
+
 def test_had_bits_reads_a_table_once_for_both_directions(monkeypatch):
     """A training step needs a table and its transpose: the caller's copy is read back and checked once."""
     from qtip_amd.utils import matmul_had as mh
