@@ -750,7 +750,7 @@ int launch_mix(const RhtParams& P, const MixShape& M, int kt, int rows, int cus,
 bool mix_shape(int n, int order, int rows, MixShape& M, int& kt) {
   int logp = 0;
   while ((n / order) >> (logp + 1)) ++logp;
-  if (logp < 3 || order > 32 * kMixMaxKT) return false;
+  if (logp < 3 || order > kMixMaxOrder) return false;
   int logpp = logp < 7 ? logp : 7;
   // fill the 32 rows of a wave before widening the columns
   while (logpp > 3 && ((long)order << (logp - logpp)) < 32) --logpp;
@@ -993,7 +993,7 @@ hipError_t qtip_rht_allow_lds() {
                        QTIP_MIX3(float, _Float16, PRE_NONE),       QTIP_MIX3(float, float, PRE_NONE)};
 #undef QTIP_MIX3
   for (const void* f : fns) {
-    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix_lds(kMixMaxKT, 172));
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix_lds(kMixMaxKT, kMixMaxOrder));
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -37,6 +37,7 @@ typedef uint32_t u32x4m __attribute__((ext_vector_type(4)));
 
 constexpr int kMixCols = 128;
 constexpr int kMixMaxKT = 8;
+constexpr int kMixMaxOrder = 32 * kMixMaxKT;  // table orders, built in or a caller's own
 
 struct MixShape {
   int logpp, logA2, logS;  // n = order << (logS + logA2 + logpp)

@@ -178,3 +178,24 @@ def test_many_rows_that_start_off_16_bytes(n, dtype):
     got, want = (ops.linear(x[i], packed, tlut, pre[i], sv[i], bits, K, None, 1, m, n, 2, n**-0.5 / 32, m**-0.5 * 32)
                  for i in (0, 1))
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("K,p", [(256, 8), (256, 128), (250, 16), (173, 64), (6, 32), (1, 8), (1, 16), (1, 64), (12, 8)])
+@pytest.mark.parametrize("rows", [24, 61])
+def test_any_order_of_signs(K, p, rows):
+    """A caller's own +-1 matrix of any order up to the largest the matrix form takes, and short rows, against float64."""
+    from qtip_amd import ops
+    from qtip_amd.utils.matmul_had import had_bits
+    n = K * p
+    g = torch.Generator(device="cuda").manual_seed(n + rows)
+    had = torch.randint(0, 2, (K, K), generator=g, device="cuda").float() * 2 - 1 if K > 1 else torch.ones(1, 1, device="cuda")
+    h64 = torch.from_numpy(scipy.linalg.hadamard(p).astype(np.float64)).cuda()
+    for dtype in (torch.float16, torch.float32):
+        x = torch.randn(rows, n, generator=g, device="cuda").to(dtype)
+        for transpose in (False, True):
+            bits = had_bits(had, K, transpose, "cuda") if K > 1 else None
+            z = (had.T if transpose else had).double() @ (x.double().view(rows, K, p) @ h64)
+            ref = z.reshape(rows, n) / n**0.5
+            y = ops.rht(x, order=K, had_bits=bits, out_dtype=torch.float32)
+            # exact products, fp32 sums of n terms
+            assert float((y.double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
