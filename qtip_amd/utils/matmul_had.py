@@ -68,7 +68,7 @@ def had_bits(hadK, K, transpose, device):
 
     hadK may be None (the built-in table of order K is used) or the caller's
     K x K tensor (as QuantizedLinear hands in); a caller-supplied tensor is
-    packed once per storage, for both directions, and must be a +-1 matrix.
+    read back once per storage, packed once per direction asked for, and must be a +-1 matrix.
     """
     dev = torch.device(device)
     if hadK is None or (K in _float_tables and hadK.data_ptr() == _float_tables[K].data_ptr()):
@@ -89,16 +89,20 @@ def had_bits(hadK, K, transpose, device):
         if h.shape != (K, K) or not np.all(np.abs(h) == 1.0):
             raise ValueError("hadK must be a K x K matrix of +-1")
         neg = h < 0
-        # a K x K table equal to the built-in one shares the built-in entry
+        # a K x K table equal to the built-in one shares the built-in entries
         if K in _ORDERS and np.array_equal(neg, _table_signs(K)):
-            bits = tuple(had_bits(None, K, t, dev) for t in (False, True))
-        else:
-            bits = tuple(torch.from_numpy(_pack_bits(b)).to(dev) for b in (neg, neg.T))
+            neg = None
         if hit is None or hit[0]() is not st:
             weakref.finalize(st, _bit_cache.pop, key, None)
-        hit = (weakref.ref(st), hadK._version, bits)
+        hit = (weakref.ref(st), hadK._version, neg, {})
         _bit_cache[key] = hit
-    return hit[2][bool(transpose)]
+    # (a forward pass asks for one direction: packing and copying the other would be paid by every first call)
+    neg, packed = hit[2:]
+    if neg is None:
+        return had_bits(None, K, transpose, dev)
+    if bool(transpose) not in packed:
+        packed[bool(transpose)] = torch.from_numpy(_pack_bits(neg.T if transpose else neg)).to(dev)
+    return packed[bool(transpose)]
 
 
 _dense_cache = {}

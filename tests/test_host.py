@@ -323,3 +323,23 @@ def test_had_bits_reads_a_table_once_for_both_directions(monkeypatch):
         monkeypatch.undo()
         assert not reads and torch.equal(bt, torch.from_numpy(mh._pack_bits((own.numpy() < 0).T)))
     assert not mh._table_signs(K).flags.writeable
+
+
+def test_had_bits_packs_the_direction_asked_for(monkeypatch):
+    """A forward pass asks for one direction of a table; the other is packed when something asks for it."""
+    from qtip_amd.utils import matmul_had as mh
+    h, K = mh.get_hadK(20 * 64)
+    packed, pack = [], mh._pack_bits
+    monkeypatch.setattr(mh, "_pack_bits", lambda neg: packed.append(1) or pack(neg))
+    monkeypatch.setattr(mh, "_bit_cache", {})
+    for own in (h.clone(), h.flip(0).contiguous()):
+        mh._bit_cache.clear()
+        for calls, transpose in ((1, True), (1, True), (2, False), (2, False)):
+            bits = mh.had_bits(own, K, transpose, "cpu")
+            assert len(packed) == calls
+            neg = own.numpy() < 0
+            assert torch.equal(bits, torch.from_numpy(pack(neg.T if transpose else neg)))
+        packed.clear()
+        own.neg_()
+        assert torch.equal(mh.had_bits(own, K, False, "cpu"), torch.from_numpy(pack(~neg)))
+        packed.clear()
