@@ -770,12 +770,36 @@ bool mix_shape(int n, int order, int rows, MixShape& M, int& kt) {
 // rows from which the one-workgroup-per-row form is used for the power-of-two sizes it covers
 constexpr int kRowsFormMin = 8;
 
-// Rows from which the matrix form is faster than one launch of order * A workgroups per row, which
-// each read the whole row.  Measured (us, that form / matrix form): fp16 rows of 12288 = 12 * 1024
-// 7.1 / 6.9 at 8 rows, 9.8 / 6.9 at 16; 28672 = 28 * 1024 9.2 / 11.2 at 8, 16.5 / 11.3 at 16;
-// 11008 = 172 * 64 15.4 / 10.8 at 8.  fp32 rows take three planes: 28672 16.5 / 21 at 16, 42 / 22 at
-// 45; 11008 15.4 / 19 at 8, 26 / 19 at 16.
-constexpr int mix_rows_min(int order, bool f16) { return order >= 100 ? (f16 ? 8 : 12) : (f16 ? 12 : 24); }
+// Rows from which the matrix form is faster than one launch of order * A workgroups per row (`wgs`), which each read
+// the whole row: its time hardly grows with the rows, theirs with rows * wgs once that passes what the chip holds.  fp32
+// rows take three planes.  Short rows cost either form little beside the launch, so the line is a count of workgroups
+// there; large orders over few points leave most of a wave's columns to other rows.  us in a graph, that form / matrix form:
+//   fp16  64 = 1 * 64, 400 rows 3.8/4.1, 600 4.7/4.1; 1024, 32 rows 3.9/4.4, 48 4.9/4.5; 1280 = 20 * 64, 32 rows 5.1/5.4,
+//         40 5.7/5.4; 3072 = 12 * 256, 16 rows 5.2/5.7, 20 5.9/5.7; 5120 = 20 * 256, 12 rows 4.8/5.9, 18 6.1/6.0;
+//         6144, 12 rows 6.0/5.9; 57344 = 28 * 2048, two slices, 12 rows 18.8/21.8, 16 24.2/22.1; 30720 = 60 * 512, 12 rows
+//         12.3/14.8, 16 16.0/15.0
+//         928 = 116 * 8, 8 rows 5.8/6.5, 12 7.2/6.9; 2240 = 140 * 16, 16 rows 8.0/8.7, 20 8.2/8.7, 24 9.7/8.7;
+//         4992 = 156 * 32, 8 rows 8.4/8.8, 12 11.7/8.8; 11008 = 172 * 64, 8 rows 14.8/10.1
+//   fp32  64, 1000 rows 5.4/6.3, 1600 7.8/6.3; 1024, 64 rows 5.4/6.3, 96 7.1/6.4; 3072, 32 rows 7.8/8.2, 36 8.7/8.2;
+//         5120, 28 rows 8.3/8.5, 36 9.4/8.5; 6144, 24 rows 8.3/8.4; 28672, 24 rows 19.8/19.6; 32768, 24 rows 17.9/22.6, 32
+//         25.2/23.1
+//         928, 32 rows 11.4/12.0, 48 15.6/12.0; 2240, 36 rows 11.6/13.9, 48 14.9/13.9; 4992, 16 rows 13.9/14.2, 18
+//         15.7/14.2; 8960 = 140 * 64, 8 rows 12.4/14, 12 16.8/14.4
+// With an element-wise prologue or a residual the matrix form is the one that covers every size, from 12 rows on.
+int mix_rows_min(int order, int n, long wgs, bool f16, bool fused, int kt, int slices) {
+  if (fused) return order >= 100 ? 8 : 12;
+  if (order >= 100) {
+    if (n <= 4096) return f16 ? (n < 1400 ? 14 : 20) : 42;
+    if (n < 8192) return f16 ? 9 : 18;
+    return f16 ? 8 : 12;
+  }
+  if (n <= 4096) return (int)(((f16 ? 512 + n / 10 : 1100 + n / 6) + wgs - 1) / wgs);
+  if (n < 6144) return f16 ? 16 : 32;
+  // (the largest workgroup, one to a CU; slices, which take three planes of either type)
+  const bool full = kt == kMixMaxKT && slices == 1;
+  if (f16) return slices > 1 || (full && order > 1) ? 16 : 12;
+  return full ? 28 : 24;
+}
 
 int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream) {
   if (!P.out || !P.in) return QTIP_E_NULL;
@@ -819,7 +843,7 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
       return launch_rht_rows<float, float>(P, rows, st);
     }
   }
-  if (rows >= mix_rows_min(order, in_dtype == QTIP_F16)) {
+  if (rows >= 8) {
     const size_t ez = in_dtype == QTIP_F16 ? 2 : 4;
     MixShape M{};
     int kt = 0;
@@ -828,7 +852,9 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
                     ((P.in_row_stride * ez) & 15u) == 0 && ((P.part_stride * ez) & 15u) == 0 &&
                     ((P.pre_row_stride * 2) & 15u) == 0 && ((P.post_row_stride * 4) & 15u) == 0 &&
                     !(P.pre_mode != PRE_NONE && in_dtype != QTIP_F16) && !(fused && out_dtype != QTIP_F16) &&
-                    mix_shape(n, order, rows, M, kt);
+                    mix_shape(n, order, rows, M, kt) &&
+                    rows >= mix_rows_min(order, n, OT, in_dtype == QTIP_F16, fused,
+                                         kt, 1 << M.logS);
     if (ok) {
       int cus = 0;
       const int rc = qtip_device_ready(stream, &cus);

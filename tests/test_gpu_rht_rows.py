@@ -25,6 +25,18 @@ def _transform(x, n, transpose):
                                53248, 57344])
 @pytest.mark.parametrize("rows", [24, 37])
 def test_rows_against_float64(n, rows):
+    _check_rows(n, rows)
+
+
+# short rows, which take the matrix form from more rows on: either side of the line for fp16 and for fp32 values
+@pytest.mark.parametrize("n,rows", [(64, 515), (64, 519), (64, 1107), (64, 1131), (256, 130), (256, 160), (256, 290),
+                                    (512, 147), (768, 48), (768, 103), (832, 61), (1024, 81), (1248, 13), (1248, 41),
+                                    (1280, 69), (2240, 17), (2240, 39), (3072, 35), (3456, 40), (4992, 19)])
+def test_short_rows_against_float64(n, rows):
+    _check_rows(n, rows)
+
+
+def _check_rows(n, rows):
     from qtip_amd import ops
     from qtip_amd.utils.matmul_had import get_hadK, had_bits
     had, K = get_hadK(n)
