@@ -204,11 +204,11 @@ class DecoderLayer(nn.Module):
         return _rows_linear(self.down, F.silu(gate) * up, residual=x)
 
     def forward(self, x, cos, sin, k_cache, v_cache, cache_position, attn_mask, causal=False):
-        """causal (or attn_mask None): a query attends to the cache slots up to its position, and attn_mask is that
-        mask or a function that makes it, called if the layer goes module by module."""
+        """attn_mask (tokens, slots), None for every slot.  causal: the mask is that of the slots up to each position, and
+        attn_mask is it, a function that makes it or None: asked for only if the layer goes module by module."""
         cfg = self.cfg
-        if causal or attn_mask is None:
-            if x.shape[0] == 1 and self.rows_ok(x[0], k_cache, v_cache, cache_position):
+        if causal:
+            if x.shape[0] == 1 and self.rows_ok(x[0], k_cache, v_cache, cache_position) and _rotary_ok(cos, sin, x, cfg):
                 return self._forward_rows(x[0], cos[0, 0], sin[0, 0], k_cache, v_cache, cache_position)[None]
             if attn_mask is None:
                 attn_mask = _causal_mask(k_cache.shape[2], cache_position)
@@ -437,6 +437,12 @@ class DecoderLayer(nn.Module):
         return f['down'].transform_out(pd, residual=x), None
 
 
+def _rotary_ok(cos, sin, x, cfg):
+    """The tables of a rotary embedding as the attention kernel reads them (a caller's own `rope` may make others)."""
+    return all(t.shape == (1, 1, x.shape[1], cfg.head_dim) and t.dtype == torch.float16 and t.device == x.device
+               and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (cos, sin))
+
+
 def _watched(module):
     """Something runs beside, or in place of, the module's own forward."""
     return bool(module._forward_hooks or module._forward_pre_hooks or 'forward' in module.__dict__)
@@ -647,16 +653,16 @@ class LlamaDecoder(nn.Module):
             raise ValueError(f"{cache_position.numel()} tokens do not fit the key / value cache of {self.max_cache_len} slots")
         x = self.embed[ids]
         cos, sin = self.rope(cache_position)
-        # one mask for all layers, made if something asks for it: from ROWS_MIN tokens on a layer may go without; hooks
-        # and anyone's own layers are handed the tensor
+        # one mask for all layers, made if something asks for it: from ROWS_MIN tokens on a layer may go without.  Hooks
+        # and anyone's own layers are handed the tensor, and a hook in front of a layer may hand on another one
         mask = functools.lru_cache(maxsize=1)(lambda: _causal_mask(self.max_cache_len, cache_position))
         few, hooked = ids.shape[-1] < ROWS_MIN or not ids.is_cuda, _all_modules_hooked()
         for i, layer in enumerate(self.layers):
             args = (x, cos, sin, self.k_cache[i], self.v_cache[i], cache_position)
-            if few or type(layer) is not DecoderLayer or 'forward' in layer.__dict__:
+            if few or hooked or type(layer) is not DecoderLayer or 'forward' in layer.__dict__ or layer._forward_pre_hooks:
                 x = layer(*args, mask())
             else:
-                x = layer(*args, mask() if hooked or _watched(layer) else mask, causal=True)
+                x = layer(*args, mask() if layer._forward_hooks else mask, causal=True)
         x = self.norm(x)
         return (x @ self.lm_head.T).float()
 

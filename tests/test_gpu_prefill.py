@@ -166,7 +166,8 @@ def test_layer_input_that_starts_off_16_bytes():
     x.copy_(torch.randn(x.shape, generator=torch.Generator().manual_seed(0)))
     assert not model.layers[0].rows_ok(x[0], model.k_cache[0], model.v_cache[0], at)
     with torch.no_grad():
-        got, want = (model.layers[0](t, cos, sin, model.k_cache[0], model.v_cache[0], at, None) for t in (x, x.clone()))
+        got, want = (model.layers[0](t, cos, sin, model.k_cache[0], model.v_cache[0], at, None, causal=True)
+                     for t in (x, x.clone()))
     assert float((got.double() - want.double()).norm() / want.double().norm()) <= 5e-3
 
 
@@ -211,3 +212,65 @@ def test_one_mask_for_all_layers(monkeypatch):
     got = run()
     assert len(made) == 1 and float((got - want).norm() / want.norm()) <= 5e-3
     assert len(masks) == 2 and all(torch.equal(m, make(32, at)) for m in masks)
+
+
+def test_a_layer_without_a_mask_attends_to_every_slot():
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=1, ffn=832, vocab=96), max_cache_len=32)
+    g = torch.Generator(device="cuda").manual_seed(0)
+    at, x = torch.arange(20, device="cuda"), torch.randn(1, 20, 256, generator=g, device="cuda").half()
+    cos, sin = model.rope(at)
+    k, v = (torch.randn(1, 2, 32, 64, generator=g, device="cuda").half() for _ in range(2))
+    layer = model.layers[0]
+    every = torch.ones(1, 1, 20, 32, dtype=torch.bool, device="cuda")
+    with torch.no_grad():
+        got, want, causal = (layer(x, cos, sin, k, v, at, mask, causal=c) for mask, c in ((None, False), (every, False), (None, True)))
+    far = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm())
+    assert far(got, want) <= 5e-3 < far(causal, want)
+
+
+def test_a_hook_in_front_of_a_layer_may_replace_the_mask():
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=2, ffn=832, vocab=96), max_cache_len=32)
+    ids, at = torch.arange(20, device="cuda")[None], torch.arange(20, device="cuda")
+    near = (at[:, None] - torch.arange(32, device="cuda")[None, :]).abs()[None, None] < 4
+
+    def window(mod, args):
+        return args[:6] + (args[6] & near,)
+
+    with torch.no_grad():
+        plain = model(ids, at)
+        hook = model.layers[1].register_forward_pre_hook(window)
+        got = model(ids, at)
+        hook.remove()
+        # the same mask by hand
+        x, (cos, sin) = model.embed[ids], model.rope(at)
+        causal = torch.arange(32, device="cuda")[None, :] <= at[:, None]
+        for layer, mask, k, v in zip(model.layers, (causal, causal & near), model.k_cache, model.v_cache):
+            x = layer(x, cos, sin, k, v, at, mask.view(1, 1, 20, 32))
+        want = (model.norm(x) @ model.lm_head.T).float()
+    far = lambda a, b: float((a - b).norm() / b.norm())
+    assert far(got, want) <= 5e-3 < far(plain, want)
+
+
+@pytest.mark.parametrize("form", ["strided", "off", "shared"])
+def test_rotary_tables_of_the_callers_own(form):
+    """Tables the attention kernel does not read as they stand go module by module."""
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=2, ffn=832, vocab=96), max_cache_len=32)
+    ids, at = torch.arange(20, device="cuda")[None], torch.arange(20, device="cuda")
+    rope = model.rope
+
+    def own(positions):
+        if form == "strided":
+            return tuple(t.transpose(2, 3).contiguous().transpose(2, 3) for t in rope(positions))
+        if form == "off":
+            return tuple(torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view_as(t).copy_(t) for t in rope(positions))
+        return tuple(t[:, :, :1] for t in rope(positions))  # one angle for every token
+
+    with torch.no_grad():
+        want = model(ids, at)
+        model.rope = own
+        got = model(ids, at)
+    far = float((got - want).norm() / want.norm())
+    assert got.isfinite().all() and (far > 5e-3 if form == "shared" else far <= 5e-3)
