@@ -65,10 +65,11 @@ __global__ __launch_bounds__(kBlock) void cache_rows_kernel(
 // consecutive dims per register.  Scores, softmax and sums in fp32; a probability enters the second product as two fp16
 // numbers, its rounded value and the rest, 22 bits of it or 2^-25 of the largest: rounded to one, outputs
 // were up to 1.013 times as far from float64 as the library's attention (2.38e-4 and 2.35e-4 at 150 tokens of 32
-// heads of 128), with two they are the correctly rounded ones (1.96e-4).
+// heads of 128), with two they are the correctly rounded ones (1.96e-4).  The rests have accumulators of their own: an
+// infinite value times a rest of zero is a NaN where times the probability it is infinite, and is left out.
 // Bound by a wave's chain through a tile (products, maximum, exponentials, products): the latest queries
 // run first, and 16-query waves give two workgroups per CU at 1000 tokens of 32 heads.  us, 1000 tokens, 32
-// heads of 128: 46 (42 with one fp16 number per probability) and 8 for the caches, where the library's attention
+// heads of 128: 45 (42 with one fp16 number per probability) and 8 for the caches, where the library's attention
 // under a dense mask took 193 beside about 150 of small passes (rotation, cache writes, copies of heads).
 constexpr int kQ = 64, kKeys = 64;
 
@@ -155,9 +156,9 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
     }
   };
 
-  float4v o[NE];
+  float4v o[NE], rest_o[NE];
 #pragma unroll
-  for (int e = 0; e < NE; ++e) o[e] = float4v{0.f, 0.f, 0.f, 0.f};
+  for (int e = 0; e < NE; ++e) o[e] = rest_o[e] = float4v{0.f, 0.f, 0.f, 0.f};
   float mx = -__builtin_inff(), sum = 0.f;  // the query's maximum; this lane's share of its sum
   load_tile(0);
   for (int kk0 = 0; kk0 < kmax; kk0 += kKeys) {
@@ -186,17 +187,21 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
       }
     tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16));
     tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
-    const float fade = __builtin_amdgcn_exp2f(mx - tile_max);  // (key 0 is in every query's range: finite from the first tile)
+    const float base = fmaxf(tile_max, -3.0e38f);  // (nothing but scores of -inf so far)
+    const float fade = __builtin_amdgcn_exp2f(mx - base);
     mx = tile_max;
     sum *= fade;
 #pragma unroll
-    for (int e = 0; e < NE; ++e) o[e] *= fade;
+    for (int e = 0; e < NE; ++e) {
+      o[e] *= fade;
+      rest_o[e] *= fade;
+    }
     half8v p[2], rest[2];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float x = __builtin_amdgcn_exp2f(s[t][r] - mx);
+        const float x = __builtin_amdgcn_exp2f(s[t][r] - base);
         sum += x;
         const _Float16 h = (_Float16)x;
         p[t >> 1][4 * (t & 1) + r] = h;
@@ -205,19 +210,23 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int e0 = 0; e0 < NE; e0 += 4) {  // (four accumulators apart, the two products of one do not wait for each other)
+      for (int e0 = 0; e0 < NE; e0 += 4) {  // (four reads in flight)
         half8v a[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) a[e] = *reinterpret_cast<const half8v*>(lds_v + (16 * (e0 + e) + ql) * VSTR + 64 * kk + 16 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e0 + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[e], rest[kk], o[e0 + e], 0, 0, 0);
-#pragma unroll
         for (int e = 0; e < 4; ++e) o[e0 + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[e], p[kk], o[e0 + e], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rest_o[e0 + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[e], rest[kk], rest_o[e0 + e], 0, 0, 0);
       }
   }
   sum += __shfl_xor(sum, 16);
   sum += __shfl_xor(sum, 32);
   const float inv = 1.f / sum;
+#pragma unroll
+  for (int e = 0; e < NE; ++e)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[e][r] += __builtin_isfinite(rest_o[e][r]) ? rest_o[e][r] : 0.f;
   if (i >= n) return;
   // row 16 e + x of V^T is dim 8 c + e' with e' * CPK + c = 16 e + x
   _Float16* dst = out + ((size_t)i * heads + h) * HD;

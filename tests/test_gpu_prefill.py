@@ -274,3 +274,60 @@ def test_rotary_tables_of_the_callers_own(form):
         got = model(ids, at)
     far = float((got - want).norm() / want.norm())
     assert got.isfinite().all() and (far > 5e-3 if form == "shared" else far <= 5e-3)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_infinite_values_and_scores(hd):
+    """An infinite value makes the outputs infinite that weigh it, and only those; keys with a score of minus infinity, however
+    many come first, do not count; a NaN key leaves the queries before its tile alone."""
+    from qtip_amd import ops
+    past, n, heads, inf = 70, 150, 3, float("inf")
+    slots = past + n
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    q, k, v = (torch.randn(heads, m, hd, generator=g, device="cuda").half() for m in (n, slots, slots))
+    v[0, 140, 5], v[0, 200, 9] = inf, -inf  # of queries 70 and 130
+    q[1, :, 3] = q[1, :, 3].abs() + 0.01
+    k[1, :past, 3] = -inf
+    k[2, 160, 7] = math.nan
+    pos = torch.arange(past, slots, device="cuda")
+    one = torch.ones(n, hd, device="cuda").half()
+    kc, vc = k[None].clone(), v[None].clone()
+    rows = lambda t: t.transpose(0, 1).reshape(n, heads * hd).contiguous()
+    out = ops.prefill_attention(rows(q), rows(k[:, past:]), rows(v[:, past:]), one, torch.zeros_like(one), kc, vc, pos, heads, heads, hd)
+    out = out.view(n, heads, hd).transpose(0, 1)
+    s = (q.double() @ k.double().transpose(1, 2).contiguous() / math.sqrt(hd))
+    p = s.masked_fill(torch.arange(slots, device="cuda")[None, :] > pos[:, None], -inf).softmax(-1)
+    want = p @ v.double().nan_to_num(posinf=0.0, neginf=0.0)
+    size = p @ v.double().abs().nan_to_num(posinf=0.0)
+    want[0, 70:, 5], want[0, 130:, 9] = inf, -inf
+    # probabilities (2^-11 each where an infinity is about) and the result rounded to fp16
+    near = lambda h, at: bool(((out[h][at].double() - want[h][at]).abs() <= 2.0**-10 * size[h][at]).all())
+    assert torch.equal(out[0, 70:, 5].float(), want[0, 70:, 5].float()) and torch.equal(out[0, 130:, 9].float(), want[0, 130:, 9].float())
+    finite = torch.tensor([c not in (5, 9) for c in range(hd)], device="cuda")
+    assert near(0, (slice(None), finite)) and near(0, slice(0, 64))
+    assert near(1, slice(None))
+    assert near(2, slice(0, 64)) and out[2, 90:].isnan().all()
+
+
+@pytest.mark.parametrize("order", ["descending", "gaps", "shuffled", "late"])
+def test_positions_in_any_order(order):
+    """Keys go to the slots of their positions and a query sees the slots up to its own, whatever order they come in."""
+    from qtip_amd import ops
+    n, slots, heads, kv, hd = 90, 300, 4, 2, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn(n, h * hd, generator=g, device="cuda").half() for h in (heads, kv, kv))
+    kc, vc = (torch.randn(1, kv, slots, hd, generator=g, device="cuda").half() for _ in range(2))
+    pos = {"descending": torch.arange(n).flip(0), "gaps": torch.arange(n) * 3 + 1, "late": torch.arange(slots - n, slots),
+           "shuffled": torch.randperm(slots, generator=torch.Generator().manual_seed(1))[:n]}[order].cuda()
+    one = torch.ones(n, hd, device="cuda").half()
+    wk, wv = kc.clone(), vc.clone()
+    wk[0, :, pos] = k.view(n, kv, hd).transpose(0, 1)
+    wv[0, :, pos] = v.view(n, kv, hd).transpose(0, 1)
+    out = ops.prefill_attention(q, k, v, one, torch.zeros_like(one), kc, vc, pos, heads, kv, hd)
+    assert torch.equal(kc, wk) and torch.equal(vc, wv)
+    kk, vv = (t[0].double().repeat_interleave(heads // kv, 0) for t in (wk, wv))
+    s = q.double().view(n, heads, hd).transpose(0, 1) @ kk.transpose(1, 2).contiguous() / math.sqrt(hd)
+    p = s.masked_fill(torch.arange(slots, device="cuda")[None, :] > pos[:, None], -math.inf).softmax(-1)
+    want, size = ((p @ t).transpose(0, 1).reshape(n, -1) for t in (vv, vv.abs()))
+    # the rounding of the result and fp32 scores (as test_prefill_probabilities_are_not_rounded_to_fp16 derives)
+    assert bool(((out.double() - want).abs() <= 2.0**-11 * want.abs() + 2.0**-25 + 2.0**-18 * size).all())
