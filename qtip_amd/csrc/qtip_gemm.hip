@@ -300,6 +300,12 @@ __global__ __launch_bounds__(256) void sum_parts_round_kernel(TOut* __restrict__
 // S k ranges of wl_per 64-column wave-loads.  Few pairs are cut along k as well (only when the caller
 // provides room for the partial results).
 constexpr int kGemmRows = 128;
+// ... and fewer where that many activations pass what a buffer's 32-bit offsets reach (2 GiB less the offset that
+// stands for padding): from k = 2^23 on
+int pass_rows(int k) {
+  const long fit = 0x7FFFFF00L / (2L * k);
+  return fit < kGemmRows ? (int)fit : kGemmRows;
+}
 struct GemmPlan {
   int NB, waves, RG, S, wl_per, ngroups;
 };
@@ -340,8 +346,9 @@ int run_gemm(TOut* out, const void* packed, const void* x_f16, const void* tlut,
   hipStream_t st = (hipStream_t)stream;
   auto* p = (const uint8_t*)packed;
   auto* t = (const uint32_t*)tlut;
-  for (int b0 = 0; b0 < batch; b0 += kGemmRows) {
-    const int nb = batch - b0 < kGemmRows ? batch - b0 : kGemmRows;
+  const int step = pass_rows(k);
+  for (int b0 = 0; b0 < batch; b0 += step) {
+    const int nb = batch - b0 < step ? batch - b0 : step;
     const GemmPlan g = gemm_plan(m, k, nb, cus, workspace != nullptr);
     const long units = (long)g.ngroups * g.S;
     long grid = units < cus ? units : cus;
@@ -417,7 +424,8 @@ size_t qtip_gemm_workspace_bytes(int m, int k, int bits, int batch) {
   const int cus = qtip_device_cus();
   if (!cus) return 0;
   size_t need = 0;  // the largest pass: full ones and the remainder
-  for (int nb : {batch < kGemmRows ? batch : kGemmRows, batch % kGemmRows}) {
+  const int step = pass_rows(k);
+  for (int nb : {batch < step ? batch : step, batch % step}) {
     if (nb < 1) continue;
     const GemmPlan g = gemm_plan(m, k, nb, cus, true);
     const size_t bytes = g.S > 1 ? (size_t)g.S * nb * m * sizeof(float) : 0;

@@ -33,3 +33,23 @@ def test_fp16_results_are_rounded_ones():
     with pytest.raises(ValueError):
         ops.decompress_gemm(packed, x, torch.zeros(1024, dtype=torch.float16, device="cuda"), 64, 64, 2, round_f16=False,
                             out_dtype=torch.float16)
+
+
+@pytest.mark.parametrize("k", [1 << 23, (1 << 24) + 32])
+def test_activations_beyond_two_gib(k):
+    """As many rows as pass the reach of 32-bit offsets (128 of 2^23 columns, 64 of 2^24) against float64 in pieces."""
+    from qtip_amd import ops
+    m, bits, rows = 32, 2, 128
+    g = torch.Generator(device="cuda").manual_seed(k)
+    packed = torch.randint(-32768, 32768, (m * k * bits // 16,), dtype=torch.int16, generator=g, device="cuda")
+    tlut = torch.randn(1024, generator=g, device="cuda").half()
+    x = torch.randn(rows, k, generator=g, device="cuda", dtype=torch.float16)
+    y = ops.decompress_gemm(packed, x, tlut, m, k, bits, round_f16=False).double()
+    w = ops.decode(packed, tlut, m, k, bits)
+    want, size = torch.zeros(2, rows, m, dtype=torch.float64, device="cuda")
+    for c in range(0, k, 1 << 20):
+        a, b = x[:, c:c + (1 << 20)].double(), w[:, c:c + (1 << 20)].double().T.contiguous()
+        want += a @ b
+        size += a.abs() @ b.abs()
+    # fp32 sums in chains of a few thousand products whose errors add like their square roots: 2^-20 of the magnitudes
+    assert bool(((y - want).abs() <= 2.0**-20 * size).all())
