@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kBlock) void sum_rows_kernel(float* __restrict__ gs
 }
 
 // Rows of a workgroup: about 1024 workgroups (four a CU) where there are enough rows, at least four rows per wave,
-// so that the partial sums are a sixteenth of what is read at most.
+// so that the partial sums are a sixteenth of what is read at most from 8 rows on (one row of n for fewer).
 int chunk_rows(int rows, int n) {
   const int colb = (n + kCols - 1) / kCols;
   const int chunks = (1024 + colb - 1) / colb;
