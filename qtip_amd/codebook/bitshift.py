@@ -362,7 +362,8 @@ class BitshiftLinear(nn.Module):
         128 rows, the dense route writes and reads 2 m n bytes once, and the library's product takes long where a
         large n meets few output tiles and, with some widths, at multiples of 32 rows.  us of the products at 2 / 3 / 4
         bits, in a graph, dense / fused:
-          4096x4096    129 rows 36/41 35/42 35/40; 176 rows 35/47 35/48 34/47; 192 rows 46/48 45/49 45/48; 193 rows 35/56 34/58 34/55
+          4096x4096    129 rows 36/41 35/42 35/40; 176 rows 35/47 35/48 34/47; 192 rows 46/48 45/49 45/48;
+                       193 rows 35/56 34/58 34/55
           22016x4096   193 rows 100/103 98/119 101/104; 256 rows 106/107 103/124 102/110
           8192x8192    256 rows 105/89 105/96 107/89; 257 rows 94/100 95/109 96/101
           5120x13824   256 rows 150/99 151/114 152/100; 257 rows 104/115 106/131 105/115
@@ -370,7 +371,8 @@ class BitshiftLinear(nn.Module):
           8192x28672   320 rows 344/215 343/247 345/226; 512 rows 427/331 429/391 433/355; 513 rows 366/356 370/418 375/380
         A call that is not recorded waits for the host on small matrices, and the dense route's launches cost it twice
         what `ops.linear` does: whole calls, dense / fused, 2048x2048 129 rows 74/39 and 192 rows 72/42 (the products alone
-        19/31 and 19/35), 4096x4096 129 rows 73/48 and 192 rows 74/57.  So the line is where a third pass starts there too."""
+        19/31 and 19/35), 4096x4096 129 rows 73/48 and 192 rows 74/57.  So the line stays there at the rows from which the
+        second pass runs the kernel of more than 64."""
         if n < 5120 or m * n < 1 << 26:
             return rows_min
         if n < 8192 or m * n < 1 << 27:
