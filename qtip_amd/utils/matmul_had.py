@@ -98,11 +98,12 @@ def had_bits(hadK, K, transpose, device):
         _bit_cache[key] = hit
     # (a forward pass asks for one direction: packing and copying the other would be paid by every first call)
     neg, packed = hit[2:]
-    if neg is None:
-        return had_bits(None, K, transpose, dev)
-    if bool(transpose) not in packed:
-        packed[bool(transpose)] = torch.from_numpy(_pack_bits(neg.T if transpose else neg)).to(dev)
-    return packed[bool(transpose)]
+    bits = packed.get(bool(transpose))
+    if bits is None:
+        bits = had_bits(None, K, transpose, dev) if neg is None else \
+            torch.from_numpy(_pack_bits(neg.T if transpose else neg)).to(dev)
+        packed[bool(transpose)] = bits
+    return bits
 
 
 _dense_cache = {}
