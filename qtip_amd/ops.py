@@ -318,7 +318,7 @@ def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, 
             if bits_t.numel() * 32 < order * order:
                 raise ValueError("sign bits too short")
     dt = _DT[x.dtype]
-    if rows >= _ALIGN_ROWS:
+    if rows >= _ALIGN_ROWS and (x.data_ptr() | su.data_ptr() | sv.data_ptr()) & 15:
         x, su, sv = map(aligned16, (x, su, sv))
     out = torch.empty((rows, m), dtype=x.dtype, device=dev)
     L = lib()
@@ -388,7 +388,8 @@ def rht(x, order=1, had_bits=None, pre=None, post=None, scale=None, out_dtype=No
         return out
     if scale is None:
         scale = n ** -0.5
-    if rows >= _ALIGN_ROWS and n % 8 == 0:
+    if rows >= _ALIGN_ROWS and n % 8 == 0 and (x.data_ptr() | (_ptr(pre) or 0) | (_ptr(post) or 0) |
+                                               (_ptr(norm_weight) or 0) | (_ptr(residual) or 0)) & 15:
         x, pre, post, norm_weight, residual = map(aligned16, (x, pre, post, norm_weight, residual))
     L = lib()
     with _on(x.device):
