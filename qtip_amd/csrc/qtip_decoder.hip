@@ -334,8 +334,8 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
   // KU keys per thread group and round, all of their loads issued before the first use: two, or one where no more than
   // RK are left.  (Four keys and eight values in flight, and 64-bit addresses for each, did not fit a thread's 128
   // registers: the spills cost more than the wider rounds gained.  us, spilling / now, 32 heads of 128 on 32 kv heads,
-  // cold caches: 60 keys 5.8 / 4.4, 500 9.3 / 8.8, 1000 19.4 / 13.7; 64 heads on 8, 900 keys 16.5 / 12.2; 32 heads on 8 in 8
-  // ranges, 2000 keys 14.9 / 14.1, 4000 20.0 / 18.8.)
+  // cold caches: 60 keys 6.6 / 5.3, 300 8.3 / 9.2 (the second round of either), 500 11.1 / 10.3, 1000 21.9 / 15.6; 64 heads
+  // on 8, 900 keys 19.4 / 13.8; 32 heads on 8 in 8 ranges, 2000 keys 17.5 / 16.2, 4000 21.3 / 20.0.)
   constexpr int KU = 2, RK = kAttnThreads / 8;
   auto cache_row = [&](const _Float16* base, int t, int d) {  // 32-bit offset from a uniform base
     const int tc = (t < k1 && t != pos) ? t : 0;              // clamped: the new key comes from LDS
