@@ -388,9 +388,11 @@ def rht(x, order=1, had_bits=None, pre=None, post=None, scale=None, out_dtype=No
         return out
     if scale is None:
         scale = n ** -0.5
-    if rows >= _ALIGN_ROWS and n % 8 == 0 and (x.data_ptr() | (_ptr(pre) or 0) | (_ptr(post) or 0) |
-                                               (_ptr(norm_weight) or 0) | (_ptr(residual) or 0)) & 15:
+    p_pre, p_post = _ptr(pre), _ptr(post)
+    if rows >= _ALIGN_ROWS and n % 8 == 0 and (x.data_ptr() | (p_pre or 0) | (p_post or 0) | (
+            fused and ((_ptr(norm_weight) or 0) | (_ptr(residual) or 0)))) & 15:
         x, pre, post, norm_weight, residual = map(aligned16, (x, pre, post, norm_weight, residual))
+        p_pre, p_post = _ptr(pre), _ptr(post)
     L = lib()
     with _on(x.device):
         width = x.shape[-1]
@@ -405,13 +407,13 @@ def rht(x, order=1, had_bits=None, pre=None, post=None, scale=None, out_dtype=No
             src = xf if in_parts > 1 else xf[r0:r1]
             if fused:
                 check(L.qtip_rht_fused(_ptr(of[r0:r1]), _DT[out_dtype], _ptr(src), _DT[x.dtype], in_parts, r1 - r0, n,
-                                       order, _ptr(had_bits), _ptr(pre), _ptr(post), ctypes.c_float(scale), pre_mode,
+                                       order, _ptr(had_bits), p_pre, p_post, ctypes.c_float(scale), pre_mode,
                                        _ptr(norm_weight), ctypes.c_float(eps),
                                        _ptr(rf[r0:r1]) if rf is not None else _ptr(None),
                                        stream_ptr(x.device)), "qtip_rht_fused")
             else:
                 check(L.qtip_rht(_ptr(of[r0:r1]), _DT[out_dtype], _ptr(src), _DT[x.dtype], in_parts, r1 - r0, n,
-                                 order, _ptr(had_bits), _ptr(pre), _ptr(post), ctypes.c_float(scale),
+                                 order, _ptr(had_bits), p_pre, p_post, ctypes.c_float(scale),
                                  stream_ptr(x.device)), "qtip_rht")
     return out
 
