@@ -291,7 +291,7 @@ class BitshiftLinear(nn.Module):
                      and n in ops.RHT_IN_MATVEC_SIZES)
         if in_matvec:
             xt = None
-        elif fused_in and by_library(bs, n, K_left):
+        elif fused_in and by_library(bs, n, K_left, x.is_cuda):
             xt = rht_many_rows(x.contiguous(), had_left, K_left, True, pre=SU, scale=(n**-0.5) / self.scale,
                                out_dtype=torch.float16)
         elif fused_in:
@@ -335,7 +335,7 @@ class BitshiftLinear(nn.Module):
         # ---- output transform: (H_R y / sqrt(m)) * SV * 32, cast
         fused_out = (rcp != 2 and SV.dtype == torch.float32 and SV.device == dev
                      and input.dtype in (torch.float16, torch.float32))
-        if fused_out and in_parts == 1 and by_library(bs, m, K_right):
+        if fused_out and in_parts == 1 and by_library(bs, m, K_right, x.is_cuda):
             out = rht_many_rows(y.reshape(bs, m), had_right, K_right, False, post=SV, scale=(m**-0.5) * self.scale,
                                 out_dtype=input.dtype)
         elif fused_out:

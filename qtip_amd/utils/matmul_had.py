@@ -123,13 +123,14 @@ def _dense_sylvester(p, device):
 _MANY_ROWS_DENSE_P = 256
 
 
-def by_library(rows, n, K):
+def by_library(rows, n, K, on_gpu=True):
     """A transform of `rows` vectors of n = K * p runs as library products (rht_many_rows): orders and parts which
     the matrix form of the transform kernel does not take (p < 8, K > 256), from the rows on from which the
     products are faster than the kernel's one set of workgroups per row.  us, kernel / products, fp16: 688 = 172 * 4,
     96 / 300 / 1000 rows 43/61 123/60 382/61; 432 = 108 * 4 30/61 80/61 242/61; 172 * 1, 96 rows 67/63; 2048 = 512 * 4,
-    96 rows 119/60; 4800 = 300 * 16, 96 rows 137/61."""
-    return rows >= 96 and K >= 100 and rows * K >= 24000 and (n // K < 8 or K > 256)
+    96 rows 119/60; 4800 = 300 * 16, 96 rows 137/61.  In host memory, where the kernel does not run, from 96 rows on at
+    every order from 100 on."""
+    return rows >= 96 and K >= 100 and (not on_gpu or (rows * K >= 24000 and (n // K < 8 or K > 256)))
 
 
 def rht_many_rows(x, hadK, K, transpose, pre=None, post=None, scale=None, out_dtype=None):
@@ -196,7 +197,7 @@ def _hadU(X, hadK, K, transpose):
     if K == 1:
         return torch.ops.hadamard.hadamard(X.contiguous(), n**(-0.5))
     x = X if X.dtype in (torch.float16, torch.float32) else X.float()
-    if by_library(x.numel() // n, n, K):
+    if by_library(x.numel() // n, n, K, x.is_cuda):
         return rht_many_rows(x.reshape(-1, n).contiguous(), hadK, K, transpose).to(X.dtype).reshape(X.shape)
     out = ops.rht(x.contiguous(), order=K, had_bits=had_bits(hadK, K, transpose, X.device), out_dtype=x.dtype)
     return out.to(X.dtype).reshape(X.shape)
@@ -222,7 +223,7 @@ class _HadamardCastFn(torch.autograd.Function):
 
 def _hadU_cast(X, hadK, K, transpose, scale, out_dtype):
     n = X.shape[-1]
-    if by_library(X.shape[0], n, K):
+    if by_library(X.shape[0], n, K, X.is_cuda):
         return rht_many_rows(X.contiguous(), hadK, K, transpose, scale=n**-0.5 * scale, out_dtype=out_dtype)
     bits = had_bits(hadK, K, transpose, X.device) if K > 1 else None
     return ops.rht(X.contiguous(), order=K, had_bits=bits, scale=n**-0.5 * scale, out_dtype=out_dtype)

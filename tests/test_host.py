@@ -343,3 +343,45 @@ def test_had_bits_packs_the_direction_asked_for(monkeypatch):
         own.neg_()
         assert torch.equal(mh.had_bits(own, K, False, "cpu"), torch.from_numpy(pack(~neg)))
         packed.clear()
+
+
+@pytest.mark.parametrize("n,K", [(11008, 172), (1248, 156), (624, 156)])
+def test_large_orders_in_host_memory(n, K):
+    """From 96 rows on, orders from 100 on are products, which run on the CPU too; against float64."""
+    from qtip_amd.utils import matmul_had as mh
+    had, order = mh.get_hadK(n)
+    assert order == K
+    p = n // K
+    h = torch.ones(1, 1, dtype=torch.float64)
+    while h.shape[0] < p:
+        h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)])
+    x = torch.randn(96, n, generator=torch.Generator().manual_seed(n))
+    for t in (False, True):
+        ref = ((had.T if t else had).double() @ (x.double().view(96, K, p) @ h)).reshape(96, n) / n**0.5
+        y = x.clone().requires_grad_()
+        for out in (mh.matmul_hadU_cuda(x, had, K, t), mh.hadU_cast(x, had, K, t, 1.0, torch.float32), mh.matmul_hadU_cuda(y, had, K, t)):
+            assert float((out.detach().double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
+        (g,) = torch.autograd.grad(out, y, x)
+        back = ((had if t else had.T).double() @ (x.double().view(96, K, p) @ h)).reshape(96, n) / n**0.5
+        assert float((g.double() - back).abs().max()) <= 1e-5 * float(back.abs().max())
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_module_without_a_kernel_in_host_memory(grad):
+    """Projection of large table orders on the CPU, 96 rows or more: input and output transforms are products."""
+    from qtip_amd.codebook.bitshift import BitshiftLinear
+    from qtip_amd.utils import matmul_had as mh
+    m, k, K = 928, 1248, 2
+    g = torch.Generator().manual_seed(2)
+    mod = BitshiftLinear(16, 16, 16, K, 2, 9, "quantlut_sym", tlut=torch.randn(512, 2, generator=g).half(), has_kernel=False)
+    states = torch.randint(0, 1 << 16, (m // 16 * k // 16, 128), generator=g)
+    x = torch.randn(100, k, generator=g)
+    SU, SV = torch.randn(k, generator=g).sign().half(), torch.randn(m, generator=g).requires_grad_(grad)
+    (hl, kl), (hr, kr) = mh.get_hadK(k), mh.get_hadK(m)
+    y = mod(x, states, SU, SV, hl, hr, kl, kr, 0, 8, mode="train-recons")
+    w = mod.get_hatW(states, m, k).double()
+    h8 = torch.tensor([[(-1.0)**bin(i & j).count("1") for j in range(8)] for i in range(8)], dtype=torch.float64)
+    t = lambda v, had, n: (had.double() @ (v.reshape(-1, had.shape[0], 8) @ h8)).reshape(-1, n) / n**0.5
+    want = t((t(x.double() * SU.double(), hl.T, k) / 32).half().double() @ w.T, hr, m) * SV.detach().double() * 32
+    assert y.requires_grad == grad
+    assert float((y.detach().double() - want).norm() / want.norm()) <= 2.0**-10  # the product's rounding to fp16, once
