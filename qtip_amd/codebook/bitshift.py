@@ -142,7 +142,7 @@ class bitshift_codebook(nn.Module):
         t = self.tlut
         if (self.decode_mode == 'quantlut_sym' and t.is_cuda and t.dtype in (torch.float16, torch.float32)
                 and t.shape == (1 << self.tlut_bits, 2) and self.tlut_bits < 16 and t.is_contiguous()
-                and not (torch.is_grad_enabled() and t.requires_grad)):
+                and not (torch.is_grad_enabled() and t.requires_grad) and ops.launchable(t)):
             self.lut = ops.expand_table(t, self.tlut_bits)
         else:
             self.lut = self._expand().T.contiguous()

@@ -70,6 +70,17 @@ def aligned16(t):
     return t if t is None or t.data_ptr() % 16 == 0 else t.clone()
 
 
+def launchable(*tensors):
+    """The tensors are memory that a launch can be given: nothing traces the program, and none of them is a wrapper
+    (batched gradients, fake tensors).  What passes by torch's own or registered operations asks this first."""
+    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack():
+        return False
+    try:
+        return all(t.data_ptr() or t.numel() == 0 for t in tensors)
+    except RuntimeError:
+        return False
+
+
 def _check_packed(packed, m, k, bits):
     require_cuda(packed, "packed trellis", (torch.int16, torch.uint16, torch.int32, torch.uint8))
     if bits not in (2, 3, 4):

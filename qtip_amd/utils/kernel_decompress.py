@@ -36,7 +36,7 @@ def tlut_from_expanded(expanded_lut):
     (inverse of quantlut_sym, lib/codebook/bitshift.py:72-80).  Indices no
     state hashes to cannot occur in a stream and are left at zero."""
     if expanded_lut.is_cuda and expanded_lut.dtype in (torch.float16, torch.float32) \
-            and expanded_lut.shape == (1 << 16, 2):
+            and expanded_lut.shape == (1 << 16, 2) and ops.launchable(expanded_lut):
         return ops.fold_table(expanded_lut)
     rep, neg, seen = _representatives()
     dev = expanded_lut.device

@@ -215,6 +215,8 @@ class _HadamardCastFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad):
         hadK, K, transpose, scale, in_dtype = ctx.args
+        if not ops.launchable(grad):
+            return (_hadU(grad.float().contiguous(), hadK, K, not transpose) * scale).to(in_dtype), None, None, None, None, None
         args = (grad, hadK, K, not transpose, scale, in_dtype)
         # (with create_graph the way back is itself recorded)
         gx = _HadamardCastFn.apply(*args) if torch.is_grad_enabled() else _hadU_cast(*args)
@@ -231,7 +233,7 @@ def _hadU_cast(X, hadK, K, transpose, scale, out_dtype):
 
 def hadU_cast(X, hadK, K, transpose, scale, out_dtype):
     """out_dtype(scale * matmul_hadU_cuda(X)), one launch; differentiable with respect to X."""
-    if X.dtype not in (torch.float16, torch.float32):
+    if X.dtype not in (torch.float16, torch.float32) or not ops.launchable(X):
         return (matmul_hadU_cuda(X, hadK, K, transpose) * scale).to(out_dtype)
     return _HadamardCastFn.apply(X, hadK, K, transpose, scale, out_dtype)
 
@@ -247,7 +249,7 @@ class _ScaleColumnsFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad):
         x, s = ctx.saved_tensors
-        if torch.is_grad_enabled() or grad.numel() == 0:
+        if torch.is_grad_enabled() or grad.numel() == 0 or not ops.launchable(grad, x, s):
             return grad * s, (grad * x).sum(0).to(s.dtype)
         gx, gs = ops.scale_columns_grad(*(ops.aligned16(t.contiguous()) for t in (grad, x, s)))
         return gx, gs.to(s.dtype)
@@ -257,7 +259,7 @@ def scale_columns(x, s):
     """x * s for x (rows, n) and s (n,)."""
     if (x.requires_grad and s.requires_grad and x.is_cuda and s.device == x.device and x.dim() == 2
             and x.dtype == torch.float32 and s.dtype in (torch.float16, torch.float32) and s.shape == x.shape[1:]
-            and x.shape[1] % 4 == 0):
+            and x.shape[1] % 4 == 0 and ops.launchable(x, s)):
         return _ScaleColumnsFn.apply(x, s)
     return x * s
 

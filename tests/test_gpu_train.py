@@ -124,3 +124,65 @@ def test_second_derivatives_pass_through_the_fused_steps():
     plain = grads(lambda x, s: (x * s) @ M.T * 0.25)
     for a, b in zip(fused, plain):
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-4 * float(b.abs().max()))
+
+
+def _module(m, k, kernel):
+    from qtip_amd.codebook.bitshift import BitshiftLinear
+    from qtip_amd.utils import matmul_had as mh
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    mod = BitshiftLinear(16, 16, 16, 2, 2, 9, "quantlut_sym", tlut=rand(512, 2).half(), has_kernel=kernel)
+    tr = torch.randint(-32768, 32768, (m // 16 * k // 16, 32), dtype=torch.int16, generator=g, device="cuda")
+    if not kernel:
+        tr = mod.cb.unpack_trellis(tr, 256)
+    (hl, kl), (hr, kr) = mh.get_hadK(k), mh.get_hadK(m)
+    call = lambda *a: mod(a[0], tr, a[1], a[2], hl, hr, kl, kr, 0, 8, mode="train-recons")
+    return call, [rand(20, k), rand(k).sign(), rand(m) / k**0.5], rand(3, 20, m)
+
+
+def _gradients(call, leaves, gy, **kw):
+    leaves = [t.detach().clone().requires_grad_() for t in leaves]
+    return torch.autograd.grad(call(*leaves), leaves, gy, **kw)
+
+
+def _close(a, b):  # (the same roundings to fp16 along either route, sums of a few hundred in another order)
+    a, b = ([t.detach().double() for t in l] for l in (a, b))
+    return all(float((p - q).norm() / q.norm()) <= 2.0**-10 for p, q in zip(a, b))
+
+
+@pytest.mark.parametrize("kernel", [True, False])
+def test_batched_gradients(kernel):
+    """A batch of output gradients in one call is the calls one by one: nothing is launched on what has no memory."""
+    call, leaves, gy = _module(256, 512, kernel)
+    got = _gradients(call, leaves, gy, is_grads_batched=True)
+    each = [_gradients(call, leaves, g) for g in gy]
+    assert _close(got, [torch.stack(t) for t in zip(*each)])
+
+
+def test_traced_and_fake_training_step():
+    """The step of a module without a kernel can be traced, compiled and run on fake tensors, as it consists of torch's and
+    registered operations then."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    call, leaves, gy = _module(256, 512, False)
+    want = _gradients(call, leaves, gy[0])
+    for backend in ("eager", "aot_eager"):
+        torch._dynamo.reset()
+        assert _close(_gradients(torch.compile(call, backend=backend), leaves, gy[0]), want)
+    torch._dynamo.reset()
+    graph = make_fx(call)(*[t.clone().requires_grad_() for t in leaves])
+    assert sum("hadamard" in str(n.target) for n in graph.graph.nodes) == 2
+    other = [t * 1.5 for t in leaves]
+    assert _close([graph(*other)], [call(*other)])
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        fake = [mode.from_tensor(t.detach().clone().requires_grad_()) for t in leaves]
+        grads = torch.autograd.grad(call(*fake), fake, mode.from_tensor(gy[0]))
+    assert [g.shape for g in grads] == [t.shape for t in leaves]
+
+
+def test_step_over_a_batch_of_inputs():
+    call, leaves, _ = _module(256, 512, False)
+    x = torch.stack([leaves[0], 2 * leaves[0]])
+    su = leaves[1].clone().requires_grad_()
+    y = torch.func.vmap(lambda t: call(t, su, leaves[2]))(x)
+    assert _close([y], [torch.stack([call(t, su, leaves[2]) for t in x])])
