@@ -70,15 +70,21 @@ def aligned16(t):
     return t if t is None or t.data_ptr() % 16 == 0 else t.clone()
 
 
+_is_compiling, _modes = torch.compiler.is_compiling, torch._C._len_torch_dispatch_stack
+
+
 def launchable(*tensors):
     """The tensors are memory that a launch can be given: nothing traces the program, and none of them is a wrapper
     (batched gradients, fake tensors).  What passes by torch's own or registered operations asks this first."""
-    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack():
+    if _is_compiling() or _modes():
         return False
     try:
-        return all(t.data_ptr() or t.numel() == 0 for t in tensors)
+        for t in tensors:
+            if not t.data_ptr() and t.numel():
+                return False
     except RuntimeError:
         return False
+    return True
 
 
 def _check_packed(packed, m, k, bits):
