@@ -176,12 +176,22 @@ class bitshift_codebook(nn.Module):
     viterbi = update = quantize_seq = quantize
 
 
+# Rows up to which a product decodes the matrix as it multiplies (gemm_rows_kernel): once per 64 to 128 rows, where the
+# dense route writes and reads 2 m n bytes once and then multiplies at the library's rate.  us at 2000 rows, dense / fused:
+# 4096x4096 73/66, 12288x4096 197/184, 22016x4096 446/317, 4096x11008 190/156, 28672x8192 805/770, 512x2048 20/15, 1728x832
+# 22/15; at 3000 rows 92/96, 270/279, 528/507, 221/231, 8192x8192 337/339, 2048x2048 38/34.  Matrices of few columns
+# end a unit after few steps: 11008x2048 83/66 at 1400 rows, 102/102 at 2000 (whole calls 147/150), so their line is
+# at 2^24 results.
+_FUSED_ROWS_MAX = 2048
+_DENSE_ROWS_MIN = 193
+
+
 class BitshiftLinear(nn.Module):
 
     max_rows = 65535  # rows per launch of the transform / GEMM kernels (grid limit)
-    # from this many rows on the dense decode + library GEMM is taken instead of the fused
-    # decompress-GEMM, for matrices of ordinary size (dense_rows_from)
-    dense_rows_min = 193
+    # A caller's own value asks for the dense decode + library GEMM instead of the fused decompress-GEMM from this many
+    # rows on, for matrices of ordinary size (dense_rows_from); as it stands, takes_dense decides.
+    dense_rows_min = _DENSE_ROWS_MIN
 
     def __init__(self, td_x, td_y, L, K, V, tlut_bits, decode_mode, dtype=torch.float16, tlut=None,
                  has_kernel=False):
@@ -272,10 +282,10 @@ class BitshiftLinear(nn.Module):
                                  rcp, tp_rank, mode=mode, **kwargs) for i in range(0, bs, self.max_rows)]
             return torch.cat(outs, dim=0).view(*input.shape[:-1], m)
 
-        if (self.has_kernel and rcp not in (1, 2) and bs < self.dense_rows_from(m, n) and SU.dtype == torch.float16
+        if (self.has_kernel and rcp not in (1, 2) and not self.takes_dense(bs, m, n) and SU.dtype == torch.float16
                 and SV.dtype == torch.float32 and SV.device == dev and x.dtype in (torch.float16, torch.float32)):
             # both transforms and the product by one call of the library: what bounds such a call otherwise is the
-            # host.  (From dense_rows_from rows on the product is the BLAS library's.)  us per call, launch by launch /
+            # host.  (Where takes_dense holds the product is the BLAS library's.)  us per call, launch by launch /
             # here: 4096x4096, 2 bits, one row 40 / 27; 28672x8192, 4 bits, 16 rows 59 / 44; 4096x11008, 3 bits, 45
             # rows 65 / 35
             return ops.linear(x.contiguous(), trellis.contiguous(), self._tlut16(dev), SU.contiguous(), SV.contiguous(),
@@ -357,22 +367,8 @@ class BitshiftLinear(nn.Module):
 
     @staticmethod
     def _dense_rows_from(m, n, rows_min):
-        """The row count from which an (m, n) matrix is decoded to dense fp16 for a library product: rows_min, and
-        4/3, 5/3 or 8/3 of it (257, 321, 514) for larger matrices.  The fused kernel decodes the matrix once per
-        128 rows, the dense route writes and reads 2 m n bytes once, and the library's product takes long where a
-        large n meets few output tiles and, with some widths, at multiples of 32 rows.  us of the products at 2 / 3 / 4
-        bits, in a graph, dense / fused:
-          4096x4096    129 rows 36/41 35/42 35/40; 176 rows 35/47 35/48 34/47; 192 rows 46/48 45/49 45/48;
-                       193 rows 35/56 34/58 34/55
-          22016x4096   193 rows 100/103 98/119 101/104; 256 rows 106/107 103/124 102/110
-          8192x8192    256 rows 105/89 105/96 107/89; 257 rows 94/100 95/109 96/101
-          5120x13824   256 rows 150/99 151/114 152/100; 257 rows 104/115 106/131 105/115
-          28672x8192   320 rows 257/227 270/266 267/237; 321 rows 269/258 274/311 277/269; 385 rows 294/290 304/345 309/305
-          8192x28672   320 rows 344/215 343/247 345/226; 512 rows 427/331 429/391 433/355; 513 rows 366/356 370/418 375/380
-        A call that is not recorded waits for the host on small matrices, and the dense route's launches cost it twice
-        what `ops.linear` does: whole calls, dense / fused, 2048x2048 129 rows 74/39 and 192 rows 72/42 (the products alone
-        19/31 and 19/35), 4096x4096 129 rows 73/48 and 192 rows 74/57.  So the line stays there at the rows from which the
-        second pass runs the kernel of more than 64."""
+        """rows_min for an (m, n) matrix of ordinary size, and 4/3, 5/3 or 8/3 of it for larger ones, which the
+        dense route writes and reads in full: where a caller that sets dense_rows_min = rows_min wants that route."""
         if n < 5120 or m * n < 1 << 26:
             return rows_min
         if n < 8192 or m * n < 1 << 27:
@@ -382,11 +378,21 @@ class BitshiftLinear(nn.Module):
     def dense_rows_from(self, m, n):
         return self._dense_rows_from(m, n, self.dense_rows_min)
 
+    @classmethod
+    def _takes_dense(cls, rows, m, n, rows_min):
+        if rows_min != _DENSE_ROWS_MIN:
+            return rows >= cls._dense_rows_from(m, n, rows_min)
+        return rows > _FUSED_ROWS_MAX or (n < 4096 and rows * m > 1 << 24)
+
+    def takes_dense(self, rows, m, n):
+        """The product of `rows` rows decodes an (m, n) matrix to dense fp16 and hands it to the BLAS library."""
+        return self._takes_dense(rows, m, n, self.dense_rows_min)
+
     def rows_product(self, xt, trellis, tlut, m, n):
         """(rows, m) fp16 = xt (rows, n) fp16 @ decode(trellis)^T, for two rows or more."""
-        if xt.shape[0] < self.dense_rows_from(m, n):
+        if not self.takes_dense(xt.shape[0], m, n):
             return ops.decompress_gemm(trellis.reshape(-1), xt, tlut, m, n, self.cb.K, out_dtype=torch.float16)
-        # many rows: decode once to dense fp16 and let the BLAS library multiply, which is what the reference does
+        # decode once to dense fp16 and let the BLAS library multiply, which is what the reference does
         # for every batch (bitshift.py:476-489); fp16, which the output transform takes as it is
         return xt @ ops.decode(trellis.reshape(-1), tlut.reshape(-1), m, n, self.cb.K).T
 
@@ -430,7 +436,7 @@ class BitshiftLinearKernelAG(torch.autograd.Function):
         if x.shape[0] == 1:
             y = ops.decompress_matvec(trellis.reshape(-1), x.reshape(-1), tlut.reshape(-1), m, n, K).view(1, m)
             y = y.to(torch.float16)
-        elif x.shape[0] < BitshiftLinear._dense_rows_from(m, n, BitshiftLinear.dense_rows_min):
+        elif not BitshiftLinear._takes_dense(x.shape[0], m, n, BitshiftLinear.dense_rows_min):
             y = ops.decompress_gemm(trellis.reshape(-1), x, tlut.reshape(-1), m, n, K, out_dtype=torch.float16)
         else:
             y = x @ ops.decode(trellis.reshape(-1), tlut.reshape(-1), m, n, K).T

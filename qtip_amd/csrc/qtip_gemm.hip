@@ -10,10 +10,9 @@ using namespace qtip;
 
 namespace {
 
-constexpr int kWaves = 16, kThreads = 64 * kWaves;
-constexpr int kMaxSplit = 16;
+constexpr int kWaves = 16, kThreads = 64 * kWaves;  // of gemm_kernel
 
-// Batched decompress + fp16 MFMA GEMM: out[b][row] = sum_col x[b][col] * W[row][col].
+// Batched decompress + fp16 MFMA GEMM: out[b][row] = sum_col x[b][col] * W[row][col], up to 16 batch rows.
 //
 // A wave works on a pair of 32-row blocks (64 rows) and 64 columns at a time: two 2x2 tile blocks of
 // either row block, 512*K bytes.  Lane bits: 0..2 row r8, 3 row block of the pair, 4 column half c,
@@ -27,41 +26,31 @@ constexpr int kMaxSplit = 16;
 // and twice the accumulators.)  The successor chunk a lane's last reference lane needs sits 16 lanes
 // away or one row on: ds_bpermute.
 //
-// A workgroup of WAVES waves: RG row-block pairs x KS = WAVES / RG column slices of 64.  The activations of
-// a stage (16*NB batch rows x 64*KS columns) are shared through LDS, each 16-byte chunk holding the
-// eight values one lane's A operand needs, chunk index xor-ed with the row (conflict-free both ways).
-// The next tile waits in registers; with room for two tiles in LDS there is one barrier per stage,
-// else two.  Work unit = (group of RG pairs, k range s); a workgroup keeps one s, so the pipeline runs
+// A workgroup of 16 waves: two row-block pairs x KS = 8 column slices of 64.  The activations of a stage (16
+// batch rows x 512 columns) are shared through LDS, each 16-byte chunk holding the eight values one lane's A operand
+// needs, chunk index xor-ed with the row (conflict-free both ways).  The next tile waits in registers; two tiles in
+// LDS, one barrier per stage.  Work unit = (two pairs, k range s); a workgroup keeps one s, so the pipeline runs
 // across unit boundaries.  The k slices of a unit meet in the tile buffer at its end.
 // S > 1 (few row blocks): fp32 partial results go to parts[s][batch][m] and are summed afterwards.
-//
-// Up to 32 batch rows on 16 waves of 128 registers (NB = 1, 2; RG = 2), 33-64 on 8 waves of 256
-// (NB = 4, RG = 2: 64 accumulators and the words of a half block do not fit 128), 65-128 on 8 waves
-// (NB = 8, RG = 4: a 32 KiB tile of 128 columns).  What bounds it: at up to 16 rows the decode, as in
-// the matvec; beyond, the sum of the stage's phases - decode, LDS reads, products, tile - because the
-// waves of a workgroup pass a stage's barriers together: each phase left out alone takes 4-13 us off
-// the 52 us of 64 rows.  us per launch, 28672x8192 at 2 / 4 bits, batch 16 / 32 / 64 / 128 (the
-// lane map with doubled products in passes of 32 rows, a row-split one at 4 bits, before):
-// 28 / 35 / 53 / 90 and 30 / 37 / 53 / 100 (33 / 50 / 94 / 183 and 33 / 39 / 75 / 143).
+// Bound by the decode, as the matvec: 28672x8192 at 2 / 4 bits 28 / 30 us.
 constexpr size_t kGemmTileBytes = 32 * 1024;
 constexpr size_t kGemmLds = kLut128Bytes + kGemmTileBytes;
 
-template <int K, int NB, int WAVES, int RG, typename TOut>
-__global__ __launch_bounds__(WAVES * 64, 1) void gemm_kernel(
+template <int K, typename TOut>
+__global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
     TOut* __restrict__ dst, const uint8_t* __restrict__ packed, const uint16_t* __restrict__ x,
-    const uint32_t* __restrict__ tlut, int m, int k, int batch, int round_f16, int wl_per, int upw_q, int upw_r) {
-  constexpr int THREADS = WAVES * 64, DEPTH = 2;
+    const uint32_t* __restrict__ tlut, int m, int k, int batch, long ldo, int round_f16, int wl_per, int upw_q, int upw_r) {
+  constexpr int NB = 1, WAVES = kWaves, RG = 2, THREADS = kThreads, DEPTH = 2;
   constexpr int KS = WAVES / RG;
   constexpr int ROWB = KS * 128;               // bytes per tile row
   constexpr int CPR = ROWB / 16;               // 16-byte chunks per tile row
   constexpr uint32_t TILE = 16 * NB * ROWB;
-  constexpr bool DB = 2 * TILE <= kGemmTileBytes && TILE >= WAVES * 1024;
   constexpr int CHUNKS = 16 * NB * CPR;
   constexpr int NX = (CHUNKS + THREADS - 1) / THREADS;  // chunks per thread
-  static_assert(TILE <= kGemmTileBytes, "tile does not fit");
+  static_assert(2 * TILE <= kGemmTileBytes, "two tiles do not fit");
   extern __shared__ __align__(16) uint8_t smem[];
   uint32_t* lut = reinterpret_cast<uint32_t*>(smem);
-  uint8_t* tile = smem + kLut128Bytes;  // [1 or 2][16*NB rows][ROWB bytes]
+  uint8_t* tile = smem + kLut128Bytes;  // [2][16 rows][ROWB bytes]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rg = wave % RG, ks = wave / RG;
@@ -87,7 +76,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void gemm_kernel(
   const int nst = wl1 > wl0 ? (wl1 - wl0 + KS - 1) / KS : 0;  // stages per unit
   const int upw = upw_q + (u0 < upw_r ? 1 : 0);
   const int T = upw * nst;
-  TOut* out_s = dst + (size_t)s * batch * m;
+  TOut* out_s = dst + (size_t)s * batch * ldo;
 
   // ---- weight stream of this wave, DEPTH stages in flight
   int l_t = 0, l_q = 0, l_u = u0;
@@ -179,7 +168,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void gemm_kernel(
     for (int d = 0; d < DEPTH; ++d) {
       // (an odd last stage: nothing to multiply, but its loads and barriers stay unconditional - see load_tile)
       const bool live = q + d < T;  // uniform over the workgroup
-      const uint32_t cb = DB ? (uint32_t)(d & 1) * TILE : 0u;  // this stage's tile
+      const uint32_t cb = (uint32_t)(d & 1) * TILE;  // this stage's tile
       if (live) {
         const int pair = c_u * RG + rg;
         const int wl = wl0 + KS * c_t + ks;
@@ -225,19 +214,17 @@ __global__ __launch_bounds__(WAVES * 64, 1) void gemm_kernel(
         int t2 = c_t + 2;  // the tile that replaces the next one in its registers
         if (t2 >= nst) t2 -= nst;
         if (t2 >= nst) t2 -= nst;  // nst == 1
-        if constexpr (DB) {
-          // the next tile (in registers since the previous stage) into the other buffer, the one after it on its way
-          store_tile((uint32_t)((d + 1) & 1) * TILE);
-          load_tile(t2);
-          issue(d);
-        }
-        __syncthreads();  // every wave has read this stage's tile (and, with two buffers, written the next)
+        // the next tile (in registers since the previous stage) into the other buffer, the one after it on its way
+        store_tile((uint32_t)((d + 1) & 1) * TILE);
+        load_tile(t2);
+        issue(d);
+        __syncthreads();  // every wave has read this stage's tile and written the next
         const bool unit_end = live && c_t + 1 == nst;
         if (unit_end) {
           // ---- end of a unit: the k slices meet in this stage's tile buffer, TI accumulator vectors of every
           // wave at a time, summed in slice order
-          constexpr int TI = DB ? TILE / (WAVES * 1024) : kGemmTileBytes / (WAVES * 1024);  // vectors that fit
-          static_assert(WAVES * TI * 1024 <= (DB ? TILE : kGemmTileBytes), "the exchange does not fit");
+          constexpr int TI = TILE / (WAVES * 1024);  // vectors that fit
+          static_assert(WAVES * TI * 1024 <= TILE, "the exchange does not fit");
           float* xch = reinterpret_cast<float*>(tile + cb);
           const float4_t* av = &acc[0][0][0];
 #pragma unroll
@@ -263,7 +250,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void gemm_kernel(
                 if constexpr (sizeof(TOut) == 4) {
                   if (round_f16) sum = (float)(_Float16)sum;
                 }
-                if (bb < batch && row < m) out_s[(size_t)bb * m + row] = (TOut)sum;
+                if (bb < batch && row < m) out_s[(size_t)bb * ldo + row] = (TOut)sum;
               }
             }
             __syncthreads();
@@ -273,58 +260,188 @@ __global__ __launch_bounds__(WAVES * 64, 1) void gemm_kernel(
           c_u += ustep;
         }
         c_t = unit_end ? 0 : c_t + (live ? 1 : 0);
-        if constexpr (!DB) {
-          store_tile(0);
-          load_tile(t2);
-          issue(d);
-          __syncthreads();  // the next tile is complete
-        }
       }
     }
   }
 }
 
-// out[i] = parts[0][i] + ... (+ rounding through fp16) for the split-k GEMM
+#include "qtip_gemm_rows.h"
+
+// out[row][i] = parts[0][row][i] + ... (+ rounding through fp16) for products cut along k, four at a time: mq = m / 4,
+// parts[s] dense, rows of out ldo apart
 template <typename TOut>
-__global__ __launch_bounds__(256) void sum_parts_round_kernel(TOut* __restrict__ out,
-                                                              const float* __restrict__ parts, long n,
-                                                              int S, int round_f16) {
+__global__ __launch_bounds__(256) void sum_parts_round_kernel(TOut* __restrict__ out, const float4_t* __restrict__ parts,
+                                                              long n, int mq, long ldo, int S, int round_f16) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  float sum = parts[i];
+  float4_t sum = parts[i];
   for (int s = 1; s < S; ++s) sum += parts[(size_t)s * n + i];
-  out[i] = (TOut)(round_f16 ? (float)(_Float16)sum : sum);
+  typedef TOut out4_t __attribute__((ext_vector_type(4), aligned(sizeof(TOut))));  // (out may start anywhere)
+  out4_t r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = (TOut)(round_f16 ? (float)(_Float16)sum[e] : sum[e]);
+  *reinterpret_cast<out4_t*>(out + (i / mq) * ldo + 4 * (i % mq)) = r;
 }
 
-// How a pass of nb <= kGemmRows batch rows runs: NB 16-row batch tiles, RG row-block pairs per workgroup,
-// S k ranges of wl_per 64-column wave-loads.  Few pairs are cut along k as well (only when the caller
-// provides room for the partial results).
-constexpr int kGemmRows = 128;
-// ... and fewer where that many activations pass what a buffer's 32-bit offsets reach (2 GiB less the offset that
-// stands for padding): from k = 2^23 on
-int pass_rows(int k) {
-  const long fit = 0x7FFFFF00L / (2L * k);
-  return fit < kGemmRows ? (int)fit : kGemmRows;
-}
+// How nb batch rows of an m-row matrix run in one launch: NB 16-row batch tiles, RG row-block pairs per workgroup,
+// S k ranges of wl_per 64-column wave-loads (S > 1 only when the caller provides room for the partial results).
 struct GemmPlan {
-  int NB, waves, RG, S, wl_per, ngroups;
+  int NB, RG, S, wl_per, nbt, ngroups;
+  float us;  // what it is expected to take
 };
-GemmPlan gemm_plan(int m, int k, int nb, int cus, bool split) {
-  GemmPlan g;
-  g.NB = nb <= 16 ? 1 : (nb <= 32 ? 2 : (nb <= 64 ? 4 : 8));
-  g.waves = nb <= 32 ? 16 : 8;
-  g.RG = nb <= 64 ? 2 : 4;
-  const int KS = g.waves / g.RG;
-  g.ngroups = (((m >> 5) + 1) / 2 + g.RG - 1) / g.RG;
+constexpr int kMaxSplit = 16;
+
+GemmPlan gemm_split(int m, int k, int nb, int NB, int RG, int KS, int S) {
+  GemmPlan g{};
+  g.NB = NB;
+  g.RG = RG;
+  g.nbt = (nb + 16 * NB - 1) / (16 * NB);
+  g.ngroups = (((m >> 5) + 1) / 2 + RG - 1) / RG;
   const int nwl = ((k >> 5) + 1) >> 1;
-  // columns a range keeps: 1024 up to 32 rows, 512 beyond (4096x4096 at 2 bits, 512 / 1024 / 2048 columns: 11.3 /
-  // 10.4 / 12.0 us for 16 rows, 17.1 / 16.6 / 20.3 for 64, 31 / 34 / 46 for 128)
-  const int min_wl = nb <= 32 ? 16 : 8;
-  int S = 1;
-  while (split && S < kMaxSplit && g.ngroups * S * 2 <= cus && nwl / (S * 2) >= min_wl) S *= 2;
   g.wl_per = ((nwl + S - 1) / S + KS - 1) / KS * KS;  // stages are groups of KS wave-loads
   g.S = (nwl + g.wl_per - 1) / g.wl_per;              // rounding up may have emptied the last ranges
   return g;
+}
+
+// up to 16 rows: gemm_kernel
+GemmPlan gemm_plan16(int m, int k, int nb, int cus, bool split) {
+  const int nwl = ((k >> 5) + 1) >> 1, ngroups = (((m >> 5) + 1) / 2 + 1) / 2;
+  int S = 1;
+  // columns a range keeps: 1024 (4096x4096 at 2 bits, 512 / 1024 / 2048 columns: 11.3 / 10.4 / 12.0 us)
+  while (split && S < kMaxSplit && ngroups * S * 2 <= cus && nwl / (S * 2) >= 16) S *= 2;
+  return gemm_split(m, k, nb, 1, 2, 8, S);
+}
+
+// What a launch of gemm_rows_kernel (and the one that adds its k ranges) takes, in us.  The terms are fitted to 4000
+// measured launches (2 and 4 bits, 17 to 2000 rows, matrices of 512x2048 to 28672x8192): 5 % root mean square, and the
+// form with the least of it takes 0.4 % longer than the best one on average.  A fixed part, per unit its
+// stores, per wave-load the step, faster where part of the chip idles (the clock), slower where a stage is half
+// a wave-load or its pieces of activations do not come out even; for k ranges the partial results and their launch.
+float rows_time(const GemmPlan& g, int m, int nb, int cus) {
+  const int KS = kRowsWaves / g.RG, NB = g.NB;
+  const long units = (long)g.ngroups * g.nbt, per = cus / g.S < units ? cus / g.S : units;
+  const float form = NB == 6 ? 1.06f : rows_stage_halves(NB, g.RG) == 2 ? 1.f : NB == 4 ? 1.24f : 1.057f;
+  const float steps = (float)(g.wl_per / KS) * (0.64f + 0.099f * NB) * form, store = 0.19f + 0.724f * NB;
+  auto round = [&](long n) { return steps * (0.8f + 0.2f * (float)(n * g.S) / cus) + store; };
+  float us = 5.2f + (float)(units / per) * round(per);
+  if (units % per) us += round(units % per);
+  if (g.S > 1) us += 1.07f + 0.265f * g.S + (float)nb * m * (1.26e-6f * g.S + 0.77e-6f);
+  return us;
+}
+
+// From 17 rows on: the form with the least expected time.
+GemmPlan rows_plan(int m, int k, int nb, int cus, bool split) {
+  static const int kForms[][2] = {{8, 8}, {8, 4}, {6, 8}, {4, 8}, {4, 4}, {4, 2}, {2, 4}, {2, 2}};
+  const int nwl = ((k >> 5) + 1) >> 1;
+  GemmPlan best{};
+  for (const auto& f : kForms) {
+    for (int S = 1; S <= (split ? kMaxSplit : 1) && (S == 1 || nwl / S >= 4); S *= 2) {
+      GemmPlan g = gemm_split(m, k, nb, f[0], f[1], kRowsWaves / f[1], S);
+      if (S > 1 && (g.S == 1 || (long)g.ngroups * g.nbt * S > cus + cus / 8)) break;
+      g.us = rows_time(g, m, nb, cus);
+      if (best.NB == 0 || g.us < best.us) best = g;
+    }
+  }
+  return best;
+}
+
+// A product in up to two launches over the matrix rows: [0, m0) and [m0, m).
+struct GemmParts {
+  int m0;
+  GemmPlan first, rest;
+};
+
+GemmParts make_plan(int m, int k, int nb, int cus, bool split) {
+  GemmParts p{m, {}, {}};
+  if (nb <= 16) {
+    p.first = gemm_plan16(m, k, nb, cus, split);
+    return p;
+  }
+  p.first = rows_plan(m, k, nb, cus, split);
+  // Units beyond whole rounds of the chip as a launch of their own, in the form that suits what is left: 22016x4096,
+  // 700 rows (258 units of 512 matrix by 128 batch rows on 256 CUs) 144 -> 129 us, 12288x4096, 1400 rows 172 -> 136.
+  // Where it should give a twelfth at least: at 0.97 22016x4096 lost 4 % at 1000 to 2000 rows (the clock makes up for
+  // part of an idle chip).  Tried where the gain covers the host's search.
+  if (p.first.us < 40.f) return p;
+  float least = 0.92f * p.first.us;
+  for (int NB = 8; NB >= 4; NB -= 2) {
+    const int per = cus / ((nb + 16 * NB - 1) / (16 * NB));  // groups a round
+    for (int rounds = 1; per && rounds <= 3; ++rounds) {
+      const long m0 = (long)per * rounds * kRowsWaves * 64;
+      if (m0 >= m) break;
+      GemmPlan a = gemm_split((int)m0, k, nb, NB, kRowsWaves, 1, 1);
+      a.us = rows_time(a, (int)m0, nb, cus);
+      if (a.us >= least) break;
+      const GemmPlan b = rows_plan(m - (int)m0, k, nb, cus, split);
+      if (a.us + b.us < least) {
+        least = a.us + b.us;
+        p = {(int)m0, a, b};
+      }
+    }
+  }
+  return p;
+}
+
+// The plan of a call is asked for by its size queries and by its launches; a search takes 1 to 15 us, so each thread
+// keeps those of the last sizes.
+GemmParts gemm_plan(int m, int k, int nb, int cus, bool split) {
+  struct Held {
+    int m, k, nb, cus;  // (of split plans; the others come from callers without scratch)
+    GemmParts plan;
+  };
+  static thread_local Held held[64];
+  if (!split) return make_plan(m, k, nb, cus, false);
+  Held& h = held[((uint32_t)m * 0x9E3779B1u ^ (uint32_t)k * 0x85EBCA77u ^ (uint32_t)nb * 0xC2B2AE3Du) >> 26];
+  if (h.m != m || h.k != k || h.nb != nb || h.cus != cus) h = {m, k, nb, cus, make_plan(m, k, nb, cus, true)};
+  return h.plan;
+}
+
+// Rows of one pass: as many as 32-bit buffer offsets reach (2 GiB less the offset that stands for padding)
+int pass_rows(int k) {
+  const long fit = 0x7FFFFF00L / (2L * k);
+  return fit >= 65536 ? 65536 : fit >= 128 ? (int)(fit & ~127L) : (int)fit;
+}
+
+size_t parts_bytes(const GemmPlan& g, int m, int nb) { return g.S > 1 ? (size_t)g.S * nb * m * sizeof(float) : 0; }
+
+template <int K, typename T>
+void launch_gemm(const GemmPlan& g, T* dst, long ldo, const uint8_t* p, const uint16_t* x, const uint32_t* t, int m, int k,
+                 int nb, int round_f16, int cus, hipStream_t st) {
+  const long units = (long)g.ngroups * g.nbt;
+  const int per = (int)(cus / g.S < units ? cus / g.S : units);  // workgroups per k range
+  const dim3 grid((unsigned)g.S, (unsigned)per);
+  const int uq = (int)(units / per), ur = (int)(units % per);
+  if (nb <= 16) {
+    gemm_kernel<K, T><<<grid, kThreads, kGemmLds, st>>>(dst, p, x, t, m, k, nb, ldo, round_f16, g.wl_per, uq, ur);
+    return;
+  }
+#define QTIP_ROWS(NBV, RGV)                                                                                       \
+  gemm_rows_kernel<K, NBV, RGV, T><<<grid, 64 * kRowsWaves, kGemmLds, st>>>(dst, p, x, t, m, k, nb, g.nbt, ldo,   \
+                                                                            round_f16, g.wl_per, uq, ur)
+  if (g.NB == 8) {
+    if (g.RG == 8) QTIP_ROWS(8, 8);
+    else QTIP_ROWS(8, 4);
+  } else if (g.NB == 6) {
+    QTIP_ROWS(6, 8);
+  } else if (g.NB == 4) {
+    if (g.RG == 8) QTIP_ROWS(4, 8);
+    else if (g.RG == 4) QTIP_ROWS(4, 4);
+    else QTIP_ROWS(4, 2);
+  } else {
+    if (g.RG == 4) QTIP_ROWS(2, 4);
+    else QTIP_ROWS(2, 2);
+  }
+#undef QTIP_ROWS
+}
+
+template <typename T>
+void launch_gemm(int bits, const GemmPlan& g, T* dst, long ldo, const uint8_t* p, const uint16_t* x, const uint32_t* t,
+                 int m, int k, int nb, int round_f16, int cus, hipStream_t st) {
+  switch (bits) {
+    case 2: return launch_gemm<2, T>(g, dst, ldo, p, x, t, m, k, nb, round_f16, cus, st);
+    case 3: return launch_gemm<3, T>(g, dst, ldo, p, x, t, m, k, nb, round_f16, cus, st);
+    default: return launch_gemm<4, T>(g, dst, ldo, p, x, t, m, k, nb, round_f16, cus, st);
+  }
 }
 
 template <typename TOut>
@@ -344,50 +461,29 @@ int run_gemm(TOut* out, const void* packed, const void* x_f16, const void* tlut,
     if (!aligned16(workspace)) return QTIP_E_ALIGN;
   }
   hipStream_t st = (hipStream_t)stream;
-  auto* p = (const uint8_t*)packed;
   auto* t = (const uint32_t*)tlut;
   const int step = pass_rows(k);
   for (int b0 = 0; b0 < batch; b0 += step) {
     const int nb = batch - b0 < step ? batch - b0 : step;
-    const GemmPlan g = gemm_plan(m, k, nb, cus, workspace != nullptr);
-    const long units = (long)g.ngroups * g.S;
-    long grid = units < cus ? units : cus;
-    grid -= grid % g.S;  // a workgroup keeps one k range
-    const int per_range = (int)(grid / g.S);
-    const dim3 g2((unsigned)g.S, (unsigned)per_range);
-    const int uq = g.ngroups / per_range, ur = g.ngroups % per_range;
+    const GemmParts parts = gemm_plan(m, k, nb, cus, workspace != nullptr);
     const uint16_t* xx = (const uint16_t*)x_f16 + (size_t)b0 * k;
-    TOut* o = out + (size_t)b0 * m;
-#define QTIP_GEMM_L(KB, NBT, WV, RGT, T, D, RND) \
-  gemm_kernel<KB, NBT, WV, RGT, T><<<g2, WV * 64, kGemmLds, st>>>(D, p, xx, t, m, k, nb, RND, g.wl_per, uq, ur)
-#define QTIP_GEMM_NB(KB, T, D, RND)                       \
-  switch (g.NB) {                                         \
-    case 1: QTIP_GEMM_L(KB, 1, 16, 2, T, D, RND); break; \
-    case 2: QTIP_GEMM_L(KB, 2, 16, 2, T, D, RND); break; \
-    case 4: QTIP_GEMM_L(KB, 4, 8, 2, T, D, RND); break;  \
-    default: QTIP_GEMM_L(KB, 8, 8, 4, T, D, RND); break; \
-  }
-#define QTIP_GEMM(T, D, RND)                      \
-  switch (bits) {                                 \
-    case 2: QTIP_GEMM_NB(2, T, D, RND) break;     \
-    case 3: QTIP_GEMM_NB(3, T, D, RND) break;     \
-    default: QTIP_GEMM_NB(4, T, D, RND) break;    \
-  }
-    if (g.S > 1) {
-      QTIP_GEMM(float, (float*)workspace, 0)
-    } else {
-      QTIP_GEMM(TOut, o, round_f16)
-    }
-#undef QTIP_GEMM
-#undef QTIP_GEMM_NB
-#undef QTIP_GEMM_L
-    hipError_t le = hipGetLastError();
-    if (le != hipSuccess) return (int)le;
-    if (g.S > 1) {
-      const long n = (long)nb * m;
-      sum_parts_round_kernel<TOut><<<(int)((n + 255) / 256), 256, 0, st>>>(o, (const float*)workspace, n, g.S, round_f16);
-      le = hipGetLastError();
+    for (int part = 0; part < 2; ++part) {
+      const int first = part ? parts.m0 : 0, rows = part ? m - parts.m0 : parts.m0;
+      if (!rows) continue;
+      const GemmPlan& g = part ? parts.rest : parts.first;
+      const uint8_t* p = (const uint8_t*)packed + (size_t)first * k * bits / 8;
+      TOut* o = out + (size_t)b0 * m + first;
+      if (g.S > 1) launch_gemm<float>(bits, g, (float*)workspace, rows, p, xx, t, rows, k, nb, 0, cus, st);
+      else launch_gemm<TOut>(bits, g, o, m, p, xx, t, rows, k, nb, round_f16, cus, st);
+      hipError_t le = hipGetLastError();
       if (le != hipSuccess) return (int)le;
+      if (g.S > 1) {
+        const long n = (long)nb * rows / 4;
+        sum_parts_round_kernel<TOut><<<(int)((n + 255) / 256), 256, 0, st>>>(o, (const float4_t*)workspace, n, rows / 4, m,
+                                                                             g.S, round_f16);
+        le = hipGetLastError();
+        if (le != hipSuccess) return (int)le;
+      }
     }
   }
   return QTIP_OK;
@@ -401,11 +497,16 @@ hipError_t qtip_gemm_allow_lds() {
   if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,   \
                                (int)bytes)) != hipSuccess)                                                       \
     return e;
-#define QTIP_ALLOW_GEMM(KB, T)                         \
-  QTIP_ALLOW((gemm_kernel<KB, 1, 16, 2, T>), kGemmLds) \
-  QTIP_ALLOW((gemm_kernel<KB, 2, 16, 2, T>), kGemmLds) \
-  QTIP_ALLOW((gemm_kernel<KB, 4, 8, 2, T>), kGemmLds)  \
-  QTIP_ALLOW((gemm_kernel<KB, 8, 8, 4, T>), kGemmLds)
+#define QTIP_ALLOW_GEMM(KB, T)                        \
+  QTIP_ALLOW((gemm_kernel<KB, T>), kGemmLds)            \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 8, 8, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 8, 4, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 6, 8, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 8, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 4, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 2, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 2, 4, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 2, 2, T>), kGemmLds)
   QTIP_ALLOW_GEMM(2, float)
   QTIP_ALLOW_GEMM(3, float)
   QTIP_ALLOW_GEMM(4, float)
@@ -427,9 +528,9 @@ size_t qtip_gemm_workspace_bytes(int m, int k, int bits, int batch) {
   const int step = pass_rows(k);
   for (int nb : {batch < step ? batch : step, batch % step}) {
     if (nb < 1) continue;
-    const GemmPlan g = gemm_plan(m, k, nb, cus, true);
-    const size_t bytes = g.S > 1 ? (size_t)g.S * nb * m * sizeof(float) : 0;
-    need = bytes > need ? bytes : need;
+    const GemmParts p = gemm_plan(m, k, nb, cus, true);
+    for (size_t bytes : {parts_bytes(p.first, p.m0, nb), p.m0 < m ? parts_bytes(p.rest, m - p.m0, nb) : 0})
+      need = bytes > need ? bytes : need;
   }
   return need;
 }

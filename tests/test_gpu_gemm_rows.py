@@ -53,3 +53,43 @@ def test_activations_beyond_two_gib(k):
         size += a.abs() @ b.abs()
     # fp32 sums in chains of a few thousand products whose errors add like their square roots: 2^-20 of the magnitudes
     assert bool(((y - want).abs() <= 2.0**-20 * size).all())
+
+
+# each form of the kernel of 17 rows and more (batch tiles of 32, 64, 96 and 128 rows by 2, 4 and 8 row-block pairs, cut along k
+# or not, in one launch or two), ranges of k that end inside a stage and inside a 64-column piece
+@pytest.mark.parametrize("m,k,batch,bits", [(64, 32, 17, 2), (544, 96, 40, 3), (96, 160, 150, 4), (512, 2048, 31, 3), (4096, 4096, 45, 4),
+                                            (1056, 2080, 130, 2), (8192, 4096, 61, 3), (12288, 2144, 90, 4), (8192, 1248, 250, 3),
+                                            (5632, 992, 1000, 2), (10240, 1120, 512, 4), (22016, 4096, 700, 3), (16416, 2080, 1030, 2),
+                                            (1728, 832, 2048, 4)])
+def test_forms_of_many_rows(m, k, batch, bits):
+    from qtip_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(m + k + batch)
+    packed = torch.randint(-32768, 32768, (m * k * bits // 16,), dtype=torch.int16, generator=g, device="cuda")
+    tlut = torch.randn(1024, generator=g, device="cuda").half()
+    w = ops.decode(packed, tlut, m, k, bits).double()
+    x = torch.randn(batch, k, generator=g, device="cuda").half()
+    ref, size = x.double() @ w.T, x.double().abs() @ w.abs().T
+    got = ops.decompress_gemm(packed, x, tlut, m, k, bits, round_f16=False)
+    # exact products, fp32 sums of k terms: chains of k / 32 additions, whose errors add like their square roots
+    assert bool(((got.double() - ref).abs() <= 2.0**-21 * size).all())
+    half = ops.decompress_gemm(packed, x, tlut, m, k, bits, out_dtype=torch.float16)
+    assert torch.equal(half, got.half())
+
+
+@pytest.mark.parametrize("m,k,batch", [(64, 32, 40), (128, 96, 20), (2048, 832, 100), (1056, 928, 200)])
+def test_infinite_table_entry_stays_in_its_rows(m, k, batch):
+    """Where k ends inside a stage, what stands in for the missing weights is met by zeros: it must not be a table entry the
+    row does not hold (state 0 selects entry 0)."""
+    from qtip_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(k)
+    packed = torch.randint(-32768, 32768, (m * k * 2 // 16,), dtype=torch.int16, generator=g, device="cuda")
+    tlut = torch.randn(512, 2, generator=g, device="cuda").half()
+    tlut[0] = float("inf")
+    w = ops.decode(packed, tlut.reshape(-1), m, k, 2)
+    finite = w.isfinite().all(1)
+    assert bool(finite.any()) and not bool(finite.all())
+    x = torch.randn(batch, k, generator=g, device="cuda").half()
+    got = ops.decompress_gemm(packed, x, tlut.reshape(-1), m, k, 2, round_f16=False)
+    ref, size = x.double() @ w[finite].double().T, x.double().abs() @ w[finite].double().abs().T
+    assert bool(((got[:, finite].double() - ref).abs() <= 2.0**-21 * size).all())
+    assert not bool(got[:, ~finite].isfinite().any())
