@@ -10,31 +10,33 @@ using namespace qtip;
 
 namespace {
 
-constexpr int kWaves = 16, kThreads = 64 * kWaves;  // of gemm_kernel
-
-// Batched decompress + fp16 MFMA GEMM: out[b][row] = sum_col x[b][col] * W[row][col], up to 16 batch rows.
+// Batched decompress + fp16 MFMA GEMM: out[b][row] = sum_col x[b][col] * W[row][col].
 //
-// A wave works on a pair of 32-row blocks (64 rows) and 64 columns at a time: two 2x2 tile blocks of
+// A wave works on a pair of 32-row blocks (64 rows) and 64 columns at a time, a wave-load: two 2x2 tile blocks of
 // either row block, 512*K bytes.  Lane bits: 0..2 row r8, 3 row block of the pair, 4 column half c,
 // 5 column block; the lane loads the 8*K bytes of reference lanes 4 r8 + 2c and 4 r8 + 2c + 1 of its
 // tile block.  For a given (tile row half mh, row half rh, column half of the block kh) the lane's four
 // table words are eight weights of ONE matrix row, and the sixteen lanes of a DPP row hold the same
-// columns of sixteen different rows, with the four DPP rows holding the four column groups: a
-// v_mfma_f32_16x16x32_f16 B operand (N = lane % 16, K group = lane / 16) in which every product is
+// columns of sixteen different rows, with the four DPP rows holding the four column groups: an operand of
+// v_mfma_f32_16x16x32_f16 (row = lane % 16, K group = lane / 16) in which every product is
 // wanted, straight from the table lookups, at every bit width.  (Lanes that split a row's columns
 // inside a DPP row - the matvec's map - leave half of every product meaningless: twice the products
 // and twice the accumulators.)  The successor chunk a lane's last reference lane needs sits 16 lanes
 // away or one row on: ds_bpermute.
 //
-// A workgroup of 16 waves: two row-block pairs x KS = 8 column slices of 64.  The activations of a stage (16
+// Three kernels: gemm_few_kernel and gemm_kernel up to 16 batch rows, gemm_rows_kernel beyond.  S > 1 (few units of work): k
+// is cut into S ranges, fp32 partial results go to parts[s][batch][m] and are summed afterwards.
+constexpr size_t kGemmTileBytes = 32 * 1024;  // beside the table: tiles of activations, sums of slices
+constexpr size_t kGemmLds = kLut128Bytes + kGemmTileBytes;
+
+// Up to 16 batch rows of the largest matrices at 3 and 4 bits (see shared_rows).  A workgroup of 16 waves: two row-block
+// pairs x KS = 8 column slices of 64.  The activations of a stage (16
 // batch rows x 512 columns) are shared through LDS, each 16-byte chunk holding the eight values one lane's A operand
 // needs, chunk index xor-ed with the row (conflict-free both ways).  The next tile waits in registers; two tiles in
 // LDS, one barrier per stage.  Work unit = (two pairs, k range s); a workgroup keeps one s, so the pipeline runs
 // across unit boundaries.  The k slices of a unit meet in the tile buffer at its end.
-// S > 1 (few row blocks): fp32 partial results go to parts[s][batch][m] and are summed afterwards.
-// Bound by the decode, as the matvec: 28672x8192 at 2 / 4 bits 28 / 30 us.
-constexpr size_t kGemmTileBytes = 32 * 1024;
-constexpr size_t kGemmLds = kLut128Bytes + kGemmTileBytes;
+// Bound by the weight stream (28672x8192 at 4 bits, from cold memory: 28 us, 4.2 TB/s; the matvec 24).
+constexpr int kWaves = 16, kThreads = 64 * kWaves;
 
 template <int K, typename TOut>
 __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
@@ -266,6 +268,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
 }
 
 #include "qtip_gemm_rows.h"
+#include "qtip_gemm_few.h"
 
 // out[row][i] = parts[0][row][i] + ... (+ rounding through fp16) for products cut along k, four at a time: mq = m / 4,
 // parts[s] dense, rows of out ldo apart
@@ -283,11 +286,12 @@ __global__ __launch_bounds__(256) void sum_parts_round_kernel(TOut* __restrict__
   *reinterpret_cast<out4_t*>(out + (i / mq) * ldo + 4 * (i % mq)) = r;
 }
 
-// How nb batch rows of an m-row matrix run in one launch: NB 16-row batch tiles, RG row-block pairs per workgroup,
-// S k ranges of wl_per 64-column wave-loads (S > 1 only when the caller provides room for the partial results).
+// How nb batch rows of an m-row matrix run in one launch: NB 16-row batch tiles of gemm_rows_kernel (0: gemm_few_kernel, 1:
+// gemm_kernel), RG row-block pairs per workgroup, S k ranges of wl_per 64-column wave-loads (S > 1 only when the
+// caller provides room for the partial results).
 struct GemmPlan {
   int NB, RG, S, wl_per, nbt, ngroups;
-  float us;  // what it is expected to take
+  float us;  // what it is expected to take, with the launch that adds the ranges
 };
 constexpr int kMaxSplit = 16;
 
@@ -295,7 +299,7 @@ GemmPlan gemm_split(int m, int k, int nb, int NB, int RG, int KS, int S) {
   GemmPlan g{};
   g.NB = NB;
   g.RG = RG;
-  g.nbt = (nb + 16 * NB - 1) / (16 * NB);
+  g.nbt = NB ? (nb + 16 * NB - 1) / (16 * NB) : 1;
   g.ngroups = (((m >> 5) + 1) / 2 + RG - 1) / RG;
   const int nwl = ((k >> 5) + 1) >> 1;
   g.wl_per = ((nwl + S - 1) / S + KS - 1) / KS * KS;  // stages are groups of KS wave-loads
@@ -303,13 +307,39 @@ GemmPlan gemm_split(int m, int k, int nb, int NB, int RG, int KS, int S) {
   return g;
 }
 
-// up to 16 rows: gemm_kernel
-GemmPlan gemm_plan16(int m, int k, int nb, int cus, bool split) {
-  const int nwl = ((k >> 5) + 1) >> 1, ngroups = (((m >> 5) + 1) / 2 + 1) / 2;
-  int S = 1;
-  // columns a range keeps: 1024 (4096x4096 at 2 bits, 512 / 1024 / 2048 columns: 11.3 / 10.4 / 12.0 us)
-  while (split && S < kMaxSplit && ngroups * S * 2 <= cus && nwl / (S * 2) >= 16) S *= 2;
-  return gemm_split(m, k, nb, 1, 2, 8, S);
+// Up to 16 rows: where the weight stream is the bound and the activations would be in its way, they are shared.  us from cold
+// memory, gemm_kernel / gemm_few_kernel: 28672x8192 at 4 bits 2 rows 27.5/27.7, 6 27.9/27.9, 9 28.5/29.1, 16 28.0/34.2; at
+// 3 bits 2 rows 28.5/27.6, 6 28.3/28.6, 16 27.9/30.0; 22016x4096 at 4 bits 6 rows 15.4/14.7, 9 15.6/15.1, 16 15.9/16.8;
+// 10240x8192 at 4 bits 16 rows 18.2/16.9.
+bool shared_rows(int m, int k, int bits, int nb) {
+  const long n = (long)m * k;
+  return bits > 2 && ((n >= 1L << 27 && nb > 4) || (n >= 85000000L && nb > 12));
+}
+
+// The form of gemm_few_kernel with the least expected time.  Fitted to 540 launches from cold memory (2 to 16 rows, all widths,
+// 512x2048 to 57344x8192; 7 % root mean square, 0.1 % longer than the best form on average).
+GemmPlan few_plan(int m, int k, int bits, int nb, int cus, bool split) {
+  if (shared_rows(m, k, bits, nb)) {
+    const int nwl = ((k >> 5) + 1) >> 1, ngroups = (((m >> 5) + 1) / 2 + 1) / 2;
+    int S = 1;
+    while (split && S < kMaxSplit && ngroups * S * 2 <= cus && nwl / (S * 2) >= 16) S *= 2;
+    return gemm_split(m, k, nb, 1, 2, 8, S);
+  }
+  const int nwl = ((k >> 5) + 1) >> 1;
+  const float step = (bits == 2 ? 0.989f : 1.208f) + (nb > 8 ? (float)(nb - 8) * (bits == 2 ? 0.008f : 0.033f) : 0.f);
+  GemmPlan best{};
+  for (int RG = 1; RG <= 2; ++RG) {
+    const int KS = kFewWaves / RG;
+    for (int S = 1; S <= (split ? kMaxSplit : 1) && (S == 1 || nwl / S >= 2); S *= 2) {
+      GemmPlan g = gemm_split(m, k, nb, 0, RG, 1, S);
+      if (S > 1 && (g.S == 1 || (long)g.ngroups * S > cus + cus / 8)) break;
+      const long per = cus / g.S < g.ngroups ? cus / g.S : g.ngroups;
+      g.us = 1.12f + (float)((g.ngroups + per - 1) / per) * ((float)((g.wl_per + KS - 1) / KS) * step + 3.f);
+      if (g.S > 1) g.us += 1.51f + g.S * (0.21f + 3.23e-6f * nb * m);
+      if (best.RG == 0 || g.us < best.us) best = g;
+    }
+  }
+  return best;
 }
 
 // What a launch of gemm_rows_kernel (and the one that adds its k ranges) takes, in us.  The terms are fitted to 4000
@@ -351,10 +381,10 @@ struct GemmParts {
   GemmPlan first, rest;
 };
 
-GemmParts make_plan(int m, int k, int nb, int cus, bool split) {
+GemmParts make_plan(int m, int k, int bits, int nb, int cus, bool split) {
   GemmParts p{m, {}, {}};
   if (nb <= 16) {
-    p.first = gemm_plan16(m, k, nb, cus, split);
+    p.first = few_plan(m, k, bits, nb, cus, split);
     return p;
   }
   p.first = rows_plan(m, k, nb, cus, split);
@@ -384,15 +414,16 @@ GemmParts make_plan(int m, int k, int nb, int cus, bool split) {
 
 // The plan of a call is asked for by its size queries and by its launches; a search takes 1 to 15 us, so each thread
 // keeps those of the last sizes.
-GemmParts gemm_plan(int m, int k, int nb, int cus, bool split) {
+GemmParts gemm_plan(int m, int k, int bits, int nb, int cus, bool split) {
   struct Held {
-    int m, k, nb, cus;  // (of split plans; the others come from callers without scratch)
+    int m, k, bits, nb, cus;  // (of split plans; the others come from callers without scratch)
     GemmParts plan;
   };
   static thread_local Held held[64];
-  if (!split) return make_plan(m, k, nb, cus, false);
-  Held& h = held[((uint32_t)m * 0x9E3779B1u ^ (uint32_t)k * 0x85EBCA77u ^ (uint32_t)nb * 0xC2B2AE3Du) >> 26];
-  if (h.m != m || h.k != k || h.nb != nb || h.cus != cus) h = {m, k, nb, cus, make_plan(m, k, nb, cus, true)};
+  if (!split) return make_plan(m, k, bits, nb, cus, false);
+  Held& h = held[((uint32_t)m * 0x9E3779B1u ^ (uint32_t)k * 0x85EBCA77u ^ (uint32_t)(4 * nb + bits) * 0xC2B2AE3Du) >> 26];
+  if (h.m != m || h.k != k || h.bits != bits || h.nb != nb || h.cus != cus)
+    h = {m, k, bits, nb, cus, make_plan(m, k, bits, nb, cus, true)};
   return h.plan;
 }
 
@@ -411,8 +442,17 @@ void launch_gemm(const GemmPlan& g, T* dst, long ldo, const uint8_t* p, const ui
   const int per = (int)(cus / g.S < units ? cus / g.S : units);  // workgroups per k range
   const dim3 grid((unsigned)g.S, (unsigned)per);
   const int uq = (int)(units / per), ur = (int)(units % per);
-  if (nb <= 16) {
-    gemm_kernel<K, T><<<grid, kThreads, kGemmLds, st>>>(dst, p, x, t, m, k, nb, ldo, round_f16, g.wl_per, uq, ur);
+  if constexpr (K > 2) {
+    if (g.NB == 1) {
+      gemm_kernel<K, T><<<grid, kThreads, kGemmLds, st>>>(dst, p, x, t, m, k, nb, ldo, round_f16, g.wl_per, uq, ur);
+      return;
+    }
+  }
+  if (g.NB == 0) {
+    if (g.RG == 2)
+      gemm_few_kernel<K, 2, T><<<grid, 64 * kFewWaves, kGemmLds, st>>>(dst, p, x, t, m, k, nb, ldo, round_f16, g.wl_per, uq, ur);
+    else
+      gemm_few_kernel<K, 1, T><<<grid, 64 * kFewWaves, kGemmLds, st>>>(dst, p, x, t, m, k, nb, ldo, round_f16, g.wl_per, uq, ur);
     return;
   }
 #define QTIP_ROWS(NBV, RGV)                                                                                       \
@@ -465,7 +505,7 @@ int run_gemm(TOut* out, const void* packed, const void* x_f16, const void* tlut,
   const int step = pass_rows(k);
   for (int b0 = 0; b0 < batch; b0 += step) {
     const int nb = batch - b0 < step ? batch - b0 : step;
-    const GemmParts parts = gemm_plan(m, k, nb, cus, workspace != nullptr);
+    const GemmParts parts = gemm_plan(m, k, bits, nb, cus, workspace != nullptr);
     const uint16_t* xx = (const uint16_t*)x_f16 + (size_t)b0 * k;
     for (int part = 0; part < 2; ++part) {
       const int first = part ? parts.m0 : 0, rows = part ? m - parts.m0 : parts.m0;
@@ -498,7 +538,8 @@ hipError_t qtip_gemm_allow_lds() {
                                (int)bytes)) != hipSuccess)                                                       \
     return e;
 #define QTIP_ALLOW_GEMM(KB, T)                        \
-  QTIP_ALLOW((gemm_kernel<KB, T>), kGemmLds)            \
+  QTIP_ALLOW((gemm_few_kernel<KB, 1, T>), kGemmLds)     \
+  QTIP_ALLOW((gemm_few_kernel<KB, 2, T>), kGemmLds)     \
   QTIP_ALLOW((gemm_rows_kernel<KB, 8, 8, T>), kGemmLds) \
   QTIP_ALLOW((gemm_rows_kernel<KB, 8, 4, T>), kGemmLds) \
   QTIP_ALLOW((gemm_rows_kernel<KB, 6, 8, T>), kGemmLds) \
@@ -513,6 +554,10 @@ hipError_t qtip_gemm_allow_lds() {
   QTIP_ALLOW_GEMM(2, _Float16)
   QTIP_ALLOW_GEMM(3, _Float16)
   QTIP_ALLOW_GEMM(4, _Float16)
+  QTIP_ALLOW((gemm_kernel<3, float>), kGemmLds)
+  QTIP_ALLOW((gemm_kernel<4, float>), kGemmLds)
+  QTIP_ALLOW((gemm_kernel<3, _Float16>), kGemmLds)
+  QTIP_ALLOW((gemm_kernel<4, _Float16>), kGemmLds)
 #undef QTIP_ALLOW_GEMM
 #undef QTIP_ALLOW
   return hipSuccess;
@@ -528,7 +573,7 @@ size_t qtip_gemm_workspace_bytes(int m, int k, int bits, int batch) {
   const int step = pass_rows(k);
   for (int nb : {batch < step ? batch : step, batch % step}) {
     if (nb < 1) continue;
-    const GemmParts p = gemm_plan(m, k, nb, cus, true);
+    const GemmParts p = gemm_plan(m, k, bits, nb, cus, true);
     for (size_t bytes : {parts_bytes(p.first, p.m0, nb), p.m0 < m ? parts_bytes(p.rest, m - p.m0, nb) : 0})
       need = bytes > need ? bytes : need;
   }

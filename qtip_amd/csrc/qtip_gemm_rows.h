@@ -1,10 +1,9 @@
 // Batched decompress + fp16 MFMA GEMM from 17 batch rows on.  Included by qtip_gemm.hip inside its namespace.
 //
-// The lane map of gemm_kernel (a wave takes 64 matrix rows by 64 columns, the table words are MFMA operands as
-// they come out of LDS), but the matrix cores do not wait for the decode: a wave multiplies one column half (16 of the 32
+// The matrix cores do not wait for the decode: a wave multiplies one column half (16 of the 32
 // columns of either tile block, 16 table words) while it looks up the words of the next, and the instructions of
-// both, with the LDS reads of the activations two groups ahead, are issued in turn.  (gemm_kernel decodes, then
-// multiplies, between two barriers, and 128 rows of 28672x8192 reached 0.67 PFLOP/s.)
+// both, with the LDS reads of the activations two groups ahead, are issued in turn.  (Decoding, then
+// multiplying, between two barriers reached 0.67 PFLOP/s at 128 rows of 28672x8192.)
 //
 // A workgroup is eight waves of up to 256 registers, two to a SIMD: RG row-block pairs by KS = 8 / RG column slices
 // of 64, a batch tile of 16 * NB rows.  The 128 KiB table leaves 32 KiB: two tiles of activations, one stage
@@ -16,7 +15,7 @@
 //
 // Unit = (group of RG pairs, batch tile); a workgroup keeps one k range and walks its units with the pipeline running
 // across their boundaries.  The slices of a unit meet in LDS at its end, each wave adding up a share.  S > 1 (few
-// units): fp32 partial results, as in gemm_kernel.
+// units): fp32 partial results.
 //
 // A wave-load of NB batch tiles takes about 0.64 + 0.099 NB us on a full chip, where the matrix cores alone need
 // 0.107 NB at 2.4 GHz and the decode by itself 0.53: it is bound by issue (95 vector instructions beside 8 NB products

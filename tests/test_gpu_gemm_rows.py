@@ -55,9 +55,11 @@ def test_activations_beyond_two_gib(k):
     assert bool(((y - want).abs() <= 2.0**-20 * size).all())
 
 
-# each form of the kernel of 17 rows and more (batch tiles of 32, 64, 96 and 128 rows by 2, 4 and 8 row-block pairs, cut along k
-# or not, in one launch or two), ranges of k that end inside a stage and inside a 64-column piece
-@pytest.mark.parametrize("m,k,batch,bits", [(64, 32, 17, 2), (544, 96, 40, 3), (96, 160, 150, 4), (512, 2048, 31, 3), (4096, 4096, 45, 4),
+# each form of the kernels: up to 16 rows one or two row-block pairs, or activations shared (the largest matrices at 3 and 4
+# bits); from 17 rows on batch tiles of 32, 64, 96 and 128 rows by 2, 4 and 8 pairs; cut along k or not, in one launch or
+# two; ranges of k that end inside a stage and inside a 64-column piece
+@pytest.mark.parametrize("m,k,batch,bits", [(1056, 928, 9, 2), (96, 32, 2, 3), (1248, 2080, 16, 4), (32768, 2144, 13, 2),
+                                            (16384, 8192, 5, 3), (22016, 4096, 16, 4), (64, 32, 17, 2), (544, 96, 40, 3), (96, 160, 150, 4), (512, 2048, 31, 3), (4096, 4096, 45, 4),
                                             (1056, 2080, 130, 2), (8192, 4096, 61, 3), (12288, 2144, 90, 4), (8192, 1248, 250, 3),
                                             (5632, 992, 1000, 2), (10240, 1120, 512, 4), (22016, 4096, 700, 3), (16416, 2080, 1030, 2),
                                             (1728, 832, 2048, 4)])
@@ -76,7 +78,8 @@ def test_forms_of_many_rows(m, k, batch, bits):
     assert torch.equal(half, got.half())
 
 
-@pytest.mark.parametrize("m,k,batch", [(64, 32, 40), (128, 96, 20), (2048, 832, 100), (1056, 928, 200)])
+@pytest.mark.parametrize("m,k,batch", [(64, 32, 5), (128, 96, 16), (1056, 928, 11), (64, 32, 40), (128, 96, 20),
+                                       (2048, 832, 100), (1056, 928, 200)])
 def test_infinite_table_entry_stays_in_its_rows(m, k, batch):
     """Where k ends inside a stage, what stands in for the missing weights is met by zeros: it must not be a table entry the
     row does not hold (state 0 selects entry 0)."""
