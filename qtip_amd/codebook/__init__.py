@@ -42,10 +42,10 @@ def _make(m, k, bits):
         # reference glue (lib/codebook/__init__.py:85-92): x.to(fp16), flat
         # codebook, (1, m) fp32 result; no zero-fill is needed here because
         # the kernel overwrites every element
-        xh = x.to(torch.float16).contiguous()
-        out = ops.decompress_matvec(compressed.reshape(-1), xh.reshape(-1), codebook.reshape(-1).contiguous(),
-                                    m, k, bits)
-        return out.view(1, m)
+        if not compressed.is_contiguous():
+            compressed = compressed.contiguous()
+        return ops.decompress_matvec(compressed, x.to(torch.float16).contiguous(), codebook.contiguous(), m, k, bits,
+                                     out=x.new_empty((1, m), dtype=torch.float32))
 
     kdict[(m, 1, k, bits)] = getattr(torch.ops.quip_lib, name)
 

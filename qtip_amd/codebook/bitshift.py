@@ -176,6 +176,10 @@ class bitshift_codebook(nn.Module):
     viterbi = update = quantize_seq = quantize
 
 
+def _contiguous(t):
+    return t if t.is_contiguous() else t.contiguous()
+
+
 # Rows up to which a product decodes the matrix as it multiplies (gemm_rows_kernel): once per 64 to 128 rows, where the
 # dense route writes and reads 2 m n bytes once and then multiplies at the library's rate.  us at 2000 rows, dense / fused:
 # 4096x4096 73/66, 12288x4096 197/184, 22016x4096 446/317, 4096x11008 190/156, 28672x8192 805/770, 512x2048 20/15, 1728x832
@@ -227,7 +231,7 @@ class BitshiftLinear(nn.Module):
         return ops.decode(trellis.reshape(-1), self._tlut16(trellis.device), m, n, self.cb.K)
 
     def _tlut16(self, device):
-        t = self.cb.tlut
+        t = self._modules["cb"].tlut
         if t.dtype != torch.float16 or t.device != device or not t.is_contiguous():
             t = t.to(device=device, dtype=torch.float16).contiguous()
         return t
@@ -257,7 +261,7 @@ class BitshiftLinear(nn.Module):
                 mode='eval', **kwargs):
         """y = (H_R [hatW fp16(H_L^T (x * SU) / 32)]) * (SV * 32), cast to input.dtype
         (lib/codebook/bitshift.py:415-472).  Launches: RHT-in, matvec or GEMM, RHT-out."""
-        n, m = len(SU), len(SV)
+        n, m = SU.shape[0], SV.shape[0]
         if mode == 'train-fixW':
             x = input.view(-1, n).to(torch.float32) * SU
             x = (x.to(self.internal_dtype) @ self.hatW.T).float()
@@ -273,7 +277,8 @@ class BitshiftLinear(nn.Module):
             return self._forward_autograd(input, trellis, SU, SV, had_left, had_right, K_left, K_right, rcp,
                                           tp_rank, mode)
         dev = input.device
-        x = input.reshape(-1, n)
+        flat = input.dim() == 2 and input.shape[1] == n  # (views and reshapes cost a call 0.5 us each)
+        x = input if flat else input.reshape(-1, n)
         bs = x.shape[0]
         if bs == 0:
             return input.new_empty(*input.shape[:-1], m)
@@ -286,13 +291,13 @@ class BitshiftLinear(nn.Module):
                 and SV.dtype == torch.float32 and SV.device == dev and x.dtype in (torch.float16, torch.float32)):
             # both transforms and the product by one call of the library: what bounds such a call otherwise is the
             # host.  (Where takes_dense holds the product is the BLAS library's.)  us per call, launch by launch /
-            # here: 4096x4096, 2 bits, one row 40 / 27; 28672x8192, 4 bits, 16 rows 59 / 44; 4096x11008, 3 bits, 45
-            # rows 65 / 35
-            return ops.linear(x.contiguous(), trellis.contiguous(), self._tlut16(dev), SU.contiguous(), SV.contiguous(),
-                              had_bits(had_left, K_left, True, dev) if K_left > 1 else None, K_left,
-                              had_bits(had_right, K_right, False, dev) if K_right > 1 else None, K_right,
-                              m, n, self.cb.K, (n**-0.5) / self.scale, (m**-0.5) * self.scale
-                              ).view(*input.shape[:-1], m)
+            # here: 4096x4096, 2 bits, one row 40 / 21; 28672x8192, 4 bits, 16 rows 59 / 43; 4096x11008, 3 bits, 45
+            # rows 65 / 32
+            y = ops.linear(_contiguous(x), _contiguous(trellis), self._tlut16(dev), _contiguous(SU), _contiguous(SV),
+                           had_bits(had_left, K_left, True, dev) if K_left > 1 else None, K_left,
+                           had_bits(had_right, K_right, False, dev) if K_right > 1 else None, K_right,
+                           m, n, self.cb.K, (n**-0.5) / self.scale, (m**-0.5) * self.scale)
+            return y if flat else y.view(*input.shape[:-1], m)
 
         # ---- input transform: fp16(H_L^T (x * SU) / sqrt(n) / 32)
         fused_in = (rcp != 1 and SU.dtype == torch.float16 and x.dtype in (torch.float16, torch.float32))

@@ -88,8 +88,17 @@ class QuantizedLinear(nn.Module):
             self.build_codebook_class()
         # the reference adds 0 so that a graph's static output is never aliased; the
         # output transform here already writes a fresh tensor
-        result = self.codebook_class(input, self.trellis, self.SU, self.SV, self.had_left, self.had_right, self.K_left,
-                                     self.K_right, self.rcp, self.tp_rank, mode=self.mode)
+        get = self._buffers.get  # (an attribute that nn.Module looks up costs a call 0.3 us)
+        trellis, SU, SV, left, right = get("trellis"), get("SU"), get("SV"), get("had_left"), get("had_right")
+        # parameters in their place, or a table order of 1
+        trellis = self.trellis if trellis is None else trellis
+        SU, SV = self.SU if SU is None else SU, self.SV if SV is None else SV
+        if left is None and self.K_left > 1:
+            left = self.had_left
+        if right is None and self.K_right > 1:
+            right = self.had_right
+        result = self.codebook_class(input, trellis, SU, SV, left, right, self.K_left, self.K_right, self.rcp, self.tp_rank,
+                                     mode=self.mode)
         if self.bias is not None:
             return result + self.bias
         return result

@@ -14,6 +14,8 @@ from . import _lib
 from ._lib import QTIP_F16, QTIP_F32, check, lib, require_cuda, stream_ptr
 
 _DT = {torch.float16: QTIP_F16, torch.float32: QTIP_F32}
+_Tensor, _F16, _F32, _BITS = torch.Tensor, torch.float16, torch.float32, (2, 3, 4)
+_PACKED_TYPES = (torch.int16, torch.uint16, torch.int32, torch.uint8)
 
 # scratch for split-k partial sums, one buffer per (device, stream): launches on one stream are
 # ordered, launches on different streams must not share partial results
@@ -88,8 +90,8 @@ def launchable(*tensors):
 
 
 def _check_packed(packed, m, k, bits):
-    require_cuda(packed, "packed trellis", (torch.int16, torch.uint16, torch.int32, torch.uint8))
-    if bits not in (2, 3, 4):
+    require_cuda(packed, "packed trellis", _PACKED_TYPES)
+    if bits not in _BITS:
         raise ValueError(f"bits must be 2, 3 or 4 (got {bits})")
     if m % 32 or k % 32 or m <= 0 or k <= 0:
         raise ValueError(f"shape {m}x{k}: m and k must be positive multiples of 32")
@@ -119,26 +121,26 @@ def decode(packed, tlut, m, k, bits):
 
 def decompress_matvec(packed, x, tlut, m, k, bits, out=None, split_k=True):
     """out[m] fp32 = decode(packed)[m,k] @ x[k]; x is fp16 with k elements."""
+    dev = packed.device
     _check_packed(packed, m, k, bits)
-    _check_tlut(tlut, packed.device)
-    require_cuda(x, "x", torch.float16)
-    if x.numel() != k or x.device != packed.device:
-        raise ValueError(f"x must hold {k} fp16 values on {packed.device}")
+    _check_tlut(tlut, dev)
+    require_cuda(x, "x", _F16)
+    if x.numel() != k or x.device != dev:
+        raise ValueError(f"x must hold {k} fp16 values on {dev}")
     if out is None:
-        out = torch.empty((m,), dtype=torch.float32, device=packed.device)
+        out = torch.empty((m,), dtype=_F32, device=dev)
     else:
-        require_cuda(out, "out", torch.float32)
+        require_cuda(out, "out", _F32)
         if out.numel() != m:
             raise ValueError(f"out must hold {m} fp32 values")
-    L = lib()
-    stream = stream_ptr(packed.device)
+    stream = stream_ptr(dev)
     wsp, wsb = None, 0
-    if split_k and matvec_split(m, k, bits, packed.device) > 1:
-        ws = _workspace(packed.device, 16 * m * 4, stream)
+    if split_k and matvec_split(m, k, bits, dev) > 1:
+        ws = _workspace(dev, 16 * m * 4, stream)
         wsp, wsb = _ptr(ws), ws.numel()
-    with _on(packed.device):
-        check(L.qtip_decompress_matvec(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, wsp, wsb, stream),
-              "qtip_decompress_matvec")
+    with _on(dev):
+        check(lib().qtip_decompress_matvec(out.data_ptr(), packed.data_ptr(), x.data_ptr(), tlut.data_ptr(), m, k, bits,
+                                           wsp, wsb, stream), "qtip_decompress_matvec")
     return out
 
 
@@ -311,11 +313,7 @@ def decompress_gemm(packed, x, tlut, m, k, bits, round_f16=True, out_dtype=torch
     return out
 
 
-def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out):
-    """A whole quantized projection in one call of the library: out (rows, m) in x's dtype = sv * scale_out * H_out(
-    fp16(scale_in * H_in(su * x)) @ decode(packed)^T) for x (rows, k) fp16 / fp32; the launches, and the results bit
-    for bit, of rht, decompress_matvec_parts[_rht] (one row) or decompress_gemm (more), rht.  had_in / had_out: sign
-    bits of the table orders (None for order 1)."""
+def _check_linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits):
     dev, rows = packed.device, x.shape[0]
     _check_packed(packed, m, k, bits)
     _check_tlut(tlut, dev)
@@ -334,6 +332,34 @@ def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, 
             require_cuda(bits_t, "sign bits", torch.int32)
             if bits_t.numel() * 32 < order * order:
                 raise ValueError("sign bits too short")
+    return dev, rows
+
+
+def _order_ok(t, order, n):
+    p = n // order
+    return not (n % order or p & (p - 1)) and (order == 1 or (
+        isinstance(t, _Tensor) and t.is_cuda and t.dtype is torch.int32 and t.is_contiguous()
+        and t.numel() * 32 >= order * order))
+
+
+def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out):
+    """A whole quantized projection in one call of the library: out (rows, m) in x's dtype = sv * scale_out * H_out(
+    fp16(scale_in * H_in(su * x)) @ decode(packed)^T) for x (rows, k) fp16 / fp32; the launches, and the results bit
+    for bit, of rht, decompress_matvec_parts[_rht] (one row) or decompress_gemm (more), rht.  had_in / had_out: sign
+    bits of the table orders (None for order 1)."""
+    # a call whose operands fit asks no more than this; what does not goes through the checks one by one
+    if not (isinstance(x, _Tensor) and isinstance(packed, _Tensor) and isinstance(tlut, _Tensor)
+            and isinstance(su, _Tensor) and isinstance(sv, _Tensor) and packed.is_cuda
+            and packed.dtype in _PACKED_TYPES and tlut.dtype is su.dtype is _F16 and sv.dtype is _F32
+            and (x.dtype is _F16 or x.dtype is _F32)
+            and x.device == (dev := packed.device) == tlut.device == su.device == sv.device
+            and packed.is_contiguous() and x.is_contiguous() and tlut.is_contiguous() and su.is_contiguous()
+            and sv.is_contiguous() and x.dim() == 2 and x.shape[1] == k and 1 <= (rows := x.shape[0]) <= 65535
+            and su.numel() == k and sv.numel() == m and tlut.numel() == 1024
+            and bits in _BITS and m > 0 and k > 0 and not (m | k) & 31
+            and packed.numel() * packed.element_size() * 8 == bits * m * k
+            and _order_ok(had_in, order_in, k) and _order_ok(had_out, order_out, m)):
+        dev, rows = _check_linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits)
     dt = _DT[x.dtype]
     if rows >= _ALIGN_ROWS and (x.data_ptr() | su.data_ptr() | sv.data_ptr()) & 15:
         x, su, sv = map(aligned16, (x, su, sv))
