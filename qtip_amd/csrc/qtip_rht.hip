@@ -30,7 +30,7 @@ constexpr int kMaxParts = 16;
 //   PRE_RMSNORM   f(x) = fp16(w * fp16(x * rsqrt(mean(x^2) + eps)))   (model/llama.py:129-135)
 //   PRE_SILU_MUL  f = fp16(fp16(silu(g)) * u), g = in[i], u = in[n + i] (model/llama.py:399-400)
 //   residual      out = fp16(residual + fp16(result))                 (model/llama.py:964,979)
-enum { PRE_NONE = 0, PRE_RMSNORM = 1, PRE_SILU_MUL = 2 };
+enum { PRE_NONE = 0, PRE_RMSNORM = 1, PRE_SILU_MUL = 2, PRE_PARTS = 3 };  // (PRE_PARTS: only as a form of rht_mix_kernel)
 
 struct RhtParams {
   void* out;
@@ -46,6 +46,7 @@ struct RhtParams {
   size_t pre_row_stride;     // the same for `pre`
   float scale, eps;
   int in_parts, n, order, logA, pp, pre_mode;
+  int round_parts;           // `in` is fp32 partial sums of an fp16 vector: added in order, then rounded to fp16
   // from the host (divisions and search loops in the prologue of a latency-bound kernel are time on
   // its critical path): log2 of the column groups (vectorised form) or of the columns (scalar form),
   // log2 of the waves holding a row in the transform, passes over the vector
@@ -696,6 +697,10 @@ __global__ __launch_bounds__(kRhtThreads) void rht_rows_kernel(const RhtParams P
 #pragma unroll
       for (int i = 0; i < EPT; ++i) v[i] += t[i];
     }
+    if (P.round_parts) {
+#pragma unroll
+      for (int i = 0; i < EPT; ++i) v[i] = (float)(_Float16)v[i];
+    }
   }
   wht_regs<EPT>(v);
 #pragma unroll
@@ -769,6 +774,9 @@ bool mix_shape(int n, int order, int rows, MixShape& M, int& kt) {
 
 // rows from which the one-workgroup-per-row form is used for the power-of-two sizes it covers
 constexpr int kRowsFormMin = 8;
+bool rows_form_size(int n, int order, int rows) {
+  return order == 1 && rows >= kRowsFormMin && (n == 2048 || n == 4096 || n == 8192);
+}
 
 // Rows from which the matrix form is faster than one launch of order * A workgroups per row (`wgs`), which each read
 // the whole row: its time hardly grows with the rows, theirs with rows * wgs once that passes what the chip holds.  fp32
@@ -830,13 +838,14 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
   hipStream_t st = (hipStream_t)stream;
   const bool fused = P.pre_mode != PRE_NONE || P.residual != nullptr;
   {
-    const size_t ez = in_dtype == QTIP_F16 ? 2 : 4;
-    const bool rows_form = !fused && order == 1 && rows >= kRowsFormMin && (n == 2048 || n == 4096 || n == 8192) &&
+    const size_t ez = in_dtype == QTIP_F16 && !P.round_parts ? 2 : 4;
+    const bool rows_form = !fused && rows_form_size(n, order, rows) &&
                            (reinterpret_cast<uintptr_t>(P.in) & 15u) == 0 && (reinterpret_cast<uintptr_t>(P.out) & 15u) == 0 &&
                            ((P.in_row_stride * ez) & 15u) == 0 && ((P.part_stride * ez) & 15u) == 0 &&
                            (!P.pre || (reinterpret_cast<uintptr_t>(P.pre) & 15u) == 0) &&
                            (!P.post || ((reinterpret_cast<uintptr_t>(P.post) & 15u) == 0 && (P.post_row_stride & 3u) == 0));
     if (rows_form) {
+      if (P.round_parts) return out_dtype == QTIP_F16 ? launch_rht_rows<float, _Float16>(P, rows, st) : launch_rht_rows<float, float>(P, rows, st);
       if (in_dtype == QTIP_F16 && out_dtype == QTIP_F16) return launch_rht_rows<_Float16, _Float16>(P, rows, st);
       if (in_dtype == QTIP_F16) return launch_rht_rows<_Float16, float>(P, rows, st);
       if (out_dtype == QTIP_F16) return launch_rht_rows<float, _Float16>(P, rows, st);
@@ -844,7 +853,7 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
     }
   }
   if (rows >= 8) {
-    const size_t ez = in_dtype == QTIP_F16 ? 2 : 4;
+    const size_t ez = in_dtype == QTIP_F16 && !P.round_parts ? 2 : 4;
     MixShape M{};
     int kt = 0;
     auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
@@ -859,6 +868,9 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
       int cus = 0;
       const int rc = qtip_device_ready(stream, &cus);
       if (rc) return rc;
+      if (P.round_parts)
+        return out_dtype == QTIP_F16 ? launch_mix<_Float16, _Float16, PRE_PARTS>(P, M, kt, rows, cus, st)
+                                     : launch_mix<_Float16, float, PRE_PARTS>(P, M, kt, rows, cus, st);
       if (P.pre_mode == PRE_RMSNORM) return launch_mix<_Float16, _Float16, PRE_RMSNORM>(P, M, kt, rows, cus, st);
       if (P.pre_mode == PRE_SILU_MUL) return launch_mix<_Float16, _Float16, PRE_SILU_MUL>(P, M, kt, rows, cus, st);
       if (in_dtype == QTIP_F16 && out_dtype == QTIP_F16) return launch_mix<_Float16, _Float16, PRE_NONE>(P, M, kt, rows, cus, st);
@@ -867,6 +879,7 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
       return launch_mix<float, float, PRE_NONE>(P, M, kt, rows, cus, st);
     }
   }
+  if (P.round_parts) return QTIP_E_SHAPE;           // (qtip_rht_takes_parts said so)
   if (fused && out_dtype != QTIP_F16) return QTIP_E_DTYPE;  // fused forms exist for the combinations the decode loop uses
   // vectorised form: 8 columns per thread, 16-byte loads
   const size_t esz = in_dtype == QTIP_F16 ? 2 : 4;
@@ -1009,6 +1022,47 @@ __global__ __launch_bounds__(kRhtThreads) void rht_chain_kernel(
 
 }  // namespace
 
+// The output transform of a product cut along k: fp32 partial sums, parts[w][row][i], are added in order and rounded to fp16 on
+// load, which is what the product leaves otherwise, one launch and one pass over it earlier.  The forms of many rows
+// take them (aligned operands).
+// us per projection in a graph, ranges added by a launch / here, rows (ranges): one workgroup per row (the orders of one), up to
+// 16 ranges: 2048 x 28672, 17 (16) 30.9/29.4, 400 (8) 90.7/89.2; 4096 x 2048, 64 (4) 18.4/16.3.
+// The matrix form has fewer loads in flight and reads a range in pieces of its columns, 2^logpp values each: up to four ranges
+// at 128 columns, two at 64: 3072 x 4096, 120 (2) 25.0/23.4; 5120 x 8192, 64 (4) 32.4/31.5, 5120 x 28672, 64 (8) 59.0/59.6;
+// 11008 x 4096, 17 (2) 28.4/27.9; 11008 x 8192, 64 (4) 45.7/47.1.  Narrower ones lose: 1728, 40 (8) 24.6/28.6; 448, 64 (4)
+// 18.3/19.1; 928 = 116 * 8, 17 (4) 19.5/24.3, 400 (2) 41.7/42.8.
+bool qtip_rht_takes_parts(int n, int order, int rows, int nparts) {
+  if (rows_form_size(n, order, rows)) return true;
+  if (rows < 8 || order < 1 || n % order || (n & 7)) return false;
+  const int p = n / order;
+  if (p & (p - 1)) return false;
+  long pp = p, OT = order;  // (the workgroups per row of the other form, as launch_rht counts them)
+  while (pp > kRhtThreads) pp >>= 1, OT <<= 1;
+  while (pp > 64 && (OT << 1) <= 64) pp >>= 1, OT <<= 1;
+  MixShape M{};
+  int kt = 0;
+  return mix_shape(n, order, rows, M, kt) && nparts << 5 <= 1 << M.logpp &&
+         rows >= mix_rows_min(order, n, OT, true, false, kt, 1 << M.logS);
+}
+
+int qtip_rht_from_parts(void* out, int out_dtype, const float* parts, int nparts, int rows, int n, int order,
+                        const uint32_t* had_bits, const float* post, float scale, void* stream) {
+  RhtParams P{};
+  P.out = out;
+  P.in = parts;
+  P.had_bits = had_bits;
+  P.post = post;
+  P.part_stride = (size_t)rows * n;
+  P.in_row_stride = (size_t)n;
+  P.scale = scale;
+  P.in_parts = nparts;
+  P.n = n;
+  P.order = order;
+  P.pre_mode = PRE_NONE;
+  P.round_parts = 1;
+  return launch_rht(P, out_dtype, QTIP_F16, rows, stream);
+}
+
 // LDS opt-in of this file's kernels, part of the device set-up
 hipError_t qtip_rht_allow_lds() {
 #define QTIP_MIX3(TI, TO, MODE)                                                                       \
@@ -1016,7 +1070,8 @@ hipError_t qtip_rht_allow_lds() {
       (const void*)rht_mix_kernel<TI, TO, MODE, 8>
   const void* fns[] = {QTIP_MIX3(_Float16, _Float16, PRE_RMSNORM), QTIP_MIX3(_Float16, _Float16, PRE_SILU_MUL),
                        QTIP_MIX3(_Float16, _Float16, PRE_NONE),    QTIP_MIX3(_Float16, float, PRE_NONE),
-                       QTIP_MIX3(float, _Float16, PRE_NONE),       QTIP_MIX3(float, float, PRE_NONE)};
+                       QTIP_MIX3(float, _Float16, PRE_NONE),       QTIP_MIX3(float, float, PRE_NONE),
+                       QTIP_MIX3(_Float16, _Float16, PRE_PARTS),   QTIP_MIX3(_Float16, float, PRE_PARTS)};
 #undef QTIP_MIX3
   for (const void* f : fns) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mix_lds(kMixMaxKT, kMixMaxOrder));

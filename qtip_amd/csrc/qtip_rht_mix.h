@@ -65,8 +65,9 @@ template <typename TIn, typename TOut, int MODE, int KTC>
 __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P, const MixShape M, int rows) {
   extern __shared__ __align__(16) uint8_t mix_smem[];
   constexpr bool F16 = sizeof(TIn) == 2;
-  constexpr bool AUX = MODE != PRE_NONE;
-  static_assert(!AUX || F16, "the element-wise prologues take fp16 rows");
+  constexpr bool PARTS = MODE == PRE_PARTS;  // rows of fp32 partial sums, summed and rounded to fp16 on load
+  constexpr bool AUX = MODE != PRE_NONE && !PARTS;
+  static_assert(MODE == PRE_NONE || F16, "the element-wise prologues take fp16 rows");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int KT = blockDim.x >> 7;
@@ -109,8 +110,35 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   auto load_patch = [&](Patch& p, int ps, uint32_t add) {
     const TIn* src = in + first_row(ps) * P.in_row_stride;
     const uint32_t lr = lane_row(ps) * (uint32_t)P.in_row_stride + add;
+    if constexpr (PARTS) {
+      const float* parts = reinterpret_cast<const float*>(P.in) + first_row(ps) * P.in_row_stride;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) p.x[i].load(src + (lr + eoff[i]));
+      for (int i0 = 0; i0 < 4; i0 += 2) {  // (two rows at a time: registers)
+        float t[2][8];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) ld_f32<8>(parts + (lr + eoff[i0 + i]), t[i]);
+        for (int w = 1; w < P.in_parts; ++w) {
+          const float* more = parts + w * P.part_stride;
+          float q[2][8];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) ld_f32<8>(more + (lr + eoff[i0 + i]), q[i]);
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) t[i][e] += q[i][e];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          half8m h;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) h[e] = (_Float16)t[i][e];
+          p.x[i0 + i] = __builtin_bit_cast(Raw8<TIn>, h);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p.x[i].load(src + (lr + eoff[i]));
+    }
     if (P.pre) {
       const _Float16* f = P.pre + first_row(ps) * P.pre_row_stride;
       const uint32_t lf = lane_row(ps) * (uint32_t)P.pre_row_stride + add;
@@ -283,7 +311,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   // ---- one plane of fp16 values: no slices or partial sums to add, and a sign vector of nothing but
   // +-1 (the same for every pass)
   if constexpr (F16) {
-    bool fast = S == 1 && P.in_parts == 1 && (!P.pre || P.pre_row_stride == 0);
+    bool fast = S == 1 && (PARTS || P.in_parts == 1) && (!P.pre || P.pre_row_stride == 0);
     if (fast && P.pre) {
       uint32_t off = 0;
 #pragma unroll
@@ -362,7 +390,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
             for (int e = 0; e < 8; ++e) t[e] = (float)x[e];
           } else {
             cur.x[i].get(t);
-            for (int w = 1; w < P.in_parts; ++w) {
+            for (int w = 1; w < (PARTS ? 1 : P.in_parts); ++w) {
               Raw8<TIn> y;
               y.load(in + w * P.part_stride + first_row(ps) * P.in_row_stride + (lr + eoff[i]));
               float q[8];
