@@ -61,8 +61,9 @@ int qtip_linear(void* out, const void* x, int x_dtype, const void* packed, const
     if (rc) return rc;
     // A product cut along k: the output transform adds the ranges on load where it is a form of many rows that takes them; a
     // launch for the sums and a pass over them less, the same bits.  us per call in a graph, fp16, m x k, rows (ranges), before
-    // -> now: 4096 x 4096, 9 (4) 14.8 -> 13.2, 64 (4) 20.4 -> 18.3, 120 (2) 23.7 -> 21.4; 4096 x 11008, 64 (4) 33.6 -> 31.6;
-    // 8192 x 28672, 400 (4) 232.7 -> 227.9; 5120 x 2048, 64 (2) 21.3 -> 19.7.
+    // -> now: 2048 x 4096, 2 (4) 13.9 -> 12.3; 4096 x 4096, 5 (4) 15.0 -> 12.9, 9 (4) 14.8 -> 13.2, 64 (4) 20.4 -> 18.3,
+    // 120 (2) 23.7 -> 21.4; 4096 x 11008, 64 (4) 33.6 -> 31.6; 8192 x 28672, 400 (4) 232.7 -> 227.9; 5120 x 2048, 64 (2)
+    // 21.3 -> 19.7.
     if (rows > 1 && p.ws_bytes && aligned16(out) && aligned16(sv)) {
       const int S = qtip_gemm_ranges(m, k, bits, rows);
       if (S > 1 && qtip_rht_takes_parts(m, order_out, rows, S)) {

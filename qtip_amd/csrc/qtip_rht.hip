@@ -772,10 +772,12 @@ bool mix_shape(int n, int order, int rows, MixShape& M, int& kt) {
   return true;
 }
 
-// rows from which the one-workgroup-per-row form is used for the power-of-two sizes it covers
-constexpr int kRowsFormMin = 8;
+// Rows from which the one-workgroup-per-row form is used for the power-of-two sizes it covers.  us in a graph, fp16 rows under a
+// sign vector, the form of n / 64 workgroups per row / this one: 2048, 2 rows 3.0/2.9, 7 rows 3.2/3.0; 4096, 2 rows 3.1/3.2,
+// 4 rows 3.2/3.2, 5 rows 3.5/3.2; 8192, 4 rows 3.8/4.5, 7 rows 4.6/4.5, to fp32 4.6/5.0.
+// Ranges of a cut product are added on load from the same rows on: a projection gives the bits of its launches.
 bool rows_form_size(int n, int order, int rows) {
-  return order == 1 && rows >= kRowsFormMin && (n == 2048 || n == 4096 || n == 8192);
+  return order == 1 && ((n == 2048 && rows >= 2) || (n == 4096 && rows >= 5) || (n == 8192 && rows >= 8));
 }
 
 // Rows from which the matrix form is faster than one launch of order * A workgroups per row (`wgs`), which each read

@@ -43,7 +43,8 @@ def test_linear_is_its_launches(m, k, rows, dtype, bits):
 
 # ranges of k added by the output transform: one workgroup per row (2, 4, 8 values a thread, 2 to 16 ranges), the matrix form at
 # 128 columns (2, 4 ranges; a last pass that is not full) and 64 (two), and the sizes on the other side of each line
-@pytest.mark.parametrize("m,k,rows", [(2048, 28672, 17), (2048, 4096, 8), (4096, 2048, 64), (4096, 4096, 7), (8192, 4096, 33),
+@pytest.mark.parametrize("m,k,rows", [(2048, 28672, 17), (2048, 4096, 8), (4096, 2048, 64), (4096, 4096, 4), (4096, 4096, 5), (2048, 4096, 2),
+                                      (8192, 11008, 7), (8192, 4096, 33),
                                       (5120, 2048, 45), (3072, 8192, 65), (3072, 4096, 17), (12288, 4096, 19), (11008, 4096, 17),
                                       (11008, 8192, 40), (928, 8192, 400), (832, 4096, 40)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
