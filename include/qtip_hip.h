@@ -196,7 +196,8 @@ int qtip_decompress_gemm_f16(void* out_f16, const void* packed, const void* x_f1
  * sv * scale_out * H_out(fp16(scale_in * H_in(su * x)) @ decode(packed)^T), H of order_in x k / order_in and
  * order_out x m / order_out with sign bits as qtip_rht takes them (NULL for order 1).  The launches are those of
  * qtip_rht, qtip_decompress_matvec_parts (one row; with the input transform inside where
- * qtip_decompress_matvec_parts_rht covers it) or qtip_decompress_gemm_f16, qtip_rht, and so are the results.
+ * qtip_decompress_matvec_parts_rht covers it) or qtip_decompress_gemm_f16, qtip_rht, and so are the results; where the
+ * product is cut along k, the output transform may add the ranges itself instead of a launch before it.
  * workspace: qtip_linear_workspace_bytes(...) bytes of scratch, 16-byte aligned, 0 bytes for a refused shape. */
 size_t qtip_linear_workspace_bytes(int m, int k, int bits, int rows, int order_in, int x_dtype);
 int qtip_linear(void* out, const void* x, int x_dtype, const void* packed, const void* tlut, const void* su_f16,

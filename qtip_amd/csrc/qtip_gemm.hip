@@ -570,8 +570,8 @@ int qtip_gemm_ranges(int m, int k, int bits, int batch) {
   return p.m0 == m ? p.first.S : 1;
 }
 
-int qtip_gemm_parts(float* parts, const void* packed, const void* x_f16, const void* tlut, int m, int k, int bits, int batch,
-                    void* stream) {
+int qtip_gemm_parts(float* parts, int nparts, const void* packed, const void* x_f16, const void* tlut, int m, int k, int bits,
+                    int batch, void* stream) {
   int rc = check_common(parts, packed, x_f16, tlut, m, k, bits);
   if (rc) return rc;
   if (!aligned16(packed) || !aligned16(x_f16) || !aligned16(parts) || (reinterpret_cast<uintptr_t>(tlut) & 3u)) return QTIP_E_ALIGN;
@@ -579,7 +579,7 @@ int qtip_gemm_parts(float* parts, const void* packed, const void* x_f16, const v
   rc = qtip_device_ready(stream, &cus);
   if (rc) return rc;
   const GemmParts p = gemm_plan(m, k, bits, batch, cus, true);
-  if (p.m0 != m || p.first.S < 2 || batch > pass_rows(k)) return QTIP_E_SHAPE;
+  if (p.m0 != m || p.first.S < 2 || p.first.S != nparts || batch > pass_rows(k)) return QTIP_E_SHAPE;
   launch_gemm<float>(bits, p.first, parts, m, (const uint8_t*)packed, (const uint16_t*)x_f16, (const uint32_t*)tlut, m, k, batch,
                      0, cus, (hipStream_t)stream);
   return (int)hipGetLastError();

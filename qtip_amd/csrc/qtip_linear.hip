@@ -68,7 +68,7 @@ int qtip_linear(void* out, const void* x, int x_dtype, const void* packed, const
       const int S = qtip_gemm_ranges(m, k, bits, rows);
       if (S > 1 && qtip_rht_takes_parts(m, order_out, rows, S)) {
         auto* parts = (float*)(ws + p.ws_off);
-        rc = qtip_gemm_parts(parts, packed, ws, tlut, m, k, bits, rows, stream);
+        rc = qtip_gemm_parts(parts, S, packed, ws, tlut, m, k, bits, rows, stream);
         if (rc) return rc;
         return qtip_rht_from_parts(out, x_dtype, parts, S, rows, m, order_out, had_out, sv, scale_out, stream);
       }

@@ -22,8 +22,8 @@ QTIP_INTERNAL hipError_t qtip_gemm_allow_lds();
 // ranges of the one launch of such a product (1: it is not cut, or runs in several launches), the launch, whether the transform
 // takes them, and its launch.
 QTIP_INTERNAL int qtip_gemm_ranges(int m, int k, int bits, int batch);
-QTIP_INTERNAL int qtip_gemm_parts(float* parts, const void* packed, const void* x_f16, const void* tlut, int m, int k, int bits,
-                                  int batch, void* stream);
+QTIP_INTERNAL int qtip_gemm_parts(float* parts, int nparts, const void* packed, const void* x_f16, const void* tlut, int m,
+                                  int k, int bits, int batch, void* stream);
 QTIP_INTERNAL bool qtip_rht_takes_parts(int n, int order, int rows, int nparts);
 QTIP_INTERNAL int qtip_rht_from_parts(void* out, int out_dtype, const float* parts, int nparts, int rows, int n, int order,
                                       const uint32_t* had_bits, const float* post, float scale, void* stream);
