@@ -15,8 +15,6 @@
 // 21.4.  At 4 bits 4096x11008 14.5 / 12.5, 10240x8192 18.2 / 16.9, but 22016x4096 15.9 / 16.8 and 28672x8192 28.0 / 34.2:
 // there the stream is the bound, and requests for 16 rows of activations are in its way.
 
-constexpr int kFewWaves = 16;
-
 template <int K, int RG, typename TOut>
 __global__ __launch_bounds__(64 * kFewWaves, 1) void gemm_few_kernel(
     TOut* __restrict__ dst, const uint8_t* __restrict__ packed, const uint16_t* __restrict__ x,

@@ -27,10 +27,6 @@
 //   28672x8192    48 rows 51 / 45, 128 90 / 69, 256 178 / 109, 1000 469 / 413, 2000 801 / 770
 //   4096x11008    48 rows 21.7 / 19.5, 128 42 / 28, 256 73 / 40, 1000 125 / 91, 2000 189 / 156
 
-constexpr int kRowsWaves = 8;
-// a whole wave-load per stage where two tiles of it fit 32 KiB
-constexpr int rows_stage_halves(int NB, int RG) { return NB * (kRowsWaves / RG) <= 8 ? 2 : 1; }
-
 template <int K>
 struct SlotMap {  // slot r = 0..7 of a column half kh: register of P, and where its two halves' words go
   static constexpr __device__ int reg(int kh, int r) {
