@@ -30,7 +30,7 @@ __global__ __launch_bounds__(64 * kFewWaves, 1) void gemm_few_kernel(
   const uint32_t slot4 = lds_address(lut) + ((uint32_t)(lane & 31) << 2);
   const int nkb = k >> 5, nwl = (nkb + 1) >> 1, nrb = m >> 5, npair = (nrb + 1) >> 1;
   const uint32_t rb_bytes = (uint32_t)nkb * 128 * K;
-  constexpr uint32_t WL_BYTES = 256 * K, OUT = 0x7FFFFF00u;
+  constexpr uint32_t WL_BYTES = 256 * K, OUT = kOutOfRange;
   const uint32_t loff = (uint32_t)pb * rb_bytes + (uint32_t)g0 * (128 * K) + (uint32_t)(2 * r8 + ch) * (8 * K);
   const int nxt4 = (ch ? ((lane & ~23) | ((r8 + 1) & 7)) : (lane | 16)) << 2;
   const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
@@ -61,10 +61,9 @@ __global__ __launch_bounds__(64 * kFewWaves, 1) void gemm_few_kernel(
     w_left = nst;
   };
   auto x_unit = [&]() {
-    x_so = (uint32_t)(wl0 + ks) * 128;
-    x_vo = x_n > 0 && (lane & 15) < batch && !(last_half && nst == 1 && g0)
-               ? ((uint32_t)(lane & 15) * (uint32_t)k + (uint32_t)(32 * g0 + 8 * ch)) * 2
-               : OUT;
+    const FewPlace p = few_activations(lane, batch, k, wl0 + ks, x_n, nst, last_half);
+    x_so = p.so;
+    x_vo = p.vo;
     x_left = nst;
   };
   auto load_x = [&](int d) {

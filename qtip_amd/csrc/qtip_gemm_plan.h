@@ -67,6 +67,23 @@ inline GemmPlan few_plan(int m, int k, int bits, int nb, int cus, bool split) {
   return best;
 }
 
+// Where a lane of gemm_few_kernel reads the activations of wave-load wl, the first of the nst of its wave in a unit, with
+// `units` units to go: scalar and lane offset of 16 bytes (16 more at + 32; the next wave-load is KS * 128 bytes on).
+// Without anything to read the lane offset is out of range by itself and the scalar one 0: the range check of a buffer load
+// need not cover the scalar offset, and one past the end leaves it nothing to check against.  That is so for rows past the
+// batch, behind the last unit, and in a wave whose slice has no wave-load in this range of k (nst 0).  last_half: the last
+// of the nst ends after 32 columns.
+struct FewPlace {
+  uint32_t so, vo;
+};
+constexpr uint32_t kOutOfRange = 0x7FFFFF00u;
+constexpr FewPlace few_activations(int lane, int batch, int k, int wl, int units, int nst, bool last_half) {
+  const int row = lane & 15, ch = (lane >> 4) & 1, g0 = lane >> 5;
+  if (units < 1 || nst < 1) return {0, kOutOfRange};
+  const bool in = row < batch && !(last_half && nst == 1 && g0);
+  return {(uint32_t)wl * 128, in ? ((uint32_t)row * (uint32_t)k + (uint32_t)(32 * g0 + 8 * ch)) * 2 : kOutOfRange};
+}
+
 // What a launch of gemm_rows_kernel (and the one that adds its k ranges) takes, in us.  The terms are fitted to 4000
 // measured launches (2 and 4 bits, 17 to 2000 rows, matrices of 512x2048 to 28672x8192): 5 % root mean square, and the
 // form with the least of it takes 0.4 % longer than the best one on average.  A fixed part, per unit its
