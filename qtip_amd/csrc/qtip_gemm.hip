@@ -60,7 +60,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
   const int r8 = lane & 7, pb = (lane >> 3) & 1, ch = (lane >> 4) & 1, g0 = lane >> 5;
   const uint32_t slot4 = lds_address(lut) + ((uint32_t)(lane & 31) << 2);
   const int nkb = k >> 5;
-  const int nwl = (nkb + 1) >> 1;  // 64-column wave-loads per row; a partial last one meets zero activations
+  const int nwl = (nkb + 1) >> 1;  // 64-column wave-loads per row
   const int nrb = m >> 5;
   const int npair = (nrb + 1) >> 1;
   const uint32_t rb_bytes = (uint32_t)nkb * 128 * K;
@@ -195,6 +195,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
                   const int wi = w_index<K>(R, 2 * kh + mh, j);  // register wi / 2, half wi % 2
                   W[mh][rh][w] = lds_word_abs((wi & 1) ? lut128_addr_hi(Q[wi >> 1], slot4) : lut128_addr_lo(Q[wi >> 1], slot4));
                 }
+            if ((nkb & 1) && wl == nwl - 1) {
+              // no second column block: its zeros decode to table entry 0, which zero activations do not cancel if
+              // it is infinite
+#pragma unroll
+              for (int i = 0; i < 16; ++i) (&W[0][0][0])[i] = g0 ? 0u : (&W[0][0][0])[i];
+            }
             __builtin_amdgcn_sched_barrier(0);
             const uint32_t ca = tile_addr + cb + ((((uint32_t)(8 * ks + 4 * g0 + 2 * kh + ch)) ^ a7) << 4);
             u32x4 xa[NB];

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(64 * kFewWaves, 1) void gemm_few_kernel(
     const int pair = w_u * RG + rg;
     const bool ok = w_n > 0 && nst > 0 && pair < npair;
     w_so = ok ? (uint32_t)(2 * pair) * rb_bytes + (uint32_t)(wl0 + ks) * WL_BYTES : 0u;
-    w_vo = ok && 2 * pair + pb < nrb ? loff - (last_half && nst == 1 && g0 ? 128u * K : 0u) : OUT;
+    w_vo = ok && 2 * pair + pb < nrb && !(last_half && nst == 1 && g0) ? loff : OUT;
     w_left = nst;
   };
   auto x_unit = [&]() {
@@ -90,8 +90,8 @@ __global__ __launch_bounds__(64 * kFewWaves, 1) void gemm_few_kernel(
         --w_n;
         w_u += ustep;
         w_unit();
-      } else if (last_half && g0 && w_vo != OUT) {
-        w_vo -= 128 * K;
+      } else if (last_half && g0) {
+        w_vo = OUT;
       }
     }
   };
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(64 * kFewWaves, 1) void gemm_few_kernel(
   float4_t acc[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-  auto work = [&](int d) {
+  auto work = [&](int d, bool cut) {  // cut: the wave-load ends after 32 columns
     load_x(d ^ 1);
     x_next();
     uint32_t P[16], W[2][16];
@@ -143,6 +143,10 @@ __global__ __launch_bounds__(64 * kFewWaves, 1) void gemm_few_kernel(
         W[kh][SlotMap<K>::word(r, 1)] = lds_word_abs(lut128_addr_hi(q, slot4));
       }
     __builtin_amdgcn_sched_barrier(0);
+    if (uni(cut)) {  // (what the missing block decodes to, table entry 0, may be infinite)
+#pragma unroll
+      for (int i = 0; i < 32; ++i) (&W[0][0])[i] = g0 ? 0u : (&W[0][0])[i];
+    }
 #pragma unroll
     for (int kh = 0; kh < 2; ++kh) {
       // a lane's eight consecutive columns to the operand's four and four
@@ -164,16 +168,16 @@ __global__ __launch_bounds__(64 * kFewWaves, 1) void gemm_few_kernel(
   for (int un = 0; un < upw; ++un, u += ustep) {
     int t = nst;
     if (par && t > 0) {
-      work(1);
+      work(1, last_half && t == 1);
       --t;
     }
     for (; t > 1; t -= 2) {
-      work(0);
-      work(1);
+      work(0, false);
+      work(1, last_half && t == 2);
     }
     par = 0;
     if (t == 1) {
-      work(0);
+      work(0, last_half);
       par = 1;
     }
     par = uni(par);

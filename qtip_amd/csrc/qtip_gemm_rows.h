@@ -103,17 +103,18 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
   constexpr uint32_t OUT = 0x7FFFFF00u;  // a lane offset that is out of range by itself
   // ---- weight stream of this wave, two wave-loads in flight
   LaneData<K> buf[2];
-  // Where a range ends inside a stage, the activations there are zeros, and the weights that meet them are others of
-  // the same rows: a slice past the end loads the range's first wave-load, and a missing second column block is the
-  // first one again.  (Zeros there would decode to table entry 0, which need not be finite in a row without it.)
+  // Where a range ends inside a stage, weights and activations there are zeros without a memory access: of every lane in a
+  // slice past the end, of the second column block where that is missing.  Such weights would decode to table entry 0,
+  // which may be infinite: see cut_words.
   const bool w_over = wl0 + KS * (nst - 1) + ks >= wl1;
-  const bool w_half = (nkb & 1) && (w_over ? wl0 : wl0 + KS * (nst - 1) + ks) == nwl - 1;
+  const bool w_half = !w_over && (nkb & 1) && wl0 + KS * (nst - 1) + ks == nwl - 1;
+  const int cut_left = w_over || w_half ? 1 : 0;  // wave-loads to go in a unit where that is so, 0: nowhere
   Unit wu = first;
   int w_left;
   uint32_t w_so, w_vo;
   auto w_last = [&]() {  // before the last wave-load of a unit
-    if (w_over) w_so -= (uint32_t)(KS * (nst - 1) + ks) * WL_BYTES;
-    if (w_half && g0 && w_vo != OUT) w_vo -= 128 * K;
+    if (w_over) w_so -= (uint32_t)(KS * (nst - 1) + ks) * WL_BYTES;  // (a place that is there)
+    if (w_over || (w_half && g0)) w_vo = OUT;
   };
   auto w_unit = [&]() {
     const int pair = wu.g * RG + rg;
@@ -251,6 +252,26 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
     w[SlotMap<K>::word(r, 0)] = lds_word_abs(lut128_addr_lo(q, slot4));
     w[SlotMap<K>::word(r, 1)] = lds_word_abs(lut128_addr_hi(q, slot4));
   };
+  // Before a wave-load that is cut short, with its first half looked up and its states at hand: finite words in place of
+  // what meets no activations.  (Words cleared before the products of either half cost every wave-load two branches: 1 % on
+  // average, 5 % at 5120x13824, 128 rows.)
+  uint32_t finite = 0;  // a state of a finite table entry, in both halves
+  if (cut_left) {
+    for (uint32_t s2 = 0; s2 < 4096u * 0x10001u; s2 += 0x10001u) {
+      const uint32_t w = uni(lds_word_abs(lut128_addr_lo(pk_hash(s2) & 0xFFC0FFC0u, slot4)));
+      if ((w & 0x7C00u) != 0x7C00u && (w & 0x7C000000u) != 0x7C000000u) {
+        finite = s2;
+        break;
+      }
+    }
+  }
+  auto cut_words = [&]() {
+    const bool none = w_over || g0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) W[0][i] = none ? 0u : W[0][i];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) P[SlotMap<K>::reg(1, r)] = none ? finite : P[SlotMap<K>::reg(1, r)];
+  };
   constexpr int GN = NB >= 4 ? 2 : 1, NG = NB / GN;  // batch tiles per group of instructions
   u32x4 xa[2 * GN];
   fetch_next(0);
@@ -267,6 +288,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
   };
   Unit cu = first;
   int c_left = nst;
+  if (nst == cut_left) cut_words();
   for (int left = T; left > 0; left -= 2) {
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
@@ -319,7 +341,8 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
       }
       w_next();
       x_next();
-      if (uni(--c_left) == 0) {
+      if (uni(--c_left) > cut_left) continue;
+      if (c_left == 0) {
         c_left = nst;
         const int pair = cu.g * RG + rg;
         const int row = 64 * pair + 32 * g0 + 4 * ch;
@@ -383,6 +406,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
         for (int i = 0; i < 4 * NB; ++i) (&acc[0][0])[i] = float4_t{0.f, 0.f, 0.f, 0.f};
         advance(cu);
       }
+      if (uni(c_left) == cut_left) cut_words();
     }
   }
 }

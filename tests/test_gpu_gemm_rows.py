@@ -96,3 +96,34 @@ def test_infinite_table_entry_stays_in_its_rows(m, k, batch):
     ref, size = x.double() @ w[finite].double().T, x.double().abs() @ w[finite].double().abs().T
     assert bool(((got[:, finite].double() - ref).abs() <= 2.0**-21 * size).all())
     assert not bool(got[:, ~finite].isfinite().any())
+
+
+# forms of up to 16 rows (the last two share their activations through LDS), from 17 rows on, cut along k or not; k that ends
+# in the middle of a 64-column piece, and slices without a piece
+@pytest.mark.parametrize("m,k,batch,bits", [(64, 32, 5, 2), (128, 96, 16, 3), (1056, 928, 11, 4), (64, 32, 40, 4), (128, 96, 20, 2),
+                                            (2048, 832, 100, 3), (1056, 928, 200, 2), (4096, 11040, 45, 2), (5632, 992, 1000, 4),
+                                            (32768, 4128, 6, 4), (32768, 4128, 16, 3)])
+@pytest.mark.parametrize("entry", [0, 5])
+def test_infinities_are_those_of_the_product(m, k, batch, bits, entry):
+    """One infinite value in the table: rows that hold it give the infinity, or NaN where two meet with opposite signs, as
+    the product of the decoded matrix does, and nothing outside the matrix adds to them."""
+    from qtip_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(k + batch)
+    packed = torch.randint(-32768, 32768, (m * k * bits // 16,), dtype=torch.int16, generator=g, device="cuda")
+    tlut = torch.randn(512, 2, generator=g, device="cuda").half()
+    tlut[entry, 0] = float("inf")
+    w = ops.decode(packed, tlut.reshape(-1), m, k, bits)
+    x = torch.randn(batch, k, generator=g, device="cuda").half()
+    x[x == 0] = 1
+    got = ops.decompress_gemm(packed, x, tlut.reshape(-1), m, k, bits, round_f16=False)
+    pos, neg = (x > 0).float(), (x < 0).float()
+    wp, wn = (w == float("inf")).float(), (w == -float("inf")).float()
+    up = (pos @ wp.T + neg @ wn.T) > 0
+    down = (pos @ wn.T + neg @ wp.T) > 0
+    fine = ~(up | down)
+    assert bool((up ^ down).any())
+    assert bool(got[up & down].isnan().all())
+    assert bool((got[up & ~down] == float("inf")).all()) and bool((got[down & ~up] == -float("inf")).all())
+    wf = w.double().nan_to_num(0, 0, 0)
+    ref, size = x.double() @ wf.T, x.double().abs() @ wf.abs().T
+    assert bool(((got.double() - ref).abs() <= 2.0**-21 * size)[fine].all())
