@@ -181,7 +181,8 @@ size_t qtip_gemm_workspace_bytes(int m, int k, int bits, int batch);
  * (lib/codebook/bitshift.py:476-489).  1 <= batch <= 65535.
  * Matrices with few rows are also cut along k; the fp32 partial results then pass through
  * `workspace` (qtip_gemm_workspace_bytes, no initialisation needed, 16-byte aligned) and one
- * more small launch adds them in a fixed order.  workspace may be NULL: k is then never split. */
+ * more small launch adds them in a fixed order.  workspace may be NULL: k is then never split.
+ * The fp32 sums are cut finely, into 2 to 8 slices and ranges of 512 to 1024 columns, whatever the number of rows. */
 int qtip_decompress_gemm(float* out, const void* packed, const void* x_f16,
                          const void* tlut, int m, int k, int bits, int batch,
                          int round_f16, void* workspace, size_t workspace_bytes, void* stream);
@@ -191,6 +192,14 @@ int qtip_decompress_gemm(float* out, const void* packed, const void* x_f16,
 int qtip_decompress_gemm_f16(void* out_f16, const void* packed, const void* x_f16, const void* tlut, int m,
                              int k, int bits, int batch, void* workspace, size_t workspace_bytes,
                              void* stream);
+
+/* The same for many rows (a prompt, a training batch), faster: fp32 sums in chains as long as those of a library product of
+ * the dense matrix, k / 32 additions at most.  From some 200 rows on the difference is before the rounding to fp16
+ * (2 to 8e-7 of the result against 1 to 3e-7; the rounding itself is 2.07e-4). */
+size_t qtip_gemm_long_workspace_bytes(int m, int k, int bits, int batch);
+int qtip_decompress_gemm_long_f16(void* out_f16, const void* packed, const void* x_f16, const void* tlut, int m,
+                                  int k, int bits, int batch, void* workspace, size_t workspace_bytes,
+                                  void* stream);
 
 /* A whole quantized projection (lib/codebook/bitshift.py:415-472 with rcp 0): out[rows][m] in x's dtype =
  * sv * scale_out * H_out(fp16(scale_in * H_in(su * x)) @ decode(packed)^T), H of order_in x k / order_in and
@@ -204,6 +213,12 @@ int qtip_linear(void* out, const void* x, int x_dtype, const void* packed, const
                 const float* sv, const uint32_t* had_in, int order_in, const uint32_t* had_out, int order_out, int m,
                 int k, int bits, int rows, float scale_in, float scale_out, void* workspace, size_t workspace_bytes,
                 void* stream);
+/* The same with the product of qtip_decompress_gemm_long_f16 (from two rows on). */
+size_t qtip_linear_long_workspace_bytes(int m, int k, int bits, int rows, int order_in, int x_dtype);
+int qtip_linear_long(void* out, const void* x, int x_dtype, const void* packed, const void* tlut, const void* su_f16,
+                     const float* sv, const uint32_t* had_in, int order_in, const uint32_t* had_out, int order_out, int m,
+                     int k, int bits, int rows, float scale_in, float scale_out, void* workspace, size_t workspace_bytes,
+                     void* stream);
 
 /* The HYB table (quantlut_sym): tlut is (2^nbits, 2), contiguous; lut holds the value pair of every 16-bit state,
  * value v of state s at element s * stride_s + v * stride_v.  dtype: of both tables (expand), of lut (fold: nbits is

@@ -50,10 +50,17 @@ _SIGNATURES = {
                              [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "qtip_decompress_gemm_f16": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 +
                                  [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "qtip_gemm_long_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 4),
+    "qtip_decompress_gemm_long_f16": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 +
+                                      [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "qtip_linear_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 6),
     "qtip_linear": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] + [ctypes.c_void_p] * 5 +
                     [ctypes.c_int, ctypes.c_void_p] + [ctypes.c_int] * 5 + [ctypes.c_float] * 2 +
                     [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "qtip_linear_long_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 6),
+    "qtip_linear_long": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] + [ctypes.c_void_p] * 5 +
+                         [ctypes.c_int, ctypes.c_void_p] + [ctypes.c_int] * 5 + [ctypes.c_float] * 2 +
+                         [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "qtip_expand_table": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2 + [ctypes.c_long] * 2 +
                           [ctypes.c_void_p]),
     "qtip_fold_table": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] + [ctypes.c_long] * 2 + [ctypes.c_void_p]),

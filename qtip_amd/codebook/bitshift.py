@@ -296,7 +296,7 @@ class BitshiftLinear(nn.Module):
             y = ops.linear(_contiguous(x), _contiguous(trellis), self._tlut16(dev), _contiguous(SU), _contiguous(SV),
                            had_bits(had_left, K_left, True, dev) if K_left > 1 else None, K_left,
                            had_bits(had_right, K_right, False, dev) if K_right > 1 else None, K_right,
-                           m, n, self.cb.K, (n**-0.5) / self.scale, (m**-0.5) * self.scale)
+                           m, n, self.cb.K, (n**-0.5) / self.scale, (m**-0.5) * self.scale, self._long_sums(bs, m, n))
             return y if flat else y.view(*input.shape[:-1], m)
 
         # ---- input transform: fp16(H_L^T (x * SU) / sqrt(n) / 32)
@@ -393,10 +393,17 @@ class BitshiftLinear(nn.Module):
         """The product of `rows` rows decodes an (m, n) matrix to dense fp16 and hands it to the BLAS library."""
         return self._takes_dense(rows, m, n, self.dense_rows_min)
 
+    @classmethod
+    def _long_sums(cls, rows, m, n):
+        """A product of so many rows that it would otherwise be the BLAS library's, as the reference's is for every batch,
+        may sum in chains as long (ops.decompress_gemm); fewer rows keep the fine sums."""
+        return rows >= cls._dense_rows_from(m, n, _DENSE_ROWS_MIN)
+
     def rows_product(self, xt, trellis, tlut, m, n):
         """(rows, m) fp16 = xt (rows, n) fp16 @ decode(trellis)^T, for two rows or more."""
         if not self.takes_dense(xt.shape[0], m, n):
-            return ops.decompress_gemm(trellis.reshape(-1), xt, tlut, m, n, self.cb.K, out_dtype=torch.float16)
+            return ops.decompress_gemm(trellis.reshape(-1), xt, tlut, m, n, self.cb.K, out_dtype=torch.float16,
+                                       long_sums=self._long_sums(xt.shape[0], m, n))
         # decode once to dense fp16 and let the BLAS library multiply, which is what the reference does
         # for every batch (bitshift.py:476-489); fp16, which the output transform takes as it is
         return xt @ ops.decode(trellis.reshape(-1), tlut.reshape(-1), m, n, self.cb.K).T
@@ -442,7 +449,8 @@ class BitshiftLinearKernelAG(torch.autograd.Function):
             y = ops.decompress_matvec(trellis.reshape(-1), x.reshape(-1), tlut.reshape(-1), m, n, K).view(1, m)
             y = y.to(torch.float16)
         elif not BitshiftLinear._takes_dense(x.shape[0], m, n, BitshiftLinear.dense_rows_min):
-            y = ops.decompress_gemm(trellis.reshape(-1), x, tlut.reshape(-1), m, n, K, out_dtype=torch.float16)
+            y = ops.decompress_gemm(trellis.reshape(-1), x, tlut.reshape(-1), m, n, K, out_dtype=torch.float16,
+                                    long_sums=BitshiftLinear._long_sums(x.shape[0], m, n))
         else:
             y = x @ ops.decode(trellis.reshape(-1), tlut.reshape(-1), m, n, K).T
         return y.view(*input.shape[:-1], m)

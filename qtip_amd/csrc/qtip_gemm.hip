@@ -25,35 +25,40 @@ namespace {
 // and twice the accumulators.)  The successor chunk a lane's last reference lane needs sits 16 lanes
 // away or one row on: ds_bpermute.
 //
-// Three kernels: gemm_few_kernel and gemm_kernel up to 16 batch rows, gemm_rows_kernel beyond.  S > 1 (few units of work): k
-// is cut into S ranges, fp32 partial results go to parts[s][batch][m] and are summed afterwards.
+// Three kernels: gemm_few_kernel up to 16 batch rows, gemm_kernel up to 32 (and up to 16 of the largest matrices),
+// gemm_rows_kernel beyond.  S > 1: k is cut into S ranges, fp32 partial results go to parts[s][batch][m] and are summed afterwards.
 constexpr size_t kGemmTileBytes = 32 * 1024;  // beside the table: tiles of activations, sums of slices
 constexpr size_t kGemmLds = kLut128Bytes + kGemmTileBytes;
 
-// Up to 16 batch rows of the largest matrices at 3 and 4 bits (see shared_rows).  A workgroup of 16 waves: two row-block
-// pairs x KS = 8 column slices of 64.  The activations of a stage (16
+// 17 to 32 batch rows (NB = 2), and up to 16 of the largest matrices at 3 and 4 bits (NB = 1, see shared_rows).  A workgroup of 16
+// waves: two row-block pairs x KS = 8 column slices of 64.  The activations of a stage (16 NB
 // batch rows x 512 columns) are shared through LDS, each 16-byte chunk holding the eight values one lane's A operand
-// needs, chunk index xor-ed with the row (conflict-free both ways).  The next tile waits in registers; two tiles in
-// LDS, one barrier per stage.  Work unit = (two pairs, k range s); a workgroup keeps one s, so the pipeline runs
-// across unit boundaries.  The k slices of a unit meet in the tile buffer at its end.
-// Bound by the weight stream (28672x8192 at 4 bits, from cold memory: 28 us, 4.2 TB/s; the matvec 24).
+// needs, chunk index xor-ed with the row (conflict-free both ways).  The next tile waits in registers; with room for two
+// tiles in LDS there is one barrier per stage, else two.  Work unit = (two pairs, k range s); a workgroup keeps one s, so the
+// pipeline runs across unit boundaries.  The k slices of a unit meet in the tile buffer at its end.
+// NB = 1 is bound by the weight stream, NB = 2 by its stages' phases.  The forms of gemm_rows_kernel at 17 to 32 rows have
+// half the slices: within what eight of them are off by (fine_error) they take 0.9 to 1.6 times as long, with chains twice as
+// long 0.87 to 1.08.  us from cold memory, launches and sums of ranges included, 32 rows at 2 bits: 4096x4096 13.4,
+// 22016x4096 19.9, 28672x8192 34, 4096x11008 17.1, 8192x28672 35.
 constexpr int kWaves = 16, kThreads = 64 * kWaves;
 
-template <int K, typename TOut>
+// CUT: k / 32 is odd.  (Looking for the last wave-load in a kernel of its own: 2 % at 17 to 32 rows, 7 % at 28672x8192.)
+template <int K, int NB, bool CUT, typename TOut>
 __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
     TOut* __restrict__ dst, const uint8_t* __restrict__ packed, const uint16_t* __restrict__ x,
     const uint32_t* __restrict__ tlut, int m, int k, int batch, long ldo, int round_f16, int wl_per, int upw_q, int upw_r) {
-  constexpr int NB = 1, WAVES = kWaves, RG = 2, THREADS = kThreads, DEPTH = 2;
+  constexpr int WAVES = kWaves, RG = 2, THREADS = kThreads, DEPTH = 2;
   constexpr int KS = WAVES / RG;
   constexpr int ROWB = KS * 128;               // bytes per tile row
   constexpr int CPR = ROWB / 16;               // 16-byte chunks per tile row
   constexpr uint32_t TILE = 16 * NB * ROWB;
+  constexpr bool DB = 2 * TILE <= kGemmTileBytes;  // two tiles fit
   constexpr int CHUNKS = 16 * NB * CPR;
   constexpr int NX = (CHUNKS + THREADS - 1) / THREADS;  // chunks per thread
-  static_assert(2 * TILE <= kGemmTileBytes, "two tiles do not fit");
+  static_assert(TILE <= kGemmTileBytes && TILE >= WAVES * 1024, "the tile, or the exchange in it, does not fit");
   extern __shared__ __align__(16) uint8_t smem[];
   uint32_t* lut = reinterpret_cast<uint32_t*>(smem);
-  uint8_t* tile = smem + kLut128Bytes;  // [2][16 rows][ROWB bytes]
+  uint8_t* tile = smem + kLut128Bytes;  // [1 or 2][16*NB rows][ROWB bytes]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rg = wave % RG, ks = wave / RG;
@@ -171,7 +176,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
     for (int d = 0; d < DEPTH; ++d) {
       // (an odd last stage: nothing to multiply, but its loads and barriers stay unconditional - see load_tile)
       const bool live = q + d < T;  // uniform over the workgroup
-      const uint32_t cb = (uint32_t)(d & 1) * TILE;  // this stage's tile
+      const uint32_t cb = DB ? (uint32_t)(d & 1) * TILE : 0u;  // this stage's tile
       if (live) {
         const int pair = c_u * RG + rg;
         const int wl = wl0 + KS * c_t + ks;
@@ -195,11 +200,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
                   const int wi = w_index<K>(R, 2 * kh + mh, j);  // register wi / 2, half wi % 2
                   W[mh][rh][w] = lds_word_abs((wi & 1) ? lut128_addr_hi(Q[wi >> 1], slot4) : lut128_addr_lo(Q[wi >> 1], slot4));
                 }
-            if ((nkb & 1) && wl == nwl - 1) {
+            if constexpr (CUT) {
               // no second column block: its zeros decode to table entry 0, which zero activations do not cancel if
               // it is infinite
+              if (wl == nwl - 1) {
 #pragma unroll
-              for (int i = 0; i < 16; ++i) (&W[0][0][0])[i] = g0 ? 0u : (&W[0][0][0])[i];
+                for (int i = 0; i < 16; ++i) (&W[0][0][0])[i] = g0 ? 0u : (&W[0][0][0])[i];
+              }
             }
             __builtin_amdgcn_sched_barrier(0);
             const uint32_t ca = tile_addr + cb + ((((uint32_t)(8 * ks + 4 * g0 + 2 * kh + ch)) ^ a7) << 4);
@@ -223,17 +230,18 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
         int t2 = c_t + 2;  // the tile that replaces the next one in its registers
         if (t2 >= nst) t2 -= nst;
         if (t2 >= nst) t2 -= nst;  // nst == 1
-        // the next tile (in registers since the previous stage) into the other buffer, the one after it on its way
-        store_tile((uint32_t)((d + 1) & 1) * TILE);
-        load_tile(t2);
-        issue(d);
-        __syncthreads();  // every wave has read this stage's tile and written the next
+        if constexpr (DB) {
+          // the next tile (in registers since the previous stage) into the other buffer, the one after it on its way
+          store_tile((uint32_t)((d + 1) & 1) * TILE);
+          load_tile(t2);
+          issue(d);
+        }
+        __syncthreads();  // every wave has read this stage's tile (and, with two buffers, written the next)
         const bool unit_end = live && c_t + 1 == nst;
         if (unit_end) {
           // ---- end of a unit: the k slices meet in this stage's tile buffer, TI accumulator vectors of every
           // wave at a time, summed in slice order
           constexpr int TI = TILE / (WAVES * 1024);  // vectors that fit
-          static_assert(WAVES * TI * 1024 <= TILE, "the exchange does not fit");
           float* xch = reinterpret_cast<float*>(tile + cb);
           const float4_t* av = &acc[0][0][0];
 #pragma unroll
@@ -269,6 +277,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
           c_u += ustep;
         }
         c_t = unit_end ? 0 : c_t + (live ? 1 : 0);
+        if constexpr (!DB) {
+          store_tile(0);
+          load_tile(t2);
+          issue(d);
+          __syncthreads();  // the next tile is complete
+        }
       }
     }
   }
@@ -300,13 +314,14 @@ void launch_gemm(const GemmPlan& g, T* dst, long ldo, const uint8_t* p, const ui
   const int per = (int)(cus / g.S < units ? cus / g.S : units);  // workgroups per k range
   const dim3 grid((unsigned)g.S, (unsigned)per);
   const int uq = (int)(units / per), ur = (int)(units % per);
-  if constexpr (K > 2) {
-    if (g.NB == 1) {
-      gemm_kernel<K, T><<<grid, kThreads, kGemmLds, st>>>(dst, p, x, t, m, k, nb, ldo, round_f16, g.wl_per, uq, ur);
-      return;
-    }
+  if (g.form == kShared) {
+    auto* kernel = (k >> 5) & 1 ? gemm_kernel<K, 2, true, T> : gemm_kernel<K, 2, false, T>;
+    if constexpr (K > 2)
+      if (g.NB == 1) kernel = (k >> 5) & 1 ? gemm_kernel<K, 1, true, T> : gemm_kernel<K, 1, false, T>;
+    kernel<<<grid, kThreads, kGemmLds, st>>>(dst, p, x, t, m, k, nb, ldo, round_f16, g.wl_per, uq, ur);
+    return;
   }
-  if (g.NB == 0) {
+  if (g.form == kFew) {
     if (g.RG == 2)
       gemm_few_kernel<K, 2, T><<<grid, 64 * kFewWaves, kGemmLds, st>>>(dst, p, x, t, m, k, nb, ldo, round_f16, g.wl_per, uq, ur);
     else
@@ -342,7 +357,7 @@ void launch_gemm(int bits, const GemmPlan& g, T* dst, long ldo, const uint8_t* p
   }
 }
 
-template <typename TOut>
+template <typename TOut, bool kFine = true>
 int run_gemm(TOut* out, const void* packed, const void* x_f16, const void* tlut, int m, int k, int bits, int batch,
                     int round_f16, void* workspace, size_t workspace_bytes, void* stream) {
   int rc = check_common(out, packed, x_f16, tlut, m, k, bits);
@@ -354,16 +369,16 @@ int run_gemm(TOut* out, const void* packed, const void* x_f16, const void* tlut,
   int cus = 0;
   rc = qtip_device_ready(stream, &cus);
   if (rc) return rc;
+  const bool split = workspace != nullptr;
   if (workspace) {
-    if (workspace_bytes < qtip_gemm_workspace_bytes(m, k, bits, batch)) return QTIP_E_WORKSPACE;
+    if (workspace_bytes < qtip_gemm_scratch(m, k, bits, batch, kFine)) return QTIP_E_WORKSPACE;
     if (!aligned16(workspace)) return QTIP_E_ALIGN;
   }
   hipStream_t st = (hipStream_t)stream;
   auto* t = (const uint32_t*)tlut;
-  const int step = pass_rows(k);
-  for (int b0 = 0; b0 < batch; b0 += step) {
-    const int nb = batch - b0 < step ? batch - b0 : step;
-    const GemmParts parts = gemm_plan(m, k, bits, nb, cus, workspace != nullptr);
+  for (int b0 = 0, nb; b0 < batch; b0 += nb) {
+    nb = next_pass(m, k, bits, batch - b0, cus, split, kFine);
+    const GemmParts parts = gemm_plan(m, k, bits, nb, cus, split, kFine);
     const uint16_t* xx = (const uint16_t*)x_f16 + (size_t)b0 * k;
     for (int part = 0; part < 2; ++part) {
       const int first = part ? parts.m0 : 0, rows = part ? m - parts.m0 : parts.m0;
@@ -396,6 +411,8 @@ hipError_t qtip_gemm_allow_lds() {
                                (int)bytes)) != hipSuccess)                                                       \
     return e;
 #define QTIP_ALLOW_GEMM(KB, T)                        \
+  QTIP_ALLOW((gemm_kernel<KB, 2, false, T>), kGemmLds)  \
+  QTIP_ALLOW((gemm_kernel<KB, 2, true, T>), kGemmLds)   \
   QTIP_ALLOW((gemm_few_kernel<KB, 1, T>), kGemmLds)     \
   QTIP_ALLOW((gemm_few_kernel<KB, 2, T>), kGemmLds)     \
   QTIP_ALLOW((gemm_rows_kernel<KB, 8, 8, T>), kGemmLds) \
@@ -412,53 +429,63 @@ hipError_t qtip_gemm_allow_lds() {
   QTIP_ALLOW_GEMM(2, _Float16)
   QTIP_ALLOW_GEMM(3, _Float16)
   QTIP_ALLOW_GEMM(4, _Float16)
-  QTIP_ALLOW((gemm_kernel<3, float>), kGemmLds)
-  QTIP_ALLOW((gemm_kernel<4, float>), kGemmLds)
-  QTIP_ALLOW((gemm_kernel<3, _Float16>), kGemmLds)
-  QTIP_ALLOW((gemm_kernel<4, _Float16>), kGemmLds)
+#define QTIP_ALLOW_SHARED(KB, CUTV)                     \
+  QTIP_ALLOW((gemm_kernel<KB, 1, CUTV, float>), kGemmLds) \
+  QTIP_ALLOW((gemm_kernel<KB, 1, CUTV, _Float16>), kGemmLds)
+  QTIP_ALLOW_SHARED(3, false)
+  QTIP_ALLOW_SHARED(3, true)
+  QTIP_ALLOW_SHARED(4, false)
+  QTIP_ALLOW_SHARED(4, true)
+#undef QTIP_ALLOW_SHARED
 #undef QTIP_ALLOW_GEMM
 #undef QTIP_ALLOW
   return hipSuccess;
 }
 
-int qtip_gemm_ranges(int m, int k, int bits, int batch) {
+int qtip_gemm_ranges(int m, int k, int bits, int batch, bool fine) {
   const int cus = qtip_device_cus();
-  if (!cus || batch > pass_rows(k)) return 1;
-  const GemmParts p = gemm_plan(m, k, bits, batch, cus, true);
+  if (!cus || next_pass(m, k, bits, batch, cus, true, fine) != batch) return 1;
+  const GemmParts p = gemm_plan(m, k, bits, batch, cus, true, fine);
   return p.m0 == m ? p.first.S : 1;
 }
 
 int qtip_gemm_parts(float* parts, int nparts, const void* packed, const void* x_f16, const void* tlut, int m, int k, int bits,
-                    int batch, void* stream) {
+                    int batch, bool fine, void* stream) {
   int rc = check_common(parts, packed, x_f16, tlut, m, k, bits);
   if (rc) return rc;
   if (!aligned16(packed) || !aligned16(x_f16) || !aligned16(parts) || (reinterpret_cast<uintptr_t>(tlut) & 3u)) return QTIP_E_ALIGN;
   int cus = 0;
   rc = qtip_device_ready(stream, &cus);
   if (rc) return rc;
-  const GemmParts p = gemm_plan(m, k, bits, batch, cus, true);
-  if (p.m0 != m || p.first.S < 2 || p.first.S != nparts || batch > pass_rows(k)) return QTIP_E_SHAPE;
-  launch_gemm<float>(bits, p.first, parts, m, (const uint8_t*)packed, (const uint16_t*)x_f16, (const uint32_t*)tlut, m, k, batch,
-                     0, cus, (hipStream_t)stream);
+  if (next_pass(m, k, bits, batch, cus, true, fine) != batch) return QTIP_E_SHAPE;
+  const GemmParts p = gemm_plan(m, k, bits, batch, cus, true, fine);
+  if (p.m0 != m || p.first.S < 2 || p.first.S != nparts) return QTIP_E_SHAPE;
+  launch_gemm<float>(bits, p.first, parts, m, (const uint8_t*)packed, (const uint16_t*)x_f16, (const uint32_t*)tlut, m, k, batch, 0, cus,
+                     (hipStream_t)stream);
   return (int)hipGetLastError();
 }
 
-extern "C" {
-
-size_t qtip_gemm_workspace_bytes(int m, int k, int bits, int batch) {
+size_t qtip_gemm_scratch(int m, int k, int bits, int batch, bool fine) {
   if (m <= 0 || k <= 0 || (m & 31) || (k & 31) || bits < 2 || bits > 4 || batch < 1) return 0;
   const int cus = qtip_device_cus();
   if (!cus) return 0;
-  size_t need = 0;  // the largest pass: full ones and the remainder
-  const int step = pass_rows(k);
-  for (int nb : {batch < step ? batch : step, batch % step}) {
-    if (nb < 1) continue;
-    const GemmParts p = gemm_plan(m, k, bits, nb, cus, true);
+  size_t need = 0;
+  for (int b0 = 0, nb, seen = 0; b0 < batch; b0 += nb) {
+    nb = next_pass(m, k, bits, batch - b0, cus, true, fine);
+    if (nb == seen) continue;
+    seen = nb;
+    const GemmParts p = gemm_plan(m, k, bits, nb, cus, true, fine);
     for (size_t bytes : {parts_bytes(p.first, p.m0, nb), p.m0 < m ? parts_bytes(p.rest, m - p.m0, nb) : 0})
       need = bytes > need ? bytes : need;
   }
   return need;
 }
+
+extern "C" {
+
+size_t qtip_gemm_workspace_bytes(int m, int k, int bits, int batch) { return qtip_gemm_scratch(m, k, bits, batch, true); }
+
+size_t qtip_gemm_long_workspace_bytes(int m, int k, int bits, int batch) { return qtip_gemm_scratch(m, k, bits, batch, false); }
 
 int qtip_decompress_gemm(float* out, const void* packed, const void* x_f16, const void* tlut, int m, int k, int bits,
                          int batch, int round_f16, void* workspace, size_t workspace_bytes, void* stream) {
@@ -469,6 +496,12 @@ int qtip_decompress_gemm_f16(void* out_f16, const void* packed, const void* x_f1
                              int batch, void* workspace, size_t workspace_bytes, void* stream) {
   return run_gemm<_Float16>((_Float16*)out_f16, packed, x_f16, tlut, m, k, bits, batch, 1, workspace, workspace_bytes,
                             stream);
+}
+
+int qtip_decompress_gemm_long_f16(void* out_f16, const void* packed, const void* x_f16, const void* tlut, int m, int k,
+                                  int bits, int batch, void* workspace, size_t workspace_bytes, void* stream) {
+  return run_gemm<_Float16, false>((_Float16*)out_f16, packed, x_f16, tlut, m, k, bits, batch, 1, workspace, workspace_bytes,
+                                   stream);
 }
 
 }  // extern "C"

@@ -1,4 +1,4 @@
-// Batched decompress + fp16 MFMA GEMM from 17 batch rows on.  Included by qtip_gemm.hip inside its namespace.
+// Batched decompress + fp16 MFMA GEMM from 33 batch rows on.  Included by qtip_gemm.hip inside its namespace.
 //
 // The matrix cores do not wait for the decode: a wave multiplies one column half (16 of the 32
 // columns of either tile block, 16 table words) while it looks up the words of the next, and the instructions of
@@ -20,12 +20,14 @@
 // A wave-load of NB batch tiles takes about 0.64 + 0.099 NB us on a full chip, where the matrix cores alone need
 // 0.107 NB at 2.4 GHz and the decode by itself 0.53: it is bound by issue (95 vector instructions beside 8 NB products
 // a wave-load, a product taking the slots of two) and, with every CU busy, by the clock: 1024 rows of 8192x8192 run at
-// 1.18 PFLOP/s, the library's product of the decoded matrix at 1.20.  us per product, decode and sums included: before
-// (passes of 128 rows; from 193 to 514 rows on dense decode + library) / here, 2 bits:
-//   4096x4096     48 rows 15.6 / 13.4, 128 32 / 17, 256 35 / 20, 1000 54 / 43, 2000 73 / 66
-//   22016x4096    48 rows 29.1 / 26.1, 128 54 / 38, 256 105 / 55, 1000 205 / 181, 2000 446 / 317
-//   28672x8192    48 rows 51 / 45, 128 90 / 69, 256 178 / 109, 1000 469 / 413, 2000 801 / 770
-//   4096x11008    48 rows 21.7 / 19.5, 128 42 / 28, 256 73 / 40, 1000 125 / 91, 2000 189 / 156
+// 1.18 PFLOP/s, the library's product of the decoded matrix at 1.20.  us per product from cold memory, launches
+// and sums of ranges included, 2 bits: a kernel that decodes, then multiplies between two barriers, in passes of 128 rows / here
+// with fine sums / with long ones (qtip_gemm_plan.h):
+//   4096x4096     45 rows 15.5 / 15.8 / 13.0, 128 31 / 19 / 17, 250 60 / 30 / 20, 1000 242 / 118 / 41
+//   22016x4096    45 rows 28.3 / 26.2 / 25.6, 128 54 / 43 / 39, 250 106 / 74 / 55, 1000 423 / 291 / 180
+//   28672x8192    45 rows 51 / 45 / 45, 128 91 / 70 / 69, 250 177 / 128 / 108, 1000 704 / 522 / 415
+//   4096x11008    45 rows 20.7 / 20.0 / 18.7, 128 38 / 28 / 27, 250 73 / 47 / 38, 1000 291 / 186 / 90
+//   8192x28672    45 rows 50 / 47 / 44, 128 84 / 68 / 67, 250 168 / 122 / 111, 1000 655 / 488 / 407
 
 template <int K>
 struct SlotMap {  // slot r = 0..7 of a column half kh: register of P, and where its two halves' words go

@@ -21,12 +21,15 @@ QTIP_INTERNAL hipError_t qtip_gemm_allow_lds();
 // A product cut along k that leaves its partial sums, and the transform that adds them on load (qtip_linear): the number of
 // ranges of the one launch of such a product (1: it is not cut, or runs in several launches), the launch, whether the transform
 // takes them, and its launch.
-QTIP_INTERNAL int qtip_gemm_ranges(int m, int k, int bits, int batch);
+QTIP_INTERNAL int qtip_gemm_ranges(int m, int k, int bits, int batch, bool fine);
 QTIP_INTERNAL int qtip_gemm_parts(float* parts, int nparts, const void* packed, const void* x_f16, const void* tlut, int m,
-                                  int k, int bits, int batch, void* stream);
+                                  int k, int bits, int batch, bool fine, void* stream);
 QTIP_INTERNAL bool qtip_rht_takes_parts(int n, int order, int rows, int nparts);
 QTIP_INTERNAL int qtip_rht_from_parts(void* out, int out_dtype, const float* parts, int nparts, int rows, int n, int order,
                                       const uint32_t* had_bits, const float* post, float scale, void* stream);
+
+// Scratch of a batched product with fine or with long sums (qtip_decompress_gemm, qtip_decompress_gemm_long_f16)
+QTIP_INTERNAL size_t qtip_gemm_scratch(int m, int k, int bits, int batch, bool fine);
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -282,9 +282,10 @@ def decompress_matvec_group(packed, x, tlut, m, k, bits, nparts=None):
     return parts
 
 
-def decompress_gemm(packed, x, tlut, m, k, bits, round_f16=True, out_dtype=torch.float32):
+def decompress_gemm(packed, x, tlut, m, k, bits, round_f16=True, out_dtype=torch.float32, long_sums=False):
     """(batch, m) = x[batch,k] (fp16) @ decode(packed)[m,k]^T on the matrix cores: fp32, rounded through
-    fp16 on request, or with out_dtype=torch.float16 the rounded values themselves."""
+    fp16 on request, or with out_dtype=torch.float16 the rounded values themselves.  long_sums (fp16 results only): many
+    rows faster, with fp32 sums in chains as long as those of a library product."""
     _check_packed(packed, m, k, bits)
     _check_tlut(tlut, packed.device)
     require_cuda(x, "x", torch.float16)
@@ -292,21 +293,24 @@ def decompress_gemm(packed, x, tlut, m, k, bits, round_f16=True, out_dtype=torch
         raise ValueError(f"x must be (batch, {k}) fp16 on {packed.device}")
     if out_dtype not in _DT or (out_dtype == torch.float16 and not round_f16):
         raise ValueError("results are fp32, or fp16 when they are rounded")
+    if long_sums and out_dtype != torch.float16:
+        raise ValueError("long sums are for fp16 results")
     batch = x.shape[0]
     out = torch.empty((batch, m), dtype=out_dtype, device=packed.device)
     if batch == 0:
         return out
     L = lib()
     with _on(packed.device):
-        need = L.qtip_gemm_workspace_bytes(m, k, bits, batch)
+        need = (L.qtip_gemm_long_workspace_bytes if long_sums else L.qtip_gemm_workspace_bytes)(m, k, bits, batch)
         stream = stream_ptr(packed.device)
         wsp, wsb = None, 0
         if need:
             ws = _workspace(packed.device, need, stream)
             wsp, wsb = _ptr(ws), ws.numel()
         if out_dtype == torch.float16:
-            check(L.qtip_decompress_gemm_f16(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, batch, wsp, wsb,
-                                             stream), "qtip_decompress_gemm_f16")
+            product = L.qtip_decompress_gemm_long_f16 if long_sums else L.qtip_decompress_gemm_f16
+            check(product(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, batch, wsp, wsb, stream),
+                  "qtip_decompress_gemm_f16")
         else:
             check(L.qtip_decompress_gemm(_ptr(out), _ptr(packed), _ptr(x), _ptr(tlut), m, k, bits, batch,
                                          int(bool(round_f16)), wsp, wsb, stream), "qtip_decompress_gemm")
@@ -342,11 +346,11 @@ def _order_ok(t, order, n):
         and t.numel() * 32 >= order * order))
 
 
-def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out):
+def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out, long_sums=False):
     """A whole quantized projection in one call of the library: out (rows, m) in x's dtype = sv * scale_out * H_out(
     fp16(scale_in * H_in(su * x)) @ decode(packed)^T) for x (rows, k) fp16 / fp32; the launches, and the results bit
     for bit, of rht, decompress_matvec_parts[_rht] (one row) or decompress_gemm (more), rht.  had_in / had_out: sign
-    bits of the table orders (None for order 1)."""
+    bits of the table orders (None for order 1).  long_sums: the product is decompress_gemm's with long sums."""
     # a call whose operands fit asks no more than this; what does not goes through the checks one by one
     if not (isinstance(x, _Tensor) and isinstance(packed, _Tensor) and isinstance(tlut, _Tensor)
             and isinstance(su, _Tensor) and isinstance(sv, _Tensor) and packed.is_cuda
@@ -367,11 +371,13 @@ def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, 
     L = lib()
     with _on(dev):
         stream = stream_ptr(dev)
-        need = L.qtip_linear_workspace_bytes(m, k, bits, rows, order_in, dt)
+        size, run = ((L.qtip_linear_long_workspace_bytes, L.qtip_linear_long) if long_sums else
+                     (L.qtip_linear_workspace_bytes, L.qtip_linear))
+        need = size(m, k, bits, rows, order_in, dt)
         ws = torch.empty(need, dtype=torch.uint8, device=dev)
-        check(L.qtip_linear(out.data_ptr(), x.data_ptr(), dt, packed.data_ptr(), tlut.data_ptr(), su.data_ptr(),
-                            sv.data_ptr(), _ptr(had_in), order_in, _ptr(had_out), order_out, m, k, bits, rows, scale_in,
-                            scale_out, ws.data_ptr(), need, stream), "qtip_linear")
+        check(run(out.data_ptr(), x.data_ptr(), dt, packed.data_ptr(), tlut.data_ptr(), su.data_ptr(),
+                  sv.data_ptr(), _ptr(had_in), order_in, _ptr(had_out), order_out, m, k, bits, rows, scale_in,
+                  scale_out, ws.data_ptr(), need, stream), "qtip_linear")
     return out
 
 

@@ -11,10 +11,18 @@ CUS = 256
 SHIM = r"""
 #include "qtip_gemm_plan.h"
 using namespace qtip;
-extern "C" void plan_of(int m, int k, int bits, int nb, int cus, int split, int* out) {
-  const GemmParts p = gemm_plan(m, k, bits, nb, cus, split);
-  const int v[] = {p.m0, p.first.NB, p.first.RG, p.first.S, p.first.wl_per, p.rest.NB, p.rest.RG, p.rest.S, p.rest.wl_per};
-  for (int i = 0; i < 9; ++i) out[i] = v[i];
+static void put(const GemmPlan& g, int* out) {
+  const int v[] = {g.form, g.NB, g.RG, g.S, g.wl_per};
+  for (int i = 0; i < 5; ++i) out[i] = v[i];
+}
+extern "C" int plan_of(int m, int k, int bits, int nb, int cus, int split, int fine, int* out) {
+  const GemmParts p = gemm_plan(m, k, bits, nb, cus, split, fine);
+  put(p.first, out);
+  put(p.rest, out + 5);
+  return p.m0;
+}
+extern "C" int pass_of(int m, int k, int bits, int left, int cus, int split, int fine) {
+  return next_pass(m, k, bits, left, cus, split, fine);
 }
 extern "C" void few_place(int lane, int batch, int k, int wl, int units, int nst, int last_half, uint32_t* out) {
   const FewPlace p = few_activations(lane, batch, k, wl, units, nst, last_half);
@@ -22,21 +30,23 @@ extern "C" void few_place(int lane, int batch, int k, int wl, int units, int nst
   out[1] = p.vo;
 }
 """
+FEW, SHARED, ROWS = range(3)
 
 
 @pytest.fixture(scope="module")
 def native(tmp_path_factory):
     d = tmp_path_factory.mktemp("gemm_plan")
     (d / "shim.cpp").write_text(SHIM)
-    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-Wno-unused-function", "-shared", "-fPIC", "-I",
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I",
                     os.path.join(ROOT, "qtip_amd", "csrc"), str(d / "shim.cpp"), "-o", str(d / "shim.so")], check=True)
     return ctypes.CDLL(str(d / "shim.so"))
 
 
-def plan(native, m, k, bits, batch, split=True):
-    out = (ctypes.c_int * 9)()
-    native.plan_of(m, k, bits, batch, CUS, int(split), out)
-    return out[0], tuple(out[1:5]), tuple(out[5:])
+def plan(native, m, k, bits, batch, split=True, fine=True):
+    """Matrix rows of the first launch, (form, NB, RG, S, wl_per) of it and of the second."""
+    out = (ctypes.c_int * 10)()
+    m0 = native.plan_of(m, k, bits, batch, CUS, int(split), int(fine), out)
+    return m0, tuple(out[:5]), tuple(out[5:])
 
 
 @pytest.mark.parametrize("k", [32, 64, 96, 832, 928, 2080, 4096, 28672])
@@ -47,8 +57,8 @@ def test_few_rows_read_their_activations_only(native, m, k):
     place = (ctypes.c_uint32 * 2)()
     nwl, odd = (k // 32 + 1) // 2, k // 32 % 2
     for batch in (2, 5, 16):
-        _, (NB, RG, S, wl_per), _ = plan(native, m, k, 2, batch)
-        assert NB == 0
+        _, (form, _, RG, S, wl_per), _ = plan(native, m, k, 2, batch)
+        assert form == FEW
         KS, size = 16 // RG, batch * k * 2
         for s in sorted({0, S - 1}):
             wl1 = min((s + 1) * wl_per, nwl)
@@ -66,3 +76,46 @@ def test_few_rows_read_their_activations_only(native, m, k):
                             if vo < 0x7FFFFF00 and not (last and t):
                                 assert so + vo + 32 + 16 <= size, (batch, s, ks, lane, t)
                             so += KS * 128
+
+
+def _error(nwl, KS, wl_per, S):
+    """Chains of additions on the matrix cores (which weigh 5), slices (1.5) and ranges (1) of a sum over nwl 64-column pieces."""
+    n = min(wl_per, nwl)
+    return 10 * -(-n // KS) + min(KS, n) * 3 // 2 + S
+
+
+def _cut_error(m, k, batch, split):
+    """_error of the cut that bounds it: passes of 128 rows in 8, 4 or 2 slices and ranges of 1024 or 512 columns."""
+    if batch > 128:
+        return min(_cut_error(m, k, 128, split), _cut_error(m, k, batch - 128, split))
+    KS, RG, least = (8, 2, 16) if batch <= 32 else (4, 2, 8) if batch <= 64 else (2, 4, 8)
+    nwl, groups = (k // 32 + 1) // 2, -(-((m // 32 + 1) // 2) // RG)
+    S = 1
+    while split and S < 16 and groups * S * 2 <= CUS and nwl // (2 * S) >= least:
+        S *= 2
+    wl_per = -(-(-(-nwl // S)) // KS) * KS
+    return _error(nwl, KS, wl_per, -(-nwl // wl_per))
+
+
+@pytest.mark.parametrize("k", [32, 96, 512, 832, 1120, 2048, 3328, 4096, 5504, 8192, 11008, 28672, 1 << 20, 1 << 23])
+def test_sums_are_cut_finely(native, k):
+    """Every pass of a product: chains, slices and ranges no coarser than the bound, with scratch for ranges and without."""
+    nwl = (k // 32 + 1) // 2
+    for m in (32, 96, 512, 992, 1728, 2048, 4096, 6144, 8192, 10240, 11008, 14336, 22016, 28672, 57344):
+        for bits in (2, 4):
+            for batch in (1, 2, 5, 9, 16, 17, 20, 32, 33, 48, 64, 65, 100, 128, 129, 150, 190, 256, 1000):
+                for split in (True, False):
+                    left = batch
+                    while left:
+                        nb = native.pass_of(m, k, bits, left, CUS, int(split), 1)
+                        assert 1 <= nb <= min(left, 256) and nb * k * 2 <= 0x7FFFFF00
+                        m0, (form, NB, RG, S, wl_per), _ = plan(native, m, k, bits, nb, split)
+                        assert m0 == m and RG and (split or S == 1)
+                        KS = (8 if form == ROWS else 16) // RG
+                        assert _error(nwl, KS, wl_per, S) <= _cut_error(m, k, nb, split), (m, bits, batch, nb, split)
+                        left -= nb
+
+
+def test_long_sums_are_longer(native):
+    _, (form, NB, RG, S, wl_per), _ = plan(native, 8192, 28672, 2, 1000, fine=False)
+    assert form == ROWS and _error(448, 8 // RG, wl_per, S) > 2 * _cut_error(8192, 28672, 128, True)

@@ -127,3 +127,28 @@ def test_infinities_are_those_of_the_product(m, k, batch, bits, entry):
     wf = w.double().nan_to_num(0, 0, 0)
     ref, size = x.double() @ wf.T, x.double().abs() @ wf.abs().T
     assert bool(((got.double() - ref).abs() <= 2.0**-21 * size)[fine].all())
+
+
+@pytest.mark.parametrize("m,k,bits", [(8192, 28672, 2), (4096, 4096, 3), (11008, 2048, 4), (28672, 8192, 2)])
+def test_error_of_unrounded_results(m, k, bits):
+    """The 2-norm error of sums cut into S ranges of KS slices of chains of L additions, 1.6e-8 sqrt(5 + 5 L + 1.5 KS + S), at
+    the cut that bounds it (up to 32, 64 and 128 rows 8, 4 and 2 slices; ranges of at least 1024 and 512 columns while they fit
+    256 CUs), with a tenth more for the sample; rounded results are off by their rounding, long sums or not."""
+    from qtip_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(k)
+    packed = torch.randint(-32768, 32768, (m * k * bits // 16,), dtype=torch.int16, generator=g, device="cuda")
+    tlut = torch.randn(1024, generator=g, device="cuda").half()
+    w = ops.decode(packed, tlut, m, k, bits).double()
+    for batch in (2, 16, 24, 40, 100, 300, 1000):
+        x = torch.randn(batch, k, generator=g, device="cuda").half()
+        ref = x.double() @ w.T
+        KS, RG, least = (8, 2, 16) if batch <= 32 else (4, 2, 8) if batch <= 64 else (2, 4, 8)
+        S = 1
+        while S < 16 and -(-m // 64 // RG) * S * 2 <= 256 and k // 64 // (2 * S) >= least:
+            S *= 2
+        bound = 1.1 * 1.6e-8 * (5 + 5 * k / 32 / KS / S + 1.5 * KS + S) ** 0.5
+        y = ops.decompress_gemm(packed, x, tlut, m, k, bits, round_f16=False)
+        assert float((y.double() - ref).norm() / ref.norm()) <= bound, batch
+        for long_sums in (False, True):
+            y = ops.decompress_gemm(packed, x, tlut, m, k, bits, out_dtype=torch.float16, long_sums=long_sums)
+            assert float((y.double() - ref).norm() / ref.norm()) <= 2.1e-4
