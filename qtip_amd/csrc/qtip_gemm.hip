@@ -328,9 +328,10 @@ void launch_gemm(const GemmPlan& g, T* dst, long ldo, const uint8_t* p, const ui
       gemm_few_kernel<K, 1, T><<<grid, 64 * kFewWaves, kGemmLds, st>>>(dst, p, x, t, m, k, nb, ldo, round_f16, g.wl_per, uq, ur);
     return;
   }
-#define QTIP_ROWS(NBV, RGV)                                                                                       \
-  gemm_rows_kernel<K, NBV, RGV, T><<<grid, 64 * kRowsWaves, kGemmLds, st>>>(dst, p, x, t, m, k, nb, g.nbt, ldo,   \
-                                                                            round_f16, g.wl_per, uq, ur)
+  const bool cut = k % (64 * (kRowsWaves / g.RG)) != 0;
+#define QTIP_ROWS(NBV, RGV)                                                                                        \
+  (cut ? gemm_rows_kernel<K, NBV, RGV, true, T> : gemm_rows_kernel<K, NBV, RGV, false, T>)                        \
+      <<<grid, 64 * kRowsWaves, kGemmLds, st>>>(dst, p, x, t, m, k, nb, g.nbt, ldo, round_f16, g.wl_per, uq, ur)
   if (g.NB == 8) {
     if (g.RG == 8) QTIP_ROWS(8, 8);
     else QTIP_ROWS(8, 4);
@@ -415,14 +416,22 @@ hipError_t qtip_gemm_allow_lds() {
   QTIP_ALLOW((gemm_kernel<KB, 2, true, T>), kGemmLds)   \
   QTIP_ALLOW((gemm_few_kernel<KB, 1, T>), kGemmLds)     \
   QTIP_ALLOW((gemm_few_kernel<KB, 2, T>), kGemmLds)     \
-  QTIP_ALLOW((gemm_rows_kernel<KB, 8, 8, T>), kGemmLds) \
-  QTIP_ALLOW((gemm_rows_kernel<KB, 8, 4, T>), kGemmLds) \
-  QTIP_ALLOW((gemm_rows_kernel<KB, 6, 8, T>), kGemmLds) \
-  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 8, T>), kGemmLds) \
-  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 4, T>), kGemmLds) \
-  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 2, T>), kGemmLds) \
-  QTIP_ALLOW((gemm_rows_kernel<KB, 2, 4, T>), kGemmLds) \
-  QTIP_ALLOW((gemm_rows_kernel<KB, 2, 2, T>), kGemmLds)
+  QTIP_ALLOW((gemm_rows_kernel<KB, 8, 8, false, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 8, 8, true, T>), kGemmLds)  \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 8, 4, false, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 8, 4, true, T>), kGemmLds)  \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 6, 8, false, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 6, 8, true, T>), kGemmLds)  \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 8, false, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 8, true, T>), kGemmLds)  \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 4, false, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 4, true, T>), kGemmLds)  \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 2, false, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 4, 2, true, T>), kGemmLds)  \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 2, 4, false, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 2, 4, true, T>), kGemmLds)  \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 2, 2, false, T>), kGemmLds) \
+  QTIP_ALLOW((gemm_rows_kernel<KB, 2, 2, true, T>), kGemmLds)
   QTIP_ALLOW_GEMM(2, float)
   QTIP_ALLOW_GEMM(3, float)
   QTIP_ALLOW_GEMM(4, float)

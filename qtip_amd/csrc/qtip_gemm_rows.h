@@ -41,7 +41,8 @@ struct SlotMap {  // slot r = 0..7 of a column half kh: register of P, and where
   }
 };
 
-template <int K, int NB, int RG, typename TOut>
+// CUT: k ends inside a stage (k no multiple of 64 KS).
+template <int K, int NB, int RG, bool CUT, typename TOut>
 __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
     TOut* __restrict__ dst, const uint8_t* __restrict__ packed, const uint16_t* __restrict__ x,
     const uint32_t* __restrict__ tlut, int m, int k, int batch, int nbt, long ldo, int round_f16, int wl_per, int upw_q,
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
   const int T = upw * nst;
   TOut* out_s = dst + (size_t)s * batch * ldo;
   const int kend = 64 * wl1 < k ? 64 * wl1 : k;
-  const int last_cols = kend - 64 * (wl0 + KS * (nst - 1));  // columns of the last stage, 64 KS if it is whole
+  const int last_cols = CUT ? kend - 64 * (wl0 + KS * (nst - 1)) : 64 * KS;  // columns of the last stage
 
   // ---- units of this workgroup; the weights, the activations and the products each have a place of their own in
   // them, one ahead of the other.  Inside a unit only a scalar offset changes.  (The compiler takes what comes
@@ -108,8 +109,8 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
   // Where a range ends inside a stage, weights and activations there are zeros without a memory access: of every lane in a
   // slice past the end, of the second column block where that is missing.  Such weights would decode to table entry 0,
   // which may be infinite: see cut_words.
-  const bool w_over = wl0 + KS * (nst - 1) + ks >= wl1;
-  const bool w_half = !w_over && (nkb & 1) && wl0 + KS * (nst - 1) + ks == nwl - 1;
+  const bool w_over = CUT && wl0 + KS * (nst - 1) + ks >= wl1;
+  const bool w_half = CUT && !w_over && (nkb & 1) && wl0 + KS * (nst - 1) + ks == nwl - 1;
   const int cut_left = w_over || w_half ? 1 : 0;  // wave-loads to go in a unit where that is so, 0: nowhere
   Unit wu = first;
   int w_left;
@@ -256,9 +257,9 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
   };
   // Before a wave-load that is cut short, with its first half looked up and its states at hand: finite words in place of
   // what meets no activations.  (Words cleared before the products of either half cost every wave-load two branches: 1 % on
-  // average, 5 % at 5120x13824, 128 rows.)
+  // average, 5 % at 128 rows of 5120x13824; this costs 0.7 % at 1000 rows of 4096x22016, so whole stages have kernels without.)
   uint32_t finite = 0;  // a state of a finite table entry, in both halves
-  if (cut_left) {
+  if (CUT && cut_left) {
     for (uint32_t s2 = 0; s2 < 4096u * 0x10001u; s2 += 0x10001u) {
       const uint32_t w = uni(lds_word_abs(lut128_addr_lo(pk_hash(s2) & 0xFFC0FFC0u, slot4)));
       if ((w & 0x7C00u) != 0x7C00u && (w & 0x7C000000u) != 0x7C000000u) {
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
   };
   Unit cu = first;
   int c_left = nst;
-  if (nst == cut_left) cut_words();
+  if (CUT && nst == cut_left) cut_words();
   for (int left = T; left > 0; left -= 2) {
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
       }
       w_next();
       x_next();
-      if (uni(--c_left) > cut_left) continue;
+      if (uni(--c_left) > (CUT ? cut_left : 0)) continue;
       if (c_left == 0) {
         c_left = nst;
         const int pair = cu.g * RG + rg;
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 1) void gemm_rows_kernel(
         for (int i = 0; i < 4 * NB; ++i) (&acc[0][0])[i] = float4_t{0.f, 0.f, 0.f, 0.f};
         advance(cu);
       }
-      if (uni(c_left) == cut_left) cut_words();
+      if (CUT && uni(c_left) == cut_left) cut_words();
     }
   }
 }
