@@ -288,9 +288,11 @@ class BitshiftLinear(nn.Module):
             return torch.cat(outs, dim=0).view(*input.shape[:-1], m)
 
         if (self.has_kernel and rcp not in (1, 2) and not self.takes_dense(bs, m, n) and SU.dtype == torch.float16
-                and SV.dtype == torch.float32 and SV.device == dev and x.dtype in (torch.float16, torch.float32)):
+                and SV.dtype == torch.float32 and SV.device == dev and x.dtype in (torch.float16, torch.float32)
+                and not by_library(bs, n, K_left) and not by_library(bs, m, K_right)):
             # both transforms and the product by one call of the library: what bounds such a call otherwise is the
-            # host.  (Where takes_dense holds the product is the BLAS library's.)  us per call, launch by launch /
+            # host.  (Where takes_dense holds the product is the BLAS library's, where by_library holds a transform is: a
+            # caller's table of order 300, 4800x4800, 1000 rows 435 against 2850 in the one call.)  us, launch by launch /
             # here: 4096x4096, 2 bits, one row 40 / 21; 28672x8192, 4 bits, 16 rows 59 / 43; 4096x11008, 3 bits, 45
             # rows 65 / 32
             y = ops.linear(_contiguous(x), _contiguous(trellis), self._tlut16(dev), _contiguous(SU), _contiguous(SV),

@@ -158,6 +158,30 @@ def test_projection_whose_orders_the_matrix_form_does_not_take(monkeypatch):
     assert len(taken) == 2 and float((got.float() - want.float()).norm() / want.float().norm()) <= 2.0**-10
 
 
+@pytest.mark.parametrize("rows", [150, 300])
+def test_kernel_projection_of_a_callers_large_order(rows, monkeypatch):
+    """A table of order 300 from the caller on both sides of a kernel-packed projection: its transforms run as library products, as
+    they do without a kernel; 50 rows at a time take the kernel's (another order of sums, fp16 activations and results)."""
+    from qtip_amd.codebook import bitshift
+    m = k = 4800
+    g = torch.Generator(device="cuda").manual_seed(2)
+    tr = torch.randint(-32768, 32768, (m * k * 2 // 16,), dtype=torch.int16, generator=g, device="cuda")
+    mod = bitshift.BitshiftLinear(16, 16, 16, 2, 2, 9, "quantlut_sym", has_kernel=True,
+                                  tlut=torch.randn(512, 2, generator=g, device="cuda").half())
+    had = torch.randint(0, 2, (300, 300), generator=g, device="cuda").float() * 2 - 1
+    su = torch.randint(0, 2, (k,), generator=g, device="cuda").half() * 2 - 1
+    sv = torch.randn(m, generator=g, device="cuda")
+    x = torch.randn(rows, k, generator=g, device="cuda").half()
+    taken, many = [], bitshift.rht_many_rows
+    monkeypatch.setattr(bitshift, "rht_many_rows", lambda *a, **kw: taken.append(1) or many(*a, **kw))
+    call = lambda t: mod(t, tr, su, sv, had, had, 300, 300, 0, 8)
+    with torch.no_grad():
+        want = torch.cat([call(x[i:i + 50]) for i in range(0, rows, 50)])
+        assert not taken
+        got = call(x)
+    assert len(taken) == 2 and float((got.float() - want.float()).norm() / want.float().norm()) <= 2.0**-10
+
+
 @pytest.mark.parametrize("n", [11008, 4096, 12288])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_many_rows_that_start_off_16_bytes(n, dtype):
