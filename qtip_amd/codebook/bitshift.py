@@ -404,8 +404,10 @@ class BitshiftLinear(nn.Module):
     def rows_product(self, xt, trellis, tlut, m, n):
         """(rows, m) fp16 = xt (rows, n) fp16 @ decode(trellis)^T, for two rows or more."""
         if not self.takes_dense(xt.shape[0], m, n):
-            return ops.decompress_gemm(trellis.reshape(-1), xt, tlut, m, n, self.cb.K, out_dtype=torch.float16,
-                                       long_sums=self._long_sums(xt.shape[0], m, n))
+            long_sums = self._long_sums(xt.shape[0], m, n)
+            if long_sums:  # (rows at any place, as the library's product takes them)
+                xt = ops.aligned16(xt.contiguous())
+            return ops.decompress_gemm(trellis.reshape(-1), xt, tlut, m, n, self.cb.K, out_dtype=torch.float16, long_sums=long_sums)
         # decode once to dense fp16 and let the BLAS library multiply, which is what the reference does
         # for every batch (bitshift.py:476-489); fp16, which the output transform takes as it is
         return xt @ ops.decode(trellis.reshape(-1), tlut.reshape(-1), m, n, self.cb.K).T
@@ -451,8 +453,9 @@ class BitshiftLinearKernelAG(torch.autograd.Function):
             y = ops.decompress_matvec(trellis.reshape(-1), x.reshape(-1), tlut.reshape(-1), m, n, K).view(1, m)
             y = y.to(torch.float16)
         elif not BitshiftLinear._takes_dense(x.shape[0], m, n, BitshiftLinear.dense_rows_min):
-            y = ops.decompress_gemm(trellis.reshape(-1), x, tlut.reshape(-1), m, n, K, out_dtype=torch.float16,
-                                    long_sums=BitshiftLinear._long_sums(x.shape[0], m, n))
+            long_sums = BitshiftLinear._long_sums(x.shape[0], m, n)
+            y = ops.decompress_gemm(trellis.reshape(-1), ops.aligned16(x) if long_sums else x, tlut.reshape(-1), m, n, K,
+                                    out_dtype=torch.float16, long_sums=long_sums)
         else:
             y = x @ ops.decode(trellis.reshape(-1), tlut.reshape(-1), m, n, K).T
         return y.view(*input.shape[:-1], m)

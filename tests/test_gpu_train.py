@@ -186,3 +186,25 @@ def test_step_over_a_batch_of_inputs():
     su = leaves[1].clone().requires_grad_()
     y = torch.func.vmap(lambda t: call(t, su, leaves[2]))(x)
     assert _close([y], [torch.stack([call(t, su, leaves[2]) for t in x])])
+
+
+@pytest.mark.parametrize("rows", [250, 3000])
+def test_kernel_product_of_rows_that_start_anywhere(rows):
+    """BitshiftLinearKernelAG and rows_product of many rows take rows off 16 bytes and rows that are not contiguous, as a library
+    product does: the values of an aligned copy."""
+    from qtip_amd.codebook.bitshift import BitshiftLinear, BitshiftLinearKernelAG
+    m, k = 256, 512
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    tr = torch.randint(-32768, 32768, (m * k * 2 // 16,), dtype=torch.int16, generator=g, device="cuda")
+    mod = BitshiftLinear(16, 16, 16, 2, 2, 9, "quantlut_sym", has_kernel=True,
+                         tlut=torch.randn(512, 2, generator=g, device="cuda").half()).cuda()
+    x = torch.randn(rows, k, generator=g, device="cuda").half()
+    off = torch.empty(rows * k + 3, dtype=torch.float16, device="cuda")[3:].view(rows, k).copy_(x)
+    wide = torch.stack([x, x], -1)[..., 0]
+    tlut = mod._tlut16(x.device)
+    with torch.no_grad():
+        mod.cb.recons_lut()
+        for form in (off, wide):
+            a, b = (BitshiftLinearKernelAG.apply(t, tr, m, k, 16, 9, 2, 2, mod.cb.lut) for t in (x, form))
+            assert torch.equal(a, b)
+            assert torch.equal(mod.rows_product(x, tr, tlut, m, k), mod.rows_product(form, tr, tlut, m, k))
