@@ -165,3 +165,19 @@ def test_launchers_on_two_streams_do_not_disturb_each_other():
         for a, b in zip(alone, got):
             for ta, tb in zip(a, b):
                 assert torch.equal(ta, tb)
+
+
+def test_torch_op_copies_or_refuses_a_packed_tensor_that_is_not_contiguous():
+    """As `compressed.reshape(-1)` does for the reference's op (lib/codebook/__init__.py:85-92): a transposed tensor is copied, every
+    other word of a larger one stays a view and is refused."""
+    import torch
+    import qtip_amd.codebook as codebook
+    op = codebook.register_shape(256, 256, 2)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    pk = torch.randint(-32768, 32768, (256, 32), dtype=torch.int16, generator=g, device="cuda")
+    x = torch.randn(1, 256, generator=g, device="cuda").half()
+    tl = torch.randn(512, 2, generator=g, device="cuda").half()
+    want = op(pk, x, tl)
+    assert torch.equal(op(pk.T.contiguous().T, x, tl), want) and torch.equal(op(pk, x, tl.T.contiguous().T), want)
+    with pytest.raises(ValueError):
+        op(torch.stack([pk, pk], -1)[..., 0], x, tl)
