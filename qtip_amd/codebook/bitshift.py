@@ -180,22 +180,24 @@ def _contiguous(t):
     return t if t.is_contiguous() else t.contiguous()
 
 
-# Rows up to which a product decodes the matrix as it multiplies (gemm_rows_kernel): once per 64 to 128 rows, where the
-# dense route writes and reads 2 m n bytes once and then multiplies at the library's rate.  us at 2000 rows, dense / fused:
-# 4096x4096 73/66, 12288x4096 197/184, 22016x4096 446/317, 4096x11008 190/156, 28672x8192 805/770, 512x2048 20/15, 1728x832
-# 22/15; at 3000 rows 92/96, 270/279, 528/507, 221/231, 8192x8192 337/339, 2048x2048 38/34.  Matrices of few columns
-# end a unit after few steps: 11008x2048 83/66 at 1400 rows, 102/102 at 2000 (whole calls 147/150), so their line is
-# at 2^24 results.
+# Rows up to which a product decodes the matrix as it multiplies, once per batch tile of 32 to 128 rows, where the dense route
+# writes and reads 2 m n bytes once and then multiplies at the library's rate.  us of the products at 2 bits from cold memory,
+# fused / dense, 2048 rows (16 tiles of 128) and 2049: 4096x4096 70/76 90/78, 12288x4096 194/203 216/206, 22016x4096 329/454
+# 348/450, 4096x11008 167/188 213/199, 8192x8192 228/227 263/304, 13824x5120 267/289 284/281, 28672x8192 816/810 838/845,
+# 8192x28672 753/773 830/1392; at 3000 rows 101/95, 286/274, 515/538, 248/231, 356/344, 391/399, 1210/1124, 1178/1188.
+# Matrices of few columns end a unit after few steps: 28672x1024 40/48 at 512 rows, 77/79 at 1024, 108/100 at 1400, 11008x2048
+# 68/82 at 1400, 82/88 at 1536, 104/102 at 2048, so their line is at 2^24 results.
 _FUSED_ROWS_MAX = 2048
-_DENSE_ROWS_MIN = 193
+# ... and rows from which the product would be dense if the fused one were no faster past 128 rows: see _rows_by_size
+_MANY_ROWS = 193
 
 
 class BitshiftLinear(nn.Module):
 
     max_rows = 65535  # rows per launch of the transform / GEMM kernels (grid limit)
     # A caller's own value asks for the dense decode + library GEMM instead of the fused decompress-GEMM from this many
-    # rows on, for matrices of ordinary size (dense_rows_from); as it stands, takes_dense decides.
-    dense_rows_min = _DENSE_ROWS_MIN
+    # rows on, for matrices of ordinary size (_rows_by_size); None leaves it to dense_rows_from.
+    dense_rows_min = None
 
     def __init__(self, td_x, td_y, L, K, V, tlut_bits, decode_mode, dtype=torch.float16, tlut=None,
                  has_kernel=False):
@@ -298,7 +300,7 @@ class BitshiftLinear(nn.Module):
             y = ops.linear(_contiguous(x), _contiguous(trellis), self._tlut16(dev), _contiguous(SU), _contiguous(SV),
                            had_bits(had_left, K_left, True, dev) if K_left > 1 else None, K_left,
                            had_bits(had_right, K_right, False, dev) if K_right > 1 else None, K_right,
-                           m, n, self.cb.K, (n**-0.5) / self.scale, (m**-0.5) * self.scale, self._long_sums(bs, m, n))
+                           m, n, self.cb.K, (n**-0.5) / self.scale, (m**-0.5) * self.scale, bs > 1 and self._long_sums(bs, m, n))
             return y if flat else y.view(*input.shape[:-1], m)
 
         # ---- input transform: fp16(H_L^T (x * SU) / sqrt(n) / 32)
@@ -373,33 +375,33 @@ class BitshiftLinear(nn.Module):
 
 
     @staticmethod
-    def _dense_rows_from(m, n, rows_min):
-        """rows_min for an (m, n) matrix of ordinary size, and 4/3, 5/3 or 8/3 of it for larger ones, which the
-        dense route writes and reads in full: where a caller that sets dense_rows_min = rows_min wants that route."""
+    def _rows_by_size(m, n, rows):
+        """`rows` for an (m, n) matrix of ordinary size, and 4/3, 5/3 or 8/3 of them for larger ones, which the
+        dense route writes and reads in full."""
         if n < 5120 or m * n < 1 << 26:
-            return rows_min
+            return rows
         if n < 8192 or m * n < 1 << 27:
-            return rows_min * 4 // 3
-        return rows_min * 5 // 3 if n < 2 * m else rows_min * 8 // 3
-
-    def dense_rows_from(self, m, n):
-        return self._dense_rows_from(m, n, self.dense_rows_min)
+            return rows * 4 // 3
+        return rows * 5 // 3 if n < 2 * m else rows * 8 // 3
 
     @classmethod
-    def _takes_dense(cls, rows, m, n, rows_min):
-        if rows_min != _DENSE_ROWS_MIN:
-            return rows >= cls._dense_rows_from(m, n, rows_min)
-        return rows > _FUSED_ROWS_MAX or (n < 4096 and rows * m > 1 << 24)
+    def _dense_rows_from(cls, m, n, rows_min):
+        if rows_min is not None:
+            return cls._rows_by_size(m, n, rows_min)
+        return _FUSED_ROWS_MAX + 1 if n >= 4096 else min(_FUSED_ROWS_MAX, (1 << 24) // m) + 1
+
+    def dense_rows_from(self, m, n):
+        """The row count from which the product decodes an (m, n) matrix to dense fp16 and hands it to the BLAS library."""
+        return self._dense_rows_from(m, n, self.dense_rows_min)
 
     def takes_dense(self, rows, m, n):
-        """The product of `rows` rows decodes an (m, n) matrix to dense fp16 and hands it to the BLAS library."""
-        return self._takes_dense(rows, m, n, self.dense_rows_min)
+        return rows >= self._dense_rows_from(m, n, self.dense_rows_min)
 
     @classmethod
     def _long_sums(cls, rows, m, n):
         """A product of so many rows that it would otherwise be the BLAS library's, as the reference's is for every batch,
         may sum in chains as long (ops.decompress_gemm); fewer rows keep the fine sums."""
-        return rows >= cls._dense_rows_from(m, n, _DENSE_ROWS_MIN)
+        return rows >= cls._rows_by_size(m, n, _MANY_ROWS)
 
     def rows_product(self, xt, trellis, tlut, m, n):
         """(rows, m) fp16 = xt (rows, n) fp16 @ decode(trellis)^T, for two rows or more."""
@@ -452,7 +454,7 @@ class BitshiftLinearKernelAG(torch.autograd.Function):
         if x.shape[0] == 1:
             y = ops.decompress_matvec(trellis.reshape(-1), x.reshape(-1), tlut.reshape(-1), m, n, K).view(1, m)
             y = y.to(torch.float16)
-        elif not BitshiftLinear._takes_dense(x.shape[0], m, n, BitshiftLinear.dense_rows_min):
+        elif x.shape[0] < BitshiftLinear._dense_rows_from(m, n, BitshiftLinear.dense_rows_min):
             long_sums = BitshiftLinear._long_sums(x.shape[0], m, n)
             y = ops.decompress_gemm(trellis.reshape(-1), ops.aligned16(x) if long_sums else x, tlut.reshape(-1), m, n, K,
                                     out_dtype=torch.float16, long_sums=long_sums)

@@ -66,21 +66,29 @@ def test_linear_refuses_what_does_not_fit():
 
 
 def test_dense_rows_rule():
-    """The row count of the dense route grows with the matrix and follows an instance's own dense_rows_min."""
+    """The row count of the dense route: past 2048 rows, or 2^24 results of fewer than 4096 columns; an instance's own
+    dense_rows_min (whatever its value) grows with the matrix."""
     lin = QuantizedLinear(1024, 512, 16, 16, 16, 2, 2, 9, "quantlut_sym", dtype=torch.float16).cuda()
     with torch.no_grad():
         lin(torch.zeros(1, 1024, device="cuda", dtype=torch.float16))
     book = lin.codebook_class
-    assert [book.dense_rows_from(m, n) for m, n in ((4096, 4096), (57344, 4096), (8192, 8192), (8160, 8192), (28672, 8192),
-                                                    (8192, 28672), (16384, 8192))] == [193, 193, 257, 193, 321, 514, 321]
+    shapes = ((4096, 4096), (57344, 4096), (8192, 8192), (8160, 8192), (28672, 8192), (8192, 28672), (16384, 8192))
+    assert book.dense_rows_min is None and {book.dense_rows_from(m, n) for m, n in shapes} == {2049}
+    assert [book.dense_rows_from(m, n) for m, n in ((8192, 2048), (8224, 2048), (28672, 1024), (512, 32))] == [2049, 2041, 586, 2049]
+    for rows_min in (193, 194):
+        book.dense_rows_min = rows_min
+        assert [book.dense_rows_from(m, n) for m, n in shapes[:5]] == [rows_min, rows_min, rows_min * 4 // 3, rows_min, rows_min * 5 // 3]
+        assert book.dense_rows_from(8192, 28672) == rows_min * 8 // 3 and book.takes_dense(rows_min, 512, 1024)
     book.dense_rows_min = 2
     assert book.dense_rows_from(4096, 4096) == 2 and book.dense_rows_from(28672, 8192) == 3
 
 
-@pytest.mark.parametrize("m,k,bits", [(13824, 5120, 3), (16384, 8192, 2), (8192, 16384, 4)])
-def test_rows_around_the_dense_route(m, k, bits):
-    """Either side of the row count from which a large matrix is decoded to dense fp16, against float64 from the decoded
-    weights: fp32 sums of k products (error at most k 2^-24 of the sum of magnitudes, far less in fact) and a rounding to fp16."""
+@pytest.mark.parametrize("m,k,bits", [(13824, 5120, 3), (16384, 8192, 2), (8192, 16384, 4), (28672, 1024, 2), (512, 1024, 3)])
+def test_rows_around_the_dense_route(m, k, bits, monkeypatch):
+    """Either side of the row count from which a matrix is decoded to dense fp16 (2049, 586 for the short rows of 28672x1024),
+    against float64 from the decoded weights: fp32 sums of k products (error at most k 2^-24 of the sum of magnitudes, far
+    less in fact) and a rounding to fp16."""
+    from qtip_amd.codebook.bitshift import BitshiftLinearKernelAG
     g = torch.Generator(device="cuda").manual_seed(m)
     lin = QuantizedLinear(k, m, 16, 16, 16, bits, 2, 9, "quantlut_sym", dtype=torch.float16).cuda()
     lin.trellis.copy_(torch.randint(-32768, 32768, lin.trellis.shape, dtype=torch.int16, generator=g, device="cuda"))
@@ -88,14 +96,21 @@ def test_rows_around_the_dense_route(m, k, bits):
     with torch.no_grad():
         lin(torch.zeros(1, k, device="cuda", dtype=torch.float16))
         book = lin.codebook_class
+        book.cb.recons_lut()
         edge = book.dense_rows_from(m, k)
-        assert edge > book.dense_rows_min
+        assert edge == (586 if m == 28672 else 2049) and book.takes_dense(edge, m, k) and not book.takes_dense(edge - 1, m, k)
         tl = book._tlut16(torch.device("cuda", 0))
         pick = torch.arange(0, m, 37, device="cuda")
         w = ops.decode(lin.trellis.reshape(-1), tl.reshape(-1), m, k, bits)[pick].double()
+        dense, decode = [], ops.decode
+        monkeypatch.setattr(ops, "decode", lambda *a: dense.append(1) or decode(*a))
         for rows in (edge - 1, edge):
             x = torch.randn(rows, k, generator=g, device="cuda").half()
-            y = book.rows_product(x, lin.trellis, tl, m, k)
-            assert y.shape == (rows, m) and y.dtype == torch.float16
             want, size = x.double() @ w.T, x.double().abs() @ w.abs().T
-            assert bool(((y[:, pick].double() - want).abs() <= 2.0**-11 * want.abs() + 2.0**-20 * size).all())
+            for product in (lambda: book.rows_product(x, lin.trellis, tl, m, k),
+                            lambda: BitshiftLinearKernelAG.apply(x, lin.trellis, m, k, 16, 9, bits, 2, book.cb.lut)):
+                dense.clear()
+                y = product()
+                assert len(dense) == (1 if rows == edge else 0)
+                assert y.shape == (rows, m) and y.dtype == torch.float16
+                assert bool(((y[:, pick].double() - want).abs() <= 2.0**-11 * want.abs() + 2.0**-20 * size).all())

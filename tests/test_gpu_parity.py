@@ -1215,7 +1215,7 @@ def test_input_transforms_of_several_layers_in_one_launch(n):
 
 
 def test_forward_many_rows_decodes_and_multiplies():
-    """From BitshiftLinear.dense_rows_min rows on the layer decodes to dense fp16 and multiplies
+    """From its own dense_rows_min rows on the layer decodes to dense fp16 and multiplies
     with the BLAS library (the reference's route for every batch, bitshift.py:476-489): same
     result as the fused decompress-GEMM and as the oracle's dense layer."""
     from qtip_amd.codebook.bitshift import BitshiftLinear, BitshiftLinearKernelAG
@@ -1226,10 +1226,13 @@ def test_forward_many_rows_decodes_and_multiplies():
     hl, Kl = mh.get_hadK(k)
     hr, Kr = mh.get_hadK(m)
     args = (dev(L["packed"]), dev(L["SU"]), dev(L["SV"]), hl, hr, Kl, Kr, 0, 8)
-    rows = BitshiftLinear.dense_rows_min + 9
+    rows = 202
     x = torch.randn(rows, k, generator=torch.Generator().manual_seed(2)).half()
+    mod.dense_rows_min = rows - 9
+    assert mod.takes_dense(rows, m, k) and not mod.takes_dense(rows - 10, m, k)
     dense = mod(x.cuda(), *args)
     mod.dense_rows_min = 10**9
+    assert not mod.takes_dense(rows, m, k)
     fused = mod(x.cuda(), *args)
     assert dense.shape == fused.shape == (rows, m)
     assert_close(dense.float().cpu().numpy(), fused.float().cpu().numpy(), 5e-3, 5e-4)
