@@ -210,19 +210,28 @@ inline GemmParts long_plan(int m, int k, int nb, int cus, bool split) {
   return p;
 }
 
-// The plan of a call is asked for by its size queries and by its launches; a search takes 1 to 15 us, so each thread
-// keeps those of the last sizes.
+// The plan of a call is asked for by its size queries and by its launches; a search takes up to 3 us (of 1000 rows; 0.1 to 1
+// of few), so each thread keeps those of the last sizes.  The slot: sizes that share one at some row count and bit width (as
+// 11008x4096 and 4096x11008 at all of them, if every size had a factor of its own) must not do so at the next.
+inline unsigned plan_slot(int m, int k, int bits, int nb, bool split, bool fine) {
+  uint32_t h = 0;
+  for (uint32_t v : {(uint32_t)m, (uint32_t)k, (uint32_t)(16 * nb + 4 * bits + 2 * split + fine)}) {
+    h = (h + v) * 0x9E3779B1u;
+    h ^= h >> 15;
+  }
+  return (h * 0x85EBCA77u) >> 26;
+}
 inline GemmParts gemm_plan(int m, int k, int bits, int nb, int cus, bool split, bool fine) {
   struct Held {
-    int m, k, bits, nb, cus;  // (of split plans; the others come from callers without scratch)
-    bool fine;
+    int m, k, bits, nb, cus;
+    bool split, fine;
     GemmParts plan;
   };
   static thread_local Held held[64];
-  auto make = [&]() { return fine ? GemmParts{m, fine_plan(m, k, bits, nb, cus, split), {}} : long_plan(m, k, nb, cus, split); };
-  if (!split) return make();
-  Held& h = held[((uint32_t)m * 0x9E3779B1u ^ (uint32_t)k * 0x85EBCA77u ^ (uint32_t)(4 * nb + bits) * 0xC2B2AE3Du) >> 26];
-  if (h.m != m || h.k != k || h.bits != bits || h.nb != nb || h.cus != cus || h.fine != fine) h = {m, k, bits, nb, cus, fine, make()};
+  Held& h = held[plan_slot(m, k, bits, nb, split, fine)];
+  if (h.m != m || h.k != k || h.bits != bits || h.nb != nb || h.cus != cus || h.split != split || h.fine != fine)
+    h = {m, k, bits, nb, cus, split, fine,
+         fine ? GemmParts{m, fine_plan(m, k, bits, nb, cus, split), {}} : long_plan(m, k, nb, cus, split)};
   return h.plan;
 }
 

@@ -24,6 +24,7 @@ extern "C" int plan_of(int m, int k, int bits, int nb, int cus, int split, int f
 extern "C" int pass_of(int m, int k, int bits, int left, int cus, int split, int fine) {
   return next_pass(m, k, bits, left, cus, split, fine);
 }
+extern "C" int slot_of(int m, int k, int bits, int nb, int split, int fine) { return plan_slot(m, k, bits, nb, split, fine); }
 extern "C" void few_place(int lane, int batch, int k, int wl, int units, int nst, int last_half, uint32_t* out) {
   const FewPlace p = few_activations(lane, batch, k, wl, units, nst, last_half);
   out[0] = p.so;
@@ -119,3 +120,18 @@ def test_sums_are_cut_finely(native, k):
 def test_long_sums_are_longer(native):
     _, (form, NB, RG, S, wl_per), _ = plan(native, 8192, 28672, 2, 1000, fine=False)
     assert form == ROWS and _error(448, 8 // RG, wl_per, S) > 2 * _cut_error(8192, 28672, 128, True)
+
+
+def test_sizes_that_share_a_slot_of_held_plans_part_again(native):
+    """The plans of a thread's last sizes are held in 64 slots: no two projections share one at more than a sixteenth of the row
+    counts (a sixty-fourth by chance), and a plan asked for again is the same after others have taken its slot."""
+    sizes = [(m, k) for d, f, kv in ((4096, 11008, 4096), (2048, 5504, 512), (8192, 28672, 1024), (5120, 13824, 5120))
+             for m, k in ((d, d), (kv, d), (f, d), (2 * f, d), (d, f))] + [(m, k) for m in (832, 928, 1120) for k in (832, 928, 1120)]
+    slots = {s: [native.slot_of(*s, bits, nb, 1, 1) for nb in range(1, 513) for bits in (2, 4)] for s in set(sizes)}
+    assert all(0 <= v < 64 for l in slots.values() for v in l)
+    for a in slots:
+        for b in slots:
+            assert a == b or sum(x == y for x, y in zip(slots[a], slots[b])) <= 1024 // 16, (a, b)
+    cases = [(m, k, bits, nb, split, fine) for m, k in sizes for bits in (2, 3) for nb in (5, 40, 300) for split in (0, 1) for fine in (0, 1)]
+    first = [plan(native, *c) for c in cases]
+    assert [plan(native, *c) for c in reversed(cases)] == first[::-1]
