@@ -1,53 +1,27 @@
 """How the batched product is cut into launches and where its waves read (qtip_gemm_plan.h), compiled for the host."""
 import ctypes
-import os
-import subprocess
 
 import pytest
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-CUS = 256
-
-SHIM = r"""
-#include "qtip_gemm_plan.h"
-using namespace qtip;
-static void put(const GemmPlan& g, int* out) {
-  const int v[] = {g.form, g.NB, g.RG, g.S, g.wl_per};
-  for (int i = 0; i < 5; ++i) out[i] = v[i];
-}
-extern "C" int plan_of(int m, int k, int bits, int nb, int cus, int split, int fine, int* out) {
-  const GemmParts p = gemm_plan(m, k, bits, nb, cus, split, fine);
-  put(p.first, out);
-  put(p.rest, out + 5);
-  return p.m0;
-}
-extern "C" int pass_of(int m, int k, int bits, int left, int cus, int split, int fine) {
-  return next_pass(m, k, bits, left, cus, split, fine);
-}
-extern "C" int slot_of(int m, int k, int bits, int nb, int split, int fine) { return plan_slot(m, k, bits, nb, split, fine); }
-extern "C" void few_place(int lane, int batch, int k, int wl, int units, int nst, int last_half, uint32_t* out) {
-  const FewPlace p = few_activations(lane, batch, k, wl, units, nst, last_half);
-  out[0] = p.so;
-  out[1] = p.vo;
-}
-"""
-FEW, SHARED, ROWS = range(3)
+import gemm_plan as G
+from gemm_plan import CUS, FEW, ROWS, SHARED, plan
 
 
 @pytest.fixture(scope="module")
-def native(tmp_path_factory):
-    d = tmp_path_factory.mktemp("gemm_plan")
-    (d / "shim.cpp").write_text(SHIM)
-    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I",
-                    os.path.join(ROOT, "qtip_amd", "csrc"), str(d / "shim.cpp"), "-o", str(d / "shim.so")], check=True)
-    return ctypes.CDLL(str(d / "shim.so"))
+def native():
+    return G.library()
 
 
-def plan(native, m, k, bits, batch, split=True, fine=True):
-    """Matrix rows of the first launch, (form, NB, RG, S, wl_per) of it and of the second."""
-    out = (ctypes.c_int * 10)()
-    m0 = native.plan_of(m, k, bits, batch, CUS, int(split), int(fine), out)
-    return m0, tuple(out[:5]), tuple(out[5:])
+def test_cases_reach_every_kernel():
+    """The cases that the GPU runs reach the form they are listed for at every bit width, and between them every compiled one."""
+    for m, k, rows, long_sums, form in G.FORMS + G.SHARED_FORMS:
+        for bits in (3, 4) if form[:2] == (SHARED, 1) else (2, 3, 4):
+            assert form in G.launches(m, k, bits, rows, not long_sums), (m, k, rows, bits)
+    compiled = {(FEW, 1, 1), (FEW, 1, 2), (SHARED, 1, 2), (SHARED, 2, 2)} | {
+        (ROWS, NB, RG) for NB, RG in ((8, 8), (8, 4), (6, 8), (4, 8), (4, 4), (4, 2), (2, 4), (2, 2))}
+    reached = {(form[:3], form[4]) for *_, form in G.FORMS + G.SHARED_FORMS}
+    assert reached == {(f, inside) for f in compiled for inside in (False, True)}
+    assert any(G.plan(m, k, 2, rows, fine=False)[0] < m for m, k, rows, long_sums, _ in G.FORMS if long_sums)  # two launches
 
 
 @pytest.mark.parametrize("k", [32, 64, 96, 832, 928, 2080, 4096, 28672])
@@ -58,7 +32,7 @@ def test_few_rows_read_their_activations_only(native, m, k):
     place = (ctypes.c_uint32 * 2)()
     nwl, odd = (k // 32 + 1) // 2, k // 32 % 2
     for batch in (2, 5, 16):
-        _, (form, _, RG, S, wl_per), _ = plan(native, m, k, 2, batch)
+        _, (form, _, RG, S, wl_per), _ = plan(m, k, 2, batch)
         assert form == FEW
         KS, size = 16 // RG, batch * k * 2
         for s in sorted({0, S - 1}):
@@ -110,7 +84,7 @@ def test_sums_are_cut_finely(native, k):
                     while left:
                         nb = native.pass_of(m, k, bits, left, CUS, int(split), 1)
                         assert 1 <= nb <= min(left, 256) and nb * k * 2 <= 0x7FFFFF00
-                        m0, (form, NB, RG, S, wl_per), _ = plan(native, m, k, bits, nb, split)
+                        m0, (form, NB, RG, S, wl_per), _ = plan(m, k, bits, nb, split)
                         assert m0 == m and RG and (split or S == 1)
                         KS = (8 if form == ROWS else 16) // RG
                         assert _error(nwl, KS, wl_per, S) <= _cut_error(m, k, nb, split), (m, bits, batch, nb, split)
@@ -118,7 +92,7 @@ def test_sums_are_cut_finely(native, k):
 
 
 def test_long_sums_are_longer(native):
-    _, (form, NB, RG, S, wl_per), _ = plan(native, 8192, 28672, 2, 1000, fine=False)
+    _, (form, NB, RG, S, wl_per), _ = plan(8192, 28672, 2, 1000, fine=False)
     assert form == ROWS and _error(448, 8 // RG, wl_per, S) > 2 * _cut_error(8192, 28672, 128, True)
 
 
@@ -133,5 +107,5 @@ def test_sizes_that_share_a_slot_of_held_plans_part_again(native):
         for b in slots:
             assert a == b or sum(x == y for x, y in zip(slots[a], slots[b])) <= 1024 // 16, (a, b)
     cases = [(m, k, bits, nb, split, fine) for m, k in sizes for bits in (2, 3) for nb in (5, 40, 300) for split in (0, 1) for fine in (0, 1)]
-    first = [plan(native, *c) for c in cases]
-    assert [plan(native, *c) for c in reversed(cases)] == first[::-1]
+    first = [plan(*c) for c in cases]
+    assert [plan(*c) for c in reversed(cases)] == first[::-1]

@@ -3,6 +3,8 @@ the decoded weights (bit-exact elsewhere) multiplied in float64."""
 import pytest
 import torch
 
+from gemm_plan import FORMS, SHARED_FORMS
+
 pytestmark = pytest.mark.gpu
 
 
@@ -55,9 +57,48 @@ def test_activations_beyond_two_gib(k):
     assert bool(((y - want).abs() <= 2.0**-20 * size).all())
 
 
-# each form of the kernels: up to 16 rows one or two row-block pairs, or activations shared (the largest matrices at 3 and 4
-# bits); from 17 rows on batch tiles of 32, 64, 96 and 128 rows by 2, 4 and 8 pairs; cut along k or not, in one launch or
-# two; ranges of k that end inside a stage and inside a 64-column piece
+def _check_product(m, k, batch, bits, long_sums):
+    from qtip_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(m + k + batch)
+    packed = torch.randint(-32768, 32768, (m * k * bits // 16,), dtype=torch.int16, generator=g, device="cuda")
+    tlut = torch.randn(1024, generator=g, device="cuda").half()
+    w = ops.decode(packed, tlut, m, k, bits).double()
+    x = torch.randn(batch, k, generator=g, device="cuda").half()
+    ref, size = x.double() @ w.T, x.double().abs() @ w.abs().T
+    half = ops.decompress_gemm(packed, x, tlut, m, k, bits, out_dtype=torch.float16, long_sums=long_sums)
+    # exact products, fp32 sums of k terms: chains of at most k / 32 additions, whose errors add like their square roots;
+    # rounding to fp16 (normal numbers: the smallest are 2^-14)
+    assert bool(((half.double() - ref).abs() <= 2.0**-11 * ref.abs() + 2.0**-24 + 2.0**-20 * size).all())
+    if not long_sums:
+        got = ops.decompress_gemm(packed, x, tlut, m, k, bits, round_f16=False)
+        assert bool(((got.double() - ref).abs() <= 2.0**-21 * size).all())
+        assert torch.equal(half, got.half())
+
+
+@pytest.mark.parametrize("m,k,batch,long_sums", [c[:4] for c in FORMS])
+@pytest.mark.parametrize("bits", [2, 3, 4])
+def test_every_form(m, k, batch, long_sums, bits):
+    """Every kernel of the batched product, cut along k and not, k ending inside a stage and not (FORMS says which case is which,
+    and a test without a GPU that it is)."""
+    _check_product(m, k, batch, bits, long_sums)
+
+
+@pytest.mark.parametrize("m,k,batch", [c[:3] for c in SHARED_FORMS])
+@pytest.mark.parametrize("bits", [3, 4])
+def test_every_form_of_the_largest_matrices(m, k, batch, bits):
+    _check_product(m, k, batch, bits, False)
+
+
+def test_long_sums_are_for_fp16_results():
+    from qtip_amd import ops
+    x = torch.zeros(2, 64, dtype=torch.float16, device="cuda")
+    packed = torch.zeros(64 * 64 * 2 // 16, dtype=torch.int16, device="cuda")
+    with pytest.raises(ValueError):
+        ops.decompress_gemm(packed, x, torch.zeros(1024, dtype=torch.float16, device="cuda"), 64, 64, 2, long_sums=True)
+
+
+# row counts between and at the edges of batch tiles, odd numbers of row-block pairs, ranges of k that end inside a stage and
+# inside a 64-column piece
 @pytest.mark.parametrize("m,k,batch,bits", [(1056, 928, 9, 2), (96, 32, 2, 3), (1248, 2080, 16, 4), (32768, 2144, 13, 2),
                                             (16384, 8192, 5, 3), (22016, 4096, 16, 4), (64, 32, 17, 2), (544, 96, 40, 3), (96, 160, 150, 4), (512, 2048, 31, 3), (4096, 4096, 45, 4),
                                             (1056, 2080, 130, 2), (8192, 4096, 61, 3), (12288, 2144, 90, 4), (8192, 1248, 250, 3),
@@ -101,7 +142,7 @@ def test_infinite_table_entry_stays_in_its_rows(m, k, batch):
 # forms of up to 16 rows (the last two share their activations through LDS), from 17 rows on, cut along k or not; k that ends
 # in the middle of a 64-column piece, and slices without a piece
 @pytest.mark.parametrize("m,k,batch,bits", [(64, 32, 5, 2), (128, 96, 16, 3), (1056, 928, 11, 4), (64, 32, 40, 4), (128, 96, 20, 2),
-                                            (2048, 832, 100, 3), (1056, 928, 200, 2), (4096, 11040, 45, 2), (5632, 992, 1000, 4),
+                                            (2048, 832, 100, 3), (1056, 928, 200, 2), (4096, 11040, 45, 2), (5632, 992, 1000, 4), (22016, 96, 509, 2), (12288, 928, 650, 3),
                                             (32768, 4128, 6, 4), (32768, 4128, 16, 3)])
 @pytest.mark.parametrize("entry", [0, 5])
 def test_infinities_are_those_of_the_product(m, k, batch, bits, entry):
@@ -122,11 +163,13 @@ def test_infinities_are_those_of_the_product(m, k, batch, bits, entry):
     down = (pos @ wn.T + neg @ wp.T) > 0
     fine = ~(up | down)
     assert bool((up ^ down).any())
-    assert bool(got[up & down].isnan().all())
-    assert bool((got[up & ~down] == float("inf")).all()) and bool((got[down & ~up] == -float("inf")).all())
     wf = w.double().nan_to_num(0, 0, 0)
     ref, size = x.double() @ wf.T, x.double().abs() @ wf.abs().T
-    assert bool(((got.double() - ref).abs() <= 2.0**-21 * size)[fine].all())
+    for got, off in ((got, 0), (ops.decompress_gemm(packed, x, tlut.reshape(-1), m, k, bits, out_dtype=torch.float16,
+                                                    long_sums=True), 2.0**-11)):
+        assert bool(got[up & down].isnan().all())
+        assert bool((got[up & ~down] == float("inf")).all()) and bool((got[down & ~up] == -float("inf")).all())
+        assert bool(((got.double() - ref).abs() <= off * ref.abs() + 2.0**-20 * size + 2.0**-24)[fine].all())
 
 
 @pytest.mark.parametrize("m,k,bits", [(8192, 28672, 2), (4096, 4096, 3), (11008, 2048, 4), (28672, 8192, 2)])

@@ -52,6 +52,26 @@ def test_linear_cut_along_k_is_its_launches(m, k, rows, dtype):
     test_linear_is_its_launches(m, k, rows, dtype, 2)
 
 
+@pytest.mark.parametrize("m,k,rows", [(928, 8192, 400), (4096, 4096, 250), (2048, 28672, 300), (11008, 2048, 1000), (64, 96, 7)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_linear_with_long_sums_is_its_launches(m, k, rows, dtype):
+    """ops.linear(long_sums=True) gives the bits of decompress_gemm(long_sums=True) between its transforms."""
+    bits = 2
+    g = torch.Generator(device=DEV).manual_seed(m + k + rows)
+    packed = torch.randint(-32768, 32768, (m * k * bits // 16,), dtype=torch.int16, generator=g, device=DEV)
+    tlut = torch.randn(1024, generator=g, device=DEV).half()
+    su = (torch.randint(0, 2, (k,), generator=g, device=DEV) * 2 - 1).half()
+    sv, x = torch.randn(m, generator=g, device=DEV), torch.randn(rows, k, generator=g, device=DEV).to(dtype)
+    (_, oin), (_, oout) = get_hadK(k), get_hadK(m)
+    bin_ = had_bits(None, oin, True, DEV) if oin > 1 else None
+    bout = had_bits(None, oout, False, DEV) if oout > 1 else None
+    s_in, s_out = k**-0.5 / 32, m**-0.5 * 32
+    got = ops.linear(x, packed, tlut, su, sv, bin_, oin, bout, oout, m, k, bits, s_in, s_out, long_sums=True)
+    xt = ops.rht(x, order=oin, had_bits=bin_, pre=su, scale=s_in, out_dtype=torch.float16)
+    y = ops.decompress_gemm(packed, xt, tlut, m, k, bits, out_dtype=torch.float16, long_sums=True)
+    assert torch.equal(got, ops.rht(y, order=oout, had_bits=bout, post=sv, scale=s_out, out_dtype=dtype))
+
+
 def test_linear_refuses_what_does_not_fit():
     packed = torch.zeros(64 * 64 * 2 // 16, dtype=torch.int16, device=DEV)
     args = dict(tlut=torch.zeros(1024, dtype=torch.float16, device=DEV), su=torch.ones(64, dtype=torch.float16, device=DEV),
