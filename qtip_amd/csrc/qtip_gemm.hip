@@ -38,11 +38,11 @@ constexpr size_t kGemmLds = kLut128Bytes + kGemmTileBytes;
 // pipeline runs across unit boundaries.  The k slices of a unit meet in the tile buffer at its end.
 // NB = 1 is bound by the weight stream, NB = 2 by its stages' phases.  The forms of gemm_rows_kernel at 17 to 32 rows have
 // half the slices: within what eight of them are off by (fine_error) they take 0.9 to 1.6 times as long, with chains twice as
-// long 0.87 to 1.08.  us from cold memory, launches and sums of ranges included, 32 rows at 2 bits: 4096x4096 13.4,
-// 22016x4096 19.9, 28672x8192 34, 4096x11008 17.1, 8192x28672 35.
+// long 0.87 to 1.08.  us from cold memory, launches and sums of ranges included, 32 rows at 2 bits: 4096x4096 13.1,
+// 22016x4096 19.7, 28672x8192 34, 4096x11008 17.1, 8192x28672 36.
 constexpr int kWaves = 16, kThreads = 64 * kWaves;
 
-// CUT: k / 32 is odd.  (Looking for the last wave-load in a kernel of its own: 2 % at 17 to 32 rows, 7 % at 28672x8192.)
+// CUT: k / 32 is odd.  (A kernel of its own: looking for the last wave-load costs 2 % at 17 to 32 rows.)
 template <int K, int NB, bool CUT, typename TOut>
 __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(
     TOut* __restrict__ dst, const uint8_t* __restrict__ packed, const uint16_t* __restrict__ x,

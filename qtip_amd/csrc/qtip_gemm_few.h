@@ -9,11 +9,11 @@
 // (28672x8192 at 2 bits, 16 rows: 38 us).
 //
 // 16 waves of 128 registers: RG row-block pairs by KS = 16 / RG column slices, which meet in LDS at a unit's end.  One
-// wave-load of weights in flight per wave instead of two: 10 % more from cold memory at 4 bits.  us per launch from cold
-// memory, sums of k ranges included, gemm_kernel / here at 2 bits: 28672x8192 16 rows 27.0 / 22.6, 57344x8192 49.8 / 43.0,
-// 12288x4096 12.4 / 8.8, 4096x4096 10.0 / 8.4, 4096x11008 13.4 / 10.4, 8192x28672 28.1 / 24.0; 6 rows of 28672x8192 24.6 /
-// 21.4.  At 4 bits 4096x11008 14.5 / 12.5, 10240x8192 18.2 / 16.9, but 22016x4096 15.9 / 16.8 and 28672x8192 28.0 / 34.2:
-// there the stream is the bound, and requests for 16 rows of activations are in its way.
+// wave-load of weights in flight per wave instead of two: 10 % more from cold memory at 4 bits.  us per product of 16 rows from
+// cold memory, launches and sums of ranges included, gemm_kernel / here with fine sums, 2 bits: 28672x8192 27.6 / 24.6,
+// 22016x4096 15.9 / 13.0, 4096x4096 10.5 / 9.7, 4096x11008 13.8 / 12.2, 8192x28672 26.8 / 26.7.  At 4 bits 4096x4096 10.8 / 9.9,
+// 4096x11008 15.2 / 14.2, but of the largest (launch alone) 22016x4096 15.9 / 16.8 and 28672x8192 28.0 / 34.2: there the
+// stream is the bound, and requests for 16 rows of activations are in its way (shared_rows).
 
 template <int K, int RG, typename TOut>
 __global__ __launch_bounds__(64 * kFewWaves, 1) void gemm_few_kernel(

@@ -90,8 +90,8 @@ inline GemmPlan shared_plan(int m, int k, int bits, int nb, int cus, bool split)
   return g;
 }
 
-// The form of gemm_few_kernel with the least expected time, of those off by no more than `most`: 2 to 3 % longer than any form on
-// average, up to 30 % (2048x11008).  Fitted to 540 launches from
+// The form of gemm_few_kernel with the least expected time, of those off by no more than `most`: fine sums take 7 % longer than
+// the fastest form on average, up to 30 % (2048x11008).  Fitted to 540 launches from
 // cold memory (2 to 16 rows, all widths, 512x2048 to 57344x8192; 7 % root mean square).
 inline GemmPlan few_plan(int m, int k, int bits, int nb, int cus, bool split, int most) {
   const int nwl = ((k >> 5) + 1) >> 1;

@@ -23,11 +23,11 @@
 // 1.18 PFLOP/s, the library's product of the decoded matrix at 1.20.  us per product from cold memory, launches
 // and sums of ranges included, 2 bits: a kernel that decodes, then multiplies between two barriers, in passes of 128 rows / here
 // with fine sums / with long ones (qtip_gemm_plan.h):
-//   4096x4096     45 rows 15.5 / 15.8 / 13.0, 128 31 / 19 / 17, 250 60 / 30 / 20, 1000 242 / 118 / 41
-//   22016x4096    45 rows 28.3 / 26.2 / 25.6, 128 54 / 43 / 39, 250 106 / 74 / 55, 1000 423 / 291 / 180
-//   28672x8192    45 rows 51 / 45 / 45, 128 91 / 70 / 69, 250 177 / 128 / 108, 1000 704 / 522 / 415
-//   4096x11008    45 rows 20.7 / 20.0 / 18.7, 128 38 / 28 / 27, 250 73 / 47 / 38, 1000 291 / 186 / 90
-//   8192x28672    45 rows 50 / 47 / 44, 128 84 / 68 / 67, 250 168 / 122 / 111, 1000 655 / 488 / 407
+//   4096x4096     45 rows 15.4 / 15.1 / 12.5, 128 31 / 19 / 17, 250 60 / 30 / 20, 1000 242 / 115 / 42
+//   22016x4096    45 rows 28.7 / 24.8 / 24.4, 128 53 / 42 / 37, 250 105 / 72 / 55, 1000 420 / 286 / 181
+//   28672x8192    45 rows 51 / 45 / 46, 128 92 / 69 / 70, 250 178 / 127 / 111, 1000 701 / 510 / 419
+//   4096x11008    45 rows 20.9 / 19.6 / 18.4, 128 38 / 28 / 27, 250 73 / 46 / 39, 1000 289 / 183 / 93
+//   8192x28672    45 rows 51 / 46 / 45, 128 85 / 68 / 69, 250 166 / 122 / 115, 1000 653 / 479 / 409
 
 template <int K>
 struct SlotMap {  // slot r = 0..7 of a column half kh: register of P, and where its two halves' words go
