@@ -194,8 +194,8 @@ int qtip_decompress_gemm_f16(void* out_f16, const void* packed, const void* x_f1
                              void* stream);
 
 /* The same for many rows (a prompt, a training batch), faster: fp32 sums in chains as long as those of a library product of
- * the dense matrix, k / 32 additions at most.  From some 200 rows on the difference is before the rounding to fp16
- * (2 to 8e-7 of the result against 1 to 3e-7; the rounding itself is 2.07e-4). */
+ * the dense matrix, k / 32 additions at most.  They are off by 2 to 8e-7 of the result before it is rounded to fp16, those of
+ * qtip_decompress_gemm by 1 to 3e-7; the rounding is 2.07e-4. */
 size_t qtip_gemm_long_workspace_bytes(int m, int k, int bits, int batch);
 int qtip_decompress_gemm_long_f16(void* out_f16, const void* packed, const void* x_f16, const void* tlut, int m,
                                   int k, int bits, int batch, void* workspace, size_t workspace_bytes,
