@@ -242,17 +242,25 @@ struct ChainRegs {  // a thread's operands, k / 1024 <= 8 consecutive elements e
   float v[8], pv[8], rv[8], wv[8], sv[8];
 };
 
+// Where the operands of the boundary's middle part are read.  It works in the swapped layout, in which
+// the lanes of a wave hold 16 runs of 4 * EPT consecutive elements: with eight elements a thread a
+// run is 64 bytes of fp16 and the operands are read there, with two or four it is half that or less
+// and a load touches four to eight times the cache lines it needs, so that they are read in the
+// natural layout and change over in LDS.  A token of 8 layers of 4096 (16 boundaries): 583 -> 565 us;
+// of layers of 8192, with the change-over in LDS or without, the same.
+template <int EPT>
+constexpr bool kChainStaged = EPT < 8;
+
 template <int EPT>
 __device__ __forceinline__ void chain_load(const ChainArgs& c, const _Float16* su, int tid, int lane,
                                            int wave, ChainRegs& r) {
   using namespace qtip_wht;
   const int e_nat = tid * EPT;
-  const int e_swp = (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
-  // operands of the middle part in the swapped layout, the partial results in the natural one
-  ld_f32<EPT>(c.post + e_swp, r.pv);
-  ld_f16<EPT>(c.residual + e_swp, r.rv);
-  ld_f16<EPT>(c.norm_w + e_swp, r.wv);
-  ld_f16<EPT>(su + e_swp, r.sv);
+  const int e_mid = kChainStaged<EPT> ? e_nat : (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
+  ld_f32<EPT>(c.post + e_mid, r.pv);
+  ld_f16<EPT>(c.residual + e_mid, r.rv);
+  ld_f16<EPT>(c.norm_w + e_mid, r.wv);
+  ld_f16<EPT>(su + e_mid, r.sv);
   ld_f32<EPT>(c.parts + e_nat, r.v);
   for (int w = 1; w < c.in_parts; ++w) {
     float t[EPT];
@@ -262,13 +270,26 @@ __device__ __forceinline__ void chain_load(const ChainArgs& c, const _Float16* s
   }
 }
 
-// xbuf: k + k/64 floats of exchange buffer, wsum: 16 floats, xs: the k fp16 activations of the matvec
+// index of element e of an operand that changes over in LDS: a pad of four lanes per 64 puts the 16
+// runs of a read on banks of their own
+template <int EPT>
+__device__ __forceinline__ int sidx(int e) {
+  return e + 4 * EPT * (e / (64 * EPT));
+}
+// the floats of LDS behind xbuf and wsum that the operands take: one of fp32, three of fp16
+template <int EPT>
+constexpr int kChainStage = (kThreads + 64) * EPT * 5 / 2;
+
+// xbuf: k + k/64 floats of exchange buffer, wsum behind it: 16 floats and kChainStage of operands, all where the
+// table will be; xs: the k fp16 activations of the matvec
 template <int EPT>
 __device__ __forceinline__ void chain_compute(ChainRegs& r, const ChainArgs& c, float scale_in, float* xbuf,
                                               float* wsum, _Float16* xs, int tid, int lane, int wave,
                                               bool write_x, unsigned long long* sv = nullptr) {
   using namespace qtip_wht;
   constexpr int N = kThreads * EPT;
+  static_assert((N + N / 64 + kWaves + (kChainStaged<EPT> ? kChainStage<EPT> : 0)) * sizeof(float) <= kLut128Bytes,
+                "the boundary's buffers fit the table's LDS");
   (void)sv;
   QTIP_STAMP_SV(6)
   const int e_nat = tid * EPT;
@@ -282,8 +303,30 @@ __device__ __forceinline__ void chain_compute(ChainRegs& r, const ChainArgs& c, 
   for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(v[i], 6, lane);
 #pragma unroll
   for (int i = 0; i < EPT; ++i) xbuf[xidx<EPT>(e_nat + i)] = v[i];
+  float* post_s = wsum + kWaves;
+  _Float16* half_s = reinterpret_cast<_Float16*>(post_s + sidx<EPT>(N));  // residual, norm weight, sign vector
+  if constexpr (kChainStaged<EPT>) {
+    _Float16 h[EPT];
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) post_s[sidx<EPT>(e_nat) + i] = r.pv[i];
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) h[i] = (_Float16)r.rv[i];
+    st_f16<EPT>(half_s + sidx<EPT>(e_nat), h);
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) h[i] = (_Float16)r.wv[i];
+    st_f16<EPT>(half_s + sidx<EPT>(N) + sidx<EPT>(e_nat), h);
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) h[i] = (_Float16)r.sv[i];
+    st_f16<EPT>(half_s + 2 * sidx<EPT>(N) + sidx<EPT>(e_nat), h);
+  }
   __syncthreads();
   QTIP_STAMP_SV(7)
+  if constexpr (kChainStaged<EPT>) {
+    ld_f32<EPT>(post_s + sidx<EPT>(e_swp), r.pv);
+    ld_f16<EPT>(half_s + sidx<EPT>(e_swp), r.rv);
+    ld_f16<EPT>(half_s + sidx<EPT>(N) + sidx<EPT>(e_swp), r.wv);
+    ld_f16<EPT>(half_s + 2 * sidx<EPT>(N) + sidx<EPT>(e_swp), r.sv);
+  }
 #pragma unroll
   for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(xbuf[xidx<EPT>(e_swp + i)], 4, lane);
   // ---- residual, RMSNorm, sign vector of this layer
