@@ -734,17 +734,35 @@ int launch_rht_rows(const RhtParams& P, int rows, hipStream_t st) {
 
 #include "qtip_rht_mix.h"
 
+// whether the output touches the rows that are read (each workgroup of a shared pass reads them after others wrote theirs)
+bool in_place(const RhtParams& P, int rows, size_t in_size, size_t out_size) {
+  const char *in = (const char*)P.in, *out = (const char*)P.out;
+  if (P.round_parts) in_size = 4;
+  const size_t width = (size_t)P.n * (P.pre_mode == PRE_SILU_MUL ? 2 : 1);
+  const size_t in_bytes = ((size_t)(P.in_parts - 1) * P.part_stride + (size_t)(rows - 1) * P.in_row_stride + width) * in_size;
+  return in < out + (size_t)rows * P.n * out_size && out < in + in_bytes;
+}
+
 constexpr int mix_class(int kt) { return kt <= 2 ? 2 : (kt <= 4 ? 4 : 8); }
 
 template <typename TI, typename TO, int MODE>
-int launch_mix(const RhtParams& P, const MixShape& M, int kt, int rows, int cus, hipStream_t st) {
+int launch_mix(const RhtParams& P, MixShape M, int kt, int rows, int cus, hipStream_t st) {
   const int ktc = mix_class(kt);
   const size_t lds = mix_lds(ktc, P.order);
   // workgroups a CU holds: LDS, and four waves of 128 registers per SIMD
   const int fit = (int)((160u * 1024) / lds) < kMixMaxKT / kt ? (int)((160u * 1024) / lds) : kMixMaxKT / kt;
   const int most = cus * (fit < 1 ? 1 : fit) >> M.logS;
   const int gx = M.npass < most ? M.npass : (most < 1 ? 1 : most);
-  const dim3 grid((unsigned)gx, 1u << M.logS);
+  // Few passes leave CUs idle, and a pass is a chain (signs, plane, products, butterflies, stores) that twelve to sixteen
+  // waves on one CU slow down for each other: as many workgroups as the chip has room for share the output rows
+  // of a pass, two waves or more each, and all of them read the whole rows.  us in a graph, shared or not: 28672, 16 fp16
+  // rows 7.0/10.2, 45 rows 7.7/10.8; 11008, 45 rows 7.6/9.8, 128 rows 8.2/10.4; fp32 45 rows 12.0/15.8.  Not where
+  // they would be more than one to a CU: 14336, 180 rows 8.8/8.4.
+  const int eights = (gx + 7) >> 3;
+  const int z = (cus >> M.logS) / (8 * eights);
+  M.share = z > 1 && !in_place(P, rows, sizeof(TI), sizeof(TO)) ? (2 * kt + z - 1) / z : 2 * kt;
+  if (M.share < 2) M.share = 2;
+  const dim3 grid(8, (unsigned)((2 * kt + M.share - 1) / M.share), (unsigned)eights << M.logS);
   if (ktc == 2) rht_mix_kernel<TI, TO, MODE, 2><<<grid, 128 * kt, lds, st>>>(P, M, rows);
   else if (ktc == 4) rht_mix_kernel<TI, TO, MODE, 4><<<grid, 128 * kt, lds, st>>>(P, M, rows);
   else rht_mix_kernel<TI, TO, MODE, 8><<<grid, 128 * kt, lds, st>>>(P, M, rows);
@@ -781,34 +799,41 @@ bool rows_form_size(int n, int order, int rows) {
 }
 
 // Rows from which the matrix form is faster than one launch of order * A workgroups per row (`wgs`), which each read
-// the whole row: its time hardly grows with the rows, theirs with rows * wgs once that passes what the chip holds.  fp32
-// rows take three planes.  Short rows cost either form little beside the launch, so the line is a count of workgroups
-// there; large orders over few points leave most of a wave's columns to other rows.  us in a graph, that form / matrix form:
-//   fp16  64 = 1 * 64, 400 rows 3.8/4.1, 600 4.7/4.1; 1024, 32 rows 3.9/4.4, 48 4.9/4.5; 1280 = 20 * 64, 32 rows 5.1/5.4,
-//         40 5.7/5.4; 3072 = 12 * 256, 16 rows 5.2/5.7, 20 5.9/5.7; 5120 = 20 * 256, 12 rows 4.8/5.9, 18 6.1/6.0;
-//         6144, 12 rows 6.0/5.9; 57344 = 28 * 2048, two slices, 12 rows 18.8/21.8, 16 24.2/22.1; 30720 = 60 * 512, 12 rows
-//         12.3/14.8, 16 16.0/15.0
-//         928 = 116 * 8, 8 rows 5.8/6.5, 12 7.2/6.9; 2240 = 140 * 16, 16 rows 8.0/8.7, 20 8.2/8.7, 24 9.7/8.7;
-//         4992 = 156 * 32, 8 rows 8.4/8.8, 12 11.7/8.8; 11008 = 172 * 64, 8 rows 14.8/10.1
-//   fp32  64, 1000 rows 5.4/6.3, 1600 7.8/6.3; 1024, 64 rows 5.4/6.3, 96 7.1/6.4; 3072, 32 rows 7.8/8.2, 36 8.7/8.2;
-//         5120, 28 rows 8.3/8.5, 36 9.4/8.5; 6144, 24 rows 8.3/8.4; 28672, 24 rows 19.8/19.6; 32768, 24 rows 17.9/22.6, 32
-//         25.2/23.1
-//         928, 32 rows 11.4/12.0, 48 15.6/12.0; 2240, 36 rows 11.6/13.9, 48 14.9/13.9; 4992, 16 rows 13.9/14.2, 18
-//         15.7/14.2; 8960 = 140 * 64, 8 rows 12.4/14, 12 16.8/14.4
-// With an element-wise prologue or a residual the matrix form is the one that covers every size, from 12 rows on.
-int mix_rows_min(int order, int n, long wgs, bool f16, bool fused, int kt, int slices) {
-  if (fused) return order >= 100 ? 8 : 12;
-  if (order >= 100) {
-    if (n <= 4096) return f16 ? (n < 1400 ? 14 : 20) : 42;
-    if (n < 8192) return f16 ? 9 : 18;
-    return f16 ? 8 : 12;
+// the whole row: its time hardly grows with the rows, theirs in steps of the workgroups that the chip holds, the higher
+// the longer a row is.  So the line is a count of workgroups, rows * wgs, by the size of a row.  fp32 rows take three planes.
+// us in a graph, that form / matrix form:
+//   fp16  order < 100:   64 = 1 * 64, 400 rows 3.8/4.1, 600 4.7/4.1; 1024, 32 rows 3.9/4.4, 48 4.9/4.5; 3072 = 12 * 256, 16 rows
+//         5.3/5.3; 5120 = 20 * 256, 12 rows 4.9/5.6, 14 6.2/5.6; 6144, 10 rows 4.9/5.5, 12 6.2/5.5; 10240, 6 rows 4.4/6.0,
+//         7 6.5/6.0; 14336, 4 rows 4.4/6.3, 5 6.5/6.3, 8 6.8/6.3; 28672, 4 rows 5.4/7.2, 5 8.7/7.3, 8 9.0/7.3; two slices:
+//         57344, 8 rows 14.0/15.5, 10 19.4/16.0
+//         order >= 100:  1248 = 156 * 8, 6 rows 5.9/6.2, 7 7.2/6.2; 1728, 8 rows 5.0/5.6, 10 6.4/5.5; 4992, 4 rows 6.2/6.5, 5
+//         7.1/6.5; 11008 = 172 * 64, 2 rows 6.1/7.1, 3 8.1/7.2, 8 14.8/7.3; 22016, 2 rows 8.8/7.4, 8 23.7/7.5
+//   fp32  order < 100:   64, 1000 rows 5.4/6.3, 1600 7.8/6.3; 1024, 64 rows 5.4/6.3, 96 7.1/6.4; 5120, 24 rows 7.3/7.7, 28
+//         8.5/7.7; 14336, 10 rows 8.9/9.4, 14 11.6/9.5; 28672, 8 rows 9.9/12.9, 10 13.3/12.9; 57344, 8 rows 14.8/14.8
+//         order >= 100:  1248, 16 rows 9.5/11.2, 20 11.3/11.2; 4992, 10 rows 10.5/10.8, 12 11.6/10.8; 11008, 5 rows 10.6/11.7,
+//         6 12.6/11.6; 22016, 2 rows 8.8/11.9, 3 12.4/11.9
+// With an element-wise prologue or a residual the matrix form is the one that covers every size, from 12 rows on at the
+// latest (8 at orders from 100 on).  Prologue SiLU: 5120, 6 rows 4.8/6.1, 7 7.3/6.0; 11008, 2 rows 8.7/8.8, 3 12.2/8.9;
+// 14336, 4 rows 5.8/7.3, 5 9.2/7.3; 28672, 4 rows 7.7/9.4, 5 13.1/9.4.
+int mix_rows_min(int order, int n, long wgs, bool f16, bool fused, int slices) {
+  const bool large = order >= 100;
+  auto above = [&](int count) { return (int)(count / wgs) + 1; };  // the first row count of more than `count` workgroups
+  if (fused) {
+    const int most = large ? 8 : 12;
+    if (n <= 4096) return most;
+    const int line = above(large ? 360 : 256);
+    return line < most ? line : most;
+  }
+  if (slices > 1) return above(510);
+  if (large) {
+    if (n <= 4096) return above(f16 ? 1024 : 3400);
+    if (n < 8192) return above(f16 ? 700 : 1800);
+    if (n < 16384) return above(f16 ? 430 : 860);
+    return above(f16 ? 256 : 400);
   }
   if (n <= 4096) return (int)(((f16 ? 512 + n / 10 : 1100 + n / 6) + wgs - 1) / wgs);
-  if (n < 6144) return f16 ? 16 : 32;
-  // (the largest workgroup, one to a CU; slices, which take three planes of either type)
-  const bool full = kt == kMixMaxKT && slices == 1;
-  if (f16) return slices > 1 || (full && order > 1) ? 16 : 12;
-  return full ? 28 : 24;
+  if (n < 10000) return above(f16 ? 512 : 1024);
+  return above(f16 ? 256 : 600);
 }
 
 int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream) {
@@ -854,7 +879,8 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
       return launch_rht_rows<float, float>(P, rows, st);
     }
   }
-  if (rows >= 8) {
+  // (rows with vectors of their own are layers that share a launch: up to seven have the bits of launches of their own)
+  if (rows >= (P.pre_row_stride || P.post_row_stride ? 8 : 2)) {
     const size_t ez = in_dtype == QTIP_F16 && !P.round_parts ? 2 : 4;
     MixShape M{};
     int kt = 0;
@@ -864,8 +890,7 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
                     ((P.pre_row_stride * 2) & 15u) == 0 && ((P.post_row_stride * 4) & 15u) == 0 &&
                     !(P.pre_mode != PRE_NONE && in_dtype != QTIP_F16) && !(fused && out_dtype != QTIP_F16) &&
                     mix_shape(n, order, rows, M, kt) &&
-                    rows >= mix_rows_min(order, n, OT, in_dtype == QTIP_F16, fused,
-                                         kt, 1 << M.logS);
+                    rows >= mix_rows_min(order, n, OT, in_dtype == QTIP_F16, fused, 1 << M.logS);
     if (ok) {
       int cus = 0;
       const int rc = qtip_device_ready(stream, &cus);
@@ -1035,7 +1060,7 @@ __global__ __launch_bounds__(kRhtThreads) void rht_chain_kernel(
 // 18.3/19.1; 928 = 116 * 8, 17 (4) 19.5/24.3, 400 (2) 41.7/42.8.
 bool qtip_rht_takes_parts(int n, int order, int rows, int nparts) {
   if (rows_form_size(n, order, rows)) return true;
-  if (rows < 8 || order < 1 || n % order || (n & 7)) return false;
+  if (rows < 2 || order < 1 || n % order || (n & 7)) return false;
   const int p = n / order;
   if (p & (p - 1)) return false;
   long pp = p, OT = order;  // (the workgroups per row of the other form, as launch_rht counts them)
@@ -1044,7 +1069,7 @@ bool qtip_rht_takes_parts(int n, int order, int rows, int nparts) {
   MixShape M{};
   int kt = 0;
   return mix_shape(n, order, rows, M, kt) && nparts << 5 <= 1 << M.logpp &&
-         rows >= mix_rows_min(order, n, OT, true, false, kt, 1 << M.logS);
+         rows >= mix_rows_min(order, n, OT, true, false, 1 << M.logS);
 }
 
 int qtip_rht_from_parts(void* out, int out_dtype, const float* parts, int nparts, int rows, int n, int order,

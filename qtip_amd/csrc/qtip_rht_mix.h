@@ -42,6 +42,7 @@ constexpr int kMixMaxOrder = 32 * kMixMaxKT;  // table orders, built in or a cal
 struct MixShape {
   int logpp, logA2, logS;  // n = order << (logS + logA2 + logpp)
   int npass;               // 128-column groups
+  int share;               // waves of a workgroup that produce output rows: from share * blockIdx.y on
 };
 
 constexpr uint32_t mix_stride(int ktc) { return 64 * ktc + 16; }  // bytes per column
@@ -74,7 +75,9 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   const int a = lane & 15, g = lane >> 4;
   const int logA2 = M.logA2, logpp = M.logpp, logS = M.logS;
   const int order = P.order, S = 1 << logS, on = order << logA2;
-  const int n = P.n, s = blockIdx.y;
+  const int n = P.n;
+  // grid (8, shares, eights of passes * slices): the workgroups that read the same rows are on one XCD
+  const int s = blockIdx.z & (S - 1), step = 8 * (gridDim.z >> logS);
   constexpr uint32_t stride = mix_stride(KTC);
   uint32_t* hb = reinterpret_cast<uint32_t*>(mix_smem + kMixCols * stride);
   const int nw = (order * order + 31) >> 5;
@@ -96,7 +99,8 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   for (int i = 0; i < 4; ++i) eoff[i] = element(j0 + i < on ? j0 + i : 0, 0);
   const int nlive = on - j0;                          // patch rows i < nlive are rows of v
   const bool edge = 16 * wave + 16 > on;              // the wave holds padding rows
-  const bool idle = 16 * wave >= on;                  // nothing but padding (the second wave of the last k tile)
+  // no output rows here: padding (the second wave of the last k tile), or another workgroup's share
+  const bool idle = 16 * wave >= on || (unsigned)(wave - (int)blockIdx.y * M.share) >= (unsigned)M.share;
   const uint32_t slice_step = 1u << (logA2 + logpp);  // elements between slices
 
   // Addresses are a uniform base (the pass's first row) and a 32-bit lane offset.
@@ -155,46 +159,84 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
     }
   };
   Patch cur;
-  int ps = blockIdx.x;
-  if (F16 && ps < M.npass) load_patch(cur, ps, 0);
+  int ps = blockIdx.x + 8 * (blockIdx.z >> logS);
+  if (ps >= M.npass) return;
+  if (F16) load_patch(cur, ps, 0);
+
+  // the output vector is needed last, behind a chain as long as a cold read: its cache lines are asked for now
+  // (a dword of each: rows 16 * wave + lane / 4 of the mix, 32 columns a lane)
+  float line = 0.f;
+  if (!AUX && P.post && !idle) {
+    const int i = 16 * wave + (lane >> 2), c = 32 * (lane & 3) & ((1 << logpp) - 1);
+    line = P.post[first_row(ps) * P.post_row_stride + element(i < on ? i : 0, s) - c0 + c];
+  }
 
   for (int i = tid; i < nw; i += blockDim.x) hb[i] = order > 1 ? P.had_bits[i] : 0u;
   if (tid < 2) flag[tid] = 0;
   __syncthreads();
-  // ---- signs of output row 16 * wave + a against v rows 32 * kt + 8 * g + e
-  // (the lookups of a k tile are issued together: a wait per lookup costs more than the transform)
-  uint32_t sb[2] = {0u, 0u};
-  {
-    const int i = 16 * wave + a;
-    const int iK = (i < on ? i : 0) >> logA2, iA = i & Am;
+  // ---- signs of output row 16 * wave + a against v rows 32 * kt + 8 * g + e: byte kt of sb, bit e
+  // (the lookups of all k tiles are issued together: a wait per lookup costs more than the transform)
+  uint32_t sb0 = 0, sb1 = 0;
+  if (!idle) {
+    uint32_t sb[2] = {0u, 0u};
     // H_A: within eight rows a pattern of iA's low bits (the rows differ in theirs), and for A > 8 a
     // sign per eight rows
+    const int i = 16 * wave + a, iA = i & Am;
     const uint32_t pat = ((iA & 1) ? 0xAAu : 0u) ^ ((iA & 2) ? 0xCCu : 0u) ^ ((iA & 4) ? 0xF0u : 0u);
-    for (int kt = 0; kt < KT; ++kt) {
-      const int jb = 32 * kt + 8 * g;
-      uint32_t byte = pat;
-      if (logA2 >= 3) {  // one table column
-        const int w = ((jb >> logA2) * order + iK) >> 5;
-        const uint32_t b = (hb[w < nw ? w : 0] >> (((jb >> logA2) * order + iK) & 31)) ^ (uint32_t)__builtin_popcount(iA & jb & Am);
-        byte ^= (0u - (b & 1u)) & 0xFFu;
-      } else {
-        // (word and shift of each row's bit; rows past the table meet zeros of v)
-        uint32_t w[8];
-        const int q0 = (jb >> logA2) * order + iK;
+    uint32_t f[KTC];
+    if (logA2 >= 3) {  // one table column
+      const int iK = (i < on ? i : 0) >> logA2;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int q = (q0 + (e >> logA2) * order) >> 5;
-          w[e] = hb[q < nw ? q : 0];
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) byte ^= ((w[e] >> ((q0 + (e >> logA2) * order) & 31)) & 1u) << e;
+      for (int kt = 0; kt < KTC; ++kt) {
+        const int q = ((32 * kt + 8 * g) >> logA2) * order + iK;
+        f[kt] = hb[q >> 5 < nw ? q >> 5 : 0] >> (q & 31);
       }
-      const uint32_t sh = byte << (8 * (kt & 3));
-      if (kt < 4) sb[0] |= sh;
-      else sb[1] |= sh;
+#pragma unroll
+      for (int kt = 0; kt < KTC; ++kt) {
+        const uint32_t b = f[kt] ^ (uint32_t)__builtin_popcount(iA & (32 * kt + 8 * g) & Am);
+        sb[kt >> 2] |= ((0u - (b & 1u)) & 0xFFu) << (8 * (kt & 3));
+      }
+    } else {
+      // lane e = a % 8 takes the bits of the eight output rows of its half of the wave against v row
+      // 32 * kt + 8 * g + e, adjacent in the table's words, and the eight lanes transpose their bytes
+      const int iK = (16 * wave + (a & 8)) >> logA2;
+      uint32_t hi[KTC], sh[KTC];
+#pragma unroll
+      for (int kt = 0; kt < KTC; ++kt) {
+        const int q = ((32 * kt + 8 * g + (a & 7)) >> logA2) * order + iK, w = q >> 5;
+        f[kt] = hb[w < nw ? w : 0];  // (rows past the table meet zeros of v, or are not stored)
+        hi[kt] = hb[w + 1 < nw ? w + 1 : 0];
+        sh[kt] = q & 31;
+      }
+#pragma unroll
+      for (int kt = 0; kt < KTC; ++kt) {
+        uint32_t x = __builtin_amdgcn_alignbit(hi[kt], f[kt], sh[kt]);
+        if (logA2 == 0) x &= 0xFFu;
+        else if (logA2 == 1) {  // four bits, each for two rows
+          x = (x & 3u) | ((x & 0xCu) << 2);
+          x = (x & 0x11u) | ((x & 0x22u) << 1);
+          x *= 3u;
+        } else x = (x & 1u) * 0x0Fu | (x & 2u) * 0x78u;  // two bits, each for four rows
+        sb[kt >> 2] |= x << (8 * (kt & 3));
+      }
+#pragma unroll
+      for (int h = 0; h < (KTC > 4 ? 2 : 1); ++h) {
+        auto step = [&](int b, uint32_t m) {  // the off-diagonal quarters change places
+          const int s = 1 << b;
+          const uint32_t o = __builtin_bit_cast(uint32_t, lane_xor(__builtin_bit_cast(float, sb[h]), b));
+          sb[h] = (a & s) ? (sb[h] & ~m) | ((o >> s) & m) : (sb[h] & m) | ((o & m) << s);
+        };
+        step(2, 0x0F0F0F0Fu);
+        step(1, 0x33333333u);
+        step(0, 0x55555555u);
+      }
     }
+    sb0 = sb[0] ^ pat * 0x01010101u;
+    sb1 = sb[1] ^ pat * 0x01010101u;
   }
-  auto signs = [&](int kt, uint32_t one) { return expand_signs(((kt & 4 ? sb[1] : sb[0]) >> (8 * (kt & 3))) & 0xFFu, one); };
+  auto signs = [&](int kt, uint32_t one) {
+    return expand_signs(((KTC > 4 && (kt & 4) ? sb1 : sb0) >> (8 * (kt & 3))) & 0xFFu, one);
+  };
   // the wave's reciprocal RMS of the lane's row: every slice, all waves, the lanes of the row
   auto row_rs = [&](const Patch& p, int ps) {
     float ss = 0.f;
@@ -249,6 +291,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   // H_pp on the products (register e is column bits 0..2, lane bit b of a column bit 3 + b) and the results
   auto finish = [&](float4v acc[8], int ps) {
     if (idle) return;
+    if constexpr (!AUX) asm volatile("" ::"v"(line));
 #pragma unroll
     for (int h = 1; h < 8; h <<= 1)
 #pragma unroll
@@ -307,6 +350,22 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   };
   uint8_t* wr = mix_smem + (uint32_t)a * stride + (uint32_t)(4 * wave + g) * 8;
   const uint8_t* rd = mix_smem + (uint32_t)a * stride + (uint32_t)g * 16;
+  // the plane's products: a column group's next operand is requested as soon as its present one is used
+  auto products = [&](float4v acc[8], uint32_t one, auto mfma) {
+    if (idle) return;
+    u32x4m b[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) b[e] = *reinterpret_cast<const u32x4m*>(rd + e * 16 * stride);
+    for (int kt = 0; kt < KT; ++kt) {
+      const u32x4m fa = signs(kt, one);
+      const uint8_t* next = rd + (kt + 1 < KT ? kt + 1 : kt) * 64;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        acc[e] = mfma(fa, b[e], acc[e]);
+        b[e] = *reinterpret_cast<const u32x4m*>(next + e * 16 * stride);
+      }
+    }
+  };
 
   // ---- one plane of fp16 values: no slices or partial sums to add, and a sign vector of nothing but
   // +-1 (the same for every pass)
@@ -325,7 +384,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
       fast = flag[1] == 0;
     }
     if (fast) {
-      for (; ps < M.npass; ps += gridDim.x) {
+      for (; ps < M.npass; ps += step) {
         float rs = 1.f;
         if constexpr (MODE == PRE_RMSNORM) rs = row_rs(cur, ps);
         u32x4m h[4];
@@ -346,20 +405,14 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
           w.y = __builtin_amdgcn_perm(h[3][e >> 1], h[2][e >> 1], (e & 1) ? 0x07060302u : 0x05040100u);
           *reinterpret_cast<uint2*>(wr + e * 16 * stride) = w;
         }
-        if (ps + (int)gridDim.x < M.npass) load_patch(cur, ps + gridDim.x, 0);
+        if (ps + step < M.npass) load_patch(cur, ps + step, 0);
         __syncthreads();
         float4v acc[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = float4v{0.f, 0.f, 0.f, 0.f};
-        if (!idle)
-          for (int kt = 0; kt < KT; ++kt) {
-            const half8m fa = __builtin_bit_cast(half8m, signs(kt, 0x3C003C00u));
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const half8m b0 = *reinterpret_cast<const half8m*>(rd + e * 16 * stride + kt * 64);
-              acc[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, b0, acc[e], 0, 0, 0);
-            }
-          }
+        products(acc, 0x3C003C00u, [](u32x4m fa, u32x4m b, float4v c) {
+          return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8m, fa), __builtin_bit_cast(half8m, b), c, 0, 0, 0);
+        });
         __syncthreads();  // the plane is free
         finish(acc, ps);
       }
@@ -368,7 +421,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   }
 
   // ---- three bf16 planes of fp32 values
-  for (; ps < M.npass; ps += gridDim.x) {
+  for (; ps < M.npass; ps += step) {
     float v[4][8];
     {
       float rs = 1.f;
@@ -445,15 +498,9 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
       }
       if (p == 1 && __any((left & 0x7FFFFFFFu) != 0) && lane == 0) flag[0] = 1;
       __syncthreads();
-      if (!idle)
-        for (int kt = 0; kt < KT; ++kt) {
-          const bf16x8 fa = __builtin_bit_cast(bf16x8, signs(kt, 0x3F803F80u));
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(rd + e * 16 * stride + kt * 64);
-            acc[e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, b0, acc[e], 0, 0, 0);
-          }
-        }
+      products(acc, 0x3F803F80u, [](u32x4m fa, u32x4m b, float4v c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fa), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+      });
       const bool last = p == 2 || (p == 1 && flag[0] == 0);  // the same for the whole workgroup
       if (p == 2 && tid == 0) flag[0] = 0;                   // (everyone read it before the barrier of this plane)
       __syncthreads();                                       // the plane is free

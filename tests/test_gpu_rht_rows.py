@@ -36,6 +36,28 @@ def test_short_rows_against_float64(n, rows):
     _check_rows(n, rows)
 
 
+# few rows, whose passes are shared by several workgroups: one pass and many, shares that do not divide a pass's waves
+@pytest.mark.parametrize("n,rows", [(928, 9), (1248, 7), (4992, 5), (5504, 5), (10240, 7), (11008, 3), (11008, 130),
+                                    (13824, 5), (14336, 67), (22016, 2), (28672, 6), (28672, 100), (57344, 11)])
+def test_few_rows_against_float64(n, rows):
+    _check_rows(n, rows)
+
+
+def test_rows_in_place():
+    """A transform over its own input, which workgroups that share a row cannot be given."""
+    from qtip_amd import _lib
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    n, rows = 11008, 20
+    had, K = get_hadK(n)
+    x = torch.randn(rows, n, generator=torch.Generator(device="cuda").manual_seed(0), device="cuda").half()
+    ref = _transform(x.double(), n, True) * n**-0.5
+    bits = had_bits(had, K, True, "cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    assert _lib.lib().qtip_rht(x.data_ptr(), _lib.QTIP_F16, x.data_ptr(), _lib.QTIP_F16, 1, rows, n, K, bits.data_ptr(), None, None,
+                               n**-0.5, st) == 0
+    assert float((x.double() - ref).abs().max()) <= 1e-3 * float(ref.abs().max())  # fp16 results
+
+
 def _check_rows(n, rows):
     from qtip_amd import ops
     from qtip_amd.utils.matmul_had import get_hadK, had_bits
