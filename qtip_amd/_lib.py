@@ -4,6 +4,7 @@ There is no CPU or pure-PyTorch fallback: if the shared library is missing or
 a launcher reports an error, the call raises.
 """
 import ctypes
+import importlib.util
 import os
 
 import torch  # must be imported first so that its bundled HIP runtime is the one libqtip_hip.so binds to
@@ -11,11 +12,14 @@ import torch  # must be imported first so that its bundled HIP runtime is the on
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("QTIP_HIP_LIBRARY") or os.path.join(_HERE, "libqtip_hip.so")
 
+HOST_PATH = os.path.join(_HERE, "_qtip_host.so")
+
 QTIP_F16 = 0
 QTIP_F32 = 1
 ABI_VERSION = 24
 
 _lib = None
+_host = None
 
 
 class QtipLibraryError(RuntimeError):
@@ -128,6 +132,22 @@ def lib():
             raise QtipLibraryError(f"libqtip_hip.so ABI {got}, Python side expects {ABI_VERSION}: rebuild")
         _lib = handle
     return _lib
+
+
+def host():
+    """The native host module (csrc/qtip_host.cpp), bound to the loaded library."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise QtipLibraryError(f"{HOST_PATH} not found: build it with `python -m qtip_amd.build`")
+        spec = importlib.util.spec_from_file_location("_qtip_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.bind(*(ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
+                      for name in ("qtip_linear", "qtip_linear_long", "qtip_linear_workspace_bytes",
+                                   "qtip_linear_long_workspace_bytes", "qtip_decompress_matvec")))
+        _host = module
+    return _host
 
 
 _INITIALISED = set()

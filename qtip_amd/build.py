@@ -1,4 +1,4 @@
-"""Compile libqtip_hip.so for gfx950 in-tree:  python -m qtip_amd.build"""
+"""Compile libqtip_hip.so for gfx950 and the host module in-tree:  python -m qtip_amd.build"""
 import os
 import subprocess
 import sys
@@ -10,6 +10,8 @@ SRCS = [os.path.join(HERE, "csrc", f)
         for f in ("qtip_hip.hip", "qtip_gemm.hip", "qtip_rht.hip", "qtip_decoder.hip", "qtip_pack.hip", "qtip_prefill.hip", "qtip_train.hip",
                   "qtip_linear.hip")]
 OUT = os.path.join(HERE, "libqtip_hip.so")
+HOST_SRC = os.path.join(HERE, "csrc", "qtip_host.cpp")
+HOST_OUT = os.path.join(HERE, "_qtip_host.so")
 
 # packed fp32 VALU forms are switched off for every HIP translation unit
 HIPCC_FLAGS = [
@@ -41,7 +43,23 @@ def compile_library(out, extra=(), verbose=True):
     return out
 
 
+def build_host(verbose=True):
+    """The native side of the wrappers' short ways (no device code), against the installed torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    dirs = include_paths() + [sysconfig.get_paths()["include"]]
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + [a for d in dirs for a in ("-isystem", d)] +
+         [HOST_SRC, "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10",
+          "-o", HOST_OUT + ".tmp"], verbose)
+    os.replace(HOST_OUT + ".tmp", HOST_OUT)
+    return HOST_OUT
+
+
 def build(verbose=True):
+    build_host(verbose)
     return compile_library(OUT, verbose=verbose)
 
 

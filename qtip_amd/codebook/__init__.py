@@ -42,6 +42,9 @@ def _make(m, k, bits):
         # reference glue (lib/codebook/__init__.py:85-92): x.to(fp16), flat
         # codebook, (1, m) fp32 result; no zero-fill is needed here because
         # the kernel overwrites every element
+        y = ops.matvec_row(compressed, x, codebook, m, k, bits)
+        if y is not None:
+            return y
         if not compressed.is_contiguous():  # (a flat view of strided words stays one, and is refused)
             compressed = compressed.reshape(-1)
         return ops.decompress_matvec(compressed, x.to(torch.float16).contiguous(), codebook.contiguous(), m, k, bits,

@@ -289,18 +289,19 @@ class BitshiftLinear(nn.Module):
                                  rcp, tp_rank, mode=mode, **kwargs) for i in range(0, bs, self.max_rows)]
             return torch.cat(outs, dim=0).view(*input.shape[:-1], m)
 
-        if (self.has_kernel and rcp not in (1, 2) and not self.takes_dense(bs, m, n) and SU.dtype == torch.float16
-                and SV.dtype == torch.float32 and SV.device == dev and x.dtype in (torch.float16, torch.float32)
-                and not by_library(bs, n, K_left) and not by_library(bs, m, K_right)):
+        if (self.has_kernel and rcp not in (1, 2) and not self.takes_dense(bs, m, n) and SU.dtype is torch.float16
+                and SV.dtype is torch.float32 and SV.device == dev and x.dtype in (torch.float16, torch.float32)
+                and (bs < 96 or not (by_library(bs, n, K_left) or by_library(bs, m, K_right)))):
             # both transforms and the product by one call of the library: what bounds such a call otherwise is the
             # host.  (Where takes_dense holds the product is the BLAS library's, where by_library holds a transform is: a
             # caller's table of order 300, 4800x4800, 1000 rows 435 against 2850 in the one call.)  us, launch by launch /
-            # here: 4096x4096, 2 bits, one row 40 / 21; 28672x8192, 4 bits, 16 rows 59 / 43; 4096x11008, 3 bits, 45
-            # rows 65 / 32
+            # here: 4096x4096, 2 bits, one row 40 / 13; 28672x8192, 4 bits, 16 rows 59 / 40; 4096x11008, 3 bits, 45
+            # rows 65 / 29
             y = ops.linear(_contiguous(x), _contiguous(trellis), self._tlut16(dev), _contiguous(SU), _contiguous(SV),
                            had_bits(had_left, K_left, True, dev) if K_left > 1 else None, K_left,
                            had_bits(had_right, K_right, False, dev) if K_right > 1 else None, K_right,
-                           m, n, self.cb.K, (n**-0.5) / self.scale, (m**-0.5) * self.scale, bs > 1 and self._long_sums(bs, m, n))
+                           m, n, self._modules["cb"].K, (n**-0.5) / self.scale, (m**-0.5) * self.scale,
+                           bs > 1 and self._long_sums(bs, m, n))
             return y if flat else y.view(*input.shape[:-1], m)
 
         # ---- input transform: fp16(H_L^T (x * SU) / sqrt(n) / 32)

@@ -11,7 +11,7 @@ import math
 import torch
 
 from . import _lib
-from ._lib import QTIP_F16, QTIP_F32, check, lib, require_cuda, stream_ptr
+from ._lib import QTIP_F16, QTIP_F32, check, host, lib, require_cuda, stream_ptr
 
 _DT = {torch.float16: QTIP_F16, torch.float32: QTIP_F32}
 _Tensor, _F16, _F32, _BITS = torch.Tensor, torch.float16, torch.float32, (2, 3, 4)
@@ -142,6 +142,20 @@ def decompress_matvec(packed, x, tlut, m, k, bits, out=None, split_k=True):
         check(lib().qtip_decompress_matvec(out.data_ptr(), packed.data_ptr(), x.data_ptr(), tlut.data_ptr(), m, k, bits,
                                            wsp, wsb, stream), "qtip_decompress_matvec")
     return out
+
+
+def matvec_row(packed, x, tlut, m, k, bits):
+    """decompress_matvec of operands that fit as they are, as a (1, m) tensor, in one native function; None for any other."""
+    if not (isinstance(packed, _Tensor) and packed.is_cuda) or _is_compiling() or bits not in _BITS or (m | k) & 31:
+        return None
+    dev = packed.device
+    stream = stream_ptr(dev)
+    wsp, wsb = 0, 0
+    if matvec_split(m, k, bits, dev) > 1:
+        ws = _workspace(dev, 16 * m * 4, stream)
+        wsp, wsb = ws.data_ptr(), ws.numel()
+    y = host().matvec(packed, x, tlut, m, k, bits, wsp, wsb, stream)
+    return y if y is None or isinstance(y, _Tensor) else check(y, "qtip_decompress_matvec")
 
 
 def decompress_matvec_parts(packed, x, tlut, m, k, bits, nparts=None):
@@ -351,7 +365,12 @@ def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, 
     fp16(scale_in * H_in(su * x)) @ decode(packed)^T) for x (rows, k) fp16 / fp32; the launches, and the results bit
     for bit, of rht, decompress_matvec_parts[_rht] (one row) or decompress_gemm (more), rht.  had_in / had_out: sign
     bits of the table orders (None for order 1).  long_sums: the product is decompress_gemm's with long sums."""
-    # a call whose operands fit asks no more than this; what does not goes through the checks one by one
+    # a call whose operands fit is one native function's; any other goes through the checks one by one
+    if isinstance(x, _Tensor) and x.is_cuda and not _is_compiling():
+        y = host().linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out,
+                          long_sums, _ALIGN_ROWS, stream_ptr(x.device))
+        if y is not None:
+            return y if isinstance(y, _Tensor) else check(y, "qtip_linear")
     if not (isinstance(x, _Tensor) and isinstance(packed, _Tensor) and isinstance(tlut, _Tensor)
             and isinstance(su, _Tensor) and isinstance(sv, _Tensor) and packed.is_cuda
             and packed.dtype in _PACKED_TYPES and tlut.dtype is su.dtype is _F16 and sv.dtype is _F32

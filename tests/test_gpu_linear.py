@@ -134,3 +134,44 @@ def test_rows_around_the_dense_route(m, k, bits, monkeypatch):
                 assert len(dense) == (1 if rows == edge else 0)
                 assert y.shape == (rows, m) and y.dtype == torch.float16
                 assert bool(((y[:, pick].double() - want).abs() <= 2.0**-11 * want.abs() + 2.0**-20 * size).all())
+
+
+def test_native_call_takes_what_fits_and_leaves_the_rest():
+    """The native functions behind a projection and the torch op: the bits of the way through the checks where the
+    operands fit, None for everything that they do not describe."""
+    from qtip_amd import _lib, ops
+    m, k, bits, rows = 96, 256, 3, 5
+    g = torch.Generator(device="cuda").manual_seed(3)
+    packed = torch.randint(-32768, 32768, (m * k * bits // 16,), dtype=torch.int16, generator=g, device="cuda")
+    tlut = torch.randn(512, 2, generator=g, device="cuda").half()
+    su, sv = torch.ones(k, device="cuda").half(), torch.ones(m, device="cuda")
+    x = torch.randn(rows, k, generator=g, device="cuda").half()
+    st = torch.cuda.current_stream().cuda_stream
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    order = get_hadK(m)[1]
+    table = had_bits(get_hadK(m)[0], order, False, "cuda")
+
+    def call(x=x, packed=packed, tlut=tlut, su=su, sv=sv, table=table, m=m, k=k, bits=bits, copy_rows=96):
+        return _lib.host().linear(x, packed, tlut, su, sv, None, 1, table, order, m, k, bits, 0.5, 2.0, False, copy_rows, st)
+
+    want = ops.rht(ops.decompress_gemm(packed, ops.rht(x, pre=su, scale=0.5, out_dtype=torch.float16), tlut, m, k, bits,
+                                       out_dtype=torch.float16), order=order, had_bits=table, post=sv, scale=2.0)
+    assert torch.equal(call(), want) and torch.equal(call(packed=packed.view(torch.uint8)), want)
+    wide = torch.zeros(rows, 2 * k, device="cuda").half()
+    off = torch.zeros(k + 1, device="cuda").half()[1:]
+    for kw in (dict(x=wide[:, ::2]), dict(x=wide[:, :k]), dict(x=x.double()), dict(x=x[0]), dict(x=x[:0]), dict(x=x.cpu()),
+               dict(packed=packed[:-1]), dict(packed=packed.float()), dict(packed=None), dict(tlut=tlut.float()),
+               dict(su=su.float()), dict(su=su[:-1]), dict(su=off, copy_rows=1), dict(sv=sv.half()), dict(table=None),
+               dict(table=table[:1] if table.numel() > 1 else table.float()), dict(m=m + 1), dict(k=k - 32), dict(bits=5),
+               dict(x=x.to_sparse())):
+        assert call(**kw) is None, kw
+    seen = []
+    torch.vmap(lambda v: seen.append(call(x=v)) or v)(x.expand(2, rows, k))
+    assert seen == [None]
+    row = x[:1]
+    assert torch.equal(_lib.host().matvec(packed, row, tlut, m, k, bits, 0, 0, st)[0],
+                       ops.decompress_matvec(packed, row, tlut, m, k, bits, split_k=False))
+    for args in ((packed, row.float(), tlut), (packed, x, tlut), (packed.cpu(), row, tlut), (packed, row, tlut[:256])):
+        assert _lib.host().matvec(*args, m, k, bits, 0, 0, st) is None
+    with pytest.raises(TypeError):
+        _lib.host().matvec(packed, row, tlut)

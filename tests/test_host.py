@@ -385,3 +385,11 @@ def test_module_without_a_kernel_in_host_memory(grad):
     want = t((t(x.double() * SU.double(), hl.T, k) / 32).half().double() @ w.T, hr, m) * SV.detach().double() * 32
     assert y.requires_grad == grad
     assert float((y.detach().double() - want).norm() / want.norm()) <= 2.0**-10  # the product's rounding to fp16, once
+
+
+def test_native_host_module_leaves_host_tensors_to_the_checks():
+    from qtip_amd import _lib
+    x = torch.zeros(1, 256, dtype=torch.float16)
+    packed, tlut = torch.zeros(256 * 256 // 8, dtype=torch.int16), torch.zeros(512, 2, dtype=torch.float16)
+    assert _lib.host().matvec(packed, x, tlut, 256, 256, 2, 0, 0, 0) is None
+    assert _lib.host().linear(x, packed, tlut, x[0], x[0].float(), None, 1, None, 1, 256, 256, 2, 1.0, 1.0, False, 96, 0) is None
