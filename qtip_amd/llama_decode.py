@@ -124,6 +124,8 @@ class DecoderLayer(nn.Module):
             self.qkv = proj('qkv', d, d + 2 * kvd)
             self.up_gate = proj('up_gate', d, 2 * cfg.ffn)
         else:
+            # (what stands for a product in front of the first layer's boundary)
+            self.register_buffer('no_parts', torch.zeros(2, d, dtype=torch.float32, device=device), persistent=False)
             self.q_proj = proj('q', d, d)
             self.k_proj = proj('k', d, kvd)
             self.v_proj = proj('v', d, kvd, K_v)
@@ -399,33 +401,37 @@ class DecoderLayer(nn.Module):
     def _group_chain(self, names, prev_parts, prev, residual, norm_weight):
         """One launch: boundary after `prev` (its output transform, residual, RMSNorm) and the
         matvecs of the projections `names`, which share that input."""
+        return self._chain_group(names, prev_parts, prev.SV, (prev.m**-0.5) * 32.0, residual, norm_weight)
+
+    def _chain_group(self, names, prev_parts, post, scale, residual, norm_weight):
         f = self._fused_linears()
         ls = [f[n] for n in names]
         return ops.decompress_matvec_group_chain(
-            [l.trellis for l in ls], [l.tlut for l in ls], [l.m for l in ls], ls[0].n, ls[0].K, prev_parts, prev.SV,
-            (prev.m**-0.5) * 32.0, residual, norm_weight, self.cfg.eps, [l.SU for l in ls], (ls[0].n**-0.5) / 32.0)
+            [l.trellis for l in ls], [l.tlut for l in ls], [l.m for l in ls], ls[0].n, ls[0].K, prev_parts, post, scale,
+            residual, norm_weight, self.cfg.eps, [l.SU for l in ls], (ls[0].n**-0.5) / 32.0)
 
     def _decode_grouped(self, x, k_cache, v_cache, pos, inv_freq, qkv_parts, next_layer):
         """decode_fused for separate projections, 8 launches: [boundary + q, k, v matvecs] (by the
-        previous layer), attention with the three output transforms in its prologue, o matvec with
+        previous layer, or the first for itself), attention with the three output transforms in its prologue, o matvec with
         its input transform, [boundary + gate, up matvecs], both output transforms (with SiLU * up in
         the same launch for vectors above 4096), [SiLU * up +] input transform of down, down
         matvec.  Returns (x, partial sums of the next layer's q, k, v)."""
         cfg = self.cfg
         f = self._fused_linears()
         qkv = [f[n] for n in ('q_proj', 'k_proj', 'v_proj')]
-        if qkv_parts is None:  # first layer: no boundary in front of it
-            vec = torch.cat([l(x, ops.PRE_RMSNORM, self.input_norm.weight, cfg.eps) for l in qkv], dim=-1)
-            attn = ops.decode_attention(vec.reshape(-1), k_cache, v_cache, pos, inv_freq, cfg.heads, cfg.kv_heads,
-                                        cfg.head_dim, key_splits=cfg.attn_key_splits)
-        else:
-            views, off = [], 0
-            for l in qkv:
-                views.append(qkv_parts[:, off:off + l.m])
-                off += l.m
-            attn = ops.decode_attention_rht3(views, [l.SV for l in qkv], [(l.m**-0.5) * 32.0 for l in qkv],
-                                             [l.br for l in qkv], [l.Kr for l in qkv], k_cache, v_cache, pos, inv_freq,
-                                             cfg.heads, cfg.kv_heads, cfg.head_dim, key_splits=cfg.attn_key_splits)
+        if qkv_parts is None:
+            # first layer: nothing in front of its boundary, which a vector of zeros leaves as it is (x + 0, RMSNorm, the
+            # input transforms).  us a token, three times [transform, matvec, transform], their concatenation and
+            # the plain attention / this one launch, 4 layers of 8192, 4 bits: 686 / 650
+            zeros = self.no_parts
+            qkv_parts, x = self._chain_group(('q_proj', 'k_proj', 'v_proj'), zeros[:1], zeros[1], 1.0, x, self.input_norm.weight)
+        views, off = [], 0
+        for l in qkv:
+            views.append(qkv_parts[:, off:off + l.m])
+            off += l.m
+        attn = ops.decode_attention_rht3(views, [l.SV for l in qkv], [(l.m**-0.5) * 32.0 for l in qkv],
+                                         [l.br for l in qkv], [l.Kr for l in qkv], k_cache, v_cache, pos, inv_freq,
+                                         cfg.heads, cfg.kv_heads, cfg.head_dim, key_splits=cfg.attn_key_splits)
         po = f['o'].matvec_from(attn.reshape(1, -1))
         gu_parts, x = self._group_chain(('gate_proj', 'up_proj'), po, f['o'], x, self.post_norm.weight)
         h, pre = self._gate_up_out(gu_parts)
