@@ -219,6 +219,15 @@ int qtip_linear_long(void* out, const void* x, int x_dtype, const void* packed, 
                      const float* sv, const uint32_t* had_in, int order_in, const uint32_t* had_out, int order_out, int m,
                      int k, int bits, int rows, float scale_in, float scale_out, void* workspace, size_t workspace_bytes,
                      void* stream);
+/* The same for fp16 rows, two or more, with the element-wise work around the projection inside the transforms' launches
+ * (pre_mode, norm_weight_f16, eps, residual_f16 as qtip_rht_fused takes them; x holds 2 k values a row with SiLU).  Results bit
+ * for bit those of qtip_rht_fused, qtip_decompress_gemm_f16 (long_sums: qtip_decompress_gemm_long_f16), qtip_rht_fused.
+ * workspace: that of qtip_linear or qtip_linear_long. */
+int qtip_linear_rows(void* out_f16, const void* x_f16, const void* packed, const void* tlut, const void* su_f16,
+                     const float* sv, const uint32_t* had_in, int order_in, const uint32_t* had_out, int order_out, int m,
+                     int k, int bits, int rows, float scale_in, float scale_out, int pre_mode,
+                     const void* norm_weight_f16, float eps, const void* residual_f16, int long_sums, void* workspace,
+                     size_t workspace_bytes, void* stream);
 
 /* The HYB table (quantlut_sym): tlut is (2^nbits, 2), contiguous; lut holds the value pair of every 16-bit state,
  * value v of state s at element s * stride_s + v * stride_v.  dtype: of both tables (expand), of lut (fold: nbits is

@@ -16,7 +16,7 @@ HOST_PATH = os.path.join(_HERE, "_qtip_host.so")
 
 QTIP_F16 = 0
 QTIP_F32 = 1
-ABI_VERSION = 24
+ABI_VERSION = 25
 
 _lib = None
 _host = None
@@ -61,6 +61,9 @@ _SIGNATURES = {
     "qtip_linear": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] + [ctypes.c_void_p] * 5 +
                     [ctypes.c_int, ctypes.c_void_p] + [ctypes.c_int] * 5 + [ctypes.c_float] * 2 +
                     [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "qtip_linear_rows": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int, ctypes.c_void_p] + [ctypes.c_int] * 5 +
+                         [ctypes.c_float] * 2 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p, ctypes.c_int,
+                                                 ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "qtip_linear_long_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int] * 6),
     "qtip_linear_long": (ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_int] + [ctypes.c_void_p] * 5 +
                          [ctypes.c_int, ctypes.c_void_p] + [ctypes.c_int] * 5 + [ctypes.c_float] * 2 +
@@ -145,7 +148,7 @@ def host():
         spec.loader.exec_module(module)
         module.bind(*(ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
                       for name in ("qtip_linear", "qtip_linear_long", "qtip_linear_workspace_bytes",
-                                   "qtip_linear_long_workspace_bytes", "qtip_decompress_matvec")))
+                                   "qtip_linear_long_workspace_bytes", "qtip_decompress_matvec", "qtip_linear_rows")))
         _host = module
     return _host
 

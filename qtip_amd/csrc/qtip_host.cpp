@@ -21,6 +21,7 @@ namespace {
 decltype(&qtip_linear) run_linear = nullptr, run_linear_long = nullptr;
 decltype(&qtip_linear_workspace_bytes) linear_bytes = nullptr, linear_long_bytes = nullptr;
 decltype(&qtip_decompress_matvec) run_matvec = nullptr;
+decltype(&qtip_linear_rows) run_rows = nullptr;
 
 // a tensor that a launch can be given: strided, contiguous GPU memory behind no wrapper (batches, fake or traced tensors)
 const at::Tensor* plain(PyObject* o, at::ScalarType type, int64_t numel) {
@@ -64,12 +65,16 @@ bool shape_ok(long m, long k, long bits) { return m > 0 && k > 0 && !((m | k) & 
 PyObject* failed(int rc) { return PyLong_FromLong(rc); }  // (the wrapper raises)
 
 // linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out, long_sums,
-// copy_rows, stream) -> tensor, an error code, or None.  From copy_rows rows on operands must start on 16 bytes.
+// copy_rows, stream[, pre_mode, norm_weight, eps, residual]) -> tensor, an error code, or None.  From copy_rows rows on
+// operands must start on 16 bytes.  With the last four: fp16 rows through qtip_linear_rows.
 PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
-  if (nargs != 17 || !run_linear) {
-    PyErr_SetString(PyExc_TypeError, "linear: 17 arguments, behind bind()");
+  const bool fused = nargs == 21;
+  if ((nargs != 17 && !fused) || !run_linear) {
+    PyErr_SetString(PyExc_TypeError, "linear: 17 or 21 arguments, behind bind()");
     return nullptr;
   }
+  const long pre_mode = fused ? PyLong_AsLong(a[17]) : 0;
+  const double eps = fused ? PyFloat_AsDouble(a[19]) : 0.;
   const long order_in = PyLong_AsLong(a[6]), order_out = PyLong_AsLong(a[8]), m = PyLong_AsLong(a[9]), k = PyLong_AsLong(a[10]),
              bits = PyLong_AsLong(a[11]), copy_rows = PyLong_AsLong(a[15]);
   const double scale_in = PyFloat_AsDouble(a[12]), scale_out = PyFloat_AsDouble(a[13]);
@@ -82,8 +87,10 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     if (xt.dim() != 2) Py_RETURN_NONE;
     const int64_t rows = xt.sym_sizes()[0].is_symbolic() ? 0 : xt.size(0);
     const at::ScalarType type = xt.scalar_type();
-    if (rows < 1 || rows > 65535 || xt.size(1) != k || (type != at::kHalf && type != at::kFloat)) Py_RETURN_NONE;
-    const at::Tensor *x = plain(a[0], type, rows * k), *packed = packed_words(a[1], m * k / 8 * bits),
+    const int64_t width = pre_mode == 2 ? 2 * k : k;  // [gate | up]
+    if (rows < (fused ? 2 : 1) || rows > 65535 || xt.size(1) != width || (type != at::kHalf && (type != at::kFloat || fused)))
+      Py_RETURN_NONE;
+    const at::Tensor *x = plain(a[0], type, rows * width), *packed = packed_words(a[1], m * k / 8 * bits),
                      *tlut = plain(a[2], at::kHalf, 1024), *su = plain(a[3], at::kHalf, k), *sv = plain(a[4], at::kFloat, m);
     if (!x || !packed || !tlut || !su || !sv) Py_RETURN_NONE;
     const c10::Device dev = packed->device();
@@ -93,6 +100,16 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
       Py_RETURN_NONE;
     const void *xp = x->data_ptr(), *pp = packed->data_ptr(), *tp = tlut->data_ptr(), *up = su->data_ptr();
     const float* vp = (const float*)sv->data_ptr();
+    const void *np = nullptr, *rp = nullptr;
+    if (fused) {
+      const at::Tensor *norm = a[18] == Py_None ? nullptr : plain(a[18], at::kHalf, k),
+                       *res = a[20] == Py_None ? nullptr : plain(a[20], at::kHalf, rows * m);
+      if ((a[18] != Py_None && (!norm || norm->device() != dev)) || (a[20] != Py_None && (!res || res->device() != dev)))
+        Py_RETURN_NONE;
+      if (norm) np = norm->data_ptr();
+      if (res) rp = res->data_ptr();
+      if (((uintptr_t)np | (uintptr_t)rp) & 15) Py_RETURN_NONE;
+    }
     if (rows >= copy_rows && (((uintptr_t)xp | (uintptr_t)up | (uintptr_t)vp) & 15)) Py_RETURN_NONE;
     const int dtype = type == at::kHalf ? QTIP_F16 : QTIP_F32;
     const size_t need = (long_sums ? linear_long_bytes : linear_bytes)((int)m, (int)k, (int)bits, (int)rows, (int)order_in, dtype);
@@ -101,9 +118,13 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     void *op = out.data_ptr(), *wp = ws.data_ptr();
     int rc;
     Py_BEGIN_ALLOW_THREADS;
-    rc = (long_sums ? run_linear_long : run_linear)(op, xp, dtype, pp, tp, up, vp, had_in, (int)order_in, had_out, (int)order_out,
-                                                    (int)m, (int)k, (int)bits, (int)rows, (float)scale_in, (float)scale_out, wp,
-                                                    need, stream);
+    if (fused)
+      rc = run_rows(op, xp, pp, tp, up, vp, had_in, (int)order_in, had_out, (int)order_out, (int)m, (int)k, (int)bits, (int)rows,
+                    (float)scale_in, (float)scale_out, (int)pre_mode, np, (float)eps, rp, long_sums, wp, need, stream);
+    else
+      rc = (long_sums ? run_linear_long : run_linear)(op, xp, dtype, pp, tp, up, vp, had_in, (int)order_in, had_out,
+                                                      (int)order_out, (int)m, (int)k, (int)bits, (int)rows, (float)scale_in,
+                                                      (float)scale_out, wp, need, stream);
     Py_END_ALLOW_THREADS;
     return rc ? failed(rc) : THPVariable_Wrap(out);
   } catch (const std::exception&) {  // (out of memory among them: the wrapper's way meets it again, and raises)
@@ -141,20 +162,21 @@ PyObject* matvec(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   }
 }
 
-// bind(addresses of qtip_linear, qtip_linear_long, their workspace sizes, qtip_decompress_matvec)
+// bind(addresses of qtip_linear, qtip_linear_long, their workspace sizes, qtip_decompress_matvec, qtip_linear_rows)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
-  if (nargs != 5) {
-    PyErr_SetString(PyExc_TypeError, "bind: 5 addresses");
+  if (nargs != 6) {
+    PyErr_SetString(PyExc_TypeError, "bind: 6 addresses");
     return nullptr;
   }
-  void* p[5];
-  for (int i = 0; i < 5; ++i) p[i] = PyLong_AsVoidPtr(a[i]);
+  void* p[6];
+  for (int i = 0; i < 6; ++i) p[i] = PyLong_AsVoidPtr(a[i]);
   if (PyErr_Occurred()) return nullptr;
   run_linear = (decltype(run_linear))p[0];
   run_linear_long = (decltype(run_linear_long))p[1];
   linear_bytes = (decltype(linear_bytes))p[2];
   linear_long_bytes = (decltype(linear_long_bytes))p[3];
   run_matvec = (decltype(run_matvec))p[4];
+  run_rows = (decltype(run_rows))p[5];
   Py_RETURN_NONE;
 }
 

@@ -1058,8 +1058,8 @@ __global__ __launch_bounds__(kRhtThreads) void rht_chain_kernel(
 // at 128 columns, two at 64: 3072 x 4096, 120 (2) 25.0/23.4; 5120 x 8192, 64 (4) 32.4/31.5, 5120 x 28672, 64 (8) 59.0/59.6;
 // 11008 x 4096, 17 (2) 28.4/27.9; 11008 x 8192, 64 (4) 45.7/47.1.  Narrower ones lose: 1728, 40 (8) 24.6/28.6; 448, 64 (4)
 // 18.3/19.1; 928 = 116 * 8, 17 (4) 19.5/24.3, 400 (2) 41.7/42.8.
-bool qtip_rht_takes_parts(int n, int order, int rows, int nparts) {
-  if (rows_form_size(n, order, rows)) return true;
+bool qtip_rht_takes_parts(int n, int order, int rows, int nparts, bool residual) {
+  if (!residual && rows_form_size(n, order, rows)) return true;
   if (rows < 2 || order < 1 || n % order || (n & 7)) return false;
   const int p = n / order;
   if (p & (p - 1)) return false;
@@ -1069,14 +1069,15 @@ bool qtip_rht_takes_parts(int n, int order, int rows, int nparts) {
   MixShape M{};
   int kt = 0;
   return mix_shape(n, order, rows, M, kt) && nparts << 5 <= 1 << M.logpp &&
-         rows >= mix_rows_min(order, n, OT, true, false, 1 << M.logS);
+         rows >= mix_rows_min(order, n, OT, true, residual, 1 << M.logS);
 }
 
 int qtip_rht_from_parts(void* out, int out_dtype, const float* parts, int nparts, int rows, int n, int order,
-                        const uint32_t* had_bits, const float* post, float scale, void* stream) {
+                        const uint32_t* had_bits, const float* post, float scale, const void* residual_f16, void* stream) {
   RhtParams P{};
   P.out = out;
   P.in = parts;
+  P.residual = (const _Float16*)residual_f16;
   P.had_bits = had_bits;
   P.post = post;
   P.part_stride = (size_t)rows * n;

@@ -24,9 +24,9 @@ QTIP_INTERNAL hipError_t qtip_gemm_allow_lds();
 QTIP_INTERNAL int qtip_gemm_ranges(int m, int k, int bits, int batch, bool fine);
 QTIP_INTERNAL int qtip_gemm_parts(float* parts, int nparts, const void* packed, const void* x_f16, const void* tlut, int m,
                                   int k, int bits, int batch, bool fine, void* stream);
-QTIP_INTERNAL bool qtip_rht_takes_parts(int n, int order, int rows, int nparts);
+QTIP_INTERNAL bool qtip_rht_takes_parts(int n, int order, int rows, int nparts, bool residual);
 QTIP_INTERNAL int qtip_rht_from_parts(void* out, int out_dtype, const float* parts, int nparts, int rows, int n, int order,
-                                      const uint32_t* had_bits, const float* post, float scale, void* stream);
+                                      const uint32_t* had_bits, const float* post, float scale, const void* residual_f16, void* stream);
 
 // Scratch of a batched product with fine or with long sums (qtip_decompress_gemm, qtip_decompress_gemm_long_f16)
 QTIP_INTERNAL size_t qtip_gemm_scratch(int m, int k, int bits, int batch, bool fine);

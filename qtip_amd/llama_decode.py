@@ -468,10 +468,18 @@ ROWS_MIN = 12
 def _rows_linear(lin, x, pre_mode=ops.PRE_NONE, norm=None, residual=None):
     """lin(f(x)) (+ residual) for x (rows, .) fp16: input transform with f in front, product, output transform."""
     n, m, dev = lin.in_features, lin.out_features, x.device
-    xt = ops.rht(x.contiguous(), order=lin.K_left, had_bits=had_bits(lin.had_left, lin.K_left, True, dev) if lin.K_left > 1 else None,
+    book, x = lin.codebook_class, x.contiguous()
+    if not book.takes_dense(x.shape[0], m, n):  # by one call of the library, which adds the ranges of a cut product on the way out
+        y = ops.linear_rows(x, lin.trellis, book._tlut16(dev), lin.SU, lin.SV,
+                            had_bits(lin.had_left, lin.K_left, True, dev) if lin.K_left > 1 else None, lin.K_left,
+                            had_bits(lin.had_right, lin.K_right, False, dev) if lin.K_right > 1 else None, lin.K_right, m, n,
+                            lin.K, (n**-0.5) / 32.0, (m**-0.5) * 32.0, book._long_sums(x.shape[0], m, n), pre_mode,
+                            None if norm is None else norm.weight, 0.0 if norm is None else norm.eps, residual)
+        if y is not None:
+            return y
+    xt = ops.rht(x, order=lin.K_left, had_bits=had_bits(lin.had_left, lin.K_left, True, dev) if lin.K_left > 1 else None,
                  pre=lin.SU, scale=(n**-0.5) / 32.0, out_dtype=torch.float16, pre_mode=pre_mode,
                  norm_weight=None if norm is None else norm.weight, eps=0.0 if norm is None else norm.eps)
-    book = lin.codebook_class
     y = book.rows_product(xt, lin.trellis, book._tlut16(dev), m, n)
     return ops.rht(y, order=lin.K_right, had_bits=had_bits(lin.had_right, lin.K_right, False, dev) if lin.K_right > 1 else None,
                    post=lin.SV, scale=(m**-0.5) * 32.0, out_dtype=torch.float16, residual=residual)

@@ -403,6 +403,17 @@ def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, 
 PRE_NONE, PRE_RMSNORM, PRE_SILU_MUL = 0, 1, 2
 
 
+def linear_rows(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out, long_sums,
+                pre_mode, norm_weight, eps, residual):
+    """linear() for fp16 rows, two or more, with the element-wise work around the projection in the transforms (as rht takes
+    it); None where an operand is not as the launches need it (contiguous, on 16 bytes)."""
+    if not (isinstance(x, _Tensor) and x.is_cuda) or _is_compiling():
+        return None
+    y = host().linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out, long_sums, 0,
+                      stream_ptr(x.device), pre_mode, norm_weight, eps, residual)
+    return y if y is None or isinstance(y, _Tensor) else check(y, "qtip_linear_rows")
+
+
 def rht(x, order=1, had_bits=None, pre=None, post=None, scale=None, out_dtype=None, in_parts=1, pre_mode=PRE_NONE,
         norm_weight=None, eps=0.0, residual=None):
     """out[r] = post * scale * (H_order (x) H_p)(pre * f(x[r])) (+ residual) over the last axis.

@@ -331,3 +331,30 @@ def test_positions_in_any_order(order):
     want, size = ((p @ t).transpose(0, 1).reshape(n, -1) for t in (vv, vv.abs()))
     # the rounding of the result and fp32 scores (as test_prefill_probabilities_are_not_rounded_to_fp16 derives)
     assert bool(((out.double() - want).abs() <= 2.0**-11 * want.abs() + 2.0**-25 + 2.0**-18 * size).all())
+
+
+@pytest.mark.parametrize("k,m,rows,mode,residual", [
+    (4096, 4096, 40, 0, True), (11008, 4096, 100, 2, True), (4096, 22016, 17, 1, False), (928, 1248, 33, 1, True),
+    (5120, 1728, 200, 2, False), (2048, 8192, 12, 1, True), (28672, 8192, 70, 2, True)])
+def test_projection_of_a_prompt_in_one_call(k, m, rows, mode, residual):
+    """linear_rows gives the bits of its launches one by one, the ranges of a cut product added on the way or not."""
+    from qtip_amd import ops
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    g = torch.Generator(device="cuda").manual_seed(k + rows)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    packed = torch.randint(-32768, 32768, (m * k * 2 // 16,), dtype=torch.int16, generator=g, device="cuda")
+    tlut, su, sv = rnd(512, 2).half(), torch.sign(rnd(k)).half(), rnd(m)
+    x, w = rnd(rows, 2 * k if mode == 2 else k).half(), (1 + 0.1 * rnd(k)).half()
+    res = rnd(rows, m).half() if residual else None
+    (hk, ki), (hm, ko) = get_hadK(k), get_hadK(m)
+    bi, bo = (had_bits(h, o, t, "cuda") if o > 1 else None for h, o, t in ((hk, ki, True), (hm, ko, False)))
+    for long_sums in (False, True):
+        got = ops.linear_rows(x, packed, tlut, su, sv, bi, ki, bo, ko, m, k, 2, 0.01, 0.02, long_sums, mode,
+                              w if mode == 1 else None, 1e-5, res)
+        xt = ops.rht(x, order=ki, had_bits=bi, pre=su, scale=0.01, out_dtype=torch.float16, pre_mode=mode,
+                     norm_weight=w if mode == 1 else None, eps=1e-5)
+        y = ops.decompress_gemm(packed, xt, tlut, m, k, 2, out_dtype=torch.float16, long_sums=long_sums)
+        want = ops.rht(y, order=ko, had_bits=bo, post=sv, scale=0.02, out_dtype=torch.float16, residual=res)
+        assert torch.equal(got, want), long_sums
+    assert ops.linear_rows(x[:, ::2], packed, tlut, su, sv, bi, ki, bo, ko, m, k, 2, 1.0, 1.0, False, 0, None, 0.0, None) is None
+    assert ops.linear_rows(x, packed, tlut, su, sv, bi, ki, bo, ko, m, k, 2, 1.0, 1.0, False, mode, w[1:], 0.0, res) is None
