@@ -241,6 +241,11 @@ size_t qtip_scale_columns_grad_workspace_bytes(int rows, int n);
 int qtip_scale_columns_grad(float* gx, float* gs, const float* g, const float* x, const void* s, int s_dtype, int rows,
                             int n, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Rotary tables of a prompt (model/llama.py:215-262): cos and sin, [n][2 half] fp16, of the fp32 products
+ * float(positions[i]) * inv_freq[d], d < half, each twice. */
+int qtip_rotary_tables(void* cos_f16, void* sin_f16, const void* positions_i64, const float* inv_freq, int n, int half,
+                       void* stream);
+
 /* Attention of n new tokens (a prompt, or a piece of one): rotary embedding of q and k (fp16 arithmetic; cos and sin
  * (n, head_dim) fp16), k and v into slots pos[0..n) of the caches (kv_heads, slots, head_dim), then every query i
  * against the cache slots up to pos[i].  q, k, v: fp16 rows, strides in elements (multiples of 8); out (n, heads *
@@ -379,6 +384,8 @@ int qtip_decode_attention_rht3(void* out_f16, const float* const* parts, int in_
 /* Final RMSNorm of the decoder for one vector: out = weight * fp16(x * rsqrt(mean(x^2) + eps))
  * (model/llama.py:129-135), n <= 16384, one launch instead of the module's six. */
 int qtip_rmsnorm(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int n, void* stream);
+/* The same for each of `rows` rows of n values, one after the other in memory. */
+int qtip_rmsnorm_rows(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int rows, int n, void* stream);
 
 /* Greedy token pick of the generation loop (eval/interactive_gen.py:43-69: argmax of the last
  * position's logits, copy into the next step's input, position + 1), all in device memory so a

@@ -602,9 +602,10 @@ namespace {
 
 constexpr int kHeadThreads = 1024;
 
-// out = w * fp16(x * rsqrt(mean(x^2) + eps)) for one vector (model/llama.py:129-135), one workgroup.
+// out = w * fp16(x * rsqrt(mean(x^2) + eps)) for a row of n (model/llama.py:129-135), one workgroup.
 // Bound by one cold read: V elements a load, 8 where the vectors start on 16 bytes and n is a multiple of 8 (one
-// element at a time, sixteen loads of either vector: 4096 6.1 us in a token, 8192 9.7; now 5.0 and 5.2).
+// element at a time, sixteen loads of either vector: 4096 6.1 us in a token, 8192 9.7; now 5.0 and 5.2).  Workgroups are as
+// wide as the row: 1000 rows of 4096 take 6 us, the eight library passes of the module's formula 64.
 template <int V>
 __global__ __launch_bounds__(kHeadThreads) void rmsnorm_kernel(_Float16* __restrict__ out,
                                                                const _Float16* __restrict__ x,
@@ -612,12 +613,14 @@ __global__ __launch_bounds__(kHeadThreads) void rmsnorm_kernel(_Float16* __restr
                                                                int n) {
   __shared__ float wsum[16];
   typedef _Float16 vec __attribute__((ext_vector_type(V)));
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+  x += (size_t)blockIdx.x * n;
+  out += (size_t)blockIdx.x * n;
   constexpr int MAXE = 16 / V;  // n <= 16384
   vec v[MAXE], g[MAXE];
 #pragma unroll
   for (int e = 0; e < MAXE; ++e) {
-    const int i = (tid + e * kHeadThreads) * V;
+    const int i = (tid + e * (int)blockDim.x) * V;
     v[e] = vec{};
     if (i < n) {
       v[e] = *reinterpret_cast<const vec*>(x + i);
@@ -634,11 +637,11 @@ __global__ __launch_bounds__(kHeadThreads) void rmsnorm_kernel(_Float16* __restr
   __syncthreads();
   float tot = 0.f;
 #pragma unroll
-  for (int q = 0; q < 16; ++q) tot += wsum[q];
+  for (int q = 0; q < 16; ++q) tot += q < waves ? wsum[q] : 0.f;
   const float rs = __builtin_amdgcn_rsqf(tot / (float)n + eps);
 #pragma unroll
   for (int e = 0; e < MAXE; ++e) {
-    const int i = (tid + e * kHeadThreads) * V;
+    const int i = (tid + e * (int)blockDim.x) * V;
     if (i < n) {
       vec y;
 #pragma unroll
@@ -712,16 +715,22 @@ __global__ __launch_bounds__(kHeadThreads) void greedy_pick_kernel(const _Float1
 
 }  // namespace
 
-extern "C" int qtip_rmsnorm(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int n,
-                            void* stream) {
+extern "C" int qtip_rmsnorm_rows(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int rows, int n,
+                                 void* stream) {
   if (!out_f16 || !x_f16 || !weight_f16) return QTIP_E_NULL;
-  if (n < 1 || n > 16 * kHeadThreads) return QTIP_E_SHAPE;
+  if (n < 1 || n > 16 * kHeadThreads || rows < 1) return QTIP_E_SHAPE;
   const bool wide = !(n & 7) && !((reinterpret_cast<uintptr_t>(out_f16) | reinterpret_cast<uintptr_t>(x_f16) |
                                    reinterpret_cast<uintptr_t>(weight_f16)) & 15);
   auto* kernel = wide ? rmsnorm_kernel<8> : rmsnorm_kernel<1>;
-  kernel<<<1, kHeadThreads, 0, (hipStream_t)stream>>>((_Float16*)out_f16, (const _Float16*)x_f16,
-                                                      (const _Float16*)weight_f16, eps, n);
+  const int loads = wide ? n >> 3 : n;
+  const int threads = loads < kHeadThreads ? (loads + 63) & ~63 : kHeadThreads;
+  kernel<<<rows, threads, 0, (hipStream_t)stream>>>((_Float16*)out_f16, (const _Float16*)x_f16,
+                                                    (const _Float16*)weight_f16, eps, n);
   return (int)hipGetLastError();
+}
+
+extern "C" int qtip_rmsnorm(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int n, void* stream) {
+  return qtip_rmsnorm_rows(out_f16, x_f16, weight_f16, eps, 1, n, stream);
 }
 
 extern "C" int qtip_greedy_pick(const void* logits_f16, int vocab, void* tok_i64, void* pos_i64,

@@ -735,6 +735,36 @@ def rmsnorm(x, weight, eps):
     return out
 
 
+def rmsnorm_rows(x, weight, eps):
+    """rmsnorm of every row of x (..., n)."""
+    require_cuda(x, "x", torch.float16)
+    require_cuda(weight, "weight", torch.float16)
+    n = weight.numel()
+    if x.dim() < 1 or x.shape[-1] != n or x.device != weight.device:
+        raise ValueError(f"rmsnorm: rows must hold {n} values and be where the weight is")
+    out = torch.empty_like(x)
+    if x.numel():
+        with _on(x.device):
+            check(lib().qtip_rmsnorm_rows(_ptr(out), _ptr(x), _ptr(weight), float(eps), x.numel() // n, n, stream_ptr(x.device)),
+                  "qtip_rmsnorm_rows")
+    return out
+
+
+def rotary_tables(positions, inv_freq):
+    """(cos, sin), each (n, 2 * len(inv_freq)) fp16, of float(positions) * inv_freq, every angle twice."""
+    require_cuda(positions, "positions", torch.int64)
+    require_cuda(inv_freq, "inv_freq", torch.float32)
+    n, half = positions.numel(), inv_freq.numel()
+    cos, sin = (torch.empty((n, 2 * half), dtype=torch.float16, device=positions.device) for _ in range(2))
+    if positions.device != inv_freq.device:
+        raise ValueError("positions and inv_freq are on different devices")
+    if n:
+        with _on(positions.device):
+            check(lib().qtip_rotary_tables(_ptr(cos), _ptr(sin), _ptr(positions), _ptr(inv_freq), n, half,
+                                           stream_ptr(positions.device)), "qtip_rotary_tables")
+    return cos, sin
+
+
 def greedy_pick(logits, tok, pos, history=None, history_base=0):
     """tok[0] = argmax(logits) (fp16 logits of one position, first index among equal maxima),
     history[pos - history_base] = tok when that slot exists, pos += 1 - the per-token bookkeeping

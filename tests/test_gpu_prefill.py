@@ -358,3 +358,35 @@ def test_projection_of_a_prompt_in_one_call(k, m, rows, mode, residual):
         assert torch.equal(got, want), long_sums
     assert ops.linear_rows(x[:, ::2], packed, tlut, su, sv, bi, ki, bo, ko, m, k, 2, 1.0, 1.0, False, 0, None, 0.0, None) is None
     assert ops.linear_rows(x, packed, tlut, su, sv, bi, ki, bo, ko, m, k, 2, 1.0, 1.0, False, mode, w[1:], 0.0, res) is None
+
+
+@pytest.mark.parametrize("rows,n", [(1, 8), (3, 17), (5, 1024), (2, 4096), (7, 8200), (1000, 4096), (2, 16384), (3, 16383)])
+def test_norm_of_rows(rows, n):
+    """rmsnorm_rows (and the module, which calls it) against the formula in float64 with its fp16 rounding points."""
+    from qtip_amd import ops
+    from qtip_amd.llama_decode import RMSNorm
+    g = torch.Generator(device="cuda").manual_seed(n)
+    store = torch.randn(rows * n + 1, generator=g, device="cuda").half()
+    mod = RMSNorm(n, 1e-5).cuda()
+    mod.weight.data = (1 + 0.1 * torch.randn(n, generator=g, device="cuda")).half()
+    for x in (store[:-1].view(rows, n), store[1:].view(rows, n)):  # on 16 bytes, and not
+        h = x.double()
+        ref = mod.weight.double() * (h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-5)).half().double()
+        got = ops.rmsnorm_rows(x, mod.weight, 1e-5)
+        assert torch.equal(mod(x), got) and torch.equal(mod(x.view(1, rows, n))[0], got)
+        # two roundings to fp16, either of which a value on the edge may take the other way
+        assert bool(((got.double() - ref).abs() <= 2e-3 * ref.abs() + 1e-7).all())
+    assert torch.equal(mod(x.float().half().requires_grad_(True)), mod.weight * (
+        x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-5)).half())  # gradients: the formula
+    assert mod(x.float()).dtype == torch.float32 and mod(x[:0]).shape == (0, n)
+
+
+@pytest.mark.parametrize("n,half", [(1, 32), (33, 64), (1000, 64), (5, 3)])
+def test_rotary_tables(n, half):
+    """The tables of the library passes, the angles' fp32 products and their cosines rounded to fp16, bit for bit."""
+    from qtip_amd import ops
+    inv = 10000.0 ** (-torch.arange(half, device="cuda", dtype=torch.float32) / half)
+    pos = torch.randint(0, 4096, (n,), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+    emb = torch.cat([pos.float()[:, None] * inv[None]] * 2, dim=-1)
+    cos, sin = ops.rotary_tables(pos, inv)
+    assert torch.equal(cos, emb.cos().half()) and torch.equal(sin, emb.sin().half())
