@@ -794,19 +794,18 @@ def generate(model, prompt_ids, max_new_tokens, use_graph=True, fused=True, temp
         return lg if sampling else pick(lg)
 
     def capture():
-        """Two eager steps (allocations, set-up), then the step recorded into a graph; the decode
+        """An eager step (allocations, set-up), then the step recorded into a graph; the decode
         state is put back afterwards, so a capture in the middle of a run leaves it untouched."""
         keep = (static_tok.clone(), static_pos.clone(), history.clone(), draw_counter.clone())
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
-            for _ in range(2):
-                step()
-                if on_device:  # the warm-up steps must not advance the decode
-                    static_tok.copy_(keep[0])
-                    static_pos.copy_(keep[1])
-                    history.copy_(keep[2])
-                    draw_counter.copy_(keep[3])
+            step()
+            if on_device:  # the warm-up step must not advance the decode
+                static_tok.copy_(keep[0])
+                static_pos.copy_(keep[1])
+                history.copy_(keep[2])
+                draw_counter.copy_(keep[3])
         torch.cuda.current_stream().wait_stream(s)
         # the warm-up wrote the cache slot of the current position with this token's k/v, which the
         # next step rewrites identically
