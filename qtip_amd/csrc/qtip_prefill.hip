@@ -262,8 +262,8 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
 
 }  // namespace
 
-extern "C" int qtip_rotary_tables(void* cos_f16, void* sin_f16, const void* positions_i64, const float* inv_freq, int n, int half,
-                       void* stream) {
+extern "C" int qtip_rotary_tables(void* cos_f16, void* sin_f16, const void* positions_i64, const float* inv_freq, int n,
+                                  int half, void* stream) {
   if (!cos_f16 || !sin_f16 || !positions_i64 || !inv_freq) return QTIP_E_NULL;
   if (n < 1 || half < 1 || (long)n * half > (1L << 38)) return QTIP_E_SHAPE;
   rotary_tables_kernel<<<(unsigned)(((long)n * half + kBlock - 1) / kBlock), kBlock, 0, (hipStream_t)stream>>>(
@@ -271,7 +271,7 @@ extern "C" int qtip_rotary_tables(void* cos_f16, void* sin_f16, const void* posi
   return (int)hipGetLastError();
 }
 
-int qtip_prefill_attention(void* out_f16, const void* q_f16, const void* k_f16, const void* v_f16,
+extern "C" int qtip_prefill_attention(void* out_f16, const void* q_f16, const void* k_f16, const void* v_f16,
                                       int q_stride, int k_stride, int v_stride, const void* cos_f16,
                                       const void* sin_f16, void* k_cache_f16, void* v_cache_f16, const int64_t* pos,
                                       int n, int heads, int kv_heads, int head_dim, int slots, void* stream) {
