@@ -6,8 +6,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <type_traits>
-
 #include "../../include/qtip_hip.h"
 #include "qtip_wht.h"
 
@@ -54,6 +52,13 @@ struct AttnXf {
 };
 
 typedef float float4a __attribute__((ext_vector_type(4)));
+typedef uint32_t uint4a __attribute__((ext_vector_type(4)));
+typedef _Float16 half8a __attribute__((ext_vector_type(8)));
+
+// value of lane 7 - i of the eight lanes (sums of four equal lanes: the other four)
+__device__ __forceinline__ float dpp_half_mirror(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));
+}
 
 // One workgroup per query head and key range.  qkv: [H*D | Hkv*D | Hkv*D] fp16 of the new
 // token; k_cache / v_cache: [Hkv][max_len][D] fp16; pos_ptr: position of the
@@ -70,41 +75,69 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
     const float* __restrict__ inv_freq, int H, int Hkv, int max_len, const AttnXf X, int nsplit,
     int keys_per_split, float* __restrict__ split_ws) {
   extern __shared__ __align__(16) uint8_t smem[];
-  float* q_s = reinterpret_cast<float*>(smem);   // [D] rotated query (as fp16 values)
-  float* k_s = q_s + kMaxHeadDim;                // [D] rotated new key
-  float* v_s = k_s + kMaxHeadDim;                // [D] new value
-  float* red = v_s + kMaxHeadDim;                // [32] reductions
-  float* acc = red + 32;                         // [TG][D] partial outputs, TG*D = 8192
-  float* p_s = acc + 8192;                       // [max_len] scores / probabilities
+  float* new_s = reinterpret_cast<float*>(smem);  // [3][kMaxHeadDim] rotated query, rotated new key, new value (fp16 values)
+  float* swap_s = new_s + 3 * kMaxHeadDim;        // [3][kMaxHeadDim] last level of the prologue's transform
+  float* red = swap_s + 3 * kMaxHeadDim;          // [2][16] maxima and sums of the waves
+  float* acc = red + 32;                          // [16][D] outputs of the waves; the prologue's [3][16][D] before that
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // grid = (query heads per kv head, kv heads): no integer division on the way to the loads
   const int rep = gridDim.x, kvh = blockIdx.y, h = kvh * rep + blockIdx.x;
   const int pos = (int)pos_ptr[0];
+  constexpr int LOGD = D == 64 ? 6 : (D == 128 ? 7 : 8);
   constexpr int half = D >> 1;
-  const _Float16* q_in = qkv + (size_t)h * D;
-  const _Float16* k_in = qkv + (size_t)H * D + (size_t)kvh * D;
-  const _Float16* v_in = qkv + (size_t)(H + Hkv) * D + (size_t)kvh * D;
   _Float16* kc = k_cache + (size_t)kvh * max_len * D;
   _Float16* vc = v_cache + (size_t)kvh * max_len * D;
+  // threads tid < 3 * D hold element c of the new token's query (s3 = 0), key (1) and value (2)
+  const int s3 = tid >> LOGD, c = tid & (D - 1);
+  const float freq = tid < 2 * D ? inv_freq[c & (half - 1)] : 0.f;
+  float postv = 1.f, postp = 1.f;
+  _Float16 own = (_Float16)0.f, pair = (_Float16)0.f;  // element c and the one that it is rotated with
+  if constexpr (!XF) {
+    if (tid < 3 * D) {
+      const _Float16* e = qkv + (size_t)(s3 == 0 ? h : (s3 == 1 ? H + kvh : H + Hkv + kvh)) * D;
+      own = e[c];
+      pair = e[c ^ half];
+    }
+  }
 
-  // rotary angle of this thread's dimension, requested before anything else: the angle is the fp32
-  // product the reference forms; its reduction to a fraction of a turn is done in fp64 (exact to
-  // 2^-29 of a turn at position 4096), the hardware cos / sin take turns.  (cosf / sinf with their
-  // large-argument paths cost ~0.5 us on this kernel's critical path.)
+  // rotary angle of the thread's element: the fp32 product the reference forms; its reduction to a fraction of a
+  // turn is done in fp64 (exact to 2^-29 of a turn at position 4096), the hardware cos / sin take
+  // turns.  (cosf / sinf with their large-argument paths cost ~0.5 us on this kernel's critical path.)
   _Float16 rc = (_Float16)1.f, rs = (_Float16)0.f;
-  if (tid < D) {
-    const float ang = (float)pos * inv_freq[tid < half ? tid : tid - half];
+  auto rotary = [&] {
+    const float ang = (float)pos * freq;
     const double turns = (double)ang * 0.15915494309189535;
     const float fr = (float)(turns - __builtin_floor(turns));
     rc = (_Float16)__builtin_amdgcn_cosf(fr);
     rs = (_Float16)__builtin_amdgcn_sinf(fr);
-  }
+  };
+
+  // ---- the cached keys [k0, kend) of this workgroup, in units of U: wave w takes keys t0 + w * KPW .. + KPW - 1 of
+  // a unit, a key of D values on D / 8 lanes.  One pass with a running maximum, a wave by itself, NU units of keys and
+  // values in flight, the first ones from before the transform's last levels and the rotary embedding on.  The part of the
+  // launch that grows with the keys is what one CU draws from memory, 50 to 60 bytes a ns: more in flight is no
+  // faster (a token of 8 layers, 500 keys: two units 548 us, four 549, eight 560), and loads of nothing take the
+  // memory unit 0.15 us a unit.  us a token of 8 layers of 4096 (32 heads of 128), 60 / 200 / 500 / 900 keys, scores and
+  // values in two passes over all keys with six barriers / here: 531 537 562 599 / 523 529 549 587; separate
+  // projections 528 537 562 / 520 527 547.
+  constexpr int LPK = D / 8, KPW = 64 / LPK, U = 16 * KPW, NU = 2;
+  const int nkeys = pos + 1 < max_len ? pos + 1 : max_len;
+  const int k0 = (int)blockIdx.z * keys_per_split;  // this workgroup's keys: [k0, k1)
+  const int k1 = k0 + keys_per_split < nkeys ? k0 + keys_per_split : nkeys;
+  const int kend = k1 < pos ? k1 : pos;             // (the new key comes from LDS)
+  const __amdgpu_buffer_rsrc_t rs_k = __builtin_amdgcn_make_buffer_rsrc(kc, 0, max_len * D * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_v = __builtin_amdgcn_make_buffer_rsrc(vc, 0, max_len * D * 2, 0x00020000);
+  const int tl = wave * KPW + lane / LPK, dl = lane & (LPK - 1);
+  // the keys and values of a unit are requested together; a lane offset past the end of the cache returns zeros
+  auto request = [&](uint4a& k, uint4a& v, int t0) {
+    const int off = t0 + tl < kend ? ((t0 + tl) * D + dl * 8) * 2 : 0x7FFFFF00;
+    k = __builtin_amdgcn_raw_buffer_load_b128(rs_k, off, 0, 0);
+    v = __builtin_amdgcn_raw_buffer_load_b128(rs_v, off, 0, 0);
+  };
 
   if constexpr (XF) {
     static_assert(D == 64 || D == 128, "the transform prologue holds 3 x 16 x D partial sums in LDS");
-    constexpr int LOGD = D == 64 ? 6 : 7;
     constexpr int G = D / 4, R = kAttnThreads / G;  // float4 column groups, chunk rows per pass
-    constexpr int QP = 4, WP = 2;                   // chunk rows and partial sums in flight per thread
     constexpr bool SEP = XF == 2;
     const int g = tid & (G - 1), r = tid >> (LOGD - 2);
     // slices: q of head h, k and v of its kv head - of the one vector, or each of its own
@@ -118,155 +151,103 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
       bb[s3] = (off[s3] >> LOGD) & ((1 << lgb[s3]) - 1);
     }
     // the epilogue's operands, requested with everything else
-    const int s3 = tid >> LOGD, c = tid & (D - 1);
     const int sx = SEP ? (s3 < 3 ? s3 : 0) : 0;  // descriptor of this thread's slice
-    float postv = 1.f;
-    const float* postp = sx == 0 ? X.post[0] : (sx == 1 ? X.post[1] : X.post[2]);
-    if (tid < 3 * D && postp) postv = postp[off[s3 < 3 ? s3 : 0] + c];
-    const float scalev = sx == 0 ? X.scale[0] : (sx == 1 ? X.scale[1] : X.scale[2]);
+    const float* post = sx == 0 ? X.post[0] : (sx == 1 ? X.post[1] : X.post[2]);
+    if (tid < 3 * D && post) {
+      const float* e = post + (s3 == 0 ? off[0] : (s3 == 1 ? off[1] : off[2]));
+      postv = e[c];
+      postp = e[c ^ half];
+    }
     float a[3][4];  // (plain arrays: element-wise bit operations on vector-typed values went wrong in the compiler)
 #pragma unroll
-    for (int s3 = 0; s3 < 3; ++s3)
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) a[s3][e] = 0.f;
-    if constexpr (SEP) {
-      // three vectors: the rows of all three are requested in one go, one chunk row and two
-      // partial sums per slice in flight (more would spill)
-      constexpr int Q2 = 1, W2 = 2;
-      int nrows[3], maxrows = 0;
+      for (int e = 0; e < 4; ++e) a[i][e] = 0.f;
+    // (chunk rows past the last are out of the descriptor's range and come back as zeros)
+    // NV vectors, QP chunk rows and WP partial sums of each in flight (more would spill)
+    constexpr int NV = SEP ? 3 : 1, QP = SEP ? 1 : 4, WP = 2;
+    auto load = [&](float4a (&raw)[NV][QP][WP], int j0, int w0) {
 #pragma unroll
-      for (int s3 = 0; s3 < 3; ++s3) {
-        nrows[s3] = X.n[s3] >> LOGD;
-        maxrows = nrows[s3] > maxrows ? nrows[s3] : maxrows;
-      }
-      for (int j0 = 0; j0 < maxrows; j0 += Q2 * R) {
-        float v[3][Q2][4];
-        uint32_t hw[3][Q2];
+      for (int u = 0; u < WP; ++u)
 #pragma unroll
-        for (int s3 = 0; s3 < 3; ++s3) {
-          // table words: with order 1 the index is 0 and the word is masked out (any readable address does)
-          const uint32_t* hb = X.order[s3] > 1 ? X.had_bits[s3] : reinterpret_cast<const uint32_t*>(X.parts[s3]);
-#pragma unroll
-          for (int q = 0; q < Q2; ++q) {
-            const int j = j0 + r + q * R;
-            const int jc = j < nrows[s3] ? j : 0;
-            const unsigned bit = (unsigned)(jc >> lgb[s3]) * X.order[s3] + iK[s3];
-            hw[s3][q] = hb[bit >> 5] >> (bit & 31);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[s3][q][e] = 0.f;
-          }
-        }
-        for (int w0 = 0; w0 < X.in_parts; w0 += W2) {
-          float4a raw[3][Q2][W2];
-#pragma unroll
-          for (int u = 0; u < W2; ++u) {
-            if (w0 + u < X.in_parts) {
-#pragma unroll
-              for (int s3 = 0; s3 < 3; ++s3)
-#pragma unroll
-                for (int q = 0; q < Q2; ++q) {
-                  const int j = j0 + r + q * R;
-                  const int jc = j < nrows[s3] ? j : 0;
-                  raw[s3][q][u] = *reinterpret_cast<const float4a*>(
-                      X.parts[s3] + (size_t)(w0 + u) * X.part_stride + ((size_t)jc << LOGD) + 4 * g);
-                }
-            } else {
-#pragma unroll
-              for (int s3 = 0; s3 < 3; ++s3)
-#pragma unroll
-                for (int q = 0; q < Q2; ++q) raw[s3][q][u] = float4a{0.f, 0.f, 0.f, 0.f};
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < W2; ++u)
-#pragma unroll
-            for (int s3 = 0; s3 < 3; ++s3)
-#pragma unroll
-              for (int q = 0; q < Q2; ++q) {
-                v[s3][q][0] += raw[s3][q][u].x;
-                v[s3][q][1] += raw[s3][q][u].y;
-                v[s3][q][2] += raw[s3][q][u].z;
-                v[s3][q][3] += raw[s3][q][u].w;
-              }
-        }
-#pragma unroll
-        for (int s3 = 0; s3 < 3; ++s3) {
-          const uint32_t omask = X.order[s3] > 1 ? 1u : 0u;
-          const int bmask = (1 << lgb[s3]) - 1;
-#pragma unroll
-          for (int q = 0; q < Q2; ++q) {
-            const int j = j0 + r + q * R;
-            if (j < nrows[s3]) {
-              const uint32_t sg = (((hw[s3][q] & omask) ^ (uint32_t)__builtin_popcount(bb[s3] & j & bmask)) & 1u) << 31;
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                a[s3][e] += __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[s3][q][e]) ^ sg);
-            }
-          }
-        }
-      }
-    } else {
-    const int logb = lgb[0], bmask = (1 << logb) - 1;
-    const int nrows = X.n[0] >> LOGD;
-    // table words: with order 1 the index is 0 and the word is masked out (any readable address does)
-    const uint32_t* hb = X.order[0] > 1 ? X.had_bits[0] : reinterpret_cast<const uint32_t*>(X.parts[0]);
-    const uint32_t omask = X.order[0] > 1 ? 1u : 0u;
-    for (int j0 = 0; j0 < nrows; j0 += QP * R) {
-      float v[QP][4];
-      uint32_t hw[QP][3];
-#pragma unroll
-      for (int q = 0; q < QP; ++q) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[q][e] = 0.f;
-        const int j = j0 + r + q * R;
-        const int jc = j < nrows ? j : 0;
-#pragma unroll
-        for (int s3 = 0; s3 < 3; ++s3) {
-          const unsigned bit = (unsigned)(jc >> logb) * X.order[0] + iK[s3];
-          hw[q][s3] = hb[bit >> 5] >> (bit & 31);
-        }
-      }
-      for (int w0 = 0; w0 < X.in_parts; w0 += WP) {
-        float4a raw[QP][WP];
-#pragma unroll
-        for (int u = 0; u < WP; ++u) {
+        for (int i = 0; i < NV; ++i) {
           if (w0 + u < X.in_parts) {
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>(X.parts[i] + (size_t)(w0 + u) * X.part_stride), 0, X.n[i] * 4, 0x00020000);
 #pragma unroll
-            for (int q = 0; q < QP; ++q) {
-              const int j = j0 + r + q * R;
-              const int jc = j < nrows ? j : 0;
-              raw[q][u] = *reinterpret_cast<const float4a*>(X.parts[0] + (size_t)(w0 + u) * X.part_stride +
-                                                            ((size_t)jc << LOGD) + 4 * g);
-            }
+            for (int q = 0; q < QP; ++q)
+              raw[i][q][u] = __builtin_bit_cast(
+                  float4a, __builtin_amdgcn_raw_buffer_load_b128(rs, (((j0 + r + q * R) << LOGD) + 4 * g) * 4, 0, 0));
           } else {
 #pragma unroll
-            for (int q = 0; q < QP; ++q) raw[q][u] = float4a{0.f, 0.f, 0.f, 0.f};
+            for (int q = 0; q < QP; ++q) raw[i][q][u] = float4a{0.f, 0.f, 0.f, 0.f};
           }
         }
+    };
+    // the table words of the rows.  (With order 1 the index is 0 and the word is masked out: any readable address does.)
+    auto words = [&](uint32_t (&hw)[QP][3], int j0) {
 #pragma unroll
-        for (int u = 0; u < WP; ++u)
+      for (int i = 0; i < 3; ++i) {
+        const int x = SEP ? i : 0;
+        const uint32_t* hb = X.order[x] > 1 ? X.had_bits[x] : reinterpret_cast<const uint32_t*>(X.parts[x]);
+        const int nrows = X.n[x] >> LOGD;
 #pragma unroll
-          for (int q = 0; q < QP; ++q) {
-            v[q][0] += raw[q][u].x;
-            v[q][1] += raw[q][u].y;
-            v[q][2] += raw[q][u].z;
-            v[q][3] += raw[q][u].w;
-          }
-      }
-#pragma unroll
-      for (int q = 0; q < QP; ++q) {
-        const int j = j0 + r + q * R;
-        if (j < nrows) {
-#pragma unroll
-          for (int s3 = 0; s3 < 3; ++s3) {
-            const uint32_t sg = (((hw[q][s3] & omask) ^ (uint32_t)__builtin_popcount(bb[s3] & j & bmask)) & 1u) << 31;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              a[s3][e] += __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[q][e]) ^ sg);
-          }
+        for (int q = 0; q < QP; ++q) {
+          const int j = j0 + r + q * R;
+          const unsigned bit = (unsigned)((j < nrows ? j : 0) >> lgb[x]) * X.order[x] + iK[i];
+          hw[q][i] = hb[bit >> 5] >> (bit & 31);
         }
       }
+    };
+    auto add = [&](float (&v)[NV][QP][4], const float4a (&raw)[NV][QP][WP]) {
+#pragma unroll
+      for (int u = 0; u < WP; ++u)
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+          for (int q = 0; q < QP; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[i][q][e] += raw[i][q][u][e];
+    };
+    auto pass = [&](float4a (&raw)[NV][QP][WP], const uint32_t (&hw)[QP][3], int j0) {
+      float v[NV][QP][4] = {};
+      add(v, raw);
+      for (int w0 = WP; w0 < X.in_parts; w0 += WP) {
+        load(raw, j0, w0);
+        add(v, raw);
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int x = SEP ? i : 0;
+        const uint32_t omask = X.order[x] > 1 ? 1u : 0u;
+        const int bmask = (1 << lgb[x]) - 1;
+#pragma unroll
+        for (int q = 0; q < QP; ++q) {
+          const uint32_t sg =
+              (((hw[q][i] & omask) ^ (uint32_t)__builtin_popcount(bb[i] & (j0 + r + q * R) & bmask)) & 1u) << 31;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            a[i][e] += __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[x][q][e]) ^ sg);
+        }
+      }
+    };
+    int maxrows = X.n[0] >> LOGD;
+    if constexpr (SEP) {
+      maxrows = X.n[1] >> LOGD > maxrows ? X.n[1] >> LOGD : maxrows;
+      maxrows = X.n[2] >> LOGD > maxrows ? X.n[2] >> LOGD : maxrows;
     }
+    {
+      float4a raw[NV][QP][WP];
+      uint32_t hw[QP][3];
+      words(hw, 0);
+      load(raw, 0, 0);
+      rotary();
+      pass(raw, hw, 0);
+      for (int j0 = QP * R; j0 < maxrows; j0 += QP * R) {
+        words(hw, j0);
+        load(raw, j0, 0);
+        pass(raw, hw, j0);
+      }
     }
     // rows that share a wave, then one partial slice per wave
 #pragma unroll
@@ -281,184 +262,153 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
         *reinterpret_cast<float4a*>(acc + (s3 * 16 + wave) * D + 4 * g) =
             float4a{a[s3][0], a[s3][1], a[s3][2], a[s3][3]};
     }
+  } else {
+    rotary();
+  }
+
+  // (the registers of the partial sums are free)
+  uint4a kb[NU], vb[NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) request(kb[u], vb[u], k0 + u * U);
+  if constexpr (XF) {
+    constexpr bool SEP = XF == 2;
+    const int sx = SEP ? (s3 < 3 ? s3 : 0) : 0;
+    const float scalev = sx == 0 ? X.scale[0] : (sx == 1 ? X.scale[1] : X.scale[2]);
     __syncthreads();
-    float y = 0.f;
+    // the other half of a slice, behind the last level of the transform, is what an element is rotated with
+    float y = 0.f, z = 0.f;
     if (tid < 3 * D) {
 #pragma unroll
       for (int w = 0; w < 16; ++w) y += acc[(s3 * 16 + w) * D + c];
       y = qtip_wht::wht_lanes(y, 6, lane);
-      if (D > 64) q_s[s3 * kMaxHeadDim + c] = y;
+      if constexpr (D > 64) swap_s[s3 * kMaxHeadDim + c] = y;
+      else z = qtip_wht::lane_xor(y, 5);
     }
-    __syncthreads();  // the partial slices are consumed: their space takes the fp16 result
-    _Float16* h_s = reinterpret_cast<_Float16*>(acc);
-    if (tid < 3 * D) {
-      if (D > 64) {
-        const float other = q_s[s3 * kMaxHeadDim + (c ^ 64)];
+    if constexpr (D > 64) {
+      __syncthreads();
+      if (tid < 3 * D) {
+        const float other = swap_s[s3 * kMaxHeadDim + (c ^ 64)];
+        z = (c & 64) ? other + y : y - other;
         y = (c & 64) ? other - y : y + other;
       }
-      h_s[s3 * D + c] = (_Float16)(y * scalev * postv);
     }
-    __syncthreads();
+    own = (_Float16)(y * scalev * postv);
+    pair = (_Float16)(z * scalev * postp);
   }
-  const _Float16* h_s = reinterpret_cast<const _Float16*>(acc);
-  auto QV = [&](int i) -> _Float16 { return XF ? h_s[i] : q_in[i]; };
-  auto KV = [&](int i) -> _Float16 { return XF ? h_s[D + i] : k_in[i]; };
-  auto VV = [&](int i) -> _Float16 { return XF ? h_s[2 * D + i] : v_in[i]; };
 
   // ---- rotary embedding in fp16 arithmetic: x*cos + rotate_half(x)*sin
-  if (tid < D) {
-    const _Float16 c = rc, s = rs;
-    const _Float16 q0 = QV(tid), k0 = KV(tid), v0 = VV(tid);
-    const _Float16 qr = tid < half ? (_Float16)(-(float)QV(tid + half)) : QV(tid - half);
-    const _Float16 kr = tid < half ? (_Float16)(-(float)KV(tid + half)) : KV(tid - half);
-    const _Float16 qe = (_Float16)((float)(_Float16)((float)q0 * (float)c) + (float)(_Float16)((float)qr * (float)s));
-    const _Float16 ke = (_Float16)((float)(_Float16)((float)k0 * (float)c) + (float)(_Float16)((float)kr * (float)s));
-    q_s[tid] = (float)qe;
-    k_s[tid] = (float)ke;
-    v_s[tid] = (float)v0;
-    if (blockIdx.x == 0 && blockIdx.z == 0 && pos < max_len) {
-      kc[(size_t)pos * D + tid] = ke;
-      vc[(size_t)pos * D + tid] = v0;
-    }
+  if (tid < 3 * D) {
+    const _Float16 rot = c < half ? (_Float16)(-(float)pair) : pair;
+    _Float16 e = (_Float16)((float)(_Float16)((float)own * (float)rc) + (float)(_Float16)((float)rot * (float)rs));
+    if (s3 == 2) e = own;
+    new_s[s3 * kMaxHeadDim + c] = (float)e;
+    if (s3 && blockIdx.x == 0 && blockIdx.z == 0 && pos < max_len) (s3 == 1 ? kc : vc)[(size_t)pos * D + c] = e;
   }
   __syncthreads();
 
-  // ---- scores: 8 lanes per key (16 dims each), 128 keys per pass
+  // ---- softmax(q k) v of the lane group's keys with a running maximum: mx, the sum of exponentials l and the
+  // unnormalised outputs o (dims 8 * dl ..); the first group of wave 0 starts with the new key
   const float sm_scale = rsqrtf((float)D);
-  const int nkeys = pos + 1 < max_len ? pos + 1 : max_len;
-  const int k0 = (int)blockIdx.z * keys_per_split;                       // this workgroup's keys: [k0, k1)
-  const int k1 = k0 + keys_per_split < nkeys ? k0 + keys_per_split : nkeys;
-  const int sub = tid & 7, kq = tid >> 3;
-  constexpr int dper = D >> 3;  // dims per lane (multiple of 8: D % 64 == 0)
-  float mx = -INFINITY;
-  // KU keys per thread group and round, all of their loads issued before the first use: two, or one where no more than
-  // RK are left.  (Four keys and eight values in flight, and 64-bit addresses for each, did not fit a thread's 128
-  // registers: the spills cost more than the wider rounds gained.  us, spilling / now, 32 heads of 128 on 32 kv heads,
-  // cold caches: 60 keys 6.6 / 5.3, 300 8.3 / 9.2 (the second round of either), 500 11.1 / 10.3, 1000 21.9 / 15.6; 64 heads
-  // on 8, 900 keys 19.4 / 13.8; 32 heads on 8 in 8 ranges, 2000 keys 17.5 / 16.2, 4000 21.3 / 20.0.)
-  constexpr int KU = 2, RK = kAttnThreads / 8;
-  auto cache_row = [&](const _Float16* base, int t, int d) {  // 32-bit offset from a uniform base
-    const int tc = (t < k1 && t != pos) ? t : 0;              // clamped: the new key comes from LDS
-    return reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base) + (uint32_t)(tc * D + d) * 2u);
+  float q[8], o[8], mx = -INFINITY, l = 0.f;
+  auto row_sum = [&](float s) {  // over the lanes of a key
+    s += qtip_wht::lane_xor(s, 0);
+    s += qtip_wht::lane_xor(s, 1);
+    s += dpp_half_mirror(s);
+    if constexpr (LPK >= 16) s += qtip_wht::lane_xor(s, 3);
+    if constexpr (LPK >= 32) s += qtip_wht::lane_xor(s, 4);
+    return s;
   };
-  auto key_round = [&](auto n, int t0) {
-    constexpr int N = decltype(n)::value;
-    uint4 raw[N][dper / 8];
-#pragma unroll
-    for (int u = 0; u < N; ++u) {
-      const uint4* kr = cache_row(kc, t0 + kq + u * RK, sub * dper);
-#pragma unroll
-      for (int d8 = 0; d8 < dper / 8; ++d8) raw[u][d8] = kr[d8];
-    }
-#pragma unroll
-    for (int u = 0; u < N; ++u) {
-      const int t = t0 + kq + u * RK;
-      float s = 0.f;
-      if (t == pos) {
-        for (int d = 0; d < dper; ++d) s += q_s[sub * dper + d] * k_s[sub * dper + d];
-      } else {
-#pragma unroll
-        for (int d8 = 0; d8 < dper / 8; ++d8) {
-          const _Float16* hv = reinterpret_cast<const _Float16*>(&raw[u][d8]);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) s += q_s[sub * dper + d8 * 8 + e] * (float)hv[e];
-        }
-      }
-      s += qtip_wht::lane_xor(s, 0);
-      s += qtip_wht::lane_xor(s, 1);
-      s += qtip_wht::lane_xor(s, 2);
-      s *= sm_scale;
-      if (t < k1) {
-        if (sub == 0) p_s[t - k0] = s;
-        mx = fmaxf(mx, s);
-      }
-    }
-  };
-  for (int t0 = k0; t0 < k1; t0 += KU * RK) {
-    if (k1 - t0 <= RK) key_round(std::integral_constant<int, 1>{}, t0);
-    else key_round(std::integral_constant<int, KU>{}, t0);
-  }
-  // the values of the first round (keys tg, tg + TG, ...: all of them up to 256 keys of 128 values) are requested
-  // here, before the softmax reductions: their addresses do not depend on the scores.  (Requesting
-  // the first round of keys ahead of the rotary embedding in the same way measured slower.)
-  constexpr int DG = D >> 3, TG = kAttnThreads / DG;  // 16 dim groups, 64 key groups for D = 128
-  constexpr int VU = 4;  // values per thread and round, loaded before the first use
-  const int dg = tid % DG, tg = tid / DG;
-  uint4 vfirst[VU];
-#pragma unroll
-  for (int u = 0; u < VU; ++u) vfirst[u] = *cache_row(vc, k0 + tg + u * TG, dg * 8);
-  mx = wave_reduce_max(mx);
-  if (lane == 0) red[wave] = mx;
-  __syncthreads();
-  mx = red[0];
-#pragma unroll
-  for (int w = 1; w < 16; ++w) mx = fmaxf(mx, red[w]);
-  float sum = 0.f;
-  for (int t = tid; t < k1 - k0; t += kAttnThreads) {
-    const float e = __expf(p_s[t] - mx);
-    p_s[t] = e;
-    sum += e;
-  }
-  sum = wave_reduce_sum(sum);
-  __syncthreads();  // everyone has read red[] (max) and written p_s
-  if (lane == 0) red[16 + wave] = sum;
-  __syncthreads();
-  float tot = 0.f;
-#pragma unroll
-  for (int w = 0; w < 16; ++w) tot += red[16 + w];
-  const float inv = 1.f / tot;
-
-  // ---- output: thread (tg, dg) sums keys tg, tg+TG, ... for dims 8*dg .. 8*dg+7
-  float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int t0 = k0 + tg; t0 < k1; t0 += VU * TG) {
-    uint4 raw[VU];
-    if (t0 == k0 + tg) {
-#pragma unroll
-      for (int u = 0; u < VU; ++u) raw[u] = vfirst[u];
-    } else {
-#pragma unroll
-      for (int u = 0; u < VU; ++u) raw[u] = *cache_row(vc, t0 + u * TG, dg * 8);
-    }
-#pragma unroll
-    for (int u = 0; u < VU; ++u) {
-      const int t = t0 + u * TG;
-      if (t < k1) {
-        const float pt = p_s[t - k0];
-        if (t == pos) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] += pt * v_s[dg * 8 + e];
-        } else {
-          const _Float16* hv = reinterpret_cast<const _Float16*>(&raw[u]);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) o[e] += pt * (float)hv[e];
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) acc[tg * D + dg * 8 + e] = o[e];
-  __syncthreads();
-  // two-level sum over the TG partial rows: thread (part, d) adds TG/PARTS rows, then PARTS rows
   {
-    constexpr int PARTS = kAttnThreads / D;  // 8 for D = 128 (TG = 64 rows)
-    const int d = tid % D, part = tid / D;
-    constexpr int per = TG / PARTS;
-    float sum = 0.f;
-    for (int r = 0; r < per; ++r) sum += acc[(part * per + r) * D + d];
-    __syncthreads();
-    acc[part * D + d] = sum;
-    __syncthreads();
-    if (tid < D) {
-      float tot2 = 0.f;
-      for (int r = 0; r < PARTS; ++r) tot2 += acc[r * D + tid];
-      acc[tid] = tot2;  // only read by this thread below
+    const bool fresh = tl == 0 && pos >= k0 && pos < k1;
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      q[e] = new_s[dl * 8 + e];
+      s += q[e] * new_s[kMaxHeadDim + dl * 8 + e];
     }
+    s = row_sum(s) * sm_scale;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = 0.f;
+    if (fresh) {
+      mx = s;
+      l = __expf(s - (s == -INFINITY ? 0.f : s));  // 1; 0 for -inf, NaN for NaN and inf
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = l * new_s[2 * kMaxHeadDim + dl * 8 + e];
+    }
+  }
+  for (int t0 = k0;;) {
+    float s[NU], m = mx;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const half8a kv = __builtin_bit_cast(half8a, kb[u]);
+      float d = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) d += q[e] * (float)kv[e];
+      d = row_sum(d) * sm_scale;
+      s[u] = t0 + u * U + tl < kend ? d : -INFINITY;
+      m = fmaxf(m, s[u]);
+    }
+    const float ms = m == -INFINITY ? 0.f : m;  // (nothing but scores of -inf so far: all of weight 0)
+    const float keep = __expf(mx - ms);
+    mx = m;
+    l *= keep;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] *= keep;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const half8a vv = __builtin_bit_cast(half8a, vb[u]);
+      const float pt = __expf(s[u] - ms);
+      l += pt;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] += pt * (float)vv[e];
+    }
+    t0 += NU * U;
+    if (t0 >= kend) break;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) request(kb[u], vb[u], t0 + u * U);
+  }
+
+  // ---- the lane groups of a wave, then the waves
+  {
+    float m = mx;
+#pragma unroll
+    for (int b = 5; (1 << b) >= LPK; --b) m = fmaxf(m, qtip_wht::lane_xor(m, b));
+    const float f = m == -INFINITY ? 0.f : __expf(mx - m);
+    l *= f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] *= f;
+#pragma unroll
+    for (int b = 5; (1 << b) >= LPK; --b) {
+      l += qtip_wht::lane_xor(l, b);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] += qtip_wht::lane_xor(o[e], b);
+    }
+    if (lane < LPK) {
+      *reinterpret_cast<float4a*>(acc + wave * D + dl * 8) = float4a{o[0], o[1], o[2], o[3]};
+      *reinterpret_cast<float4a*>(acc + wave * D + dl * 8 + 4) = float4a{o[4], o[5], o[6], o[7]};
+    }
+    if (lane == 0) {
+      red[wave] = m;
+      red[16 + wave] = l;
+    }
+  }
+  __syncthreads();
+  if (tid >= D) return;
+  mx = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) mx = fmaxf(mx, red[w]);
+  float sum = 0.f, tot = 0.f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    const float f = red[w] == -INFINITY ? 0.f : __expf(red[w] - mx);
+    tot += f * red[16 + w];
+    sum += f * acc[w * D + tid];
   }
   if (nsplit == 1) {
-    if (tid < D) out[(size_t)h * D + tid] = (_Float16)(acc[tid] * inv);
-  } else if (tid < D) {
+    out[(size_t)h * D + tid] = (_Float16)(sum * (1.f / tot));
+  } else {
     float* w = split_ws + ((size_t)h * nsplit + blockIdx.z) * (D + 2);
-    w[tid] = acc[tid];  // 0 for a range past the last key
+    w[tid] = sum;       // 0 for a range past the last key
     if (tid == 0) {
       w[D] = mx;        // -inf for an empty range
       w[D + 1] = tot;
@@ -498,7 +448,7 @@ static int launch_attention(void* out_f16, const void* qkv_f16, const AttnXf* xf
   if (heads < 1 || kv_heads < 1 || heads % kv_heads || head_dim < 64 || head_dim > kMaxHeadDim ||
       (head_dim & (head_dim - 1)) || max_len < 1 || max_len > 4096)
     return QTIP_E_SHAPE;
-  const size_t lds = (size_t)(3 * kMaxHeadDim + 32 + 8192 + max_len) * sizeof(float);
+  const size_t lds = (size_t)(6 * kMaxHeadDim + 32 + (xf ? 3 : 1) * 16 * head_dim) * sizeof(float);
   const dim3 grid((unsigned)(heads / kv_heads), (unsigned)kv_heads, (unsigned)key_splits);
   const int kps = (max_len + key_splits - 1) / key_splits;  // keys per range
 #define QTIP_ATTN(DD, XX, ARG)                                                                      \

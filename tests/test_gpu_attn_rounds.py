@@ -33,3 +33,30 @@ def test_rounds(heads, kv, D, splits):
         err = (got.view(heads, D).double() - ref).abs().max()
         assert float(err) <= 2**-8 * float(ref.abs().max()), (pos, float(err))
         assert torch.equal(v1[0, :, pos], qkv[(heads + kv) * D:].view(kv, D))
+
+
+@pytest.mark.parametrize("splits", [1, 4])
+@pytest.mark.parametrize("pos", [3, 130, 700])
+def test_infinite_scores_and_stale_slots(pos, splits):
+    """Keys whose score is -inf weigh nothing (the first ones a wave meets among them), an infinite value stays one, a score of
+    +inf or NaN makes its head NaN, and what stands in slots from the position on is not looked at."""
+    heads, D, slots = 4, 128, 1024
+    g = torch.Generator(device=DEV).manual_seed(pos)
+    qkv = torch.randn(3 * heads * D, generator=g, device=DEV).half()
+    qkv[:heads * D] = qkv[:heads * D].abs() + 0.5  # with no rotation every element of a query is positive
+    freq = torch.zeros(D // 2, device=DEV)
+    kc = torch.randn(1, heads, slots, D, generator=g, device=DEV).half()
+    vc = torch.randn(1, heads, slots, D, generator=g, device=DEV).half()
+    kc[:, :, pos:], vc[:, :, pos:] = float("nan"), float("nan")
+    low = torch.arange(0, pos, 2, device=DEV)  # head 0, 2: every other key at -inf, head 1: one of +inf, head 2: an infinite value
+    kc[0, 0, low, 5] = kc[0, 2, low, 5] = -float("inf")
+    kc[0, 1, pos - 1, 7] = float("inf")
+    vc[0, 2, 1, 9] = float("inf")
+    out = ops.decode_attention(qkv, kc, vc, torch.tensor([pos], device=DEV), freq, heads, heads, D, key_splits=splits).view(heads, D)
+    q = qkv[:heads * D].view(heads, 1, D).double()
+    p = torch.softmax((kc[0, :, :pos + 1].double() @ q.transpose(1, 2).contiguous())[..., 0] / D**0.5, -1)
+    ref = (p[:, None] @ vc[0, :, :pos + 1].double())[:, 0]
+    assert bool(out[1].isnan().all()) and bool(ref[1].isnan().all())
+    for h in (0, 3):
+        assert float((out[h].double() - ref[h]).abs().max()) <= 2**-9 * float(ref[h].abs().max())
+    assert float(out[2, 9]) == float(ref[2, 9]) == float("inf") and bool(out[2, :9].isfinite().all())
