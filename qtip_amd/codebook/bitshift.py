@@ -295,7 +295,7 @@ class BitshiftLinear(nn.Module):
             # both transforms and the product by one call of the library: what bounds such a call otherwise is the
             # host.  (Where takes_dense holds the product is the BLAS library's, where by_library holds a transform is: a
             # caller's table of order 300, 4800x4800, 1000 rows 435 against 2850 in the one call.)  us, launch by launch /
-            # here: 4096x4096, 2 bits, one row 40 / 13; 28672x8192, 4 bits, 16 rows 59 / 40; 4096x11008, 3 bits, 45
+            # here: 4096x4096, 2 bits, one row 40 / 15; 28672x8192, 4 bits, 16 rows 59 / 40; 4096x11008, 3 bits, 45
             # rows 65 / 29
             y = ops.linear(_contiguous(x), _contiguous(trellis), self._tlut16(dev), _contiguous(SU), _contiguous(SV),
                            had_bits(had_left, K_left, True, dev) if K_left > 1 else None, K_left,

@@ -26,9 +26,10 @@
 // Bound by a wave's instructions, so 16-row waves with 128 registers, four to a SIMD (32-row waves of
 // 256 registers read LDS half as often and took 45 instead of 41 us below).  us per launch, fp16 rows
 // under a +-1 sign vector, with the one-workgroup-set-per-row form (or, at order 172, the best of it
-// and fp32 library products) before: 28672 = 28 * 1024, 1000 rows 772 -> 41 (2.8 TB/s), 45 rows
-// 38 -> 11; 11008 = 172 * 64, 1000 rows ~150 -> 20, 45 rows 67 -> 11; 12288, 1000 rows 471 -> 18.
-// fp32 rows: 28672, 1000 rows 811 -> 82; 11008, 2048 rows ~240 -> 64.
+// and fp32 library products) before: 28672 = 28 * 1024, 1000 rows 772 -> 39 (2.9 TB/s), 45 rows
+// 38 -> 7.7; 11008 = 172 * 64, 1000 rows ~150 -> 19, 45 rows 67 -> 7.5; 12288, 1000 rows 471 -> 17.
+// fp32 rows: 28672, 1000 rows 811 -> 82; 11008, 2048 rows ~240 -> 64.  Few rows: the workgroups of a pass share its
+// output rows (launch_mix), each with all of the plane.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half8m __attribute__((ext_vector_type(8)));
