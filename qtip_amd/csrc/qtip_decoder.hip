@@ -60,6 +60,15 @@ __device__ __forceinline__ float dpp_half_mirror(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));
 }
 
+// x * c + y * s, both products and the sum rounded to fp16 as in the prompt's kernels and the module's own arithmetic.  (Left
+// to itself the compiler makes one product and the sum a single operation of one rounding, in some instances of a kernel and
+// not in others.)
+__device__ __forceinline__ _Float16 rotated(_Float16 x, _Float16 c, _Float16 y, _Float16 s) {
+#pragma clang fp contract(off)
+  const _Float16 a = x * c, b = y * s;
+  return a + b;
+}
+
 // One workgroup per query head and key range.  qkv: [H*D | Hkv*D | Hkv*D] fp16 of the new
 // token; k_cache / v_cache: [Hkv][max_len][D] fp16; pos_ptr: position of the
 // new token (device memory, so that a recorded graph follows the position).
@@ -299,7 +308,7 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
   // ---- rotary embedding in fp16 arithmetic: x*cos + rotate_half(x)*sin
   if (tid < 3 * D) {
     const _Float16 rot = c < half ? (_Float16)(-(float)pair) : pair;
-    _Float16 e = (_Float16)((float)(_Float16)((float)own * (float)rc) + (float)(_Float16)((float)rot * (float)rs));
+    _Float16 e = rotated(own, rc, rot, rs);
     if (s3 == 2) e = own;
     new_s[s3 * kMaxHeadDim + c] = (float)e;
     if (s3 && blockIdx.x == 0 && blockIdx.z == 0 && pos < max_len) (s3 == 1 ? kc : vc)[(size_t)pos * D + c] = e;

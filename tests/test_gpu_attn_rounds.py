@@ -60,3 +60,44 @@ def test_infinite_scores_and_stale_slots(pos, splits):
     for h in (0, 3):
         assert float((out[h].double() - ref[h]).abs().max()) <= 2**-9 * float(ref[h].abs().max())
     assert float(out[2, 9]) == float(ref[2, 9]) == float("inf") and bool(out[2, :9].isfinite().all())
+
+
+@pytest.mark.parametrize("form,D", [("plain", 64), ("plain", 128), ("plain", 256), ("rht", 64), ("rht", 128), ("rht3", 64),
+                                    ("rht3", 128)])
+def test_rotation_rounds_every_product(form, D):
+    """The cached key of a token is fp16(fp16(k * cos) + fp16(rotate_half(k) * sin)) bit for bit in every form of the launch."""
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    heads, kv, slots, pos = 8, 2, 64, 37
+    g = torch.Generator(device=DEV).manual_seed(D)
+    n = (heads + 2 * kv) * D
+    freq = 1.0 / (10000.0**(torch.arange(0, D, 2, device=DEV).float() / D))
+    where = torch.tensor([pos], device=DEV)
+    caches = lambda: [torch.zeros(1, kv, slots, D, device=DEV).half() for _ in range(2)]
+    probe = torch.zeros(n, device=DEV).half()
+    probe[heads * D:heads * D + D // 2] = 1  # a key of ones in front of zeros: cosines in its first half, sines in the other
+    kc, vc = caches()
+    ops.decode_attention(probe, kc, vc, where, freq, heads, kv, D)
+    c, s = (t.repeat(2) for t in kc[0, 0, pos].split(D // 2))
+    kc, vc = caches()
+    if form == "plain":
+        qkv = torch.randn(n, generator=g, device=DEV).half()
+        ops.decode_attention(qkv, kc, vc, where, freq, heads, kv, D)
+    else:  # whole numbers, whose transforms are exact in fp32 and in fp16 after the division by 8
+        parts = torch.randint(-8, 9, (2, n), generator=g, device=DEV).float()
+        sizes = [n] if form == "rht" else [heads * D, kv * D, kv * D]
+        views = parts.split(sizes, dim=1)
+        tables = [get_hadK(m) for m in sizes]
+        bits = [had_bits(h, o, False, DEV) if o > 1 else None for h, o in tables]
+        qkv = torch.cat([ops.rht(v.sum(0, keepdim=True), order=o, had_bits=b, scale=0.125, out_dtype=torch.float32)[0]
+                         for v, (_, o), b in zip(views, tables, bits)])
+        assert torch.equal(qkv, qkv.half().float())
+        qkv = qkv.half()
+        if form == "rht":
+            ops.decode_attention_rht(parts, None, 0.125, bits[0], tables[0][1], kc, vc, where, freq, heads, kv, D)
+        else:
+            ops.decode_attention_rht3(list(views), [None] * 3, [0.125] * 3, bits, [o for _, o in tables], kc, vc, where, freq,
+                                      heads, kv, D)
+    k = qkv[heads * D:(heads + kv) * D].view(kv, D)
+    turned = torch.cat((-k[:, D // 2:], k[:, :D // 2]), 1)
+    assert torch.equal(kc[0, :, pos], k * c + turned * s)
+    assert torch.equal(vc[0, :, pos], qkv[(heads + kv) * D:].view(kv, D))
