@@ -9,6 +9,7 @@ import ctypes
 import math
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._lib import QTIP_F16, QTIP_F32, check, host, lib, require_cuda, stream_ptr
@@ -77,16 +78,18 @@ _is_compiling, _modes = torch.compiler.is_compiling, torch._C._len_torch_dispatc
 
 def launchable(*tensors):
     """The tensors are memory that a launch can be given: nothing traces the program, and none of them is a wrapper
-    (batched gradients, fake tensors).  What passes by torch's own or registered operations asks this first."""
+    (batched gradients, fake tensors) or carries a tangent.  What passes by torch's own or registered operations asks this
+    first."""
     if _is_compiling() or _modes():
         return False
     try:
         for t in tensors:
             if not t.data_ptr() and t.numel():
                 return False
+        # (forward-mode derivatives: such a tensor has ordinary memory and no requires_grad)
+        return forward_ad._current_level < 0 or all(forward_ad.unpack_dual(t).tangent is None for t in tensors)
     except RuntimeError:
         return False
-    return True
 
 
 def _check_packed(packed, m, k, bits):

@@ -390,3 +390,23 @@ def test_rotary_tables(n, half):
     emb = torch.cat([pos.float()[:, None] * inv[None]] * 2, dim=-1)
     cos, sin = ops.rotary_tables(pos, inv)
     assert torch.equal(cos, emb.cos().half()) and torch.equal(sin, emb.sin().half())
+
+
+def test_norm_carries_tangents():
+    """Forward-mode derivatives of the norm, of its input and of its weight, against reverse mode."""
+    from torch.autograd import forward_ad
+    from qtip_amd.llama_decode import RMSNorm
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, t = (torch.randn(4, 512, generator=g, device="cuda").half() for _ in range(2))
+    mod = RMSNorm(512, 1e-5).cuda()
+    w = (1 + 0.1 * torch.randn(512, generator=g, device="cuda")).half()
+    for dual in ("input", "weight"):
+        f = lambda v: torch.func.functional_call(mod, {"weight": w}, v) if dual == "input" else \
+            torch.func.functional_call(mod, {"weight": v}, x)
+        at, along = (x, t) if dual == "input" else (w, t[0])
+        with forward_ad.dual_level():
+            y, tangent = forward_ad.unpack_dual(f(forward_ad.make_dual(at, along)))
+        want = torch.autograd.functional.jvp(f, at, along)  # by reverse mode, twice
+        assert torch.equal(y, want[0]) and tangent is not None
+        # fp16 products and roundings on the way, in another order
+        assert float((tangent.float() - want[1].float()).norm()) <= 2.0**-8 * float(want[1].float().norm())

@@ -393,3 +393,17 @@ def test_native_host_module_leaves_host_tensors_to_the_checks():
     packed, tlut = torch.zeros(256 * 256 // 8, dtype=torch.int16), torch.zeros(512, 2, dtype=torch.float16)
     assert _lib.host().matvec(packed, x, tlut, 256, 256, 2, 0, 0, 0) is None
     assert _lib.host().linear(x, packed, tlut, x[0], x[0].float(), None, 1, None, 1, 256, 256, 2, 1.0, 1.0, False, 96, 0) is None
+
+
+def test_a_tensor_with_a_tangent_is_not_launchable():
+    from torch.autograd import forward_ad
+    from qtip_amd import ops
+    x = torch.randn(3, 8)
+    assert ops.launchable(x)
+    with forward_ad.dual_level():
+        d = forward_ad.make_dual(x, torch.ones_like(x))
+        assert not d.requires_grad and not ops.launchable(d) and not ops.launchable(x, d) and ops.launchable(x)
+    assert ops.launchable(x)
+    seen = []
+    torch.func.jvp(lambda v: seen.append(ops.launchable(v)) or v, (x,), (x,))
+    assert seen == [False]
