@@ -73,14 +73,14 @@ def aligned16(t):
     return t if t is None or t.data_ptr() % 16 == 0 else t.clone()
 
 
-_is_compiling, _modes = torch.compiler.is_compiling, torch._C._len_torch_dispatch_stack
+_is_compiling, _is_tracing, _modes = torch.compiler.is_compiling, torch.jit.is_tracing, torch._C._len_torch_dispatch_stack
 
 
 def launchable(*tensors):
     """The tensors are memory that a launch can be given: nothing traces the program, and none of them is a wrapper
     (batched gradients, fake tensors) or carries a tangent.  What passes by torch's own or registered operations asks this
     first."""
-    if _is_compiling() or _modes():
+    if _is_compiling() or _modes() or _is_tracing():
         return False
     try:
         for t in tensors:

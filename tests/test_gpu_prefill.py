@@ -410,3 +410,16 @@ def test_norm_carries_tangents():
         assert torch.equal(y, want[0]) and tangent is not None
         # fp16 products and roundings on the way, in another order
         assert float((tangent.float() - want[1].float()).norm()) <= 2.0**-8 * float(want[1].float().norm())
+
+
+def test_traced_norm_and_rotary_tables_follow_their_input():
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder, RMSNorm
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x, other = (torch.randn(4, 512, generator=g, device="cuda").half() for _ in range(2))
+    mod = RMSNorm(512, 1e-5).cuda()
+    # (a product of two values and a sum of 512 of them in another order: a value on the edge rounds the other way)
+    assert float((torch.jit.trace(mod, x)(other).float() - mod(other).float()).abs().max()) <= 2.0**-9 * float(mod(other).abs().max())
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=1, ffn=512, vocab=64, K=2), 64, device="cuda")
+    pos = torch.arange(9, device="cuda")
+    traced = torch.jit.trace(lambda p: model.rope(p), (pos,))
+    assert all(torch.equal(a, b) for a, b in zip(traced(pos + 30), model.rope(pos + 30)))

@@ -407,3 +407,11 @@ def test_a_tensor_with_a_tangent_is_not_launchable():
     seen = []
     torch.func.jvp(lambda v: seen.append(ops.launchable(v)) or v, (x,), (x,))
     assert seen == [False]
+
+
+def test_nothing_is_launchable_while_a_trace_records():
+    """(A recorded program would hold the output's allocation and not the launch that fills it.)"""
+    from qtip_amd import ops
+    x, seen = torch.randn(3, 8), []
+    torch.jit.trace(lambda v: seen.append(ops.launchable(v)) or v + 1, (x,), check_trace=False)
+    assert seen == [False] and ops.launchable(x)
