@@ -97,8 +97,9 @@ class RMSNorm(nn.Module):
 
     def forward(self, x):
         w = self.weight
-        if (x.is_cuda and x.dtype == w.dtype == torch.float16 and x.device == w.device and x.shape[-1:] == w.shape
-                and w.shape[0] <= 16384 and x.is_contiguous() and w.is_contiguous() and ops.launchable(x, w)
+        # (a symbolic trace hands in what is no tensor, and records the formula)
+        if (isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == w.dtype == torch.float16 and x.device == w.device
+                and x.shape[-1:] == w.shape and w.shape[0] <= 16384 and x.is_contiguous() and w.is_contiguous() and ops.launchable(x, w)
                 and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
             return ops.rmsnorm_rows(x, w, self.eps)
         h = x.float()
@@ -662,8 +663,8 @@ class LlamaDecoder(nn.Module):
 
     def rope(self, positions):
         f = self.inv_freq
-        if (positions.is_cuda and positions.dtype == torch.int64 and positions.dim() == 1 and f.dtype == torch.float32
-                and positions.device == f.device and positions.is_contiguous() and f.is_contiguous()
+        if (isinstance(positions, torch.Tensor) and positions.is_cuda and positions.dtype == torch.int64
+                and positions.dim() == 1 and f.dtype == torch.float32 and positions.device == f.device and positions.is_contiguous() and f.is_contiguous()
                 and ops.launchable(positions, f)):
             return tuple(t[None, None] for t in ops.rotary_tables(positions, f))
         freqs = positions.float()[:, None] * self.inv_freq[None, :]

@@ -415,3 +415,19 @@ def test_nothing_is_launchable_while_a_trace_records():
     x, seen = torch.randn(3, 8), []
     torch.jit.trace(lambda v: seen.append(ops.launchable(v)) or v + 1, (x,), check_trace=False)
     assert seen == [False] and ops.launchable(x)
+
+
+def test_symbolic_traces_of_the_norm_and_the_rotary_tables():
+    import torch.fx
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder, RMSNorm
+
+    class Rope(torch.nn.Module):
+
+        def forward(self, p):
+            return model.rope(p)
+
+    x, mod = torch.randn(3, 8).half(), RMSNorm(8, 1e-5)
+    assert torch.equal(torch.fx.symbolic_trace(mod)(x), mod(x))
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=0, ffn=512, vocab=64, K=2), 64, device="cpu")
+    pos = torch.arange(9)
+    assert all(torch.equal(a, b) for a, b in zip(torch.fx.symbolic_trace(Rope())(pos), model.rope(pos)))
