@@ -95,13 +95,17 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(n, dtype=torch.float16), requires_grad=False)
         self.eps = eps
 
-    def forward(self, x):
+    def _launches(self, x):
         w = self.weight
         # (a symbolic trace hands in what is no tensor, and records the formula)
-        if (isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == w.dtype == torch.float16 and x.device == w.device
-                and x.shape[-1:] == w.shape and w.shape[0] <= 16384 and x.is_contiguous() and w.is_contiguous() and ops.launchable(x, w)
-                and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
-            return ops.rmsnorm_rows(x, w, self.eps)
+        return (isinstance(x, torch.Tensor) and x.is_cuda and x.dtype == w.dtype == torch.float16 and x.device == w.device
+                and x.shape[-1:] == w.shape and w.shape[0] <= 16384 and x.is_contiguous() and w.is_contiguous()
+                and ops.launchable(x, w) and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)))
+
+    def forward(self, x):
+        if not torch.jit.is_scripting():  # (a scripted module holds the formula)
+            if self._launches(x):
+                return ops.rmsnorm_rows(x, self.weight, self.eps)
         h = x.float()
         h = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + self.eps)
         return self.weight * h.to(x.dtype)
@@ -664,8 +668,8 @@ class LlamaDecoder(nn.Module):
     def rope(self, positions):
         f = self.inv_freq
         if (isinstance(positions, torch.Tensor) and positions.is_cuda and positions.dtype == torch.int64
-                and positions.dim() == 1 and f.dtype == torch.float32 and positions.device == f.device and positions.is_contiguous() and f.is_contiguous()
-                and ops.launchable(positions, f)):
+                and positions.dim() == 1 and f.dtype == torch.float32 and positions.device == f.device
+                and positions.is_contiguous() and f.is_contiguous() and ops.launchable(positions, f)):
             return tuple(t[None, None] for t in ops.rotary_tables(positions, f))
         freqs = positions.float()[:, None] * self.inv_freq[None, :]
         emb = torch.cat((freqs, freqs), dim=-1)

@@ -431,3 +431,9 @@ def test_symbolic_traces_of_the_norm_and_the_rotary_tables():
     model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=0, ffn=512, vocab=64, K=2), 64, device="cpu")
     pos = torch.arange(9)
     assert all(torch.equal(a, b) for a, b in zip(torch.fx.symbolic_trace(Rope())(pos), model.rope(pos)))
+
+
+def test_scripted_norm():
+    from qtip_amd.llama_decode import RMSNorm
+    x, mod = torch.randn(3, 8).half(), RMSNorm(8, 1e-5)
+    assert torch.equal(torch.jit.script(mod)(x), mod(x))
