@@ -437,3 +437,11 @@ def test_scripted_norm():
     from qtip_amd.llama_decode import RMSNorm
     x, mod = torch.randn(3, 8).half(), RMSNorm(8, 1e-5)
     assert torch.equal(torch.jit.script(mod)(x), mod(x))
+
+
+@pytest.mark.parametrize("fused", [True, False])
+def test_a_layer_holds_its_projections_and_norms(fused):
+    """(A model saved whole by an earlier version has no more than these.)"""
+    from qtip_amd.llama_decode import DecoderLayer, LlamaConfig
+    layer = DecoderLayer(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=1, ffn=512, vocab=64, K=2), None, "cpu", fused=fused)
+    assert not dict(layer.named_buffers(recurse=False)) and not dict(layer.named_parameters(recurse=False))
