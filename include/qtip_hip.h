@@ -243,7 +243,7 @@ int qtip_scale_columns_grad(float* gx, float* gs, const float* g, const float* x
 
 /* Rotary tables of a prompt (model/llama.py:215-262): cos and sin, [n][2 half] fp16, of the fp32 products
  * float(positions[i]) * inv_freq[d], d < half, each twice. */
-int qtip_rotary_tables(void* cos_f16, void* sin_f16, const void* positions_i64, const float* inv_freq, int n, int half,
+int qtip_rotary_tables(void* cos_f16, void* sin_f16, const void* positions_i64, const float* inv_freq, long n, int half,
                        void* stream);
 
 /* Attention of n new tokens (a prompt, or a piece of one): rotary embedding of q and k (fp16 arithmetic; cos and sin
@@ -385,7 +385,7 @@ int qtip_decode_attention_rht3(void* out_f16, const float* const* parts, int in_
  * (model/llama.py:129-135), n <= 16384, one launch instead of the module's six. */
 int qtip_rmsnorm(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int n, void* stream);
 /* The same for each of `rows` rows of n values, one after the other in memory. */
-int qtip_rmsnorm_rows(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int rows, int n, void* stream);
+int qtip_rmsnorm_rows(void* out_f16, const void* x_f16, const void* weight_f16, float eps, long rows, int n, void* stream);
 
 /* Greedy token pick of the generation loop (eval/interactive_gen.py:43-69: argmax of the last
  * position's logits, copy into the next step's input, position + 1), all in device memory so a

@@ -674,7 +674,7 @@ __global__ __launch_bounds__(kHeadThreads) void greedy_pick_kernel(const _Float1
 
 }  // namespace
 
-extern "C" int qtip_rmsnorm_rows(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int rows, int n,
+extern "C" int qtip_rmsnorm_rows(void* out_f16, const void* x_f16, const void* weight_f16, float eps, long rows, int n,
                                  void* stream) {
   if (!out_f16 || !x_f16 || !weight_f16) return QTIP_E_NULL;
   if (n < 1 || n > 16 * kHeadThreads || rows < 1) return QTIP_E_SHAPE;
@@ -683,9 +683,12 @@ extern "C" int qtip_rmsnorm_rows(void* out_f16, const void* x_f16, const void* w
   auto* kernel = wide ? rmsnorm_kernel<8> : rmsnorm_kernel<1>;
   const int loads = wide ? n >> 3 : n;
   const int threads = loads < kHeadThreads ? (loads + 63) & ~63 : kHeadThreads;
-  kernel<<<rows, threads, 0, (hipStream_t)stream>>>((_Float16*)out_f16, (const _Float16*)x_f16,
-                                                    (const _Float16*)weight_f16, eps, n);
-  return (int)hipGetLastError();
+  for (long r = 0; r < rows; r += 1 << 20) {  // (a launch holds fewer than 2^32 threads)
+    kernel<<<(unsigned)(rows - r < 1 << 20 ? rows - r : 1 << 20), threads, 0, (hipStream_t)stream>>>(
+        (_Float16*)out_f16 + r * n, (const _Float16*)x_f16 + r * n, (const _Float16*)weight_f16, eps, n);
+    if (const hipError_t e = hipGetLastError()) return (int)e;
+  }
+  return 0;
 }
 
 extern "C" int qtip_rmsnorm(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int n, void* stream) {

@@ -262,13 +262,19 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
 
 }  // namespace
 
-extern "C" int qtip_rotary_tables(void* cos_f16, void* sin_f16, const void* positions_i64, const float* inv_freq, int n,
+extern "C" int qtip_rotary_tables(void* cos_f16, void* sin_f16, const void* positions_i64, const float* inv_freq, long n,
                                   int half, void* stream) {
   if (!cos_f16 || !sin_f16 || !positions_i64 || !inv_freq) return QTIP_E_NULL;
-  if (n < 1 || half < 1 || (long)n * half > (1L << 38)) return QTIP_E_SHAPE;
-  rotary_tables_kernel<<<(unsigned)(((long)n * half + kBlock - 1) / kBlock), kBlock, 0, (hipStream_t)stream>>>(
-      (_Float16*)cos_f16, (_Float16*)sin_f16, (const int64_t*)positions_i64, inv_freq, n, half);
-  return (int)hipGetLastError();
+  if (n < 1 || half < 1 || half > 1 << 20) return QTIP_E_SHAPE;
+  const long step = (1 << 30) / half;  // (a launch holds fewer than 2^32 threads)
+  for (long i = 0; i < n; i += step) {
+    const long m = n - i < step ? n - i : step;
+    rotary_tables_kernel<<<(unsigned)((m * half + kBlock - 1) / kBlock), kBlock, 0, (hipStream_t)stream>>>(
+        (_Float16*)cos_f16 + i * 2 * half, (_Float16*)sin_f16 + i * 2 * half, (const int64_t*)positions_i64 + i, inv_freq,
+        (int)m, half);
+    if (const hipError_t e = hipGetLastError()) return (int)e;
+  }
+  return 0;
 }
 
 extern "C" int qtip_prefill_attention(void* out_f16, const void* q_f16, const void* k_f16, const void* v_f16,

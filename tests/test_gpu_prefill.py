@@ -423,3 +423,18 @@ def test_traced_norm_and_rotary_tables_follow_their_input():
     pos = torch.arange(9, device="cuda")
     traced = torch.jit.trace(lambda p: model.rope(p), (pos,))
     assert all(torch.equal(a, b) for a, b in zip(traced(pos + 30), model.rope(pos + 30)))
+
+
+def test_more_rows_and_positions_than_a_launch_has_threads():
+    """2^26 + 3 rows of 8 values (a wave each), and 2^26 + 3 positions of 64 angles: past 2^32 threads, the first and the last ones."""
+    from qtip_amd import ops
+    rows = 2**26 + 3
+    pick = torch.tensor([0, 1, 2**20 - 1, 2**20, 2**26 - 1, 2**26, rows - 1], device="cuda")
+    w = (1 + 0.1 * torch.randn(8, device="cuda")).half()
+    x = torch.randn(rows, 8, device="cuda", dtype=torch.float16)
+    assert torch.equal(ops.rmsnorm_rows(x, w, 1e-5)[pick], ops.rmsnorm_rows(x[pick], w, 1e-5))
+    del x
+    inv = 10000.0 ** (-torch.arange(64, device="cuda", dtype=torch.float32) / 64)
+    pos = torch.randint(0, 4096, (rows,), device="cuda")
+    for big, few in zip(ops.rotary_tables(pos, inv), ops.rotary_tables(pos[pick], inv)):
+        assert torch.equal(big[pick], few)
