@@ -6,6 +6,7 @@ a launcher reports an error, the call raises.
 import ctypes
 import importlib.util
 import os
+import warnings
 
 import torch  # must be imported first so that its bundled HIP runtime is the one libqtip_hip.so binds to
 
@@ -140,19 +141,27 @@ def lib():
 
 
 def host():
-    """The native host module (csrc/qtip_host.cpp), bound to the loaded library."""
+    """The native host module (csrc/qtip_host.cpp), bound to the loaded library; False where there is none that loads.  It
+    shortens the way to the library's launches, which every one of its callers knows by itself: the results are the same."""
     global _host
     if _host is None:
-        if not os.path.exists(HOST_PATH):
-            raise QtipLibraryError(f"{HOST_PATH} not found: build it with `python -m qtip_amd.build`")
+        _host = _load_host()
+    return _host
+
+
+def _load_host():
+    try:
         spec = importlib.util.spec_from_file_location("_qtip_host", HOST_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
-        module.bind(*(ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
-                      for name in ("qtip_linear", "qtip_linear_long", "qtip_linear_workspace_bytes",
-                                   "qtip_linear_long_workspace_bytes", "qtip_decompress_matvec", "qtip_linear_rows")))
-        _host = module
-    return _host
+    except (ImportError, OSError) as e:
+        warnings.warn(f"{HOST_PATH} does not load, calls of a few rows take longer on the host: build it with "
+                      f"`python -m qtip_amd.build` ({e})", RuntimeWarning, stacklevel=3)
+        return False
+    module.bind(*(ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
+                  for name in ("qtip_linear", "qtip_linear_long", "qtip_linear_workspace_bytes",
+                               "qtip_linear_long_workspace_bytes", "qtip_decompress_matvec", "qtip_linear_rows")))
+    return module
 
 
 _INITIALISED = set()

@@ -151,13 +151,16 @@ def matvec_row(packed, x, tlut, m, k, bits):
     """decompress_matvec of operands that fit as they are, as a (1, m) tensor, in one native function; None for any other."""
     if not (isinstance(packed, _Tensor) and packed.is_cuda) or _is_compiling() or bits not in _BITS or (m | k) & 31:
         return None
+    native = host()
+    if not native:
+        return None
     dev = packed.device
     stream = stream_ptr(dev)
     wsp, wsb = 0, 0
     if matvec_split(m, k, bits, dev) > 1:
         ws = _workspace(dev, 16 * m * 4, stream)
         wsp, wsb = ws.data_ptr(), ws.numel()
-    y = host().matvec(packed, x, tlut, m, k, bits, wsp, wsb, stream)
+    y = native.matvec(packed, x, tlut, m, k, bits, wsp, wsb, stream)
     return y if y is None or isinstance(y, _Tensor) else check(y, "qtip_decompress_matvec")
 
 
@@ -369,8 +372,8 @@ def linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, 
     for bit, of rht, decompress_matvec_parts[_rht] (one row) or decompress_gemm (more), rht.  had_in / had_out: sign
     bits of the table orders (None for order 1).  long_sums: the product is decompress_gemm's with long sums."""
     # a call whose operands fit is one native function's; any other goes through the checks one by one
-    if isinstance(x, _Tensor) and x.is_cuda and not _is_compiling():
-        y = host().linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out,
+    if isinstance(x, _Tensor) and x.is_cuda and not _is_compiling() and (native := host()):
+        y = native.linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out,
                           long_sums, _ALIGN_ROWS, stream_ptr(x.device))
         if y is not None:
             return y if isinstance(y, _Tensor) else check(y, "qtip_linear")
@@ -409,10 +412,10 @@ PRE_NONE, PRE_RMSNORM, PRE_SILU_MUL = 0, 1, 2
 def linear_rows(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out, long_sums,
                 pre_mode, norm_weight, eps, residual):
     """linear() for fp16 rows, two or more, with the element-wise work around the projection in the transforms (as rht takes
-    it); None where an operand is not as the launches need it (contiguous, on 16 bytes)."""
-    if not (isinstance(x, _Tensor) and x.is_cuda) or _is_compiling():
+    it); None where an operand is not as the launches need it (contiguous, on 16 bytes), or without the native module."""
+    if not (isinstance(x, _Tensor) and x.is_cuda) or _is_compiling() or not (native := host()):
         return None
-    y = host().linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out, long_sums, 0,
+    y = native.linear(x, packed, tlut, su, sv, had_in, order_in, had_out, order_out, m, k, bits, scale_in, scale_out, long_sums, 0,
                       stream_ptr(x.device), pre_mode, norm_weight, eps, residual)
     return y if y is None or isinstance(y, _Tensor) else check(y, "qtip_linear_rows")
 

@@ -175,3 +175,31 @@ def test_native_call_takes_what_fits_and_leaves_the_rest():
         assert _lib.host().matvec(*args, m, k, bits, 0, 0, st) is None
     with pytest.raises(TypeError):
         _lib.host().matvec(packed, row, tlut)
+
+
+def test_without_the_native_module(monkeypatch):
+    """Every caller of the native functions has its own way to the same launches: the same bits."""
+    from qtip_amd import _lib, ops
+    from qtip_amd.codebook import register_shape
+    from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder
+    m, k, bits = 96, 256, 3
+    g = torch.Generator(device="cuda").manual_seed(4)
+    packed = torch.randint(-32768, 32768, (m // 16 * k // 16, 16 * bits), dtype=torch.int16, generator=g, device="cuda")
+    tlut = torch.randn(512, 2, generator=g, device="cuda").half()
+    su, sv = torch.ones(k, device="cuda").half(), torch.ones(m, device="cuda")
+    xs = [torch.randn(rows, k, generator=g, device="cuda").half() for rows in (1, 5, 40)]
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    order = get_hadK(m)[1]
+    table = had_bits(get_hadK(m)[0], order, False, "cuda")
+    model = LlamaDecoder(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=1, ffn=512, vocab=64, K=2), 64, device="cuda")
+    ids, pos = torch.arange(20, device="cuda")[None], torch.arange(20, device="cuda")
+
+    def outputs():
+        with torch.no_grad():
+            return [ops.linear(x, packed.reshape(-1), tlut, su, sv, None, 1, table, order, m, k, bits, 0.5, 2.0) for x in xs] + [
+                register_shape(m, k, bits)(packed, xs[0], tlut), model(ids, pos)]
+
+    native = outputs()
+    assert _lib.host()
+    monkeypatch.setattr(_lib, "_host", False)
+    assert all(torch.equal(a, b) for a, b in zip(native, outputs()))

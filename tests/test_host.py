@@ -445,3 +445,17 @@ def test_a_layer_holds_its_projections_and_norms(fused):
     from qtip_amd.llama_decode import DecoderLayer, LlamaConfig
     layer = DecoderLayer(LlamaConfig(hidden=256, heads=4, kv_heads=2, layers=1, ffn=512, vocab=64, K=2), None, "cpu", fused=fused)
     assert not dict(layer.named_buffers(recurse=False)) and not dict(layer.named_parameters(recurse=False))
+
+
+@pytest.mark.parametrize("there", [False, True])
+def test_library_without_a_host_module_that_loads(there, tmp_path, monkeypatch):
+    """The native host module shortens calls; a tree that holds the library alone has all of them."""
+    from qtip_amd import _lib
+    path = tmp_path / "_qtip_host.so"
+    if there:
+        path.write_bytes(b"for another interpreter")
+    monkeypatch.setattr(_lib, "HOST_PATH", str(path))
+    monkeypatch.setattr(_lib, "_host", None)
+    with pytest.warns(RuntimeWarning, match="qtip_amd.build"):
+        assert not _lib.host()
+    assert not _lib.host()  # (asked once)
