@@ -32,6 +32,8 @@
 extern "C" {
 #endif
 
+#define QTIP_ABI_VERSION 26 /* of this header; a library tells its own by qtip_abi_version() */
+
 #define QTIP_OK 0
 #define QTIP_E_SHAPE (-1)     /* m % 32, k % 32, bits, batch or n out of range */
 #define QTIP_E_NULL (-2)      /* a required pointer is NULL */

@@ -154,6 +154,13 @@ def _load_host():
         spec = importlib.util.spec_from_file_location("_qtip_host", HOST_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        # a module of another version calls the library with other arguments, one built for another torch reads other tensors
+        got = getattr(module, "abi_version", None)
+        if got != ABI_VERSION:
+            raise QtipLibraryError(f"{HOST_PATH}: ABI {got}, Python side expects {ABI_VERSION}: rebuild with "
+                                   "`python -m qtip_amd.build`")
+        if module.torch_version != torch.__version__:
+            raise ImportError(f"built for torch {module.torch_version}, this is {torch.__version__}")
     except (ImportError, OSError) as e:
         warnings.warn(f"{HOST_PATH} does not load, calls of a few rows take longer on the host: build it with "
                       f"`python -m qtip_amd.build` ({e})", RuntimeWarning, stacklevel=3)

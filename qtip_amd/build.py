@@ -51,7 +51,7 @@ def build_host(verbose=True):
     from torch.utils.cpp_extension import include_paths
     dirs = include_paths() + [sysconfig.get_paths()["include"]]
     _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
-          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] + [a for d in dirs for a in ("-isystem", d)] +
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DQTIP_TORCH_VERSION="{torch.__version__}"'] + [a for d in dirs for a in ("-isystem", d)] +
          [HOST_SRC, "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10",
           "-o", HOST_OUT + ".tmp"], verbose)
     os.replace(HOST_OUT + ".tmp", HOST_OUT)

@@ -911,7 +911,7 @@ int qtip_device_ready(void* stream, int* cus) {
 
 extern "C" {
 
-int qtip_abi_version(void) { return 26; }
+int qtip_abi_version(void) { return QTIP_ABI_VERSION; }
 
 int qtip_init(void) { return ready(false, nullptr).rc; }
 

@@ -189,4 +189,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_qtip_host", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__qtip_host() { return PyModule_Create(&module); }
+// (abi_version, torch_version: of the header and of the torch that this was compiled against, for the loader to compare)
+PyMODINIT_FUNC PyInit__qtip_host() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && (PyModule_AddIntConstant(m, "abi_version", QTIP_ABI_VERSION) ||
+            PyModule_AddStringConstant(m, "torch_version", QTIP_TORCH_VERSION))) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

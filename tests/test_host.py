@@ -459,3 +459,27 @@ def test_library_without_a_host_module_that_loads(there, tmp_path, monkeypatch):
     with pytest.warns(RuntimeWarning, match="qtip_amd.build"):
         assert not _lib.host()
     assert not _lib.host()  # (asked once)
+
+
+def test_host_module_of_another_version(tmp_path, monkeypatch):
+    """A module for another version of the library is refused; one for another torch is left alone."""
+    from qtip_amd import _lib
+    for abi, version in ((None, None), (_lib.ABI_VERSION - 1, torch.__version__), (_lib.ABI_VERSION, "1.0")):
+        path = tmp_path / f"host_{abi}_{version}.py"
+        text = "def bind(*a): raise AssertionError('bound')\n"
+        path.write_text(text if abi is None else text + f"abi_version = {abi}\ntorch_version = {str(version)!r}\n")
+        monkeypatch.setattr(_lib, "HOST_PATH", str(path))
+        monkeypatch.setattr(_lib, "_host", None)
+        if abi == _lib.ABI_VERSION:
+            with pytest.warns(RuntimeWarning, match="torch 1.0"):
+                assert not _lib.host()
+        else:
+            with pytest.raises(_lib.QtipLibraryError, match="rebuild"):
+                _lib.host()
+
+
+def test_header_and_host_module_are_of_one_version():
+    from qtip_amd import _lib
+    text = open(os.path.join(ROOT, "include", "qtip_hip.h")).read()
+    assert int(re.search(r"#define QTIP_ABI_VERSION (\d+)", text)[1]) == _lib.ABI_VERSION == _lib.host().abi_version
+    assert _lib.host().torch_version == torch.__version__
