@@ -813,15 +813,20 @@ bool rows_form_size(int n, int order, int rows) {
 //         order >= 100:  1248, 16 rows 9.5/11.2, 20 11.3/11.2; 4992, 10 rows 10.5/10.8, 12 11.6/10.8; 11008, 5 rows 10.6/11.7,
 //         6 12.6/11.6; 22016, 2 rows 8.8/11.9, 3 12.4/11.9
 // With an element-wise prologue or a residual the matrix form is the one that covers every size, from 12 rows on at the
-// latest (8 at orders from 100 on).  Prologue SiLU: 5120, 6 rows 4.8/6.1, 7 7.3/6.0; 11008, 2 rows 8.7/8.8, 3 12.2/8.9;
-// 14336, 4 rows 5.8/7.3, 5 9.2/7.3; 28672, 4 rows 7.7/9.4, 5 13.1/9.4.
-int mix_rows_min(int order, int n, long wgs, bool f16, bool fused, int slices) {
+// latest (8 at orders from 100 on).  Prologue SiLU: 5120, 6 rows 4.6/5.8, 7 7.1/5.8; 11008, 2 rows 8.7/8.4, 3 11.8/8.6;
+// 14336, 4 rows 5.6/7.0, 5 8.9/6.9; 28672, 4 rows 7.4/9.0, 5 12.6/9.0; two slices: 57344, 4 rows 12.1/18.6, 5 22.5/18.5.  RMSNorm:
+// 5120, 6 rows 4.7/6.9, 7 7.3/6.9; 11008, 2 rows 8.4/9.7, 3 11.5/9.9; 14336, 4 rows 5.5/8.1, 5 8.8/8.1.  A residual alone, fp16
+// rows: 5120, 6 rows 4.0/5.9, 7 5.9/5.9; 11008, 2 rows 6.0/7.2, 3 7.9/7.4; 14336, 4 rows 4.3/6.5, 5 6.5/6.5; 28672, 4 rows 5.0/7.1,
+// 5 8.0/7.1; two slices, which take three planes: 57344, 9 rows 13.7/14.8, 10 19.4/15.1.  A residual and fp32 rows, three planes
+// as well: 5120, 11 rows 6.0/8.3; 11008, 5 rows 11.1/12.1, 8 16.1/12.1; 28672, 11 rows 11.2/13.3, 57344, 10 rows 18.5/13.9.
+int mix_rows_min(int order, int n, long wgs, bool f16, bool pre, bool residual,
+                 int slices) {
   const bool large = order >= 100;
   auto above = [&](int count) { return (int)(count / wgs) + 1; };  // the first row count of more than `count` workgroups
-  if (fused) {
+  if (pre || residual) {
     const int most = large ? 8 : 12;
-    if (n <= 4096) return most;
-    const int line = above(large ? 360 : 256);
+    if (n <= 4096 || (!f16 && slices == 1)) return most;
+    const int line = above(large ? 360 : (slices > 1 && !pre ? 510 : 256));
     return line < most ? line : most;
   }
   if (slices > 1) return above(510);
@@ -890,7 +895,8 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
                     ((P.pre_row_stride * 2) & 15u) == 0 && ((P.post_row_stride * 4) & 15u) == 0 &&
                     !(P.pre_mode != PRE_NONE && in_dtype != QTIP_F16) && !(fused && out_dtype != QTIP_F16) &&
                     mix_shape(n, order, rows, M, kt) &&
-                    rows >= mix_rows_min(order, n, OT, in_dtype == QTIP_F16, fused, 1 << M.logS);
+                    rows >= mix_rows_min(order, n, OT, in_dtype == QTIP_F16, P.pre_mode != PRE_NONE, P.residual != nullptr,
+                                         1 << M.logS);
     if (ok) {
       int cus = 0;
       const int rc = qtip_device_ready(stream, &cus);
@@ -1069,7 +1075,7 @@ bool qtip_rht_takes_parts(int n, int order, int rows, int nparts, bool residual)
   MixShape M{};
   int kt = 0;
   return mix_shape(n, order, rows, M, kt) && nparts << 5 <= 1 << M.logpp &&
-         rows >= mix_rows_min(order, n, OT, true, residual, 1 << M.logS);
+         rows >= mix_rows_min(order, n, OT, true, false, residual, 1 << M.logS);
 }
 
 int qtip_rht_from_parts(void* out, int out_dtype, const float* parts, int nparts, int rows, int n, int order,

@@ -257,3 +257,22 @@ def test_any_order_of_signs(K, p, rows):
             y = ops.rht(x, order=K, had_bits=bits, out_dtype=torch.float32)
             # exact products, fp32 sums of n terms
             assert float((y.double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("n,line16,line32", [(5120, 7, 12), (11008, 3, 8), (28672, 5, 12), (57344, 10, 10)])
+def test_rows_with_a_residual_either_side_of_the_line(n, line16, line32):
+    """A residual behind few rows: below the line between the forms every row has the bits of a launch of its own, on it the
+    matrix form rounds some of them to the neighbouring fp16 value."""
+    from qtip_amd import ops
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    had, K = get_hadK(n)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    kw = dict(order=K, had_bits=had_bits(had, K, False, "cuda"), post=rnd(n), out_dtype=torch.float16)
+    for dtype, line in ((torch.float16, line16), (torch.float32, line32)):
+        x, res = rnd(line, n).to(dtype), rnd(line, n).half()
+        one = torch.cat([ops.rht(x[i:i + 1], residual=res[i:i + 1], **kw) for i in range(line)])
+        assert torch.equal(ops.rht(x[:-1], residual=res[:-1], **kw), one[:-1])
+        got = ops.rht(x, residual=res, **kw)
+        # (exact values within half an fp16 step and the fp32 sums' error of each other; twice for a rounding of two sums)
+        assert not torch.equal(got, one) and float((got.float() - one.float()).abs().max()) <= 2.0**-9 * float(one.abs().max())
