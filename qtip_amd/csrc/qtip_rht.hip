@@ -809,36 +809,40 @@ bool rows_form_size(int n, int order, int rows) {
 //         order >= 100:  1248 = 156 * 8, 6 rows 5.9/6.2, 7 7.2/6.2; 1728, 8 rows 5.0/5.6, 10 6.4/5.5; 4992, 4 rows 6.2/6.5, 5
 //         7.1/6.5; 11008 = 172 * 64, 2 rows 6.1/7.1, 3 8.1/7.2, 8 14.8/7.3; 22016, 2 rows 8.8/7.4, 8 23.7/7.5
 //   fp32  order < 100:   64, 1000 rows 5.4/6.3, 1600 7.8/6.3; 1024, 64 rows 5.4/6.3, 96 7.1/6.4; 5120, 24 rows 7.3/7.7, 28
-//         8.5/7.7; 14336, 10 rows 8.9/9.4, 14 11.6/9.5; 28672, 8 rows 9.9/12.9, 10 13.3/12.9; 57344, 8 rows 14.8/14.8
-//         order >= 100:  1248, 16 rows 9.5/11.2, 20 11.3/11.2; 4992, 10 rows 10.5/10.8, 12 11.6/10.8; 11008, 5 rows 10.6/11.7,
-//         6 12.6/11.6; 22016, 2 rows 8.8/11.9, 3 12.4/11.9
+//         8.5/7.7; with a vector on the way out (on the way in): 10240, 18 rows 8.3/9.0 (9.1/8.7), 20 10.2/9.0 (11.3/8.7);
+//         14336, 13 rows 8.3/9.7 (9.1/9.2), 14 10.2/9.7 (11.2/9.2); 16384, 12 rows 8.0/9.4 (8.9/9.2), 13 9.8/9.4 (10.7/9.2);
+//         28672, 13 rows 10.9/13.0 (12.8/12.8), 14 13.7/13.0 (16.3/12.7); two slices: 57344, 9 rows 12.0/13.6, 10 16.7/13.7
+//         order >= 100:  1248, 16 rows 9.5/11.2, 20 11.3/11.2; 4992, 10 rows 10.5/10.8, 12 11.6/10.8; a vector on the way in, which
+//         that form reads again in every workgroup: 11008, 5 rows 10.6/11.5, 6 12.6/11.5; 13824, 7 rows 9.4/9.3, 8 11.6/9.2; 22016,
+//         2 rows 8.8/11.7, 3 12.3/11.7; none: 11008, 7 rows 11.5/11.2, 8 13.3/11.2; 13824, 7 rows 8.5/9.6, 8 10.5/9.6; 22016, 4 rows
+//         11.1/12.0, 5 14.0/12.0
 // With an element-wise prologue or a residual the matrix form is the one that covers every size, from 12 rows on at the
 // latest (8 at orders from 100 on).  Prologue SiLU: 5120, 6 rows 4.6/5.8, 7 7.1/5.8; 11008, 2 rows 8.7/8.4, 3 11.8/8.6;
 // 14336, 4 rows 5.6/7.0, 5 8.9/6.9; 28672, 4 rows 7.4/9.0, 5 12.6/9.0; two slices: 57344, 4 rows 12.1/18.6, 5 22.5/18.5.  RMSNorm:
 // 5120, 6 rows 4.7/6.9, 7 7.3/6.9; 11008, 2 rows 8.4/9.7, 3 11.5/9.9; 14336, 4 rows 5.5/8.1, 5 8.8/8.1.  A residual alone, fp16
 // rows: 5120, 6 rows 4.0/5.9, 7 5.9/5.9; 11008, 2 rows 6.0/7.2, 3 7.9/7.4; 14336, 4 rows 4.3/6.5, 5 6.5/6.5; 28672, 4 rows 5.0/7.1,
-// 5 8.0/7.1; two slices, which take three planes: 57344, 9 rows 13.7/14.8, 10 19.4/15.1.  A residual and fp32 rows, three planes
+// 5 8.0/7.1; orders from 100 on over fewer points: 4992, 3 rows 7.6/8.5 (RMSNorm; SiLU 7.1/7.8, a residual 6.0/6.7), 4 10.2/8.5;
+// 9984, 3 rows 8.8/9.4, 4 12.1/9.4; two slices, which take three planes: 57344, 9 rows 13.7/14.8, 10 19.4/15.1.  A residual and fp32 rows, three planes
 // as well: 5120, 11 rows 6.0/8.3; 11008, 5 rows 11.1/12.1, 8 16.1/12.1; 28672, 11 rows 11.2/13.3, 57344, 10 rows 18.5/13.9.
-int mix_rows_min(int order, int n, long wgs, bool f16, bool pre, bool residual,
-                 int slices) {
+int mix_rows_min(int order, int n, long wgs, bool f16, bool vector_in, bool prologue, bool residual, int slices) {
   const bool large = order >= 100;
   auto above = [&](int count) { return (int)(count / wgs) + 1; };  // the first row count of more than `count` workgroups
-  if (pre || residual) {
+  if (prologue || residual) {
     const int most = large ? 8 : 12;
     if (n <= 4096 || (!f16 && slices == 1)) return most;
-    const int line = above(large ? 360 : (slices > 1 && !pre ? 510 : 256));
+    const int line = above(large ? (n < 10000 ? 470 : 360) : (slices > 1 && !prologue ? 510 : 256));
     return line < most ? line : most;
   }
   if (slices > 1) return above(510);
   if (large) {
     if (n <= 4096) return above(f16 ? 1024 : 3400);
     if (n < 8192) return above(f16 ? 700 : 1800);
-    if (n < 16384) return above(f16 ? 430 : 860);
-    return above(f16 ? 256 : 400);
+    if (n < 16384) return f16 ? above(430) : (vector_in ? above(860) : 8);
+    return above(f16 ? 256 : (vector_in ? 400 : 768));
   }
   if (n <= 4096) return (int)(((f16 ? 512 + n / 10 : 1100 + n / 6) + wgs - 1) / wgs);
   if (n < 10000) return above(f16 ? 512 : 1024);
-  return above(f16 ? 256 : 600);
+  return above(f16 ? 256 : 768);
 }
 
 int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream) {
@@ -895,8 +899,8 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
                     ((P.pre_row_stride * 2) & 15u) == 0 && ((P.post_row_stride * 4) & 15u) == 0 &&
                     !(P.pre_mode != PRE_NONE && in_dtype != QTIP_F16) && !(fused && out_dtype != QTIP_F16) &&
                     mix_shape(n, order, rows, M, kt) &&
-                    rows >= mix_rows_min(order, n, OT, in_dtype == QTIP_F16, P.pre_mode != PRE_NONE, P.residual != nullptr,
-                                         1 << M.logS);
+                    rows >= mix_rows_min(order, n, OT, in_dtype == QTIP_F16, P.pre != nullptr, P.pre_mode != PRE_NONE,
+                                         P.residual != nullptr, 1 << M.logS);
     if (ok) {
       int cus = 0;
       const int rc = qtip_device_ready(stream, &cus);
@@ -1075,7 +1079,7 @@ bool qtip_rht_takes_parts(int n, int order, int rows, int nparts, bool residual)
   MixShape M{};
   int kt = 0;
   return mix_shape(n, order, rows, M, kt) && nparts << 5 <= 1 << M.logpp &&
-         rows >= mix_rows_min(order, n, OT, true, false, residual, 1 << M.logS);
+         rows >= mix_rows_min(order, n, OT, true, false, false, residual, 1 << M.logS);
 }
 
 int qtip_rht_from_parts(void* out, int out_dtype, const float* parts, int nparts, int rows, int n, int order,

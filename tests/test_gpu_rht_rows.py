@@ -276,3 +276,34 @@ def test_rows_with_a_residual_either_side_of_the_line(n, line16, line32):
         got = ops.rht(x, residual=res, **kw)
         # (exact values within half an fp16 step and the fp32 sums' error of each other; twice for a rounding of two sums)
         assert not torch.equal(got, one) and float((got.float() - one.float()).abs().max()) <= 2.0**-9 * float(one.abs().max())
+
+
+@pytest.mark.parametrize("n,kind,line", [(10240, "post32", 20), (14336, "post32", 14), (14336, "pre32", 14), (16384, "post32", 13),
+                                         (28672, "post32", 14), (11008, "post32", 8), (11008, "pre32", 6), (22016, "post32", 5),
+                                         (22016, "pre32", 3), (57344, "post32", 10), (4992, "norm", 4), (9984, "silu", 4),
+                                         (11008, "norm", 3), (14336, "silu", 5), (5120, "norm", 7)])
+def test_rows_either_side_of_the_line(n, kind, line):
+    """The row counts from which few rows take the matrix form: one below it every row has the bits of a launch of its own,
+    on it the sums run in another order, with the same rounding points."""
+    from qtip_amd import ops
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    had, K = get_hadK(n)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    kw = dict(order=K, had_bits=had_bits(had, K, True, "cuda") if K > 1 else None)
+    x = rnd(line, 2 * n if kind == "silu" else n)
+    if kind == "post32":
+        kw.update(post=rnd(n))
+    else:
+        kw.update(pre=torch.sign(rnd(n) + 1e-5).half())
+    if kind in ("norm", "silu"):
+        x = x.half()
+        kw.update(dict(pre_mode=ops.PRE_SILU_MUL) if kind == "silu" else
+                  dict(pre_mode=ops.PRE_RMSNORM, norm_weight=(1 + 0.1 * rnd(n)).half(), eps=1e-5))
+    one = torch.cat([ops.rht(x[i:i + 1], **kw) for i in range(line)])
+    assert torch.equal(ops.rht(x[:-1], **kw), one[:-1])
+    got = ops.rht(x, **kw)
+    # fp32 sums of n terms; a prologue's fp16 values may round the other way (a norm's sum of squares in another order)
+    tol = 2e-3 if kind in ("norm", "silu") else 1e-5
+    assert float((got.float() - one.float()).abs().max()) <= tol * float(one.abs().max())
+    assert kind in ("norm", "silu") or not torch.equal(got, one)  # (fp16 results may all round the same way)
