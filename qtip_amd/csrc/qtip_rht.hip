@@ -759,7 +759,10 @@ int launch_mix(const RhtParams& P, MixShape M, int kt, int rows, int cus, hipStr
   // rows 7.0/10.2, 45 rows 7.7/10.8; 11008, 45 rows 7.6/9.8, 128 rows 8.2/10.4; fp32 45 rows 12.0/15.8.  Not where
   // they would be more than one to a CU: 14336, 180 rows 8.8/8.4.
   const int eights = (gx + 7) >> 3;
-  const int z = (cus >> M.logS) / (8 * eights);
+  int z = (cus >> M.logS) / (8 * eights);
+  // Nor behind a norm, whose sum of squares every workgroup of a pass takes over the whole row, where a pass is four k tiles at most:
+  // 16384, 32 rows 8.6/8.4, 64 9.4/8.6, 128 9.7/9.3; 14336, 64 rows 9.5/9.0 (24 rows 8.7/8.7; seven tiles, 28672, 64 rows 12.6/13.3).
+  if (MODE == PRE_RMSNORM && kt <= 4 && M.npass >= 32) z = 1;
   M.share = z > 1 && !in_place(P, rows, sizeof(TI), sizeof(TO)) ? (2 * kt + z - 1) / z : 2 * kt;
   if (M.share < 2) M.share = 2;
   const dim3 grid(8, (unsigned)((2 * kt + M.share - 1) / M.share), (unsigned)eights << M.logS);
