@@ -761,8 +761,8 @@ int launch_mix(const RhtParams& P, MixShape M, int kt, int rows, int cus, hipStr
   const int eights = (gx + 7) >> 3;
   int z = (cus >> M.logS) / (8 * eights);
   // Nor behind a norm, whose sum of squares every workgroup of a pass takes over the whole row, where a pass is four k tiles at most:
-  // 16384, 32 rows 8.6/8.4, 64 9.4/8.6, 128 9.7/9.3; 14336, 64 rows 9.5/9.0 (24 rows 8.7/8.7; seven tiles, 28672, 64 rows 12.6/13.3).
-  if (MODE == PRE_RMSNORM && kt <= 4 && M.npass >= 32) z = 1;
+  // 16384, 45 rows 7.9/7.9, 64 8.2/7.9; 14336, 45 rows 8.2/8.2, 64 8.5/8.3, 128 8.9/8.7 (seven tiles: 28672, 64 rows 11.7/12.9).
+  if (MODE == PRE_RMSNORM && kt <= 4 && M.npass >= 48) z = 1;
   M.share = z > 1 && !in_place(P, rows, sizeof(TI), sizeof(TO)) ? (2 * kt + z - 1) / z : 2 * kt;
   if (M.share < 2) M.share = 2;
   const dim3 grid(8, (unsigned)((2 * kt + M.share - 1) / M.share), (unsigned)eights << M.logS);
@@ -822,10 +822,10 @@ bool rows_form_size(int n, int order, int rows) {
 // With an element-wise prologue or a residual the matrix form is the one that covers every size, from 12 rows on at the
 // latest (8 at orders from 100 on).  Prologue SiLU: 5120, 6 rows 4.6/5.8, 7 7.1/5.8; 11008, 2 rows 8.7/8.4, 3 11.8/8.6;
 // 14336, 4 rows 5.6/7.0, 5 8.9/6.9; 28672, 4 rows 7.4/9.0, 5 12.6/9.0; two slices: 57344, 4 rows 12.1/18.6, 5 22.5/18.5.  RMSNorm:
-// 5120, 6 rows 4.7/6.9, 7 7.3/6.9; 11008, 2 rows 8.4/9.7, 3 11.5/9.9; 14336, 4 rows 5.5/8.1, 5 8.8/8.1.  A residual alone, fp16
+// 5120, 6 rows 4.8/6.4, 7 7.4/6.4; 11008, 2 rows 8.5/9.7, 3 11.7/9.8; 14336, 4 rows 5.5/7.6, 5 9.0/7.6.  A residual alone, fp16
 // rows: 5120, 6 rows 4.0/5.9, 7 5.9/5.9; 11008, 2 rows 6.0/7.2, 3 7.9/7.4; 14336, 4 rows 4.3/6.5, 5 6.5/6.5; 28672, 4 rows 5.0/7.1,
-// 5 8.0/7.1; orders from 100 on over fewer points: 4992, 3 rows 7.6/8.5 (RMSNorm; SiLU 7.1/7.8, a residual 6.0/6.7), 4 10.2/8.5;
-// 9984, 3 rows 8.8/9.4, 4 12.1/9.4; two slices, which take three planes: 57344, 9 rows 13.7/14.8, 10 19.4/15.1.  A residual and fp32 rows, three planes
+// 5 8.0/7.1; orders from 100 on over fewer points: 4992, 3 rows 7.5/8.3 (RMSNorm; SiLU 7.1/7.8, a residual 6.0/6.7), 4 10.2/8.3;
+// 9984, 3 rows 8.8/9.3, 4 12.0/9.3; two slices, which take three planes: 57344, 9 rows 13.7/14.8, 10 19.4/15.1.  A residual and fp32 rows, three planes
 // as well: 5120, 11 rows 6.0/8.3; 11008, 5 rows 11.1/12.1, 8 16.1/12.1; 28672, 11 rows 11.2/13.3, 57344, 10 rows 18.5/13.9.
 int mix_rows_min(int order, int n, long wgs, bool f16, bool vector_in, bool prologue, bool residual, int slices) {
   const bool large = order >= 100;

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   };
   auto first_row = [&](int ps) { return (size_t)ps << lrows; };
   auto lane_row = [&](int ps) { return (int)first_row(ps) + rsub < rows ? (uint32_t)rsub : 0u; };  // (a row to read)
-  auto load_patch = [&](Patch& p, int ps, uint32_t add) {
+  auto load_patch = [&](Patch& p, int ps, uint32_t add, bool vectors = true) {
     const TIn* src = in + first_row(ps) * P.in_row_stride;
     const uint32_t lr = lane_row(ps) * (uint32_t)P.in_row_stride + add;
     if constexpr (PARTS) {
@@ -144,6 +144,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
 #pragma unroll
       for (int i = 0; i < 4; ++i) p.x[i].load(src + (lr + eoff[i]));
     }
+    if (!vectors) return;
     if (P.pre) {
       const _Float16* f = P.pre + first_row(ps) * P.pre_row_stride;
       const uint32_t lf = lane_row(ps) * (uint32_t)P.pre_row_stride + add;
@@ -385,6 +386,15 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
       fast = flag[1] == 0;
     }
     if (fast) {
+      // behind a norm the signs go into its weights, which every pass has in common: read again for each and kept beside the
+      // products' operands they cost 13 to 16 registers of scratch (us, 1000 rows, then / now: 28672 51.1/41.4, 4096 9.5/8.5)
+      constexpr bool NORM = MODE == PRE_RMSNORM;
+      if (NORM && P.pre) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          cur.u[AUX ? i : 0].a = __builtin_bit_cast(uint4, __builtin_bit_cast(u32x4m, cur.u[AUX ? i : 0].a) ^
+                                                      (__builtin_bit_cast(u32x4m, cur.f[i].a) & 0x80008000u));
+      }
       for (; ps < M.npass; ps += step) {
         float rs = 1.f;
         if constexpr (MODE == PRE_RMSNORM) rs = row_rs(cur, ps);
@@ -392,7 +402,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           h[i] = __builtin_bit_cast(u32x4m, prologue(cur.x[i], cur.u[AUX ? i : 0], rs));
-          if (P.pre) h[i] ^= __builtin_bit_cast(u32x4m, cur.f[i].a) & 0x80008000u;
+          if (!NORM && P.pre) h[i] ^= __builtin_bit_cast(u32x4m, cur.f[i].a) & 0x80008000u;
         }
         if (edge) {
 #pragma unroll
@@ -406,7 +416,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
           w.y = __builtin_amdgcn_perm(h[3][e >> 1], h[2][e >> 1], (e & 1) ? 0x07060302u : 0x05040100u);
           *reinterpret_cast<uint2*>(wr + e * 16 * stride) = w;
         }
-        if (ps + step < M.npass) load_patch(cur, ps + step, 0);
+        if (ps + step < M.npass) load_patch(cur, ps + step, 0, !NORM);
         __syncthreads();
         float4v acc[8];
 #pragma unroll
