@@ -344,7 +344,7 @@ int qtip_rht_chain(void* xt_out_f16, void* x_out_f16, const float* parts, int in
  * caches are [kv_heads][max_len][d] fp16, pos_i64 points to the position in DEVICE memory (a
  * recorded graph then follows the position), inv_freq[d/2] fp32.  out_f16 = [heads*d].
  * key_splits (1..16): 1 = one workgroup per head walks the whole context (right up to a few
- * hundred keys: 32 heads of 128, 5 us at 150, 9 us at 500, 14 us at 1000); > 1 = the cache slots are cut into
+ * hundred keys: 32 heads of 128, 5 us at 150, 7 us at 500, 13 us at 1000); > 1 = the cache slots are cut into
  * key_splits equal ranges of max_len / key_splits slots, one workgroup per head and range, and a
  * second small launch combines the ranges' softmax shares, which pass through split_workspace:
  * heads * key_splits * (head_dim + 2) floats, 16-byte aligned, no initialisation needed (may be

@@ -824,9 +824,9 @@ def generate(model, prompt_ids, max_new_tokens, use_graph=True, fused=True, temp
         return g, nxt
 
     # the fused attention has two forms (one workgroup per head; key ranges for long contexts): a run
-    # that crosses ops.ATTN_SPLIT_FROM records its step again there, so short contexts never pay
+    # that crosses the line between them records its step again there, so short contexts never pay
     # for the second launch of the long form
-    splits_at = lambda ctx: ops.attention_key_splits(ctx) if fused else 1
+    splits_at = lambda ctx: ops.attention_key_splits(ctx, model.cfg.heads) if fused else 1
     model.cfg.attn_key_splits = splits_at(n + 1)
     graph = static_next = None
     if use_graph:

@@ -587,14 +587,21 @@ def rht_silu_pair_ok(n, order, two_vectors):
 ATTN_MAX_KEY_SPLITS = 16
 
 
-ATTN_SPLIT_FROM = 1024  # context length from which the key-range form is faster
+ATTN_SPLIT_FROM = 1024  # context length from which the key-range form is faster, of heads whose ranges fit the chip side by side
+ATTN_SPLIT_FROM_MANY = 2560  # and of more heads than that
 
 
-def attention_key_splits(context):
-    """Key ranges per head for decode attention over a context of `context` tokens: one workgroup
-    per head below ATTN_SPLIT_FROM keys (the ranges cost a second small launch: 32 heads of 128, 250 keys
-    5.5 vs 7.9 us; 64 heads on 8, 1000 keys 12.6 vs 14.6), 8 ranges from there on (32 heads on 8, 2000 keys
-    22 -> 14 us, 4000 keys 40 -> 19 us)."""
+def attention_key_splits(context, heads=None):
+    """Key ranges per head for decode attention over a context of `context` tokens: one workgroup per head below
+    ATTN_SPLIT_FROM keys, 8 ranges from there on.  The ranges cost a second small launch, and every one of them repeats the
+    transform of the new token: more than 40 heads (of `heads`, where given) keep one workgroup up to ATTN_SPLIT_FROM_MANY
+    keys and then have as many ranges as 256 compute units hold.  us a launch with that transform, one range / eight: 32 heads
+    of 128, 250 keys 9.0/11.7; 32 on 8, 900 keys 12.0/12.7, 1200 13.4/12.9, 2000 18.1/15.0, 4000 29.3/20.3; 32 on 32, 900
+    12.0/12.6, 1200 16.5/13.9; 40, 900 13.8/15.5, 1200 17.8/15.8.  One / four / eight: 64 on 8, 1024 keys 12.5/16.2/21.2, 2000
+    18.7/19.2/25.3, 2500 21.8/20.3/27.1, 4000 30.7/26.1/31.1; one / two / four: 128 on 8, 2500 23.1/24.0/29.3, 3000
+    26.1/25.5/32.5."""
+    if heads is not None and heads > 40:
+        return 1 if context < ATTN_SPLIT_FROM_MANY else max(1, 256 // heads)
     return 1 if context < ATTN_SPLIT_FROM else 8
 
 

@@ -483,3 +483,15 @@ def test_header_and_host_module_are_of_one_version():
     text = open(os.path.join(ROOT, "include", "qtip_hip.h")).read()
     assert int(re.search(r"#define QTIP_ABI_VERSION (\d+)", text)[1]) == _lib.ABI_VERSION == _lib.host().abi_version
     assert _lib.host().torch_version == torch.__version__
+
+
+def test_key_ranges_of_a_context():
+    """One workgroup a head for short contexts; ranges fit the chip side by side, as many as the kernel takes."""
+    from qtip_amd import ops
+    line, many = ops.ATTN_SPLIT_FROM, ops.ATTN_SPLIT_FROM_MANY
+    for heads in (None, 1, 8, 32, 40):
+        assert [ops.attention_key_splits(c, heads) for c in (1, line - 1, line, 4096)] == [1, 1, 8, 8]
+    assert ops.attention_key_splits(line) == 8
+    for heads, ranges in ((41, 6), (64, 4), (128, 2), (256, 1), (300, 1)):
+        assert [ops.attention_key_splits(c, heads) for c in (line, many - 1, many, 4096)] == [1, 1, ranges, ranges]
+        assert ranges <= ops.ATTN_MAX_KEY_SPLITS
