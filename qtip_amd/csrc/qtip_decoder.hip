@@ -20,17 +20,6 @@ constexpr int kMaxHeadDim = 256;
 __device__ __forceinline__ int lane_xor_i(int v, int b) {
   return __builtin_bit_cast(int, qtip_wht::lane_xor(__builtin_bit_cast(float, v), b));
 }
-__device__ __forceinline__ float wave_reduce_max(float v) {
-#pragma unroll
-  for (int b = 5; b >= 0; --b) v = fmaxf(v, qtip_wht::lane_xor(v, b));
-  return v;
-}
-__device__ __forceinline__ float wave_reduce_sum(float v) {
-#pragma unroll
-  for (int b = 5; b >= 0; --b) v += qtip_wht::lane_xor(v, b);
-  return v;
-}
-
 // The qkv projection's output transform, for the XF form of the kernel: the new token's
 // [q | k | v] vector (n = order * 2^logp2 elements) is
 //   post * scale * (H_order (x) H_{2^logp2}) (sum of the in_parts partial sums),
@@ -455,7 +444,7 @@ static int launch_attention(void* out_f16, const void* qkv_f16, const AttnXf* xf
   if (key_splits > 1 && !split_ws) return QTIP_E_NULL;
   if (key_splits > 1 && (reinterpret_cast<uintptr_t>(split_ws) & 15)) return QTIP_E_ALIGN;
   if (heads < 1 || kv_heads < 1 || heads % kv_heads || head_dim < 64 || head_dim > kMaxHeadDim ||
-      (head_dim & (head_dim - 1)) || max_len < 1 || max_len > 4096)
+      (head_dim & (head_dim - 1)) || max_len < 1 || max_len > 4096)  // (positions the rotary reduction is stated for)
     return QTIP_E_SHAPE;
   const size_t lds = (size_t)(6 * kMaxHeadDim + 32 + (xf ? 3 : 1) * 16 * head_dim) * sizeof(float);
   const dim3 grid((unsigned)(heads / kv_heads), (unsigned)kv_heads, (unsigned)key_splits);

@@ -628,7 +628,8 @@ class _FusedLinear:
         return self.transform_out(self.matvec(self.transform_in(x, pre_mode, norm_weight, eps)), residual)
 
 
-# the decode attention kernel keeps one score per cache slot in LDS
+# the positions for which the decode attention states its rotary angles (to 2^-29 of a turn) and is tested; its launcher takes
+# no longer caches
 FUSED_MAX_CACHE_LEN = 4096
 
 

@@ -438,3 +438,10 @@ def test_more_rows_and_positions_than_a_launch_has_threads():
     pos = torch.randint(0, 4096, (rows,), device="cuda")
     for big, few in zip(ops.rotary_tables(pos, inv), ops.rotary_tables(pos[pick], inv)):
         assert torch.equal(big[pick], few)
+
+
+@pytest.mark.parametrize("k,m,rows,mode,residual", [(4096, 4096, 2, 0, True), (4096, 22016, 5, 1, False), (11008, 4096, 3, 2, True),
+                                                    (5120, 28672, 9, 1, False), (28672, 8192, 11, 2, True), (928, 1248, 7, 2, True)])
+def test_projection_of_few_rows_in_one_call(k, m, rows, mode, residual):
+    """(The rows below those of a prompt, for callers of the native entry: the same check.)"""
+    test_projection_of_a_prompt_in_one_call(k, m, rows, mode, residual)

@@ -307,3 +307,34 @@ def test_rows_either_side_of_the_line(n, kind, line):
     tol = 2e-3 if kind in ("norm", "silu") else 1e-5
     assert float((got.float() - one.float()).abs().max()) <= tol * float(one.abs().max())
     assert kind in ("norm", "silu") or not torch.equal(got, one)  # (fp16 results may all round the same way)
+
+
+@pytest.mark.parametrize("n,rows", [(928, 3), (4992, 4), (5120, 2), (5120, 7), (8960, 6), (11008, 3), (11008, 11), (14336, 5), (16384, 6),
+                                    (16384, 48), (28672, 9), (57344, 5), (57344, 9), (57344, 11)])
+@pytest.mark.parametrize("sign", [True, False])
+def test_few_rows_with_prologue_and_residual_against_float64(n, rows, sign):
+    """Either form of few rows with element-wise neighbours, sharing workgroups among them."""
+    from qtip_amd import ops
+    from qtip_amd.utils.matmul_had import get_hadK, had_bits
+    had, K = get_hadK(n)
+    g = torch.Generator(device="cuda").manual_seed(n + rows)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    bits = {t: had_bits(had, K, t, "cuda") if K > 1 else None for t in (True, False)}
+    pre = torch.sign(rnd(n) + 1e-5)
+    pre = (pre if sign else pre * (0.5 + torch.rand(n, generator=g, device="cuda"))).half()
+    w, post = (1 + 0.1 * rnd(n)).half(), rnd(n)
+    x, gu, res = rnd(rows, n).half(), rnd(rows, 2 * n).half(), rnd(rows, n).half()
+    d = x.double()
+    normed = w.double() * (d * torch.rsqrt(d.pow(2).mean(-1, keepdim=True) + 1e-5)).half().double()
+    gate, up = gu.double().split(n, -1)
+    cases = [(x, dict(pre=pre, residual=res), d * pre.double(), res.double()), (x, dict(post=post, residual=res), d, res.double()),
+             (gu, dict(pre=pre, pre_mode=ops.PRE_SILU_MUL),
+              ((gate * torch.sigmoid(gate)).half().double() * up).half().double() * pre.double(), 0.0)]
+    if n <= 16384 or rows >= 5:  # (the norm of longer rows has the matrix form alone)
+        cases.append((x, dict(pre=pre, pre_mode=ops.PRE_RMSNORM, norm_weight=w, eps=1e-5), normed.half().double() * pre.double(), 0.0))
+    for src, kw, ref, more in cases:
+        t = "pre" in kw
+        got = ops.rht(src, order=K, had_bits=bits[t], out_dtype=torch.float16, **kw)
+        ref = _transform(ref, n, t) * n**-0.5 * (post.double() if "post" in kw else 1.0) + more
+        # fp16 results; a prologue's fp16 values on the edge that round the other way move all elements of a row by 2^-11 / sqrt(n) each
+        assert float((got.double() - ref).abs().max()) <= 1e-3 * float(ref.abs().max()), kw.keys()
