@@ -36,7 +36,8 @@ constexpr size_t kGemmLds = kLut128Bytes + kGemmTileBytes;
 // needs, chunk index xor-ed with the row (conflict-free both ways).  The next tile waits in registers; with room for two
 // tiles in LDS there is one barrier per stage, else two.  Work unit = (two pairs, k range s); a workgroup keeps one s, so the
 // pipeline runs across unit boundaries.  The k slices of a unit meet in the tile buffer at its end.
-// NB = 1 is bound by the weight stream, NB = 2 by its stages' phases.  The forms of gemm_rows_kernel at 17 to 32 rows have
+// NB = 1 waits at its barriers and for LDS (28672x8192, 4 bits, 16 rows: 4.0 TB/s of weights, waits 48 % of the waves' cycles, LDS busy
+// 54 %, a fifth of that conflicts; the kernel of one row streams 5.5), NB = 2 for its stages' phases.  The forms of gemm_rows_kernel at 17 to 32 rows have
 // half the slices: within what eight of them are off by (fine_error) they take 0.9 to 1.6 times as long, with chains twice as
 // long 0.87 to 1.08.  us from cold memory, launches and sums of ranges included, 32 rows at 2 bits: 4096x4096 13.1,
 // 22016x4096 19.7, 28672x8192 34, 4096x11008 17.1, 8192x28672 36.

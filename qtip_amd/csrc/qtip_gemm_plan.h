@@ -72,7 +72,7 @@ inline int fine_error(int m, int k, int nb, int cus, bool split) {
   return sum_error(k, KS, wl_per, (nwl + wl_per - 1) / wl_per);
 }
 
-// Up to 16 rows: where the weight stream is the bound and the activations would be in its way, they are shared.  us from cold
+// Up to 16 rows: where the stream of weights is long and a wave's own reads of the activations would stand in its way, they are shared.  us from cold
 // memory, gemm_kernel / gemm_few_kernel: 28672x8192 at 4 bits 2 rows 27.5/27.7, 6 27.9/27.9, 9 28.5/29.1, 16 28.0/34.2; at
 // 3 bits 2 rows 28.5/27.6, 6 28.3/28.6, 16 27.9/30.0; 22016x4096 at 4 bits 6 rows 15.4/14.7, 9 15.6/15.1, 16 15.9/16.8;
 // 10240x8192 at 4 bits 16 rows 18.2/16.9.
