@@ -36,7 +36,8 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this script, each calibrated
 # against a 256 MiB copy) are read from this summary, which names the kernel sources it was taken on
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "matvec_k2_llama70b_set_traffic.txt")
-KERNEL_SOURCES = ("qtip_amd/csrc/qtip_hip.hip", "qtip_amd/csrc/qtip_device.h", "qtip_amd/csrc/qtip_wht.h")
+KERNEL_SOURCES = ("qtip_amd/csrc/qtip_hip.hip", "qtip_amd/csrc/qtip_device.h", "qtip_amd/csrc/qtip_wht.h",
+                  "qtip_amd/csrc/qtip_chain.h")
 
 
 def kernel_source_digest():

@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define QTIP_ABI_VERSION 26 /* of this header; a library tells its own by qtip_abi_version() */
+#define QTIP_ABI_VERSION 27 /* of this header; a library tells its own by qtip_abi_version() */
 
 #define QTIP_OK 0
 #define QTIP_E_SHAPE (-1)     /* m % 32, k % 32, bits, batch or n out of range */
@@ -388,6 +388,15 @@ int qtip_decode_attention_rht3(void* out_f16, const float* const* parts, int in_
 int qtip_rmsnorm(void* out_f16, const void* x_f16, const void* weight_f16, float eps, int n, void* stream);
 /* The same for each of `rows` rows of n values, one after the other in memory. */
 int qtip_rmsnorm_rows(void* out_f16, const void* x_f16, const void* weight_f16, float eps, long rows, int n, void* stream);
+
+/* The end of a decoded token in one launch (model/llama.py:1466-1467 behind the last decoder layer):
+ *   logits = fp16(head . fp16(weight * fp16(y * rsqrt(mean(y^2) + eps)))),  out_dtype QTIP_F16 or QTIP_F32 (the fp16 values)
+ * head fp16 [vocab][n], sums fp32.  y is x itself where parts is NULL (n a multiple of 8 up to 8192), else the last layer's
+ * boundary as in qtip_rht_fused: y = fp16(x + fp16(post * scale_out * H_n (sum over in_parts of parts))), parts
+ * [in_parts][n] with part_stride floats between them, n in {2048, 4096, 8192}. */
+int qtip_token_head(void* out, int out_dtype, const void* head_f16, int vocab, int n, const void* x_f16,
+                    const float* parts, int in_parts, size_t part_stride, const float* post_f32, float scale_out,
+                    const void* norm_weight_f16, float eps, void* stream);
 
 /* Greedy token pick of the generation loop (eval/interactive_gen.py:43-69: argmax of the last
  * position's logits, copy into the next step's input, position + 1), all in device memory so a

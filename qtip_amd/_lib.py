@@ -17,7 +17,7 @@ HOST_PATH = os.path.join(_HERE, "_qtip_host.so")
 
 QTIP_F16 = 0
 QTIP_F32 = 1
-ABI_VERSION = 26
+ABI_VERSION = 27
 
 _lib = None
 _host = None
@@ -105,6 +105,9 @@ _SIGNATURES = {
     "qtip_rmsnorm_rows": (ctypes.c_int, [ctypes.c_void_p] * 3 + [ctypes.c_float, ctypes.c_long, ctypes.c_int, ctypes.c_void_p]),
     "qtip_rotary_tables": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_long, ctypes.c_int, ctypes.c_void_p]),
     "qtip_rmsnorm": (ctypes.c_int, [ctypes.c_void_p] * 3 + [ctypes.c_float, ctypes.c_int, ctypes.c_void_p]),
+    "qtip_token_head": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_int] +
+                        [ctypes.c_void_p] * 2 + [ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_float,
+                                                 ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p]),
     "qtip_greedy_pick": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int] + [ctypes.c_void_p] * 3 +
                          [ctypes.c_long, ctypes.c_long, ctypes.c_void_p]),
     "qtip_sample_pick": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_int, ctypes.c_uint] +

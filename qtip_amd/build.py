@@ -8,7 +8,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRCS = [os.path.join(HERE, "csrc", f)
         for f in ("qtip_hip.hip", "qtip_gemm.hip", "qtip_rht.hip", "qtip_decoder.hip", "qtip_pack.hip", "qtip_prefill.hip", "qtip_train.hip",
-                  "qtip_linear.hip")]
+                  "qtip_linear.hip", "qtip_head.hip")]
 OUT = os.path.join(HERE, "libqtip_hip.so")
 HOST_SRC = os.path.join(HERE, "csrc", "qtip_host.cpp")
 HOST_OUT = os.path.join(HERE, "_qtip_host.so")

@@ -13,12 +13,19 @@
 #include "qtip_setup.h"
 #include "qtip_wht.h"
 
+#ifdef QTIP_STAMPS  // (the timeline build, see QTIP_STAMP)
+// inside the layer boundary of the prologue (sv = the kernel's stamp_v): 6 entered, 7 / 8 / 9 past its
+// first / second / third barrier (first transform, RMSNorm sum, second transform), 10 left
+#define QTIP_STAMP_SV(i) if (wave == 0 && sv) sv[i] = __builtin_amdgcn_s_memrealtime();
+#endif
+#include "qtip_chain.h"
+
 using namespace qtip;
+using namespace qtip_chain;
 
 namespace {
 
-constexpr int kThreads = 1024;  // 16 waves per workgroup, one workgroup per CU
-constexpr int kWaves = kThreads / 64;
+// kThreads = 1024: 16 waves per workgroup, one workgroup per CU
 constexpr int kMaxSplit = 16;
 
 __device__ __forceinline__ float dpp_xor1(float v) {
@@ -173,24 +180,13 @@ __device__ __forceinline__ void xform_prologue(const float v_in[8], float scale,
   __syncthreads();  // xchg is free for the table, xs is complete
 }
 
-// XFORM == 2: the whole boundary between two linear layers of a decoder in front of the matvec,
-//   x_new = residual + fp16(scale_out * post * H_k (sum of the previous layer's partial results)),
-//   x_t   = fp16(scale_in * H_k (su * RMSNorm(x_new) * norm_w)),    parts_out = hatW . x_t
-// i.e. the output transform of the previous QuantizedLinear with the residual addition, the
-// RMSNorm and the input transform of this one (what rht_chain_kernel does in a launch of its
-// own).  Every workgroup recomputes the k-point boundary - a few microseconds of work on 1024
-// threads, most of it while the first stream requests are in flight - and workgroup (0, 0)
-// stores x_new for the layers that follow.
-struct ChainArgs {
-  const float* parts;        // [in_parts][k] fp32 partial results of the previous linear layer
-  const float* post;         // its output sign vector times its scale (SV), k fp32
-  const _Float16* residual;  // the residual stream, k fp16
-  const _Float16* norm_w;    // RMSNorm weight, k fp16
-  _Float16* x_out;           // the new residual stream, k fp16
-  size_t part_stride;        // floats between partial results
-  float scale_out, eps;
-  int in_parts;
-};
+// XFORM == 2: the whole boundary between two linear layers of a decoder (qtip_chain.h) in front of the matvec, what
+// rht_chain_kernel does in a launch of its own.  Every workgroup recomputes the k-point boundary - a few microseconds of
+// work on 1024 threads, most of it while the first stream requests are in flight - and workgroup (0, 0) stores x_new for
+// the layers that follow.
+static_assert(sizeof(float) * kChainFloats<4> <= kLut128Bytes && sizeof(float) * kChainFloats<8> <= kLut128Bytes,
+              "the boundary's buffers fit the table's LDS");
+
 // Up to three matrices with the same k and bit width in one launch (the separate q / k / v or
 // gate / up projections of a decoder layer): the workgroups blockIdx.y in
 // [wg_begin[g], wg_begin[g + 1]) serve matrix g with its own stream, table, sign vector and
@@ -222,153 +218,16 @@ __device__ unsigned long long g_stamps[kStampSlots][kStampWgs][kStampN];
 #define QTIP_STAMP_DECL unsigned long long stamp_v[kStampN] = {};
 #define QTIP_STAMP(i) if (wave == 0 || (i == 0 && wave == kWaves - 1)) stamp_v[i] = __builtin_amdgcn_s_memrealtime();
 #define QTIP_STAMP_FIRST_LOAD() if (wave == 0) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DEPTH - 1)); stamp_v[15] = __builtin_amdgcn_s_memrealtime(); }
-// inside the layer boundary of the prologue (sv = the kernel's stamp_v): 6 entered, 7 / 8 / 9 past its
-// first / second / third barrier (first transform, RMSNorm sum, second transform), 10 left
-#define QTIP_STAMP_SV(i) if (wave == 0 && sv) sv[i] = __builtin_amdgcn_s_memrealtime();
 #define QTIP_STAMP_PTR stamp_v
 #else
 #define QTIP_STAMP_DECL
 #define QTIP_STAMP(i)
 #define QTIP_STAMP_FIRST_LOAD()
-#define QTIP_STAMP_SV(i)
 #define QTIP_STAMP_PTR nullptr
 #endif
 template <typename T>
 __device__ __forceinline__ T pick3(const T (&a)[3], int g) {
   return g == 0 ? a[0] : (g == 1 ? a[1] : a[2]);
-}
-
-struct ChainRegs {  // a thread's operands, k / 1024 <= 8 consecutive elements each
-  float v[8], pv[8], rv[8], wv[8], sv[8];
-};
-
-// Where the operands of the boundary's middle part are read.  It works in the swapped layout, in which
-// the lanes of a wave hold 16 runs of 4 * EPT consecutive elements: with eight elements a thread a
-// run is 64 bytes of fp16 and the operands are read there, with two or four it is half that or less
-// and a load touches four to eight times the cache lines it needs, so that they are read in the
-// natural layout and change over in LDS.  A token of 8 layers of 4096 (16 boundaries): 583 -> 565 us;
-// of layers of 8192, with the change-over in LDS or without, the same.
-template <int EPT>
-constexpr bool kChainStaged = EPT < 8;
-
-template <int EPT>
-__device__ __forceinline__ void chain_load(const ChainArgs& c, const _Float16* su, int tid, int lane,
-                                           int wave, ChainRegs& r) {
-  using namespace qtip_wht;
-  const int e_nat = tid * EPT;
-  const int e_mid = kChainStaged<EPT> ? e_nat : (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
-  ld_f32<EPT>(c.post + e_mid, r.pv);
-  ld_f16<EPT>(c.residual + e_mid, r.rv);
-  ld_f16<EPT>(c.norm_w + e_mid, r.wv);
-  ld_f16<EPT>(su + e_mid, r.sv);
-  ld_f32<EPT>(c.parts + e_nat, r.v);
-  for (int w = 1; w < c.in_parts; ++w) {
-    float t[EPT];
-    ld_f32<EPT>(c.parts + w * c.part_stride + e_nat, t);
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) r.v[i] += t[i];
-  }
-}
-
-// index of element e of an operand that changes over in LDS: a pad of four lanes per 64 puts the 16
-// runs of a read on banks of their own
-template <int EPT>
-__device__ __forceinline__ int sidx(int e) {
-  return e + 4 * EPT * (e / (64 * EPT));
-}
-// the floats of LDS behind xbuf and wsum that the operands take: one of fp32, three of fp16
-template <int EPT>
-constexpr int kChainStage = (kThreads + 64) * EPT * 5 / 2;
-
-// xbuf: k + k/64 floats of exchange buffer, wsum behind it: 16 floats and kChainStage of operands, all where the
-// table will be; xs: the k fp16 activations of the matvec
-template <int EPT>
-__device__ __forceinline__ void chain_compute(ChainRegs& r, const ChainArgs& c, float scale_in, float* xbuf,
-                                              float* wsum, _Float16* xs, int tid, int lane, int wave,
-                                              bool write_x, unsigned long long* sv = nullptr) {
-  using namespace qtip_wht;
-  constexpr int N = kThreads * EPT;
-  static_assert((N + N / 64 + kWaves + (kChainStaged<EPT> ? kChainStage<EPT> : 0)) * sizeof(float) <= kLut128Bytes,
-                "the boundary's buffers fit the table's LDS");
-  (void)sv;
-  QTIP_STAMP_SV(6)
-  const int e_nat = tid * EPT;
-  const int e_swp = (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
-  float v[EPT];
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = r.v[i];
-  // ---- first transform (natural -> swapped layout)
-  wht_regs<EPT>(v);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(v[i], 6, lane);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) xbuf[xidx<EPT>(e_nat + i)] = v[i];
-  float* post_s = wsum + kWaves;
-  _Float16* half_s = reinterpret_cast<_Float16*>(post_s + sidx<EPT>(N));  // residual, norm weight, sign vector
-  if constexpr (kChainStaged<EPT>) {
-    _Float16 h[EPT];
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) post_s[sidx<EPT>(e_nat) + i] = r.pv[i];
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) h[i] = (_Float16)r.rv[i];
-    st_f16<EPT>(half_s + sidx<EPT>(e_nat), h);
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) h[i] = (_Float16)r.wv[i];
-    st_f16<EPT>(half_s + sidx<EPT>(N) + sidx<EPT>(e_nat), h);
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) h[i] = (_Float16)r.sv[i];
-    st_f16<EPT>(half_s + 2 * sidx<EPT>(N) + sidx<EPT>(e_nat), h);
-  }
-  __syncthreads();
-  QTIP_STAMP_SV(7)
-  if constexpr (kChainStaged<EPT>) {
-    ld_f32<EPT>(post_s + sidx<EPT>(e_swp), r.pv);
-    ld_f16<EPT>(half_s + sidx<EPT>(e_swp), r.rv);
-    ld_f16<EPT>(half_s + sidx<EPT>(N) + sidx<EPT>(e_swp), r.wv);
-    ld_f16<EPT>(half_s + 2 * sidx<EPT>(N) + sidx<EPT>(e_swp), r.sv);
-  }
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(xbuf[xidx<EPT>(e_swp + i)], 4, lane);
-  // ---- residual, RMSNorm, sign vector of this layer
-  float ss = 0.f;
-  _Float16 xn[EPT];
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) {
-    const float o = v[i] * c.scale_out * r.pv[i];
-    xn[i] = (_Float16)(r.rv[i] + (float)(_Float16)o);
-    v[i] = (float)xn[i];
-    ss += v[i] * v[i];
-  }
-  if (write_x) st_f16<EPT>(c.x_out + e_swp, xn);
-  ss = wave_sum(ss);
-  if (lane == 0) wsum[wave] = ss;
-  __syncthreads();  // also: every read of xbuf above is done
-  QTIP_STAMP_SV(8)
-  float tot = 0.f;
-#pragma unroll
-  for (int w = 0; w < 16; ++w) tot += wsum[w];
-  const float rs = __builtin_amdgcn_rsqf(tot / (float)N + c.eps);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = (float)(_Float16)(r.wv[i] * (float)(_Float16)(v[i] * rs)) * r.sv[i];
-  // ---- second transform (swapped -> natural layout)
-  wht_regs<EPT>(v);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(v[i], 6, lane);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) xbuf[xidx<EPT>(e_swp + i)] = v[i];
-  __syncthreads();
-  QTIP_STAMP_SV(9)
-  // the bits still missing are the top four of the element's lane field = lane bits 2..5 here
-  _Float16 xo[EPT];
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) {
-    float y = xbuf[xidx<EPT>(e_nat + i)];
-    y = wht_lanes(y, 6, lane, 2);
-    xo[i] = (_Float16)(y * scale_in);
-  }
-  st_f16<EPT>(xs + e_nat, xo);
-  __syncthreads();  // the exchange buffer is free for the table, xs is complete
-  QTIP_STAMP_SV(10)
 }
 
 // Work unit = (32-row block rb, k split s).  The 16 waves of a workgroup take

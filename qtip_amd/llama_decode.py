@@ -257,7 +257,7 @@ class DecoderLayer(nn.Module):
             self._fused = {n: _FusedLinear(getattr(self, n)) for n in names}
         return self._fused
 
-    def decode_fused(self, x, k_cache, v_cache, pos, inv_freq, qkv_parts=None, next_layer=None):
+    def decode_fused(self, x, k_cache, v_cache, pos, inv_freq, qkv_parts=None, next_layer=None, open_end=False):
         """One new token, x (1, hidden) fp16, on the fused transforms: 12 launches for the fused
         layout (4 x [transform, matvec, transform] + attention, the attention kernel doing the qkv
         output transform itself), 24 for the separate projections.
@@ -266,11 +266,13 @@ class DecoderLayer(nn.Module):
         input inside the matvec (9 per layer); where it pays, that one launch is the following
         matvec itself (7 per layer): `qkv_parts` are then the partial sums of this layer's qkv matvec
         (launched by the previous layer with the layer boundary in its prologue) and `next_layer` the
-        layer whose qkv matvec this one launches.  Returns (x, qkv partial sums for the next layer)."""
+        layer whose qkv matvec this one launches.  Returns (x, qkv partial sums for the next layer).
+        open_end (no next layer): where down's output transform and the residual addition can be left to the caller, x is
+        the residual stream in front of them and the partial sums are down's."""
         cfg = self.cfg
         f = self._fused_linears()
         if self.grouped_ok():
-            return self._decode_grouped(x, k_cache, v_cache, pos, inv_freq, qkv_parts, next_layer)
+            return self._decode_grouped(x, k_cache, v_cache, pos, inv_freq, qkv_parts, next_layer, open_end)
         if self.grouped_plain_ok():
             return self._decode_grouped_plain(x, k_cache, v_cache, pos, inv_freq), None
         if self.fused:
@@ -308,6 +310,8 @@ class DecoderLayer(nn.Module):
         if nq is not None and not f['down'].dense and f['down'].can_chain_into(nq):
             parts = f['down'].matvec(f['down'].transform_in(ug, pre))
             return f['down'].chain_matvec(parts, x, nq, next_layer.input_norm.weight, cfg.eps)
+        if open_end and f['down'].can_end_open():
+            return x, f['down'].matvec(f['down'].transform_in(ug, pre))
         return f['down'](ug, pre, residual=x), None
 
     # ---- separate projections (the layout of the published checkpoints) in grouped launches
@@ -418,7 +422,7 @@ class DecoderLayer(nn.Module):
             [l.trellis for l in ls], [l.tlut for l in ls], [l.m for l in ls], ls[0].n, ls[0].K, prev_parts, post, scale,
             residual, norm_weight, self.cfg.eps, [l.SU for l in ls], (ls[0].n**-0.5) / 32.0)
 
-    def _decode_grouped(self, x, k_cache, v_cache, pos, inv_freq, qkv_parts, next_layer):
+    def _decode_grouped(self, x, k_cache, v_cache, pos, inv_freq, qkv_parts, next_layer, open_end=False):
         """decode_fused for separate projections, 8 launches: [boundary + q, k, v matvecs] (by the
         previous layer, or the first for itself), attention with the three output transforms in its prologue, o matvec with
         its input transform, [boundary + gate, up matvecs], both output transforms (with SiLU * up in
@@ -449,6 +453,8 @@ class DecoderLayer(nn.Module):
             parts, x = next_layer._group_chain(('q_proj', 'k_proj', 'v_proj'), pd, f['down'], x,
                                                next_layer.input_norm.weight)
             return x, parts
+        if open_end and f['down'].can_end_open():
+            return x, pd
         return f['down'].transform_out(pd, residual=x), None
 
 
@@ -604,6 +610,11 @@ class _FusedLinear:
         return (not self.dense and not nxt.dense and self.Kr == 1 and nxt.Kl == 1 and self.m == nxt.n
                 and self.m in (2048, 4096, 8192) and not self.shard_out and not nxt.shard_in)
 
+    def can_end_open(self):
+        """The token head can do this layer's output transform."""
+        return (not self.dense and not self.shard_out and self.Kr == 1 and self.m in ops.RHT_IN_MATVEC_SIZES
+                and self.SV.dtype == torch.float32 and self.SV.is_contiguous() and self.SV.data_ptr() % 16 == 0)
+
     def chain(self, parts, residual, nxt, norm_weight, eps):
         """(x_new, xt): transform_out(parts) + residual, then nxt.transform_in(RMSNorm(x_new))."""
         return ops.rht_chain(parts, self.SV, (self.m**-0.5) * 32.0, residual, norm_weight, eps, nxt.SU,
@@ -708,6 +719,16 @@ class LlamaDecoder(nn.Module):
             return False
         return True
 
+    def _head_launches(self, x):
+        """The last boundary, the norm and the output matrix of a token run as one launch (ops.token_head)."""
+        h, w = self.lm_head, self.norm.weight
+        return (len(self.layers) > 0 and x.shape == (1, self.cfg.hidden) and all(
+            type(t) in (torch.Tensor, nn.Parameter) and t.is_cuda and t.dtype == torch.float16 and t.device == x.device
+            and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (h, w, x))
+                and h.dim() == 2 and 0 < h.shape[0] < 2**30 and w.shape == h.shape[1:] == x.shape[1:] and h.shape[1] % 8 == 0
+                and h.shape[1] <= ops.TOKEN_HEAD_MAX and not (torch.is_grad_enabled() and h.requires_grad)
+                and ops.launchable(h, w, x))
+
     def decode_fused(self, tok, pos, float_logits=True):
         """tok (1,1) int64, pos (1,) int64 device tensors -> logits (1, 1, vocab), fused kernels;
         fp32 as the reference returns them, or the fp16 values the lm_head product yields
@@ -717,9 +738,18 @@ class LlamaDecoder(nn.Module):
                              f"(this model has {self.max_cache_len}); decode module by module")
         x = self.embed[tok.reshape(-1)]
         qp = None
+        head = self._head_launches(x)
         for i, layer in enumerate(self.layers):
             nxt = self.layers[i + 1] if i + 1 < len(self.layers) else None
-            x, qp = layer.decode_fused(x, self.k_cache[i], self.v_cache[i], pos, self.inv_freq, qp, nxt)
+            # (anyone's own last layer is not asked to leave its end open)
+            end = head and nxt is None and type(layer) is DecoderLayer and 'decode_fused' not in layer.__dict__
+            x, qp = layer.decode_fused(x, self.k_cache[i], self.v_cache[i], pos, self.inv_freq, qp, nxt,
+                                       **({'open_end': True} if end else {}))
+        if head and self._head_launches(x):
+            d, qp = (layer._fused_linears()['down'], qp) if end and qp is not None else (None, None)
+            return ops.token_head(self.lm_head, x, self.norm.weight, self.norm.eps, qp, None if d is None else d.SV,
+                                  0.0 if d is None else (d.m**-0.5) * 32.0,
+                                  torch.float32 if float_logits else torch.float16).reshape(1, 1, -1)
         x = ops.rmsnorm(x, self.norm.weight, self.norm.eps)
         lg = (x @ self.lm_head.T).reshape(1, 1, -1)
         return lg.float() if float_logits else lg

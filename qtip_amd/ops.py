@@ -778,6 +778,38 @@ def rotary_tables(positions, inv_freq):
     return cos, sin
 
 
+TOKEN_HEAD_MAX = 8192  # values of a row that the waves of token_head hold in flight
+
+
+def token_head(head, x, norm_weight, eps, parts=None, post=None, scale_out=0.0, out_dtype=torch.float16):
+    """fp16(head @ rmsnorm(y)) as out_dtype (fp16 or fp32), (vocab,), for one token: y = x, or behind the last layer's
+    projection y = fp16(x + fp16(post * scale_out * H(sum(parts)))).  head (vocab, n) fp16; parts (S, n) fp32, n in
+    RHT_IN_MATVEC_SIZES."""
+    require_cuda(head, "head", torch.float16)
+    require_cuda(x, "x", torch.float16)
+    require_cuda(norm_weight, "norm_weight", torch.float16)
+    if head.dim() != 2 or out_dtype not in _DT:
+        raise ValueError("head must be a matrix, out_dtype fp16 or fp32")
+    vocab, n = head.shape
+    if x.numel() != n or norm_weight.numel() != n or x.device != head.device or norm_weight.device != head.device:
+        raise ValueError(f"x and norm_weight must hold {n} values on {head.device}")
+    nparts, stride = 0, 0
+    if parts is not None:
+        require_cuda(parts, "parts", torch.float32)
+        require_cuda(post, "post", torch.float32)
+        parts = parts.reshape(parts.shape[0], -1)
+        nparts, stride = parts.shape[0], parts.stride(0)
+        if n not in RHT_IN_MATVEC_SIZES or parts.shape[1] != n or post.numel() != n or parts.device != head.device \
+                or post.device != head.device:
+            raise ValueError(f"parts and post must hold vectors of {n} values on {head.device}, n in {RHT_IN_MATVEC_SIZES}")
+    out = torch.empty((vocab,), dtype=out_dtype, device=head.device)
+    with _on(head.device):
+        check(lib().qtip_token_head(_ptr(out), _DT[out_dtype], _ptr(head), vocab, n, _ptr(x), _ptr(parts), nparts,
+                                    ctypes.c_size_t(stride), _ptr(post), float(scale_out), _ptr(norm_weight), float(eps),
+                                    stream_ptr(head.device)), "qtip_token_head")
+    return out
+
+
 def greedy_pick(logits, tok, pos, history=None, history_base=0):
     """tok[0] = argmax(logits) (fp16 logits of one position, first index among equal maxima),
     history[pos - history_base] = tok when that slot exists, pos += 1 - the per-token bookkeeping
