@@ -1,7 +1,13 @@
 // The boundary between two linear layers of a decoder in one workgroup of 1024 threads:
 //   x_new = residual + fp16(scale_out * post * H_k (sum of the previous layer's partial results)),
 //   x_t   = fp16(scale_in * H_k (su * RMSNorm(x_new) * norm_w))
-// for k = 1024 * EPT, shared by the matvec prologue (all of it) and the token head (x_new and its norm).
+// for k = 1024 * EPT, shared by the matvec prologue and the boundary's own launch (all of it) and the token head (x_new
+// and its norm).
+// Bound by latency: one cold round trip for the operands, three barriers, and between them some 70 vector instructions on
+// four waves a SIMD.  Nothing in it waits for the LDS crossbar (wht_place), no load waits for another, and no conversion
+// for a load.  us, a 2-bit launch of 12288 or 22016 rows of 4096 with the boundary in front, on average: 13.45 -> 12.33, past
+// the barrier behind its table after 5.8 -> 4.1; 57344 and 10240 rows of 8192 at 4 bits 51.9 -> 48.4 and
+// 21.2 -> 18.3.  A token of 8 layers of 4096 496 -> 473, of 4 layers of 8192 594 -> 584.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -28,163 +34,115 @@ struct ChainArgs {
   int in_parts;
 };
 
-struct ChainRegs {  // a thread's operands, k / 1024 <= 8 consecutive elements each
-  float v[8], pv[8], rv[8], wv[8], sv[8];
+template <int EPT>
+struct ChainRegs {  // a thread's operands, EPT consecutive elements each
+  typedef _Float16 hvec __attribute__((ext_vector_type(EPT)));
+  float v[EPT], v1[EPT];  // the first two partial results, where the first transform takes them
+  float pv[EPT];          // of the middle part
+  hvec rv, wv, sv;        // (as loaded: a conversion would wait for the load)
 };
 
-// Where the operands of the boundary's middle part are read.  It works in the swapped layout, in which
-// the lanes of a wave hold 16 runs of 4 * EPT consecutive elements: with eight elements a thread a
-// run is 64 bytes of fp16 and the operands are read there, with two or four it is half that or less
-// and a load touches four to eight times the cache lines it needs, so that they are read in the
-// natural layout and change over in LDS.  A token of 8 layers of 4096 (16 boundaries): 583 -> 565 us;
-// of layers of 8192, with the change-over in LDS or without, the same.
+// A thread holds EPT consecutive elements, those of thread index t (ten bits, e = t * EPT) of one of two layouts:
+//   natural   t = [wave 4 | place 6]
+//   swapped   t = [place 3..0 | wave 4 | place 5..4]
+// with place = wht_place(lane).  A transform does its register and place bits in one of them, changes over to the other
+// through LDS, and finds the bits that were the wave's among its places.  The boundary runs swapped -> natural -> swapped:
+// the partial results are read in runs of 4 * EPT floats, and the four operands of the middle part and the new residual
+// stream, which are fp16 but for one, whole cache lines at a time.  (The other way round they had to change over in LDS as well.)
 template <int EPT>
-constexpr bool kChainStaged = EPT < 8;
+__device__ __forceinline__ int nat_index(int place, int wave) {
+  return (wave * 64 + place) * EPT;
+}
+template <int EPT>
+__device__ __forceinline__ int swp_index(int place, int wave) {
+  return (((place & 15) << 6) | ((wave & 15) << 2) | (place >> 4)) * EPT;
+}
 
-// the operands but for the partial results past the first
-template <int EPT>
-__device__ __forceinline__ void chain_load_first(const ChainArgs& c, const _Float16* su, int tid, int lane,
-                                                 int wave, ChainRegs& r) {
+// All loads of the boundary but the partial results past the second, without a wait between them (SU: the sign vector too).
+template <int EPT, bool SU = true>
+__device__ __forceinline__ void chain_load(const ChainArgs& c, const _Float16* su, int place, int wave, ChainRegs<EPT>& r) {
   using namespace qtip_wht;
-  const int e_nat = tid * EPT;
-  const int e_mid = kChainStaged<EPT> ? e_nat : (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
-  ld_f32<EPT>(c.post + e_mid, r.pv);
-  ld_f16<EPT>(c.residual + e_mid, r.rv);
-  ld_f16<EPT>(c.norm_w + e_mid, r.wv);
-  ld_f16<EPT>(su + e_mid, r.sv);
-  ld_f32<EPT>(c.parts + e_nat, r.v);
+  const int e_nat = nat_index<EPT>(place, wave), e_swp = swp_index<EPT>(place, wave);
+  ld_f32<EPT>(c.parts + e_swp, r.v);
+  ld_f32<EPT>(c.parts + (c.in_parts > 1 ? c.part_stride : 0) + e_swp, r.v1);
+  ld_f32<EPT>(c.post + e_nat, r.pv);
+  typedef typename ChainRegs<EPT>::hvec hvec;
+  r.rv = *reinterpret_cast<const hvec*>(c.residual + e_nat);
+  r.wv = *reinterpret_cast<const hvec*>(c.norm_w + e_nat);
+  if constexpr (SU) r.sv = *reinterpret_cast<const hvec*>(su + e_nat);
 }
 
-// adds the partial results from `w` on
-template <int EPT>
-__device__ __forceinline__ void chain_load_parts(const ChainArgs& c, int w, int tid, ChainRegs& r) {
-  for (; w < c.in_parts; ++w) {
-    float t[EPT];
-    qtip_wht::ld_f32<EPT>(c.parts + w * c.part_stride + tid * EPT, t);
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) r.v[i] += t[i];
-  }
-}
+// floats of LDS: the exchange buffer and, behind it, the waves' sums
+constexpr int chain_floats(int k) { return k + k / 64 + kWaves; }
 
+// x_new in v (natural layout) and the reciprocal of its RMS.  xbuf: chain_floats(k) floats; the exchange buffer in
+// it is free again afterwards.
 template <int EPT>
-__device__ __forceinline__ void chain_load(const ChainArgs& c, const _Float16* su, int tid, int lane,
-                                           int wave, ChainRegs& r) {
-  chain_load_first<EPT>(c, su, tid, lane, wave, r);
-  chain_load_parts<EPT>(c, 1, tid, r);
-}
-
-// index of element e of an operand that changes over in LDS: a pad of four lanes per 64 puts the 16
-// runs of a read on banks of their own
-template <int EPT>
-__device__ __forceinline__ int sidx(int e) {
-  return e + 4 * EPT * (e / (64 * EPT));
-}
-// the floats of LDS behind xbuf and wsum that the operands take: one of fp32, three of fp16
-template <int EPT>
-constexpr int kChainStage = (kThreads + 64) * EPT * 5 / 2;
-
-// floats of LDS behind xbuf: k + k/64 of exchange buffer, the waves' sums, the operands that change over
-template <int EPT>
-constexpr int kChainFloats = kThreads * EPT + kThreads * EPT / 64 + kWaves + (kChainStaged<EPT> ? kChainStage<EPT> : 0);
-
-// x_new in v (swapped layout: element e_swp + i of thread tid) and the reciprocal of its RMS.  xbuf: k + k/64 floats of
-// exchange buffer, wsum behind it: 16 floats and kChainStage of operands; xbuf and the operands are free again, the sums
-// are not.  Leaves the norm weights (and the sign vector) of the layout in r.
-template <int EPT>
-__device__ __forceinline__ float chain_residual(ChainRegs& r, const ChainArgs& c, float* xbuf, float* wsum, float (&v)[EPT],
-                                                int tid, int lane, int wave, bool write_x, unsigned long long* sv = nullptr) {
+__device__ __forceinline__ float chain_residual(const ChainRegs<EPT>& r, const ChainArgs& c, float* xbuf, float (&v)[EPT], int lane, int place,
+                                                int wave, bool write_x, unsigned long long* sv = nullptr) {
   using namespace qtip_wht;
   constexpr int N = kThreads * EPT;
   (void)sv;
   QTIP_STAMP_SV(6)
-  const int e_nat = tid * EPT;
-  const int e_swp = (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
+  const int e_nat = nat_index<EPT>(place, wave), e_swp = swp_index<EPT>(place, wave);
+  float* wsum = xbuf + N + N / 64;
 #pragma unroll
   for (int i = 0; i < EPT; ++i) v[i] = r.v[i];
-  // ---- first transform (natural -> swapped layout)
-  wht_regs<EPT>(v);
+  if (c.in_parts > 1) {
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(v[i], 6, lane);
+    for (int i = 0; i < EPT; ++i) v[i] += r.v1[i];
+    for (int w = 2; w < c.in_parts; ++w) {
+      float t[EPT];
+      ld_f32<EPT>(c.parts + w * c.part_stride + e_swp, t);
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) xbuf[xidx<EPT>(e_nat + i)] = v[i];
-  float* post_s = wsum + kWaves;
-  _Float16* half_s = reinterpret_cast<_Float16*>(post_s + sidx<EPT>(N));  // residual, norm weight, sign vector
-  if constexpr (kChainStaged<EPT>) {
-    _Float16 h[EPT];
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) post_s[sidx<EPT>(e_nat) + i] = r.pv[i];
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) h[i] = (_Float16)r.rv[i];
-    st_f16<EPT>(half_s + sidx<EPT>(e_nat), h);
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) h[i] = (_Float16)r.wv[i];
-    st_f16<EPT>(half_s + sidx<EPT>(N) + sidx<EPT>(e_nat), h);
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) h[i] = (_Float16)r.sv[i];
-    st_f16<EPT>(half_s + 2 * sidx<EPT>(N) + sidx<EPT>(e_nat), h);
+      for (int i = 0; i < EPT; ++i) v[i] += t[i];
+    }
   }
+  // ---- first transform (swapped -> natural layout)
+  wht_regs<EPT>(v);
+  wht_places<EPT>(v, 6, place);
+  st_f32<EPT>(xbuf + xidx<EPT>(e_swp), v);
   __syncthreads();
   QTIP_STAMP_SV(7)
-  if constexpr (kChainStaged<EPT>) {
-    ld_f32<EPT>(post_s + sidx<EPT>(e_swp), r.pv);
-    ld_f16<EPT>(half_s + sidx<EPT>(e_swp), r.rv);
-    ld_f16<EPT>(half_s + sidx<EPT>(N) + sidx<EPT>(e_swp), r.wv);
-    ld_f16<EPT>(half_s + 2 * sidx<EPT>(N) + sidx<EPT>(e_swp), r.sv);
-  }
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(xbuf[xidx<EPT>(e_swp + i)], 4, lane);
-  // ---- residual, RMSNorm, sign vector of this layer
+  ld_f32<EPT>(xbuf + xidx<EPT>(e_nat), v);
+  wht_places<EPT>(v, 6, place, 2);
+  // ---- residual, RMSNorm
   float ss = 0.f;
   _Float16 xn[EPT];
 #pragma unroll
   for (int i = 0; i < EPT; ++i) {
     const float o = v[i] * c.scale_out * r.pv[i];
-    xn[i] = (_Float16)(r.rv[i] + (float)(_Float16)o);
+    xn[i] = (_Float16)((float)r.rv[i] + (float)(_Float16)o);
     v[i] = (float)xn[i];
     ss += v[i] * v[i];
   }
-  if (write_x) st_f16<EPT>(c.x_out + e_swp, xn);
+  if (write_x) st_f16<EPT>(c.x_out + e_nat, xn);
   ss = wave_sum(ss);
   if (lane == 0) wsum[wave] = ss;
   __syncthreads();  // also: every read of xbuf above is done
   QTIP_STAMP_SV(8)
-  float tot = 0.f;
-#pragma unroll
-  for (int w = 0; w < 16; ++w) tot += wsum[w];
-  return __builtin_amdgcn_rsqf(tot / (float)N + c.eps);
+  return __builtin_amdgcn_rsqf(waves16_sum(wsum, lane) / (float)N + c.eps);
 }
 
-// xbuf, wsum: as in chain_residual; xs: the k fp16 activations of the matvec
+// The whole boundary; x_t in the swapped layout, scaled and rounded, in xo.
 template <int EPT>
-__device__ __forceinline__ void chain_compute(ChainRegs& r, const ChainArgs& c, float scale_in, float* xbuf,
-                                              float* wsum, _Float16* xs, int tid, int lane, int wave,
-                                              bool write_x, unsigned long long* sv = nullptr) {
+__device__ __forceinline__ void chain_compute(const ChainRegs<EPT>& r, const ChainArgs& c, float scale_in, float* xbuf, _Float16 (&xo)[EPT],
+                                              int lane, int place, int wave, bool write_x, unsigned long long* sv = nullptr) {
   using namespace qtip_wht;
-  const int e_nat = tid * EPT;
-  const int e_swp = (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
   float v[EPT];
-  const float rs = chain_residual<EPT>(r, c, xbuf, wsum, v, tid, lane, wave, write_x, sv);
+  const float rs = chain_residual<EPT>(r, c, xbuf, v, lane, place, wave, write_x, sv);
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = (float)(_Float16)(r.wv[i] * (float)(_Float16)(v[i] * rs)) * r.sv[i];
-  // ---- second transform (swapped -> natural layout)
+  for (int i = 0; i < EPT; ++i) v[i] = (float)(_Float16)((float)r.wv[i] * (float)(_Float16)(v[i] * rs)) * (float)r.sv[i];
+  // ---- second transform (natural -> swapped layout)
   wht_regs<EPT>(v);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(v[i], 6, lane);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) xbuf[xidx<EPT>(e_swp + i)] = v[i];
+  wht_places<EPT>(v, 6, place);
+  st_f32<EPT>(xbuf + xidx<EPT>(nat_index<EPT>(place, wave)), v);
   __syncthreads();
   QTIP_STAMP_SV(9)
-  // the bits still missing are the top four of the element's lane field = lane bits 2..5 here
-  _Float16 xo[EPT];
+  ld_f32<EPT>(xbuf + xidx<EPT>(swp_index<EPT>(place, wave)), v);
+  wht_places<EPT>(v, 4, place);
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) {
-    float y = xbuf[xidx<EPT>(e_nat + i)];
-    y = wht_lanes(y, 6, lane, 2);
-    xo[i] = (_Float16)(y * scale_in);
-  }
-  st_f16<EPT>(xs + e_nat, xo);
-  __syncthreads();  // the exchange buffer is free for the table, xs is complete
-  QTIP_STAMP_SV(10)
+  for (int i = 0; i < EPT; ++i) xo[i] = (_Float16)(v[i] * scale_in);
 }
 
 }  // namespace qtip_chain

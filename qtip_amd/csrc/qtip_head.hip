@@ -29,7 +29,7 @@ constexpr int kMaxLoads = 16;  // 16-byte loads of a lane per matrix row: n <= 8
 template <int EPT, int NL, typename TOut>
 __global__ __launch_bounds__(kThreads, 1) void token_head_kernel(TOut* __restrict__ out, const _Float16* __restrict__ head,
                                                                  int vocab, int n, const ChainArgs c) {
-  __shared__ __align__(16) float smem[EPT ? kChainFloats<EPT ? EPT : 2> : kMaxLoads * 256 + kWaves];
+  __shared__ __align__(16) float smem[EPT ? chain_floats(kThreads * EPT) : kMaxLoads * 256 + kWaves];
   _Float16* xs = reinterpret_cast<_Float16*>(smem);  // n values, padded with zeros to whole loads
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -37,14 +37,12 @@ __global__ __launch_bounds__(kThreads, 1) void token_head_kernel(TOut* __restric
   int row = (int)blockIdx.x * kWaves + wave;
 
   // the operands of the norm first: a CU's requests return in order
-  ChainRegs r;
-  float* wsum = smem + (EPT ? n + (n >> 6) : kMaxLoads * 256);
+  const int place = qtip_wht::wht_place(lane);
   half8h px = {}, pw = {};
   constexpr int E = EPT ? EPT : 2;
-  float p1[E];  // the second of the partial results
+  ChainRegs<E> r;
   if constexpr (EPT != 0) {
-    chain_load_first<E>(c, c.norm_w, tid, lane, wave, r);  // (there is no sign vector here)
-    qtip_wht::ld_f32<E>(c.parts + (c.in_parts > 1 ? c.part_stride : 0) + tid * E, p1);
+    chain_load<E, false>(c, nullptr, place, wave, r);
   } else if (tid * 8 < n) {
     px = *reinterpret_cast<const half8h*>(c.residual + tid * 8);
     pw = *reinterpret_cast<const half8h*>(c.norm_w + tid * 8);
@@ -64,27 +62,21 @@ __global__ __launch_bounds__(kThreads, 1) void token_head_kernel(TOut* __restric
   }
 
   if constexpr (EPT != 0) {
-#pragma unroll
-    for (int i = 0; i < E; ++i) r.v[i] += c.in_parts > 1 ? p1[i] : 0.f;
-    chain_load_parts<E>(c, 2, tid, r);
-    const int e_swp = (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * E;
     float v[E];
-    const float rs = chain_residual<E>(r, c, smem, wsum, v, tid, lane, wave, false);
+    const float rs = chain_residual<E>(r, c, smem, v, lane, place, wave, false);
     _Float16 h[E];
 #pragma unroll
-    for (int i = 0; i < E; ++i) h[i] = (_Float16)(r.wv[i] * (float)(_Float16)(v[i] * rs));
-    qtip_wht::st_f16<E>(xs + e_swp, h);
+    for (int i = 0; i < E; ++i) h[i] = (_Float16)((float)r.wv[i] * (float)(_Float16)(v[i] * rs));
+    qtip_wht::st_f16<E>(xs + nat_index<E>(place, wave), h);
   } else {
     float ss = 0.f;
 #pragma unroll
     for (int q = 0; q < 8; ++q) ss += (float)px[q] * (float)px[q];
     ss = qtip_wht::wave_sum(ss);
+    float* wsum = smem + kMaxLoads * 256;
     if (lane == 0) wsum[wave] = ss;
     __syncthreads();
-    float tot = 0.f;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) tot += wsum[w];
-    const float rs = __builtin_amdgcn_rsqf(tot / (float)n + c.eps);
+    const float rs = __builtin_amdgcn_rsqf(qtip_wht::waves16_sum(wsum, lane) / (float)n + c.eps);
     half8h y;
 #pragma unroll
     for (int q = 0; q < 8; ++q) y[q] = (_Float16)((float)pw[q] * (float)(_Float16)((float)px[q] * rs));

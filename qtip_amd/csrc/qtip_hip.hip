@@ -155,37 +155,41 @@ __device__ __forceinline__ void load_x_buf(__amdgpu_buffer_rsrc_t rsrc, uint32_t
 // xs[e] = fp16(scale * (H_k (su * x))[e]) for the whole vector, written to LDS where the
 // kernel keeps its activations.  Every workgroup computes the whole transform (a few thousand
 // butterflies per thread, hidden behind the latency of the first weight loads) - it replaces
-// a separate transform launch.  `xchg` (k + k/64 floats) is the table's LDS, not yet built.
-// Element e = [wave 4][lane 6][i]: butterflies over the register bits, the six lane bits and,
-// after one exchange through LDS that swaps the wave bits with the low four lane bits, the rest.
+// a separate transform launch.  `xchg`: k + k/64 floats.
+// Natural to swapped layout (qtip_chain.h).
 template <int EPT>
-__device__ __forceinline__ void xform_prologue(const float v_in[8], float scale, float* xchg,
-                                               _Float16* xs, int tid, int lane, int wave) {
+__device__ __forceinline__ void xform_compute(float (&v)[EPT], float scale, float* xchg, _Float16 (&xo)[EPT], int place,
+                                              int wave) {
   using namespace qtip_wht;
-  float v[EPT];
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = v_in[i];
-  const int e_nat = tid * EPT;
-  const int e_swp = (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
   wht_regs<EPT>(v);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(v[i], 6, lane);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) xchg[xidx<EPT>(e_nat + i)] = v[i];
+  wht_places<EPT>(v, 6, place);
+  st_f32<EPT>(xchg + xidx<EPT>(nat_index<EPT>(place, wave)), v);
   __syncthreads();
-  _Float16 o[EPT];
+  ld_f32<EPT>(xchg + xidx<EPT>(swp_index<EPT>(place, wave)), v);
+  wht_places<EPT>(v, 4, place);
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) o[i] = (_Float16)(wht_lanes(xchg[xidx<EPT>(e_swp + i)], 4, lane) * scale);
-  st_f16<EPT>(xs + e_swp, o);
-  __syncthreads();  // xchg is free for the table, xs is complete
+  for (int i = 0; i < EPT; ++i) xo[i] = (_Float16)(v[i] * scale);
 }
+
+// Transformed activations lie in LDS with 16 bytes between wave-loads: a transform ends in the swapped layout, whose
+// sixteen lanes store 64 * EPT elements apart, on one bank without them.
+constexpr uint32_t kXsStride = 256 + 16;
+// LDS of a matvec with a transform in front: where the table leaves room (k <= 4096) the exchange buffer is beside it
+// and the table is written while the operands are on their way; at 8192 it lies under the table, whose first items
+// wait for it.
+constexpr uint32_t xform_lds_bytes(int k) { return (uint32_t)k / 128 * kXsStride; }
+constexpr bool xform_beside(int k) { return k <= 4096; }
+constexpr size_t xform_lds(int k) {
+  return kMatvecLds + xform_lds_bytes(k) + (xform_beside(k) ? chain_floats(k) * sizeof(float) : 0);
+}
+constexpr int kLateItems = 3;  // items of 16 KiB of the table that the exchange buffer of 8192 covers
+static_assert(xform_lds(4096) <= kMatvecLds + kMatvecXBytes && xform_lds(8192) <= kMatvecLds + kMatvecXBytes &&
+              chain_floats(8192) * sizeof(float) <= kLateItems * 16 * kThreads, "the transform's buffers fit");
 
 // XFORM == 2: the whole boundary between two linear layers of a decoder (qtip_chain.h) in front of the matvec, what
 // rht_chain_kernel does in a launch of its own.  Every workgroup recomputes the k-point boundary - a few microseconds of
 // work on 1024 threads, most of it while the first stream requests are in flight - and workgroup (0, 0) stores x_new for
 // the layers that follow.
-static_assert(sizeof(float) * kChainFloats<4> <= kLut128Bytes && sizeof(float) * kChainFloats<8> <= kLut128Bytes,
-              "the boundary's buffers fit the table's LDS");
 
 // Up to three matrices with the same k and bit width in one launch (the separate q / k / v or
 // gate / up projections of a decoder layer): the workgroups blockIdx.y in
@@ -225,9 +229,18 @@ __device__ unsigned long long g_stamps[kStampSlots][kStampWgs][kStampN];
 #define QTIP_STAMP_FIRST_LOAD()
 #define QTIP_STAMP_PTR nullptr
 #endif
+// (read and selected: left to itself the compiler selects an address and reads there, a round trip more)
+__device__ __forceinline__ int pick3(const int (&a)[3], int g) {
+  int x = a[0], y = a[1], z = a[2];
+  asm("" : "+s"(x), "+s"(y), "+s"(z));
+  return g == 0 ? x : (g == 1 ? y : z);
+}
 template <typename T>
-__device__ __forceinline__ T pick3(const T (&a)[3], int g) {
-  return g == 0 ? a[0] : (g == 1 ? a[1] : a[2]);
+__device__ __forceinline__ T* pick3(T* const (&a)[3], int g) {
+  uint64_t x = (uint64_t)a[0], y = (uint64_t)a[1], z = (uint64_t)a[2];
+  asm("" : "+s"(x), "+s"(y), "+s"(z));
+  // (device memory, which the statement above hides from the compiler)
+  return (T*)(__attribute__((address_space(1))) T*)(g == 0 ? x : (g == 1 ? y : z));
 }
 
 // Work unit = (32-row block rb, k split s).  The 16 waves of a workgroup take
@@ -250,6 +263,7 @@ __device__ __forceinline__ T pick3(const T (&a)[3], int g) {
 // (needs 256 bytes per wave-load of the range) and read from there.
 // XFORM: 0 = x is the matvec's fp16 input, 1 = x is the layer's raw input (input transform in the
 // prologue), 2 = the previous layer's partial results (whole layer boundary in the prologue).
+// EPT = k / 1024 with either, a kernel each: behind a switch over it the compiler waits for everything in flight.
 // XHALF: the k range needs up to twice the staging area and every workgroup has exactly one unit:
 // x is staged in two halves, the second replacing the first in the middle of the unit (two more
 // barriers per launch instead of x travelling through vector loads with every wave-load, which
@@ -260,13 +274,16 @@ __device__ __forceinline__ T pick3(const T (&a)[3], int g) {
 // whole stream but decodes half of its states (about 0.55 of a unit's time), and its rows are
 // complete sums, so nothing has to be combined across workgroups: 320 row blocks on 256
 // workgroups take 1.55 units of time instead of 2, 128 row blocks 0.55 instead of 1.
-template <int K, int DEPTH, bool XLDS, int XFORM = 0, bool XHALF = false, bool GROUP = false, bool HALF = false>
+template <int K, int DEPTH, bool XLDS, int XFORM = 0, bool XHALF = false, bool GROUP = false, bool HALF = false,
+          int EPT = 0>
 __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
     float* __restrict__ dst_, const uint8_t* __restrict__ packed_, const uint16_t* __restrict__ x_,
-    const uint32_t* __restrict__ tlut_, int m_, int k, int wl_per, int upw_q_, int upw_r_,
+    const uint32_t* __restrict__ tlut_, int m_, int k_, int wl_per, int upw_q_, int upw_r_,
     const uint16_t* __restrict__ su_ = nullptr, float xscale = 1.f, const ChainArgs chain = ChainArgs{},
     const GroupArgs grp = GroupArgs{}) {
   static_assert(!XFORM || XLDS, "the transformed activations live in LDS");
+  static_assert((XFORM != 0) == (EPT != 0), "a transform in front knows its size");
+  const int k = EPT ? 1024 * EPT : k_;
   static_assert(!GROUP || XFORM == 2 || (XFORM == 0 && XLDS && !XHALF),
                 "grouped launches exist for the layer-boundary form and the plain form with x in LDS");
   // the matrix this workgroup serves (uniform: scalar selects on kernel arguments)
@@ -366,18 +383,20 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
   uint32_t tw[4];  // item it*1024 + tid belongs to entry it*128 + tid/8; entries e and e+512 share a word
   // the wave's eight words of a pass come through the scalar cache (uniform address), which
   // keeps them out of the vector-memory queue that the stream requests fill
+  if constexpr (!XFORM) {
 #pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    const uint32_t* tp = tlut + it * 128 + wave * 8;
-    // one 32-byte scalar load (the table needs dword alignment only).  Loaded word by word, the
-    // compiler may fold the first select below into a per-lane load of tp[lane >> 3], and the wait
-    // for that vector load also waits for the stream loads requested before it.
-    typedef uint32_t u32x8_dw __attribute__((ext_vector_type(8), aligned(4)));
-    const u32x8_dw sw = *reinterpret_cast<const u32x8_dw*>(tp);
-    uint32_t v = sw[0];
+    for (int it = 0; it < 4; ++it) {
+      const uint32_t* tp = tlut + it * 128 + wave * 8;
+      // one 32-byte scalar load (the table needs dword alignment only).  Loaded word by word, the
+      // compiler may fold the first select below into a per-lane load of tp[lane >> 3], and the wait
+      // for that vector load also waits for the stream loads requested before it.
+      typedef uint32_t u32x8_dw __attribute__((ext_vector_type(8), aligned(4)));
+      const u32x8_dw sw = *reinterpret_cast<const u32x8_dw*>(tp);
+      uint32_t v = sw[0];
 #pragma unroll
-    for (int j = 1; j < 8; ++j) v = ((lane >> 3) == j) ? sw[j] : v;
-    tw[it] = v;
+      for (int j = 1; j < 8; ++j) v = ((lane >> 3) == j) ? sw[j] : v;
+      tw[it] = v;
+    }
   }
   QTIP_STAMP(1)
   u32x4 xstage[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
@@ -385,29 +404,7 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
   const int jh = XHALF ? (npw + 1) >> 1 : npw;  // items per wave served by the first staging
   // wave-loads of the first staging (all of the range unless XHALF)
   const int wlx = XHALF ? ((wl1 - wl0) < jh * kWaves ? (wl1 - wl0) : jh * kWaves) : (wl1 - wl0);
-  float xraw[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  ChainRegs cr;
-  if constexpr (XFORM == 2) {
-    const _Float16* sr = reinterpret_cast<const _Float16*>(su);
-    switch (k >> 10) {
-      case 2: chain_load<2>(chain, sr, tid, lane, wave, cr); break;
-      case 4: chain_load<4>(chain, sr, tid, lane, wave, cr); break;
-      default: chain_load<8>(chain, sr, tid, lane, wave, cr); break;
-    }
-  } else if constexpr (XFORM == 1) {
-    // the raw activations and the sign vector of the layer, k / 1024 consecutive elements per thread
-    using namespace qtip_wht;
-    float sv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const _Float16* xr = reinterpret_cast<const _Float16*>(x);
-    const _Float16* sr = reinterpret_cast<const _Float16*>(su);
-    switch (k >> 10) {
-      case 2: ld_f16<2>(xr + tid * 2, xraw); ld_f16<2>(sr + tid * 2, sv); break;
-      case 4: ld_f16<4>(xr + tid * 4, xraw); ld_f16<4>(sr + tid * 4, sv); break;
-      default: ld_f16<8>(xr + tid * 8, xraw); ld_f16<8>(sr + tid * 8, sv); break;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) xraw[i] *= sv[i];  // entries past k / 1024 are never read
-  } else if constexpr (XLDS) {
+  if constexpr (XLDS && !XFORM) {
     // x of wave-loads [wl0, wl0 + wlx): 16 bytes per thread and pass, at most 2 passes (28 KiB)
     const int xbytes = wlx * 256;
     const int kbytes = k * 2;
@@ -428,35 +425,59 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
       }
     }
   }
-#pragma unroll
-  for (int d = 0; d < FIRST; ++d) issue(d);
-
-  if constexpr (XFORM == 2) {
-    float* xbuf = reinterpret_cast<float*>(smem);
-    float* wsum = xbuf + k + (k >> 6);
-    _Float16* xs = reinterpret_cast<_Float16*>(xs_lds);
-    const bool write_x = blockIdx.x == 0 && blockIdx.y == 0;
-    switch (k >> 10) {
-      case 2: chain_compute<2>(cr, chain, xscale, xbuf, wsum, xs, tid, lane, wave, write_x, QTIP_STAMP_PTR); break;
-      case 4: chain_compute<4>(cr, chain, xscale, xbuf, wsum, xs, tid, lane, wave, write_x, QTIP_STAMP_PTR); break;
-      default: chain_compute<8>(cr, chain, xscale, xbuf, wsum, xs, tid, lane, wave, write_x, QTIP_STAMP_PTR); break;
-    }
-  } else if constexpr (XFORM == 1) {
-    QTIP_STAMP(6)
-    float* xchg = reinterpret_cast<float*>(smem);
-    _Float16* xs = reinterpret_cast<_Float16*>(xs_lds);
-    switch (k >> 10) {
-      case 2: xform_prologue<2>(xraw, xscale, xchg, xs, tid, lane, wave); break;
-      case 4: xform_prologue<4>(xraw, xscale, xchg, xs, tid, lane, wave); break;
-      default: xform_prologue<8>(xraw, xscale, xchg, xs, tid, lane, wave); break;
-    }
-    QTIP_STAMP(10)
-  }
-#pragma unroll
-  for (int it = 0; it < 8; ++it) {
+  auto table_item = [&](int it) {
     const uint32_t w = tw[it & 3] ^ ((uint32_t)(it >> 2) << 15);
     const u32x4 v = {w, w, w, w};
     reinterpret_cast<u32x4*>(lut)[it * kThreads + tid] = v;
+  };
+  if constexpr (XFORM) {
+    constexpr bool BESIDE = xform_beside(1024 * EPT);
+    const int place = qtip_wht::wht_place(lane);
+    // (vector loads: the scalar ones of the plain form are four round trips in a row where registers are short)
+#pragma unroll
+    for (int it = 0; it < 4; ++it) tw[it] = tlut[it * 128 + (tid >> 3)];
+    const _Float16* sr = reinterpret_cast<const _Float16*>(su);
+    float* xbuf = reinterpret_cast<float*>(BESIDE ? xs_lds + xform_lds_bytes(1024 * EPT) : smem);
+    _Float16 xo[EPT];
+    auto requested = [&] {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < FIRST; ++d) issue(d);
+#pragma unroll
+      for (int it = BESIDE ? 0 : kLateItems; it < 8; ++it) table_item(it);
+      __builtin_amdgcn_sched_barrier(0);  // (the table's writes wait for its words only)
+      QTIP_STAMP(6)
+    };
+    if constexpr (XFORM == 2) {
+      ChainRegs<EPT> cr;
+      chain_load<EPT>(chain, sr, place, wave, cr);
+      requested();
+      chain_compute<EPT>(cr, chain, xscale, xbuf, xo, lane, place, wave, blockIdx.x == 0 && blockIdx.y == 0, QTIP_STAMP_PTR);
+    } else {
+      // the raw activations and the sign vector of the layer
+      typedef _Float16 hvec __attribute__((ext_vector_type(EPT)));
+      const int e = nat_index<EPT>(place, wave);
+      const hvec xr = *reinterpret_cast<const hvec*>(reinterpret_cast<const _Float16*>(x) + e);
+      const hvec sv = *reinterpret_cast<const hvec*>(sr + e);
+      requested();
+      float v[EPT];
+#pragma unroll
+      for (int i = 0; i < EPT; ++i) v[i] = (float)xr[i] * (float)sv[i];
+      xform_compute<EPT>(v, xscale, xbuf, xo, place, wave);
+    }
+    const int e = swp_index<EPT>(place, wave);
+    qtip_wht::st_f16<EPT>(reinterpret_cast<_Float16*>(xs_lds) + e + 8 * (e >> 7), xo);
+    QTIP_STAMP(10)
+    if constexpr (!BESIDE) {
+      __syncthreads();  // the exchange buffer has been read
+#pragma unroll
+      for (int it = 0; it < kLateItems; ++it) table_item(it);
+    }
+  } else {
+#pragma unroll
+    for (int d = 0; d < FIRST; ++d) issue(d);
+#pragma unroll
+    for (int it = 0; it < 8; ++it) table_item(it);
   }
   if constexpr (XLDS && !XFORM) {
     const int xbytes = wlx * 256;
@@ -474,7 +495,8 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
   QTIP_STAMP_FIRST_LOAD()
 
   // wave-load w_first (the transformed vector is stored whole, a staged one from wl0 on)
-  const uint32_t xs_lane = lds_address(xs_lds) + xoff + (uint32_t)(XFORM ? w_first : wave) * 256u;
+  constexpr uint32_t xs_stride = XFORM ? kXsStride : 256u;
+  const uint32_t xs_lane = lds_address(xs_lds) + xoff + (uint32_t)(XFORM ? w_first : wave) * xs_stride;
 
   float4_t acc[4];  // [2*mh + rh]: rows 16*mh + 8*rh + a/2 of the unit's 32-row block
 #pragma unroll
@@ -507,7 +529,7 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
           if constexpr (XLDS) {
             typedef __attribute__((address_space(3))) const u32x2 lds_u32x2_t;
             u32x2 xv[4];
-            const uint32_t xa = xs_lane + (uint32_t)(c_j - c_jbase) * (kWaves * 256u);
+            const uint32_t xa = xs_lane + (uint32_t)(c_j - c_jbase) * (kWaves * xs_stride);
 #pragma unroll
             for (int q = 0; q < 4; ++q) xv[q] = *(lds_u32x2_t*)(uintptr_t)(xa + 16u * q);
             accumulate(buf[d], xv);
@@ -643,18 +665,17 @@ hipError_t allow_lds_all() {
   QTIP_ALLOW((matvec_kernel<2, 2, true, 0, false, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<3, 2, true, 0, false, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<4, 2, true, 0, false, true>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<2, 2, true, 2, false, true>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<3, 2, true, 2, false, true>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<4, 2, true, 2, false, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<2, 2, true, 0, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<3, 2, true, 0, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<4, 2, true, 0, true>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<2, 2, true, 1>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<3, 2, true, 1>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<4, 2, true, 1>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<2, 2, true, 2>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<3, 2, true, 2>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<4, 2, true, 2>), kMatvecLds + kMatvecXBytes)
+#define QTIP_ALLOW_XFORM(BITS, EPT)                                                                       \
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 1, false, false, false, EPT>), xform_lds(1024 * EPT))           \
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 2, false, false, false, EPT>), xform_lds(1024 * EPT))           \
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 2, false, true, false, EPT>), xform_lds(1024 * EPT))
+  QTIP_ALLOW_XFORM(2, 2) QTIP_ALLOW_XFORM(2, 4) QTIP_ALLOW_XFORM(2, 8)
+  QTIP_ALLOW_XFORM(3, 2) QTIP_ALLOW_XFORM(3, 4) QTIP_ALLOW_XFORM(3, 8)
+  QTIP_ALLOW_XFORM(4, 2) QTIP_ALLOW_XFORM(4, 4) QTIP_ALLOW_XFORM(4, 8)
+#undef QTIP_ALLOW_XFORM
 #undef QTIP_ALLOW
   return hipSuccess;
 }
@@ -829,6 +850,20 @@ size_t qtip_matvec_workspace_bytes(int m, int k, int bits) {
   return S > 1 ? (size_t)S * m * sizeof(float) : 0;
 }
 
+// the kernel with a transform in front for `bits` and k = 2048, 4096 or 8192, on grid g2 with lds bytes
+#define QTIP_XFORM(MODE, GROUP, ARGS)                                                       \
+  switch (16 * bits + (k >> 10)) {                                                          \
+    case 34: matvec_kernel<2, 2, true, MODE, false, GROUP, false, 2><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 36: matvec_kernel<2, 2, true, MODE, false, GROUP, false, 4><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 40: matvec_kernel<2, 2, true, MODE, false, GROUP, false, 8><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 50: matvec_kernel<3, 2, true, MODE, false, GROUP, false, 2><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 52: matvec_kernel<3, 2, true, MODE, false, GROUP, false, 4><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 56: matvec_kernel<3, 2, true, MODE, false, GROUP, false, 8><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 66: matvec_kernel<4, 2, true, MODE, false, GROUP, false, 2><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 68: matvec_kernel<4, 2, true, MODE, false, GROUP, false, 4><<<g2, kThreads, lds, st>>>ARGS; break; \
+    default: matvec_kernel<4, 2, true, MODE, false, GROUP, false, 8><<<g2, kThreads, lds, st>>>ARGS; break; \
+  }
+
 static int launch_matvec(const Ready& di, float* dst, const void* packed, const void* x_f16, const void* tlut,
                          int m, int k, int bits, int S, hipStream_t st, const void* su_f16 = nullptr,
                          float xscale = 1.f, const ChainArgs* chain = nullptr) {
@@ -845,21 +880,13 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
   const int uq = (m >> 5) / per_range, ur = (m >> 5) % per_range;
   if (su_f16) {
     // input transform inside the prologue: the whole transformed vector lives in LDS
-    const size_t lds = kMatvecLds + (size_t)k * 2;
+    const size_t lds = xform_lds(k);
     auto* sg = (const uint16_t*)su_f16;
     if (chain) {
-      switch (bits) {
-        case 2: matvec_kernel<2, 2, true, 2><<<g2, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale, *chain); break;
-        case 3: matvec_kernel<3, 2, true, 2><<<g2, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale, *chain); break;
-        default: matvec_kernel<4, 2, true, 2><<<g2, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale, *chain); break;
-      }
+      QTIP_XFORM(2, false, (dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale, *chain))
       return (int)hipGetLastError();
     }
-    switch (bits) {
-      case 2: matvec_kernel<2, 2, true, 1><<<g2, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale); break;
-      case 3: matvec_kernel<3, 2, true, 1><<<g2, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale); break;
-      default: matvec_kernel<4, 2, true, 1><<<g2, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale); break;
-    }
+    QTIP_XFORM(1, false, (dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale))
     return (int)hipGetLastError();
   }
   const size_t xbytes = (size_t)wl_per * 256;
@@ -1097,13 +1124,9 @@ int qtip_decompress_matvec_group_chain(float* parts, int ngroups, const void* co
   const int nwl = ((k >> 5) + 3) >> 2;
   const int wl_per = (nwl + S - 1) / S;
   const dim3 g2((unsigned)S, (unsigned)used);
-  const size_t lds = kMatvecLds + (size_t)k * 2;
+  const size_t lds = xform_lds(k);
   hipStream_t st = (hipStream_t)stream;
-  switch (bits) {
-    case 2: matvec_kernel<2, 2, true, 2, false, true><<<g2, kThreads, lds, st>>>(nullptr, nullptr, nullptr, nullptr, 0, k, wl_per, 0, 0, nullptr, scale_in, c, ga); break;
-    case 3: matvec_kernel<3, 2, true, 2, false, true><<<g2, kThreads, lds, st>>>(nullptr, nullptr, nullptr, nullptr, 0, k, wl_per, 0, 0, nullptr, scale_in, c, ga); break;
-    default: matvec_kernel<4, 2, true, 2, false, true><<<g2, kThreads, lds, st>>>(nullptr, nullptr, nullptr, nullptr, 0, k, wl_per, 0, 0, nullptr, scale_in, c, ga); break;
-  }
+  QTIP_XFORM(2, true, (nullptr, nullptr, nullptr, nullptr, 0, k, wl_per, 0, 0, nullptr, scale_in, c, ga))
   return (int)hipGetLastError();
 }
 

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "../../include/qtip_hip.h"
+#include "qtip_chain.h"
 #include "qtip_setup.h"
 #include "qtip_wht.h"
 
@@ -976,88 +977,30 @@ int launch_rht(RhtParams P, int out_dtype, int in_dtype, int rows, void* stream)
 // next linear layer (all four are separate launches otherwise, each with its own cold operands):
 //   x_new = fp16(residual + fp16(post * scale_out * H (sum of parts)))
 //   xt    = fp16(scale_in * H (pre * fp16(w * fp16(x_new * rsqrt(mean(x_new^2) + eps)))))
-// n = 1024 * EPT is a power of two (both transforms of order 1).  Element e = [wave 4][lane 6][i]
-// (i = log2 EPT register bits).  A transform runs its butterflies over the register bits, the six
-// lane bits, and - after one exchange through LDS that swaps the wave bits with the low four
-// lane bits - the remaining four bits.  The first transform leaves the data in the swapped
-// layout, which is as good as any for the element-wise middle part; the second transform swaps
-// back, so xt is stored in natural order.
+// n = 1024 * EPT is a power of two (both transforms of order 1); the steps are those of qtip_chain.h.
 template <int EPT>
 __global__ __launch_bounds__(kRhtThreads) void rht_chain_kernel(
     _Float16* __restrict__ xt_out, _Float16* __restrict__ x_out, const float* __restrict__ parts,
     int in_parts, size_t part_stride, const float* __restrict__ post, float scale_out,
     const _Float16* __restrict__ residual, const _Float16* __restrict__ norm_w, float eps,
     const _Float16* __restrict__ pre, float scale_in) {
+  using namespace qtip_chain;
   constexpr int N = kRhtThreads * EPT;
-  __shared__ __align__(16) float xbuf[N + N / 64];
-  __shared__ float wsum[16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  static_assert(kRhtThreads == kThreads, "one workgroup is a boundary");
+  __shared__ __align__(16) float xbuf[chain_floats(N)];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), place = wht_place(lane);
   const size_t row = blockIdx.x;
-  parts += row * N;
-  // natural layout: e = tid * EPT + i;  swapped layout: wave bits <-> low four lane bits
-  const int e_nat = tid * EPT;
-  const int e_swp = (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
-  // ---- operands of the middle part, in the swapped layout (issued first: they are cold)
-  float pv[EPT], rv[EPT], wv[EPT], sv[EPT];
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) pv[i] = sv[i] = 1.f;
-  if (post) ld_f32<EPT>(post + e_swp, pv);
-  ld_f16<EPT>(residual + row * N + e_swp, rv);
-  ld_f16<EPT>(norm_w + e_swp, wv);
-  if (pre) ld_f16<EPT>(pre + e_swp, sv);
-  // ---- first transform
-  float v[EPT];
-  ld_f32<EPT>(parts + e_nat, v);
-  for (int w = 1; w < in_parts; ++w) {
-    float t[EPT];
-    ld_f32<EPT>(parts + w * part_stride + e_nat, t);
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) v[i] += t[i];
-  }
-  wht_regs<EPT>(v);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(v[i], 6, lane);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) xbuf[xidx<EPT>(e_nat + i)] = v[i];
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(xbuf[xidx<EPT>(e_swp + i)], 4, lane);
-  // ---- residual, RMSNorm, sign vector of the next layer
-  float ss = 0.f;
-  _Float16 xn[EPT];
+  ChainRegs<EPT> r;
+  const ChainArgs c = {parts + row * N, post ? post : parts, residual + row * N, norm_w, x_out + row * N, part_stride, scale_out, eps, in_parts};
+  chain_load<EPT>(c, pre ? pre : norm_w, place, wave, r);
 #pragma unroll
   for (int i = 0; i < EPT; ++i) {
-    const float o = v[i] * scale_out * pv[i];
-    xn[i] = (_Float16)(rv[i] + (float)(_Float16)o);
-    v[i] = (float)xn[i];
-    ss += v[i] * v[i];
+    if (!post) r.pv[i] = 1.f;
+    if (!pre) r.sv[i] = (_Float16)1.f;
   }
-  st_f16<EPT>(x_out + row * N + e_swp, xn);
-  ss = wave_sum(ss);
-  if (lane == 0) wsum[wave] = ss;
-  __syncthreads();  // also: every read of xbuf above is done
-  float tot = 0.f;
-#pragma unroll
-  for (int w = 0; w < 16; ++w) tot += wsum[w];
-  const float rs = __builtin_amdgcn_rsqf(tot / (float)N + eps);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = (float)(_Float16)(wv[i] * (float)(_Float16)(v[i] * rs)) * sv[i];
-  // ---- second transform, from the swapped layout back to the natural one
-  wht_regs<EPT>(v);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(v[i], 6, lane);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) xbuf[xidx<EPT>(e_swp + i)] = v[i];
-  __syncthreads();
-  // the bits still missing are the top four of the element's lane field = lane bits 2..5 here
   _Float16 xo[EPT];
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) {
-    float y = xbuf[xidx<EPT>(e_nat + i)];
-    y = wht_lanes(y, 6, lane, 2);
-    xo[i] = (_Float16)(y * scale_in);
-  }
-  st_f16<EPT>(xt_out + row * N + e_nat, xo);
+  chain_compute<EPT>(r, c, scale_in, xbuf, xo, lane, place, wave, true);
+  st_f16<EPT>(xt_out + row * N + swp_index<EPT>(place, wave), xo);
 }
 
 }  // namespace

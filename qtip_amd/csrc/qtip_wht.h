@@ -56,10 +56,56 @@ __device__ __forceinline__ float wht_lanes(float v, int nbits, int lane, int lo 
   return v;
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
+// Transforms whose elements may sit in any lane keep element `place` of a wave in lane place ^ (3 if bit 2 of it is set).
+// A step over bit 2 of the place then exchanges lanes l and l ^ 7, a mirror of eight lanes that rides on the addition
+// as a DPP operand, and the one over bit 4 is a row swap: no step goes through the LDS crossbar, whose round trip (a wave
+// of a boundary waited for sixteen of them in a row) was most of a transform's time.  The additions are those of wht_lanes.
+__device__ __forceinline__ int wht_place(int lane) {
+  return lane ^ ((lane & 4) ? 3 : 0);
+}
+__device__ __forceinline__ float half_mirror(float v) {  // value of lane ^ 7
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float wht_place_stage(float v, int b, int place) {
+  const uint32_t flip = ((uint32_t)place << (31 - b)) & 0x80000000u;
+  const uint32_t u = __builtin_bit_cast(uint32_t, v), f = u ^ flip;
+  if (b >= 4) {
+    auto sw = b == 4 ? __builtin_amdgcn_permlane16_swap(u, f, false, false) : __builtin_amdgcn_permlane32_swap(u, f, false, false);
+    return __builtin_bit_cast(float, (uint32_t)sw[0]) + __builtin_bit_cast(float, (uint32_t)sw[1]);
+  }
+  return (b == 2 ? half_mirror(v) : lane_xor(v, b)) + __builtin_bit_cast(float, f);
+}
+// butterflies over place bits lo .. nbits-1 of EPT values
+template <int EPT>
+__device__ __forceinline__ void wht_places(float (&v)[EPT], int nbits, int place, int lo = 0) {
 #pragma unroll
-  for (int b = 0; b < 6; ++b) v += lane_xor(v, b);
-  return v;
+  for (int b = 0; b < 6; ++b)
+    if (b >= lo && b < nbits) {
+#pragma unroll
+      for (int i = 0; i < EPT; ++i) v[i] = wht_place_stage(v[i], b, place);
+    }
+}
+
+// the sum over the lanes of a wave (four lanes hold the same sum when eight are mirrored)
+__device__ __forceinline__ float wave_sum(float v) {
+  v += lane_xor(v, 0);
+  v += lane_xor(v, 1);
+  v += half_mirror(v);
+  v += lane_xor(v, 3);
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  auto s16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __builtin_bit_cast(float, (uint32_t)s16[0]) + __builtin_bit_cast(float, (uint32_t)s16[1]);
+  const uint32_t t = __builtin_bit_cast(uint32_t, v);
+  auto s32 = __builtin_amdgcn_permlane32_swap(t, t, false, false);
+  return __builtin_bit_cast(float, (uint32_t)s32[0]) + __builtin_bit_cast(float, (uint32_t)s32[1]);
+}
+// the sum of values that a workgroup's 16 waves left in LDS, the same in every lane
+__device__ __forceinline__ float waves16_sum(const float* w, int lane) {
+  float v = w[lane & 15];
+  v += lane_xor(v, 0);
+  v += lane_xor(v, 1);
+  v += half_mirror(v);
+  return v + lane_xor(v, 3);
 }
 
 // EPT consecutive elements as floats, with the widest loads the alignment (EPT elements) allows
@@ -76,6 +122,16 @@ __device__ __forceinline__ void ld_f32(const float* p, float v[EPT]) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[4 * q + e] = t[e];
     }
+  }
+}
+template <int EPT>
+__device__ __forceinline__ void st_f32(float* p, const float v[EPT]) {
+  if constexpr (EPT == 2) {
+    *reinterpret_cast<float2*>(p) = float2{v[0], v[1]};
+  } else {
+#pragma unroll
+    for (int q = 0; q < EPT / 4; ++q)
+      *reinterpret_cast<float4w*>(p + 4 * q) = float4w{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
   }
 }
 template <int EPT>
