@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define QTIP_ABI_VERSION 27 /* of this header; a library tells its own by qtip_abi_version() */
+#define QTIP_ABI_VERSION 28 /* of this header; a library tells its own by qtip_abi_version() */
 
 #define QTIP_OK 0
 #define QTIP_E_SHAPE (-1)     /* m % 32, k % 32, bits, batch or n out of range */
@@ -130,6 +130,16 @@ int qtip_decompress_matvec_parts(float* parts, const void* packed, const void* x
 int qtip_decompress_matvec_parts_rht(float* parts, const void* packed, const void* x_raw_f16,
                                      const void* su_f16, float scale, const void* tlut, int m, int k,
                                      int bits, int nparts, void* stream);
+
+/* qtip_decompress_matvec_parts_rht for k = order * 2^a, H_k = table (x) H_{2^a}.  Every workgroup makes the range of x_t that
+ * it reads.  With c = qtip_matvec_mix_columns(k, order, nparts), sign_rows holds k / c rows of 8 words: bit j of row i is set
+ * where entry (i, j) of table (x) H_{k / c / order} is -1, and 0 past the last column.  x_raw, su and sign_rows are 16-byte
+ * aligned.  c is 32 or 64, or 0 where the form does not apply (QTIP_E_SHAPE): k not a multiple of 128, 2^a below c, more
+ * than 256 rows, a range of k of more than 14336 elements. */
+int qtip_matvec_mix_columns(int k, int order, int nparts);
+int qtip_decompress_matvec_parts_mix(float* parts, const void* packed, const void* x_raw_f16, const void* su_f16, float scale,
+                                     const uint32_t* sign_rows, int order, const void* tlut, int m, int k, int bits, int nparts,
+                                     void* stream);
 
 /* qtip_decompress_matvec_parts with the whole boundary between two linear layers of a decoder
  * in front of it (k in {2048, 4096, 8192}):

@@ -19,6 +19,7 @@
 #define QTIP_STAMP_SV(i) if (wave == 0 && sv) sv[i] = __builtin_amdgcn_s_memrealtime();
 #endif
 #include "qtip_chain.h"
+#include "qtip_mix.h"
 
 using namespace qtip;
 using namespace qtip_chain;
@@ -183,6 +184,8 @@ constexpr size_t xform_lds(int k) {
   return kMatvecLds + xform_lds_bytes(k) + (xform_beside(k) ? chain_floats(k) * sizeof(float) : 0);
 }
 constexpr int kLateItems = 3;  // items of 16 KiB of the table that the exchange buffer of 8192 covers
+static_assert(qtip_mix::mix_in_lds(qtip_mix::kMixInMaxRows, 4).bytes <= kMatvecLds + kMatvecXBytes - 7 * 16 * kThreads &&
+              qtip_mix::mix_in_lds(qtip_mix::kMixInMaxRows, 4).bytes % 16 == 0, "a mix leaves the table but for its last item");
 static_assert(xform_lds(4096) <= kMatvecLds + kMatvecXBytes && xform_lds(8192) <= kMatvecLds + kMatvecXBytes &&
               chain_floats(8192) * sizeof(float) <= kLateItems * 16 * kThreads, "the transform's buffers fit");
 
@@ -263,7 +266,9 @@ __device__ __forceinline__ T* pick3(T* const (&a)[3], int g) {
 // (needs 256 bytes per wave-load of the range) and read from there.
 // XFORM: 0 = x is the matvec's fp16 input, 1 = x is the layer's raw input (input transform in the
 // prologue), 2 = the previous layer's partial results (whole layer boundary in the prologue).
-// EPT = k / 1024 with either, a kernel each: behind a switch over it the compiler waits for everything in flight.
+// 3 = as 1, for a table order times a power of two (qtip_mix.h); every workgroup makes the range of the vector that it reads
+// and x is staged as in the plain form.  EPT is a sixteenth of the columns there.
+// EPT = k / 1024 with 1 and 2, a kernel each: behind a switch over it the compiler waits for everything in flight.
 // XHALF: the k range needs up to twice the staging area and every workgroup has exactly one unit:
 // x is staged in two halves, the second replacing the first in the middle of the unit (two more
 // barriers per launch instead of x travelling through vector loads with every wave-load, which
@@ -280,10 +285,11 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
     float* __restrict__ dst_, const uint8_t* __restrict__ packed_, const uint16_t* __restrict__ x_,
     const uint32_t* __restrict__ tlut_, int m_, int k_, int wl_per, int upw_q_, int upw_r_,
     const uint16_t* __restrict__ su_ = nullptr, float xscale = 1.f, const ChainArgs chain = ChainArgs{},
-    const GroupArgs grp = GroupArgs{}) {
+    const GroupArgs grp = GroupArgs{}, const qtip_mix::MixArgs mix = qtip_mix::MixArgs{}) {
   static_assert(!XFORM || XLDS, "the transformed activations live in LDS");
   static_assert((XFORM != 0) == (EPT != 0), "a transform in front knows its size");
-  const int k = EPT ? 1024 * EPT : k_;
+  constexpr bool POW2 = XFORM == 1 || XFORM == 2;  // the whole transformed vector, in padded wave-loads
+  const int k = POW2 ? 1024 * EPT : k_;
   static_assert(!GROUP || XFORM == 2 || (XFORM == 0 && XLDS && !XHALF),
                 "grouped launches exist for the layer-boundary form and the plain form with x in LDS");
   // the matrix this workgroup serves (uniform: scalar selects on kernel arguments)
@@ -298,7 +304,7 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
   const int upw_q = GROUP ? pick3(grp.upw_q, gi) : upw_q_;
   const int upw_r = GROUP ? pick3(grp.upw_r, gi) : upw_r_;
   static_assert(!XHALF || (XLDS && !XFORM), "two-half staging is a form of the plain staged x");
-  static_assert(!HALF || (XLDS && !XFORM && !XHALF && !GROUP), "half units exist for the plain form with x in LDS");
+  static_assert(!HALF || (XLDS && !POW2 && !XHALF && !GROUP), "half units exist for the plain form with x in LDS and behind a mix");
   // wave-loads requested before the table is built.  With half units both: a half wave-load is
   // decoded in half the time, which no longer covers the latency of a load requested after the barrier.
   constexpr int FIRST = (DEPTH > 2 || HALF) ? 2 : 1;
@@ -430,7 +436,30 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
     const u32x4 v = {w, w, w, w};
     reinterpret_cast<u32x4*>(lut)[it * kThreads + tid] = v;
   };
-  if constexpr (XFORM) {
+  if constexpr (XFORM == 3) {
+#pragma unroll
+    for (int it = 0; it < 4; ++it) tw[it] = tlut[it * 128 + (tid >> 3)];
+    const int row0 = wl0 * (8 / EPT), row1 = wl1 * (8 / EPT);  // of the range
+    qtip_mix::MixInRegs<EPT> r;
+    const _Float16* xr = reinterpret_cast<const _Float16*>(x);
+    const _Float16* sr = reinterpret_cast<const _Float16*>(su);
+    qtip_mix::mix_in_load<EPT>(r, mix, xr, sr, row0, tid);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 0; d < FIRST; ++d) issue(d);
+    // The transform's buffers end where the LDS does: on the staging area and the waves' sums, which are free, and, from 224
+    // rows of 64 on, a part of the table's last item, which is written behind the transform then.
+    const int buffers = (int)(kMatvecLds + kMatvecXBytes) - qtip_mix::mix_in_lds(mix.on, EPT).bytes;
+    const bool all = buffers >= 8 * 16 * kThreads;
+#pragma unroll
+    for (int it = 0; it < 7; ++it) table_item(it);
+    if (all) table_item(7);
+    __builtin_amdgcn_sched_barrier(0);
+    qtip_mix::mix_in_compute<EPT>(r, mix, xscale, smem + buffers, reinterpret_cast<_Float16*>(xs_lds), xr, sr, row0, row1, tid,
+                                  QTIP_STAMP_PTR);
+    QTIP_STAMP(10)
+    if (!all) table_item(7);
+  } else if constexpr (XFORM) {
     constexpr bool BESIDE = xform_beside(1024 * EPT);
     const int place = qtip_wht::wht_place(lane);
     // (vector loads: the scalar ones of the plain form are four round trips in a row where registers are short)
@@ -495,8 +524,8 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
   QTIP_STAMP_FIRST_LOAD()
 
   // wave-load w_first (the transformed vector is stored whole, a staged one from wl0 on)
-  constexpr uint32_t xs_stride = XFORM ? kXsStride : 256u;
-  const uint32_t xs_lane = lds_address(xs_lds) + xoff + (uint32_t)(XFORM ? w_first : wave) * xs_stride;
+  constexpr uint32_t xs_stride = POW2 ? kXsStride : 256u;
+  const uint32_t xs_lane = lds_address(xs_lds) + xoff + (uint32_t)(POW2 ? w_first : wave) * xs_stride;
 
   float4_t acc[4];  // [2*mh + rh]: rows 16*mh + 8*rh + a/2 of the unit's 32-row block
 #pragma unroll
@@ -676,6 +705,11 @@ hipError_t allow_lds_all() {
   QTIP_ALLOW_XFORM(3, 2) QTIP_ALLOW_XFORM(3, 4) QTIP_ALLOW_XFORM(3, 8)
   QTIP_ALLOW_XFORM(4, 2) QTIP_ALLOW_XFORM(4, 4) QTIP_ALLOW_XFORM(4, 8)
 #undef QTIP_ALLOW_XFORM
+#define QTIP_ALLOW_MIX(BITS, HALF)                                                                         \
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 3, false, false, HALF, 2>), kMatvecLds + kMatvecXBytes)         \
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 3, false, false, HALF, 4>), kMatvecLds + kMatvecXBytes)
+  QTIP_ALLOW_MIX(2, false) QTIP_ALLOW_MIX(2, true) QTIP_ALLOW_MIX(3, false) QTIP_ALLOW_MIX(4, false)
+#undef QTIP_ALLOW_MIX
 #undef QTIP_ALLOW
   return hipSuccess;
 }
@@ -866,7 +900,7 @@ size_t qtip_matvec_workspace_bytes(int m, int k, int bits) {
 
 static int launch_matvec(const Ready& di, float* dst, const void* packed, const void* x_f16, const void* tlut,
                          int m, int k, int bits, int S, hipStream_t st, const void* su_f16 = nullptr,
-                         float xscale = 1.f, const ChainArgs* chain = nullptr) {
+                         float xscale = 1.f, const ChainArgs* chain = nullptr, const qtip_mix::MixArgs* mix = nullptr) {
   const long units = (long)(m >> 5) * S;
   long grid = units < di.cus ? units : di.cus;
   grid -= grid % S;  // a workgroup keeps one k range (units is a multiple of S, so grid >= S)
@@ -878,7 +912,7 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
   const int per_range = (int)(grid / S);  // workgroups per k range, each walks row blocks rb0, rb0 + per_range, ...
   const dim3 g2((unsigned)S, (unsigned)per_range);
   const int uq = (m >> 5) / per_range, ur = (m >> 5) % per_range;
-  if (su_f16) {
+  if (su_f16 && !mix) {
     // input transform inside the prologue: the whole transformed vector lives in LDS
     const size_t lds = xform_lds(k);
     auto* sg = (const uint16_t*)su_f16;
@@ -902,6 +936,30 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
   const int left = full_range > 0 ? (m >> 5) % full_range : 0;
   const int whole = full_range > 0 ? (m >> 5) / full_range : 0;
   const bool even_items = (((wl_per + kWaves - 1) / kWaves) & 1) == 0;
+  if (mix) {
+    const int cols = k / mix->on;
+    const size_t lds = kMatvecLds + kMatvecXBytes;
+    auto* sg = (const uint16_t*)su_f16;
+    const bool half = bits == 2 && left > 0 && 2 * left <= full_range && (whole == 0 || even_items);
+    const dim3 gh = half ? dim3((unsigned)S, (unsigned)(whole > 0 ? full_range : 2 * left)) : g2;
+    const int q = half ? whole : uq, r = half ? 2 * left : ur;
+#define QTIP_MIX(BITS, HALF)                                                                                                     \
+  if (cols == 64) matvec_kernel<BITS, 2, true, 3, false, false, HALF, 4><<<gh, kThreads, lds, st>>>(                            \
+      dst, p, xx, t, m, k, wl_per, q, r, sg, xscale, ChainArgs{}, GroupArgs{}, *mix);                                            \
+  else matvec_kernel<BITS, 2, true, 3, false, false, HALF, 2><<<gh, kThreads, lds, st>>>(                                        \
+      dst, p, xx, t, m, k, wl_per, q, r, sg, xscale, ChainArgs{}, GroupArgs{}, *mix)
+    if (half) {
+      QTIP_MIX(2, true);
+    } else {
+      switch (bits) {
+        case 2: QTIP_MIX(2, false); break;
+        case 3: QTIP_MIX(3, false); break;
+        default: QTIP_MIX(4, false); break;
+      }
+    }
+#undef QTIP_MIX
+    return (int)hipGetLastError();
+  }
   if (bits == 2 && xbytes <= kMatvecXBytes && left > 0 && 2 * left <= full_range && (whole == 0 || even_items)) {
     const dim3 gh((unsigned)S, (unsigned)(whole > 0 ? full_range : 2 * left));
     matvec_kernel<2, 2, true, 0, false, false, true><<<gh, kThreads, kMatvecLds + xbytes, st>>>(
@@ -931,6 +989,18 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
     }
   }
   return (int)hipGetLastError();
+}
+
+// Columns (32 or 64) of a transform of k elements in front of a matvec cut in S ranges of k, or 0: at most 256 rows (few columns
+// are many rows, which more waves share), whole wave-loads in every range and a range that fits the staging area.  With
+// 128 columns, for k up to 32768, the launch is slower than its two: one wave a tile goes through eight values of four rows.  us from cold
+// memory at 2 bits, two launches / one with 128 columns: 5120 x 5120 9.0 / 10.5, 14336 -> 4096 10.5 / 12.1, 28672 -> 8192 23.6 / 25.9.
+static int matvec_mix_cols(int k, int order, int S) {
+  if (order < 1 || k < 128 || (k & 127) || k % order || S < 1 || S > kMaxSplit || S > (k >> 7)) return 0;
+  const int p2 = k / order;
+  if ((p2 & (p2 - 1)) || p2 < 32 || (size_t)(((k >> 7) + S - 1) / S) * 256 > kMatvecXBytes) return 0;
+  if (k / 32 <= qtip_mix::kMixInMaxRows) return 32;
+  return p2 >= 64 && k / 64 <= qtip_mix::kMixInMaxRows ? 64 : 0;
 }
 
 static int check_matvec(const void* out, const void* packed, const void* x_f16, const void* tlut,
@@ -976,6 +1046,23 @@ int qtip_decompress_matvec_parts_rht(float* parts, const void* packed, const voi
   const Ready rd = ready(stream);
   if (rd.rc) return rd.rc;
   return launch_matvec(rd, parts, packed, x_raw_f16, tlut, m, k, bits, nparts, (hipStream_t)stream, su_f16, scale);
+}
+
+int qtip_matvec_mix_columns(int k, int order, int nparts) { return matvec_mix_cols(k, order, nparts); }
+
+int qtip_decompress_matvec_parts_mix(float* parts, const void* packed, const void* x_raw_f16, const void* su_f16, float scale,
+                                     const uint32_t* sign_rows, int order, const void* tlut, int m, int k, int bits, int nparts,
+                                     void* stream) {
+  int rc = check_matvec(parts, packed, x_raw_f16, tlut, m, k, bits);
+  if (rc) return rc;
+  if (!su_f16 || !sign_rows) return QTIP_E_NULL;
+  const int cols = matvec_mix_cols(k, order, nparts);
+  if (!cols) return QTIP_E_SHAPE;
+  if (!aligned16(x_raw_f16) || !aligned16(su_f16) || !aligned16(sign_rows)) return QTIP_E_ALIGN;
+  const qtip_mix::MixArgs mix = {sign_rows, k / cols};
+  const Ready rd = ready(stream);
+  if (rd.rc) return rd.rc;
+  return launch_matvec(rd, parts, packed, x_raw_f16, tlut, m, k, bits, nparts, (hipStream_t)stream, su_f16, scale, nullptr, &mix);
 }
 
 int qtip_decompress_matvec_parts_chain(float* parts, const void* packed, const void* tlut, int m, int k,

@@ -5,6 +5,7 @@
 
 #include "../../include/qtip_hip.h"
 #include "qtip_chain.h"
+#include "qtip_mix.h"
 #include "qtip_setup.h"
 #include "qtip_wht.h"
 

@@ -31,11 +31,11 @@
 // fp32 rows: 28672, 1000 rows 811 -> 82; 11008, 2048 rows ~240 -> 64.  Few rows: the workgroups of a pass share its
 // output rows (launch_mix), each with all of the plane.
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half8m __attribute__((ext_vector_type(8)));
-typedef _Float16 half2m __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4m __attribute__((ext_vector_type(4)));
-
+using qtip_mix::bf16x8;
+using qtip_mix::half8m;
+using qtip_mix::u32x4m;
+using qtip_mix::expand_signs;
+using qtip_mix::mix_signs;
 constexpr int kMixCols = 128;
 constexpr int kMixMaxKT = 8;
 constexpr int kMixMaxOrder = 32 * kMixMaxKT;  // table orders, built in or a caller's own
@@ -52,15 +52,6 @@ constexpr uint32_t mix_stride(int ktc) { return 64 * ktc + 16; }  // bytes per c
 constexpr size_t mix_lds(int ktc, int order) {
   return (size_t)kMixCols * mix_stride(ktc) + (((size_t)order * order + 31) / 32 * 4 + 15) / 16 * 16 +
          32 * kMixMaxKT * sizeof(float) + 16;
-}
-
-// eight +-1 values (`one` = twice the 16-bit pattern of 1) from the bits of a byte (1 = -1)
-__device__ __forceinline__ u32x4m expand_signs(uint32_t b, uint32_t one) {
-  const uint32_t u = b | (b << 15);
-  u32x4m r;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) r[q] = ((u << (15 - 2 * q)) & 0x80008000u) | one;
-  return r;
 }
 
 template <typename TIn, typename TOut, int MODE, int KTC>
@@ -177,65 +168,8 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   if (tid < 2) flag[tid] = 0;
   __syncthreads();
   // ---- signs of output row 16 * wave + a against v rows 32 * kt + 8 * g + e: byte kt of sb, bit e
-  // (the lookups of all k tiles are issued together: a wait per lookup costs more than the transform)
   uint32_t sb0 = 0, sb1 = 0;
-  if (!idle) {
-    uint32_t sb[2] = {0u, 0u};
-    // H_A: within eight rows a pattern of iA's low bits (the rows differ in theirs), and for A > 8 a
-    // sign per eight rows
-    const int i = 16 * wave + a, iA = i & Am;
-    const uint32_t pat = ((iA & 1) ? 0xAAu : 0u) ^ ((iA & 2) ? 0xCCu : 0u) ^ ((iA & 4) ? 0xF0u : 0u);
-    uint32_t f[KTC];
-    if (logA2 >= 3) {  // one table column
-      const int iK = (i < on ? i : 0) >> logA2;
-#pragma unroll
-      for (int kt = 0; kt < KTC; ++kt) {
-        const int q = ((32 * kt + 8 * g) >> logA2) * order + iK;
-        f[kt] = hb[q >> 5 < nw ? q >> 5 : 0] >> (q & 31);
-      }
-#pragma unroll
-      for (int kt = 0; kt < KTC; ++kt) {
-        const uint32_t b = f[kt] ^ (uint32_t)__builtin_popcount(iA & (32 * kt + 8 * g) & Am);
-        sb[kt >> 2] |= ((0u - (b & 1u)) & 0xFFu) << (8 * (kt & 3));
-      }
-    } else {
-      // lane e = a % 8 takes the bits of the eight output rows of its half of the wave against v row
-      // 32 * kt + 8 * g + e, adjacent in the table's words, and the eight lanes transpose their bytes
-      const int iK = (16 * wave + (a & 8)) >> logA2;
-      uint32_t hi[KTC], sh[KTC];
-#pragma unroll
-      for (int kt = 0; kt < KTC; ++kt) {
-        const int q = ((32 * kt + 8 * g + (a & 7)) >> logA2) * order + iK, w = q >> 5;
-        f[kt] = hb[w < nw ? w : 0];  // (rows past the table meet zeros of v, or are not stored)
-        hi[kt] = hb[w + 1 < nw ? w + 1 : 0];
-        sh[kt] = q & 31;
-      }
-#pragma unroll
-      for (int kt = 0; kt < KTC; ++kt) {
-        uint32_t x = __builtin_amdgcn_alignbit(hi[kt], f[kt], sh[kt]);
-        if (logA2 == 0) x &= 0xFFu;
-        else if (logA2 == 1) {  // four bits, each for two rows
-          x = (x & 3u) | ((x & 0xCu) << 2);
-          x = (x & 0x11u) | ((x & 0x22u) << 1);
-          x *= 3u;
-        } else x = (x & 1u) * 0x0Fu | (x & 2u) * 0x78u;  // two bits, each for four rows
-        sb[kt >> 2] |= x << (8 * (kt & 3));
-      }
-#pragma unroll
-      for (int h = 0; h < (KTC > 4 ? 2 : 1); ++h) {
-        auto step = [&](int b, uint32_t m) {  // the off-diagonal quarters change places
-          const int s = 1 << b;
-          const uint32_t o = __builtin_bit_cast(uint32_t, lane_xor(__builtin_bit_cast(float, sb[h]), b));
-          sb[h] = (a & s) ? (sb[h] & ~m) | ((o >> s) & m) : (sb[h] & m) | ((o & m) << s);
-        };
-        step(2, 0x0F0F0F0Fu);
-        step(1, 0x33333333u);
-        step(0, 0x55555555u);
-      }
-    }
-    sb0 = sb[0] ^ pat * 0x01010101u;
-    sb1 = sb[1] ^ pat * 0x01010101u;
-  }
+  if (!idle) mix_signs<KTC>(sb0, sb1, hb, order, logA2, 16 * wave, on, lane);
   auto signs = [&](int kt, uint32_t one) {
     return expand_signs(((KTC > 4 && (kt & 4) ? sb1 : sb0) >> (8 * (kt & 3))) & 0xFFu, one);
   };

@@ -24,7 +24,7 @@ import torch.nn.functional as F
 
 from . import ops
 from .linear.quantized_linear import QuantizedLinear
-from .utils.matmul_had import had_bits
+from .utils.matmul_had import had_bits, sign_rows
 
 
 class LlamaConfig:
@@ -266,7 +266,8 @@ class DecoderLayer(nn.Module):
         input inside the matvec (9 per layer); where it pays, that one launch is the following
         matvec itself (7 per layer): `qkv_parts` are then the partial sums of this layer's qkv matvec
         (launched by the previous layer with the layer boundary in its prologue) and `next_layer` the
-        layer whose qkv matvec this one launches.  Returns (x, qkv partial sums for the next layer).
+        layer whose qkv matvec this one launches.  A table transform in front of down (ops.matvec_mix_columns) is inside down's
+        matvec, a launch less.  Returns (x, qkv partial sums for the next layer).
         open_end (no next layer): where down's output transform and the residual addition can be left to the caller, x is
         the residual stream in front of them and the partial sums are down's."""
         cfg = self.cfg
@@ -308,10 +309,10 @@ class DecoderLayer(nn.Module):
         pre = ops.PRE_SILU_MUL if ug.shape[-1] == 2 * cfg.ffn else ops.PRE_NONE
         nq = next_layer._fused_linears().get('qkv') if (next_layer is not None and next_layer.fused) else None
         if nq is not None and not f['down'].dense and f['down'].can_chain_into(nq):
-            parts = f['down'].matvec(f['down'].transform_in(ug, pre))
+            parts = f['down'].matvec_behind(ug, pre)
             return f['down'].chain_matvec(parts, x, nq, next_layer.input_norm.weight, cfg.eps)
         if open_end and f['down'].can_end_open():
-            return x, f['down'].matvec(f['down'].transform_in(ug, pre))
+            return x, f['down'].matvec_behind(ug, pre)
         return f['down'](ug, pre, residual=x), None
 
     # ---- separate projections (the layout of the published checkpoints) in grouped launches
@@ -448,7 +449,7 @@ class DecoderLayer(nn.Module):
         po = f['o'].matvec_from(attn.reshape(1, -1))
         gu_parts, x = self._group_chain(('gate_proj', 'up_proj'), po, f['o'], x, self.post_norm.weight)
         h, pre = self._gate_up_out(gu_parts)
-        pd = f['down'].matvec(f['down'].transform_in(h, pre))
+        pd = f['down'].matvec_behind(h, pre)
         if next_layer is not None and next_layer.grouped_ok():
             parts, x = next_layer._group_chain(('q_proj', 'k_proj', 'v_proj'), pd, f['down'], x,
                                                next_layer.input_norm.weight)
@@ -538,6 +539,11 @@ class _FusedLinear:
         self.Kl, self.Kr = lin.K_left, lin.K_right
         self.bl = had_bits(lin.had_left, self.Kl, True, dev) if self.Kl > 1 else None
         self.br = had_bits(lin.had_right, self.Kr, False, dev) if self.Kr > 1 else None
+        # the table of an input transform that runs in front of the matvec, in its launch
+        cols = 0
+        if dev.type == "cuda" and not self.shard_in:
+            cols = ops.matvec_mix_columns(self.n, self.Kl, ops.matvec_split(self.m, self.n, self.K, dev))
+        self.mix_rows = sign_rows(self.bl, self.Kl, self.n // cols // self.Kl, dev) if cols else None
 
     def _dense(self, x, pre_mode, norm_weight, eps, residual):
         if pre_mode == ops.PRE_RMSNORM:
@@ -568,13 +574,21 @@ class _FusedLinear:
         return ops.decompress_matvec_parts(self.trellis, xt.reshape(-1), self.tlut, self.m, self.n, self.K).unsqueeze(1)
 
     def matvec_from(self, x):
-        """matvec(transform_in(x)) for a plain input; one launch when the transform is a power of
-        two the matvec kernel computes in its prologue."""
+        """matvec(transform_in(x)) for a plain input; one launch where the matvec kernel computes the transform in its
+        prologue."""
         if (self.Kl == 1 and self.n in ops.RHT_IN_MATVEC_SIZES and x.dtype == torch.float16
                 and self.SU.dtype == torch.float16 and not self.shard_in):
             return ops.decompress_matvec_parts_rht(self.trellis, x.reshape(-1), self.SU, (self.n**-0.5) / 32.0,
                                                    self.tlut, self.m, self.n, self.K).unsqueeze(1)
+        if (self.mix_rows is not None and x.dtype == self.SU.dtype == torch.float16 and self.SU.is_contiguous()
+                and x.data_ptr() % 16 == self.SU.data_ptr() % 16 == 0):
+            return ops.decompress_matvec_parts_mix(self.trellis, x.reshape(-1), self.SU, (self.n**-0.5) / 32.0, self.mix_rows,
+                                                   self.Kl, self.tlut, self.m, self.n, self.K).unsqueeze(1)
         return self.matvec(self.transform_in(x))
+
+    def matvec_behind(self, x, pre_mode):
+        """matvec(transform_in(x, pre_mode))"""
+        return self.matvec_from(x) if pre_mode == ops.PRE_NONE else self.matvec(self.transform_in(x, pre_mode))
 
     def transform_out(self, parts, residual=None):
         if self.shard_out:

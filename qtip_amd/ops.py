@@ -203,6 +203,36 @@ def decompress_matvec_parts_rht(packed, x_raw, su, scale, tlut, m, k, bits, npar
     return parts
 
 
+def decompress_matvec_parts_mix(packed, x_raw, su, scale, sign_rows, order, tlut, m, k, bits, nparts=None):
+    """decompress_matvec_parts_rht for k = order * 2^a where matvec_mix_columns(k, order, nparts) is not 0; sign_rows as
+    utils.matmul_had.sign_rows makes them for that many columns."""
+    _check_packed(packed, m, k, bits)
+    _check_tlut(tlut, packed.device)
+    require_cuda(x_raw, "x", torch.float16)
+    require_cuda(su, "su", torch.float16)
+    require_cuda(sign_rows, "sign_rows", torch.int32)
+    S = int(nparts) if nparts is not None else matvec_split(m, k, bits, packed.device)
+    cols = matvec_mix_columns(k, order, S)
+    if x_raw.numel() != k or su.numel() != k:
+        raise ValueError(f"x and su must hold k = {k} fp16 values")
+    if not cols or sign_rows.numel() != k // cols * 8:
+        raise ValueError(f"no transform of {k} = {order} * 2^a elements with such a table in front of {S} ranges")
+    if any(t.device != packed.device for t in (x_raw, su, sign_rows)):
+        raise ValueError(f"x, su and sign_rows must be on {packed.device}")
+    parts = torch.empty((S, m), dtype=torch.float32, device=packed.device)
+    with _on(packed.device):
+        check(lib().qtip_decompress_matvec_parts_mix(_ptr(parts), _ptr(packed), _ptr(x_raw), _ptr(su), ctypes.c_float(scale),
+                                                     _ptr(sign_rows), order, _ptr(tlut), m, k, bits, S,
+                                                     stream_ptr(packed.device)), "qtip_decompress_matvec_parts_mix")
+    return parts
+
+
+def matvec_mix_columns(k, order, nparts):
+    """Columns of the transform of k = order * 2^a elements that decompress_matvec_parts_mix runs in front of a matvec of nparts
+    ranges; 0 where it does not."""
+    return lib().qtip_matvec_mix_columns(k, order, nparts)
+
+
 def decompress_matvec_parts_chain(packed, tlut, m, k, bits, prev_parts, post, scale_out, residual, norm_weight, eps,
                                   su, scale_in, nparts=None):
     """(parts, x_new): the boundary between two linear layers and the second layer's matvec in

@@ -63,6 +63,30 @@ def _pack_bits(neg):
     return np.ascontiguousarray(words).view("<u4").reshape(-1).view(np.int32)
 
 
+def sign_rows(bits, K, A, device):
+    """Signs of (table (x) H_A), K * A <= 256 rows of 8 words with bit j of row i set for -1, from the table's `bits` as had_bits
+    returns them (None for K = 1); kept for the built-in tables."""
+    dev = torch.device(device)
+    own = [t for t in (False, True) if bits is not None and bits is _bit_cache.get((K, t, dev))]
+    key = ("rows", K, A, own[0], dev) if own else None
+    if key in _bit_cache:
+        return _bit_cache[key]
+    words = np.zeros(1, np.uint32) if bits is None else bits.cpu().numpy().view(np.uint32)
+    table = np.unpackbits(words.view(np.uint8), bitorder="little")[:K * K].reshape(K, K).T
+    i = np.arange(A)
+    parity = i[:, None] & i[None, :]
+    for s in (4, 2, 1):
+        parity ^= parity >> s
+    parity &= 1
+    neg = (table[:, None, :, None] ^ parity[None, :, None, :]).reshape(K * A, K * A)
+    rows = np.zeros((K * A, 256), np.uint8)
+    rows[:, :K * A] = neg
+    out = torch.from_numpy(np.packbits(rows, axis=1, bitorder="little").view(np.int32)).to(dev)
+    if key:
+        _bit_cache[key] = out
+    return out
+
+
 def had_bits(hadK, K, transpose, device):
     """Device int32 tensor of sign bits for the kernel, cached.
 

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from qtip_amd import ops
+from qtip_amd.utils.matmul_had import had_bits, sign_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +56,37 @@ def test_input_transform_in_front_of_a_matvec(bits, k):
     x, su = (torch.randn(k, generator=g, device="cuda").half() for _ in range(2))
     parts = ops.decompress_matvec_parts_rht(packed, x, su, k**-0.5, tlut, 96, k, bits)
     _close(parts, w, _hadamard(k) @ (x.double() * su.double()) * k**-0.5)
+
+
+# (k, table order, ranges): 64 and 32 columns, rows that do and do not fill a tile of 16 or a k tile of 32, A from 1 to 256,
+# ranges that start inside a tile, buffers that do and do not reach into the table (from 224 rows of 64 on)
+MIXES = ((5504, 172, 2), (11008, 172, 2), (11008, 172, 1), (13824, 108, 3), (14336, 28, 2), (14336, 28, 1), (7168, 28, 5),
+         (5120, 20, 1), (4992, 156, 2), (3328, 52, 1), (1280, 20, 4), (1536, 12, 1), (1024, 1, 1), (16384, 1, 2), (128, 1, 1))
+
+
+@pytest.mark.parametrize("bits,m", ((2, 96), (2, 3232), (3, 96), (4, 96)))
+@pytest.mark.parametrize("k,order,ranges", MIXES)
+@pytest.mark.parametrize("signs", (True, False))
+def test_table_transform_in_front_of_a_matvec(k, order, ranges, m, bits, signs):
+    """Against the transform's own launch in fp32.  A sign vector of other values than +-1 takes three planes."""
+    g = torch.Generator(device="cuda").manual_seed(k + 10 * bits + ranges)
+    packed, tlut, w = _matrix(m, k, bits, g)
+    x, su = (torch.randn(k, generator=g, device="cuda").half() for _ in range(2))
+    if signs:
+        su = torch.where(su < 0, -1.0, 1.0).half()
+    hb = had_bits(None, order, True, "cuda") if order > 1 else None
+    rows = sign_rows(hb, order, k // ops.matvec_mix_columns(k, order, ranges) // order, "cuda")
+    parts = ops.decompress_matvec_parts_mix(packed, x, su, k**-0.5, rows, order, tlut, m, k, bits, ranges)
+    assert parts.shape == (ranges, m)
+    xt = ops.rht((x.float() * su.float())[None], order=order, had_bits=hb, scale=k**-0.5, out_dtype=torch.float32)
+    _close(parts, w, xt.reshape(-1).double())
+
+
+def test_table_transform_refusals():
+    """Fewer than 32 columns, more than 256 rows of 64, a range past the staging area, k inside a wave-load."""
+    for k, order, ranges in ((832, 52, 1), (28672, 28, 4), (16384, 1, 1), (4800, 150, 1), (4096 + 32, 129, 1), (11008, 172, 0)):
+        assert ops.matvec_mix_columns(k, order, ranges) == 0
+    z = torch.zeros(11008, device="cuda").half()
+    packed, tlut, _ = _matrix(32, 11008, 2, torch.Generator(device="cuda").manual_seed(0))
+    with pytest.raises(ValueError):
+        ops.decompress_matvec_parts_mix(packed, z, z, 1.0, torch.zeros(171, 8, dtype=torch.int32, device="cuda"), 172, tlut, 32, 11008, 2)

@@ -495,3 +495,15 @@ def test_key_ranges_of_a_context():
     for heads, ranges in ((41, 6), (64, 4), (128, 2), (256, 1), (300, 1)):
         assert [ops.attention_key_splits(c, heads) for c in (line, many - 1, many, 4096)] == [1, 1, ranges, ranges]
         assert ranges <= ops.ATTN_MAX_KEY_SPLITS
+
+
+@pytest.mark.parametrize("K,A", ((172, 1), (28, 8), (20, 4), (108, 2), (1, 256), (1, 1)))
+@pytest.mark.parametrize("transpose", (True, False))
+def test_sign_rows_of_a_table(K, A, transpose):
+    from scipy.linalg import hadamard
+    from qtip_amd.utils import matmul_had as mh
+    rows = mh.sign_rows(mh.had_bits(None, K, transpose, "cpu") if K > 1 else None, K, A, "cpu")
+    neg = mh._table_signs(K).astype(bool) if K > 1 else np.zeros((1, 1), bool)
+    full = np.kron(np.where(neg.T if transpose else neg, -1, 1), hadamard(A)) < 0
+    bits = np.unpackbits(rows.numpy().view(np.uint8).reshape(K * A, 32), axis=1, bitorder="little").astype(bool)
+    assert np.array_equal(bits[:, :K * A], full) and not bits[:, K * A:].any()
