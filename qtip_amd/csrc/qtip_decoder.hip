@@ -86,7 +86,7 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
   _Float16* kc = k_cache + (size_t)kvh * max_len * D;
   _Float16* vc = v_cache + (size_t)kvh * max_len * D;
   // threads tid < 3 * D hold element c of the new token's query (s3 = 0), key (1) and value (2)
-  const int s3 = tid >> LOGD, c = tid & (D - 1);
+  const int s3 = tid >> LOGD, place = qtip_wht::wht_place(lane), c = ((tid & ~63) | place) & (D - 1);
   const float freq = tid < 2 * D ? inv_freq[c & (half - 1)] : 0.f;
   float postv = 1.f, postp = 1.f;
   _Float16 own = (_Float16)0.f, pair = (_Float16)0.f;  // element c and the one that it is rotated with
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
     if (tid < 3 * D) {
 #pragma unroll
       for (int w = 0; w < 16; ++w) y += acc[(s3 * 16 + w) * D + c];
-      y = qtip_wht::wht_lanes(y, 6, lane);
+      y = qtip_wht::wht_places(y, 6, place);
       if constexpr (D > 64) swap_s[s3 * kMaxHeadDim + c] = y;
       else z = qtip_wht::lane_xor(y, 5);
     }

@@ -186,14 +186,15 @@ __global__ __launch_bounds__(kRhtThreads) void rht_kernel(const RhtParams P) {
     __syncthreads();
   }
   // ---- thread t < RI*pp takes row t / pp, column t % pp
-  const int row = tid >> logc, col = tid & (pp - 1);  // col keeps the lane index in its low bits
+  const int place = wht_place(lane);  // (a permutation inside eight lanes; columns are no fewer)
+  const int row = tid >> logc, col = ((tid & ~63) | place) & (pp - 1);  // col keeps the place in its low bits
   const bool active = tid < RI * pp;
   float y = 0.f;
   if (active) {
     if (JG > 1) {
       for (int q = 0; q < JG; ++q) y += red[row][q * pp + col];
     } else {
-      y = z[0];  // JG == 1 implies pp == 1024 and RI == 1
+      y = wht_to_place(z[0], lane);  // JG == 1 implies pp == 1024 and RI == 1
     }
   }
   // ---- pp-point transform
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(kRhtThreads) void rht_kernel(const RhtParams P) {
   const int nb0 = logc < 6 ? logc : 6;
   int cfin = col;
   if (active) {
-    y = wht_lanes(y, nb0, lane);
+    y = wht_places(y, nb0, place);
     if (W > 1) red[row][col] = y;
   }
   if (W > 1) {
@@ -211,11 +212,11 @@ __global__ __launch_bounds__(kRhtThreads) void rht_kernel(const RhtParams P) {
     if (active) {
       // transposed read: the wave index of the element becomes the low lane bits
       const int wv = col >> 6;
-      const int ew = lane & (W - 1);              // wave part of the element index
-      const int el = (lane >> logw) + (64 >> logw) * wv;  // lane part of the element index
+      const int ew = place & (W - 1);             // wave part of the element index
+      const int el = (place >> logw) + (64 >> logw) * wv;  // lane part of the element index
       cfin = 64 * ew + el;
       y = red[row][cfin];
-      y = wht_lanes(y, logw, lane);
+      y = wht_places(y, logw, place);
     }
   }
   if (active) {
@@ -295,12 +296,13 @@ __global__ __launch_bounds__(kRhtThreads) void rht_vec_kernel(const RhtParams P)
 
   // ---- this thread's output element and its operands
   const bool active = tid < pp;
+  const int place = wht_place(lane), col = (tid & ~63) | place;  // the thread's column (pp is a multiple of 8)
   const int logw = P.logw;
   const int W = 1 << logw;  // waves holding the row in the transform
-  int cfin = tid;
+  int cfin = col;
   if (W > 1) {
     const int wv = tid >> 6;
-    cfin = 64 * (lane & (W - 1)) + (lane >> logw) + (64 >> logw) * wv;  // after the transposed read
+    cfin = 64 * (place & (W - 1)) + (place >> logw) + (64 >> logw) * wv;  // after the transposed read
   }
   const size_t oidx = ((size_t)iK * A + iA) * pp + cfin;
   float postv = 1.f, resv = 0.f;
@@ -439,20 +441,20 @@ __global__ __launch_bounds__(kRhtThreads) void rht_vec_kernel(const RhtParams P)
   __syncthreads();
   float y = 0.f;
   if (active) {
-    for (int q = 0; q < NP; ++q) y += red[q * pp + tid];
+    for (int q = 0; q < NP; ++q) y += red[q * pp + col];
   }
   if (W > 1) __syncthreads();  // the buffer is reused only when a row spans several waves
   // ---- pp-point transform of column tid
   const int nb0 = lcg + 3 < 6 ? lcg + 3 : 6;  // log2(pp), at most the six lane bits
   if (active) {
-    y = wht_lanes(y, nb0, lane);
-    if (W > 1) red[tid] = y;
+    y = wht_places(y, nb0, place);
+    if (W > 1) red[col] = y;
   }
   if (W > 1) {
     __syncthreads();
     if (active) {
       y = red[cfin];
-      y = wht_lanes(y, logw, lane);
+      y = wht_places(y, logw, place);
     }
   }
   if (active) {
@@ -488,10 +490,11 @@ __global__ __launch_bounds__(kRhtThreads) void rht_vec_silu_pair_kernel(const Rh
   const int JG = kRhtThreads >> lcg;
   const int cg = tid & (CG - 1), jg = tid >> lcg;
   const bool active = tid < pp;
+  const int place = wht_place(lane), col = (tid & ~63) | place;  // the thread's column (pp is a multiple of 8)
   const int logw = P.logw;
   const int W = 1 << logw;
-  int cfin = tid;
-  if (W > 1) cfin = 64 * (lane & (W - 1)) + (lane >> logw) + (64 >> logw) * wave;
+  int cfin = col;
+  if (W > 1) cfin = 64 * (place & (W - 1)) + (place >> logw) + (64 >> logw) * wave;
   const size_t oidx1 = ((size_t)iK * A + iA) * pp + cfin;
   const size_t oidx2 = ((size_t)iK2 * A + iA) * pp + cfin;
   float post1 = 1.f, post2 = 1.f;
@@ -597,24 +600,24 @@ __global__ __launch_bounds__(kRhtThreads) void rht_vec_silu_pair_kernel(const Rh
   float y1 = 0.f, y2 = 0.f;
   if (active) {
     for (int q = 0; q < NP; ++q) {
-      y1 += red1[q * pp + tid];
-      y2 += red2[q * pp + tid];
+      y1 += red1[q * pp + col];
+      y2 += red2[q * pp + col];
     }
   }
   if (W > 1) __syncthreads();  // the partial vectors are consumed before the buffers are reused
   if (active) {
-    y1 = wht_lanes(y1, nb0, lane);
-    y2 = wht_lanes(y2, nb0, lane);
+    y1 = wht_places(y1, nb0, place);
+    y2 = wht_places(y2, nb0, place);
     if (W > 1) {
-      red1[tid] = y1;
-      red2[tid] = y2;
+      red1[col] = y1;
+      red2[col] = y2;
     }
   }
   if (W > 1) {
     __syncthreads();
     if (active) {
-      y1 = wht_lanes(red1[cfin], logw, lane);
-      y2 = wht_lanes(red2[cfin], logw, lane);
+      y1 = wht_places(red1[cfin], logw, place);
+      y2 = wht_places(red2[cfin], logw, place);
     }
   }
   if (active) {
@@ -667,10 +670,9 @@ template <int EPT, typename TIn, typename TOut>
 __global__ __launch_bounds__(kRhtThreads) void rht_rows_kernel(const RhtParams P) {
   constexpr int N = kRhtThreads * EPT;
   __shared__ __align__(16) float xbuf[N + N / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wave = threadIdx.x >> 6, place = wht_place(threadIdx.x & 63);
   const size_t r = blockIdx.x;
-  const int e_nat = tid * EPT;
-  const int e_swp = (((lane & 15) << 6) | ((wave & 15) << 2) | (lane >> 4)) * EPT;
+  const int e_nat = qtip_chain::nat_index<EPT>(place, wave), e_swp = qtip_chain::swp_index<EPT>(place, wave);
   const TIn* src = reinterpret_cast<const TIn*>(P.in) + r * P.in_row_stride;
   float v[EPT], pv[EPT];
   auto load = [&](const TIn* p, float t[EPT]) {
@@ -705,13 +707,13 @@ __global__ __launch_bounds__(kRhtThreads) void rht_rows_kernel(const RhtParams P
     }
   }
   wht_regs<EPT>(v);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(v[i], 6, lane);
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) xbuf[xidx<EPT>(e_nat + i)] = v[i];
+  wht_places<EPT>(v, 6, place);
+  st_f32<EPT>(xbuf + xidx<EPT>(e_nat), v);
   __syncthreads();
+  ld_f32<EPT>(xbuf + xidx<EPT>(e_swp), v);
+  wht_places<EPT>(v, 4, place);
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) v[i] = wht_lanes(xbuf[xidx<EPT>(e_swp + i)], 4, lane) * P.scale * pv[i];
+  for (int i = 0; i < EPT; ++i) v[i] = v[i] * P.scale * pv[i];
   TOut* dst = reinterpret_cast<TOut*>(P.out) + r * (size_t)N + e_swp;
   if constexpr (sizeof(TOut) == 2) {
     _Float16 h[EPT];
@@ -719,8 +721,7 @@ __global__ __launch_bounds__(kRhtThreads) void rht_rows_kernel(const RhtParams P
     for (int i = 0; i < EPT; ++i) h[i] = (_Float16)v[i];
     st_f16<EPT>(reinterpret_cast<_Float16*>(dst), h);
   } else {
-#pragma unroll
-    for (int i = 0; i < EPT; ++i) reinterpret_cast<float*>(dst)[i] = v[i];
+    st_f32<EPT>(reinterpret_cast<float*>(dst), v);
   }
 }
 

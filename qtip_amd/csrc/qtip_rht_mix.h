@@ -80,6 +80,8 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   // ---- this lane's patch of v: row j = 16 * wave + 4 * g + i, columns c0 .. c0 + 7 of row rsub of the pass
   const int lrows = 7 - logpp;  // log2 of the rows per pass
   const int rsub = (8 * a) >> logpp, c0 = (8 * a) & ((1 << logpp) - 1);
+  // a result's columns are those of the lane's place, which the operands are read for
+  const int pa = wht_place(lane) & 15, rsub_out = (8 * pa) >> logpp, c0_out = (8 * pa) & ((1 << logpp) - 1);
   const int Am = (1 << logA2) - 1;
   // element j, slice part sl inside a row
   auto element = [&](int j, int sl) {
@@ -224,7 +226,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
     }
     return x;
   };
-  // H_pp on the products (register e is column bits 0..2, lane bit b of a column bit 3 + b) and the results
+  // H_pp on the products (register e is column bits 0..2, bit b of a lane's place column bit 3 + b) and the results
   auto finish = [&](float4v acc[8], int ps) {
     if (idle) return;
     if constexpr (!AUX) asm volatile("" ::"v"(line));
@@ -243,18 +245,18 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
 #pragma unroll
         for (int e = 0; e < 8; ++e)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) acc[e][q] = wht_stage(acc[e][q], b, lane);
+          for (int q = 0; q < 4; ++q) acc[e][q] = wht_place_stage(acc[e][q], b, pa);
       }
     // output rows 16 * wave + 4 * g + q of the mix
-    const bool row_ok = (int)first_row(ps) + rsub < rows;
-    const uint32_t lr = lane_row(ps);
+    const bool row_ok = (int)first_row(ps) + rsub_out < rows;
+    const uint32_t lr = row_ok ? (uint32_t)rsub_out : 0u;
     const float* post = P.post ? P.post + first_row(ps) * P.post_row_stride : nullptr;
     const _Float16* res = P.residual ? P.residual + first_row(ps) * n : nullptr;
     TOut* out = reinterpret_cast<TOut*>(P.out) + first_row(ps) * n;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int i = j0 + q;
-      const uint32_t o = element(i < on ? i : 0, s);
+      const uint32_t o = element(i < on ? i : 0, s) - c0 + c0_out;
       float y[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) y[e] = acc[e][q] * P.scale;
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
     }
   };
   uint8_t* wr = mix_smem + (uint32_t)a * stride + (uint32_t)(4 * wave + g) * 8;
-  const uint8_t* rd = mix_smem + (uint32_t)a * stride + (uint32_t)g * 16;
+  const uint8_t* rd = mix_smem + (uint32_t)pa * stride + (uint32_t)g * 16;
   // the plane's products: a column group's next operand is requested as soon as its present one is used
   auto products = [&](float4v acc[8], uint32_t one, auto mfma) {
     if (idle) return;

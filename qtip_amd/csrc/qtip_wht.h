@@ -30,42 +30,27 @@ __device__ __forceinline__ float lane_xor(float v, int b) {
   return __builtin_bit_cast(float, r);
 }
 
-// One butterfly over lane bit b: lanes with the bit clear get v + partner, the others partner - v.
-// Written as partner + (v with its sign flipped where the bit is set): an xor and an addition (the
-// exchange rides on the addition as a DPP operand) instead of an addition, a subtraction and a
-// select; the sums are the same floating-point operations on the same operands.
-__device__ __forceinline__ float wht_stage(float v, int b, int lane) {
-  const uint32_t flip = ((uint32_t)lane << (31 - b)) & 0x80000000u;
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  if (b == 5) {
-    // the swap exchanges the upper half of its first operand with the lower half of its second:
-    // with (v, flipped v) the first result holds the lower half's values in either half and the
-    // second the upper half's, negated where they stayed at home - their sum is the butterfly
-    auto sw = __builtin_amdgcn_permlane32_swap(u, u ^ flip, false, false);
-    return __builtin_bit_cast(float, (uint32_t)sw[0]) + __builtin_bit_cast(float, (uint32_t)sw[1]);
-  }
-  return lane_xor(v, b) + __builtin_bit_cast(float, u ^ flip);
-}
-
-// Walsh-Hadamard butterflies over lane bits lo .. nbits-1 (natural order)
-__device__ __forceinline__ float wht_lanes(float v, int nbits, int lane, int lo = 0) {
-#pragma unroll
-  for (int b = 0; b < 6; ++b) {
-    if (b >= lo && b < nbits) v = wht_stage(v, b, lane);
-  }
-  return v;
-}
-
 // Transforms whose elements may sit in any lane keep element `place` of a wave in lane place ^ (3 if bit 2 of it is set).
 // A step over bit 2 of the place then exchanges lanes l and l ^ 7, a mirror of eight lanes that rides on the addition
 // as a DPP operand, and the one over bit 4 is a row swap: no step goes through the LDS crossbar, whose round trip (a wave
-// of a boundary waited for sixteen of them in a row) was most of a transform's time.  The additions are those of wht_lanes.
+// of a boundary waited for sixteen of them in a row) was most of a transform's time.
 __device__ __forceinline__ int wht_place(int lane) {
   return lane ^ ((lane & 4) ? 3 : 0);
+}
+// the value of element `lane` of a wave -> that of element wht_place(lane), in every lane
+__device__ __forceinline__ float wht_to_place(float v, int lane) {
+  const float m = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x1B, 0xF, 0xF, false));
+  return (lane & 4) ? m : v;  // (quads with bit 2 set run backwards)
 }
 __device__ __forceinline__ float half_mirror(float v) {  // value of lane ^ 7
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));
 }
+// One butterfly over bit b of the place: lanes with the bit clear get v + partner, the others partner - v.
+// Written as partner + (v with its sign flipped where the bit is set): an xor and an addition (the
+// exchange rides on the addition as a DPP operand) instead of an addition, a subtraction and a
+// select; the sums are the same floating-point operations on the same operands.  The swaps exchange odd rows (or the
+// upper half) of their first operand with even rows (the lower half) of their second: with (v, flipped v) the first result holds
+// the lower partner's values in either and the second the upper one's, negated where they stayed at home - their sum is the butterfly.
 __device__ __forceinline__ float wht_place_stage(float v, int b, int place) {
   const uint32_t flip = ((uint32_t)place << (31 - b)) & 0x80000000u;
   const uint32_t u = __builtin_bit_cast(uint32_t, v), f = u ^ flip;
@@ -84,6 +69,13 @@ __device__ __forceinline__ void wht_places(float (&v)[EPT], int nbits, int place
 #pragma unroll
       for (int i = 0; i < EPT; ++i) v[i] = wht_place_stage(v[i], b, place);
     }
+}
+
+__device__ __forceinline__ float wht_places(float v, int nbits, int place, int lo = 0) {
+#pragma unroll
+  for (int b = 0; b < 6; ++b)
+    if (b >= lo && b < nbits) v = wht_place_stage(v, b, place);
+  return v;
 }
 
 // the sum over the lanes of a wave (four lanes hold the same sum when eight are mirrored)
