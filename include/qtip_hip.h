@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define QTIP_ABI_VERSION 28 /* of this header; a library tells its own by qtip_abi_version() */
+#define QTIP_ABI_VERSION 29 /* of this header; a library tells its own by qtip_abi_version() */
 
 #define QTIP_OK 0
 #define QTIP_E_SHAPE (-1)     /* m % 32, k % 32, bits, batch or n out of range */
@@ -379,6 +379,20 @@ int qtip_decode_attention_rht(void* out_f16, const float* parts, int in_parts, s
                               void* k_cache_f16, void* v_cache_f16, const void* pos_i64,
                               const float* inv_freq, int heads, int kv_heads, int head_dim, int max_len,
                               int key_splits, float* split_workspace, void* stream);
+
+/* qtip_decode_attention_rht (vectors = 1) or _rht3 (vectors = 3) over up to `ranges` (1..4) ranges of the keys, by the position in
+ * device memory: one up to 379 keys (639 with more than 40 heads), then one for every 160, of equal length.  What it leaves in `shares` is read by
+ * qtip_decompress_matvec_parts_shares: heads * ranges * (head_dim + 4) floats, 16-byte aligned. */
+int qtip_decode_attention_shares(float* shares, int ranges, int vectors, const float* const* parts, int in_parts, size_t part_stride,
+                                 const float* const* post_f32, const float* scale, const uint32_t* const* had_bits, const int* order,
+                                 void* k_cache_f16, void* v_cache_f16, const void* pos_i64, const float* inv_freq, int heads,
+                                 int kv_heads, int head_dim, int max_len, void* stream);
+
+/* qtip_decompress_matvec_parts_rht on the attention output of k / head_dim heads that those shares give, rounded to fp16; the same
+ * ranges, head_dim, position and max_len. */
+int qtip_decompress_matvec_parts_shares(float* parts, const void* packed, const float* shares, int ranges, int head_dim,
+                                        const void* pos_i64, int max_len, const void* su_f16, float scale, const void* tlut, int m,
+                                        int k, int bits, int nparts, void* stream);
 
 /* qtip_decode_attention_rht for separate q / k / v projections: three raw matvec results, each
  * with the output transform of its own QuantizedLinear (q: heads * head_dim elements, k and v:

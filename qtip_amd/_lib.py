@@ -17,7 +17,7 @@ HOST_PATH = os.path.join(_HERE, "_qtip_host.so")
 
 QTIP_F16 = 0
 QTIP_F32 = 1
-ABI_VERSION = 28
+ABI_VERSION = 29
 
 _lib = None
 _host = None
@@ -37,6 +37,11 @@ _SIGNATURES = {
     "qtip_decompress_matvec_parts": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 + [ctypes.c_void_p]),
     "qtip_decompress_matvec_parts_rht": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_float, ctypes.c_void_p] +
                                          [ctypes.c_int] * 4 + [ctypes.c_void_p]),
+    "qtip_decode_attention_shares": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int,
+                                     ctypes.c_size_t] + [ctypes.c_void_p] * 8 + [ctypes.c_int] * 4 + [ctypes.c_void_p]),
+    "qtip_decompress_matvec_parts_shares": (ctypes.c_int, [ctypes.c_void_p] * 3 + [ctypes.c_int] * 2 +
+                                            [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p] +
+                                            [ctypes.c_int] * 4 + [ctypes.c_void_p]),
     "qtip_matvec_mix_columns": (ctypes.c_int, [ctypes.c_int] * 3),
     "qtip_decompress_matvec_parts_mix": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_float, ctypes.c_void_p, ctypes.c_int,
                                          ctypes.c_void_p] + [ctypes.c_int] * 4 + [ctypes.c_void_p]),

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include "../../include/qtip_hip.h"
+#include "qtip_shares.h"
 #include "qtip_wht.h"
 
 namespace {
@@ -66,6 +67,8 @@ __device__ __forceinline__ _Float16 rotated(_Float16 x, _Float16 c, _Float16 y, 
 // sums, its score maximum and its sum of exponentials - in split_ws[head][z][D + 2] for
 // attn_combine_kernel; every workgroup repeats the prologue (transform, rotary embedding), the
 // one of range 0 writes the cache.
+// keys_per_split = 0: the ranges of qtip_shares.h, whose shares the next matvec reads; no workgroup past those in use does
+// anything.
 template <int D, int XF>
 __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
     _Float16* __restrict__ out, const _Float16* __restrict__ qkv, _Float16* __restrict__ k_cache,
@@ -120,8 +123,12 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
   // projections 528 537 562 / 520 527 547.
   constexpr int LPK = D / 8, KPW = 64 / LPK, U = 16 * KPW, NU = 2;
   const int nkeys = pos + 1 < max_len ? pos + 1 : max_len;
-  const int k0 = (int)blockIdx.z * keys_per_split;  // this workgroup's keys: [k0, k1)
-  const int k1 = k0 + keys_per_split < nkeys ? k0 + keys_per_split : nkeys;
+  const bool open = keys_per_split == 0;
+  const int used = open ? qtip_shares::active(nkeys, nsplit, H) : nsplit;
+  if ((int)blockIdx.z >= used) return;
+  const int kps = open ? qtip_shares::keys_of(nkeys, used) : keys_per_split;
+  const int k0 = (int)blockIdx.z * kps;  // this workgroup's keys: [k0, k1)
+  const int k1 = k0 + kps < nkeys ? k0 + kps : nkeys;
   const int kend = k1 < pos ? k1 : pos;             // (the new key comes from LDS)
   const __amdgpu_buffer_rsrc_t rs_k = __builtin_amdgcn_make_buffer_rsrc(kc, 0, max_len * D * 2, 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_v = __builtin_amdgcn_make_buffer_rsrc(vc, 0, max_len * D * 2, 0x00020000);
@@ -402,10 +409,10 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
     tot += f * red[16 + w];
     sum += f * acc[w * D + tid];
   }
-  if (nsplit == 1) {
+  if (nsplit == 1 && !open) {
     out[(size_t)h * D + tid] = (_Float16)(sum * (1.f / tot));
   } else {
-    float* w = split_ws + ((size_t)h * nsplit + blockIdx.z) * (D + 2);
+    float* w = split_ws + ((size_t)h * nsplit + blockIdx.z) * (open ? qtip_shares::floats(D) : D + 2);
     w[tid] = sum;       // 0 for a range past the last key
     if (tid == 0) {
       w[D] = mx;        // -inf for an empty range
@@ -438,17 +445,17 @@ __global__ __launch_bounds__(kMaxHeadDim) void attn_combine_kernel(_Float16* __r
 static int launch_attention(void* out_f16, const void* qkv_f16, const AttnXf* xf, int xf_mode, void* k_cache_f16,
                             void* v_cache_f16, const void* pos_i64, const float* inv_freq, int heads,
                             int kv_heads, int head_dim, int max_len, int key_splits, float* split_ws,
-                            void* stream) {
-  if (!out_f16 || !k_cache_f16 || !v_cache_f16 || !pos_i64 || !inv_freq) return QTIP_E_NULL;
+                            void* stream, bool open = false) {
+  if ((!out_f16 && !open) || !k_cache_f16 || !v_cache_f16 || !pos_i64 || !inv_freq) return QTIP_E_NULL;
   if (key_splits < 1 || key_splits > 16) return QTIP_E_SHAPE;
-  if (key_splits > 1 && !split_ws) return QTIP_E_NULL;
-  if (key_splits > 1 && (reinterpret_cast<uintptr_t>(split_ws) & 15)) return QTIP_E_ALIGN;
+  if ((key_splits > 1 || open) && !split_ws) return QTIP_E_NULL;
+  if ((key_splits > 1 || open) && (reinterpret_cast<uintptr_t>(split_ws) & 15)) return QTIP_E_ALIGN;
   if (heads < 1 || kv_heads < 1 || heads % kv_heads || head_dim < 64 || head_dim > kMaxHeadDim ||
       (head_dim & (head_dim - 1)) || max_len < 1 || max_len > 4096)  // (positions the rotary reduction is stated for)
     return QTIP_E_SHAPE;
   const size_t lds = (size_t)(6 * kMaxHeadDim + 32 + (xf ? 3 : 1) * 16 * head_dim) * sizeof(float);
   const dim3 grid((unsigned)(heads / kv_heads), (unsigned)kv_heads, (unsigned)key_splits);
-  const int kps = (max_len + key_splits - 1) / key_splits;  // keys per range
+  const int kps = open ? 0 : (max_len + key_splits - 1) / key_splits;  // keys per range
 #define QTIP_ATTN(DD, XX, ARG)                                                                      \
   decode_attn_kernel<DD, XX><<<grid, kAttnThreads, lds, (hipStream_t)stream>>>(                      \
       (_Float16*)out_f16, (const _Float16*)qkv_f16, (_Float16*)k_cache_f16, (_Float16*)v_cache_f16,  \
@@ -469,7 +476,7 @@ static int launch_attention(void* out_f16, const void* qkv_f16, const AttnXf* xf
   }
 #undef QTIP_ATTN
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || key_splits == 1) return (int)e;
+  if (e != hipSuccess || key_splits == 1 || open) return (int)e;
   attn_combine_kernel<<<heads, head_dim, 0, (hipStream_t)stream>>>((_Float16*)out_f16, split_ws, key_splits,
                                                                    head_dim);
   return (int)hipGetLastError();
@@ -542,6 +549,27 @@ extern "C" int qtip_decode_attention_rht3(void* out_f16, const float* const* par
   x.in_parts = in_parts;
   return launch_attention(out_f16, nullptr, &x, 2, k_cache_f16, v_cache_f16, pos_i64, inv_freq, heads, kv_heads,
                           head_dim, max_len, key_splits, split_workspace, stream);
+}
+
+extern "C" int qtip_decode_attention_shares(float* shares, int ranges, int vectors, const float* const* parts, int in_parts,
+                                            size_t part_stride, const float* const* post_f32, const float* scale,
+                                            const uint32_t* const* had_bits, const int* order, void* k_cache_f16,
+                                            void* v_cache_f16, const void* pos_i64, const float* inv_freq, int heads, int kv_heads,
+                                            int head_dim, int max_len, void* stream) {
+  if (!parts || !post_f32 || !scale || !had_bits || !order) return QTIP_E_NULL;
+  if ((vectors != 1 && vectors != 3) || ranges < 1 || ranges > qtip_shares::kMaxRanges || in_parts < 1 || in_parts > 16 ||
+      heads < 1 || kv_heads < 1 || head_dim < 64 || head_dim > 128 || (part_stride & 3))
+    return QTIP_E_SHAPE;
+  AttnXf x = {};
+  for (int s = 0; s < vectors; ++s) {
+    const long n = (long)(vectors == 1 ? heads + 2 * kv_heads : (s == 0 ? heads : kv_heads)) * head_dim;
+    const int rc = fill_xf_slot(x, s, parts[s], post_f32[s], had_bits[s], scale[s], order[s], n, head_dim);
+    if (rc) return rc;
+  }
+  x.part_stride = part_stride;
+  x.in_parts = in_parts;
+  return launch_attention(nullptr, nullptr, &x, vectors == 1 ? 1 : 2, k_cache_f16, v_cache_f16, pos_i64, inv_freq, heads, kv_heads,
+                          head_dim, max_len, ranges, shares, stream, true);
 }
 
 // ---- token head of the decode loop: final RMSNorm and the greedy pick ------------------------

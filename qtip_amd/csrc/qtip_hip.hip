@@ -11,6 +11,7 @@
 #include "../../include/qtip_hip.h"
 #include "qtip_device.h"
 #include "qtip_setup.h"
+#include "qtip_shares.h"
 #include "qtip_wht.h"
 
 #ifdef QTIP_STAMPS  // (the timeline build, see QTIP_STAMP)
@@ -268,7 +269,8 @@ __device__ __forceinline__ T* pick3(T* const (&a)[3], int g) {
 // prologue), 2 = the previous layer's partial results (whole layer boundary in the prologue).
 // 3 = as 1, for a table order times a power of two (qtip_mix.h); every workgroup makes the range of the vector that it reads
 // and x is staged as in the plain form.  EPT is a sixteenth of the columns there.
-// EPT = k / 1024 with 1 and 2, a kernel each: behind a switch over it the compiler waits for everything in flight.
+// 4 = as 1, on the attention output that the shares of the key ranges give (qtip_shares.h).
+// EPT = k / 1024 with 1, 2 and 4, a kernel each: behind a switch over it the compiler waits for everything in flight.
 // XHALF: the k range needs up to twice the staging area and every workgroup has exactly one unit:
 // x is staged in two halves, the second replacing the first in the middle of the unit (two more
 // barriers per launch instead of x travelling through vector loads with every wave-load, which
@@ -285,10 +287,11 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
     float* __restrict__ dst_, const uint8_t* __restrict__ packed_, const uint16_t* __restrict__ x_,
     const uint32_t* __restrict__ tlut_, int m_, int k_, int wl_per, int upw_q_, int upw_r_,
     const uint16_t* __restrict__ su_ = nullptr, float xscale = 1.f, const ChainArgs chain = ChainArgs{},
-    const GroupArgs grp = GroupArgs{}, const qtip_mix::MixArgs mix = qtip_mix::MixArgs{}) {
+    const GroupArgs grp = GroupArgs{}, const qtip_mix::MixArgs mix = qtip_mix::MixArgs{},
+    const qtip_shares::ShareArgs sh = qtip_shares::ShareArgs{}) {
   static_assert(!XFORM || XLDS, "the transformed activations live in LDS");
   static_assert((XFORM != 0) == (EPT != 0), "a transform in front knows its size");
-  constexpr bool POW2 = XFORM == 1 || XFORM == 2;  // the whole transformed vector, in padded wave-loads
+  constexpr bool POW2 = XFORM != 0 && XFORM != 3;  // the whole transformed vector, in padded wave-loads
   const int k = POW2 ? 1024 * EPT : k_;
   static_assert(!GROUP || XFORM == 2 || (XFORM == 0 && XLDS && !XHALF),
                 "grouped launches exist for the layer-boundary form and the plain form with x in LDS");
@@ -482,6 +485,49 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
       chain_load<EPT>(chain, sr, place, wave, cr);
       requested();
       chain_compute<EPT>(cr, chain, xscale, xbuf, xo, lane, place, wave, blockIdx.x == 0 && blockIdx.y == 0, QTIP_STAMP_PTR);
+    } else if constexpr (XFORM == 4) {
+      typedef _Float16 hvec __attribute__((ext_vector_type(EPT)));
+      const int e = nat_index<EPT>(place, wave), dim = 1 << sh.log_dim, step = qtip_shares::floats(dim);
+      const float* w = sh.shares + (size_t)(e >> sh.log_dim) * sh.ranges * step;
+      const int d = e & (dim - 1);
+      const hvec sv = *reinterpret_cast<const hvec*>(sr + e);
+      constexpr int R = qtip_shares::kMaxRanges;
+      float o[R][EPT] = {};
+      float2 ml[R] = {};
+      qtip_wht::ld_f32<EPT>(w + d, o[0]);
+      ml[0] = *reinterpret_cast<const float2*>(w + dim);
+      const int pos = (int)sh.pos[0], nkeys = pos + 1 < sh.max_len ? pos + 1 : sh.max_len;
+      const int used = qtip_shares::active(nkeys, sh.ranges, k >> sh.log_dim);
+      if (used > 1) {  // (the position is as far away as the first share: short contexts wait for nothing more)
+#pragma unroll
+        for (int z = 1; z < R; ++z) {
+          const float* wz = w + (z < used ? z : 0) * step;
+          qtip_wht::ld_f32<EPT>(wz + d, o[z]);
+          ml[z] = *reinterpret_cast<const float2*>(wz + dim);
+        }
+      }
+      requested();
+      float v[EPT];
+      if (used == 1) {
+        const float f = 1.f / ml[0].y;
+#pragma unroll
+        for (int i = 0; i < EPT; ++i) v[i] = (float)(_Float16)(o[0][i] * f) * (float)sv[i];
+      } else {
+        float M = ml[0].x;
+#pragma unroll
+        for (int z = 1; z < R; ++z) M = z < used ? fmaxf(M, ml[z].x) : M;
+        float num[EPT] = {}, den = 0.f;
+#pragma unroll
+        for (int z = 0; z < R; ++z) {
+          const float f = z < used && ml[z].x != -INFINITY ? __expf(ml[z].x - M) : 0.f;
+          den += z < used ? f * ml[z].y : 0.f;
+#pragma unroll
+          for (int i = 0; i < EPT; ++i) num[i] += z < used ? f * o[z][i] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < EPT; ++i) v[i] = (float)(_Float16)(num[i] / den) * (float)sv[i];
+      }
+      xform_compute<EPT>(v, xscale, xbuf, xo, place, wave);
     } else {
       // the raw activations and the sign vector of the layer
       typedef _Float16 hvec __attribute__((ext_vector_type(EPT)));
@@ -700,7 +746,8 @@ hipError_t allow_lds_all() {
 #define QTIP_ALLOW_XFORM(BITS, EPT)                                                                       \
   QTIP_ALLOW((matvec_kernel<BITS, 2, true, 1, false, false, false, EPT>), xform_lds(1024 * EPT))           \
   QTIP_ALLOW((matvec_kernel<BITS, 2, true, 2, false, false, false, EPT>), xform_lds(1024 * EPT))           \
-  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 2, false, true, false, EPT>), xform_lds(1024 * EPT))
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 2, false, true, false, EPT>), xform_lds(1024 * EPT))            \
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 4, false, false, false, EPT>), xform_lds(1024 * EPT))
   QTIP_ALLOW_XFORM(2, 2) QTIP_ALLOW_XFORM(2, 4) QTIP_ALLOW_XFORM(2, 8)
   QTIP_ALLOW_XFORM(3, 2) QTIP_ALLOW_XFORM(3, 4) QTIP_ALLOW_XFORM(3, 8)
   QTIP_ALLOW_XFORM(4, 2) QTIP_ALLOW_XFORM(4, 4) QTIP_ALLOW_XFORM(4, 8)
@@ -900,7 +947,8 @@ size_t qtip_matvec_workspace_bytes(int m, int k, int bits) {
 
 static int launch_matvec(const Ready& di, float* dst, const void* packed, const void* x_f16, const void* tlut,
                          int m, int k, int bits, int S, hipStream_t st, const void* su_f16 = nullptr,
-                         float xscale = 1.f, const ChainArgs* chain = nullptr, const qtip_mix::MixArgs* mix = nullptr) {
+                         float xscale = 1.f, const ChainArgs* chain = nullptr, const qtip_mix::MixArgs* mix = nullptr,
+                         const qtip_shares::ShareArgs* shares = nullptr) {
   const long units = (long)(m >> 5) * S;
   long grid = units < di.cus ? units : di.cus;
   grid -= grid % S;  // a workgroup keeps one k range (units is a multiple of S, so grid >= S)
@@ -918,6 +966,10 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
     auto* sg = (const uint16_t*)su_f16;
     if (chain) {
       QTIP_XFORM(2, false, (dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale, *chain))
+      return (int)hipGetLastError();
+    }
+    if (shares) {
+      QTIP_XFORM(4, false, (dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale, ChainArgs{}, GroupArgs{}, qtip_mix::MixArgs{}, *shares))
       return (int)hipGetLastError();
     }
     QTIP_XFORM(1, false, (dst, p, xx, t, m, k, wl_per, uq, ur, sg, xscale))
@@ -1046,6 +1098,22 @@ int qtip_decompress_matvec_parts_rht(float* parts, const void* packed, const voi
   const Ready rd = ready(stream);
   if (rd.rc) return rd.rc;
   return launch_matvec(rd, parts, packed, x_raw_f16, tlut, m, k, bits, nparts, (hipStream_t)stream, su_f16, scale);
+}
+
+int qtip_decompress_matvec_parts_shares(float* parts, const void* packed, const float* shares, int ranges, int head_dim,
+                                        const void* pos_i64, int max_len, const void* su_f16, float scale, const void* tlut, int m,
+                                        int k, int bits, int nparts, void* stream) {
+  int rc = check_matvec(parts, packed, shares, tlut, m, k, bits);
+  if (rc) return rc;
+  if (!su_f16 || !pos_i64) return QTIP_E_NULL;
+  if ((k != 2048 && k != 4096 && k != 8192) || (head_dim != 64 && head_dim != 128)) return QTIP_E_SHAPE;
+  if (nparts < 1 || nparts > kMaxSplit || nparts > (k >> 7) || ranges < 1 || ranges > qtip_shares::kMaxRanges || max_len < 1)
+    return QTIP_E_SHAPE;
+  if (!aligned16(shares) || !aligned16(su_f16)) return QTIP_E_ALIGN;
+  const qtip_shares::ShareArgs sh = {shares, (const long*)pos_i64, ranges, head_dim == 64 ? 6 : 7, max_len};
+  const Ready rd = ready(stream);
+  if (rd.rc) return rd.rc;
+  return launch_matvec(rd, parts, packed, shares, tlut, m, k, bits, nparts, (hipStream_t)stream, su_f16, scale, nullptr, nullptr, &sh);
 }
 
 int qtip_matvec_mix_columns(int k, int order, int nparts) { return matvec_mix_cols(k, order, nparts); }

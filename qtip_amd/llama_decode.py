@@ -283,7 +283,11 @@ class DecoderLayer(nn.Module):
         else:
             qkv = torch.cat([f[n](x, ops.PRE_RMSNORM, self.input_norm.weight, cfg.eps)
                              for n in ('q_proj', 'k_proj', 'v_proj')], dim=-1)
-        if qkv is None:
+        attn = o_parts = None
+        if qkv is None and self._o_takes_shares() and f['qkv'].SV.dtype == torch.float32:
+            q = f['qkv']
+            o_parts = self._attend_into_o([qkv_parts.reshape(-1, q.m)], [q], k_cache, v_cache, pos, inv_freq)
+        elif qkv is None:
             # the attention kernel transforms the head-sized slices it needs itself
             q = f['qkv']
             attn = ops.decode_attention_rht(qkv_parts, q.SV, (q.m**-0.5) * 32.0, q.br, q.Kr, k_cache, v_cache, pos,
@@ -292,11 +296,11 @@ class DecoderLayer(nn.Module):
             attn = ops.decode_attention(qkv.reshape(-1), k_cache, v_cache, pos, inv_freq, cfg.heads, cfg.kv_heads,
                                         cfg.head_dim, key_splits=cfg.attn_key_splits)
         if self.fused and f['o'].can_chain_into(f['up_gate']):
-            parts = f['o'].matvec_from(attn.reshape(1, -1))
+            parts = f['o'].matvec_from(attn.reshape(1, -1)) if o_parts is None else o_parts
             x, ug_parts = f['o'].chain_matvec(parts, x, f['up_gate'], self.post_norm.weight, cfg.eps)
             ug = f['up_gate'].transform_out_silu(ug_parts)
         else:
-            x = f['o'](attn.reshape(1, -1), residual=x)
+            x = f['o'](attn.reshape(1, -1), residual=x) if o_parts is None else f['o'].transform_out(o_parts, x)
             if self.fused and not f['up_gate'].dense:
                 u = f['up_gate']
                 ug = u.transform_out_silu(u.matvec(u.transform_in(x, ops.PRE_RMSNORM, self.post_norm.weight, cfg.eps)))
@@ -314,6 +318,29 @@ class DecoderLayer(nn.Module):
         if open_end and f['down'].can_end_open():
             return x, f['down'].matvec_behind(ug, pre)
         return f['down'](ug, pre, residual=x), None
+
+    def _o_takes_shares(self):
+        """The attention may cut the keys in ranges by the position alone: o's matvec puts their shares together.  A count of
+        ranges that a caller set (cfg.attn_key_splits) is one for the attention's own launch."""
+        return self.cfg.attn_key_splits == 1 and self._fused_linears()['o'].takes_shares(self.cfg.head_dim)
+
+    def attends_into_o(self):
+        """Every context takes the one form of the attention whose shares o's matvec reads."""
+        f = self._fused_linears()
+        if not f['o'].takes_shares(self.cfg.head_dim):
+            return False
+        return self.grouped_ok() or (self.fused and f['qkv'].out_transform_fits_attention(self.cfg.head_dim)
+                                     and f['qkv'].SV.dtype == torch.float32)
+
+    def _attend_into_o(self, views, lins, k_cache, v_cache, pos, inv_freq):
+        """o's partial sums (S, 1, hidden) from those of the q / k / v projections: two launches."""
+        cfg = self.cfg
+        o = self._fused_linears()['o']
+        shares = ops.decode_attention_shares(views, [l.SV for l in lins], [(l.m**-0.5) * 32.0 for l in lins], [l.br for l in lins],
+                                             [l.Kr for l in lins], k_cache, v_cache, pos, inv_freq, cfg.heads, cfg.kv_heads,
+                                             cfg.head_dim)
+        return ops.decompress_matvec_parts_shares(o.trellis, shares, pos, k_cache.shape[-2], o.SU, (o.n**-0.5) / 32.0, o.tlut, o.m,
+                                                  o.n, o.K).unsqueeze(1)
 
     # ---- separate projections (the layout of the published checkpoints) in grouped launches
 
@@ -443,10 +470,13 @@ class DecoderLayer(nn.Module):
         for l in qkv:
             views.append(qkv_parts[:, off:off + l.m])
             off += l.m
-        attn = ops.decode_attention_rht3(views, [l.SV for l in qkv], [(l.m**-0.5) * 32.0 for l in qkv],
-                                         [l.br for l in qkv], [l.Kr for l in qkv], k_cache, v_cache, pos, inv_freq,
-                                         cfg.heads, cfg.kv_heads, cfg.head_dim, key_splits=cfg.attn_key_splits)
-        po = f['o'].matvec_from(attn.reshape(1, -1))
+        if self._o_takes_shares():
+            po = self._attend_into_o(views, qkv, k_cache, v_cache, pos, inv_freq)
+        else:
+            attn = ops.decode_attention_rht3(views, [l.SV for l in qkv], [(l.m**-0.5) * 32.0 for l in qkv],
+                                             [l.br for l in qkv], [l.Kr for l in qkv], k_cache, v_cache, pos, inv_freq,
+                                             cfg.heads, cfg.kv_heads, cfg.head_dim, key_splits=cfg.attn_key_splits)
+            po = f['o'].matvec_from(attn.reshape(1, -1))
         gu_parts, x = self._group_chain(('gate_proj', 'up_proj'), po, f['o'], x, self.post_norm.weight)
         h, pre = self._gate_up_out(gu_parts)
         pd = f['down'].matvec_behind(h, pre)
@@ -623,6 +653,11 @@ class _FusedLinear:
         transforms of one hidden-size vector: one launch does both plus residual and RMSNorm."""
         return (not self.dense and not nxt.dense and self.Kr == 1 and nxt.Kl == 1 and self.m == nxt.n
                 and self.m in (2048, 4096, 8192) and not self.shard_out and not nxt.shard_in)
+
+    def takes_shares(self, head_dim):
+        """The matvec's launch puts the attention's shares together in front of its input transform."""
+        return (not self.dense and not self.shard_in and self.Kl == 1 and self.n in ops.RHT_IN_MATVEC_SIZES and head_dim in (64, 128)
+                and self.SU.dtype == torch.float16 and self.SU.is_contiguous() and self.SU.data_ptr() % 16 == 0)
 
     def can_end_open(self):
         """The token head can do this layer's output transform."""
@@ -868,10 +903,11 @@ def generate(model, prompt_ids, max_new_tokens, use_graph=True, fused=True, temp
             draw_counter.copy_(keep[3])
         return g, nxt
 
-    # the fused attention has two forms (one workgroup per head; key ranges for long contexts): a run
-    # that crosses the line between them records its step again there, so short contexts never pay
+    # the fused attention has two forms where o's matvec does not put the shares of key ranges together (one workgroup per head; key
+    # ranges for long contexts): a run that crosses the line between them records its step again there, so short contexts never pay
     # for the second launch of the long form
-    splits_at = lambda ctx: ops.attention_key_splits(ctx, model.cfg.heads) if fused else 1
+    by_context = fused and not all(layer.attends_into_o() for layer in model.layers)
+    splits_at = lambda ctx: ops.attention_key_splits(ctx, model.cfg.heads) if by_context else 1
     model.cfg.attn_key_splits = splits_at(n + 1)
     graph = static_next = None
     if use_graph:

@@ -737,6 +737,68 @@ def decode_attention_rht3(parts, post, scale, had_bits, order, k_cache, v_cache,
     return out
 
 
+def attention_share_ranges(heads):
+    """Ranges of the keys that decode_attention_shares has room for: as many as leave the chip's 256 CUs a workgroup each."""
+    return max(1, min(4, 256 // heads))
+
+
+def decode_attention_shares(parts, post, scale, had_bits, order, k_cache, v_cache, pos, inv_freq, heads, kv_heads, head_dim):
+    """decode_attention_rht (one-element lists) or _rht3 (three) for decompress_matvec_parts_shares: the shares of the ranges
+    of keys, (heads, ranges, head_dim + 4) fp32, as many of them in use as the position gives."""
+    vectors = len(parts)
+    dev = parts[0].device
+    for i in range(vectors):
+        require_cuda(parts[i], "parts", torch.float32, contiguous=False)
+        require_cuda(post[i], "post", torch.float32)
+        if had_bits[i] is not None:
+            require_cuda(had_bits[i], "had_bits", torch.int32)
+        n = (heads + 2 * kv_heads if vectors == 1 else heads if i == 0 else kv_heads) * head_dim
+        if parts[i].dim() != 2 or parts[i].shape[1] != n or parts[i].stride(1) != 1 \
+                or parts[i].shape[0] != parts[0].shape[0] or parts[i].stride(0) != parts[0].stride(0) \
+                or post[i].numel() != n or (order[i] > 1 and had_bits[i] is None):
+            raise ValueError("decode_attention_shares: inconsistent shapes")
+    require_cuda(k_cache, "k_cache", torch.float16)
+    require_cuda(v_cache, "v_cache", torch.float16)
+    require_cuda(pos, "pos", torch.int64)
+    require_cuda(inv_freq, "inv_freq", torch.float32)
+    max_len = k_cache.shape[-2]
+    if k_cache.numel() != kv_heads * max_len * head_dim or v_cache.shape != k_cache.shape \
+            or inv_freq.numel() != head_dim // 2 or pos.numel() != 1:
+        raise ValueError("decode_attention_shares: inconsistent shapes")
+    ranges = attention_share_ranges(heads)
+    shares = torch.empty((heads, ranges, head_dim + 4), dtype=torch.float32, device=dev)
+    vp = lambda ts: (ctypes.c_void_p * vectors)(*[t.data_ptr() if t is not None else None for t in ts])
+    with _on(dev):
+        check(lib().qtip_decode_attention_shares(_ptr(shares), ranges, vectors, vp(parts), parts[0].shape[0], parts[0].stride(0),
+                                                 vp(post), (ctypes.c_float * vectors)(*[float(v) for v in scale]), vp(had_bits),
+                                                 (ctypes.c_int * vectors)(*[int(v) for v in order]), _ptr(k_cache), _ptr(v_cache),
+                                                 _ptr(pos), _ptr(inv_freq), heads, kv_heads, head_dim, max_len, stream_ptr(dev)),
+              "qtip_decode_attention_shares")
+    return shares
+
+
+def decompress_matvec_parts_shares(packed, shares, pos, max_len, su, scale, tlut, m, k, bits, nparts=None):
+    """decompress_matvec_parts_rht on the attention output that the shares of decode_attention_shares give, with the position and
+    the cache slots of that call."""
+    _check_packed(packed, m, k, bits)
+    _check_tlut(tlut, packed.device)
+    require_cuda(shares, "shares", torch.float32)
+    require_cuda(su, "su", torch.float16)
+    require_cuda(pos, "pos", torch.int64)
+    heads, ranges, dim = shares.shape[0], shares.shape[1], shares.shape[2] - 4
+    if k not in RHT_IN_MATVEC_SIZES or heads * dim != k or su.numel() != k or pos.numel() != 1:
+        raise ValueError(f"shares and su must be of k = {k} values, k in {RHT_IN_MATVEC_SIZES}")
+    if any(t.device != packed.device for t in (shares, su, pos)):
+        raise ValueError(f"shares, su and pos must be on {packed.device}")
+    S = int(nparts) if nparts is not None else matvec_split(m, k, bits, packed.device)
+    parts = torch.empty((S, m), dtype=torch.float32, device=packed.device)
+    with _on(packed.device):
+        check(lib().qtip_decompress_matvec_parts_shares(_ptr(parts), _ptr(packed), _ptr(shares), ranges, dim, _ptr(pos), max_len,
+                                                        _ptr(su), ctypes.c_float(scale), _ptr(tlut), m, k, bits, S,
+                                                        stream_ptr(packed.device)), "qtip_decompress_matvec_parts_shares")
+    return parts
+
+
 def prefill_attention(q, k, v, cos, sin, k_cache, v_cache, pos, heads, kv_heads, head_dim):
     """Causal attention of n new tokens against the cache, which gets their keys and values first: q (n, heads *
     head_dim), k / v (n, kv_heads * head_dim) fp16 with contiguous rows, cos / sin (n, head_dim) fp16, pos (n,) int64
