@@ -81,3 +81,24 @@ def test_a_callers_own_ranges_keep_their_launch():
         cfg.attn_key_splits = 3
         b = model.decode_fused(tok, pos)
     assert (a - b).norm() <= 4e-3 * a.norm()
+
+
+def test_a_further_request_needs_no_eager_step(monkeypatch):
+    """The step of a further request is recorded at once, and with an eager step again where a layer has been replaced."""
+    cfg = LlamaConfig(hidden=2048, heads=16, kv_heads=4, layers=2, ffn=172 * 32, vocab=512)
+    g = torch.Generator().manual_seed(3)
+    a, b = (torch.randint(0, cfg.vocab, (1, n), generator=g).cuda() for n in (20, 33))
+    model = LlamaDecoder(cfg, max_cache_len=64)
+    steps = []
+    inner = model.decode_fused
+    monkeypatch.setattr(model, "decode_fused", lambda *args, **kw: steps.append(torch.cuda.is_current_stream_capturing()) or
+                        inner(*args, **kw))
+    for ids in (a, b, a):
+        got, _, _ = generate(model, ids, 12)
+        assert torch.equal(got, generate(LlamaDecoder(cfg, max_cache_len=64), ids, 12, use_graph=False)[0])
+    assert steps == [False, True, True, True]
+    del steps[:]
+    model.layers[1] = LlamaDecoder(cfg, max_cache_len=64).layers[1]
+    assert torch.equal(generate(model, a, 12)[0], got) and steps == [False, True]
+    drawn = [generate(model, b, 12, temperature=0.7, top_k=4)[0] for _ in range(2) if torch.manual_seed(7)]
+    assert torch.equal(*drawn)
