@@ -5,6 +5,7 @@
 
 #include "../../include/qtip_hip.h"
 #include "qtip_setup.h"
+#include "qtip_wht.h"
 
 namespace {
 
@@ -81,17 +82,24 @@ __global__ __launch_bounds__(kBlock) void cache_rows_kernel(
 // were up to 1.013 times as far from float64 as the library's attention (2.38e-4 and 2.35e-4 at 150 tokens of 32
 // heads of 128), with two they are the correctly rounded ones (1.96e-4).  The rests have accumulators of their own: an
 // infinite value times a rest of zero is a NaN where times the probability it is infinite, and is left out.
-// Bound by a wave's chain through a tile (products, maximum, exponentials, products): the latest queries
-// run first, and 16-query waves give two workgroups per CU at 1000 tokens of 32 heads.  us, 1000 tokens, 32
-// heads of 128: 45 (42 with one fp16 number per probability) and 8 for the caches, where the library's attention
-// under a dense mask took 193 beside about 150 of small passes (rotation, cache writes, copies of heads).
+// Bound by a wave's chain through a tile (products, maximum, exponentials, products), and 16-query waves give two workgroups
+// per CU at 1000 tokens of 32 heads: so it matters which two.  With a head's workgroups side by side an XCD had those of two lengths
+// only, 2.4 times as many keys as another, and a CU two of the same length.  us, 1000 tokens, 32 heads of 128: 46.7, in the order
+// below, with no mask where every key is seen and no product where the maximum stays, 36.8; and 8 for the caches, where the
+// library's attention under a dense mask took 193 beside about 150 of small passes (rotation, cache writes, copies of heads).
 constexpr int kQ = 64, kKeys = 64;
+
+// the larger of v and lane ^ 16 (b = 4) or lane ^ 32 (5)
+__device__ __forceinline__ float lane_max(float v, int b) {
+  const auto s = qtip_wht::lane_pair(v, b);
+  return fmaxf(s.x, s.y);
+}
 
 template <int HD>
 __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
     _Float16* __restrict__ out, const _Float16* __restrict__ q, int q_stride, const _Float16* __restrict__ cos_t,
     const _Float16* __restrict__ sin_t, const _Float16* __restrict__ k_cache, const _Float16* __restrict__ v_cache,
-    const int64_t* __restrict__ pos, int n, int heads, int group, int slots, float scale_log2) {
+    const int64_t* __restrict__ pos, int n, int heads, int group, int slots, float scale_log2, int turn) {
   constexpr int KSTR = HD * 2 + 16, VSTR = kKeys * 2 + 16;  // bytes per key, per dim
   constexpr int NS = HD / 32, NE = HD / 16;                 // K steps of the scores, dim tiles
   constexpr int CPK = HD / 8;                               // 16-byte chunks per key
@@ -100,7 +108,10 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
   __shared__ __align__(16) uint8_t lds_v[HD * VSTR];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ql = lane & 15, g = lane >> 4;
-  const int h = blockIdx.y, qt = gridDim.x - 1 - blockIdx.x;
+  // rank 0 has the most keys; heads side by side, so that an XCD (every eighth workgroup) has the same mix of ranks as the others
+  // and, of eight heads or a multiple, heads of its own
+  const int id = blockIdx.x, rank = id < turn ? id : (int)gridDim.x - 1 - (id - turn);
+  const int h = rank % heads, qt = ((int)gridDim.x - 1 - rank) / heads;
   const size_t head = (size_t)(h / group) * slots * HD;
   const _Float16* kc = k_cache + head;
   const _Float16* vc = v_cache + head;
@@ -192,24 +203,31 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
     }
     float tile_max = mx;
 #pragma unroll
+    for (int t = 0; t < 4; ++t) s[t] *= scale_log2;
+    if (__any(kk0 + kKeys - 1 > limit)) {  // (a tile that every query of the wave sees all of needs no mask)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (kk0 + 16 * t + 4 * g + r > limit) s[t][r] = -__builtin_inff();
+    }
+#pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float x = s[t][r] * scale_log2;
-        s[t][r] = kk0 + 16 * t + 4 * g + r <= limit ? x : -__builtin_inff();
-        tile_max = fmaxf(tile_max, s[t][r]);
-      }
-    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16));
-    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
+      for (int r = 0; r < 4; ++r) tile_max = fmaxf(tile_max, s[t][r]);
+    tile_max = lane_max(tile_max, 4);
+    tile_max = lane_max(tile_max, 5);
     const float base = fmaxf(tile_max, -3.0e38f);  // (nothing but scores of -inf so far)
-    const float fade = __builtin_amdgcn_exp2f(mx - base);
-    mx = tile_max;
-    sum *= fade;
+    if (__any(tile_max != mx)) {  // (a maximum that stays leaves the outputs as they are)
+      const float fade = __builtin_amdgcn_exp2f(mx - base);
+      sum *= fade;
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      o[e] *= fade;
-      rest_o[e] *= fade;
+      for (int e = 0; e < NE; ++e) {
+        o[e] *= fade;
+        rest_o[e] *= fade;
+      }
     }
+    mx = tile_max;
     half8v p[2], rest[2];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -234,8 +252,8 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
         for (int e = 0; e < 4; ++e) rest_o[e0 + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[e], rest[kk], rest_o[e0 + e], 0, 0, 0);
       }
   }
-  sum += __shfl_xor(sum, 16);
-  sum += __shfl_xor(sum, 32);
+  sum = qtip_wht::lane_add(sum, 4);
+  sum = qtip_wht::lane_add(sum, 5);
   const float inv = 1.f / sum;
 #pragma unroll
   for (int e = 0; e < NE; ++e)
@@ -301,14 +319,18 @@ extern "C" int qtip_prefill_attention(void* out_f16, const void* q_f16, const vo
       kc, vc, (const _Float16*)k_f16, (const _Float16*)v_f16, k_stride, v_stride, c, s, pos, n, kv_heads, head_dim, slots);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
-  const dim3 grid((unsigned)((n + kQ - 1) / kQ), (unsigned)heads);
+  const long wgs = (long)((n + kQ - 1) / kQ) * heads;
+  const dim3 grid((unsigned)wgs);
+  // Two workgroups a CU at most: the second ones come shortest first, beside the longest (32 heads, 1000 tokens: 16 tiles of keys
+  // and 1 to 9 and 8).  More of them take the place of those that end, longest first.
+  const int cus = qtip_device_cus(), turn = cus > 0 && wgs <= 2L * cus ? cus : (int)wgs;
   const int group = heads / kv_heads;
   const float log2e = 1.44269504088896340736f;
   if (head_dim == 128)
     prefill_attn_kernel<128><<<grid, kBlock, 0, st>>>((_Float16*)out_f16, (const _Float16*)q_f16, q_stride, c, s, kc, vc, pos,
-                                                      n, heads, group, slots, log2e * 0.08838834764831845f);
+                                                      n, heads, group, slots, log2e * 0.08838834764831845f, turn);
   else
     prefill_attn_kernel<64><<<grid, kBlock, 0, st>>>((_Float16*)out_f16, (const _Float16*)q_f16, q_stride, c, s, kc, vc, pos,
-                                                     n, heads, group, slots, log2e * 0.125f);
+                                                     n, heads, group, slots, log2e * 0.125f, turn);
   return (int)hipGetLastError();
 }

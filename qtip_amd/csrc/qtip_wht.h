@@ -78,18 +78,24 @@ __device__ __forceinline__ float wht_places(float v, int nbits, int place, int l
   return v;
 }
 
+// a lane's value and that of lane ^ 16 (b = 4) or lane ^ 32 (5), the lower lane's first
+__device__ __forceinline__ float2 lane_pair(float v, int b) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  auto sw = b == 4 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return float2{__builtin_bit_cast(float, (uint32_t)sw[0]), __builtin_bit_cast(float, (uint32_t)sw[1])};
+}
+__device__ __forceinline__ float lane_add(float v, int b) {
+  const float2 s = lane_pair(v, b);
+  return s.x + s.y;
+}
+
 // the sum over the lanes of a wave (four lanes hold the same sum when eight are mirrored)
 __device__ __forceinline__ float wave_sum(float v) {
   v += lane_xor(v, 0);
   v += lane_xor(v, 1);
   v += half_mirror(v);
   v += lane_xor(v, 3);
-  const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  auto s16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = __builtin_bit_cast(float, (uint32_t)s16[0]) + __builtin_bit_cast(float, (uint32_t)s16[1]);
-  const uint32_t t = __builtin_bit_cast(uint32_t, v);
-  auto s32 = __builtin_amdgcn_permlane32_swap(t, t, false, false);
-  return __builtin_bit_cast(float, (uint32_t)s32[0]) + __builtin_bit_cast(float, (uint32_t)s32[1]);
+  return lane_add(lane_add(v, 4), 5);
 }
 // the sum of values that a workgroup's 16 waves left in LDS, the same in every lane
 __device__ __forceinline__ float waves16_sum(const float* w, int lane) {
