@@ -276,8 +276,7 @@ __device__ __forceinline__ T* pick3(T* const (&a)[3], int g) {
 // barriers per launch instead of x travelling through vector loads with every wave-load, which
 // made the 28672-wide matrices 15-20 % slower).
 // HALF: the row blocks that do not fill a last round of whole units (at most half a round of
-// them) are cut by row half instead: workgroup w < upw_r takes the rows with rh = w % 2 of row
-// block upw_q * rb_step + w / 2 after its upw_q whole units.  Such a half unit reads the block's
+// them) are cut by row half instead: a workgroup w < upw_r takes the rows of one rh of one of them after its upw_q whole units.  Such a half unit reads the block's
 // whole stream but decodes half of its states (about 0.55 of a unit's time), and its rows are
 // complete sums, so nothing has to be combined across workgroups: 320 row blocks on 256
 // workgroups take 1.55 units of time instead of 2, 128 row blocks 0.55 instead of 1.
@@ -345,8 +344,13 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
   const int upw = HALF ? upw_q : upw_q + (rb0 < upw_r ? 1 : 0);
   const int T_full = upw * npw;
   const bool has_half = HALF && rb0 < upw_r;
-  const int half_rh = rb0 & 1;
-  const int half_rb = upw_q * rb_step + (rb0 >> 1);
+  // Nothing but half units: the two of a block on one XCD (workgroups go round the eight of them), where the second reading of
+  // its stream hits in L2; the last ones, less than a round of pairs, side by side.  Behind whole units they lie side by side too: a
+  // pair on one XCD starts together and is 1 % slower.
+  const int lg = upw_q ? 0 : (gridDim.x == 1 ? 3 : (gridDim.x == 2 ? 2 : (gridDim.x == 4 ? 1 : 0)));
+  const bool paired = rb0 < (upw_r >> (lg + 1)) << (lg + 1);
+  const int half_rh = (paired ? rb0 >> lg : rb0) & 1;
+  const int half_rb = upw_q * rb_step + (paired ? ((rb0 >> (lg + 1)) << lg) + (rb0 & ((1 << lg) - 1)) : rb0 >> 1);
   const int T = T_full + (has_half ? npw : 0);
   const int w_first = wl0 + wave;
   const int nvj = w_first < wl1f ? (wl1f - w_first + kWaves - 1) / kWaves : 0;  // real items per unit
@@ -737,6 +741,8 @@ hipError_t allow_lds_all() {
   QTIP_ALLOW((matvec_kernel<3, 2, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<4, 2, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<2, 2, true, 0, false, false, true>), kMatvecLds + kMatvecXBytes)
+  QTIP_ALLOW((matvec_kernel<3, 2, true, 0, false, false, true>), kMatvecLds + kMatvecXBytes)
+  QTIP_ALLOW((matvec_kernel<4, 2, true, 0, false, false, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<2, 2, true, 0, false, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<3, 2, true, 0, false, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<4, 2, true, 0, false, true>), kMatvecLds + kMatvecXBytes)
@@ -981,9 +987,11 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
   // the whole ones in the same two-stage load pipeline, so the whole units must end on an even
   // item.  Measured at 2 bits: 10240x8192 11.1 -> 9.8 us, 12288x4096 7.15 -> 6.6 us, and matrices
   // that do not fill one round - 4096x4096 4.8 -> 4.55 us, 4096x11008 7.9 -> 6.9 us (half the
-  // decode per workgroup on twice the workgroups).  At 3 and 4 bits the doubled stream of the
-  // left-over blocks costs what the halved decode saves (slower on the 4096-wide matrices, 2-4 %
-  // faster on 10240x8192 only), so those keep whole units.
+  // decode per workgroup on twice the workgroups), 6.8 -> 6.5 with both halves of a block on one XCD.
+  // At 3 and 4 bits the left-over blocks behind whole units stay whole: the doubled stream costs what the halved decode saves
+  // (12288x4096 at 3 bits 7.8 / 8.0).  Matrices that do not fill one round, us, whole units / halves on one XCD, 3 and 4 bits: 4096x11008
+  // 8.65 / 8.2 and 8.9 / 8.4, 4096x14336 10.3 / 10.0 and 10.3 / 9.8, 2048x5504 5.9 / 5.7 and 5.9 / 5.4, 1024x8192 7.2 / 6.3 and
+  // 6.75 / 5.6; 4096x4096 5.16 / 5.24 and 5.4 / 5.3, so at 3 bits from three wave-loads a wave on.
   const int full_range = di.cus / S;
   const int left = full_range > 0 ? (m >> 5) % full_range : 0;
   const int whole = full_range > 0 ? (m >> 5) / full_range : 0;
@@ -1012,10 +1020,15 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
 #undef QTIP_MIX
     return (int)hipGetLastError();
   }
-  if (bits == 2 && xbytes <= kMatvecXBytes && left > 0 && 2 * left <= full_range && (whole == 0 || even_items)) {
+  const bool half = whole > 0 ? bits == 2 && even_items : bits != 3 || wl_per > 2 * kWaves;
+  if (xbytes <= kMatvecXBytes && left > 0 && 2 * left <= full_range && half) {
     const dim3 gh((unsigned)S, (unsigned)(whole > 0 ? full_range : 2 * left));
-    matvec_kernel<2, 2, true, 0, false, false, true><<<gh, kThreads, kMatvecLds + xbytes, st>>>(
-        dst, p, xx, t, m, k, wl_per, whole, 2 * left);
+    const size_t lds = kMatvecLds + xbytes;
+    switch (bits) {
+      case 2: matvec_kernel<2, 2, true, 0, false, false, true><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, 2 * left); break;
+      case 3: matvec_kernel<3, 2, true, 0, false, false, true><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, 2 * left); break;
+      default: matvec_kernel<4, 2, true, 0, false, false, true><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, 2 * left); break;
+    }
     return (int)hipGetLastError();
   }
   if (xbytes <= kMatvecXBytes) {

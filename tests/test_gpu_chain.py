@@ -90,3 +90,19 @@ def test_table_transform_refusals():
     packed, tlut, _ = _matrix(32, 11008, 2, torch.Generator(device="cuda").manual_seed(0))
     with pytest.raises(ValueError):
         ops.decompress_matvec_parts_mix(packed, z, z, 1.0, torch.zeros(171, 8, dtype=torch.int32, device="cuda"), 172, tlut, 32, 11008, 2)
+
+
+# row blocks that fill less than half of the chip: pairs of halves on one XCD and side by side, one to four ranges of k
+@pytest.mark.parametrize("bits", (2, 3, 4))
+@pytest.mark.parametrize("m,k,ranges", ((32, 4224, 1), (288, 8192, 1), (4096, 4608, 1), (256, 8192, 2), (160, 8320, 3), (1024, 16384, 4)))
+def test_half_units_of_matrices_that_do_not_fill_the_chip(m, k, ranges, bits):
+    """Every row once: sums of k exact products in fp32 against float64 (a chain of k / 64 on the matrix cores and 16 waves)."""
+    g = torch.Generator(device="cuda").manual_seed(m + k + bits)
+    packed, tlut, w = _matrix(m, k, bits, g)
+    x = torch.randn(k, generator=g, device="cuda").half()
+    got = ops.decompress_matvec_parts(packed, x, tlut, m, k, bits, ranges).double().sum(0)
+    want, size = w @ x.double(), w.abs() @ x.double().abs()
+    assert ((got - want).abs() <= size * (k / 64 + 24) * 2.0**-24).all()
+    if ranges == 1:
+        one = ops.decompress_matvec(packed, x, tlut, m, k, bits).reshape(-1).double()
+        assert ((one - want).abs() <= size * (k / 64 + 24) * 2.0**-24).all()
