@@ -455,7 +455,7 @@ class DecoderLayer(nn.Module):
         previous layer, or the first for itself), attention with the three output transforms in its prologue, o matvec with
         its input transform, [boundary + gate, up matvecs], both output transforms (with SiLU * up in
         the same launch for vectors above 4096), [SiLU * up +] input transform of down, down
-        matvec.  Returns (x, partial sums of the next layer's q, k, v)."""
+        matvec; 7 where down's matvec transforms its input itself.  Returns (x, partial sums of the next layer's q, k, v)."""
         cfg = self.cfg
         f = self._fused_linears()
         qkv = [f[n] for n in ('q_proj', 'k_proj', 'v_proj')]
