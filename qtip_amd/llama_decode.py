@@ -255,7 +255,15 @@ class DecoderLayer(nn.Module):
             names = ('qkv', 'o', 'up_gate', 'down') if self.fused else \
                 ('q_proj', 'k_proj', 'v_proj', 'o', 'gate_proj', 'up_proj', 'down')
             self._fused = {n: _FusedLinear(getattr(self, n)) for n in names}
+            self._recorded = set()
         return self._fused
+
+    def recorded_forms(self):
+        """Forms of decode_fused that have been recorded into a graph with the set-up that the layer keeps, all of which exists
+        behind this call: dropped set-up is made anew, outside of a recording, and with no form."""
+        self._fused_linears()
+        self.grouped_ok() or self.grouped_plain_ok()
+        return self.__dict__.setdefault('_recorded', set())  # (a layer from a file may have set-up alone)
 
     def decode_fused(self, x, k_cache, v_cache, pos, inv_freq, qkv_parts=None, next_layer=None, open_end=False):
         """One new token, x (1, hidden) fp16, on the fused transforms: 12 launches for the fused
@@ -822,6 +830,9 @@ def sample(logits, temperature=1.0, top_k=None):
     return torch.argmax(probs / q, dim=-1, keepdim=True), probs
 
 
+_PROCESS = object()  # (part of a recorded form, which a copy or a file of a layer brings along: it is equal to itself alone)
+
+
 @torch.no_grad()
 def generate(model, prompt_ids, max_new_tokens, use_graph=True, fused=True, temperature=None, top_k=None,
              callback=None):
@@ -881,9 +892,10 @@ def generate(model, prompt_ids, max_new_tokens, use_graph=True, fused=True, temp
         """The step recorded into a graph, behind an eager step (allocations, set-up) where one of the layers has not had this form
         of it recorded yet; the decode state is put back afterwards, so a capture in the middle of a run leaves it untouched."""
         # What an eager step sets up stays with the layers and the process; recording runs nothing.  A further request on a
-        # model of 8 layers of 4096 starts 1.6 ms earlier for it.
-        form = (sampling, model.cfg.attn_key_splits, dev)
-        ready = on_device and all(form in layer.__dict__.get("_recorded", ()) for layer in model.layers)
+        # model of 8 layers of 4096 starts 1.6 ms earlier for it.  (Only a layer of this module tells what it keeps.)
+        form = (sampling, model.cfg.attn_key_splits, dev, _PROCESS)
+        own = [layer for layer in model.layers if type(layer) is DecoderLayer and 'decode_fused' not in layer.__dict__]
+        ready = on_device and len(own) == len(model.layers) and all(form in layer.recorded_forms() for layer in own)
         keep = (static_tok.clone(), static_pos.clone(), history.clone(), draw_counter.clone())
 
         def restore():
@@ -903,24 +915,14 @@ def generate(model, prompt_ids, max_new_tokens, use_graph=True, fused=True, temp
             # the warm-up wrote the cache slot of the current position with this token's k/v, which the
             # next step rewrites identically
 
-        def record():
-            g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
-                nxt = step()
-            return g, nxt
-
         if not ready:
             eager()
-        try:
-            g, nxt = record()
-        except RuntimeError:
-            if not ready:
-                raise
-            eager()  # (something has been replaced since, and is set up by a step that runs)
-            g, nxt = record()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            nxt = step()
         if on_device:
-            for layer in model.layers:
-                layer.__dict__.setdefault("_recorded", set()).add(form)
+            for layer in own:
+                layer.recorded_forms().add(form)
             restore()  # (capture only records; in case the stream ran anything)
         return g, nxt
 
