@@ -802,11 +802,13 @@ class LlamaDecoder(nn.Module):
             end = head and nxt is None and type(layer) is DecoderLayer and 'decode_fused' not in layer.__dict__
             x, qp = layer.decode_fused(x, self.k_cache[i], self.v_cache[i], pos, self.inv_freq, qp, nxt,
                                        **({'open_end': True} if end else {}))
+        d = layer._fused_linears()['down'] if head and end and qp is not None else None  # (the last layer's end is open)
         if head and self._head_launches(x):
-            d, qp = (layer._fused_linears()['down'], qp) if end and qp is not None else (None, None)
-            return ops.token_head(self.lm_head, x, self.norm.weight, self.norm.eps, qp, None if d is None else d.SV,
-                                  0.0 if d is None else (d.m**-0.5) * 32.0,
+            return ops.token_head(self.lm_head, x, self.norm.weight, self.norm.eps, qp if d is not None else None,
+                                  None if d is None else d.SV, 0.0 if d is None else (d.m**-0.5) * 32.0,
                                   torch.float32 if float_logits else torch.float16).reshape(1, 1, -1)
+        if d is not None:
+            x = d.transform_out(qp, residual=x)
         x = ops.rmsnorm(x, self.norm.weight, self.norm.eps)
         lg = (x @ self.lm_head.T).reshape(1, 1, -1)
         return lg.float() if float_logits else lg
