@@ -784,7 +784,7 @@ class LlamaDecoder(nn.Module):
             and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (h, w, x))
                 and h.dim() == 2 and 0 < h.shape[0] < 2**30 and w.shape == h.shape[1:] == x.shape[1:] and h.shape[1] % 8 == 0
                 and h.shape[1] <= ops.TOKEN_HEAD_MAX and not (torch.is_grad_enabled() and h.requires_grad)
-                and ops.launchable(h, w, x))
+                and not torch.is_autocast_enabled("cuda") and ops.launchable(h, w, x))
 
     def decode_fused(self, tok, pos, float_logits=True):
         """tok (1,1) int64, pos (1,) int64 device tensors -> logits (1, 1, vocab), fused kernels;

@@ -26,3 +26,17 @@ def test_a_head_that_does_not_launch_reads_the_whole_stream(fused, answers, monk
         got = model.decode_fused(tok, pos)
     assert next(asked, None) is None
     assert (got - want).norm() <= 8e-4 * want.norm()
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+def test_autocast_casts_the_output_matrix(dtype):
+    """A region of autocast computes the product of the output matrix in its own type, as it does for the module's prompt."""
+    model, tok, pos = _step(True)
+    with torch.no_grad():
+        plain = model.decode_fused(tok, pos)
+        with torch.autocast("cuda", dtype=dtype):
+            got = model.decode_fused(tok, pos)
+            assert model.decode_fused(tok, pos, float_logits=False).dtype == dtype
+    assert got.dtype == torch.float32 and torch.equal(got, got.to(dtype).float())
+    # two roundings of the norm and one of the result
+    assert (got - plain).norm() <= (1e-3 if dtype == torch.float16 else 8e-3) * plain.norm()
