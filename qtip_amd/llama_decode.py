@@ -577,11 +577,19 @@ class _FusedLinear:
         self.Kl, self.Kr = lin.K_left, lin.K_right
         self.bl = had_bits(lin.had_left, self.Kl, True, dev) if self.Kl > 1 else None
         self.br = had_bits(lin.had_right, self.Kr, False, dev) if self.Kr > 1 else None
-        # the table of an input transform that runs in front of the matvec, in its launch
-        cols = 0
-        if dev.type == "cuda" and not self.shard_in:
-            cols = ops.matvec_mix_columns(self.n, self.Kl, ops.matvec_split(self.m, self.n, self.K, dev))
-        self.mix_rows = sign_rows(self.bl, self.Kl, self.n // cols // self.Kl, dev) if cols else None
+        self._mix_rows = ()  # (not asked for yet)
+
+    def mix_rows(self):
+        """The table of an input transform that runs in front of the matvec, in its launch, or None: made when the first matvec
+        reads it.  A copy from host memory has no place in a recording, which goes without where no step ran before."""
+        if type(self._mix_rows) is tuple:
+            dev, cols = self.trellis.device, 0
+            if dev.type == "cuda" and not self.shard_in:
+                if torch.cuda.is_current_stream_capturing():
+                    return None
+                cols = ops.matvec_mix_columns(self.n, self.Kl, ops.matvec_split(self.m, self.n, self.K, dev))
+            self._mix_rows = sign_rows(self.bl, self.Kl, self.n // cols // self.Kl, dev) if cols else None
+        return self._mix_rows
 
     def _dense(self, x, pre_mode, norm_weight, eps, residual):
         if pre_mode == ops.PRE_RMSNORM:
@@ -618,9 +626,9 @@ class _FusedLinear:
                 and self.SU.dtype == torch.float16 and not self.shard_in):
             return ops.decompress_matvec_parts_rht(self.trellis, x.reshape(-1), self.SU, (self.n**-0.5) / 32.0,
                                                    self.tlut, self.m, self.n, self.K).unsqueeze(1)
-        if (self.mix_rows is not None and x.dtype == self.SU.dtype == torch.float16 and self.SU.is_contiguous()
-                and x.data_ptr() % 16 == self.SU.data_ptr() % 16 == 0):
-            return ops.decompress_matvec_parts_mix(self.trellis, x.reshape(-1), self.SU, (self.n**-0.5) / 32.0, self.mix_rows,
+        if (x.dtype == self.SU.dtype == torch.float16 and self.SU.is_contiguous()
+                and x.data_ptr() % 16 == self.SU.data_ptr() % 16 == 0 and self.mix_rows() is not None):
+            return ops.decompress_matvec_parts_mix(self.trellis, x.reshape(-1), self.SU, (self.n**-0.5) / 32.0, self.mix_rows(),
                                                    self.Kl, self.tlut, self.m, self.n, self.K).unsqueeze(1)
         return self.matvec(self.transform_in(x))
 

@@ -65,9 +65,9 @@ def _pack_bits(neg):
 
 def sign_rows(bits, K, A, device):
     """Signs of (table (x) H_A), K * A <= 256 rows of 8 words with bit j of row i set for -1, from the table's `bits` as had_bits
-    returns them (None for K = 1); kept for the built-in tables."""
+    returns them (None for K = 1); kept for the built-in tables and K = 1."""
     dev = torch.device(device)
-    own = [t for t in (False, True) if bits is not None and bits is _bit_cache.get((K, t, dev))]
+    own = [None] if bits is None else [t for t in (False, True) if bits is _bit_cache.get((K, t, dev))]
     key = ("rows", K, A, own[0], dev) if own else None
     if key in _bit_cache:
         return _bit_cache[key]

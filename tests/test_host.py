@@ -507,3 +507,12 @@ def test_sign_rows_of_a_table(K, A, transpose):
     full = np.kron(np.where(neg.T if transpose else neg, -1, 1), hadamard(A)) < 0
     bits = np.unpackbits(rows.numpy().view(np.uint8).reshape(K * A, 32), axis=1, bitorder="little").astype(bool)
     assert np.array_equal(bits[:, :K * A], full) and not bits[:, K * A:].any()
+
+
+def test_sign_rows_are_made_once():
+    """Also for transforms without a table."""
+    from qtip_amd.utils import matmul_had as mh
+    for K, A in ((1, 32), (12, 4)):
+        bits = mh.had_bits(None, K, True, "cpu") if K > 1 else None
+        assert mh.sign_rows(bits, K, A, "cpu") is mh.sign_rows(bits, K, A, "cpu")
+    assert not torch.equal(mh.sign_rows(None, 1, 32, "cpu")[:256], mh.sign_rows(None, 1, 64, "cpu")[:256])

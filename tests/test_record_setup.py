@@ -7,7 +7,7 @@ import types
 import pytest
 import torch
 
-from qtip_amd import ops
+from qtip_amd import llama_decode, ops
 from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder, generate
 
 SETUP = ("_fused", "_grouped", "_grouped_plain")
@@ -139,3 +139,37 @@ def test_requests_on_dropped_set_up(cfg, names):
     if cfg.hidden == 1280:
         for layer in model.layers:
             assert torch.equal(layer._su_qkv, torch.stack([layer.q_proj.SU, layer.k_proj.SU, layer.v_proj.SU]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fused", (True, False))
+def test_sign_tables_are_made_where_a_matvec_reads_them(fused, monkeypatch):
+    """Of a layer with a power-of-two hidden size and a table order behind it: down's alone."""
+    cfg = LlamaConfig(hidden=2048, heads=16, kv_heads=4, layers=2, ffn=172 * 32, vocab=96)
+    model = LlamaDecoder(cfg, max_cache_len=64, fused=fused)
+    made, inner = [], llama_decode.sign_rows
+    monkeypatch.setattr(llama_decode, "sign_rows", lambda bits, K, A, dev: made.append(K) or inner(bits, K, A, dev))
+    generate(model, torch.zeros(1, 20, dtype=torch.int64, device="cuda"), 4)
+    assert made == [172] * cfg.layers
+
+
+@pytest.mark.gpu
+def test_a_step_recorded_behind_a_prompt():
+    """A prompt sets up the tables of the transforms, which is all that a recording of the step copies from host memory; it goes
+    without the sign tables of the transforms inside matvecs and is replayed beside steps that have them."""
+    cfg = LlamaConfig(hidden=2048, heads=16, kv_heads=4, layers=2, ffn=172 * 32, vocab=96)
+    model = LlamaDecoder(cfg, max_cache_len=64)
+    ids = torch.randint(0, cfg.vocab, (1, 20), generator=torch.Generator().manual_seed(3)).cuda()
+    tok, pos = torch.zeros(1, 1, dtype=torch.int64, device="cuda"), torch.tensor([20], device="cuda")
+    with torch.no_grad():
+        model(ids, torch.arange(20, device="cuda"))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = model.decode_fused(tok, pos)
+        for t in (3, 50, 3):
+            tok.fill_(t)
+            graph.replay()
+            want = model.decode_fused(tok, pos)
+            torch.cuda.synchronize()
+            # (down's input transform may give the neighbouring value in fp16)
+            assert (got - want).norm() <= 2.5e-3 * want.norm()
