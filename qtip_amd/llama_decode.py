@@ -939,7 +939,10 @@ def generate(model, prompt_ids, max_new_tokens, use_graph=True, fused=True, temp
     # the fused attention has two forms where o's matvec does not put the shares of key ranges together (one workgroup per head; key
     # ranges for long contexts): a run that crosses the line between them records its step again there, so short contexts never pay
     # for the second launch of the long form
-    by_context = fused and not all(layer.attends_into_o() for layer in model.layers)
+    # (anyone's own step of a layer may have its own attention, which goes by cfg.attn_key_splits)
+    own_step = lambda layer: (getattr(type(layer), 'decode_fused', None) is DecoderLayer.decode_fused
+                              and 'decode_fused' not in layer.__dict__)
+    by_context = fused and not all(own_step(layer) and layer.attends_into_o() for layer in model.layers)
     splits_at = lambda ctx: ops.attention_key_splits(ctx, model.cfg.heads) if by_context else 1
     model.cfg.attn_key_splits = splits_at(n + 1)
     graph = static_next = None

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from qtip_amd import llama_decode, ops
-from qtip_amd.llama_decode import LlamaConfig, LlamaDecoder, generate
+from qtip_amd.llama_decode import DecoderLayer, LlamaConfig, LlamaDecoder, generate
 
 SETUP = ("_fused", "_grouped", "_grouped_plain")
 TABLE_ORDER = dict(hidden=1280, heads=20, kv_heads=20, layers=2, ffn=832, vocab=96)  # 1280 = 20 * 64, stacked sign vectors
@@ -89,6 +89,41 @@ def test_a_step_of_someones_own_layers_runs_before_it_is_recorded(steps):
         del steps.seen[:]
         generate(model, torch.zeros(1, 4, dtype=torch.int64), 1)
         assert [recording for recording, _ in steps.seen] == [False, True]
+
+
+class _Foreign(torch.nn.Module):
+    """A layer that brings what the fused step asks of one, and no more."""
+    fused = False
+
+    def _fused_linears(self):
+        return {}
+
+    def grouped_ok(self):
+        return False
+
+    grouped_plain_ok = grouped_ok
+
+
+class _OwnStep(DecoderLayer):
+    def decode_fused(self, *args, **kw):
+        raise NotImplementedError
+
+
+class _OwnForward(DecoderLayer):
+    pass
+
+
+@pytest.mark.parametrize("kind,ranges", ((None, 1), (_Foreign, 8), (_OwnStep, 8), (_OwnForward, 1)))
+def test_key_ranges_of_someones_own_layers_go_by_the_context(steps, kind, ranges):
+    """Only the step of this module's layers cuts the keys by the position."""
+    model = _host_model(steps, POWER_OF_2)
+    model.max_cache_len = 2048
+    if kind is _Foreign:
+        model.layers[1] = kind()
+    elif kind is not None:
+        model.layers[1].__class__ = kind
+    generate(model, torch.zeros(1, ops.ATTN_SPLIT_FROM, dtype=torch.int64), 1, use_graph=False)
+    assert model.cfg.attn_key_splits == ranges
 
 
 @pytest.mark.parametrize("through", (copy.deepcopy, lambda layers: pickle.loads(pickle.dumps(layers))))
