@@ -10,6 +10,7 @@
 
 #include "../../include/qtip_hip.h"
 #include "qtip_device.h"
+#include "qtip_matvec_half.h"
 #include "qtip_setup.h"
 #include "qtip_shares.h"
 #include "qtip_wht.h"
@@ -982,33 +983,24 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
     return (int)hipGetLastError();
   }
   const size_t xbytes = (size_t)wl_per * 256;
-  // row blocks left over by the rounds of whole units, when they fill at most half a round of the
-  // full grid: each is cut into its two row halves (see HALF at the kernel).  The half units follow
-  // the whole ones in the same two-stage load pipeline, so the whole units must end on an even
-  // item.  Measured at 2 bits: 10240x8192 11.1 -> 9.8 us, 12288x4096 7.15 -> 6.6 us, and matrices
-  // that do not fill one round - 4096x4096 4.8 -> 4.55 us, 4096x11008 7.9 -> 6.9 us (half the
-  // decode per workgroup on twice the workgroups), 6.8 -> 6.5 with both halves of a block on one XCD.
-  // At 3 and 4 bits the left-over blocks behind whole units stay whole: the doubled stream costs what the halved decode saves
-  // (12288x4096 at 3 bits 7.8 / 8.0).  Matrices that do not fill one round, us, whole units / halves on one XCD, 3 and 4 bits: 4096x11008
-  // 8.65 / 8.2 and 8.9 / 8.4, 4096x14336 10.3 / 10.0 and 10.3 / 9.8, 2048x5504 5.9 / 5.7 and 5.9 / 5.4, 1024x8192 7.2 / 6.3 and
-  // 6.75 / 5.6; 4096x4096 5.16 / 5.24 and 5.4 / 5.3, so at 3 bits from three wave-loads a wave on.
+  // row blocks left over by the rounds of whole units may be cut into their row halves
   const int full_range = di.cus / S;
   const int left = full_range > 0 ? (m >> 5) % full_range : 0;
   const int whole = full_range > 0 ? (m >> 5) / full_range : 0;
-  const bool even_items = (((wl_per + kWaves - 1) / kWaves) & 1) == 0;
+  const bool half = half_units(bits, left, whole, full_range, S, wl_per, di.cus);
   if (mix) {
     const int cols = k / mix->on;
     const size_t lds = kMatvecLds + kMatvecXBytes;
     auto* sg = (const uint16_t*)su_f16;
-    const bool half = bits == 2 && left > 0 && 2 * left <= full_range && (whole == 0 || even_items);
-    const dim3 gh = half ? dim3((unsigned)S, (unsigned)(whole > 0 ? full_range : 2 * left)) : g2;
-    const int q = half ? whole : uq, r = half ? 2 * left : ur;
+    const bool halves = half && bits == 2;  // (not measured at 3 and 4)
+    const dim3 gh = halves ? dim3((unsigned)S, (unsigned)(whole > 0 ? full_range : 2 * left)) : g2;
+    const int q = halves ? whole : uq, r = halves ? 2 * left : ur;
 #define QTIP_MIX(BITS, HALF)                                                                                                     \
   if (cols == 64) matvec_kernel<BITS, 2, true, 3, false, false, HALF, 4><<<gh, kThreads, lds, st>>>(                            \
       dst, p, xx, t, m, k, wl_per, q, r, sg, xscale, ChainArgs{}, GroupArgs{}, *mix);                                            \
   else matvec_kernel<BITS, 2, true, 3, false, false, HALF, 2><<<gh, kThreads, lds, st>>>(                                        \
       dst, p, xx, t, m, k, wl_per, q, r, sg, xscale, ChainArgs{}, GroupArgs{}, *mix)
-    if (half) {
+    if (halves) {
       QTIP_MIX(2, true);
     } else {
       switch (bits) {
@@ -1020,8 +1012,7 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
 #undef QTIP_MIX
     return (int)hipGetLastError();
   }
-  const bool half = whole > 0 ? bits == 2 && even_items : bits != 3 || wl_per > 2 * kWaves;
-  if (xbytes <= kMatvecXBytes && left > 0 && 2 * left <= full_range && half) {
+  if (xbytes <= kMatvecXBytes && half) {
     const dim3 gh((unsigned)S, (unsigned)(whole > 0 ? full_range : 2 * left));
     const size_t lds = kMatvecLds + xbytes;
     switch (bits) {
