@@ -30,6 +30,7 @@ namespace {
 
 // kThreads = 1024: 16 waves per workgroup, one workgroup per CU
 constexpr int kMaxSplit = 16;
+constexpr int kApartShift = 16;  // upw_r of half units that lie apart holds their workgroups and, from this bit on, half_apart
 
 __device__ __forceinline__ float dpp_xor1(float v) {
   return __builtin_bit_cast(
@@ -281,7 +282,9 @@ __device__ __forceinline__ T* pick3(T* const (&a)[3], int g) {
 // whole stream but decodes half of its states (about 0.55 of a unit's time), and its rows are
 // complete sums, so nothing has to be combined across workgroups: 320 row blocks on 256
 // workgroups take 1.55 units of time instead of 2, 128 row blocks 0.55 instead of 1.
-template <int K, int DEPTH, bool XLDS, int XFORM = 0, bool XHALF = false, bool GROUP = false, bool HALF = false,
+// HALF = 1: the halves of a block lie side by side, 2: 1 << half_apart workgroups apart, but for the last ones, less than a round of pairs
+// (a form of its own: its dozen scalar instructions in a row in front of the first stream load cost the other 1 to 2 %).
+template <int K, int DEPTH, bool XLDS, int XFORM = 0, bool XHALF = false, bool GROUP = false, int HALF = 0,
           int EPT = 0>
 __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
     float* __restrict__ dst_, const uint8_t* __restrict__ packed_, const uint16_t* __restrict__ x_,
@@ -305,7 +308,7 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
   const uint16_t* __restrict__ x = (GROUP && XFORM == 0) ? pick3(grp.x, gi) : x_;
   const int m = GROUP ? pick3(grp.m, gi) : m_;
   const int upw_q = GROUP ? pick3(grp.upw_q, gi) : upw_q_;
-  const int upw_r = GROUP ? pick3(grp.upw_r, gi) : upw_r_;
+  const int upw_r = GROUP ? pick3(grp.upw_r, gi) : (HALF == 2 ? upw_r_ & ((1 << kApartShift) - 1) : upw_r_);
   static_assert(!XHALF || (XLDS && !XFORM), "two-half staging is a form of the plain staged x");
   static_assert(!HALF || (XLDS && !POW2 && !XHALF && !GROUP), "half units exist for the plain form with x in LDS and behind a mix");
   // wave-loads requested before the table is built.  With half units both: a half wave-load is
@@ -345,13 +348,10 @@ __global__ __launch_bounds__(kThreads, 1) void matvec_kernel(
   const int upw = HALF ? upw_q : upw_q + (rb0 < upw_r ? 1 : 0);
   const int T_full = upw * npw;
   const bool has_half = HALF && rb0 < upw_r;
-  // Nothing but half units: the two of a block on one XCD (workgroups go round the eight of them), where the second reading of
-  // its stream hits in L2; the last ones, less than a round of pairs, side by side.  Behind whole units they lie side by side too: a
-  // pair on one XCD starts together and is 1 % slower.
-  const int lg = upw_q ? 0 : (gridDim.x == 1 ? 3 : (gridDim.x == 2 ? 2 : (gridDim.x == 4 ? 1 : 0)));
-  const bool paired = rb0 < (upw_r >> (lg + 1)) << (lg + 1);
-  const int half_rh = (paired ? rb0 >> lg : rb0) & 1;
-  const int half_rb = upw_q * rb_step + (paired ? ((rb0 >> (lg + 1)) << lg) + (rb0 & ((1 << lg) - 1)) : rb0 >> 1);
+  const int apart = HALF == 2 ? upw_r_ >> kApartShift : 0;
+  const int lg = HALF == 2 && rb0 < (upw_r >> (apart + 1)) << (apart + 1) ? apart : 0;
+  const int half_rh = (rb0 >> lg) & 1;
+  const int half_rb = upw_q * rb_step + (HALF == 2 ? ((rb0 >> (lg + 1)) << lg) + (rb0 & ((1 << lg) - 1)) : rb0 >> 1);
   const int T = T_full + (has_half ? npw : 0);
   const int w_first = wl0 + wave;
   const int nvj = w_first < wl1f ? (wl1f - w_first + kWaves - 1) / kWaves : 0;  // real items per unit
@@ -741,9 +741,10 @@ hipError_t allow_lds_all() {
   QTIP_ALLOW((matvec_kernel<2, 2, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<3, 2, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<4, 2, true>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<2, 2, true, 0, false, false, true>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<3, 2, true, 0, false, false, true>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW((matvec_kernel<4, 2, true, 0, false, false, true>), kMatvecLds + kMatvecXBytes)
+  QTIP_ALLOW((matvec_kernel<2, 2, true, 0, false, false, 1>), kMatvecLds + kMatvecXBytes)
+  QTIP_ALLOW((matvec_kernel<2, 2, true, 0, false, false, 2>), kMatvecLds + kMatvecXBytes)
+  QTIP_ALLOW((matvec_kernel<3, 2, true, 0, false, false, 2>), kMatvecLds + kMatvecXBytes)
+  QTIP_ALLOW((matvec_kernel<4, 2, true, 0, false, false, 2>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<2, 2, true, 0, false, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<3, 2, true, 0, false, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<4, 2, true, 0, false, true>), kMatvecLds + kMatvecXBytes)
@@ -751,10 +752,10 @@ hipError_t allow_lds_all() {
   QTIP_ALLOW((matvec_kernel<3, 2, true, 0, true>), kMatvecLds + kMatvecXBytes)
   QTIP_ALLOW((matvec_kernel<4, 2, true, 0, true>), kMatvecLds + kMatvecXBytes)
 #define QTIP_ALLOW_XFORM(BITS, EPT)                                                                       \
-  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 1, false, false, false, EPT>), xform_lds(1024 * EPT))           \
-  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 2, false, false, false, EPT>), xform_lds(1024 * EPT))           \
-  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 2, false, true, false, EPT>), xform_lds(1024 * EPT))            \
-  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 4, false, false, false, EPT>), xform_lds(1024 * EPT))
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 1, false, false, 0, EPT>), xform_lds(1024 * EPT))           \
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 2, false, false, 0, EPT>), xform_lds(1024 * EPT))           \
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 2, false, true, 0, EPT>), xform_lds(1024 * EPT))            \
+  QTIP_ALLOW((matvec_kernel<BITS, 2, true, 4, false, false, 0, EPT>), xform_lds(1024 * EPT))
   QTIP_ALLOW_XFORM(2, 2) QTIP_ALLOW_XFORM(2, 4) QTIP_ALLOW_XFORM(2, 8)
   QTIP_ALLOW_XFORM(3, 2) QTIP_ALLOW_XFORM(3, 4) QTIP_ALLOW_XFORM(3, 8)
   QTIP_ALLOW_XFORM(4, 2) QTIP_ALLOW_XFORM(4, 4) QTIP_ALLOW_XFORM(4, 8)
@@ -762,7 +763,7 @@ hipError_t allow_lds_all() {
 #define QTIP_ALLOW_MIX(BITS, HALF)                                                                         \
   QTIP_ALLOW((matvec_kernel<BITS, 2, true, 3, false, false, HALF, 2>), kMatvecLds + kMatvecXBytes)         \
   QTIP_ALLOW((matvec_kernel<BITS, 2, true, 3, false, false, HALF, 4>), kMatvecLds + kMatvecXBytes)
-  QTIP_ALLOW_MIX(2, false) QTIP_ALLOW_MIX(2, true) QTIP_ALLOW_MIX(3, false) QTIP_ALLOW_MIX(4, false)
+  QTIP_ALLOW_MIX(2, 0) QTIP_ALLOW_MIX(2, 1) QTIP_ALLOW_MIX(2, 2) QTIP_ALLOW_MIX(3, 0) QTIP_ALLOW_MIX(4, 0)
 #undef QTIP_ALLOW_MIX
 #undef QTIP_ALLOW
   return hipSuccess;
@@ -941,15 +942,15 @@ size_t qtip_matvec_workspace_bytes(int m, int k, int bits) {
 // the kernel with a transform in front for `bits` and k = 2048, 4096 or 8192, on grid g2 with lds bytes
 #define QTIP_XFORM(MODE, GROUP, ARGS)                                                       \
   switch (16 * bits + (k >> 10)) {                                                          \
-    case 34: matvec_kernel<2, 2, true, MODE, false, GROUP, false, 2><<<g2, kThreads, lds, st>>>ARGS; break; \
-    case 36: matvec_kernel<2, 2, true, MODE, false, GROUP, false, 4><<<g2, kThreads, lds, st>>>ARGS; break; \
-    case 40: matvec_kernel<2, 2, true, MODE, false, GROUP, false, 8><<<g2, kThreads, lds, st>>>ARGS; break; \
-    case 50: matvec_kernel<3, 2, true, MODE, false, GROUP, false, 2><<<g2, kThreads, lds, st>>>ARGS; break; \
-    case 52: matvec_kernel<3, 2, true, MODE, false, GROUP, false, 4><<<g2, kThreads, lds, st>>>ARGS; break; \
-    case 56: matvec_kernel<3, 2, true, MODE, false, GROUP, false, 8><<<g2, kThreads, lds, st>>>ARGS; break; \
-    case 66: matvec_kernel<4, 2, true, MODE, false, GROUP, false, 2><<<g2, kThreads, lds, st>>>ARGS; break; \
-    case 68: matvec_kernel<4, 2, true, MODE, false, GROUP, false, 4><<<g2, kThreads, lds, st>>>ARGS; break; \
-    default: matvec_kernel<4, 2, true, MODE, false, GROUP, false, 8><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 34: matvec_kernel<2, 2, true, MODE, false, GROUP, 0, 2><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 36: matvec_kernel<2, 2, true, MODE, false, GROUP, 0, 4><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 40: matvec_kernel<2, 2, true, MODE, false, GROUP, 0, 8><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 50: matvec_kernel<3, 2, true, MODE, false, GROUP, 0, 2><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 52: matvec_kernel<3, 2, true, MODE, false, GROUP, 0, 4><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 56: matvec_kernel<3, 2, true, MODE, false, GROUP, 0, 8><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 66: matvec_kernel<4, 2, true, MODE, false, GROUP, 0, 2><<<g2, kThreads, lds, st>>>ARGS; break; \
+    case 68: matvec_kernel<4, 2, true, MODE, false, GROUP, 0, 4><<<g2, kThreads, lds, st>>>ARGS; break; \
+    default: matvec_kernel<4, 2, true, MODE, false, GROUP, 0, 8><<<g2, kThreads, lds, st>>>ARGS; break; \
   }
 
 static int launch_matvec(const Ready& di, float* dst, const void* packed, const void* x_f16, const void* tlut,
@@ -988,25 +989,30 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
   const int left = full_range > 0 ? (m >> 5) % full_range : 0;
   const int whole = full_range > 0 ? (m >> 5) / full_range : 0;
   const bool half = half_units(bits, left, whole, full_range, S, wl_per, di.cus);
+  const int apart = half_apart(bits, left, whole, S, wl_per, di.cus);
+  const bool aside = bits == 2 && apart == 0;  // (3 and 4 bits have the form of halves that lie apart alone)
+  const int half_r = aside ? 2 * left : 2 * left | apart << kApartShift;
   if (mix) {
     const int cols = k / mix->on;
     const size_t lds = kMatvecLds + kMatvecXBytes;
     auto* sg = (const uint16_t*)su_f16;
     const bool halves = half && bits == 2;  // (not measured at 3 and 4)
     const dim3 gh = halves ? dim3((unsigned)S, (unsigned)(whole > 0 ? full_range : 2 * left)) : g2;
-    const int q = halves ? whole : uq, r = halves ? 2 * left : ur;
+    const int q = halves ? whole : uq, r = halves ? half_r : ur;
 #define QTIP_MIX(BITS, HALF)                                                                                                     \
   if (cols == 64) matvec_kernel<BITS, 2, true, 3, false, false, HALF, 4><<<gh, kThreads, lds, st>>>(                            \
       dst, p, xx, t, m, k, wl_per, q, r, sg, xscale, ChainArgs{}, GroupArgs{}, *mix);                                            \
   else matvec_kernel<BITS, 2, true, 3, false, false, HALF, 2><<<gh, kThreads, lds, st>>>(                                        \
       dst, p, xx, t, m, k, wl_per, q, r, sg, xscale, ChainArgs{}, GroupArgs{}, *mix)
-    if (halves) {
-      QTIP_MIX(2, true);
+    if (halves && aside) {
+      QTIP_MIX(2, 1);
+    } else if (halves) {
+      QTIP_MIX(2, 2);
     } else {
       switch (bits) {
-        case 2: QTIP_MIX(2, false); break;
-        case 3: QTIP_MIX(3, false); break;
-        default: QTIP_MIX(4, false); break;
+        case 2: QTIP_MIX(2, 0); break;
+        case 3: QTIP_MIX(3, 0); break;
+        default: QTIP_MIX(4, 0); break;
       }
     }
 #undef QTIP_MIX
@@ -1016,9 +1022,12 @@ static int launch_matvec(const Ready& di, float* dst, const void* packed, const 
     const dim3 gh((unsigned)S, (unsigned)(whole > 0 ? full_range : 2 * left));
     const size_t lds = kMatvecLds + xbytes;
     switch (bits) {
-      case 2: matvec_kernel<2, 2, true, 0, false, false, true><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, 2 * left); break;
-      case 3: matvec_kernel<3, 2, true, 0, false, false, true><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, 2 * left); break;
-      default: matvec_kernel<4, 2, true, 0, false, false, true><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, 2 * left); break;
+      case 2:
+        if (aside) matvec_kernel<2, 2, true, 0, false, false, 1><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, half_r);
+        else matvec_kernel<2, 2, true, 0, false, false, 2><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, half_r);
+        break;
+      case 3: matvec_kernel<3, 2, true, 0, false, false, 2><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, half_r); break;
+      default: matvec_kernel<4, 2, true, 0, false, false, 2><<<gh, kThreads, lds, st>>>(dst, p, xx, t, m, k, wl_per, whole, half_r); break;
     }
     return (int)hipGetLastError();
   }
