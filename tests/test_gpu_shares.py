@@ -102,3 +102,29 @@ def test_a_further_request_needs_no_eager_step(monkeypatch):
     assert torch.equal(generate(model, a, 12)[0], got) and steps == [False, True]
     drawn = [generate(model, b, 12, temperature=0.7, top_k=4)[0] for _ in range(2) if torch.manual_seed(7)]
     assert torch.equal(*drawn)
+
+
+@pytest.mark.parametrize("fused", (True, False))
+def test_a_callers_own_ranges_run_in_the_attentions_own_launch(fused, monkeypatch):
+    """Which launches a token takes: ranges by the position and o's matvec on their shares, or the caller's count of ranges."""
+    cfg = LlamaConfig(hidden=2048, heads=16, kv_heads=4, layers=2, ffn=172 * 32, vocab=512)
+    model = LlamaDecoder(cfg, max_cache_len=512, fused=fused)
+    tok, pos = torch.zeros(1, 1, dtype=torch.int64, device="cuda"), torch.tensor([400], device="cuda")
+    took = []
+
+    def watch(name):
+        inner = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda *args, **kw: took.append((name, kw.get("key_splits"))) or inner(*args, **kw))
+
+    own = "decode_attention_rht" if fused else "decode_attention_rht3"
+    for name in ("decode_attention_shares", "decompress_matvec_parts_shares", "decode_attention", "decode_attention_rht",
+                 "decode_attention_rht3"):
+        watch(name)
+    with torch.no_grad():
+        model.decode_fused(tok, pos)
+        assert took == [("decode_attention_shares", None), ("decompress_matvec_parts_shares", None)] * 2
+        for ranges in (3, 8):
+            del took[:]
+            cfg.attn_key_splits = ranges
+            model.decode_fused(tok, pos)
+            assert took == [(own, ranges)] * 2
