@@ -26,6 +26,7 @@ Prints ONE JSON line:  value = packed bytes streamed per second (GB/s), plus
 import argparse
 import json
 import os
+import re
 import sys
 import time
 
@@ -36,15 +37,25 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this script, each calibrated
 # against a 256 MiB copy) are read from this summary, which names the kernel sources it was taken on
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "matvec_k2_llama70b_set_traffic.txt")
-KERNEL_SOURCES = ("qtip_amd/csrc/qtip_hip.hip", "qtip_amd/csrc/qtip_device.h", "qtip_amd/csrc/qtip_wht.h",
-                  "qtip_amd/csrc/qtip_chain.h")
+KERNEL_DIR = os.path.join(ROOT, "qtip_amd", "csrc")
+
+
+def kernel_sources(name="qtip_hip.hip", seen=()):
+    """The matvec's translation unit: its file and, in the order of their includes, the headers beside it."""
+    with open(os.path.join(KERNEL_DIR, name)) as f:
+        included = re.findall(r'^#include "([^"/]+)"', f.read(), re.M)
+    seen = (*seen, name)
+    for header in included:
+        if header not in seen:
+            seen = kernel_sources(header, seen)
+    return seen
 
 
 def kernel_source_digest():
     import hashlib
     h = hashlib.sha256()
-    for rel in KERNEL_SOURCES:
-        with open(os.path.join(ROOT, rel), "rb") as f:
+    for name in kernel_sources():
+        with open(os.path.join(KERNEL_DIR, name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]
 

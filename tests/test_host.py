@@ -516,3 +516,16 @@ def test_sign_rows_are_made_once():
         bits = mh.had_bits(None, K, True, "cpu") if K > 1 else None
         assert mh.sign_rows(bits, K, A, "cpu") is mh.sign_rows(bits, K, A, "cpu")
     assert not torch.equal(mh.sign_rows(None, 1, 32, "cpu")[:256], mh.sign_rows(None, 1, 64, "cpu")[:256])
+
+
+def test_bench_names_every_kernel_source_of_its_traffic_figure():
+    """The digest that the counter figure is tied to covers the matvec's file and every header beside it that it includes."""
+    import os
+    import bench
+    sources = bench.kernel_sources()
+    assert len(set(sources)) == len(sources) and sources[0] == "qtip_hip.hip"
+    for name in sources:
+        with open(os.path.join(bench.KERNEL_DIR, name)) as f:
+            lines = [l.split('"')[1] for l in f if l.startswith("#include \"") and "/" not in l.split('"')[1]]
+        assert set(lines) <= set(sources), name
+    assert {"qtip_chain.h", "qtip_device.h", "qtip_mix.h", "qtip_setup.h", "qtip_shares.h", "qtip_wht.h"} <= set(sources)
