@@ -84,9 +84,9 @@ __global__ __launch_bounds__(kBlock) void cache_rows_kernel(
 // infinite value times a rest of zero is a NaN where times the probability it is infinite, and is left out.
 // Bound by a wave's chain through a tile (products, maximum, exponentials, products), and 16-query waves give two workgroups
 // per CU at 1000 tokens of 32 heads: so it matters which two.  With a head's workgroups side by side an XCD had those of two lengths
-// only, 2.4 times as many keys as another, and a CU two of the same length.  us, 1000 tokens, 32 heads of 128: 46.7, in the order
-// below, with no mask where every key is seen and no product where the maximum stays, 36.8; and 8 for the caches, where the
-// library's attention under a dense mask took 193 beside about 150 of small passes (rotation, cache writes, copies of heads).
+// only, 2.4 times as many keys as another, and a CU two of the same length.  us with the launch for the caches, 1000 tokens, 32 heads
+// of 128: 50.7, with no mask where every key is seen 49.8, in the order below too 40.6; the library's attention under a dense mask
+// took 193 beside about 150 of small passes (rotation, cache writes, copies of heads).
 constexpr int kQ = 64, kKeys = 64;
 
 // the larger of v and lane ^ 16 (b = 4) or lane ^ 32 (5)
@@ -218,16 +218,16 @@ __global__ __launch_bounds__(kBlock, 2) void prefill_attn_kernel(
     tile_max = lane_max(tile_max, 4);
     tile_max = lane_max(tile_max, 5);
     const float base = fmaxf(tile_max, -3.0e38f);  // (nothing but scores of -inf so far)
-    if (__any(tile_max != mx)) {  // (a maximum that stays leaves the outputs as they are)
-      const float fade = __builtin_amdgcn_exp2f(mx - base);
-      sum *= fade;
-#pragma unroll
-      for (int e = 0; e < NE; ++e) {
-        o[e] *= fade;
-        rest_o[e] *= fade;
-      }
-    }
+    // (Also where the maximum stays, by 1: behind a branch that asks the wave for a maximum that changed the fade and the sum's first
+    // addition are two roundings, and 1000 tokens of 32 heads of 128 take 41.8 us, without it 40.6; 16 heads 33.8 and 32.8.)
+    const float fade = __builtin_amdgcn_exp2f(mx - base);
     mx = tile_max;
+    sum *= fade;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      o[e] *= fade;
+      rest_o[e] *= fade;
+    }
     half8v p[2], rest[2];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
