@@ -544,6 +544,12 @@ def _causal_mask(slots, cache_position):
     return (torch.arange(slots, device=cache_position.device)[None, :] <= cache_position[:, None])[None, None]
 
 
+# Values of a range of k up to which a transform runs inside its matvec: every workgroup makes its whole range.  us from cold memory, two
+# launches / one, to 8192 rows in one range, 2, 3 and 4 bits: 11008 12.8/12.5, 14.8/14.4 and 16.0/15.4; 13824 14.4/15.1, 16.8/17.1 and
+# 18.0/18.5; 14336 14.6/15.2, 17.5/17.5 and 18.8/18.9; in four ranges 14336 to 5120 rows 13.0/12.2, 14.4/13.6 and 15.0/13.6
+MIX_RANGE = 12288
+
+
 class _FusedLinear:
     """The three launches of a bs=1 QuantizedLinear with the neighbouring element-wise work of
     the decoder layer folded into the two transforms (RMSNorm or SiLU*up on the way in, the
@@ -587,7 +593,9 @@ class _FusedLinear:
             if dev.type == "cuda" and not self.shard_in:
                 if torch.cuda.is_current_stream_capturing():
                     return None
-                cols = ops.matvec_mix_columns(self.n, self.Kl, ops.matvec_split(self.m, self.n, self.K, dev))
+                split = ops.matvec_split(self.m, self.n, self.K, dev)
+                if self.n <= MIX_RANGE * split:
+                    cols = ops.matvec_mix_columns(self.n, self.Kl, split)
             self._mix_rows = sign_rows(self.bl, self.Kl, self.n // cols // self.Kl, dev) if cols else None
         return self._mix_rows
 

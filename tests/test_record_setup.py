@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from qtip_amd import llama_decode, ops
+from qtip_amd.linear.quantized_linear import QuantizedLinear
 from qtip_amd.llama_decode import DecoderLayer, LlamaConfig, LlamaDecoder, generate
 
 SETUP = ("_fused", "_grouped", "_grouped_plain")
@@ -208,3 +209,10 @@ def test_a_step_recorded_behind_a_prompt():
             torch.cuda.synchronize()
             # (down's input transform may give the neighbouring value in fp16)
             assert (got - want).norm() <= 2.5e-3 * want.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,inside", ((8192, 11008, True), (8192, 13824, False), (8192, 14336, False), (5120, 14336, True), (4096, 14336, True)))
+def test_a_transform_inside_a_matvec_makes_a_range_that_pays(m, k, inside):
+    lin = QuantizedLinear(k, m, 16, 16, 16, 2, 2, 9, "quantlut_sym", dtype=torch.float16, mode="eval").cuda()
+    assert (llama_decode._FusedLinear(lin).mix_rows() is not None) == inside
