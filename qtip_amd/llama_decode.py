@@ -270,12 +270,11 @@ class DecoderLayer(nn.Module):
         layout (4 x [transform, matvec, transform] + attention, the attention kernel doing the qkv
         output transform itself), 24 for the separate projections.
         With power-of-two hidden sizes the [transform-out + residual] of o / down and the
-        [RMSNorm + transform-in] that follows are one launch and the o projection transforms its
-        input inside the matvec (9 per layer); where it pays, that one launch is the following
-        matvec itself (7 per layer): `qkv_parts` are then the partial sums of this layer's qkv matvec
-        (launched by the previous layer with the layer boundary in its prologue) and `next_layer` the
-        layer whose qkv matvec this one launches.  A table transform in front of down (ops.matvec_mix_columns) is inside down's
-        matvec, a launch less.  Returns (x, qkv partial sums for the next layer).
+        [RMSNorm + transform-in] that follows run in front of the following matvec, in its launch, and o transforms its input
+        inside its own: 7 per layer, [attention, o, boundary + up_gate, its output transform with SiLU(gate) * up, down's input
+        transform, down, boundary + the next layer's qkv], or 6 where a table transform in front of down is inside down's
+        matvec (ops.matvec_mix_columns).  `qkv_parts` are the partial sums of this layer's qkv matvec (launched by the previous
+        layer) and `next_layer` the layer whose qkv matvec this one launches.  Returns (x, qkv partial sums for the next layer).
         open_end (no next layer): where down's output transform and the residual addition can be left to the caller, x is
         the residual stream in front of them and the partial sums are down's."""
         cfg = self.cfg
@@ -459,11 +458,11 @@ class DecoderLayer(nn.Module):
             residual, norm_weight, self.cfg.eps, [l.SU for l in ls], (ls[0].n**-0.5) / 32.0)
 
     def _decode_grouped(self, x, k_cache, v_cache, pos, inv_freq, qkv_parts, next_layer, open_end=False):
-        """decode_fused for separate projections, 8 launches: [boundary + q, k, v matvecs] (by the
+        """decode_fused for separate projections, 7 launches: [boundary + q, k, v matvecs] (by the
         previous layer, or the first for itself), attention with the three output transforms in its prologue, o matvec with
         its input transform, [boundary + gate, up matvecs], both output transforms (with SiLU * up in
         the same launch for vectors above 4096), [SiLU * up +] input transform of down, down
-        matvec; 7 where down's matvec transforms its input itself.  Returns (x, partial sums of the next layer's q, k, v)."""
+        matvec; 6 where down's matvec transforms its input itself.  Returns (x, partial sums of the next layer's q, k, v)."""
         cfg = self.cfg
         f = self._fused_linears()
         qkv = [f[n] for n in ('q_proj', 'k_proj', 'v_proj')]

@@ -738,7 +738,8 @@ def decode_attention_rht3(parts, post, scale, had_bits, order, k_cache, v_cache,
 
 
 def attention_share_ranges(heads):
-    """Ranges of the keys that decode_attention_shares has room for: as many as leave the chip's 256 CUs a workgroup each."""
+    """Ranges of the keys that decode_attention_shares has room for: up to four, which is what o's matvec reads, and as many as leave
+    each of 256 compute units a workgroup."""
     return max(1, min(4, 256 // heads))
 
 
