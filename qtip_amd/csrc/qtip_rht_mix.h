@@ -81,7 +81,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   const int lrows = 7 - logpp;  // log2 of the rows per pass
   const int rsub = (8 * a) >> logpp, c0 = (8 * a) & ((1 << logpp) - 1);
   // a result's columns are those of the lane's place, which the operands are read for
-  const int pa_in = wht_place(lane) & 15;
+  int pa = wht_place(lane) & 15, rsub_out = (8 * pa) >> logpp, c0_out = (8 * pa) & ((1 << logpp) - 1);
   const int Am = (1 << logA2) - 1;
   // element j, slice part sl inside a row
   auto element = [&](int j, int sl) {
@@ -230,9 +230,13 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
   auto finish = [&](float4v acc[8], int ps) {
     if (idle) return;
     if constexpr (!AUX) asm volatile("" ::"v"(line));
-    int own = lane;
-    asm("" : "+v"(own));  // (the place again: kept over the products it cost the SiLU form of 256 rows a register to scratch)
-    const int pa = wht_place(own) & 15, rsub_out = (8 * pa) >> logpp, c0_out = (8 * pa) & ((1 << logpp) - 1);
+    if constexpr (MODE == PRE_SILU_MUL && KTC == 8) {
+      // (Taken again: kept over the products they cost this form a register to scratch, 16 rows of 28672 9.8 us, so 9.3.  The
+      // other forms have the registers for them; taken again there, 1000 rows are 1 to 4 % slower.)
+      int own = lane;
+      asm("" : "+v"(own));
+      pa = wht_place(own) & 15, rsub_out = (8 * pa) >> logpp, c0_out = (8 * pa) & ((1 << logpp) - 1);
+    }
 #pragma unroll
     for (int h = 1; h < 8; h <<= 1)
 #pragma unroll
@@ -290,7 +294,7 @@ __global__ __launch_bounds__(128 * KTC, 4) void rht_mix_kernel(const RhtParams P
     }
   };
   uint8_t* wr = mix_smem + (uint32_t)a * stride + (uint32_t)(4 * wave + g) * 8;
-  const uint8_t* rd = mix_smem + (uint32_t)pa_in * stride + (uint32_t)g * 16;
+  const uint8_t* rd = mix_smem + (uint32_t)pa * stride + (uint32_t)g * 16;
   // the plane's products: a column group's next operand is requested as soon as its present one is used
   auto products = [&](float4v acc[8], uint32_t one, auto mfma) {
     if (idle) return;
