@@ -263,7 +263,14 @@ class DecoderLayer(nn.Module):
         behind this call: dropped set-up is made anew, outside of a recording, and with no form."""
         self._fused_linears()
         self.grouped_ok() or self.grouped_plain_ok()
-        return self.__dict__.setdefault('_recorded', set())  # (a layer from a file may have set-up alone)
+        return self._recorded
+
+    def __setstate__(self, state):
+        """A copy or a layer from a file makes its set-up anew: the classes of this module may have changed since it was written, and
+        what has been recorded belongs to one process."""
+        super().__setstate__(state)
+        for name in ('_fused', '_grouped', '_grouped_plain', '_recorded'):
+            self.__dict__.pop(name, None)
 
     def decode_fused(self, x, k_cache, v_cache, pos, inv_freq, qkv_parts=None, next_layer=None, open_end=False):
         """One new token, x (1, hidden) fp16, on the fused transforms: 12 launches for the fused
@@ -847,9 +854,6 @@ def sample(logits, temperature=1.0, top_k=None):
     return torch.argmax(probs / q, dim=-1, keepdim=True), probs
 
 
-_PROCESS = object()  # (part of a recorded form, which a copy or a file of a layer brings along: it is equal to itself alone)
-
-
 @torch.no_grad()
 def generate(model, prompt_ids, max_new_tokens, use_graph=True, fused=True, temperature=None, top_k=None,
              callback=None):
@@ -910,7 +914,7 @@ def generate(model, prompt_ids, max_new_tokens, use_graph=True, fused=True, temp
         of it recorded yet; the decode state is put back afterwards, so a capture in the middle of a run leaves it untouched."""
         # What an eager step sets up stays with the layers and the process; recording runs nothing.  A further request on a
         # model of 8 layers of 4096 starts 1.6 ms earlier for it.  (Only a layer of this module tells what it keeps.)
-        form = (sampling, model.cfg.attn_key_splits, dev, _PROCESS)
+        form = (sampling, model.cfg.attn_key_splits, dev)
         own = [layer for layer in model.layers if type(layer) is DecoderLayer and 'decode_fused' not in layer.__dict__]
         ready = on_device and len(own) == len(model.layers) and all(form in layer.recorded_forms() for layer in own)
         keep = (static_tok.clone(), static_pos.clone(), history.clone(), draw_counter.clone())

@@ -142,6 +142,22 @@ def test_a_copy_has_nothing_recorded(steps, through):
     assert steps.seen == [(True, True)]
 
 
+@pytest.mark.parametrize("through", (copy.copy, copy.deepcopy, lambda model: pickle.loads(pickle.dumps(model))))
+def test_a_model_from_a_file_makes_its_set_up_anew(through):
+    """Set-up written by an earlier version lacks what this one keeps with it."""
+    cfg = LlamaConfig(**TABLE_ORDER)
+    model = LlamaDecoder(cfg, max_cache_len=32, device="cpu", random_init=False, fused=False)
+    for layer in model.layers:
+        assert layer.grouped_plain_ok()
+        for lin in layer._fused_linears().values():
+            lin.__dict__.pop("_mix_rows")
+    for layer in (through(layer) for layer in model.layers):
+        assert not any(name in layer.__dict__ for name in SETUP)
+        assert all("_mix_rows" in lin.__dict__ for lin in layer._fused_linears().values()) and layer.grouped_plain_ok()
+        assert torch.equal(layer._su_qkv, torch.stack([layer.q_proj.SU, layer.k_proj.SU, layer.v_proj.SU]))
+    assert all(name in layer.__dict__ for layer in model.layers for name in SETUP)  # (the copied ones keep theirs)
+
+
 def test_a_recording_that_fails_ends_the_request(steps, monkeypatch):
     """One attempt: the library's stream is not the caller's any more after a recording that was cut off."""
     model = _host_model(steps, POWER_OF_2)
